@@ -117,9 +117,6 @@ __device__ __forceinline__ uint32_t f32_to_e4m3(float x) {
   return sign | (uint32_t)__builtin_rintf(a * 512.0f);  // sub-normal grid 2^-9, 8 -> 2^-6
 }
 
-__device__ __constant__ const float kE2M1[16] = {0.0f,  0.5f,  1.0f,  1.5f,  2.0f,  3.0f,  4.0f,  6.0f,
-                                                 -0.0f, -0.5f, -1.0f, -1.5f, -2.0f, -3.0f, -4.0f, -6.0f};
-
 // Offset of scale (r, c) of a [rows, cols] e4m3 matrix stored in 128x4 blocked order.
 __host__ __device__ __forceinline__ int64_t blocked_scale_offset(int64_t r, int64_t c, int64_t cols) {
   int64_t rb = r >> 7, ri = r & 127, cb = c >> 2, ci = c & 3;

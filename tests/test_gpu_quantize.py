@@ -142,6 +142,25 @@ def test_dequantize_matches_oracle(gpu, rule, dtype):
         assert torch.equal(got.cpu(), torch.from_numpy(ref).to(dtype))
 
 
+@pytest.mark.parametrize("shape", [(1, 16), (31, 250), (32, 256), (129, 264), (256, 520)])
+@pytest.mark.parametrize("amax", [0.0, 1e-35, 1.7, 3e35])
+def test_dequantize_every_code_and_scale_byte(gpu, shape, amax):
+    """Random bytes (all codes, all finite scale bytes of both signs) at the edges of the kernel's 32 x 256 tiles, with
+    amax values inside and outside the range in which it scales by powers of two: equal to the oracle's divisions."""
+    from longlive_amd._native import padded_shape
+    rng = np.random.default_rng(5)
+    mp, kp = padded_shape(shape)
+    v = rng.integers(0, 256, (mp, kp // 2), dtype=np.uint8)
+    s = rng.integers(0, 256, mp * kp // 16, dtype=np.uint8)
+    s[(s & 0x7F) == 0x7F] = 0x7E
+    q = QuantizedTensor(torch.from_numpy(v).to(gpu), torch.from_numpy(s).to(gpu).view(torch.float8_e4m3fn),
+                        torch.tensor([amax], device=gpu), "nvfp4", shape, "mse", (mp, kp))
+    ref = o.dequantize(v, s, np.float32(amax), "mse", (mp, kp), shape)
+    got = q.dequantize(torch.float32).cpu().numpy()
+    assert np.array_equal(got.view(np.uint32), np.ascontiguousarray(ref).view(np.uint32))
+    assert torch.equal(q.dequantize(torch.bfloat16).cpu(), torch.from_numpy(ref).bfloat16())
+
+
 def test_dequantize_golden(golden, gpu):
     for name, shape in (("randn_128x512_s1", (128, 512)), ("weights_256x512_s2", (256, 512))):
         v, s, a = (golden[f"{name}/mse/{k}"] for k in ("values", "scales", "amax"))

@@ -18,6 +18,8 @@ LIB_PATH = os.path.join(_HERE, "csrc", "libll_nvfp4.so")
 HEADER_PATH = os.path.join(os.path.dirname(_HERE), "include", "ll_nvfp4.h")
 
 RULE_IDS = {"static_6": 0, "static_4": 1, "mae": 2, "mse": 3, "abs_max": 4}
+# e2m1_max * e4m3_max of a scale rule: what the tensor amax is divided by
+DENOMINATORS = {"static_6": 2688.0, "static_4": 1792.0, "mae": 1536.0, "mse": 1536.0, "abs_max": 1536.0}
 # looks (1-2 us each) a workgroup of a launch whose workgroups exchange their maxima waits for the others
 NORM_QUANTIZE_SPIN_LIMIT = 64
 DTYPE_CODES = {torch.bfloat16: 0, torch.float16: 1, torch.float32: 2}
@@ -120,6 +122,23 @@ def load():
         fn.argtypes = args
     _lib = lib
     return lib
+
+
+_host = None
+
+
+def host():
+    """The native host path (csrc/host_ops.cpp): whole calls from tensors to launches.  Raises if it has not been built."""
+    global _host
+    if _host is None:
+        load()
+        try:
+            from . import _host_ops
+        except ImportError as e:
+            raise RuntimeError(f"longlive_amd/_host_ops.so is missing or does not load ({e}): build it with "
+                               "`python -c 'import __graft_entry__ as g; g.build()'`") from e
+        _host = _host_ops
+    return _host
 
 
 def _check(code: int, what: str) -> None:
@@ -318,6 +337,10 @@ def quantize(x: torch.Tensor, rule: str, amax: torch.Tensor | None = None, out=N
     ``out`` = (values, scale_factors, amax) buffers of exactly those shapes to write into (KV slots).
     ``amax``: a float32[1] tensor to quantize against, or the :class:`AmaxTicket` the producer of ``x`` was
     given, in which case the bytes equal those of ``amax=None``."""
+    if amax is None and out is None:
+        res = host().quantize(x, RULE_IDS[rule])
+        if res is not None:
+            return res
     ticket = amax if isinstance(amax, AmaxTicket) else None
     if ticket is not None:
         _check_consumer(ticket)
@@ -399,6 +422,9 @@ def quantize_pair(x0: torch.Tensor, x1: torch.Tensor, rule: str, ticket0: AmaxTi
 
 
 def dequantize(values, scales, amax, rule: str, padded, original, dtype: torch.dtype) -> torch.Tensor:
+    out = host().dequantize(values, scales, amax, RULE_IDS[rule], *padded, *original, DTYPE_CODES[dtype])
+    if out is not None:
+        return out
     _require_cuda(values, scales, amax)
     out = torch.empty(original, dtype=dtype, device=values.device)
     with torch.cuda.device(values.device):

@@ -54,8 +54,8 @@ def fp4_matmul(
         input.values, input.scale_factors, other.values, other.scale_factors,
         input.original_shape[0], other.original_shape[0],
         amax_a=input.amax, amax_b=other.amax,
-        denom_a=float(input.scale_rule.max_allowed_e2m1_value() * input.scale_rule.max_allowed_e4m3_value()),
-        denom_b=float(other.scale_rule.max_allowed_e2m1_value() * other.scale_rule.max_allowed_e4m3_value()),
+        denom_a=_native.DENOMINATORS[input.scale_rule.value],
+        denom_b=_native.DENOMINATORS[other.scale_rule.value],
         bias=bias,
         activation=activation,
         residual=residual,

@@ -8,8 +8,11 @@ from typing import Any
 import torch
 import torch.nn as nn
 
+from .... import _native
 from ...matmul import fp4_matmul
 from ...quantize import QuantizationConfig, QuantizedTensor, quantize_to_fp4
+from ...quantize.frontend import _unsupported
+from ...utils import DataType
 from ..config import ModuleQuantizationConfig
 from ..quantize import QuantizedModule
 
@@ -122,6 +125,16 @@ class FourOverSixLinear(nn.Linear):
         return out.reshape(*input.shape[:-1], out.shape[-1])
 
     def _forward_2d(self, x2d: torch.Tensor) -> torch.Tensor:
+        weight, config = self.quantized_weight(), self.config
+        if (isinstance(weight, QuantizedTensor) and config.output_dtype is DataType.bfloat16 and config.dtype is DataType.nvfp4
+                and weight.original_shape[1] == x2d.shape[1]):
+            # quantization and product as one native call; the operand between them has no other reader
+            rule = config.activation_scale_rule._value_
+            out = _native.host().linear(x2d, _native.RULE_IDS[rule], _native.DENOMINATORS[rule], weight.values, weight.scale_factors,
+                                        weight.amax, _native.DENOMINATORS[weight.scale_rule._value_], weight.original_shape[0],
+                                        self._parameters.get("bias"))
+            if out is not None:
+                return out
         return self.forward_quantized(self.quantize_input(x2d))
 
     def quantize_input(self, x2d: torch.Tensor, amax=None) -> QuantizedTensor:
@@ -137,9 +150,6 @@ class FourOverSixLinear(nn.Linear):
         normalization and the layer's quantization separately, wan_5b/modules/causal_model.py:869-878, 892-906,
         909-918).  The bytes are those of the separate operations.  ``None`` when that launch does not take the
         input or the activation config, and the caller runs the separate operations."""
-        from .... import _native
-        from ...quantize.frontend import _unsupported
-
         config = self.config.get_activation_config()
         if not (x.is_cuda and x.dtype == torch.bfloat16 and x.ndim == 3 and x.is_contiguous()) or \
                 _unsupported(x[0], config) is not None:
@@ -164,8 +174,6 @@ class FourOverSixLinear(nn.Linear):
         (the q / k / v projections of an attention layer): the products are computed exactly as they would be
         alone, only the cost of two launches and of two half-empty rounds of workgroups is saved.  ``amax_outs``:
         one amax ticket or ``None`` per layer."""
-        from .... import _native
-
         amax_outs = amax_outs or [None] * len(layers)
         weights = [m.quantized_weight() for m in layers]
         same = (1 < len(layers) <= 4 and all(isinstance(w, QuantizedTensor) for w in weights)
@@ -177,10 +185,9 @@ class FourOverSixLinear(nn.Linear):
                 and len({t.parts.data_ptr() for t in amax_outs if t is not None}) == sum(t is not None for t in amax_outs))
         if not same:
             return [m.forward_quantized(xq, amax_out=t) for m, t in zip(layers, amax_outs)]
-        denom = lambda q: float(q.scale_rule.max_allowed_e2m1_value() * q.scale_rule.max_allowed_e4m3_value())
-        products = [dict(values=w.values, scales=w.scale_factors, amax=w.amax, denom=denom(w), bias=m.bias, amax_out=t)
+        products = [dict(values=w.values, scales=w.scale_factors, amax=w.amax, denom=_native.DENOMINATORS[w.scale_rule.value], bias=m.bias, amax_out=t)
                     for m, w, t in zip(layers, weights, amax_outs)]
-        return _native.gemm_grouped(xq.values, xq.scale_factors, xq.amax, denom(xq), xq.original_shape[0],
+        return _native.gemm_grouped(xq.values, xq.scale_factors, xq.amax, _native.DENOMINATORS[xq.scale_rule.value], xq.original_shape[0],
                                     weights[0].original_shape[0], products)
 
     def forward_quantized(self, xq: QuantizedTensor, activation: str | None = None, *,

@@ -13,6 +13,9 @@ from .config import QuantizationConfig
 from .quantized_tensor import QuantizedTensor
 
 
+_DEFAULT = QuantizationConfig()
+
+
 def _unsupported(x: torch.Tensor, config: QuantizationConfig) -> str | None:
     if x.ndim != 2:
         return "input must be 2-D"
@@ -39,11 +42,11 @@ def quantize_to_fp4(x: torch.Tensor, config: QuantizationConfig | None = None, *
     that the kernel which produced ``x`` was given; the reduction pass over ``x`` is then skipped.
     """
     if config is None:
-        config = QuantizationConfig()
+        config = _DEFAULT
     why = _unsupported(x, config)
     if why is not None:
         backend = config.backend.value if config.backend is not None else "hip"
         raise ValueError(f"Backend {backend} does not support the given parameters: {why}")
     values, scales, amax = _native.quantize(x, config.scale_rule.value, amax=amax)
-    return QuantizedTensor(values, scales, amax, config.dtype, tuple(x.shape), config.scale_rule,
-                           _native.padded_shape(tuple(x.shape)))
+    return QuantizedTensor.of_kernel(values, scales, amax, config.dtype, tuple(x.shape), config.scale_rule,
+                                     (values.shape[0], 2 * values.shape[1]))

@@ -55,6 +55,14 @@ class QuantizedTensor:
         self.scale_factors = scale_factors
         self.amax = amax
 
+    @classmethod
+    def of_kernel(cls, values, scale_factors, amax, dtype, original_shape, scale_rule, padded_shape) -> "QuantizedTensor":
+        """A tensor from what the quantizer itself returned: nothing to convert, pad or check."""
+        q = cls.__new__(cls)
+        q.dtype, q.original_shape, q.scale_rule, q.padded_shape = dtype, original_shape, scale_rule, padded_shape
+        q.values, q.scale_factors, q.amax = values, scale_factors, amax
+        return q
+
     def dequantize(self, dtype: torch.dtype = torch.bfloat16) -> torch.Tensor:
         """``((e2m1 * e4m3) * amax) / (e2m1_max * e4m3_max)`` cast to ``dtype``, sliced to the
         original shape (HIP kernel)."""

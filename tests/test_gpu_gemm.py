@@ -670,3 +670,21 @@ def test_hand_scheduled_main_loop_is_bit_identical_to_the_compiled_one(gpu, M, N
         assert torch.equal(got, want)
     assert out["tiles"][1] == out["tiles_compiled"][1]
     assert out["tiles"][1] == [float(yi.float().abs().max()) for yi in out["tiles"][0]]
+
+
+@pytest.mark.parametrize("view", ["plain", "row_strided", "transposed", "one_row"])
+def test_native_linear_call_equals_the_separate_operations(gpu, view):
+    """FourOverSixLinear.forward as one native call (or, for a layout that call does not take, the general path) gives
+    what quantize_to_fp4 and fp4_matmul give one after the other, bit for bit, with and without bias."""
+    from longlive_amd.fouroversix import ModelQuantizationConfig
+    from longlive_amd.utils.quant import quantize_model_with_filter
+
+    torch.manual_seed(3)
+    x = activations((77, 320), 4).to(gpu)
+    x = {"plain": x, "row_strided": x[:, :192], "transposed": x[:64, :64].t(), "one_row": x[5:6]}[view]
+    for bias in (True, False):
+        model = torch.nn.Sequential(torch.nn.Linear(x.shape[1], 136, bias=bias)).to(gpu)
+        model, _ = quantize_model_with_filter(model, ModelQuantizationConfig(), materialize_for_inference=True, verbose=False)
+        with torch.no_grad():
+            want = fp4_matmul(quantize_to_fp4(x, QuantizationConfig()), model[0].quantized_weight(), bias=model[0].bias)
+            assert torch.equal(model(x), want)

@@ -135,8 +135,12 @@ inline TileKernelChoice choose_tile_kernel(int64_t M, int64_t N, int64_t Kp, int
     if (tiles <= cus && 2 * tiles > cus) return {4, true};
   }
   // Small problems: when even 128 x 128 tiles would occupy at most half of the compute units, 64 x 64 tiles (more
-  // decode work per MFMA, but four times the workgroups) finish sooner.
-  if (((M + 127) / 128) * ((N * n_products + 127) / 128) <= cus / 2) return {0, false};
+  // decode work per MFMA, but four times the workgroups) finish sooner.  Up to 0.69 of the units they still do where K is
+  // long, since each 128 x 128 tile then has a unit to itself with one wave per SIMD (880 x 3072 x 3072, 168 tiles: 24.8
+  // against 27.7 us; 1173 x 2048 x 8192, 160 tiles: 52.6 against 65.4; but 335 x 5888 x 1536, 138 tiles: 16.4 against 16.0,
+  // and 520 x 5888 x 2048, 230 tiles: 23.4 against 20.5).
+  const int64_t tiles_128 = ((M + 127) / 128) * ((N * n_products + 127) / 128);
+  if (tiles_128 <= cus / 2 || (schedule != 2 && Kp >= 2048 && tiles_128 * 16 <= 11 * (int64_t)cus)) return {0, false};
   // Two workgroups of four waves are resident per compute unit.  The 256 x 128 / 128 x 256 tiles need 6 decode
   // instructions per MFMA, the 128 x 128 tile 8, so the larger tiles win unless they fill the slots much worse.  A last
   // round of at most one workgroup per unit is cheap: alone on its unit a workgroup runs in 0.56 of the time it takes
@@ -160,6 +164,32 @@ inline TileKernelChoice choose_tile_kernel(int64_t M, int64_t N, int64_t Kp, int
     }
   }
   return {best, generated_ok && best >= 2};
+}
+
+// How the small-product kernel divides a launch: 64 x 64 tiles, each by `parts` workgroups that share its K range (steps of
+// 256 elements).  Measured: a step takes 0.55 us with one workgroup on every compute unit and 0.85 with two; handing the
+// parts over and adding them up takes 3 us and 0.1 more per part (64 x 512 x 5888: 17.7 us whole, 10.7 in four parts,
+// 10.2 in eight; 128 x 3072 x 14336: 36.4 whole, 23.9 in two, 21.8 in four; 112 x 2944 x 8192: 23.0 whole, 15.6 in four,
+// 18.0 in five; 256 x 3072 x 3072: 11.9 whole, 13.6 in two).  More workgroups than two per unit would run one after the other.
+struct SmallGemmPlan {
+  int parts;
+  int tiles_m, tiles_n_each;
+  int64_t tiles;
+};
+inline SmallGemmPlan plan_small_gemm(int64_t M, int64_t N, int64_t Kp, int n_products, int cus) {
+  SmallGemmPlan p{1, (int)((M + 63) / 64), (int)((N + 63) / 64), 0};
+  p.tiles = (int64_t)p.tiles_m * p.tiles_n_each * n_products;
+  const int64_t steps = (Kp + 255) / 256;
+  double best = 0.0;
+  for (int64_t s = 1; s <= 16 && s <= steps && (s == 1 || p.tiles * s <= 2 * cus); ++s) {
+    const double beyond = p.tiles * s <= cus ? 0.0 : (double)(p.tiles * s - cus) / cus;
+    const double time = (double)((steps + s - 1) / s) * (0.55 + 0.3 * beyond) + (s > 1 ? 3.0 + 0.1 * (double)s : 0.0);
+    if (s == 1 || time < best) {
+      best = time;
+      p.parts = (int)s;
+    }
+  }
+  return p;
 }
 
 }  // namespace ll

@@ -22,6 +22,8 @@
 #include "ll_common.h"
 #include "gemm_split.h"
 
+#include <type_traits>
+
 namespace ll {
 
 // sixteen zero bytes in global memory: what lanes load in place of K elements beyond the end of a row
@@ -726,6 +728,303 @@ __global__ __launch_bounds__(256) void gemm_w4a4_persistent_kernel(PersistentPar
 #undef LL_V10
 
 
+// ============================================================================ small products
+// 64 x 64 tiles for products that give at most half a 128 x 128 tile per compute unit.  A workgroup is four waves; each
+// holds the whole 64 x 64 tile (2 x 2 fragments) and multiplies one quarter of every K step of 256 elements, so a
+// decoded fragment serves two MFMAs (8 decode instructions per MFMA; the tile kernel above, whose four waves share the
+// tile out as 32 x 32 each, decodes 16).  With one or two waves per SIMD the kernel is bound by the instructions a wave
+// issues, one per four cycles whatever their kind: the stages of the ring are unrolled so that LDS addresses are
+// immediates, and the loads take a scalar base.  Behind the loop each wave finishes one of the four fragments: it adds
+// the other waves' parts of it, always in the order of the K quarters, from LDS.  Where there are few tiles and K is
+// long, several workgroups share the K range of a tile (plan_small_gemm).
+// Measured (this kernel / the 64 x 64 tile kernel above): 512 x 3072 x 3072 16.6 / 21.8 us, 128 x 3072 x 14336 21.8 / 58.1 us
+// (four parts), 64 x 512 x 5888 10.7 / 25.3 us (four parts), 736 x 1536 x 8960 35.2 / 56.2 us; a single K step (48 x 512 x
+// 256) 5.5 / 5.3 us, which is the launch.  The kernel above keeps this tile for LL_GEMM_TILES_COMPILED (one order of
+// summation for every shape).
+constexpr int kSmallThreads = 256;
+constexpr int kSmallStages = 4;
+constexpr int kSmallK = 256;                                  // K elements per step: 64 per wave
+constexpr int kSmallRow = kSmallK / 2;                        // bytes per row and stage; pieces stored at piece ^ (row % 8)
+constexpr int kSmallVals = 64 * kSmallRow;                    // one operand's values of a stage
+constexpr int kSmallScales = 4 * 512;                         // one operand's scales: four 128 x 4 tiles
+constexpr int kSmallStage = 2 * (kSmallVals + kSmallScales);
+constexpr int kSmallSmem = kSmallStages * kSmallStage;
+constexpr int kSmallFlag = 4 * 3 * 4096;                      // behind the exchange
+static_assert(kSmallFlag + 16 <= kSmallSmem && 2 * kSmallSmem <= 160 * 1024, "the exchange fits the ring, two workgroups fit a unit");
+
+// 16 bytes per lane from base + offset straight into LDS at lds_base + IMM + 16 * lane (see load_to_lds_b128).
+template <int IMM>
+__device__ __forceinline__ void load_to_lds_b128_at(const uint8_t* base, uint32_t offset, uint32_t lds_base) {
+  asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(offset), "s"(base), "s"(lds_base), "n"(IMM)
+               : "memory", "scc");
+}
+
+__global__ __launch_bounds__(kSmallThreads, 2) void gemm_w4a4_small_kernel(
+    const uint8_t* __restrict__ Av, const uint8_t* __restrict__ As, const uint8_t* __restrict__ Bv0,
+    const uint8_t* __restrict__ Bs0, const float* __restrict__ alpha_ptr0, const float* __restrict__ amax_a,
+    const float* __restrict__ amax_b0, float inv_denom_a, float inv_denom_b0, int M, int N, int Mp, int Np, int Kp,
+    uint16_t* __restrict__ D0, int64_t ldd0, int tiles_m, int tiles_n, GemmEpilogue epi, GemmGroups groups,
+    int parts, float* __restrict__ records, int* __restrict__ arrivals) {
+  const uint8_t* __restrict__ Bv = Bv0;
+  const uint8_t* __restrict__ Bs = Bs0;
+  const float* __restrict__ alpha_ptr = alpha_ptr0;
+  const float* __restrict__ amax_b = amax_b0;
+  float inv_denom_b = inv_denom_b0;
+  uint16_t* __restrict__ D = D0;
+  int64_t ldd = ldd0;
+  const uint16_t* __restrict__ bias = epi.bias;
+  const int act = epi.act;
+  extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+
+  // Workgroup -> (tile, part of its K range), as in gemm_w4a4_asm8_kernel: every XCD takes a run of consecutive ones.
+  const int total = tiles_m * tiles_n * parts, per_xcd = (int)gridDim.x >> 3;
+  const int unit = ((int)blockIdx.x & 7) * per_xcd + ((int)blockIdx.x >> 3);
+  if (unit >= total) return;
+  const int tile = unit / parts, part = unit - tile * parts;
+  int tile_n = tile / tiles_m;
+  const int tile_m = tile - tile_n * tiles_m;
+  if (groups.n > 1) {
+    const int g = tile_n / groups.tiles_n_each;
+    tile_n -= g * groups.tiles_n_each;
+    if (g > 0) {
+      const GemmGroup& gg = groups.more[g - 1];
+      Bv = gg.Bv;
+      Bs = gg.Bs;
+      alpha_ptr = gg.alpha;
+      amax_b = gg.amax_b;
+      inv_denom_b = gg.inv_denom_b;
+      D = gg.D;
+      ldd = gg.ldd;
+      bias = gg.bias;
+      epi.sink = gg.sink;
+    }
+  }
+  const int row0 = tile_m * 64, col0 = tile_n * 64;
+  const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, lh = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int all_steps = (Kp + kSmallK - 1) / kSmallK;
+  const int t0 = (int)((int64_t)part * all_steps / parts);             // first K step of this part
+  const int nk = (int)((int64_t)(part + 1) * all_steps / parts) - t0;  // at least one: the host sees to it
+
+  // ---- global -> LDS: a load instruction covers 1 KB = 8 rows of 128 bytes.  Wave w brings rows 8 w .. and 32 + 8 w .. of
+  // A and of B and 1 KB of scales (waves 0, 1: A, tiles 0-1 and 2-3 of the step; waves 2, 3: B).  The tiles of a matrix
+  // padded to 128 rows have all their rows.
+  const int64_t row_bytes = Kp >> 1;
+  const int piece = (lane & 7) ^ (lane >> 3);      // the row's piece that belongs at this lane's position
+  const uint8_t* a_src = Av + (int64_t)(row0 + 8 * wave) * row_bytes + (int64_t)t0 * kSmallRow;
+  const uint8_t* b_src = Bv + (int64_t)(col0 + 8 * wave) * row_bytes + (int64_t)t0 * kSmallRow;
+  const uint8_t* s_src = (wave < 2 ? As + (int64_t)(row0 >> 7) * (Kp >> 6) * 512 : Bs + (int64_t)(col0 >> 7) * (Kp >> 6) * 512) +
+                         (wave & 1) * 1024 + (int64_t)t0 * 2048;
+  const uint8_t* src[4] = {a_src, a_src + 32 * row_bytes, b_src, b_src + 32 * row_bytes};
+  uint32_t voff = (uint32_t)(lane >> 3) * (uint32_t)row_bytes + (uint32_t)piece * 16u, soff = (uint32_t)lane * 16u;
+  const uint32_t v_dst = lds_address(smem) + wave * 1024;
+  auto load_step = [&](int step, auto stage) {  // called for the steps in order
+    constexpr int kBase = decltype(stage)::value * kSmallStage;
+    const int k0 = (t0 + step) * kSmallK;
+    if (k0 + kSmallK <= Kp) {
+      load_to_lds_b128_at<kBase>(src[0], voff, v_dst);
+      load_to_lds_b128_at<kBase + 4096>(src[1], voff, v_dst);
+      load_to_lds_b128_at<kBase + 8192>(src[2], voff, v_dst);
+      load_to_lds_b128_at<kBase + 12288>(src[3], voff, v_dst);
+      load_to_lds_b128_at<kBase + 16384>(s_src, soff, v_dst);
+    } else {  // the rows end inside this step: zeros behind their end
+      const uint8_t* zero16 = reinterpret_cast<const uint8_t*>(&g_gemm_zero16);
+      const bool have = k0 + piece * 32 < Kp, have_scales = k0 + 64 * (2 * (wave & 1) + (lane >> 5)) < Kp;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) load_to_lds_b128(have ? src[i] + voff : zero16, v_dst + kBase + i * 4096);
+      load_to_lds_b128(have_scales ? s_src + soff : zero16, v_dst + kBase + 16384);
+    }
+    voff += kSmallRow;
+    soff += 2048;
+  };
+
+  // ---- the lane's LDS reads: row 32 f + l32, piece 2 wave + lh; the scale bytes of the piece's two blocks
+  const uint8_t* v_rd = smem + l32 * kSmallRow + 16 * ((2 * wave + lh) ^ (l32 & 7));
+  const uint8_t* s_rd = smem + 2 * kSmallVals + 512 * wave + l32 * 16 + 2 * lh;
+  const uint8_t* sa_rd = s_rd + ((row0 & 127) >> 5) * 4;
+  const uint8_t* sb_rd = s_rd + kSmallScales + ((col0 & 127) >> 5) * 4;
+  struct Raw {
+    uint4 v[4];  // fragments A0, A1, B0, B1
+    uint32_t sc[4];
+  };
+  auto read_raw = [&](Raw& h, auto stage) {
+    constexpr int kBase = decltype(stage)::value * kSmallStage;
+#pragma unroll
+    for (int f = 0; f < 4; ++f) {
+      h.v[f] = *reinterpret_cast<const uint4*>(v_rd + kBase + f * 4096);
+      h.sc[f] = *reinterpret_cast<const uint16_t*>((f < 2 ? sa_rd : sb_rd) + kBase + 4 * (f & 1));
+    }
+  };
+  float16v acc[2][2];
+#pragma unroll
+  for (int g = 0; g < 2; ++g)
+#pragma unroll
+    for (int f = 0; f < 2; ++f)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[g][f][i] = 0.0f;
+  half8v o[2][4];
+#pragma unroll
+  for (int f = 0; f < 4; ++f)
+#pragma unroll
+    for (int i = 0; i < 8; ++i) o[1][f][i] = (_Float16)0.0f;  // the first step's "previous sub-step" adds nothing
+  // The four MFMAs of a sub-step with the decode of the next one between them, a fragment (eight instructions) behind
+  // each; the scheduling barriers hold that order (left to itself the compiler pairs MFMAs that depend on each other).
+  auto mma_under = [&](half8v (&dst)[4], const Raw& h, const half2v (&s2)[4][2], int j, const half8v (&x)[4]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      acc[i >> 1][i & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[2 + (i >> 1)], x[i & 1], acc[i >> 1][i & 1], 0, 0, 0);
+      const uint32_t w = j == 0 ? h.v[i].x : j == 1 ? h.v[i].y : j == 2 ? h.v[i].z : h.v[i].w;
+      dst[i] = decode8(w, s2[i][j >> 1]);
+      asm volatile("" : "+v"(dst[i]));  // here, and not sunk behind the branches to the MFMA that reads it
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  // The wave's five loads of the step that comes next have landed; those of the `behind` steps after it may be under way.
+  auto wait_loads = [&](int behind) {
+    if (behind >= 3) __builtin_amdgcn_s_waitcnt(0x0F7F);       // vmcnt(15)
+    else if (behind == 2) __builtin_amdgcn_s_waitcnt(0x0F7A);  // vmcnt(10)
+    else if (behind == 1) __builtin_amdgcn_s_waitcnt(0x0F75);  // vmcnt(5)
+    else __builtin_amdgcn_s_waitcnt(0x0F70);
+  };
+  // One K step from the packed words in h; the words of the step behind it are read into `next` half way through,
+  // when every wave has its loads of that step in LDS and has read this step's stage for the last time (the stage is
+  // then refilled with the step four further on), so that neither the barrier nor the LDS latency is waited out.
+  auto step = [&](int t, auto stage, const Raw& h, Raw& next) {
+    constexpr int kStageNo = decltype(stage)::value;
+    half2v s2[4][2];
+#pragma unroll
+    for (int f = 0; f < 4; ++f) {
+      const half2v sc = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(h.sc[f], 1.0f, false);
+      s2[f][0] = half2v{sc[0], sc[0]};
+      s2[f][1] = half2v{sc[1], sc[1]};
+    }
+    mma_under(o[0], h, s2, 0, o[1]);
+    mma_under(o[1], h, s2, 1, o[0]);
+    if (t + 1 < nk) {
+      wait_loads(nk - 2 - t < 2 ? nk - 2 - t : 2);
+      __syncthreads();
+      if (t + kSmallStages < nk) load_step(t + kSmallStages, stage);
+      read_raw(next, std::integral_constant<int, (kStageNo + 1) % kSmallStages>{});
+    }
+    mma_under(o[0], h, s2, 2, o[1]);
+    mma_under(o[1], h, s2, 3, o[0]);
+  };
+  constexpr std::integral_constant<int, 0> kS0{};
+  constexpr std::integral_constant<int, 1> kS1{};
+  constexpr std::integral_constant<int, 2> kS2{};
+  constexpr std::integral_constant<int, 3> kS3{};
+  load_step(0, kS0);
+  if (1 < nk) load_step(1, kS1);
+  if (2 < nk) load_step(2, kS2);
+  if (3 < nk) load_step(3, kS3);
+  wait_loads(nk - 1);
+  __syncthreads();
+  Raw h0, h1;
+  read_raw(h0, kS0);
+  int t = 0;
+#pragma unroll 1
+  for (; t + 4 <= nk; t += 4) {
+    step(t, kS0, h0, h1);
+    step(t + 1, kS1, h1, h0);
+    step(t + 2, kS2, h0, h1);
+    step(t + 3, kS3, h1, h0);
+  }
+  if (t < nk) step(t, kS0, h0, h1);
+  if (t + 1 < nk) step(t + 1, kS1, h1, h0);
+  if (t + 2 < nk) step(t + 2, kS2, h0, h1);
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    acc[i >> 1][i & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(o[1][2 + (i >> 1)], o[1][i & 1], acc[i >> 1][i & 1], 0, 0, 0);
+  __syncthreads();  // every wave has left the ring
+
+  // ---- wave w finishes fragment (g, f) = (w / 2, w % 2): the others leave their parts of it in LDS
+  float* exchange = reinterpret_cast<float*>(smem);
+  float16v sum[1][1];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const float16v& a = acc[q >> 1][q & 1];
+    if (q == wave) {
+      sum[0][0] = a;
+    } else {
+      float* dst = exchange + (q * 3 + (wave < q ? wave : wave - 1)) * 1024 + lane * 4;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) *reinterpret_cast<float4*>(dst + i * 256) = make_float4(a[4 * i], a[4 * i + 1], a[4 * i + 2], a[4 * i + 3]);
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float* p = exchange + wave * 3 * 1024 + lane * 4 + i * 256;
+    const float4 x = *reinterpret_cast<const float4*>(p), y = *reinterpret_cast<const float4*>(p + 1024),
+                 z = *reinterpret_cast<const float4*>(p + 2048);
+    const float xs[4] = {x.x, x.y, x.z, x.w}, ys[4] = {y.x, y.y, y.z, y.w}, zs[4] = {z.x, z.y, z.z, z.w};
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {  // x, y, z: the three other waves in order; own part at its place
+      const float m = sum[0][0][4 * i + c];
+      const float s0 = wave == 0 ? m : xs[c], s1 = wave == 1 ? m : (wave == 0 ? xs[c] : ys[c]);
+      const float s2v = wave == 2 ? m : (wave == 3 ? zs[c] : ys[c]), s3 = wave == 3 ? m : zs[c];
+      sum[0][0][4 * i + c] = (s0 + s1) + (s2v + s3);
+    }
+  }
+  __syncthreads();  // the patches of the epilogue overlap the exchange
+  if (parts > 1) {
+    // Part of a tile: the workgroup that arrives last adds the parts up in the order of their K ranges, so the sum does
+    // not depend on who that is; the others leave theirs in a record.  Same protocol as in the persistent kernel:
+    // device-scope stores, every wave waits for its own, then the barrier, then thread 0 counts the arrival.
+    int* flag = reinterpret_cast<int*>(smem + kSmallFlag);
+    float* tile_records = records + (size_t)tile * parts * 4096 + wave * 1024 + lane * 4;
+    float16v& own = sum[0][0];
+    if (tid == 0) *flag = __hip_atomic_load(arrivals + tile, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == parts - 1;
+    __syncthreads();
+    bool last = *flag != 0;
+    if (!last) {
+      float* rec = tile_records + (size_t)part * 4096;
+      store_shared_f32x4<0>(rec, float4v{own[0], own[1], own[2], own[3]});
+      store_shared_f32x4<1024>(rec, float4v{own[4], own[5], own[6], own[7]});
+      store_shared_f32x4<2048>(rec, float4v{own[8], own[9], own[10], own[11]});
+      store_shared_f32x4<3072>(rec, float4v{own[12], own[13], own[14], own[15]});
+      __builtin_amdgcn_s_waitcnt(0x0F70);
+      __syncthreads();
+      if (tid == 0) *flag = __hip_atomic_fetch_add(arrivals + tile, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == parts - 1;
+      __syncthreads();
+      last = *flag != 0;
+    }
+    if (!last) return;
+    if (tid == 0) __hip_atomic_store(arrivals + tile, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // ready for the next launch
+    float16v all;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) all[i] = 0.0f;
+    for (int p0 = 0; p0 < parts; p0 += 4) {  // sixteen loads in flight
+      float4v v[4][4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const float* rec = tile_records + (size_t)min(p0 + q, parts - 1) * 4096;
+        load_shared_f32x4<0>(rec, v[q][0]);
+        load_shared_f32x4<1024>(rec, v[q][1]);
+        load_shared_f32x4<2048>(rec, v[q][2]);
+        load_shared_f32x4<3072>(rec, v[q][3]);
+      }
+      asm volatile("s_waitcnt vmcnt(0)"
+                   : "+v"(v[0][0]), "+v"(v[0][1]), "+v"(v[0][2]), "+v"(v[0][3]), "+v"(v[1][0]), "+v"(v[1][1]), "+v"(v[1][2]),
+                     "+v"(v[1][3]), "+v"(v[2][0]), "+v"(v[2][1]), "+v"(v[2][2]), "+v"(v[2][3]), "+v"(v[3][0]), "+v"(v[3][1]),
+                     "+v"(v[3][2]), "+v"(v[3][3])
+                   :
+                   : "memory");
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        if (p0 + q < parts) {
+#pragma unroll
+          for (int i = 0; i < 16; ++i) all[i] += p0 + q == part ? own[i] : v[q][i >> 2][i & 3];
+        }
+      }
+    }
+    own = all;
+  }
+  const float alpha = alpha_ptr ? alpha_ptr[0] : (amax_a[0] * amax_b[0]) * (inv_denom_a * inv_denom_b);
+  gemm_epilogue<1, 1>(sum, alpha, smem, wave, lane, row0 + 32 * (wave & 1), col0 + 32 * (wave >> 1), M, N, D, ldd, bias, act, epi,
+                      (uint32_t)blockIdx.x * 4 + wave);
+}
+
 // ============================================================================ tile kernel, hand-scheduled loop
 // gemm_w4a4_kernel<FA, FB> with its main loop replaced by a generated instruction sequence
 // (gemm_tile_loop_gen.py): the same workgroup -> tile map, the same arithmetic in the same order (the accumulators
@@ -1147,6 +1446,7 @@ extern "C" int ll_nvfp4_gemm_tnt_fused(const uint8_t* A_values, const uint8_t* A
 
 namespace ll {
 
+inline size_t small_record_bytes(const SmallGemmPlan& p) { return (size_t)p.tiles * p.parts * 64 * 64 * sizeof(float); }
 inline size_t persistent_record_bytes(const GemmDivision& d) { return (size_t)2 * d.G * kPRecordFloats * sizeof(float); }
 
 // Launches the persistent kernel if the plan says so and its memory is at hand; *launched tells.
@@ -1225,6 +1525,26 @@ int dispatch_gemm(const uint8_t* A_values, const uint8_t* A_scales, const uint8_
                        A_scales, B_values, B_scales, alpha, amax_a, amax_b, 1.0f / denom_a, 1.0f / denom_b, (int)M, (int)N, (int)Mp,
                        (int)Np, (int)Kp, static_cast<uint16_t*>(D), ldd, tiles_m, tiles_n, epi, gr);
     LL_CHECK_LAUNCH("gemm_w4a4_asm8_kernel");
+    return LL_OK;
+  }
+  if (choice.kernel == LL_GEMM_KERNEL_64X64 && g_gemm_schedule.load(std::memory_order_relaxed) != LL_GEMM_TILES_COMPILED) {
+    SmallGemmPlan plan = plan_small_gemm(M, N, Kp, groups.n, cus);
+    StreamScratch w;
+    if (plan.parts > 1) {
+      bool missing = false;
+      if (int rc = stream_scratch(dev, s, small_record_bytes(plan), (size_t)plan.tiles, !stream_is_capturing(s), w, &missing,
+                                  "ll_nvfp4_gemm_tnt")) return rc;
+      if (missing) plan.parts = 1;  // a capturing stream without the memory: one workgroup per tile, which needs none
+    }
+    GemmGroups gr = groups;
+    gr.tiles_n_each = plan.tiles_n_each;
+    static std::atomic<uint64_t> lds_allowed{0};
+    if (int rc = allow_dynamic_lds(reinterpret_cast<const void*>(&gemm_w4a4_small_kernel), kSmallSmem, lds_allowed, "ll_nvfp4_gemm_tnt")) return rc;
+    hipLaunchKernelGGL(gemm_w4a4_small_kernel, dim3((unsigned)((plan.tiles * plan.parts + 7) / 8 * 8)), dim3(kSmallThreads), kSmallSmem, s,
+                       A_values, A_scales, B_values, B_scales, alpha, amax_a, amax_b, 1.0f / denom_a, 1.0f / denom_b, (int)M, (int)N,
+                       (int)Mp, (int)Np, (int)Kp, static_cast<uint16_t*>(D), ldd, plan.tiles_m, plan.tiles_n_each * gr.n, epi, gr,
+                       plan.parts, reinterpret_cast<float*>(w.records), w.counters);
+    LL_CHECK_LAUNCH("gemm_w4a4_small_kernel");
     return LL_OK;
   }
 #define LL_GEMM_ARGS A_values, A_scales, B_values, B_scales, alpha, amax_a, amax_b, denom_a, denom_b, (int)M, (int)N, \
@@ -1337,13 +1657,24 @@ extern "C" int ll_nvfp4_gemm_reserve(int64_t M, int64_t N, int64_t Kp, int n_pro
     return LL_ELAUNCH;
   }
   if (int rc = compute_units_of(dev, cus, "ll_nvfp4_gemm_reserve")) return rc;
-  const PersistentPlan plan = plan_persistent(M, N, Kp, n_products, cus, g_gemm_schedule.load(std::memory_order_relaxed));
-  if (!plan.use) return LL_OK;
+  const int schedule = g_gemm_schedule.load(std::memory_order_relaxed);
+  size_t bytes = 0, counters = 0;
+  if (const PersistentPlan plan = plan_persistent(M, N, Kp, n_products, cus, schedule); plan.use) {
+    bytes = persistent_record_bytes(plan.d);
+    counters = gemm_split_tiles(plan.d);
+  } else if (schedule != LL_GEMM_TILES_COMPILED && choose_tile_kernel(M, N, Kp, n_products, cus, schedule).kernel == LL_GEMM_KERNEL_64X64) {
+    const SmallGemmPlan small = plan_small_gemm(M, N, Kp, n_products, cus);
+    if (small.parts > 1) {
+      bytes = small_record_bytes(small);
+      counters = (size_t)small.tiles;
+    }
+  }
+  if (bytes == 0) return LL_OK;
   if (stream_is_capturing(static_cast<hipStream_t>(stream))) {
     set_error("ll_nvfp4_gemm_reserve: the stream is being captured; reserve before the recording starts");
     return LL_ENOSUP;
   }
   StreamScratch w;
-  return stream_scratch(dev, static_cast<hipStream_t>(stream), persistent_record_bytes(plan.d), gemm_split_tiles(plan.d), true, w, nullptr,
+  return stream_scratch(dev, static_cast<hipStream_t>(stream), bytes, counters, true, w, nullptr,
                         "ll_nvfp4_gemm_reserve");
 }

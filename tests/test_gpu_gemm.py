@@ -688,3 +688,59 @@ def test_native_linear_call_equals_the_separate_operations(gpu, view):
         with torch.no_grad():
             want = fp4_matmul(quantize_to_fp4(x, QuantizationConfig()), model[0].quantized_weight(), bias=model[0].bias)
             assert torch.equal(model(x), want)
+
+
+@pytest.mark.parametrize("M,N,K,groups", [
+    (1, 8, 64, 1),            # one row, a K step that is three quarters zeros
+    (63, 65, 192, 1),         # ragged both ways, one partial K step
+    (64, 64, 256, 2),         # one tile and one whole step per product
+    (65, 200, 320, 1),        # a second row of tiles with one row, a step and a quarter
+    (130, 136, 1088, 3),      # five steps, the last a quarter; three products
+    (40, 256, 5888, 1),       # few tiles, long K: several workgroups share a tile's K range
+    (100, 72, 14400, 2),      # the same with a ragged last step and two products
+])
+def test_small_products_with_k_shared_between_waves_and_workgroups(gpu, M, N, K, groups):
+    """The small-product kernel (64 x 64 tiles, every wave a quarter of each K step, the K range of few tiles shared
+    between workgroups) adds the exact products in another order than the compiled tile kernel: within one bf16 ulp of
+    the fp32 sum of it (fp32 sums of up to 2^14 exact products of unit-scale data differ by far less than a bf16 step),
+    twice for identical bits, and recorded into a graph, with and without the memory its parts pass through."""
+    cfg = QuantizationConfig(scale_rule="mse")
+    xq = quantize_to_fp4(activations((M, K), 25).to(gpu), cfg)
+    ws = [quantize_to_fp4((weights((N, K), 26 + i) * (1 + i)).to(gpu), cfg) for i in range(groups)]
+    bias = (torch.randn(N, generator=torch.Generator().manual_seed(27)) * 0.1).to(gpu).bfloat16()
+
+    def run():
+        products = [dict(values=w.values, scales=w.scale_factors, amax=w.amax, denom=1536.0, bias=bias if i != 1 else None)
+                    for i, w in enumerate(ws)]
+        return list(_native.gemm_grouped(xq.values, xq.scale_factors, xq.amax, 1536.0, M, N, products))
+
+    assert _native.gemm_kernel(M, N, xq.padded_shape[1], groups)["kernel"] == "64x64"
+    with _native.gemm_schedule("tiles_compiled"):
+        want = run()
+    got, again = run(), run()
+    for a, b, c in zip(got, again, want):
+        assert torch.equal(a, b)
+        _ulp_close(a, c, frac=5e-3)
+    for reserve in (False, True):
+        side = torch.cuda.Stream(device=gpu)
+        side.wait_stream(torch.cuda.current_stream())
+        if reserve:
+            with torch.cuda.stream(side):
+                _native.gemm_reserve(M, N, xq.padded_shape[1], groups)
+            side.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            out = run()
+        for _ in range(3):
+            for y in out:
+                y.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            for a, b in zip(out, got):
+                if reserve:
+                    assert torch.equal(a, b)
+                else:
+                    _ulp_close(a, b, frac=5e-3)
+            run()
+        with torch.cuda.stream(side):
+            _native.release_stream_memory()

@@ -572,9 +572,10 @@ class gemm_schedule:
 
 
 def release_stream_memory(device=None) -> None:
-    """Free the memory the library holds for the current stream (partial tiles of the attention and the GEMM)."""
+    """Free the memory the library holds for the current stream (partial tiles of the attention and the GEMM, amax sink)."""
     with torch.cuda.device(device if device is not None else torch.cuda.current_device()):
         _check(load().ll_release_stream_memory(_stream()), "ll_release_stream_memory")
+        host().release_stream_sink()
 
 
 # --------------------------------------------------------------------------- KV cache
@@ -820,6 +821,25 @@ def layer_norm_quantize(x, weight, bias, rule: str, eps=1e-6, spin_limit=None):
                                              NORM_QUANTIZE_SPIN_LIMIT if spin_limit is None else int(spin_limit),
                                              _stream())
     return _norm_quantize_result(code, "ll_layer_norm_quantize", values, scales, amax)
+
+
+def block_forward(x, e, layers, norms, cos, sin, window, text, rule: str, sizes, keys_only: bool, tickets):
+    """One transformer block as one native call (``block_forward`` of csrc/host_ops.cpp, which documents the arguments):
+    (out, roped K, V, text K, text V), or None when it does not take the call.  ``tickets``: of the producers of K and V.
+    The other tensor maxima go through a sink of the current stream, or through that of an active recording."""
+    lib, graph, graph_sink = host(), _active_graph_sinks.get(_device_key(x.device)), None
+    if graph is not None:
+        graph_sink = (graph.parts, graph.entry[1], graph.offset)
+        graph.entry[1] += lib.EPOCHS_PER_CALL
+        graph.entry[2] = None
+    out = lib.block_forward(x, e, layers, norms, cos, sin, window, text,
+                            (RULE_IDS[rule], DENOMINATORS[rule], *sizes, NORM_QUANTIZE_SPIN_LIMIT, keys_only),
+                            *(None if t is None else (t.parts, t.epoch) for t in tickets), graph_sink)
+    if out is not None:
+        for t in tickets:
+            if t is not None:
+                t.entry[2] = (t.epoch, lib.current_stream())
+    return out
 
 
 def gate_residual(x, y, gate, frame_seqlen):

@@ -4,9 +4,12 @@
 // stream and hands raw pointers on.  In Python the same work costs 20 to 25 us a call (tensor factories, stream and
 // device queries, ctypes conversions), more than the kernels of a small call need on the GPU; here it is 2 to 4 us.
 //
+// A transformer block is one call too (block_forward, 21 launches): issued one by one from Python it took 600 us of host
+// time, more than the GPU needs for a block of up to about 2000 tokens.
+//
 // Every function returns None for a call it does not take (another device, type, layout or option than the common
 // one); the caller then runs the general Python path, which does the work or raises the error that belongs to it.
-// Nothing is kept between calls.
+// Nothing is kept between calls but one amax sink (8 KB) per device and stream, which release_stream_memory gives back.
 #include <Python.h>
 
 #include <ATen/hip/EmptyTensor.h>
@@ -14,6 +17,10 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
+
+#include <map>
+#include <mutex>
+#include <utility>
 
 #include "../../include/ll_nvfp4.h"
 
@@ -158,7 +165,364 @@ PyObject* py_dequantize(PyObject*, PyObject* const* args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// ------------------------------------------------------------------------------------------------ amax sinks of a block
+// The sink through which the kernels of one native call hand tensor maxima on belongs to the (device, stream) pair: launches
+// on one stream are ordered, and two streams (or the threads that drive them) never meet in one buffer.
+struct StreamSink {
+  Tensor parts;
+  uint32_t epoch = 0;
+};
+std::mutex g_sink_mutex;
+std::map<std::pair<int, void*>, StreamSink>& stream_sinks() {
+  static auto* sinks = new std::map<std::pair<int, void*>, StreamSink>;  // outlives every static that may still hold tensors
+  return *sinks;
+}
+constexpr uint32_t kEpochsPerCall = 16;
+
+// Epochs for the producers of one call, in the order in which they run.
+struct Epochs {
+  uint64_t* parts;
+  const uint32_t* offset;
+  uint32_t next;
+  ll_amax_sink take() { return ll_amax_sink{parts, ++next, offset}; }
+};
+// parts is null where the sink would have to be made while the stream is being captured (its memory would belong to the
+// capture, its clearing to every replay).
+Epochs epochs_of_stream(int dev, void* stream) {
+  std::lock_guard<std::mutex> lock(g_sink_mutex);
+  auto& sinks = stream_sinks();
+  const std::pair<int, void*> key{dev, stream};
+  auto found = sinks.find(key);
+  if (found == sinks.end() || found->second.epoch > 0xFFFFFF00u) {
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(static_cast<hipStream_t>(stream), &capture) != hipSuccess || capture != hipStreamCaptureStatusNone)
+      return Epochs{nullptr, nullptr, 0};
+    if (found == sinks.end()) found = sinks.emplace(key, StreamSink{empty({(int64_t)LL_AMAX_PARTS}, at::kLong, dev), 0}).first;
+    found->second.parts.zero_();
+    found->second.epoch = 0;
+  }
+  StreamSink& s = found->second;
+  const Epochs e{reinterpret_cast<uint64_t*>(s.parts.data_ptr<int64_t>()), nullptr, s.epoch};
+  s.epoch += kEpochsPerCall;
+  return e;
+}
+
+// ------------------------------------------------------------------------------------------------ block
+struct Layer {  // a quantized linear layer
+  const uint8_t *values, *scales;
+  const float* amax;
+  const void* bias;
+  float denom;
+  int64_t np, kp, n;
+};
+// From (values, scale_factors, amax, bias or None, denominator, out_features); false: not for this path.
+bool parse_layer(PyObject* t, int dev, Layer& l) {
+  if (!PyTuple_CheckExact(t) || PyTuple_GET_SIZE(t) != 6) return false;
+  const Tensor *v = as_tensor(PyTuple_GET_ITEM(t, 0)), *s = as_tensor(PyTuple_GET_ITEM(t, 1)), *a = as_tensor(PyTuple_GET_ITEM(t, 2));
+  PyObject* b = PyTuple_GET_ITEM(t, 3);
+  const Tensor* bias = as_tensor(b);
+  if (!v || !s || !a || (!bias && b != Py_None)) return false;
+  if (!on_device(*v, dev) || !on_device(*s, dev) || !on_device(*a, dev) || v->dim() != 2 || !v->is_contiguous() || !s->is_contiguous()) return false;
+  l.n = PyLong_AsLongLong(PyTuple_GET_ITEM(t, 5));
+  l.np = v->size(0);
+  l.kp = v->size(1) * 2;
+  if (l.np != round_up(l.n, 128) || l.n % 8) return false;
+  if (bias && (!is_bf16(*bias, dev) || bias->numel() != l.n || !bias->is_contiguous())) return false;
+  l.values = v->data_ptr<uint8_t>();
+  l.scales = static_cast<const uint8_t*>(s->data_ptr());
+  l.amax = a->data_ptr<float>();
+  l.bias = bias ? bias->data_ptr() : nullptr;
+  l.denom = (float)PyFloat_AsDouble(PyTuple_GET_ITEM(t, 4));
+  return true;
+}
+inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
+
+struct BlockCall {
+  int dev, rule;
+  float denom_a;
+  void* stream;
+  int64_t L, C;
+
+  // out = epilogue(a @ layer^T)
+  int gemm(const TempOperand& a, const Layer& w, int64_t M, void* out, ll_gemm_epilogue e) const {
+    e.bias = w.bias;
+    return ll_nvfp4_gemm_tnt_fused(a.values, a.scales, w.values, w.scales, nullptr, a.amax, w.amax, denom_a, w.denom, M, w.n, a.mp, w.np,
+                                   a.kp, out, w.n, &e, stream);
+  }
+  int grouped(const TempOperand& a, const Layer* const* w, int n, int64_t M, void* const* outs, const ll_amax_sink* sinks) const {
+    ll_gemm_product p[4];
+    for (int i = 0; i < n; ++i)
+      p[i] = ll_gemm_product{w[i]->values, w[i]->scales, nullptr, w[i]->amax, w[i]->denom, outs[i], w[i]->n, w[i]->bias,
+                             sinks ? sinks[i] : ll_amax_sink{nullptr, 0, nullptr}};
+    return ll_nvfp4_gemm_tnt_grouped(a.values, a.scales, a.amax, denom_a, M, w[0]->n, a.mp, w[0]->np, a.kp, n, p, stream);
+  }
+  TempOperand operand(int64_t m, int64_t k) const { return temp_operand(m, k, dev); }
+  int quantize_from(const Tensor& x, int64_t M, int64_t K, const TempOperand& q, const ll_amax_sink& sink) const {
+    return ll_nvfp4_quantize_from_sink(x.data_ptr(), M, K, K, rule, q.values, q.scales, q.amax, &sink, stream);
+  }
+};
+
+// block_forward(x, e, layers, norms, cos, sin, kv, text, options, k_sink, v_sink, graph_sink) ->
+//   (x_out or None, roped K [1, L, H, 128], V [1, L, H, 128], text K, text V) or None
+//   e: the six modulation vectors per frame [1, F, 6, C];  layers: q, k, v, o, cross q, k, v, o, FFN up, down;  norms: weights of
+//   norm_q, norm_k, norm3, norm3's bias, cross norm_q, cross norm_k;  kv: (table of the K slots, of the V slots, cached keys,
+//   block_token_size, e2m1_max, e4m3_max) or None;  text: the context [1, T, C] or (K, V) [1, T, H, 128];  options: (rule,
+//   denominator, heads, eps, eps of q/k norm, of norm3, of cross norm_q, of cross norm_k, spin limit, keys_only);  k_sink,
+//   v_sink: (parts, epoch) or None;  graph_sink: (parts, last epoch, offset) or None.
+// The launches and their order are those of DiTBlock.forward (longlive_amd/dit/model.py), which documents them.
+PyObject* py_block_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 12 || !plain(args[0]) || !plain(args[1])) Py_RETURN_NONE;
+  const Tensor& x = THPVariable_Unpack(args[0]);
+  const Tensor& e = THPVariable_Unpack(args[1]);
+  const int dev = current_device_of(x);
+  if (!is_bf16(x, dev) || !is_bf16(e, dev) || x.dim() != 3 || x.size(0) != 1 || !x.is_contiguous() || e.dim() != 4 || e.size(0) != 1 ||
+      e.size(2) != 6 || e.size(3) != x.size(2) || e.stride(3) != 1)
+    Py_RETURN_NONE;
+  BlockCall c;
+  c.dev = dev;
+  c.L = x.size(1);
+  c.C = x.size(2);
+  const int64_t L = c.L, C = c.C, F = e.size(1);
+  if (L == 0 || F == 0 || L % F || C % 128 || e.stride(1) % 8 || e.stride(2) % 8 || !aligned16(e.data_ptr()) || !aligned16(x.data_ptr())) Py_RETURN_NONE;
+  const int64_t frame_rows = L / F;
+  if (!PyTuple_CheckExact(args[2]) || PyTuple_GET_SIZE(args[2]) != 10 || !PyTuple_CheckExact(args[3]) || PyTuple_GET_SIZE(args[3]) != 6 ||
+      !PyTuple_CheckExact(args[8]) || PyTuple_GET_SIZE(args[8]) != 10)
+    Py_RETURN_NONE;
+  Layer w[10];
+  for (int i = 0; i < 10; ++i)
+    if (!parse_layer(PyTuple_GET_ITEM(args[2], i), dev, w[i])) Py_RETURN_NONE;
+  enum { Q, K, V, O, CQ, CK, CV, CO, UP, DOWN };
+  for (int i = 0; i < 10; ++i)
+    if (w[i].kp != round_up(i == DOWN ? w[UP].n : C, 64) || (i != UP && w[i].n != C)) Py_RETURN_NONE;
+  const void* norm[6];
+  for (int i = 0; i < 6; ++i) {
+    const Tensor* t = as_tensor(PyTuple_GET_ITEM(args[3], i));
+    if (!t || !is_bf16(*t, dev) || t->numel() != C || !t->is_contiguous() || !aligned16(t->data_ptr())) Py_RETURN_NONE;
+    norm[i] = t->data_ptr();
+  }
+  const Tensor *cos = as_tensor(args[4]), *sin = as_tensor(args[5]);
+  if (!cos || !sin || !on_device(*cos, dev) || !on_device(*sin, dev) || cos->scalar_type() != at::kFloat || sin->scalar_type() != at::kFloat ||
+      !cos->is_contiguous() || !sin->is_contiguous() || cos->numel() != L * 64 || sin->numel() != L * 64)
+    Py_RETURN_NONE;
+  PyObject* const o = args[8];
+  c.rule = (int)PyLong_AsLong(PyTuple_GET_ITEM(o, 0));
+  c.denom_a = (float)PyFloat_AsDouble(PyTuple_GET_ITEM(o, 1));
+  const int H = (int)PyLong_AsLong(PyTuple_GET_ITEM(o, 2));
+  float eps[5];
+  for (int i = 0; i < 5; ++i) eps[i] = (float)PyFloat_AsDouble(PyTuple_GET_ITEM(o, 3 + i));
+  const int64_t spin = PyLong_AsLongLong(PyTuple_GET_ITEM(o, 8));
+  const bool keys_only = PyObject_IsTrue(PyTuple_GET_ITEM(o, 9)) == 1;
+  if (PyErr_Occurred()) return nullptr;
+  if ((int64_t)H * 128 != C) Py_RETURN_NONE;
+  // the cached window
+  const uint64_t* kv[6] = {};
+  int64_t n_cached = 0;
+  int bts = 0;
+  float e2 = 6.f, e4 = 256.f;
+  if (args[6] != Py_None) {
+    if (!PyTuple_CheckExact(args[6]) || PyTuple_GET_SIZE(args[6]) != 6) Py_RETURN_NONE;
+    for (int i = 0; i < 2; ++i) {
+      const Tensor* t = as_tensor(PyTuple_GET_ITEM(args[6], i));
+      if (!t || !on_device(*t, dev) || t->scalar_type() != at::kLong || t->dim() != 2 || t->size(0) != 3 || !t->is_contiguous()) Py_RETURN_NONE;
+      for (int j = 0; j < 3; ++j) kv[3 * i + j] = reinterpret_cast<const uint64_t*>(t->data_ptr<int64_t>()) + j * t->size(1);
+    }
+    n_cached = PyLong_AsLongLong(PyTuple_GET_ITEM(args[6], 2));
+    bts = (int)PyLong_AsLong(PyTuple_GET_ITEM(args[6], 3));
+    e2 = (float)PyFloat_AsDouble(PyTuple_GET_ITEM(args[6], 4));
+    e4 = (float)PyFloat_AsDouble(PyTuple_GET_ITEM(args[6], 5));
+    if (PyErr_Occurred()) return nullptr;
+  }
+  // the text: its context, or the projected keys and values
+  const Tensor* context = as_tensor(args[7]);
+  Tensor text_k, text_v;
+  int64_t T = 0;
+  if (context) {
+    if (!is_bf16(*context, dev) || context->dim() != 3 || context->size(0) != 1 || context->size(2) != C || !context->is_contiguous() ||
+        context->size(1) == 0)
+      Py_RETURN_NONE;
+    T = context->size(1);
+  } else {
+    if (!PyTuple_CheckExact(args[7]) || PyTuple_GET_SIZE(args[7]) != 2) Py_RETURN_NONE;
+    const Tensor *tk = as_tensor(PyTuple_GET_ITEM(args[7], 0)), *tv = as_tensor(PyTuple_GET_ITEM(args[7], 1));
+    if (!tk || !tv || !is_bf16(*tk, dev) || !is_bf16(*tv, dev) || !tk->is_contiguous() || !tv->is_contiguous() || tk->dim() != 4 ||
+        tk->sizes() != tv->sizes() || tk->size(0) != 1 || tk->size(2) != H || tk->size(3) != 128 || tk->size(1) == 0)
+      Py_RETURN_NONE;
+    text_k = *tk;
+    text_v = *tv;
+    T = tk->size(1);
+  }
+  ll_amax_sink kv_sink[2] = {{nullptr, 0, nullptr}, {nullptr, 0, nullptr}};
+  for (int i = 0; i < 2; ++i) {
+    PyObject* t = args[9 + i];
+    if (t == Py_None) continue;
+    const Tensor* parts = PyTuple_CheckExact(t) && PyTuple_GET_SIZE(t) == 2 ? as_tensor(PyTuple_GET_ITEM(t, 0)) : nullptr;
+    if (!parts || !on_device(*parts, dev)) Py_RETURN_NONE;
+    kv_sink[i] = ll_amax_sink{reinterpret_cast<uint64_t*>(parts->data_ptr<int64_t>()), (uint32_t)PyLong_AsUnsignedLong(PyTuple_GET_ITEM(t, 1)), nullptr};
+    if (PyErr_Occurred()) return nullptr;
+  }
+  c.stream = stream_of(dev);
+  Epochs ep;
+  if (args[11] == Py_None) {
+    ep = epochs_of_stream(dev, c.stream);
+    if (!ep.parts) Py_RETURN_NONE;
+  } else {
+    PyObject* t = args[11];
+    const Tensor *parts = as_tensor(PyTuple_GET_ITEM(t, 0)), *offset = as_tensor(PyTuple_GET_ITEM(t, 2));
+    if (!parts || !offset || !on_device(*parts, dev) || !on_device(*offset, dev)) Py_RETURN_NONE;
+    ep = Epochs{reinterpret_cast<uint64_t*>(parts->data_ptr<int64_t>()), reinterpret_cast<const uint32_t*>(offset->data_ptr<int32_t>()),
+                (uint32_t)PyLong_AsUnsignedLong(PyTuple_GET_ITEM(t, 1))};
+    if (PyErr_Occurred()) return nullptr;
+  }
+#define LL_TRY(call, what) \
+  if (failed(call, what)) return nullptr
+
+  const uint16_t* mod = static_cast<const uint16_t*>(e.data_ptr());
+  const int64_t sb = e.stride(0), sf = e.stride(1);
+  auto modulation = [&](int i) { return mod + i * e.stride(2); };
+  // LayerNorm(h) * (1 + e[scale]) + e[shift] as an NVFP4 operand: one launch, or two where the rows do not fit one
+  auto adaln_operand = [&](const void* h, int scale, int shift, const TempOperand& q) -> int {
+    const ll_amax_sink sink = ep.take();
+    int code = ll_adaln_quantize(h, 1, L, (int)C, modulation(scale), modulation(shift), sb, sf, sb, sf, frame_rows, eps[0], 1, c.rule,
+                                 q.values, q.scales, q.amax, &sink, spin, c.stream);
+    if (code != LL_ENOSUP) return code;
+    const ll_amax_sink again = ep.take();
+    const Tensor y = empty({L, C}, at::kBFloat16, dev);
+    code = ll_adaln_modulate_amax(h, 1, L, (int)C, modulation(scale), modulation(shift), sb, sf, sb, sf, frame_rows, eps[0], 1,
+                                  y.data_ptr(), &again, c.stream);
+    return code ? code : c.quantize_from(y, L, C, q, again);
+  };
+  const TempOperand xq = c.operand(L, C);
+  LL_TRY(adaln_operand(x.data_ptr(), 1, 0, xq), "adaLN");
+
+  // ---- self-attention
+  const Tensor value = empty({1, L, H, 128}, at::kBFloat16, dev), key = empty({1, L, H, 128}, at::kBFloat16, dev);
+  Tensor attended;  // [L, C]
+  {
+    const Tensor q = empty({L, C}, at::kBFloat16, dev), k = empty({L, C}, at::kBFloat16, dev);
+    const Layer* const layers[3] = {&w[Q], &w[K], &w[V]};
+    void* const outs[3] = {q.data_ptr(), k.data_ptr(), value.data_ptr()};
+    const ll_amax_sink sinks[3] = {{nullptr, 0, nullptr}, {nullptr, 0, nullptr}, kv_sink[1]};
+    LL_TRY(c.grouped(xq, layers, 3, L, outs, sinks), "q / k / v projections");
+    const Tensor roped_q = empty({L, C}, at::kBFloat16, dev), smooth_k = empty({L, C}, at::kBFloat16, dev);
+    LL_TRY(ll_qk_norm_rope_pair_amax(q.data_ptr(), k.data_ptr(), L, H, norm[0], norm[1], eps[1], cos->data_ptr<float>(),
+                                     sin->data_ptr<float>(), L, roped_q.data_ptr(), key.data_ptr(), smooth_k.data_ptr(), &kv_sink[0],
+                                     c.stream),
+           "norm and RoPE");
+    if (keys_only) {
+      PyObject* r = PyTuple_New(5);
+      if (!r) return nullptr;
+      for (int i : {0, 3, 4}) {
+        Py_INCREF(Py_None);
+        PyTuple_SET_ITEM(r, i, Py_None);
+      }
+      PyTuple_SET_ITEM(r, 1, THPVariable_Wrap(key));
+      PyTuple_SET_ITEM(r, 2, THPVariable_Wrap(value));
+      return r;
+    }
+    attended = empty({L, C}, at::kBFloat16, dev);
+    const ll_amax_sink sink = ep.take();
+    LL_TRY(ll_kv_attention_amax(roped_q.data_ptr(), L, H, kv[0], kv[1], kv[2], kv[3], kv[4], kv[5], n_cached, bts, e2, e4,
+                                smooth_k.data_ptr(), value.data_ptr(), L, 0.08838834764831845f, attended.data_ptr(), &sink, c.stream),
+           "self-attention");
+    LL_TRY(c.quantize_from(attended, L, C, xq, sink), "quantization");
+  }
+  const Tensor x1 = empty({1, L, C}, at::kBFloat16, dev);
+  ll_gemm_epilogue plain_epilogue{}, gated{};
+  gated.gate_rows = frame_rows;
+  gated.gate_stride = sf;
+  gated.ldr = C;
+  gated.gate = modulation(2);
+  gated.residual = x.data_ptr();
+  LL_TRY(c.gemm(xq, w[O], L, x1.data_ptr(), gated), "output projection");
+
+  // ---- cross-attention
+  {
+    const ll_amax_sink sink = ep.take();
+    int code = ll_layer_norm_quantize(x1.data_ptr(), L, (int)C, norm[2], norm[3], eps[2], c.rule, xq.values, xq.scales, xq.amax, &sink, spin,
+                                      c.stream);
+    if (code == LL_ENOSUP) {
+      const ll_amax_sink again = ep.take();
+      const Tensor y = empty({L, C}, at::kBFloat16, dev);
+      code = ll_layer_norm(x1.data_ptr(), L, (int)C, norm[2], norm[3], eps[2], y.data_ptr(), &again, c.stream);
+      if (!code) code = c.quantize_from(y, L, C, xq, again);
+    }
+    LL_TRY(code, "norm3");
+  }
+  {
+    const Tensor q = empty({L, C}, at::kBFloat16, dev), qn = empty({L, C}, at::kBFloat16, dev);
+    LL_TRY(c.gemm(xq, w[CQ], L, q.data_ptr(), plain_epilogue), "cross-attention q");
+    LL_TRY(ll_rms_norm(q.data_ptr(), L, (int)C, norm[4], eps[3], qn.data_ptr(), c.stream), "cross-attention norm_q");
+    if (context) {
+      const TempOperand tq = c.operand(T, C);
+      LL_TRY(ll_nvfp4_quantize(context->data_ptr(), T, C, C, c.rule, tq.values, tq.scales, tq.amax, 0, tq.workspace, c.stream), "text quantization");
+      const Tensor k = empty({T, C}, at::kBFloat16, dev);
+      text_k = empty({1, T, H, 128}, at::kBFloat16, dev);
+      text_v = empty({1, T, H, 128}, at::kBFloat16, dev);
+      const Layer* const layers[2] = {&w[CK], &w[CV]};
+      void* const outs[2] = {k.data_ptr(), text_v.data_ptr()};
+      LL_TRY(c.grouped(tq, layers, 2, T, outs, nullptr), "text projections");
+      LL_TRY(ll_rms_norm(k.data_ptr(), T, (int)C, norm[5], eps[4], text_k.data_ptr(), c.stream), "cross-attention norm_k");
+    }
+    const ll_amax_sink sink = ep.take();
+    LL_TRY(ll_kv_attention_amax(qn.data_ptr(), L, H, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0, 6.f, 256.f,
+                                text_k.data_ptr(), text_v.data_ptr(), T, 0.08838834764831845f, attended.data_ptr(), &sink, c.stream),
+           "cross-attention");
+    LL_TRY(c.quantize_from(attended, L, C, xq, sink), "quantization");
+  }
+  const Tensor x2 = empty({1, L, C}, at::kBFloat16, dev);
+  ll_gemm_epilogue residual{};
+  residual.ldr = C;
+  residual.residual = x1.data_ptr();
+  LL_TRY(c.gemm(xq, w[CO], L, x2.data_ptr(), residual), "cross-attention output projection");
+
+  // ---- feed-forward
+  LL_TRY(adaln_operand(x2.data_ptr(), 4, 3, xq), "adaLN");
+  const Tensor hidden = empty({L, w[UP].n}, at::kBFloat16, dev);
+  ll_gemm_epilogue gelu{};
+  gelu.activation = LL_ACT_GELU_TANH;
+  gelu.amax_sink = ep.take();
+  LL_TRY(c.gemm(xq, w[UP], L, hidden.data_ptr(), gelu), "FFN up");
+  const TempOperand hq = c.operand(L, w[UP].n);
+  LL_TRY(c.quantize_from(hidden, L, w[UP].n, hq, gelu.amax_sink), "quantization");
+  const Tensor& out = attended;  // its memory is free by now
+  gated.gate = modulation(5);
+  gated.residual = x2.data_ptr();
+  LL_TRY(c.gemm(hq, w[DOWN], L, out.data_ptr(), gated), "FFN down");
+#undef LL_TRY
+
+  PyObject* r = PyTuple_New(5);
+  if (!r) return nullptr;
+  PyTuple_SET_ITEM(r, 0, THPVariable_Wrap(out.view({1, L, C})));
+  PyTuple_SET_ITEM(r, 1, THPVariable_Wrap(key));
+  PyTuple_SET_ITEM(r, 2, THPVariable_Wrap(value));
+  PyTuple_SET_ITEM(r, 3, THPVariable_Wrap(text_k));
+  PyTuple_SET_ITEM(r, 4, THPVariable_Wrap(text_v));
+  return r;
+  END_HANDLE_TH_ERRORS
+}
+
+// current_stream() -> the current HIP stream of the current device as an integer
+PyObject* py_current_stream(PyObject*, PyObject*) {
+  HANDLE_TH_ERRORS
+  return PyLong_FromVoidPtr(stream_of(c10::hip::current_device()));
+  END_HANDLE_TH_ERRORS
+}
+
+// release_stream_sink(): gives back the amax sink of (current device, current stream)
+PyObject* py_release_stream_sink(PyObject*, PyObject*) {
+  HANDLE_TH_ERRORS
+  const int dev = c10::hip::current_device();
+  std::lock_guard<std::mutex> lock(g_sink_mutex);
+  stream_sinks().erase({dev, stream_of(dev)});
+  Py_RETURN_NONE;
+  END_HANDLE_TH_ERRORS
+}
+
 PyMethodDef methods[] = {
+    {"block_forward", (PyCFunction)(void (*)(void))py_block_forward, METH_FASTCALL, nullptr},
+    {"current_stream", py_current_stream, METH_NOARGS, nullptr},
+    {"release_stream_sink", py_release_stream_sink, METH_NOARGS, nullptr},
     {"quantize", (PyCFunction)(void (*)(void))py_quantize, METH_FASTCALL, nullptr},
     {"linear", (PyCFunction)(void (*)(void))py_linear, METH_FASTCALL, nullptr},
     {"dequantize", (PyCFunction)(void (*)(void))py_dequantize, METH_FASTCALL, nullptr},
@@ -168,4 +532,8 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host_ops", nullptr, -1, methods, 
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__host_ops(void) { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__host_ops(void) {
+  PyObject* m = PyModule_Create(&module);
+  if (m) PyModule_AddIntConstant(m, "EPOCHS_PER_CALL", kEpochsPerCall);
+  return m;
+}

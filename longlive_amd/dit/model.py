@@ -144,6 +144,14 @@ class CausalSelfAttention(nn.Module):
         self.norm_q, self.norm_k = WanRMSNorm(dim, eps), WanRMSNorm(dim, eps)
         self.use_relative_rope = False  # set on the module by the pipeline (pipeline/causal_diffusion_inference.py:316)
 
+    @staticmethod
+    def amax_sinks(kv_cache: dict, device):
+        """The two sinks of a layer's cache in which the producers of K and V leave the maxima for the cache write."""
+        sinks = kv_cache.get("_amax_sinks")
+        if sinks is None:
+            sinks = kv_cache["_amax_sinks"] = (_native.PrivateAmaxSink(device), _native.PrivateAmaxSink(device))
+        return sinks
+
     def forward(self, x, cos, sin, kv_cache, current_start, sink_tokens, max_attention_size, *, input_amax=None,
                 residual=None, gate=None, gate_rows=0, global_sink_tokens=0, rope_fn=None, collect_kv_amax=True,
                 keys_only=False):
@@ -165,10 +173,7 @@ class CausalSelfAttention(nn.Module):
         fused_path = b == 1 and d == 128 and not self.use_relative_rope and self.norm_q.eps == self.norm_k.eps
         k_amax = v_amax = None
         if fused_path and collect_kv_amax and isinstance(kv_cache, dict):
-            sinks = kv_cache.get("_amax_sinks")
-            if sinks is None:
-                sinks = kv_cache["_amax_sinks"] = (_native.PrivateAmaxSink(x.device), _native.PrivateAmaxSink(x.device))
-            k_amax, v_amax = sinks[0].ticket(), sinks[1].ticket()
+            k_amax, v_amax = (sink.ticket() for sink in self.amax_sinks(kv_cache, x.device))
         (q, k, v), v_amax_written = _project_shared(x, [self.q, self.k, self.v], amax=input_amax,
                                                     amax_outs=[None, None, v_amax])
         v = v.view(b, s, n, d)
@@ -248,6 +253,13 @@ class CrossAttention(nn.Module):
         return _project_out(self.o, out.unsqueeze(0).flatten(2), out_amax, residual, None, 0)
 
 
+def _has_hooks(*modules) -> bool:
+    """Whether calling one of the modules would run more than its forward."""
+    g = torch.nn.modules.module
+    return bool(g._global_forward_hooks or g._global_forward_pre_hooks) or any(
+        m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__ for m in modules)
+
+
 class DiTBlock(nn.Module):
     # normalize and quantize in one launch where a quantized layer reads the result (the same bytes either way)
     fuse_norm_quantize = True
@@ -287,7 +299,12 @@ class DiTBlock(nn.Module):
         ``keys_only``: the block's output has no reader (last block of a pass that only rewrites the cache):
         the block stops behind the producers of the chunk's K and V and returns ``(None, update)``."""
         num_frames, frame_seqlen = e.shape[1], x.shape[1] // e.shape[1]
-        e = (self.modulation.unsqueeze(1) + e if modulated is None else modulated).chunk(6, dim=2)
+        e = self.modulation.unsqueeze(1) + e if modulated is None else modulated
+        done = self._forward_native(x, e, cos, sin, context, kv_cache, current_start, sink_tokens, max_attention_size,
+                                    crossattn_cache, global_sink_tokens, collect_kv_amax, keys_only)
+        if done is not None:
+            return done
+        e = e.chunk(6, dim=2)
         gates = [g.reshape(-1, g.shape[-1]) for g in (e[2], e[5])]  # [B*F, C] views, one row per frame
         sa = self.self_attn
         y, y_amax = self._normalized_for([sa.q, sa.k, sa.v], x, scale=e[1], shift=e[0], frame_seqlen=frame_seqlen)
@@ -305,6 +322,57 @@ class DiTBlock(nn.Module):
                                          operand_ok=fused_ffn)
         x = self._feed_forward(y, y_amax, x, gates[1], frame_seqlen)
         return x, update
+
+    def _forward_native(self, x, e, cos, sin, context, kv_cache, current_start, sink_tokens, max_attention_size,
+                        crossattn_cache, global_sink_tokens, collect_kv_amax, keys_only):
+        """:meth:`forward` as one native call (``block_forward`` of csrc/host_ops.cpp): the same kernels on the same
+        values in the same order, without Python between the launches.  ``None`` where a layer, a layout or an option
+        is not the common one; :meth:`forward` then runs the operations one by one."""
+        sa, ca, norm3, ffn = (self._modules[name] for name in ("self_attn", "cross_attn", "norm3", "ffn"))
+        if (not x.is_cuda or type(sa) is not CausalSelfAttention or type(ca) is not CrossAttention or sa.use_relative_rope
+                or type(norm3) is not WanLayerNorm or norm3.weight is None or sa.head_dim != 128 or not self.fuse_norm_quantize
+                or not isinstance(kv_cache, dict) or len(ffn) != 3 or getattr(ffn[1], "approximate", None) != "tanh"):
+            return None
+        sm, cm = sa._modules, ca._modules
+        norms = (sm["norm_q"], sm["norm_k"], cm["norm_q"], cm["norm_k"])
+        if norms[0].eps != norms[1].eps or any(type(n) is not WanRMSNorm for n in norms) or _has_hooks(sa, ca, norm3, *norms):
+            return None
+        linears = (sm["q"], sm["k"], sm["v"], sm["o"], cm["q"], cm["k"], cm["v"], cm["o"], ffn[0], ffn[2])
+        rule, layers = None, []
+        for m in linears:
+            operand = m.native_operand() if type(m) is FourOverSixLinear else None
+            if operand is None or (rule is not None and m.config.activation_scale_rule is not rule):
+                return None
+            rule = m.config.activation_scale_rule
+            layers.append(operand)
+        text = context
+        if crossattn_cache is not None and crossattn_cache.get("is_init"):
+            text = (crossattn_cache["k"], crossattn_cache["v"])
+        slot_ids, info, local_end = kvc.plan_cache_step(kv_cache, current_start, x.shape[1], sink_tokens, max_attention_size,
+                                                        global_sink_tokens)
+        window = None
+        if not keys_only:
+            if slot_ids is None:
+                return None
+            if slot_ids:
+                kt, vt = kvc._tables_for(kv_cache, slot_ids)
+                kv_rule, blk = kv_cache["k"][0].scale_rule, kv_cache["block_token_size"]
+                window = (kt.table, vt.table, len(slot_ids) * blk, blk, kv_rule.max_allowed_e2m1_value(),
+                          kv_rule.max_allowed_e4m3_value())
+        tickets = (None, None)
+        if collect_kv_amax:
+            tickets = tuple(sink.ticket() for sink in sa.amax_sinks(kv_cache, x.device))
+        out = _native.block_forward(
+            x, e, tuple(layers), (norms[0].weight, norms[1].weight, norm3.weight, norm3.bias, norms[2].weight, norms[3].weight),
+            cos, sin, window, text, rule.value, (sa.num_heads, self.eps, norms[0].eps, norm3.eps, norms[2].eps, norms[3].eps),
+            keys_only, tickets)
+        if out is None:
+            return None
+        y, info["new_k"], info["new_v"], text_k, text_v = out
+        info["new_k_amax"], info["new_v_amax"] = tickets
+        if not keys_only and crossattn_cache is not None and text is context:
+            crossattn_cache.update(is_init=True, k=text_k, v=text_v)
+        return y, (current_start + x.shape[1], local_end, info)
 
     def _normalized_for(self, layers, x, *, scale=None, shift=None, frame_seqlen=0, norm=None, operand_ok=True):
         """The adaLN modulation of ``x`` (``scale`` / ``shift`` given) or ``norm(x)`` as input of ``layers``:

@@ -137,6 +137,15 @@ class FourOverSixLinear(nn.Linear):
                 return out
         return self.forward_quantized(self.quantize_input(x2d))
 
+    def native_operand(self):
+        """(values, scale factors, amax, bias or None, denominator, out_features) for the native calls that run this
+        layer among others; ``None`` when it has no quantized weight or another type than NVFP4 in, bf16 out."""
+        config, weight = self.config, self.quantized_weight()
+        if not isinstance(weight, QuantizedTensor) or config.output_dtype is not DataType.bfloat16 or config.dtype is not DataType.nvfp4:
+            return None
+        return (weight.values, weight.scale_factors, weight.amax, self._parameters.get("bias"),
+                _native.DENOMINATORS[weight.scale_rule._value_], weight.original_shape[0])
+
     def quantize_input(self, x2d: torch.Tensor, amax=None) -> QuantizedTensor:
         """The activation operand exactly as ``forward`` would build it from a 2-D input.  ``amax`` is
         the amax ticket of the kernel that produced ``x2d``, if it was given one."""

@@ -923,3 +923,60 @@ def test_leaving_out_the_unread_tail_of_the_clean_context_pass_changes_nothing(g
         for sa, sb in zip(la["k"] + la["v"], lb["k"] + lb["v"]):
             assert torch.equal(sa.values, sb.values) and torch.equal(sa.amax, sb.amax)
             assert torch.equal(sa.scale_factors.view(torch.uint8), sb.scale_factors.view(torch.uint8))
+
+
+@pytest.mark.parametrize("F,h,w,heads,ffn,T,cached,keep_text", [
+    (1, 1, 1, 1, 64, 1, 0, False),       # one token, one head, one text token
+    (2, 23, 16, 8, 1000, 77, 2, True),   # ragged rows, FFN width and text
+    (1, 16, 24, 24, 14336, 512, 1, False),
+    (3, 1, 43, 4, 512, 16, 0, True),     # one row past a tile
+])
+def test_native_block_call_equals_the_separate_operations(gpu, F, h, w, heads, ffn, T, cached, keep_text):
+    """The block as one native call runs the same kernels on the same values as the operations one by one (taken when
+    a submodule has a hook): outputs, cache update and text K / V are the same bits, on the default and on a side
+    stream, with and without the text projections kept, and for the pass that stops at K and V."""
+    torch.manual_seed(0)
+    dim, L = heads * 128, F * h * w
+    block, _ = quantize_model_with_filter(DiTBlock(dim, ffn, heads).to(gpu), ModelQuantizationConfig(), use_default_filtered_modules=True,
+                                          materialize_for_inference=True, verbose=False)
+    g = torch.Generator().manual_seed(5)
+
+    def run(native, keys_only=False):
+        cache = kvc.initialize_kv_cache(1, L, cached + 1, heads, 128, KV, gpu)[0]
+        for name in "kv":
+            for slot, values in zip(cache[name], slots[name]):
+                slot.values.copy_(values), slot.scale_factors.fill_(1.0), slot.amax.fill_(4.0)
+        cache["_global_end"] = cache["_local_end"] = cached * L
+        hook = None if native else block.self_attn.register_forward_hook(lambda *a: None)
+        text = {"is_init": False} if keep_text else None
+        outs = []
+        for _ in range(2):  # with keep_text the second call reads the first's text K and V
+            y, (ce, le, info) = block(x, e, cos, sin, ctx, cache, cached * L, sink_tokens=0, crossattn_cache=text, keys_only=keys_only)
+            outs += [y, info["new_k"], info["new_v"]]
+            outs += [text["k"], text["v"]] if keep_text and not keys_only else []
+            assert (ce, le) == ((cached + 1) * L,) * 2 and info["new_k_amax"].parts is cache["_amax_sinks"][0].parts
+            kvc.apply_cache_update(cache, ce, le, info, KV)
+            outs += [t.clone() for n in "kv" for s in (cache[n][cached],) for t in (s.values, s.scale_factors.view(torch.uint8), s.amax)]
+            cache["_global_end"] = cache["_local_end"] = cached * L
+        if hook is not None:
+            hook.remove()
+        return outs
+
+    x = torch.randn(1, L, dim, generator=g).bfloat16().to(gpu)
+    e = torch.randn(1, F, 6, dim, generator=g).bfloat16().to(gpu)
+    ctx = torch.randn(1, T, dim, generator=g).bfloat16().to(gpu)
+    cos, sin = rope_cos_sin(build_rope_angles(128), F, h, w, cached * F, gpu)
+    rows = -(-L * heads // 128) * 128
+    slots = {n: [torch.randint(0, 256, (rows, 64), generator=g, dtype=torch.uint8).to(gpu) for _ in range(cached + 1)] for n in "kv"}
+    with torch.no_grad():
+        for keys_only in (False, True):
+            ref = run(False, keys_only)
+            side = torch.cuda.Stream()
+            side.wait_stream(torch.cuda.current_stream())
+            with torch.cuda.stream(side):
+                on_side = run(True, keys_only)
+            torch.cuda.current_stream().wait_stream(side)
+            for got in (run(True, keys_only), on_side):
+                assert len(got) == len(ref)
+                for i, (a, b) in enumerate(zip(got, ref)):
+                    assert (a is None and b is None) or torch.equal(a, b), i

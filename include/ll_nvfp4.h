@@ -131,6 +131,13 @@ int ll_nvfp4_quantize_pair_from_sinks(const void* x0, const void* x1, int64_t M,
                                       float* amax0, float* amax1, const ll_amax_sink* amax_sink0,
                                       const ll_amax_sink* amax_sink1, void* stream);
 
+/* Two ll_nvfp4_quantize calls (amax_given == 0) on tensors of the same shape, leading dimension and rule: one launch for
+ * both maxima and one for both quantizations.  workspace: 2 * ll_nvfp4_quantize_workspace_floats() floats.  The bytes equal
+ * those of the two calls. */
+int ll_nvfp4_quantize_pair(const void* x0, const void* x1, int64_t M, int64_t K, int64_t ldx, int rule,
+                           uint8_t* values0, uint8_t* values1, uint8_t* scales0, uint8_t* scales1,
+                           float* amax0, float* amax1, float* workspace, void* stream);
+
 /*
  * Replaces QuantizedTensor.dequantize (fouroversix/src/fouroversix/quantize/quantized_tensor.py:184-214):
  * out[r, c] = cast(((e2m1 * e4m3) * amax) / (e2m1_max * e4m3_max)) for r < M, c < K; ldo in elements.
@@ -275,6 +282,25 @@ int ll_nvfp4_gemm_kernel(int64_t M, int64_t N, int64_t Kp, int n_products, int c
 int ll_kv_dequantize_blocks(const uint64_t* values_ptrs, const uint64_t* scales_ptrs, const uint64_t* amax_ptrs,
                             int n_blocks, int num_heads, int block_token_size, int out_dtype,
                             float e2m1_max, float e4m3_max, void* out, void* stream);
+
+/* k - mean(k over the head dimension) of bf16 [tokens, H, 128] (utils/quant.py:797-798): fp32 sum of a head, mean rounded to
+ * bf16, difference rounded to bf16. */
+int ll_kv_smooth(const void* k, int64_t tokens, int num_heads, void* out, void* stream);
+
+/*
+ * The operands of attention with relative RoPE (wan_5b/modules/causal_model.py:486-487, 716-771) in one launch:
+ *   k_out = rope([cached K slots | ll_kv_smooth(k_new)]), v_out = [cached V slots | v_new], q_out = rope(q)
+ * with the values of ll_kv_dequantize_blocks (bf16), ll_kv_smooth and ll_rope_apply.  q bf16 [Lq, H, 128]; k_new, v_new bf16
+ * [n_new, H, 128], n_new > 0; n_cached >= 0 whole slots; cos_k / sin_k f32 [n_cached + n_new, 64], cos_q / sin_q f32 [Lq, 64];
+ * outputs bf16 [n_cached + n_new, H, 128] and [Lq, H, 128].  All pointers 16-byte aligned; slot pointer arrays as above.
+ */
+int ll_kv_window_rope(const void* q, int64_t Lq, int num_heads,
+                      const uint64_t* k_values_ptrs, const uint64_t* k_scales_ptrs, const uint64_t* k_amax_ptrs,
+                      const uint64_t* v_values_ptrs, const uint64_t* v_scales_ptrs, const uint64_t* v_amax_ptrs,
+                      int64_t n_cached, int block_token_size, float e2m1_max, float e4m3_max,
+                      const void* k_new, const void* v_new, int64_t n_new,
+                      const float* cos_k, const float* sin_k, const float* cos_q, const float* sin_q,
+                      void* q_out, void* k_out, void* v_out, void* stream);
 
 /*
  * FP4 KV-cache attention for one chunk; replaces dequantize_kv_cache + slice copies + flash attention

@@ -50,6 +50,11 @@ _SIGNATURES = {
                                         c_void_p, c_void_p]),
     "ll_nvfp4_gemm_tnt_grouped": (c_int, [c_void_p, c_void_p, c_void_p, c_float, c_int64, c_int64, c_int64, c_int64,
                                           c_int64, c_int, c_void_p, c_void_p]),
+    "ll_nvfp4_quantize_pair": (c_int, [c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int, c_void_p, c_void_p, c_void_p,
+                                       c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
+    "ll_kv_smooth": (c_int, [c_void_p, c_int64, c_int, c_void_p, c_void_p]),
+    "ll_kv_window_rope": (c_int, [c_void_p, c_int64, c_int, *[c_void_p] * 6, c_int64, c_int, c_float, c_float, c_void_p, c_void_p,
+                                  c_int64, *[c_void_p] * 8]),
     "ll_kv_dequantize_blocks": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_float, c_float,
                                         c_void_p, c_void_p]),
     "ll_kv_attention": (c_int, [c_void_p, c_int64, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
@@ -419,6 +424,22 @@ def quantize_pair(x0: torch.Tensor, x1: torch.Tensor, rule: str, ticket0: AmaxTi
             ctypes.byref(s1), _stream())
     _check(code, "ll_nvfp4_quantize_pair_from_sinks")
     return out0, out1
+
+
+def cache_write(k, v, first: int, tokens: int, rule: str, k_out, v_out, k_ticket, v_ticket) -> bool:
+    """Tokens first .. first + tokens of the chunk's K and V [1, n, H, 128] into their slots, (values, scale_factors, amax)
+    each, in one native call: both maxima in one launch unless the two producers left them behind (the tickets), both
+    quantizations in one.  False when the call is not a common one and nothing was done."""
+    if not k.is_cuda or (k_ticket is None) != (v_ticket is None):
+        return False
+    sinks = (None, None)
+    if k_ticket is not None:
+        for t in (k_ticket, v_ticket):
+            if not isinstance(t, AmaxTicket) or t.offset is not None:
+                return False
+            _check_consumer(t)
+        sinks = ((k_ticket.parts, k_ticket.epoch), (v_ticket.parts, v_ticket.epoch))
+    return host().cache_write(k, v, first, tokens, RULE_IDS[rule], k_out, v_out, *sinks) is True
 
 
 def dequantize(values, scales, amax, rule: str, padded, original, dtype: torch.dtype) -> torch.Tensor:

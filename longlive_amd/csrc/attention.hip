@@ -33,7 +33,6 @@ namespace ll {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float float16v __attribute__((ext_vector_type(16)));
-typedef float float2v __attribute__((ext_vector_type(2)));
 
 constexpr int kHeadDim = 128;
 constexpr int kTileKeys = 64;                  // keys per wave tile

@@ -44,18 +44,6 @@ __device__ __forceinline__ void store1(void* out, int64_t off, float v) {
   }
 }
 
-typedef float float2v __attribute__((ext_vector_type(2)));
-
-// The eight e2m1 values of one packed dword, exact, in four conversions.
-__device__ __forceinline__ void fp4x8_values(uint32_t w, float (&q)[8]) {
-  const float2v p0 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w, 1.0f, 0);
-  const float2v p1 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w, 1.0f, 1);
-  const float2v p2 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w, 1.0f, 2);
-  const float2v p3 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w, 1.0f, 3);
-  q[0] = p0[0]; q[1] = p0[1]; q[2] = p1[0]; q[3] = p1[1];
-  q[4] = p2[0]; q[5] = p2[1]; q[6] = p3[0]; q[7] = p3[1];
-}
-
 // out = ((q * s) * amax) / denom.  HBM bound: 0.5625 bytes in and 2 (f32: 4) out per element.  The value of an e2m1
 // number q = m * 2^k (m = 1 or 1.5) is 2^k * d(m, s) with d(m, s) = ((m * s) * amax) / denom, exactly (a power of two
 // commutes with both roundings while nothing under- or overflows, which the bound on amax guarantees), so the

@@ -235,6 +235,36 @@ bool parse_layer(PyObject* t, int dev, Layer& l) {
   l.denom = (float)PyFloat_AsDouble(PyTuple_GET_ITEM(t, 4));
   return true;
 }
+// The attended slots: (table of the K slots, of the V slots, cached keys, block_token_size, e2m1_max, e4m3_max) or None.
+struct Window {
+  const uint64_t* p[6] = {};  // K values, scales, amax, then V
+  int64_t n_cached = 0;
+  int bts = 0;
+  float e2 = 6.f, e4 = 256.f;
+};
+bool parse_window(PyObject* o, int dev, Window& w) {
+  if (o == Py_None) return true;
+  if (!PyTuple_CheckExact(o) || PyTuple_GET_SIZE(o) != 6) return false;
+  for (int i = 0; i < 2; ++i) {
+    const Tensor* t = as_tensor(PyTuple_GET_ITEM(o, i));
+    if (!t || !on_device(*t, dev) || t->scalar_type() != at::kLong || t->dim() != 2 || t->size(0) != 3 || !t->is_contiguous()) return false;
+    for (int j = 0; j < 3; ++j) w.p[3 * i + j] = reinterpret_cast<const uint64_t*>(t->data_ptr<int64_t>()) + j * t->size(1);
+  }
+  w.n_cached = PyLong_AsLongLong(PyTuple_GET_ITEM(o, 2));
+  w.bts = (int)PyLong_AsLong(PyTuple_GET_ITEM(o, 3));
+  w.e2 = (float)PyFloat_AsDouble(PyTuple_GET_ITEM(o, 4));
+  w.e4 = (float)PyFloat_AsDouble(PyTuple_GET_ITEM(o, 5));
+  return !PyErr_Occurred();
+}
+
+// A (parts, epoch) tuple as a sink; false: not one.
+bool parse_sink(PyObject* t, int dev, ll_amax_sink& s) {
+  const Tensor* parts = PyTuple_CheckExact(t) && PyTuple_GET_SIZE(t) == 2 ? as_tensor(PyTuple_GET_ITEM(t, 0)) : nullptr;
+  if (!parts || !on_device(*parts, dev)) return false;
+  s = ll_amax_sink{reinterpret_cast<uint64_t*>(parts->data_ptr<int64_t>()), (uint32_t)PyLong_AsUnsignedLong(PyTuple_GET_ITEM(t, 1)), nullptr};
+  return !PyErr_Occurred();
+}
+
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 struct BlockCall {
@@ -265,8 +295,7 @@ struct BlockCall {
 // block_forward(x, e, layers, norms, cos, sin, kv, text, options, k_sink, v_sink, graph_sink) ->
 //   (x_out or None, roped K [1, L, H, 128], V [1, L, H, 128], text K, text V) or None
 //   e: the six modulation vectors per frame [1, F, 6, C];  layers: q, k, v, o, cross q, k, v, o, FFN up, down;  norms: weights of
-//   norm_q, norm_k, norm3, norm3's bias, cross norm_q, cross norm_k;  kv: (table of the K slots, of the V slots, cached keys,
-//   block_token_size, e2m1_max, e4m3_max) or None;  text: the context [1, T, C] or (K, V) [1, T, H, 128];  options: (rule,
+//   norm_q, norm_k, norm3, norm3's bias, cross norm_q, cross norm_k;  kv: the window (see Window);  text: the context [1, T, C] or (K, V) [1, T, H, 128];  options: (rule,
 //   denominator, heads, eps, eps of q/k norm, of norm3, of cross norm_q, of cross norm_k, spin limit, keys_only);  k_sink,
 //   v_sink: (parts, epoch) or None;  graph_sink: (parts, last epoch, offset) or None.
 // The launches and their order are those of DiTBlock.forward (longlive_amd/dit/model.py), which documents them.
@@ -315,23 +344,10 @@ PyObject* py_block_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const bool keys_only = PyObject_IsTrue(PyTuple_GET_ITEM(o, 9)) == 1;
   if (PyErr_Occurred()) return nullptr;
   if ((int64_t)H * 128 != C) Py_RETURN_NONE;
-  // the cached window
-  const uint64_t* kv[6] = {};
-  int64_t n_cached = 0;
-  int bts = 0;
-  float e2 = 6.f, e4 = 256.f;
-  if (args[6] != Py_None) {
-    if (!PyTuple_CheckExact(args[6]) || PyTuple_GET_SIZE(args[6]) != 6) Py_RETURN_NONE;
-    for (int i = 0; i < 2; ++i) {
-      const Tensor* t = as_tensor(PyTuple_GET_ITEM(args[6], i));
-      if (!t || !on_device(*t, dev) || t->scalar_type() != at::kLong || t->dim() != 2 || t->size(0) != 3 || !t->is_contiguous()) Py_RETURN_NONE;
-      for (int j = 0; j < 3; ++j) kv[3 * i + j] = reinterpret_cast<const uint64_t*>(t->data_ptr<int64_t>()) + j * t->size(1);
-    }
-    n_cached = PyLong_AsLongLong(PyTuple_GET_ITEM(args[6], 2));
-    bts = (int)PyLong_AsLong(PyTuple_GET_ITEM(args[6], 3));
-    e2 = (float)PyFloat_AsDouble(PyTuple_GET_ITEM(args[6], 4));
-    e4 = (float)PyFloat_AsDouble(PyTuple_GET_ITEM(args[6], 5));
+  Window kv;
+  if (!parse_window(args[6], dev, kv)) {
     if (PyErr_Occurred()) return nullptr;
+    Py_RETURN_NONE;
   }
   // the text: its context, or the projected keys and values
   const Tensor* context = as_tensor(args[7]);
@@ -353,14 +369,11 @@ PyObject* py_block_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
     T = tk->size(1);
   }
   ll_amax_sink kv_sink[2] = {{nullptr, 0, nullptr}, {nullptr, 0, nullptr}};
-  for (int i = 0; i < 2; ++i) {
-    PyObject* t = args[9 + i];
-    if (t == Py_None) continue;
-    const Tensor* parts = PyTuple_CheckExact(t) && PyTuple_GET_SIZE(t) == 2 ? as_tensor(PyTuple_GET_ITEM(t, 0)) : nullptr;
-    if (!parts || !on_device(*parts, dev)) Py_RETURN_NONE;
-    kv_sink[i] = ll_amax_sink{reinterpret_cast<uint64_t*>(parts->data_ptr<int64_t>()), (uint32_t)PyLong_AsUnsignedLong(PyTuple_GET_ITEM(t, 1)), nullptr};
-    if (PyErr_Occurred()) return nullptr;
-  }
+  for (int i = 0; i < 2; ++i)
+    if (args[9 + i] != Py_None && !parse_sink(args[9 + i], dev, kv_sink[i])) {
+      if (PyErr_Occurred()) return nullptr;
+      Py_RETURN_NONE;
+    }
   c.stream = stream_of(dev);
   Epochs ep;
   if (args[11] == Py_None) {
@@ -422,8 +435,8 @@ PyObject* py_block_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
     }
     attended = empty({L, C}, at::kBFloat16, dev);
     const ll_amax_sink sink = ep.take();
-    LL_TRY(ll_kv_attention_amax(roped_q.data_ptr(), L, H, kv[0], kv[1], kv[2], kv[3], kv[4], kv[5], n_cached, bts, e2, e4,
-                                smooth_k.data_ptr(), value.data_ptr(), L, 0.08838834764831845f, attended.data_ptr(), &sink, c.stream),
+    LL_TRY(ll_kv_attention_amax(roped_q.data_ptr(), L, H, kv.p[0], kv.p[1], kv.p[2], kv.p[3], kv.p[4], kv.p[5], kv.n_cached, kv.bts, kv.e2,
+                                kv.e4,                                smooth_k.data_ptr(), value.data_ptr(), L, 0.08838834764831845f, attended.data_ptr(), &sink, c.stream),
            "self-attention");
     LL_TRY(c.quantize_from(attended, L, C, xq, sink), "quantization");
   }
@@ -502,6 +515,143 @@ PyObject* py_block_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// ------------------------------------------------------------------------------------------------ KV-cache step
+// A contiguous bf16 [1, tokens, H, 128] tensor of plain torch type on that device.
+const Tensor* as_chunk(PyObject* o, int dev) {
+  if (!plain(o)) return nullptr;
+  const Tensor& t = THPVariable_Unpack(o);
+  return is_bf16(t, dev) && t.dim() == 4 && t.size(0) == 1 && t.size(3) == 128 && t.numel() > 0 && t.is_contiguous() && aligned16(t.data_ptr()) ? &t
+                                                                                                                                                : nullptr;
+}
+
+// kv_attention(q, k, v, smoothed K or None, window, scale) -> [1, S, H, 128]
+PyObject* py_kv_attention(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 6 || !plain(args[0])) Py_RETURN_NONE;
+  const int dev = current_device_of(THPVariable_Unpack(args[0]));
+  if (dev < 0) Py_RETURN_NONE;
+  const Tensor *q = as_chunk(args[0], dev), *k = as_chunk(args[1], dev), *v = as_chunk(args[2], dev);
+  if (!q || !k || !v || k->sizes() != v->sizes() || k->size(2) != q->size(2)) Py_RETURN_NONE;
+  const int H = (int)q->size(2);
+  Tensor smooth;
+  if (args[3] != Py_None) {
+    const Tensor* s = as_chunk(args[3], dev);
+    if (!s || s->sizes() != k->sizes()) Py_RETURN_NONE;
+    smooth = *s;
+  }
+  Window w;
+  if (!parse_window(args[4], dev, w)) {
+    if (PyErr_Occurred()) return nullptr;
+    Py_RETURN_NONE;
+  }
+  const float scale = (float)PyFloat_AsDouble(args[5]);
+  if (PyErr_Occurred()) return nullptr;
+  void* stream = stream_of(dev);
+  if (!smooth.defined()) {
+    smooth = empty(k->sizes(), at::kBFloat16, dev);
+    if (failed(ll_kv_smooth(k->data_ptr(), k->size(1), H, smooth.data_ptr(), stream), "ll_kv_smooth")) return nullptr;
+  }
+  const Tensor out = empty(q->sizes(), at::kBFloat16, dev);
+  if (failed(ll_kv_attention(q->data_ptr(), q->size(1), H, w.p[0], w.p[1], w.p[2], w.p[3], w.p[4], w.p[5], w.n_cached, w.bts, w.e2, w.e4,
+                             smooth.data_ptr(), v->data_ptr(), k->size(1), scale, out.data_ptr(), stream),
+             "ll_kv_attention"))
+    return nullptr;
+  return THPVariable_Wrap(out);
+  END_HANDLE_TH_ERRORS
+}
+
+// kv_attention_relative(q, k, v, window, cos_k, sin_k, cos_q, sin_q, scale) -> [1, S, H, 128]
+PyObject* py_kv_attention_relative(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 9 || !plain(args[0])) Py_RETURN_NONE;
+  const int dev = current_device_of(THPVariable_Unpack(args[0]));
+  if (dev < 0) Py_RETURN_NONE;
+  const Tensor *q = as_chunk(args[0], dev), *k = as_chunk(args[1], dev), *v = as_chunk(args[2], dev);
+  if (!q || !k || !v || k->sizes() != v->sizes() || k->sizes() != q->sizes()) Py_RETURN_NONE;
+  const int H = (int)q->size(2);
+  const int64_t S = q->size(1);
+  Window w;
+  if (!parse_window(args[3], dev, w)) {
+    if (PyErr_Occurred()) return nullptr;
+    Py_RETURN_NONE;
+  }
+  const int64_t keys = w.n_cached + S;
+  const float* tables[4];
+  for (int i = 0; i < 4; ++i) {
+    const Tensor* t = as_tensor(args[4 + i]);
+    if (!t || !on_device(*t, dev) || t->scalar_type() != at::kFloat || !t->is_contiguous() || t->numel() != (i < 2 ? keys : S) * 64 ||
+        !aligned16(t->data_ptr()))
+      Py_RETURN_NONE;
+    tables[i] = t->data_ptr<float>();
+  }
+  const float scale = (float)PyFloat_AsDouble(args[8]);
+  if (PyErr_Occurred()) return nullptr;
+  void* stream = stream_of(dev);
+  const Tensor wk = empty({keys, H, 128}, at::kBFloat16, dev), wv = empty({keys, H, 128}, at::kBFloat16, dev);
+  const Tensor rq = empty(q->sizes(), at::kBFloat16, dev), out = empty(q->sizes(), at::kBFloat16, dev);
+  if (failed(ll_kv_window_rope(q->data_ptr(), S, H, w.p[0], w.p[1], w.p[2], w.p[3], w.p[4], w.p[5], w.n_cached, w.bts, w.e2, w.e4,
+                               k->data_ptr(), v->data_ptr(), S, tables[0], tables[1], tables[2], tables[3], rq.data_ptr(), wk.data_ptr(),
+                               wv.data_ptr(), stream),
+             "ll_kv_window_rope"))
+    return nullptr;
+  if (failed(ll_kv_attention(rq.data_ptr(), S, H, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0, 6.f, 256.f, wk.data_ptr(),
+                             wv.data_ptr(), keys, scale, out.data_ptr(), stream),
+             "ll_kv_attention"))
+    return nullptr;
+  return THPVariable_Wrap(out);
+  END_HANDLE_TH_ERRORS
+}
+
+// cache_write(k, v, first token, tokens, rule, (values, scales, amax) of the K slot, of the V slot, k_sink, v_sink) -> True, or
+// None when it does not take the call.  The sinks: (parts, epoch) that the producers of k and v were given, or None for both.
+PyObject* py_cache_write(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 9 || !plain(args[0])) Py_RETURN_NONE;
+  const int dev = current_device_of(THPVariable_Unpack(args[0]));
+  if (dev < 0) Py_RETURN_NONE;
+  const Tensor *k = as_chunk(args[0], dev), *v = as_chunk(args[1], dev);
+  const int64_t first = PyLong_AsLongLong(args[2]), tokens = PyLong_AsLongLong(args[3]);
+  const int rule = (int)PyLong_AsLong(args[4]);
+  if (PyErr_Occurred()) return nullptr;
+  if (!k || !v || k->sizes() != v->sizes() || first < 0 || tokens <= 0 || first + tokens > k->size(1)) Py_RETURN_NONE;
+  const int64_t M = tokens * k->size(2), Mp = round_up(M, 128);
+  uint8_t* out[2][2];
+  float* amax[2];
+  for (int i = 0; i < 2; ++i) {
+    PyObject* t = args[5 + i];
+    if (!PyTuple_CheckExact(t) || PyTuple_GET_SIZE(t) != 3) Py_RETURN_NONE;
+    const Tensor *values = as_tensor(PyTuple_GET_ITEM(t, 0)), *scales = as_tensor(PyTuple_GET_ITEM(t, 1)), *a = as_tensor(PyTuple_GET_ITEM(t, 2));
+    if (!values || !scales || !a || !on_device(*values, dev) || !on_device(*scales, dev) || !on_device(*a, dev) ||
+        values->scalar_type() != at::kByte || values->dim() != 2 || values->size(0) != Mp || values->size(1) != 64 || scales->numel() != Mp * 8 ||
+        scales->element_size() != 1 || a->numel() != 1 || a->scalar_type() != at::kFloat || !values->is_contiguous() || !scales->is_contiguous())
+      Py_RETURN_NONE;
+    out[i][0] = values->data_ptr<uint8_t>();
+    out[i][1] = static_cast<uint8_t*>(scales->data_ptr());
+    amax[i] = a->data_ptr<float>();
+  }
+  if (out[0][0] == out[1][0] || out[0][1] == out[1][1] || amax[0] == amax[1]) Py_RETURN_NONE;
+  const int64_t at = first * k->size(2) * 128;
+  const uint16_t *kx = static_cast<const uint16_t*>(k->data_ptr()) + at, *vx = static_cast<const uint16_t*>(v->data_ptr()) + at;
+  void* stream = stream_of(dev);
+  int code;
+  if (args[7] != Py_None || args[8] != Py_None) {
+    ll_amax_sink sinks[2];
+    if (!parse_sink(args[7], dev, sinks[0]) || !parse_sink(args[8], dev, sinks[1]) || sinks[0].parts == sinks[1].parts) {
+      if (PyErr_Occurred()) return nullptr;
+      Py_RETURN_NONE;
+    }
+    code = ll_nvfp4_quantize_pair_from_sinks(kx, vx, M, 128, 128, rule, out[0][0], out[1][0], out[0][1], out[1][1], amax[0], amax[1], &sinks[0],
+                                             &sinks[1], stream);
+  } else {
+    const Tensor ws = empty({2 * (int64_t)LL_AMAX_PARTS}, at::kFloat, dev);
+    code = ll_nvfp4_quantize_pair(kx, vx, M, 128, 128, rule, out[0][0], out[1][0], out[0][1], out[1][1], amax[0], amax[1], ws.data_ptr<float>(),
+                                  stream);
+  }
+  if (failed(code, "cache write")) return nullptr;
+  Py_RETURN_TRUE;
+  END_HANDLE_TH_ERRORS
+}
+
 // current_stream() -> the current HIP stream of the current device as an integer
 PyObject* py_current_stream(PyObject*, PyObject*) {
   HANDLE_TH_ERRORS
@@ -521,6 +671,9 @@ PyObject* py_release_stream_sink(PyObject*, PyObject*) {
 
 PyMethodDef methods[] = {
     {"block_forward", (PyCFunction)(void (*)(void))py_block_forward, METH_FASTCALL, nullptr},
+    {"kv_attention", (PyCFunction)(void (*)(void))py_kv_attention, METH_FASTCALL, nullptr},
+    {"kv_attention_relative", (PyCFunction)(void (*)(void))py_kv_attention_relative, METH_FASTCALL, nullptr},
+    {"cache_write", (PyCFunction)(void (*)(void))py_cache_write, METH_FASTCALL, nullptr},
     {"current_stream", py_current_stream, METH_NOARGS, nullptr},
     {"release_stream_sink", py_release_stream_sink, METH_NOARGS, nullptr},
     {"quantize", (PyCFunction)(void (*)(void))py_quantize, METH_FASTCALL, nullptr},

@@ -102,6 +102,17 @@ __device__ __forceinline__ float e4m3_to_f32(uint32_t b) {
   return (b & 0x80u) ? -v : v;
 }
 
+typedef float float2v __attribute__((ext_vector_type(2)));
+// The eight e2m1 values of one packed dword, exact, in four conversions.
+__device__ __forceinline__ void fp4x8_values(uint32_t w, float (&q)[8]) {
+  const float2v p0 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w, 1.0f, 0);
+  const float2v p1 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w, 1.0f, 1);
+  const float2v p2 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w, 1.0f, 2);
+  const float2v p3 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w, 1.0f, 3);
+  q[0] = p0[0]; q[1] = p0[1]; q[2] = p1[0]; q[3] = p1[1];
+  q[4] = p2[0]; q[5] = p2[1]; q[6] = p3[0]; q[7] = p3[1];
+}
+
 // fp32 -> e4m3fn byte, round to nearest even, |x| > 464 -> NaN (0x7F): the value torch's
 // float8_e4m3fn cast produces.
 __device__ __forceinline__ uint32_t f32_to_e4m3(float x) {

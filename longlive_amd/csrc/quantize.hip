@@ -17,8 +17,14 @@ constexpr int kThreads = 256;
 // ----------------------------------------------------------------------------- amax
 // Each workgroup folds a grid-strided share of x into one partial maximum; the quantize kernel
 // reduces the kAmaxParts partials again, so no atomics and no zero-initialised state are needed.
-__global__ __launch_bounds__(kThreads) void amax_partial_kernel(const uint16_t* __restrict__ x, int64_t M, int64_t K,
-                                                                 int64_t ldx, float* __restrict__ parts) {
+// blockIdx.y selects one of the (at most two) tensors of the launch.
+struct AmaxJobs {
+  const uint16_t* x[2];
+  float* parts[2];
+};
+__global__ __launch_bounds__(kThreads) void amax_partial_kernel(AmaxJobs jobs, int64_t M, int64_t K, int64_t ldx) {
+  const uint16_t* __restrict__ x = blockIdx.y ? jobs.x[1] : jobs.x[0];
+  float* __restrict__ parts = blockIdx.y ? jobs.parts[1] : jobs.parts[0];
   float m = 0.0f;
   const int64_t tid = (int64_t)blockIdx.x * kThreads + threadIdx.x;
   const int64_t nthreads = (int64_t)gridDim.x * kThreads;
@@ -302,6 +308,7 @@ static int quantize_impl(const QuantRequest* req, int n, int64_t M, int64_t K, i
   LL_REQUIRE(total_tiles < (1ll << 31), "ll_nvfp4_quantize: tensor too large for one launch");
   hipStream_t s = static_cast<hipStream_t>(stream);
   QuantJobs jobs{};
+  AmaxJobs amax_jobs{};
   jobs.n = n;
   bool generic = (K % 64) != 0 || (ldx % 8) != 0;
   for (int i = 0; i < n; ++i) {
@@ -322,10 +329,13 @@ static int quantize_impl(const QuantRequest* req, int n, int64_t M, int64_t K, i
     j.sink_parts = r.sink ? reinterpret_cast<const unsigned long long*>(r.sink->parts) : nullptr;
     j.sink_epoch_base = r.sink ? r.sink->epoch : 0u;
     j.sink_epoch_offset = r.sink ? r.sink->epoch_offset : nullptr;
-    if (!amax_given && !r.sink) {
-      hipLaunchKernelGGL(amax_partial_kernel, dim3(kAmaxParts), dim3(kThreads), 0, s, j.x, M, K, ldx, r.workspace);
-      LL_CHECK_LAUNCH("amax_partial_kernel");
-    }
+    LL_REQUIRE(i == 0 || !r.sink == !req[0].sink, "ll_nvfp4_quantize: the tensors of a launch need one source of the amax");
+    amax_jobs.x[i] = j.x;
+    amax_jobs.parts[i] = r.workspace;
+  }
+  if (!amax_given && !req[0].sink) {
+    hipLaunchKernelGGL(amax_partial_kernel, dim3(kAmaxParts, n), dim3(kThreads), 0, s, amax_jobs, M, K, ldx);
+    LL_CHECK_LAUNCH("amax_partial_kernel");
   }
   // One workgroup per tile up to what the chip holds at once (the launch is persistent: every workgroup has to be
   // resident from the start, or the ones that wait would run after the others have finished).
@@ -391,6 +401,17 @@ extern "C" int ll_nvfp4_quantize_from_sink(const void* x, int64_t M, int64_t K, 
   LL_REQUIRE(amax_sink, "ll_nvfp4_quantize_from_sink: null amax sink");
   const QuantRequest r{x, values, scales, amax, nullptr, amax_sink};
   return quantize_impl(&r, 1, M, K, ldx, rule, 0, stream);
+}
+
+extern "C" int ll_nvfp4_quantize_pair(const void* x0, const void* x1, int64_t M, int64_t K, int64_t ldx, int rule, uint8_t* values0,
+                                      uint8_t* values1, uint8_t* scales0, uint8_t* scales1, float* amax0, float* amax1,
+                                      float* workspace, void* stream) {
+  using namespace ll;
+  LL_REQUIRE(workspace, "ll_nvfp4_quantize_pair: workspace required");
+  LL_REQUIRE(values0 != values1 && scales0 != scales1 && amax0 != amax1, "ll_nvfp4_quantize_pair: the two tensors need outputs of their own");
+  const QuantRequest r[2] = {{x0, values0, scales0, amax0, workspace, nullptr},
+                             {x1, values1, scales1, amax1, workspace + kAmaxParts, nullptr}};
+  return quantize_impl(r, 2, M, K, ldx, rule, 0, stream);
 }
 
 extern "C" int ll_nvfp4_quantize_pair_from_sinks(const void* x0, const void* x1, int64_t M, int64_t K, int64_t ldx,

@@ -139,8 +139,6 @@ struct ScaleEntry {
   float r, d1, d3, w;  // w = d1 * d1
 };
 
-typedef float float2v __attribute__((ext_vector_type(2)));
-
 // Codes of one candidate (scale entry e) and, for the rules that choose between candidates, a cheap
 // estimate of its error in units of the candidate's own step: sum (q - y)^2, sum |q - y| or max |q - y| with
 // y = x * r the scaled value the codes were rounded from.

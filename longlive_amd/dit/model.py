@@ -354,11 +354,7 @@ class DiTBlock(nn.Module):
         if not keys_only:
             if slot_ids is None:
                 return None
-            if slot_ids:
-                kt, vt = kvc._tables_for(kv_cache, slot_ids)
-                kv_rule, blk = kv_cache["k"][0].scale_rule, kv_cache["block_token_size"]
-                window = (kt.table, vt.table, len(slot_ids) * blk, blk, kv_rule.max_allowed_e2m1_value(),
-                          kv_rule.max_allowed_e4m3_value())
+            window = kvc._window(kv_cache, slot_ids)
         tickets = (None, None)
         if collect_kv_amax:
             tickets = tuple(sink.ticket() for sink in sa.amax_sinks(kv_cache, x.device))

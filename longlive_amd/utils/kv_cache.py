@@ -76,6 +76,15 @@ def _tables_for(cache: dict, slot_ids: tuple[int, ...]):
     return entry
 
 
+def _window(cache: dict, slot_ids):
+    """The attended slots as the native calls take them, None for none."""
+    if not slot_ids:
+        return None
+    kt, vt = _tables_for(cache, slot_ids)
+    rule, blk = cache["k"][0].scale_rule, cache["block_token_size"]
+    return kt.table, vt.table, len(slot_ids) * blk, blk, rule.max_allowed_e2m1_value(), rule.max_allowed_e4m3_value()
+
+
 def plan_cache_step(cache: dict, current_start: int, num_new_tokens: int, sink_tokens: int,
                     max_attention_size: int | None = None, global_sink_tokens: int = 0):
     """Host-side cache policy for one forward of one layer (wan_5b/modules/causal_model.py:491-674): which
@@ -194,8 +203,12 @@ def kv_cache_attention(q: torch.Tensor, key_to_cache: torch.Tensor, v: torch.Ten
     slot_ids, info, local_end = plan_cache_step(cache, current_start, S, sink_tokens, max_attention_size,
                                                 global_sink_tokens)
     info["new_k"], info["new_v"] = key_to_cache, v
-    k_new = (k_smooth(key_to_cache) if smoothed_key is None else smoothed_key)[0]
     scale = D ** -0.5 if softmax_scale is None else softmax_scale
+    if slot_ids is not None and amax_out is None and q.is_cuda:   # smoothing and attention as one native call
+        out = _native.host().kv_attention(q, key_to_cache, v, smoothed_key, _window(cache, slot_ids), float(scale))
+        if out is not None:
+            return out, (current_start + S, local_end, info)
+    k_new = (k_smooth(key_to_cache) if smoothed_key is None else smoothed_key)[0]
     rule = cache["k"][0].scale_rule
     if slot_ids is None:   # part of a slot is attended: bf16 rows of the window, then the plain attention kernel
         wk, wv = _materialize_pieces(cache, info["attended_pieces"], q.dtype, q.device)
@@ -231,9 +244,9 @@ def kv_cache_attention_relative(q: torch.Tensor, k: torch.Tensor, v: torch.Tenso
     frame positions 0, 1, ... of the window itself (sink first), the chunk's queries sitting on its last frames.
 
     q, k (RMS-normed, no RoPE), v: bf16 [1, S, H, 128]; ``rope_fn(frames, start_frame) -> (cos, sin)`` gives the
-    float32 tables of a (frames, h, w) grid.  As in the reference this path materialises the window: the attended
-    slots are dequantized to bf16 in one launch, concatenated with the smoothed chunk keys, rotated, and handed
-    to the plain bf16 attention kernel.  Returns the same tuple as ``kv_cache_attention``; ``new_k`` is the
+    float32 tables of a (frames, h, w) grid.  As in the reference this path materialises the window: one launch
+    dequantizes the attended slots to bf16, appends the smoothed chunk keys and rotates, and the plain bf16 attention
+    kernel reads the result.  Returns the same tuple as ``kv_cache_attention``; ``new_k`` is the
     un-rotated ``k``."""
     if q.shape[0] != 1:
         raise ValueError("the quantized KV cache holds one sequence (batch size 1)")
@@ -244,6 +257,13 @@ def kv_cache_attention_relative(q: torch.Tensor, k: torch.Tensor, v: torch.Tenso
     slot_ids, info, local_end = plan_cache_step(cache, current_start, S, sink_tokens, max_attention_size,
                                                 global_sink_tokens)
     info["new_k"], info["new_v"] = k, v
+    scale = D ** -0.5 if softmax_scale is None else softmax_scale
+    if slot_ids is not None and q.is_cuda:   # window, rotations and attention as one native call
+        frames, new_frames = (len(slot_ids) * cache["block_token_size"] + S) // frame_seqlen, S // frame_seqlen
+        out = _native.host().kv_attention_relative(q, k, v, _window(cache, slot_ids), *rope_fn(frames, 0),
+                                                   *rope_fn(new_frames, frames - new_frames), float(scale))
+        if out is not None:
+            return out, (current_start + S, local_end, info)
     keys, values = [k_smooth(k)[0]], [v[0]]
     if info["attended_pieces"]:
         wk, wv = _materialize_pieces(cache, info["attended_pieces"], q.dtype, q.device)
@@ -256,7 +276,6 @@ def kv_cache_attention_relative(q: torch.Tensor, k: torch.Tensor, v: torch.Tenso
     from .rope import rope_apply
     roped_k = rope_apply(window_k, *rope_fn(window_frames, 0))
     roped_q = rope_apply(q[0].contiguous(), *rope_fn(new_frames, window_frames - new_frames))
-    scale = D ** -0.5 if softmax_scale is None else softmax_scale
     out = _native.attention_bf16(roped_q, roped_k, window_v.contiguous(), scale)
     return out.unsqueeze(0), (current_start + S, local_end, info)
 
@@ -297,14 +316,16 @@ def apply_cache_update(cache: dict, current_end: int, local_end_index: int, info
         n_insert = (info["local_end_index"] - info["local_start_index"]) // blk
         rule = kv_quant_config.scale_rule.value
         for bi in range(n_insert):
-            blocks, slots, tickets = [], [], []
-            for name, new in (("k", info["new_k"]), ("v", info["new_v"])):
-                slots.append(cache[name][start_blk + bi])
-                blocks.append(new[0, bi * blk:(bi + 1) * blk].reshape(-1, new.shape[-1]))
-                # A chunk of one block is quantized as a whole: if its producer left the tensor maximum behind
-                # (an amax ticket of the layer's own sink), the quantization takes it from there.
-                tickets.append(info.get(f"new_{name}_amax") if n_insert == 1 and new.shape[1] == blk else None)
+            slots = [cache[name][start_blk + bi] for name in ("k", "v")]
             outs = [(slot.values, slot.scale_factors, slot.amax) for slot in slots]
+            # A chunk of one block is quantized as a whole: if its producer left the tensor maximum behind
+            # (an amax ticket of the layer's own sink), the quantization takes it from there.
+            news = [info["new_k"], info["new_v"]]
+            tickets = [info.get(f"new_{name}_amax") if n_insert == 1 and new.shape[1] == blk else None
+                       for name, new in zip(("k", "v"), news)]
+            if _native.cache_write(*news, bi * blk, blk, rule, *outs, *tickets):
+                continue
+            blocks = [new[0, bi * blk:(bi + 1) * blk].reshape(-1, new.shape[-1]) for new in news]
             if tickets[0] is not None and tickets[1] is not None and blocks[0].shape == blocks[1].shape:
                 _native.quantize_pair(blocks[0], blocks[1], rule, tickets[0], tickets[1], outs[0], outs[1])  # one launch
             else:

@@ -892,3 +892,34 @@ def test_roll_with_stable_slot_addresses_copies_like_the_reference(gpu):
         for a, b in zip(caches[0][n], caches[1][n]):
             assert torch.equal(a.values, b.values) and torch.equal(a.scale_factors.view(torch.uint8), b.scale_factors.view(torch.uint8))
             assert torch.equal(a.amax, b.amax)
+
+
+@pytest.mark.parametrize("relative", [False, True])
+@pytest.mark.parametrize("frames,h,w,H,cached,blocks", [(1, 1, 128, 1, 0, 1), (1, 23, 16, 8, 3, 1), (2, 7, 64, 3, 2, 2), (1, 5, 43, 2, 0, 1)])
+def test_native_cache_step_equals_the_separate_operations(gpu, relative, frames, h, w, H, cached, blocks):
+    """Smoothing, window and rotations in one launch and the K and V of a chunk quantized together give the bits of the
+    separate operations (which strided operands take): attention output and slots, for chunks of one and of two blocks,
+    behind none to three cached ones.  The values are multiples of 1/4, so that the mean of a head is the same sum in any
+    order."""
+    S = frames * h * w * blocks
+    g = torch.Generator().manual_seed(S + H)
+    draw = lambda: (torch.randint(-15, 16, (1, S, H, 128), generator=g) / 4).bfloat16().to(gpu)  # noqa: E731
+    chunks = [[draw() for _ in range(3)] for _ in range(cached // blocks + 1)]
+    angles = build_rope_angles(128)
+    rope_fn = lambda n, first: rope_cos_sin(angles, n, h, w, first, gpu)  # noqa: E731
+
+    def run(strided):
+        cache = kvc.initialize_kv_cache(1, S // blocks, cached + blocks, H, 128, CFG, gpu)[0]
+        for c, (q, k, v) in enumerate(chunks):
+            if strided:
+                q, k, v = (torch.stack([t, t], -1)[..., 0] for t in (q, k, v))
+                assert not q.is_contiguous()
+            if relative:
+                out, update = kvc.kv_cache_attention_relative(q, k, v, cache, c * S, 0, rope_fn)
+            else:
+                out, update = kvc.kv_cache_attention(q, k, v, cache, c * S, 0)
+            kvc.apply_cache_update(cache, *update, CFG)
+        return [out] + [t for n in "kv" for s in cache[n] for t in (s.values, s.scale_factors.view(torch.uint8), s.amax)]
+
+    for i, (a, b) in enumerate(zip(run(False), run(True))):
+        assert torch.equal(a, b), i

@@ -334,7 +334,8 @@ int ll_kv_attention_amax(const void* q, int64_t Lq, int num_heads,
  * How ll_kv_attention / ll_kv_attention_amax / ll_attention_bf16 divide a launch between workgroups.  No
  * counterpart in the reference (it calls flash attention).  LL_ATTENTION_AUTO, the initial setting, picks per
  * launch the cheapest of the three by a cost estimate:
- *   LL_ATTENTION_NARROW  one workgroup per (head, 128 queries);
+ *   LL_ATTENTION_NARROW  one workgroup per (head, 128 queries), or, for launches of a few hundred queries over a short
+ *                        key range, per (head, 32 queries) with the keys divided between its waves;
  *   LL_ATTENTION_WIDE    one workgroup per (head, 256 queries): every decoded K/V tile serves twice as many MFMAs;
  *   LL_ATTENTION_SPLIT   256-query tiles; what does not fill whole rounds of one tile per compute unit is cut
  *                        along the key range into shares of equal cost (a head's last, partly filled group of
@@ -342,7 +343,7 @@ int ll_kv_attention_amax(const void* q, int64_t Lq, int num_heads,
  *                        workgroups pass through device memory that the library allocates on the first such
  *                        launch on a (device, stream) pair and keeps (69 MB on a 256-CU device); launches that
  *                        use it must not overlap on one stream's memory, which same-stream order guarantees.
- * The three give the same result up to the order of fp32 additions (each is deterministic).  The setting is
+ * All give the same result up to the order of fp32 additions (each is deterministic).  The setting is
  * process-wide.  A launch on a stream that is being captured into a graph never allocates: it uses the memory an
  * earlier launch or ll_kv_attention_reserve left on that stream, and without such memory the automatic choice
  * takes the cheaper of NARROW and WIDE while an explicit LL_ATTENTION_SPLIT returns LL_ENOSUP.

@@ -781,9 +781,277 @@ __global__ __launch_bounds__(kAttnThreads) void kv_attention_kernel(AttnParams p
   }  // segments
 }
 
+// ----------------------------------------------------------------------------- short launches
+// One head x 32 queries per workgroup, its keys dealt to W waves in tiles of 32 (wave w takes tiles w, w + W, ...).
+// A launch of a few hundred queries gives the kernel above a few dozen tiles of 128 or 256 queries: most compute units
+// idle, and every wave walks the whole key range or leaves 135 KB of partial results in device memory.  Here each wave
+// has LDS rows, registers and a softmax of its own, nothing but the merge at the end needs a barrier, and the longest
+// chain is (keys / 32 / W) tiles.  What it costs is the conversion of every K and V row once per 32 instead of
+// 128 or 256 queries: short_kernel_waves (attention_split.h) says up to where that pays.
+//
+// The contraction over the head dimension may run in any order as long as Q and K agree: step ks of lane half lh
+// covers elements 64 lh + 8 ks .. + 7, so the K operand of a cached row comes straight out of 32 packed bytes and four
+// scale bytes of the lane's own, without LDS.  Rows of the chunk (bf16) are loaded four whole rows per instruction
+// and pass through LDS, as V always does (its operand needs the transposing read).
+//
+// Bound by vector instructions (per tile 16 MFMAs beside about 480 others where the keys are cached, 150 where not) and,
+// for the chunk's rows, by the 64 B per clock a CU takes from its L1.  368 queries x 16 heads over 1472 bf16 keys 16.9 us
+// (36.8 in the 256-query kernel), 192 x 12 over 768 cached + 192 keys 15.5 (27.3), 64 x 2 over 128 keys 5.6 (8.0).
+constexpr int kShortKeys = 32;                                                // keys per wave tile
+constexpr int kShortWaveBytes = kShortKeys * (kKPitch + kVPitch);             // a wave's K and V rows
+constexpr int kShortRecord = 66 * 64;                                         // floats of a wave's result in the merge
+template <int W>
+constexpr size_t kShortLds = (size_t)W * kShortWaveBytes + sizeof(SlotTable);
+static_assert(kShortRecord * 4 <= kShortWaveBytes, "the merge reuses the waves' rows");
+
+// amdgpu_waves_per_eu: 256 registers per lane, two waves per SIMD (one workgroup of eight or two of four per CU)
+template <int W>
+__global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void kv_attention_short_kernel(AttnParams p) {
+  static_assert(W == 4 || W == 8, "the merge gives every wave 64 / W of the 64 output registers");
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  SlotTable& tab = *reinterpret_cast<SlotTable*>(smem + W * kShortWaveBytes);
+  if (const int t = threadIdx.x; t < p.n_slots) {
+    tab.kv[t] = reinterpret_cast<const uint8_t*>(p.kv_ptrs[t]);
+    tab.ks[t] = reinterpret_cast<const uint8_t*>(p.ks_ptrs[t]);
+    tab.vv[t] = reinterpret_cast<const uint8_t*>(p.vv_ptrs[t]);
+    tab.vs[t] = reinterpret_cast<const uint8_t*>(p.vs_ptrs[t]);
+    tab.kg[t] = load_global<float>(reinterpret_cast<const void*>(p.ka_ptrs[t])) * p.inv_denom;
+    tab.vg[t] = load_global<float>(reinterpret_cast<const void*>(p.va_ptrs[t])) * p.inv_denom;
+  }
+  const uint32_t tile_id = group_number(p.d.G);
+  const int head = (int)(tile_id / (uint32_t)p.n_qtiles), qtile = (int)(tile_id - (uint32_t)head * (uint32_t)p.n_qtiles);
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l32 = lane & 31, lh = lane >> 5;
+  const int n_cached = (int)p.n_cached, n_new = (int)p.n_new;
+  const int cached_tiles = (n_cached + kShortKeys - 1) / kShortKeys, n_tiles = cached_tiles + (n_new + kShortKeys - 1) / kShortKeys;
+  uint8_t* const krows = smem + wave * kShortWaveBytes;
+  uint8_t* const vrows = krows + kShortKeys * kKPitch;
+
+  const int64_t query = (int64_t)qtile * kWaveQueries + l32;
+  bf16x8 qf[8];
+  {
+    const uint16_t* src = p.q + ((query < p.Lq ? query : p.Lq - 1) * p.H + head) * kHeadDim + 64 * lh;
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks) qf[ks] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(src + 8 * ks));
+  }
+  __syncthreads();  // the slot table
+
+  float16v o[4];
+#pragma unroll
+  for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) o[dt][i] = 0.0f;
+  float m_run = -INFINITY, l_run = 0.0f;
+  constexpr float kRescaleStep = 8.0f;  // as in the kernel above: the reference point follows the maximum in steps
+
+  // Softmax of the wave's 32 scores per query (register r of sc: key 8 (r / 4) + 4 lh + r % 4 of the tile, `valid` keys
+  // exist) and O^T += V^T P^T from the V rows in LDS.
+  auto softmax_pv = [&](float16v& sc, int valid) __attribute__((always_inline)) {
+    typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(3))) bf16x4* lds_bf16x4_t;
+    const uint8_t* vt_lane = vrows + (4 * lh + ((lane & 15) >> 2)) * kVPitch + (16 * ((lane >> 4) & 1) + 4 * (lane & 3)) * 2;
+    bf16x4 vfr[2][4][2];
+    auto read_v = [&](int step) __attribute__((always_inline)) {
+#pragma unroll
+      for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          vfr[step][dt][j] = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4_t)(vt_lane + (16 * step + 8 * j) * kVPitch + dt * 64));
+    };
+    read_v(0);
+    if (valid < kShortKeys) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        if (8 * (r >> 2) + 4 * lh + (r & 3) >= valid) sc[r] = -INFINITY;
+    }
+    float mx = sc[0];
+#pragma unroll
+    for (int r = 1; r < 16; ++r) mx = fmaxf(mx, sc[r]);
+    mx = max_over_wave_halves(mx);
+    const bool raise = (mx - m_run) * p.scale_log2 > kRescaleStep;
+    const float m_new = raise ? mx : m_run;
+    if (__builtin_amdgcn_ballot_w64(raise) != 0) {
+      const float alpha = raise ? __builtin_amdgcn_exp2f((m_run - m_new) * p.scale_log2) : 1.0f;
+      l_run *= alpha;
+#pragma unroll
+      for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[dt][i] *= alpha;
+    }
+    m_run = m_new;
+    const float neg = -m_new * p.scale_log2;
+    read_v(1);
+#pragma unroll
+    for (int step = 0; step < 2; ++step) {
+      uint32_t w[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float p0 = __builtin_amdgcn_exp2f(fmaf(sc[8 * step + 2 * i], p.scale_log2, neg));
+        const float p1 = __builtin_amdgcn_exp2f(fmaf(sc[8 * step + 2 * i + 1], p.scale_log2, neg));
+        l_run += p0 + p1;
+        w[i] = pack_bf16(p0, p1);
+      }
+      const bf16x8 pb = __builtin_bit_cast(bf16x8, make_uint4(w[0], w[1], w[2], w[3]));
+#pragma unroll
+      for (int dt = 0; dt < 4; ++dt) {
+        const bf16x8 a = __builtin_shufflevector(vfr[step][dt][0], vfr[step][dt][1], 0, 1, 2, 3, 4, 5, 6, 7);
+        o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, pb, o[dt], 0, 0, 0);
+      }
+    }
+    // the next tile's rows are written behind these reads: LDS accesses of one wave are carried out in order
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  };
+  auto rows_written = [&]() __attribute__((always_inline)) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  };
+
+  // ---- cached keys: lane = (key l32, half lh of the head dimension) for K and V alike
+  int t = wave;
+  {
+    struct { uint4 v[2]; uint32_t scales; } kf, vf;
+    float kg = 0.0f, vg = 0.0f;
+    auto fetch = [&](int tile) __attribute__((always_inline)) {
+      const uint32_t key = (uint32_t)min(tile * kShortKeys + l32, n_cached - 1);
+      const uint32_t slot = key / (uint32_t)p.bts;
+      const int64_t row = (int64_t)(key - slot * (uint32_t)p.bts) * p.H + head;
+      const uint32_t vo = (uint32_t)row * 64u + lh * 32u, so = (uint32_t)blocked_scale_offset(row, lh * 4, 8);
+      kf.v[0] = load_global_b128(tab.kv[slot] + vo);
+      kf.v[1] = load_global_b128(tab.kv[slot] + vo + 16);
+      kf.scales = load_global<uint32_t>(tab.ks[slot] + so);
+      vf.v[0] = load_global_b128(tab.vv[slot] + vo);
+      vf.v[1] = load_global_b128(tab.vv[slot] + vo + 16);
+      vf.scales = load_global<uint32_t>(tab.vs[slot] + so);
+      kg = tab.kg[slot];
+      vg = tab.vg[slot];
+    };
+    if (t < cached_tiles) fetch(t);
+    for (; t < cached_tiles; t += W) {
+      const int valid = n_cached - t * kShortKeys;
+      float16v sc;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) sc[i] = 0.0f;
+      const uint32_t wk[8] = {kf.v[0].x, kf.v[0].y, kf.v[0].z, kf.v[0].w, kf.v[1].x, kf.v[1].y, kf.v[1].z, kf.v[1].w};
+      const bool live = l32 < valid;  // rows of keys that do not exist are zeros
+      uint32_t wv[8] = {vf.v[0].x, vf.v[0].y, vf.v[0].z, vf.v[0].w, vf.v[1].x, vf.v[1].y, vf.v[1].z, vf.v[1].w};
+#pragma unroll
+      for (int j = 0; j < 8; ++j) wv[j] = live ? wv[j] : 0u;
+      half2v ks2[4], vs2[4];
+      block_scales_f16(kf.scales, *reinterpret_cast<half2v(*)[2]>(&ks2[0]));
+      block_scales_f16(kf.scales >> 16, *reinterpret_cast<half2v(*)[2]>(&ks2[2]));
+      const uint32_t vsc = live ? vf.scales : 0u;
+      block_scales_f16(vsc, *reinterpret_cast<half2v(*)[2]>(&vs2[0]));
+      block_scales_f16(vsc >> 16, *reinterpret_cast<half2v(*)[2]>(&vs2[2]));
+      const float kgt = kg, vgt = live ? vg : 0.0f;
+      if (t + W < cached_tiles) fetch(t + W);
+      uint4* vdst = reinterpret_cast<uint4*>(vrows + l32 * kVPitch + lh * 128);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        float v8[8];
+        fp4x8_to_f32(wk[j], ks2[j >> 1], kgt, v8);
+        const bf16x8 fa = __builtin_bit_cast(bf16x8, make_uint4(pack_bf16(v8[0], v8[1]), pack_bf16(v8[2], v8[3]),
+                                                                pack_bf16(v8[4], v8[5]), pack_bf16(v8[6], v8[7])));
+        sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa, qf[j], sc, 0, 0, 0);
+        fp4x8_to_f32(wv[j], vs2[j >> 1], vgt, v8);
+        vdst[j] = make_uint4(pack_bf16(v8[0], v8[1]), pack_bf16(v8[2], v8[3]), pack_bf16(v8[4], v8[5]), pack_bf16(v8[6], v8[7]));
+      }
+      rows_written();
+      softmax_pv(sc, valid);
+    }
+  }
+  // ---- the chunk's own keys: piece j of a tile is rows 4 j + lane / 16, 16 bytes per lane
+  if (t < n_tiles) {
+    uint4 kb[8], vb[8];
+    const int64_t row_step = (int64_t)p.H * kHeadDim;
+    auto fetch = [&](int tile, const uint16_t* src, uint4 (&dst)[8]) __attribute__((always_inline)) {
+      const int key0 = (tile - cached_tiles) * kShortKeys + (lane >> 4);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int key = key0 + 4 * j;
+        dst[j] = make_uint4(0u, 0u, 0u, 0u);
+        if (key < n_new) dst[j] = load_global_b128(src + key * row_step + head * kHeadDim + (lane & 15) * 8);
+      }
+    };
+    fetch(t, p.k_new, kb);
+    fetch(t, p.v_new, vb);
+    for (; t < n_tiles; t += W) {
+      const int valid = n_new - (t - cached_tiles) * kShortKeys;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        *reinterpret_cast<uint4*>(krows + (4 * j + (lane >> 4)) * kKPitch + (lane & 15) * 16) = kb[j];
+        *reinterpret_cast<uint4*>(vrows + (4 * j + (lane >> 4)) * kVPitch + (lane & 15) * 16) = vb[j];
+      }
+      rows_written();
+      if (t + W < n_tiles) {
+        fetch(t + W, p.k_new, kb);
+        fetch(t + W, p.v_new, vb);
+      }
+      float16v sc;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) sc[i] = 0.0f;
+      const uint8_t* krow = krows + l32 * kKPitch + lh * 128;
+#pragma unroll
+      for (int ks = 0; ks < 8; ++ks)
+        sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(krow + 16 * ks)), qf[ks], sc, 0, 0, 0);
+      softmax_pv(sc, valid);
+    }
+  }
+
+  // ---- merge: every wave leaves (O^T, reference point, row sum) in LDS, wave w combines registers 64 w / W .. of all
+  l_run += __shfl_xor(l_run, 32, 64);
+  __syncthreads();  // all waves are through with their rows
+  float* const records = reinterpret_cast<float*>(smem);
+  {
+    float* mine = records + wave * kShortRecord + lane;
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) mine[(dt * 16 + i) * 64] = o[dt][i];
+    mine[64 * 64] = m_run;
+    mine[65 * 64] = l_run;
+  }
+  __syncthreads();
+  float a[W], m = -INFINITY, l = 0.0f;
+#pragma unroll
+  for (int w = 0; w < W; ++w) {
+    a[w] = records[w * kShortRecord + 64 * 64 + lane];
+    m = fmaxf(m, a[w]);
+  }
+#pragma unroll
+  for (int w = 0; w < W; ++w) {
+    a[w] = a[w] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((a[w] - m) * p.scale_log2);  // a wave without a tile: -inf
+    l += a[w] * records[w * kShortRecord + 65 * 64 + lane];
+  }
+  const float inv_l = 1.0f / l;
+  float out_max = 0.0f;
+#pragma unroll
+  for (int g = 0; g < 16 / W; ++g) {
+    const int reg = wave * (64 / W) + 4 * g;  // four registers = four neighbouring elements of the head dimension
+    float v[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      v[i] = 0.0f;
+#pragma unroll
+      for (int w = 0; w < W; ++w) v[i] += a[w] * records[w * kShortRecord + (reg + i) * 64 + lane];
+      v[i] *= inv_l;
+    }
+    if (query < p.Lq) {
+      const uint2 packed = make_uint2(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]));
+      const int d = 32 * (reg >> 4) + 8 * ((reg & 15) >> 2) + 4 * lh;
+      *reinterpret_cast<uint2*>(p.out + (query * p.H + head) * kHeadDim + d) = packed;
+      out_max = abs_max_bf16x8(make_uint4(packed.x, packed.y, 0u, 0u), out_max);
+    }
+  }
+  if (p.sink.parts) {
+    out_max = wave_max(out_max);
+    if (lane == 0) amax_sink_update(p.sink, tile_id * W + wave, out_max);
+  }
+}
+
 static std::atomic<int> g_attention_policy{LL_ATTENTION_AUTO};
 
-// Three ways to run a launch, all one workgroup per compute unit at a time (LDS):
+// Short launches take kv_attention_short_kernel, under the automatic choice and where the division without shared tiles and
+// with few queries per workgroup (LL_ATTENTION_NARROW) is asked for.  For the others there are three ways, all one workgroup per compute unit at a time (LDS):
 //  * 128 queries per workgroup, the key range halved between two sets of waves; one workgroup per tile;
 //  * 256 queries per workgroup (every decoded K/V tile serves twice as many MFMAs: an iteration takes about 1.64
 //    times as long for twice the work), one workgroup per tile;
@@ -803,6 +1071,21 @@ static int launch_attention(const AttnParams& p_in, hipStream_t stream) {
   const int64_t n_iter = (p.n_cached + p.n_new + kIterKeys - 1) / kIterKeys;
   LL_REQUIRE(p.H * ((p.Lq + kWgQueries - 1) / kWgQueries) * n_iter < (1ll << 32), "ll_kv_attention: too many (tile, iteration) units");
   const int policy = g_attention_policy.load(std::memory_order_relaxed);
+  if (const int waves = policy <= LL_ATTENTION_NARROW ? short_kernel_waves(p.Lq, p.H, p.n_cached, p.n_new, cus) : 0) {
+    p.n_qtiles = (int)((p.Lq + kWaveQueries - 1) / kWaveQueries);
+    p.d.G = (uint32_t)(p.H * p.n_qtiles);
+    static std::atomic<uint64_t> lds_allowed4{0}, lds_allowed8{0};
+    const void* kernel = waves == 8 ? reinterpret_cast<const void*>(&kv_attention_short_kernel<8>) : reinterpret_cast<const void*>(&kv_attention_short_kernel<4>);
+    const size_t lds = waves == 8 ? kShortLds<8> : kShortLds<4>;
+    if (int rc = allow_dynamic_lds(kernel, lds, waves == 8 ? lds_allowed8 : lds_allowed4, "ll_kv_attention")) return rc;
+    if (waves == 8) {
+      hipLaunchKernelGGL(kv_attention_short_kernel<8>, dim3(p.d.G), dim3(512), lds, stream, p);
+    } else {
+      hipLaunchKernelGGL(kv_attention_short_kernel<4>, dim3(p.d.G), dim3(256), lds, stream, p);
+    }
+    LL_CHECK_LAUNCH("kv_attention_short_kernel");
+    return LL_OK;
+  }
   AttentionPlan plan = plan_attention(p.Lq, p.H, p.n_cached + p.n_new, cus, policy);
   StreamScratch w;
   if (plan.mode == LL_ATTENTION_SPLIT) {
@@ -863,7 +1146,11 @@ extern "C" int ll_kv_attention_reserve(int64_t Lq, int num_heads, int64_t n_keys
     return LL_ELAUNCH;
   }
   if (int rc = compute_units_of(dev, cus, "ll_kv_attention")) return rc;
-  const AttentionPlan plan = plan_attention(Lq, num_heads, n_keys, cus, g_attention_policy.load(std::memory_order_relaxed));
+  const int policy = g_attention_policy.load(std::memory_order_relaxed);
+  const AttentionPlan plan = plan_attention(Lq, num_heads, n_keys, cus, policy);
+  // (what is cached and what is the chunk's own decides between the short kernel and the tiles: only a launch that takes
+  // the short kernel either way needs no memory; + 32: a window of both has a partly filled tile more)
+  if (policy <= LL_ATTENTION_NARROW && short_kernel_waves(Lq, num_heads, n_keys + 32, 0, cus)) return LL_OK;
   if (plan.mode != LL_ATTENTION_SPLIT) return LL_OK;
   if (stream_is_capturing(static_cast<hipStream_t>(stream))) {
     set_error("ll_kv_attention_reserve: the stream is being captured; reserve before the recording starts");
@@ -881,6 +1168,13 @@ extern "C" int ll_kv_attention_plan(int64_t Lq, int num_heads, int64_t n_keys, i
   LL_REQUIRE(Lq > 0 && num_heads > 0 && n_keys > 0 && compute_units > 0 && Lq < (1ll << 30) && n_keys < (1ll << 30),
              "ll_kv_attention_plan: bad sizes");
   LL_REQUIRE(policy >= LL_ATTENTION_AUTO && policy <= LL_ATTENTION_SPLIT, "ll_kv_attention_plan: unknown policy %d", policy);
+  if (policy <= LL_ATTENTION_NARROW && ll::short_kernel_waves(Lq, num_heads, n_keys + 32, 0, compute_units)) {
+    if (division) *division = LL_ATTENTION_NARROW;
+    if (workgroups) *workgroups = (uint32_t)(num_heads * ((Lq + 31) / 32));
+    if (whole_rounds) *whole_rounds = 1;
+    if (split_tiles) *split_tiles = 0;
+    return LL_OK;
+  }
   const ll::AttentionPlan plan = ll::plan_attention(Lq, num_heads, n_keys, compute_units, policy);
   if (division) *division = plan.mode;
   if (workgroups) *workgroups = plan.d.G;

@@ -103,6 +103,26 @@ LL_SPLIT_FN uint32_t record_of_part(uint32_t g, uint32_t split_tile, const Divis
   return 2 * g + (first_tile == split_tile ? 0u : 1u);
 }
 
+// ---- short launches (host): waves per workgroup with which kv_attention_short_kernel takes a launch, 0 for the tile
+// kernels.  It converts K and V once per 32 queries and fills a compute unit with one workgroup of eight or two of
+// four waves, so it is ahead while everything runs at once and the key range is short (us, tile kernels / 8 waves /
+// 4 waves; "a + b" = cached + chunk keys in tiles of 32):
+//   G <= CUs      368 queries x 16 heads, 0 + 46 tiles 36.8 / 16.9 / 20.3; 512 x 16, 64 + 16: 36.9 / 28.8 / 31.2;
+//                 1024 x 6, 64 + 32: 42.5 / 32.9 / 36.5, but 128 + 32: 48.5 / 50.1 / 57.7 (the divided tiles use all units)
+//   up to 12 tiles four waves have two or three tiles each and half the merge: 64 x 12, 0 + 4: 8.4 / 6.7 / 5.8
+//   G <= 2 CUs    736 x 12, 0 + 16: 16.3 / 18.4 / 13.7; 512 x 24, 32 + 16: 34.7 / 38.3 / 32.8, but 46 + 23 on 736 x 12:
+//                 38.7 / 49.9 / 43.5;   G > 2 CUs: 736 x 24, 0 + 16: 16.8 / 26.4 / 20.5
+// A cached tile costs about half as much again as one of the chunk (conversion).  Launches of more than 256 queries per
+// head for every head (700 queries of 2 heads: 27.8 / 12.9) stay with the divided tiles: programs that reserve their memory
+// ahead of a recording count on that division and its bits.
+inline int short_kernel_waves(int64_t Lq, int H, int64_t n_cached, int64_t n_new, int cus) {
+  const int64_t groups = H * ((Lq + 31) / 32), cached = (n_cached + 31) / 32, fresh = (n_new + 31) / 32;
+  const int64_t length = cached + cached / 2 + fresh;
+  if (Lq > 256 * (int64_t)H) return 0;
+  if (groups <= cus) return length > 176 ? 0 : (cached + fresh <= 12 ? 4 : 8);
+  return groups <= 2 * (int64_t)cus && length <= 64 ? 4 : 0;
+}
+
 // ---- the launcher's choice (host).  Costs are in iterations of the 128-query kernel; whole rounds of workgroups
 // count in full.
 struct AttentionPlan {

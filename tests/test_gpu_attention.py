@@ -923,3 +923,44 @@ def test_native_cache_step_equals_the_separate_operations(gpu, relative, frames,
 
     for i, (a, b) in enumerate(zip(run(False), run(True))):
         assert torch.equal(a, b), i
+
+
+@pytest.mark.parametrize("Lq,H,T,cached,n_new", [
+    (1, 1, 0, 0, 1),            # one query, one key: seven or three waves without a tile
+    (64, 2, 0, 0, 128),         # four waves, four tiles
+    (33, 4, 32, 33, 3),         # a ragged tile of either kind; keys of one tile in two slots
+    (70, 8, 48, 140, 0),        # nothing but cached keys, slots that end inside tiles
+    (368, 16, 0, 0, 417),       # eight waves, 14 tiles
+    (100, 4, 96, 257, 64),      # eight waves, cached and chunk
+    (512, 16, 512, 2048, 512),  # as many workgroups as compute units, the longest range
+    (520, 24, 0, 0, 1030),      # two workgroups of four waves per compute unit
+])
+def test_short_launches_against_fp64(gpu, Lq, H, T, cached, n_new):
+    """The kernel with 32 queries per workgroup, over the edges of its tiles and of its rule, twice for
+    identical bits, its amax sink included.  Bound: bf16 probabilities and a bf16 result, 2^-9 relative each, with
+    sum p |v| <= max |v|, and as much again for the fp32 sums and scores."""
+    q, k, v = (_randn((n, H, 128), s).to(gpu) for n, s in ((Lq, 31), (max(n_new, 1), 32), (max(n_new, 1), 33)))
+    slots, tables, K, V = -(-cached // T) if cached else 0, None, [], []
+    if cached:
+        cache = kvc.initialize_kv_cache(1, T, slots, H, 128, CFG, gpu)[0]
+        for c in range(slots):
+            kv = [_randn((1, T, H, 128), 40 + 2 * c + i).to(gpu) for i in range(2)]
+            end, local_end, info = kvc.kv_cache_update_only(*kv, cache, c * T, T)
+            kvc.apply_cache_update(cache, end, local_end, info, CFG)
+        kt, vt = kvc._tables_for(cache, tuple(range(slots)))
+        tables = (kt.values, kt.scales, kt.amax, vt.values, vt.scales, vt.amax)
+        for rows, name in ((K, "k"), (V, "v")):
+            rows.append(dequantize_kv_cache(cache[name][:slots], slots, H, T, torch.bfloat16, gpu)[0][:cached])
+    new = (k[:n_new], v[:n_new]) if n_new else (None, None)
+    if n_new:
+        K.append(k), V.append(v)
+    outs = []
+    for _ in range(2):
+        ticket = _native.amax_ticket(gpu)
+        outs.append(_native.kv_attention(q, tables, cached, T, 6.0, 256.0, *new, 128 ** -0.5, amax_out=ticket))
+        xq = quantize_to_fp4(outs[-1].flatten(1), CFG, amax=ticket)
+        assert float(xq.amax) == float(outs[-1].float().abs().max())
+    assert torch.equal(*outs)
+    K, V = torch.cat(K).double(), torch.cat(V).double()
+    ref = torch.stack([torch.softmax(q[:, h].double() @ K[:, h].T.contiguous() * 128 ** -0.5, -1) @ V[:, h] for h in range(H)], 1)
+    assert (outs[0].double() - ref).abs().max().item() <= 2 ** -7 * V.abs().max().item()

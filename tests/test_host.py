@@ -291,6 +291,17 @@ def test_attention_plan_for_the_benchmark_shapes():
         plan(0, 24, 100)
 
 
+@pytest.mark.parametrize("Lq,H,keys,short", [(192, 2, 960, True), (512, 16, 3200, True), (512, 16, 13200, False),
+                                            (1500, 24, 512, False), (700, 2, 900, False), (520, 24, 1300, True)])
+def test_short_launches_take_32_queries_per_workgroup(Lq, H, keys, short):
+    auto, narrow = (_native.attention_plan(Lq, H, keys, policy=p) for p in ("auto", "narrow"))
+    if short:
+        assert auto == narrow == {"division": "narrow", "workgroups": H * -(-Lq // 32), "whole_rounds": 1, "split_tiles": 0}
+    else:
+        assert auto["division"] != "narrow" and narrow["workgroups"] == H * -(-Lq // 128)
+    assert _native.attention_plan(Lq, H, keys, policy="wide")["division"] == "wide"
+
+
 def _check_division(plan, tiles):
     """Every (tile, iteration) in exactly one segment; whole tiles first; the parts of a split tile held by exactly
     the workgroups parts_of_tile names, one part each, in records no two parts share; at most two partial tiles

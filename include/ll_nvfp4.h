@@ -469,6 +469,23 @@ int ll_qk_norm_rope_pair_amax(const void* q, const void* k, int64_t rows, int nu
                               void* q_out, void* k_out, void* k_out_smooth, const ll_amax_sink* k_amax_sink,
                               void* stream);
 
+/* One step of the flow-matching UniPC sampler, order 1 or 2 (wan_5b/utils/fm_solvers_unipc.py:281-350, 352-486, 488-628,
+ * 657-741), as one pass over bf16 tensors of n elements: x0 prediction from the flow, corrector for the step just taken,
+ * predictor for the next one.  Every product, difference and sum is rounded to bf16, as the tensor expressions of the
+ * reference round it.  The scalars are those expressions' fp32 scalars:
+ *   converted = sample - sigma * flow
+ *   corrected = ratio * last - m0 * m1 - b * (rho * ((m2 - m1) / rk) + rho_new * (converted - m1))     [corrector]
+ *   next      = ratio * corrected - m0 * converted - b * (rho * ((m1 - converted) / rk))               [predictor]
+ * order 0 leaves the corrector out (corrected = sample; `corrected` and `last` are not touched), order 1 the rho term.
+ * m1 / m2: the newest and second newest x0 predictions of earlier steps; what no term reads may be NULL. */
+typedef struct ll_unipc_scalars {
+  int order;
+  float ratio, m0, b, rho, rk, rho_new;
+} ll_unipc_scalars;
+int ll_unipc_step(const void* flow, const void* sample, const void* last, const void* m1, const void* m2, int64_t n, float sigma,
+                  const ll_unipc_scalars* corrector, const ll_unipc_scalars* predictor, void* converted, void* corrected, void* next,
+                  void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -15,8 +15,13 @@
 #include <ATen/hip/EmptyTensor.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
+#include <ATen/PythonTorchFunctionTLS.h>
+#include <c10/core/GradMode.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/autograd/variable.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 
 #include <map>
 #include <mutex>
@@ -652,6 +657,49 @@ PyObject* py_cache_write(PyObject*, PyObject* const* args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// unipc_step(flow, sample, last or None, m1 or None, m2 or None, sigma, corrector, predictor) -> (x0 prediction, corrected
+// sample, next sample), or None when it does not take the call.  corrector, predictor: (order, ratio, m0, b, rho, rk,
+// rho_new), see ll_unipc_scalars; with a corrector of order 0 the corrected sample is `sample` itself.
+PyObject* py_unipc_step(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 8 || c10::impl::TorchDispatchModeTLS::any_modes_set() || at::impl::torch_function_mode_enabled() || torch::jit::tracer::isTracing())
+    Py_RETURN_NONE;
+  const Tensor* in[5] = {};
+  int dev = -1;
+  for (int i = 0; i < 5; ++i) {
+    if (i > 1 && args[i] == Py_None) continue;
+    if (!plain(args[i])) Py_RETURN_NONE;
+    const Tensor& t = THPVariable_Unpack(args[i]);
+    // batched and functional wrappers have no storage; gradients of either mode need torch's own operations
+    if (!t.has_storage() || (t.requires_grad() && c10::GradMode::is_enabled()) ||
+        (torch::autograd::impl::get_autograd_meta(t) && t._fw_grad(0).defined()))
+      Py_RETURN_NONE;
+    if (i == 0) dev = current_device_of(t);
+    if (!is_bf16(t, dev) || !t.is_contiguous() || t.numel() == 0 || (i > 0 && t.sizes() != in[0]->sizes())) Py_RETURN_NONE;
+    in[i] = &t;
+  }
+  const double sigma = PyFloat_AsDouble(args[5]);
+  ll_unipc_scalars s[2];
+  for (int i = 0; i < 2; ++i) {
+    PyObject* t = args[6 + i];
+    if (!PyTuple_CheckExact(t) || PyTuple_GET_SIZE(t) != 7) Py_RETURN_NONE;
+    s[i].order = (int)PyLong_AsLong(PyTuple_GET_ITEM(t, 0));
+    float* const f[6] = {&s[i].ratio, &s[i].m0, &s[i].b, &s[i].rho, &s[i].rk, &s[i].rho_new};
+    for (int j = 0; j < 6; ++j) *f[j] = (float)PyFloat_AsDouble(PyTuple_GET_ITEM(t, 1 + j));
+  }
+  if (PyErr_Occurred()) return nullptr;
+  const bool correct = s[0].order > 0;
+  const Tensor converted = empty(in[0]->sizes(), at::kBFloat16, dev), next = empty(in[0]->sizes(), at::kBFloat16, dev);
+  const Tensor corrected = correct ? empty(in[0]->sizes(), at::kBFloat16, dev) : *in[1];
+  const auto ptr = [&](int i) -> const void* { return in[i] ? in[i]->data_ptr() : nullptr; };
+  if (failed(ll_unipc_step(ptr(0), ptr(1), ptr(2), ptr(3), ptr(4), in[0]->numel(), (float)sigma, &s[0], &s[1], converted.data_ptr(),
+                           correct ? corrected.data_ptr() : nullptr, next.data_ptr(), stream_of(dev)),
+             "ll_unipc_step"))
+    return nullptr;
+  return tuple3(converted, corrected, next);
+  END_HANDLE_TH_ERRORS
+}
+
 // current_stream() -> the current HIP stream of the current device as an integer
 PyObject* py_current_stream(PyObject*, PyObject*) {
   HANDLE_TH_ERRORS
@@ -674,6 +722,7 @@ PyMethodDef methods[] = {
     {"kv_attention", (PyCFunction)(void (*)(void))py_kv_attention, METH_FASTCALL, nullptr},
     {"kv_attention_relative", (PyCFunction)(void (*)(void))py_kv_attention_relative, METH_FASTCALL, nullptr},
     {"cache_write", (PyCFunction)(void (*)(void))py_cache_write, METH_FASTCALL, nullptr},
+    {"unipc_step", (PyCFunction)(void (*)(void))py_unipc_step, METH_FASTCALL, nullptr},
     {"current_stream", py_current_stream, METH_NOARGS, nullptr},
     {"release_stream_sink", py_release_stream_sink, METH_NOARGS, nullptr},
     {"quantize", (PyCFunction)(void (*)(void))py_quantize, METH_FASTCALL, nullptr},

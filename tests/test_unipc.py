@@ -149,3 +149,35 @@ def test_the_fixed_weight_one_half_is_what_makes_the_step_second_order(which):
     for w in (0.45, 0.55):
         assert 2.8 < coarse[w] / fine[w] < 5.5, (w, coarse[w] / fine[w])
         assert abs(fine[w]) > 5 * abs(fine[0.5])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape,steps,order,solver", [((48, 3, 8, 32), 4, 2, "bh2"), ((1,), 5, 2, "bh1"), ((257,), 3, 1, "bh2"),
+                                                      ((16, 33), 6, 2, "bh2"), ((5, 8), 1, 2, "bh2")])
+def test_one_launch_step_has_the_bits_of_the_tensor_expressions(gpu, monkeypatch, shape, steps, order, solver):
+    """The step as one launch against the same scheduler's tensor expressions on the GPU, whole trajectories with all
+    history; lengths with and without whole 16-byte pieces, and an input that is not 16-byte aligned."""
+    def run(fused):
+        sch = FlowUniPCMultistepScheduler(num_train_timesteps=1000, shift=1, solver_order=order, solver_type=solver)
+        sch.set_timesteps(steps, device=gpu, shift=5.0)
+        calls, original = [], FlowUniPCMultistepScheduler._fused_step
+        with monkeypatch.context() as m:
+            m.setattr(FlowUniPCMultistepScheduler, "_fused_step",
+                      lambda self, *a: calls.append(original(self, *a) if fused else None) or calls[-1])
+            g = torch.Generator().manual_seed(5)
+            pad = torch.randn(math.prod(shape) + 1, generator=g).bfloat16().to(gpu)
+            x, trace = pad[1:].view(shape), []
+            x[..., 0] = 0.0
+            for t in sch.timesteps.tolist():
+                flow = torch.randn(shape, generator=g).bfloat16().to(gpu) * 3
+                x = sch.step(flow, t, x, return_dict=False)[0]
+                trace += [x, sch.model_outputs[-1], sch.last_sample]
+        assert all((c is not None) == fused for c in calls) and len(calls) == steps
+        return trace
+
+    for a, b in zip(run(True), run(False)):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+    sch = FlowUniPCMultistepScheduler(shift=1)   # gradients and other types keep torch's own operations
+    sch.set_timesteps(2, device=gpu)
+    flow = torch.ones(4, device=gpu, dtype=torch.bfloat16, requires_grad=True)
+    assert sch.step(flow, sch.timesteps[0], torch.ones_like(flow), return_dict=False)[0].requires_grad

@@ -156,12 +156,17 @@ __device__ __forceinline__ void fetch_row(const uint8_t* values, const uint8_t* 
   f.scales = load_global<uint16_t>(scales + so);
 }
 
-// 4 bytes per lane from global memory straight into LDS at lds_base + 4 * lane (lds_base wave-uniform).  An asm
-// statement on purpose: for the builtin the compiler's wait-count pass, which cannot tell the two LDS stages apart,
+// 16 bytes per lane from global memory (base + offset; the base wave-uniform) straight into LDS at lds_base + 16 * lane.
+// An asm statement on purpose: for the builtin the compiler's wait-count pass, which cannot tell the two LDS stages apart,
 // makes later LDS reads of the *other* stage wait for the load.  The kernel waits for these loads itself
 // (vmcnt(0) ahead of the barrier that hands the stage over).
-__device__ __forceinline__ void load_to_lds_b32(const void* src, uint32_t lds_base) {
-  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(src), "s"(lds_base) : "memory");
+__device__ __forceinline__ void load_to_lds_b128(uint32_t offset, const void* base, uint32_t lds_base) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(offset), "s"(base), "s"(lds_base) : "memory");
+}
+__device__ __forceinline__ const void* wave_uniform(const void* p) {
+  const uint64_t v = (uint64_t)(uintptr_t)p;
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+  return reinterpret_cast<const void*>((uintptr_t)(((uint64_t)hi << 32) | lo));
 }
 __device__ __forceinline__ uint32_t lds_address(const void* p) {
   return __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)p);
@@ -563,25 +568,52 @@ __global__ __launch_bounds__(kAttnThreads) void kv_attention_kernel(AttnParams p
     __syncthreads();
   }
 
+  // The rows of a chunk tile reach LDS in pieces of 1 KB, one load of 64 x 16 bytes each: 34 of K, 36 of V, the rows' padding
+  // included (its lanes fetch the row's last 16 bytes again).  Wave w takes pieces w, w + 8, w + 16, w + 24 of either and
+  // one of the six behind them; here the source offsets of its lanes.  2640 queries x 24 heads over 13200 bf16 keys take
+  // 400 us; with 32 loads of 4 bytes per lane and iteration (one row each), which cost 100 vector instructions for their
+  // addresses, 446 us; with 10560 of the keys cached 432 instead of 449 us.
+  constexpr int kKPieces = 2 * kKTileBytes / 1024, kVPieces = 2 * kVTileBytes / 1024;
+  static_assert(kKPieces * 1024 == 2 * kKTileBytes && kVPieces * 1024 == 2 * kVTileBytes && kKPieces + kVPieces <= 72, "nine pieces per wave at most");
+  const int chunk_wave = __builtin_amdgcn_readfirstlane(wave);
+  uint32_t k_piece[4], v_piece[4];
+  int piece_lane = lane;
+  auto source = [&](uint32_t piece, uint32_t pitch) __attribute__((always_inline)) {
+    const uint32_t at = piece * 1024u + piece_lane * 16u, row = at / pitch;
+    return row * ((uint32_t)p.H * (kHeadDim * 2u)) + min(at - row * pitch, kHeadDim * 2u - 16u);
+  };
+  auto locate_pieces = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      k_piece[i] = source(chunk_wave + 8 * i, kKPitch);
+      v_piece[i] = source(chunk_wave + 8 * i, kVPitch);
+    }
+  };
+  if constexpr (WIDE) locate_pieces();
+
   // Plain body: the S phase without interleaved conversion, masking in the last tile, and the successor tile
   // decoded after the MFMAs (or, for the chunk's own bf16 tiles, brought in ahead of them).
   for (; it < seg_end; ++it) {
     const uint8_t* cur = smem + (it & 1) * kStageBytes;
-    // A successor that lies wholly in the bf16 chunk is brought in ahead of the MFMAs: its K rows go
-    // and V rows go straight from global memory into the other stage (one 256-byte row per wave instruction,
-    // 16 rows of each per wave).
-    const bool next_is_chunk = it + 1 < seg_end && iter_base >= n_cached && iter_base + kIterKeys <= Lk_i;  // iter_base = first key of tile it + 1
+    // A successor that lies wholly in the bf16 chunk is brought in ahead of the MFMAs, straight from global memory into
+    // the other stage.
+    const bool next_is_chunk = it + 1 < seg_end && iter_base >= n_cached && iter_base + kIterKeys <= Lk_i && p.H <= 65536;  // iter_base = first key of tile it + 1; 32-bit offsets inside a tile
     if (next_is_chunk) {
-      uint8_t* nxt = smem + ((it + 1) & 1) * kStageBytes;
-      const int64_t src_off = ((int64_t)(iter_base + wave * 16 - n_cached) * p.H + head) * kHeadDim + lane * 2;
-      const int64_t src_step = (int64_t)p.H * kHeadDim;
-      uint8_t* kdst = nxt + (wave >> 2) * kKTileBytes + ((wave & 3) * 16) * kKPitch;
-      uint8_t* vdst = nxt + 2 * kKTileBytes + (wave >> 2) * kVTileBytes + ((wave & 3) * 16) * kVPitch;
-      const uint32_t kdst_lds = lds_address(kdst), vdst_lds = lds_address(vdst);
+      const uint32_t dst = lds_address(smem + ((it + 1) & 1) * kStageBytes) + chunk_wave * 1024;
+      const int64_t src_off = ((int64_t)(iter_base - n_cached) * p.H + head) * kHeadDim;
+      const void *k_base = wave_uniform(p.k_new + src_off), *v_base = wave_uniform(p.v_new + src_off);
+      if constexpr (!WIDE) {  // no registers to keep the offsets in: formed anew
+        asm volatile("" : "+v"(piece_lane));
+        locate_pieces();
+      }
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        load_to_lds_b32(p.k_new + src_off + r * src_step, kdst_lds + r * kKPitch);
-        load_to_lds_b32(p.v_new + src_off + r * src_step, vdst_lds + r * kVPitch);
+      for (int i = 0; i < 4; ++i) load_to_lds_b128(k_piece[i], k_base, dst + i * 8192);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) load_to_lds_b128(v_piece[i], v_base, dst + 2 * kKTileBytes + i * 8192);
+      if (chunk_wave < kKPieces - 32) {
+        load_to_lds_b128(source(32 + chunk_wave, kKPitch), k_base, dst + 32 * 1024);
+      } else if (chunk_wave < kKPieces - 32 + kVPieces - 32) {
+        load_to_lds_b128(source(64 - kKPieces + chunk_wave, kVPitch), v_base, dst + 2 * kKTileBytes + (64 - kKPieces) * 1024);
       }
     }
 #pragma unroll 1

@@ -469,6 +469,18 @@ int ll_qk_norm_rope_pair_amax(const void* q, const void* k, int64_t rows, int nu
                               void* q_out, void* k_out, void* k_out_smooth, const ll_amax_sink* k_amax_sink,
                               void* stream);
 
+/* Patch embedding (wan_5b/modules/causal_model.py:1052-1053, 1535): x [channels, F, H, W] bf16 -> out [tokens, N] bf16, token =
+ * (f, h, w) of the grid F / pt x H / ph x W / pw (what the patches do not cover is left out), weight [N, channels * pt * ph * pw]
+ * in the order of a convolution weight, bias [N] or NULL.  fp32 sums, one rounding.  LL_ENOSUP for shapes outside
+ * channels * pt * ph * pw a multiple of 16 up to 896 and N a multiple of 8. */
+int ll_patch_embed(const void* x, int channels, int F, int H, int W, int pt, int ph, int pw, const void* weight, const void* bias,
+                   int N, void* out, void* stream);
+/* The head's linear layer with its result as latents (:925-960, :1840-1857): y [tokens, K] bf16 -> out [channels, F, H, W] bf16,
+ * weight [pt * ph * pw * channels, K], bias [pt * ph * pw * channels] or NULL; F, H, W whole patches.  LL_ENOSUP unless K is a
+ * multiple of 16. */
+int ll_patch_head(const void* y, int K, const void* weight, const void* bias, int channels, int F, int H, int W, int pt, int ph, int pw,
+                  void* out, void* stream);
+
 /* One step of the flow-matching UniPC sampler, order 1 or 2 (wan_5b/utils/fm_solvers_unipc.py:281-350, 352-486, 488-628,
  * 657-741), as one pass over bf16 tensors of n elements: x0 prediction from the flow, corrector for the step just taken,
  * predictor for the next one.  Every product, difference and sum is rounded to bf16, as the tensor expressions of the

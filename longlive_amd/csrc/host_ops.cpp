@@ -16,6 +16,7 @@
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/autocast_mode.h>
 #include <c10/core/GradMode.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <torch/csrc/Exceptions.h>
@@ -657,23 +658,112 @@ PyObject* py_cache_write(PyObject*, PyObject* const* args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// Calls that took torch's own operations before stay with them where Python code or torch itself has to see each one, or
+// where a gradient is wanted.
+inline bool traced() {
+  return c10::impl::TorchDispatchModeTLS::any_modes_set() || at::impl::torch_function_mode_enabled() || torch::jit::tracer::isTracing() ||
+         at::autocast::is_autocast_enabled(c10::kCUDA);
+}
+inline bool needs_torch(const Tensor& t) {
+  // batched and functional wrappers have no storage
+  return !t.has_storage() || (t.requires_grad() && c10::GradMode::is_enabled()) ||
+         (torch::autograd::impl::get_autograd_meta(t) && t._fw_grad(0).defined());
+}
+// A bf16 matrix [rows, cols] (or, rows < 0, a vector [cols]) on the device, contiguous and 16-byte aligned; null if it is not.
+inline const Tensor* as_weight(PyObject* o, int dev, int64_t rows, int64_t cols) {
+  if (!plain(o)) return nullptr;
+  const Tensor& t = THPVariable_Unpack(o);
+  if (needs_torch(t) || !is_bf16(t, dev) || !t.is_contiguous() || t.numel() != (rows < 0 ? cols : rows * cols) || !aligned16(t.data_ptr())) return nullptr;
+  return &t;
+}
+
+// Up to this many tokens the ends of the model run on the kernels of patch_linear.hip, above it on torch's matrix products and
+// permuted copies.  On the GPU alone (us, here / torch): embedding 192 tokens x 256 9.3 / 11.5, 736 x 1536 11.5 / 13.1,
+// 2640 x 3072 28.5 / 20; head without its normalization 9.6 / 12, 16.6 / 15.9, 28.5 / 20.  With the host's part: embedding of
+// 192 tokens 9.4 / 35, of 736 11.3 / 35; head 18.7 / 75, 24.9 / 74.
+constexpr int64_t kPatchTokens = 1024;
+
+// patch_embed(x [C, F, H, W], weight, bias or None, outputs, pt, ph, pw) -> tokens [1, f h w, outputs], or None when it does not
+// take the call.
+PyObject* py_patch_embed(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 7 || !plain(args[0]) || traced()) Py_RETURN_NONE;
+  const Tensor& x = THPVariable_Unpack(args[0]);
+  const int dev = current_device_of(x);
+  if (needs_torch(x) || !is_bf16(x, dev) || x.dim() != 4 || !x.is_contiguous() || x.numel() == 0 || x.numel() >= (1ll << 31)) Py_RETURN_NONE;
+  const int64_t N = PyLong_AsLongLong(args[3]), pt = PyLong_AsLongLong(args[4]), ph = PyLong_AsLongLong(args[5]), pw = PyLong_AsLongLong(args[6]);
+  if (PyErr_Occurred()) return nullptr;
+  if (pt < 1 || ph < 1 || pw < 1 || x.size(1) < pt || x.size(2) < ph || x.size(3) < pw || N < 1 || N > (1 << 20)) Py_RETURN_NONE;
+  if ((x.size(1) / pt) * (x.size(2) / ph) * (x.size(3) / pw) > kPatchTokens) Py_RETURN_NONE;
+  const Tensor* w = as_weight(args[1], dev, N, x.size(0) * pt * ph * pw);
+  const Tensor* b = args[2] == Py_None ? nullptr : as_weight(args[2], dev, -1, N);
+  if (!w || (!b && args[2] != Py_None)) Py_RETURN_NONE;
+  const Tensor out = empty({1, (x.size(1) / pt) * (x.size(2) / ph) * (x.size(3) / pw), N}, at::kBFloat16, dev);
+  const int code = ll_patch_embed(x.data_ptr(), (int)x.size(0), (int)x.size(1), (int)x.size(2), (int)x.size(3), (int)pt, (int)ph, (int)pw,
+                                  w->data_ptr(), b ? b->data_ptr() : nullptr, (int)N, out.data_ptr(), stream_of(dev));
+  if (code == LL_ENOSUP) Py_RETURN_NONE;
+  if (failed(code, "ll_patch_embed")) return nullptr;
+  return THPVariable_Wrap(out);
+  END_HANDLE_TH_ERRORS
+}
+
+// head(x [1, L, C], e [1, F, 2, C] (shift, scale), weight, bias or None, eps, channels, (f, h, w), (pt, ph, pw)) -> latents
+// [channels, f pt, h ph, w pw], or None when it does not take the call: LayerNorm(x) * (1 + scale) + shift, linear layer, unpatchify.
+PyObject* py_head(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 8 || !plain(args[0]) || !plain(args[1]) || traced()) Py_RETURN_NONE;
+  const Tensor &x = THPVariable_Unpack(args[0]), &e = THPVariable_Unpack(args[1]);
+  const int dev = current_device_of(x);
+  if (needs_torch(x) || needs_torch(e) || !is_bf16(x, dev) || !is_bf16(e, dev) || x.dim() != 3 || x.size(0) != 1 || !x.is_contiguous() ||
+      e.dim() != 4 || e.size(0) != 1 || e.size(2) != 2 || e.size(3) != x.size(2) || !e.is_contiguous() || x.numel() == 0)
+    Py_RETURN_NONE;
+  const int64_t L = x.size(1), C = x.size(2), F = e.size(1);
+  int64_t grid[3], patch[3];
+  for (int i = 0; i < 2; ++i) {
+    PyObject* t = args[6 + i];
+    if (!PyTuple_CheckExact(t) || PyTuple_GET_SIZE(t) != 3) Py_RETURN_NONE;
+    for (int j = 0; j < 3; ++j) (i ? patch : grid)[j] = PyLong_AsLongLong(PyTuple_GET_ITEM(t, j));
+  }
+  const double eps = PyFloat_AsDouble(args[4]);
+  const int64_t channels = PyLong_AsLongLong(args[5]);
+  if (PyErr_Occurred()) return nullptr;
+  for (int j = 0; j < 3; ++j)
+    if (grid[j] < 1 || patch[j] < 1) Py_RETURN_NONE;
+  if (F < 1 || L % F || L > kPatchTokens || grid[0] * grid[1] * grid[2] != L || C % 16 || channels < 1 || !aligned16(x.data_ptr()) || !aligned16(e.data_ptr())) Py_RETURN_NONE;
+  const int64_t N = channels * patch[0] * patch[1] * patch[2];
+  if (N >= (1 << 20) || N * L >= (1ll << 31)) Py_RETURN_NONE;
+  const Tensor* w = as_weight(args[2], dev, N, C);
+  const Tensor* b = args[3] == Py_None ? nullptr : as_weight(args[3], dev, -1, N);
+  if (!w || (!b && args[3] != Py_None)) Py_RETURN_NONE;
+  void* stream = stream_of(dev);
+  const Tensor y = empty({L, C}, at::kBFloat16, dev);
+  const uint16_t* shift = static_cast<const uint16_t*>(e.data_ptr());
+  if (failed(ll_adaln_modulate_amax(x.data_ptr(), 1, L, (int)C, shift + C, shift, e.stride(0), e.stride(1), e.stride(0), e.stride(1), L / F,
+                                    (float)eps, 1, y.data_ptr(), nullptr, stream),
+             "ll_adaln_modulate"))
+    return nullptr;
+  const Tensor out = empty({channels, grid[0] * patch[0], grid[1] * patch[1], grid[2] * patch[2]}, at::kBFloat16, dev);
+  if (failed(ll_patch_head(y.data_ptr(), (int)C, w->data_ptr(), b ? b->data_ptr() : nullptr, (int)channels, (int)out.size(1), (int)out.size(2),
+                           (int)out.size(3), (int)patch[0], (int)patch[1], (int)patch[2], out.data_ptr(), stream),
+             "ll_patch_head"))
+    return nullptr;
+  return THPVariable_Wrap(out);
+  END_HANDLE_TH_ERRORS
+}
+
 // unipc_step(flow, sample, last or None, m1 or None, m2 or None, sigma, corrector, predictor) -> (x0 prediction, corrected
 // sample, next sample), or None when it does not take the call.  corrector, predictor: (order, ratio, m0, b, rho, rk,
 // rho_new), see ll_unipc_scalars; with a corrector of order 0 the corrected sample is `sample` itself.
 PyObject* py_unipc_step(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  if (n != 8 || c10::impl::TorchDispatchModeTLS::any_modes_set() || at::impl::torch_function_mode_enabled() || torch::jit::tracer::isTracing())
-    Py_RETURN_NONE;
+  if (n != 8 || traced()) Py_RETURN_NONE;
   const Tensor* in[5] = {};
   int dev = -1;
   for (int i = 0; i < 5; ++i) {
     if (i > 1 && args[i] == Py_None) continue;
     if (!plain(args[i])) Py_RETURN_NONE;
     const Tensor& t = THPVariable_Unpack(args[i]);
-    // batched and functional wrappers have no storage; gradients of either mode need torch's own operations
-    if (!t.has_storage() || (t.requires_grad() && c10::GradMode::is_enabled()) ||
-        (torch::autograd::impl::get_autograd_meta(t) && t._fw_grad(0).defined()))
-      Py_RETURN_NONE;
+    if (needs_torch(t)) Py_RETURN_NONE;
     if (i == 0) dev = current_device_of(t);
     if (!is_bf16(t, dev) || !t.is_contiguous() || t.numel() == 0 || (i > 0 && t.sizes() != in[0]->sizes())) Py_RETURN_NONE;
     in[i] = &t;
@@ -722,6 +812,8 @@ PyMethodDef methods[] = {
     {"kv_attention", (PyCFunction)(void (*)(void))py_kv_attention, METH_FASTCALL, nullptr},
     {"kv_attention_relative", (PyCFunction)(void (*)(void))py_kv_attention_relative, METH_FASTCALL, nullptr},
     {"cache_write", (PyCFunction)(void (*)(void))py_cache_write, METH_FASTCALL, nullptr},
+    {"patch_embed", (PyCFunction)(void (*)(void))py_patch_embed, METH_FASTCALL, nullptr},
+    {"head", (PyCFunction)(void (*)(void))py_head, METH_FASTCALL, nullptr},
     {"unipc_step", (PyCFunction)(void (*)(void))py_unipc_step, METH_FASTCALL, nullptr},
     {"current_stream", py_current_stream, METH_NOARGS, nullptr},
     {"release_stream_sink", py_release_stream_sink, METH_NOARGS, nullptr},

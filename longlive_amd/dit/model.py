@@ -5,8 +5,8 @@ Module and parameter names follow the reference model so that its checkpoints, i
 ``CausalWanAttentionBlock`` (wan_5b/modules/causal_model.py:794-930), ``CausalWanSelfAttention``
 (:298-791), ``MultiShotT2VCrossAttention`` (:197-262), ``CausalHead`` (:933-959), ``CausalWanModel``
 (:1040-1110, forward :1485-1654).  The ten Linear layers of every block become ``FourOverSixLinear``
-through ``quantize_model_with_filter``; norms, RoPE, adaLN and attention call the gfx950 kernels;
-the bf16 ends of the model (patch / time / text embeddings, head) are plain torch modules.
+through ``quantize_model_with_filter``; norms, RoPE, adaLN, attention, patch embedding and head call the gfx950 kernels;
+the time and text embeddings are plain torch modules.
 """
 from __future__ import annotations
 
@@ -408,6 +408,15 @@ class CausalHead(nn.Module):
             return self.head(y.unflatten(1, (num_frames, frame_seqlen)))
         return self.head(self.norm(x).unflatten(1, (num_frames, frame_seqlen)) * (1 + e[1]) + e[0])
 
+    def latents(self, x, e, grid, patch_size, channels: int):
+        """``unpatchify(forward(x, e))`` as one native call, the linear layer writing the latents in place of its rows; None
+        where the modules have to run."""
+        if not x.is_cuda or type(self.norm) is not WanLayerNorm or type(self.head) is not nn.Linear or self.norm.weight is not None \
+                or _has_hooks(self, self.norm, self.head):
+            return None
+        return _native.host().head(x, self.modulation.unsqueeze(1) + e, self.head.weight, self.head.bias, self.norm.eps, channels,
+                                   tuple(grid), tuple(patch_size))
+
 
 def sinusoidal_embedding_1d(dim: int, position: torch.Tensor) -> torch.Tensor:
     half = dim // 2
@@ -468,6 +477,11 @@ class CausalDiT(nn.Module):
         pt, ph, pw = self.cfg.patch_size
         c, fr, hh, ww = x.shape
         f, h, w = fr // pt, hh // ph, ww // pw
+        conv = self.patch_embedding
+        if x.is_cuda:   # patches gathered and multiplied in one launch
+            tokens = _native.host().patch_embed(x, conv.weight, conv.bias, conv.weight.shape[0], pt, ph, pw)
+            if tokens is not None:
+                return tokens, (f, h, w)
         patches = x[:, :f * pt, :h * ph, :w * pw].reshape(c, f, pt, h, ph, w, pw).permute(1, 3, 5, 0, 2, 4, 6)
         patches = patches.reshape(f * h * w, c * pt * ph * pw)
         weight = self.patch_embedding.weight.reshape(self.patch_embedding.weight.shape[0], -1)
@@ -556,5 +570,9 @@ class CausalDiT(nn.Module):
                 kvc.apply_cache_update(kv_cache[i], cur_end, loc_end, info, self.kv_quant_config)
         if cache_only:
             return None
+        if type(self.head) is CausalHead:
+            latents = self.head.latents(x, e.unsqueeze(2), (f, h, w), cfg.patch_size, cfg.out_dim)
+            if latents is not None:
+                return latents
         x = self.head(x, e.unsqueeze(2))
         return self.unpatchify(x[0].flatten(0, 1) if x.dim() == 4 else x[0], (f, h, w))

@@ -1,4 +1,6 @@
 """GPU tests of the DiT block and the streaming generator on top of the NVFP4 kernels."""
+import math
+
 import numpy as np
 import pytest
 import torch
@@ -980,3 +982,54 @@ def test_native_block_call_equals_the_separate_operations(gpu, F, h, w, heads, f
                 assert len(got) == len(ref)
                 for i, (a, b) in enumerate(zip(got, ref)):
                     assert (a is None and b is None) or torch.equal(a, b), i
+
+
+@pytest.mark.parametrize("dim,channels,patch,latent", [
+    (256, 48, (1, 2, 2), (3, 8, 32)),     # the suite's model: 192 tokens
+    (384, 16, (1, 2, 2), (2, 10, 14)),    # 70 tokens: ragged tiles of tokens, N = 64
+    (136, 8, (2, 1, 2), (5, 3, 7)),       # a frame and a column that no patch covers, N not a multiple of the tiles
+    (3072, 48, (1, 2, 2), (1, 6, 10)),    # full width
+    (128, 4, (1, 2, 3), (1, 2, 3)),       # K = 24: not taken by the embedding; patches three wide; one token
+])
+def test_patch_embedding_and_head_against_their_modules(gpu, monkeypatch, dim, channels, patch, latent):
+    """The two ends of the model as kernels of their own against the permuted copies and matrix products of the same model,
+    and both against fp64.  Both round one fp32 sum to bf16, so each lies within 2^-8 of fp64 relative to the sum of
+    magnitudes' share of fp32 noise: half a bf16 step plus K 2^-24 of sum |a b|."""
+    from types import SimpleNamespace
+    from longlive_amd import _native
+
+    torch.manual_seed(3)
+    cfg = DiTConfig(dim=dim, ffn_dim=dim, num_heads=dim // 128 or 1, num_layers=0, in_dim=channels, out_dim=channels, patch_size=patch,
+                    text_dim=64, text_len=4)
+    with torch.device(gpu):
+        model = CausalDiT(cfg).bfloat16()
+    x = torch.randn(channels, *latent, device=gpu).bfloat16()
+    grid = tuple(a // b for a, b in zip(latent, patch))
+    L, K = math.prod(grid), channels * math.prod(patch)
+    h, e = torch.randn(1, L, dim, device=gpu).bfloat16(), torch.randn(1, grid[0], 1, dim, device=gpu).bfloat16()
+    with torch.no_grad():
+        model.patch_embedding.bias.normal_()
+        model.head.head.bias.normal_()
+        taken = _native.host().patch_embed(x, model.patch_embedding.weight, model.patch_embedding.bias, dim, *patch)
+        assert (taken is not None) == (K % 16 == 0 and dim % 8 == 0)
+        tokens, got_grid = model.patch_embed(x)
+        assert got_grid == grid and tokens.shape == (1, L, dim)
+        latents = model.head.latents(h, e, grid, patch, channels)
+        assert (latents is not None) == (dim % 16 == 0)
+        if latents is None:
+            latents = model.unpatchify(model.head(h, e)[0].flatten(0, 1), grid)
+        monkeypatch.setattr(_native, "host", lambda: SimpleNamespace(patch_embed=lambda *a: None))
+        plain_tokens = model.patch_embed(x)[0]
+        plain = model.unpatchify(model.head(h, e)[0].flatten(0, 1), grid)
+        y = _native.adaln_modulate(h, *[(model.head.modulation.unsqueeze(1) + e)[:, :, i:i + 1] for i in (1, 0)], L // grid[0]).double()[0]
+    pt, ph, pw = patch
+    crop = x[:, :grid[0] * pt, :grid[1] * ph, :grid[2] * pw].double()
+    patches = crop.reshape(channels, grid[0], pt, grid[1], ph, grid[2], pw).permute(1, 3, 5, 0, 2, 4, 6).reshape(L, K)
+    for a, w, b, got, other, back in (
+            (patches, model.patch_embedding.weight.flatten(1), model.patch_embedding.bias, tokens[0], plain_tokens[0], lambda t: t),
+            (y, model.head.head.weight, model.head.head.bias, latents, plain, lambda t: model.unpatchify(t, grid))):
+        w, b = w.detach().double(), b.detach().double()
+        ref, size = back(a @ w.T + b), back(a.abs() @ w.abs().T + b.abs())
+        assert got.shape == other.shape == ref.shape
+        bound = ref.abs() * 2 ** -8 + size * (a.shape[1] + 2) * 2 ** -24
+        assert ((got.double() - ref).abs() <= bound).all() and ((other.double() - ref).abs() <= bound).all()

@@ -135,12 +135,15 @@ inline TileKernelChoice choose_tile_kernel(int64_t M, int64_t N, int64_t Kp, int
     if (tiles <= cus && 2 * tiles > cus) return {4, true};
   }
   // Small problems: when even 128 x 128 tiles would occupy at most half of the compute units, 64 x 64 tiles (more
-  // decode work per MFMA, but four times the workgroups) finish sooner.  Up to 0.69 of the units they still do where K is
-  // long, since each 128 x 128 tile then has a unit to itself with one wave per SIMD (880 x 3072 x 3072, 168 tiles: 24.8
-  // against 27.7 us; 1173 x 2048 x 8192, 160 tiles: 52.6 against 65.4; but 335 x 5888 x 1536, 138 tiles: 16.4 against 16.0,
-  // and 520 x 5888 x 2048, 230 tiles: 23.4 against 20.5).
+  // decode work per MFMA, but four times the workgroups) finish sooner.  Up to three of them per unit they still do where K is
+  // long, since each 128 x 128 tile then has a unit to itself with one wave per SIMD (880 x 3072 x 3072, 672 small tiles:
+  // 24.8 against 27.7 us; 1173 x 2048 x 8192, 608: 52.6 against 65.4; 1173 x 2304 x 9216, 684: 59.9 against 72.8; 1173 x 2560 x
+  // 10240, 760: 68 against 81; 368 x 8192 x 2048, 768: 22.0 against 22.2; but
+  // 1760 x 2048 x 8192, 896: 68.3 against 65.8, and 256 x 14336 x 3072, 896: 32.5 against
+  // 28.4; with K = 1536, 335 x 5888, 552: 16.4 against 16.0).
   const int64_t tiles_128 = ((M + 127) / 128) * ((N * n_products + 127) / 128);
-  if (tiles_128 <= cus / 2 || (schedule != 2 && Kp >= 2048 && tiles_128 * 16 <= 11 * (int64_t)cus)) return {0, false};
+  const int64_t tiles_64 = ((M + 63) / 64) * ((N + 63) / 64) * n_products;
+  if (tiles_128 <= cus / 2 || (schedule != 2 && Kp >= 2048 && tiles_64 <= 3 * (int64_t)cus)) return {0, false};
   // Two workgroups of four waves are resident per compute unit.  The 256 x 128 / 128 x 256 tiles need 6 decode
   // instructions per MFMA, the 128 x 128 tile 8, so the larger tiles win unless they fill the slots much worse.  A last
   // round of at most one workgroup per unit is cheap: alone on its unit a workgroup runs in 0.56 of the time it takes

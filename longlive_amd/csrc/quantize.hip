@@ -32,9 +32,20 @@ __global__ __launch_bounds__(kThreads) void amax_partial_kernel(AmaxJobs jobs, i
   if (vec) {
     const int64_t kc = K >> 3;
     const int64_t nchunks = M * kc;
+    // (r, cc): the piece's row and its place in it; a step of nthreads pieces advances both by constants.  With a 64-bit
+    // division per piece, amax and quantization of 7040 x 14336 from memory took 93.2 instead of 90.5 us (7040 x 3072: 24.6,
+    // now 24.0).  Four pieces of a lane on their way at a time: 89.7 from memory, but 81.5 instead of 78.2 where the tensor
+    // is in the last-level cache; the same with a workgroup's pieces side by side: 93.5 and 84.7.
+    const int64_t step_r = nthreads / kc, step_c = nthreads - step_r * kc;
+    int64_t r = tid / kc, cc = tid - r * kc;
     for (int64_t c = tid; c < nchunks; c += nthreads) {
-      const int64_t r = c / kc, cc = c - r * kc;
       const uint4 v = *reinterpret_cast<const uint4*>(x + r * ldx + cc * 8);
+      r += step_r;
+      cc += step_c;
+      if (cc >= kc) {
+        cc -= kc;
+        ++r;
+      }
       const uint32_t w[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
       for (int i = 0; i < 4; ++i) {

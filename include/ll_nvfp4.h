@@ -116,6 +116,13 @@ typedef struct ll_amax_sink {
  * reference. */
 int ll_amax_epoch_advance(uint32_t* epoch_offset, uint32_t step, uint64_t* parts, void* stream);
 
+/* ll_nvfp4_quantize of a small tensor as one launch whose workgroups exchange their maxima through amax_sink, which serves
+ * this launch only (a fresh epoch; nothing else reads or writes it meanwhile).  The same bytes.  spin_limit as in
+ * ll_adaln_quantize.  LL_ENOSUP for more than 256 tiles of 128 x 64 (or one per compute unit), K not a multiple of 64, ldx not
+ * a multiple of 8 or x not 16-byte aligned.  In a recording the epoch has to move between replays (epoch_offset). */
+int ll_nvfp4_quantize_once(const void* x, int64_t M, int64_t K, int64_t ldx, int rule, uint8_t* values, uint8_t* scales, float* amax,
+                           const ll_amax_sink* amax_sink, int64_t spin_limit, void* stream);
+
 /* ll_nvfp4_quantize whose tensor amax comes from an amax sink that the producer of x has filled with the
  * same epoch; amax (f32[1]) is written.  The bytes equal those of ll_nvfp4_quantize with amax_given == 0. */
 int ll_nvfp4_quantize_from_sink(const void* x, int64_t M, int64_t K, int64_t ldx, int rule,

@@ -80,6 +80,8 @@ _SIGNATURES = {
                                      c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p]),
     "ll_qk_norm_rope_pair_amax": (c_int, [c_void_p, c_void_p, c_int64, c_int, c_void_p, c_void_p, c_float, c_void_p,
                                      c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
+    "ll_nvfp4_quantize_once": (c_int, [c_void_p, c_int64, c_int64, c_int64, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_int64,
+                                       c_void_p]),
     "ll_patch_embed": (c_int, [c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_int, c_void_p,
                                c_void_p]),
     "ll_patch_head": (c_int, [c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p,

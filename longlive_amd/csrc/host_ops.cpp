@@ -99,79 +99,7 @@ inline TempOperand temp_operand(int64_t m, int64_t k, int dev) {
   return t;
 }
 
-// quantize(x, rule) -> (values, scales, amax): x bf16 [M, K] with contiguous columns.
-PyObject* py_quantize(PyObject*, PyObject* const* args, Py_ssize_t n) {
-  HANDLE_TH_ERRORS
-  if (n != 2 || !plain(args[0])) Py_RETURN_NONE;
-  const Tensor& x = THPVariable_Unpack(args[0]);
-  const int dev = current_device_of(x);
-  if (!is_bf16(x, dev) || x.dim() != 2 || x.stride(1) != 1 || x.numel() == 0) Py_RETURN_NONE;
-  const int64_t M = x.size(0), K = x.size(1), Mp = round_up(M, 128), Kp = round_up(K, 64);
-  const int rule = (int)PyLong_AsLong(args[1]);
-  const Tensor values = empty({Mp, Kp / 2}, at::kByte, dev), scales = empty({Mp * Kp / 16}, at::kFloat8_e4m3fn, dev),
-               amax = empty({1}, at::kFloat, dev), ws = empty({(int64_t)LL_AMAX_PARTS}, at::kFloat, dev);
-  if (failed(ll_nvfp4_quantize(x.data_ptr(), M, K, x.stride(0), rule, values.data_ptr<uint8_t>(), static_cast<uint8_t*>(scales.data_ptr()),
-                               amax.data_ptr<float>(), 0, ws.data_ptr<float>(), stream_of(dev)),
-             "ll_nvfp4_quantize"))
-    return nullptr;
-  return tuple3(values, scales, amax);
-  END_HANDLE_TH_ERRORS
-}
-
-// linear(x, rule, denom_a, w_values, w_scales, w_amax, denom_b, out_features, bias or None) -> bf16 [M, out_features]:
-// activation quantization and GEMM; the operand in between lives for this call.
-PyObject* py_linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
-  HANDLE_TH_ERRORS
-  if (n != 9 || !plain(args[0])) Py_RETURN_NONE;
-  const Tensor& x = THPVariable_Unpack(args[0]);
-  const Tensor *wv = as_tensor(args[3]), *ws = as_tensor(args[4]), *wa = as_tensor(args[5]), *bias = as_tensor(args[8]);
-  const int dev = current_device_of(x);
-  if (!wv || !ws || !wa || (!bias && args[8] != Py_None)) Py_RETURN_NONE;
-  if (!is_bf16(x, dev) || x.dim() != 2 || x.stride(1) != 1 || x.numel() == 0) Py_RETURN_NONE;
-  if (!on_device(*wv, dev) || !on_device(*ws, dev) || !on_device(*wa, dev) || wv->dim() != 2) Py_RETURN_NONE;
-  const int64_t M = x.size(0), K = x.size(1), N = PyLong_AsLongLong(args[7]);
-  const int rule = (int)PyLong_AsLong(args[1]);
-  const double denom_a = PyFloat_AsDouble(args[2]), denom_b = PyFloat_AsDouble(args[6]);
-  if (PyErr_Occurred()) return nullptr;
-  if (wv->size(1) * 2 != round_up(K, 64) || wv->size(0) != round_up(N, 128) || !wv->is_contiguous() || !ws->is_contiguous()) Py_RETURN_NONE;
-  if (bias && (!is_bf16(*bias, dev) || bias->numel() != N || !bias->is_contiguous())) Py_RETURN_NONE;
-  void* stream = stream_of(dev);
-  const TempOperand a = temp_operand(M, K, dev);
-  const Tensor out = empty({M, N}, at::kBFloat16, dev);
-  if (failed(ll_nvfp4_quantize(x.data_ptr(), M, K, x.stride(0), rule, a.values, a.scales, a.amax, 0, a.workspace, stream),
-             "ll_nvfp4_quantize"))
-    return nullptr;
-  if (failed(ll_nvfp4_gemm_tnt(a.values, a.scales, wv->data_ptr<uint8_t>(), static_cast<const uint8_t*>(ws->data_ptr()), nullptr,
-                               a.amax, wa->data_ptr<float>(), (float)denom_a, (float)denom_b, M, N, a.mp, wv->size(0), a.kp,
-                               out.data_ptr(), N, bias ? bias->data_ptr() : nullptr, stream),
-             "ll_nvfp4_gemm_tnt"))
-    return nullptr;
-  return THPVariable_Wrap(out);
-  END_HANDLE_TH_ERRORS
-}
-
-// dequantize(values, scales, amax, rule, Mp, Kp, M, K, dtype code) -> [M, K]
-PyObject* py_dequantize(PyObject*, PyObject* const* args, Py_ssize_t n) {
-  HANDLE_TH_ERRORS
-  if (n != 9) Py_RETURN_NONE;
-  const Tensor *values = as_tensor(args[0]), *scales = as_tensor(args[1]), *amax = as_tensor(args[2]);
-  const int dev = values ? current_device_of(*values) : -1;
-  if (!values || !scales || !amax || dev < 0 || !on_device(*scales, dev) || !on_device(*amax, dev)) Py_RETURN_NONE;
-  int64_t v[6];
-  for (int i = 0; i < 6; ++i) v[i] = PyLong_AsLongLong(args[3 + i]);
-  if (PyErr_Occurred()) return nullptr;
-  const at::ScalarType type = v[5] == LL_DTYPE_BF16 ? at::kBFloat16 : v[5] == LL_DTYPE_F16 ? at::kHalf : at::kFloat;
-  const Tensor out = empty({v[3], v[4]}, type, dev);
-  if (failed(ll_nvfp4_dequantize(static_cast<const uint8_t*>(values->data_ptr()), static_cast<const uint8_t*>(scales->data_ptr()),
-                                 amax->data_ptr<float>(), (int)v[0], v[1], v[2], v[3], v[4], out.data_ptr(), (int)v[5], v[4],
-                                 stream_of(dev)),
-             "ll_nvfp4_dequantize"))
-    return nullptr;
-  return THPVariable_Wrap(out);
-  END_HANDLE_TH_ERRORS
-}
-
-// ------------------------------------------------------------------------------------------------ amax sinks of a block
+// ------------------------------------------------------------------------------------------------ amax sinks
 // The sink through which the kernels of one native call hand tensor maxima on belongs to the (device, stream) pair: launches
 // on one stream are ordered, and two streams (or the threads that drive them) never meet in one buffer.
 struct StreamSink {
@@ -211,6 +139,97 @@ Epochs epochs_of_stream(int dev, void* stream) {
   const Epochs e{reinterpret_cast<uint64_t*>(s.parts.data_ptr<int64_t>()), nullptr, s.epoch};
   s.epoch += kEpochsPerCall;
   return e;
+}
+
+// The amax of x and its quantization: one launch for a small tensor, two otherwise and while the stream is being captured (a
+// recorded epoch would be the same in every replay).
+constexpr int64_t kSpinLimit = 64;  // looks of one to two microseconds at the other workgroups' maxima
+int quantize_operand(const void* x, int64_t M, int64_t K, int64_t ldx, int rule, uint8_t* values, uint8_t* scales, float* amax, float* workspace,
+                     int dev, void* stream) {
+  if (K % 64 == 0 && ((M + 127) / 128) * (K / 64) <= 256) {
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(static_cast<hipStream_t>(stream), &capture) == hipSuccess && capture == hipStreamCaptureStatusNone) {
+      Epochs e = epochs_of_stream(dev, stream);
+      if (e.parts) {
+        const ll_amax_sink sink = e.take();
+        const int code = ll_nvfp4_quantize_once(x, M, K, ldx, rule, values, scales, amax, &sink, kSpinLimit, stream);
+        if (code != LL_ENOSUP) return code;
+      }
+    }
+  }
+  return ll_nvfp4_quantize(x, M, K, ldx, rule, values, scales, amax, 0, workspace, stream);
+}
+
+// quantize(x, rule) -> (values, scales, amax): x bf16 [M, K] with contiguous columns.
+PyObject* py_quantize(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 2 || !plain(args[0])) Py_RETURN_NONE;
+  const Tensor& x = THPVariable_Unpack(args[0]);
+  const int dev = current_device_of(x);
+  if (!is_bf16(x, dev) || x.dim() != 2 || x.stride(1) != 1 || x.numel() == 0) Py_RETURN_NONE;
+  const int64_t M = x.size(0), K = x.size(1), Mp = round_up(M, 128), Kp = round_up(K, 64);
+  const int rule = (int)PyLong_AsLong(args[1]);
+  const Tensor values = empty({Mp, Kp / 2}, at::kByte, dev), scales = empty({Mp * Kp / 16}, at::kFloat8_e4m3fn, dev),
+               amax = empty({1}, at::kFloat, dev), ws = empty({(int64_t)LL_AMAX_PARTS}, at::kFloat, dev);
+  if (failed(quantize_operand(x.data_ptr(), M, K, x.stride(0), rule, values.data_ptr<uint8_t>(), static_cast<uint8_t*>(scales.data_ptr()),
+                              amax.data_ptr<float>(), ws.data_ptr<float>(), dev, stream_of(dev)),
+             "ll_nvfp4_quantize"))
+    return nullptr;
+  return tuple3(values, scales, amax);
+  END_HANDLE_TH_ERRORS
+}
+
+// linear(x, rule, denom_a, w_values, w_scales, w_amax, denom_b, out_features, bias or None) -> bf16 [M, out_features]:
+// activation quantization and GEMM; the operand in between lives for this call.
+PyObject* py_linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 9 || !plain(args[0])) Py_RETURN_NONE;
+  const Tensor& x = THPVariable_Unpack(args[0]);
+  const Tensor *wv = as_tensor(args[3]), *ws = as_tensor(args[4]), *wa = as_tensor(args[5]), *bias = as_tensor(args[8]);
+  const int dev = current_device_of(x);
+  if (!wv || !ws || !wa || (!bias && args[8] != Py_None)) Py_RETURN_NONE;
+  if (!is_bf16(x, dev) || x.dim() != 2 || x.stride(1) != 1 || x.numel() == 0) Py_RETURN_NONE;
+  if (!on_device(*wv, dev) || !on_device(*ws, dev) || !on_device(*wa, dev) || wv->dim() != 2) Py_RETURN_NONE;
+  const int64_t M = x.size(0), K = x.size(1), N = PyLong_AsLongLong(args[7]);
+  const int rule = (int)PyLong_AsLong(args[1]);
+  const double denom_a = PyFloat_AsDouble(args[2]), denom_b = PyFloat_AsDouble(args[6]);
+  if (PyErr_Occurred()) return nullptr;
+  if (wv->size(1) * 2 != round_up(K, 64) || wv->size(0) != round_up(N, 128) || !wv->is_contiguous() || !ws->is_contiguous()) Py_RETURN_NONE;
+  if (bias && (!is_bf16(*bias, dev) || bias->numel() != N || !bias->is_contiguous())) Py_RETURN_NONE;
+  void* stream = stream_of(dev);
+  const TempOperand a = temp_operand(M, K, dev);
+  const Tensor out = empty({M, N}, at::kBFloat16, dev);
+  if (failed(quantize_operand(x.data_ptr(), M, K, x.stride(0), rule, a.values, a.scales, a.amax, a.workspace, dev, stream),
+             "ll_nvfp4_quantize"))
+    return nullptr;
+  if (failed(ll_nvfp4_gemm_tnt(a.values, a.scales, wv->data_ptr<uint8_t>(), static_cast<const uint8_t*>(ws->data_ptr()), nullptr,
+                               a.amax, wa->data_ptr<float>(), (float)denom_a, (float)denom_b, M, N, a.mp, wv->size(0), a.kp,
+                               out.data_ptr(), N, bias ? bias->data_ptr() : nullptr, stream),
+             "ll_nvfp4_gemm_tnt"))
+    return nullptr;
+  return THPVariable_Wrap(out);
+  END_HANDLE_TH_ERRORS
+}
+
+// dequantize(values, scales, amax, rule, Mp, Kp, M, K, dtype code) -> [M, K]
+PyObject* py_dequantize(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 9) Py_RETURN_NONE;
+  const Tensor *values = as_tensor(args[0]), *scales = as_tensor(args[1]), *amax = as_tensor(args[2]);
+  const int dev = values ? current_device_of(*values) : -1;
+  if (!values || !scales || !amax || dev < 0 || !on_device(*scales, dev) || !on_device(*amax, dev)) Py_RETURN_NONE;
+  int64_t v[6];
+  for (int i = 0; i < 6; ++i) v[i] = PyLong_AsLongLong(args[3 + i]);
+  if (PyErr_Occurred()) return nullptr;
+  const at::ScalarType type = v[5] == LL_DTYPE_BF16 ? at::kBFloat16 : v[5] == LL_DTYPE_F16 ? at::kHalf : at::kFloat;
+  const Tensor out = empty({v[3], v[4]}, type, dev);
+  if (failed(ll_nvfp4_dequantize(static_cast<const uint8_t*>(values->data_ptr()), static_cast<const uint8_t*>(scales->data_ptr()),
+                                 amax->data_ptr<float>(), (int)v[0], v[1], v[2], v[3], v[4], out.data_ptr(), (int)v[5], v[4],
+                                 stream_of(dev)),
+             "ll_nvfp4_dequantize"))
+    return nullptr;
+  return THPVariable_Wrap(out);
+  END_HANDLE_TH_ERRORS
 }
 
 // ------------------------------------------------------------------------------------------------ block

@@ -1,5 +1,7 @@
 """GPU parity: NVFP4 quantize / dequantize through the C ABI against the CPU oracle and the golden
 vectors.  Bar: bit-exact packed nibbles, scale bytes and amax."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -226,3 +228,55 @@ def test_two_tensors_in_one_launch_equal_the_oracle(gpu, rows, C, rule):
         t = sinks[0].ticket()
         _native.layer_norm(xs[0], None, None, amax_out=t)
         _native.quantize_pair(ys[0], ys[1], rule, t, t, outs[0], outs[1])
+
+
+@pytest.mark.parametrize("rule", ["mse", "static_6", "static_4", "mae", "abs_max"])
+@pytest.mark.parametrize("M,K,pad", [(1, 64, 0), (48, 256, 0), (129, 192, 8), (512, 3072, 0), (1173, 1536, 0), (4096, 512, 0), (130, 8192, 24)])
+def test_small_tensors_in_one_launch_have_the_bytes_of_the_two_launches(gpu, rule, M, K, pad):
+    """Up to 256 tiles of 128 x 64, one workgroup each: ragged rows, rows with a stride, one tile, as many as the rule takes;
+    several calls on one sink with the maximum falling; with the wait's way out (every workgroup computes all maxima);
+    a tensor of zeros and one with maxima outside the fast path."""
+    lib, stream, code = _native.load(), torch.cuda.current_stream().cuda_stream, _native.RULE_IDS[rule]
+    g = torch.Generator(device=gpu).manual_seed(M + K)
+    Mp, Kp = -(-M // 128) * 128, K
+    parts = torch.zeros(1024, dtype=torch.int64, device=gpu)
+    for i, (scale, spin) in enumerate([(1e3, 64), (1.0, 64), (0.01, -1), (0.0, 64), (1e35, 64), (1.0, 0)]):
+        x = (torch.randn((M, K + pad), generator=g, device=gpu) * scale).bfloat16()[:, :K]
+        x[0, -1] *= 30
+        outs = []
+        for once in (True, False):
+            v, s, a = (torch.full((n,), 7, dtype=t, device=gpu) for n, t in ((Mp * Kp // 2, torch.uint8), (Mp * Kp // 16, torch.uint8),
+                                                                            (1, torch.float32)))
+            ws = torch.empty(1024, dtype=torch.float32, device=gpu)
+            args = (x.data_ptr(), M, K, x.stride(0), code, v.data_ptr(), s.data_ptr(), a.data_ptr())
+            if once:
+                sink = _native.AmaxSinkStruct(parts.data_ptr(), i + 1, None)
+                rc = lib.ll_nvfp4_quantize_once(*args, ctypes.byref(sink), spin, stream)
+            else:
+                rc = lib.ll_nvfp4_quantize(*args, 0, ws.data_ptr(), stream)
+            assert rc == 0, lib.ll_last_error()
+            outs.append((v, s, a))
+        assert all(torch.equal(p, q) for p, q in zip(*outs)), (i, scale, spin)
+    assert lib.ll_nvfp4_quantize_once(x.data_ptr(), 128 * 257, 64, 64, *args[4:], ctypes.byref(sink), 64, stream) == -3   # refused on the host
+
+
+def test_small_quantization_recorded_into_a_graph(gpu):
+    """While a stream is being captured the two launches are recorded: replays on a falling maximum equal the eager bytes."""
+    cfg = QuantizationConfig(scale_rule="mse")
+    xs = [(torch.randn(200, 512, generator=torch.Generator().manual_seed(i)) * s).bfloat16().to(gpu) for i, s in enumerate((8.0, 1.0, 0.1))]
+    eager = [quantize_to_fp4(x, cfg) for x in xs]
+    static, side = xs[0].clone(), torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        quantize_to_fp4(static, cfg)
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        q = quantize_to_fp4(static, cfg)
+    for x, ref in zip(xs, eager):
+        static.copy_(x)
+        graph.replay()
+        torch.cuda.synchronize()
+        quantize_to_fp4(x, cfg)
+        assert torch.equal(q.values, ref.values) and torch.equal(q.amax, ref.amax)
+        assert torch.equal(q.scale_factors.view(torch.uint8), ref.scale_factors.view(torch.uint8))

@@ -89,7 +89,7 @@ __global__ __launch_bounds__(256) void patch_embed_kernel(const uint16_t* __rest
 // ----------------------------------------------------------------------------- head
 // out[c][f pt + p][h ph + q][w pw + r] = sum_k y[m][k] weight[n][k] + bias[n], n = ((p ph + q) pw + r) C + c.  N is small
 // (192) and K long (3072): a workgroup takes 32 tokens x 64 outputs and its eight waves an eighth of K each, read straight
-// from memory; the parts meet in LDS and are added in a fixed order.  
+// from memory; the parts meet in LDS and are added in a fixed order.
 // 192 tokens x 256 9.6 us, 736 x 1536 16.6 us (12 and 15.9 as library product and permuted copy).
 constexpr int kHeadTokens = 32, kHeadOutputs = 64, kHeadWaves = 8, kHeadPitch = kHeadTokens;  // 64 KB of LDS
 

@@ -43,13 +43,15 @@ const char* ll_last_error(void);
 int ll_version(void);
 
 /*
- * Memory of the library's own.  Two kernels let several workgroups compute parts of one output tile and pass the
- * parts through device memory: the attention's split division (ll_kv_attention_set_policy) and the W4A4 GEMM at
- * sizes where whole tiles would leave compute units idle (ll_nvfp4_gemm_reserve).  That memory is allocated per
- * (device, stream) by the first launch that needs it, grown when a later launch needs more (which frees the old
- * set and so waits for the device), shared by both kernels and kept.  ll_release_stream_memory frees the set of
- * (current device, stream), if any, after waiting for the launches that still use it - for callers that create
- * streams as they go.  Launches on a stream that is being captured into a graph never allocate: they use the set a
+ * Memory of the library's own.  Three kernels let several workgroups compute parts of one output tile and pass the
+ * parts through device memory: the attention's split division (ll_kv_attention_set_policy), the persistent W4A4 GEMM
+ * (ll_nvfp4_gemm_reserve) and small W4A4 products of few tiles and long K.  That memory is allocated per
+ * (device, stream) by the first launch that needs it and kept.  The first two share one set, grown when a later launch
+ * needs more (which frees the old set and so waits for the device).  Small products have a set of their own that no
+ * recorded launch uses: on a capturing stream, or where the memory cannot be had, one workgroup computes the parts of a
+ * tile one after the other, with the same bits.  ll_release_stream_memory frees the sets of (current device, stream), if
+ * any, after waiting for the launches that still use them - for callers that create streams as they go.  Launches of the
+ * first two kernels on a stream that is being captured into a graph never allocate: they use the set a
  * reserve call or an earlier launch left on that stream, or fall back to a division of the work that needs none.
  * A set that a captured launch has used belongs to the recorded graph as well: it is not freed when the stream
  * later needs a larger one (the old set is kept aside), only by ll_release_stream_memory, which must therefore not
@@ -264,8 +266,8 @@ int ll_nvfp4_gemm_plan(int64_t M, int64_t N, int64_t Kp, int n_products, int com
  * see): *kernel = one of the codes below, *hand_scheduled = 1 if its main loop is the generated instruction sequence.
  * The 128- and 256-row four-wave tile kernels add the K steps in order, and so does every kernel under
  * LL_GEMM_TILES_COMPILED; LL_GEMM_KERNEL_64X64 (each wave a quarter of every K step; where there are few tiles and K is
- * long, several workgroups per tile), LL_GEMM_KERNEL_EIGHT_WAVES and LL_GEMM_KERNEL_PERSISTENT form partial sums over
- * parts of K, added in a fixed order.  Output pointers may be NULL.  No counterpart in the reference. */
+ * long, K ranges that several workgroups share or, on a capturing stream or without memory, one runs through),
+ * LL_GEMM_KERNEL_EIGHT_WAVES and LL_GEMM_KERNEL_PERSISTENT form partial sums over parts of K, added in a fixed order.  Output pointers may be NULL.  No counterpart in the reference. */
 #define LL_GEMM_KERNEL_64X64 0       /* four waves per workgroup, two workgroups per compute unit */
 #define LL_GEMM_KERNEL_128X128 1
 #define LL_GEMM_KERNEL_128X256 2

@@ -174,6 +174,8 @@ inline TileKernelChoice choose_tile_kernel(int64_t M, int64_t N, int64_t Kp, int
 // parts over and adding them up takes 3 us and 0.1 more per part (64 x 512 x 5888: 17.7 us whole, 10.7 in four parts,
 // 10.2 in eight; 128 x 3072 x 14336: 36.4 whole, 23.9 in two, 21.8 in four; 112 x 2944 x 8192: 23.0 whole, 15.6 in four,
 // 18.0 in five; 256 x 3072 x 3072: 11.9 whole, 13.6 in two).  More workgroups than two per unit would run one after the other.
+constexpr int kSmallRecordBytes = 64 * 64 * 4;                            // a part's fp32 sums of its tile
+inline int64_t small_product_units(int cus) { return 2 * (int64_t)cus; }  // most (tile, part) pairs of a launch with parts
 struct SmallGemmPlan {
   int parts;
   int tiles_m, tiles_n_each;
@@ -184,7 +186,7 @@ inline SmallGemmPlan plan_small_gemm(int64_t M, int64_t N, int64_t Kp, int n_pro
   p.tiles = (int64_t)p.tiles_m * p.tiles_n_each * n_products;
   const int64_t steps = (Kp + 255) / 256;
   double best = 0.0;
-  for (int64_t s = 1; s <= 16 && s <= steps && (s == 1 || p.tiles * s <= 2 * cus); ++s) {
+  for (int64_t s = 1; s <= 16 && s <= steps && (s == 1 || p.tiles * s <= small_product_units(cus)); ++s) {
     const double beyond = p.tiles * s <= cus ? 0.0 : (double)(p.tiles * s - cus) / cus;
     const double time = (double)((steps + s - 1) / s) * (0.55 + 0.3 * beyond) + (s > 1 ? 3.0 + 0.1 * (double)s : 0.0);
     if (s == 1 || time < best) {

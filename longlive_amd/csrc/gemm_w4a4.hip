@@ -751,6 +751,7 @@ constexpr int kSmallStage = 2 * (kSmallVals + kSmallScales);
 constexpr int kSmallSmem = kSmallStages * kSmallStage;
 constexpr int kSmallFlag = 4 * 3 * 4096;                      // behind the exchange
 static_assert(kSmallFlag + 16 <= kSmallSmem && 2 * kSmallSmem <= 160 * 1024, "the exchange fits the ring, two workgroups fit a unit");
+constexpr int kSmallWholeSmem = kSmallSmem + kSmallFlag;      // WHOLE: the exchange lies behind the ring, which stays full
 
 // 16 bytes per lane from base + offset straight into LDS at lds_base + IMM + 16 * lane (see load_to_lds_b128).
 template <int IMM>
@@ -759,7 +760,12 @@ __device__ __forceinline__ void load_to_lds_b128_at(const uint8_t* base, uint32_
                : "memory", "scc");
 }
 
-__global__ __launch_bounds__(kSmallThreads, 2) void gemm_w4a4_small_kernel(
+// WHOLE: one workgroup computes all parts of its tile one after the other and adds them up in their order, which gives the
+// bits of `parts` workgroups without the memory that these share.  That memory belongs to a stream, and a recorded launch
+// may be replayed on any stream beside others: two that counted their arrivals in the same words would add up each other's
+// parts.  The loads run on across the parts; what a part costs is its exchange through LDS.
+template <bool WHOLE>
+__global__ __launch_bounds__(kSmallThreads, WHOLE ? 1 : 2) void gemm_w4a4_small_kernel(
     const uint8_t* __restrict__ Av, const uint8_t* __restrict__ As, const uint8_t* __restrict__ Bv0,
     const uint8_t* __restrict__ Bs0, const float* __restrict__ alpha_ptr0, const float* __restrict__ amax_a,
     const float* __restrict__ amax_b0, float inv_denom_a, float inv_denom_b0, int M, int N, int Mp, int Np, int Kp,
@@ -777,10 +783,11 @@ __global__ __launch_bounds__(kSmallThreads, 2) void gemm_w4a4_small_kernel(
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
 
   // Workgroup -> (tile, part of its K range), as in gemm_w4a4_asm8_kernel: every XCD takes a run of consecutive ones.
-  const int total = tiles_m * tiles_n * parts, per_xcd = (int)gridDim.x >> 3;
+  const int wgs_per_tile = WHOLE ? 1 : parts;
+  const int total = tiles_m * tiles_n * wgs_per_tile, per_xcd = (int)gridDim.x >> 3;
   const int unit = ((int)blockIdx.x & 7) * per_xcd + ((int)blockIdx.x >> 3);
   if (unit >= total) return;
-  const int tile = unit / parts, part = unit - tile * parts;
+  const int tile = unit / wgs_per_tile, part = unit - tile * wgs_per_tile;
   int tile_n = tile / tiles_m;
   const int tile_m = tile - tile_n * tiles_m;
   if (groups.n > 1) {
@@ -803,8 +810,9 @@ __global__ __launch_bounds__(kSmallThreads, 2) void gemm_w4a4_small_kernel(
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, lh = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int all_steps = (Kp + kSmallK - 1) / kSmallK;
-  const int t0 = (int)((int64_t)part * all_steps / parts);             // first K step of this part
-  const int nk = (int)((int64_t)(part + 1) * all_steps / parts) - t0;  // at least one: the host sees to it
+  auto first_step = [&](int p) { return (int)((int64_t)p * all_steps / parts); };  // of part p, which has at least one: the host sees to it
+  const int t0 = WHOLE ? 0 : first_step(part);
+  const int nk = WHOLE ? all_steps : first_step(part + 1) - t0;
 
   // ---- global -> LDS: a load instruction covers 1 KB = 8 rows of 128 bytes.  Wave w brings rows 8 w .. and 32 + 8 w .. of
   // A and of B and 1 KB of scales (waves 0, 1: A, tiles 0-1 and 2-3 of the step; waves 2, 3: B).  The tiles of a matrix
@@ -818,7 +826,7 @@ __global__ __launch_bounds__(kSmallThreads, 2) void gemm_w4a4_small_kernel(
   const uint8_t* src[4] = {a_src, a_src + 32 * row_bytes, b_src, b_src + 32 * row_bytes};
   uint32_t voff = (uint32_t)(lane >> 3) * (uint32_t)row_bytes + (uint32_t)piece * 16u, soff = (uint32_t)lane * 16u;
   const uint32_t v_dst = lds_address(smem) + wave * 1024;
-  auto load_step = [&](int step, auto stage) {  // called for the steps in order
+  auto load_step = [&](int step, auto stage) __attribute__((always_inline)) {  // called for the steps in order
     constexpr int kBase = decltype(stage)::value * kSmallStage;
     const int k0 = (t0 + step) * kSmallK;
     if (k0 + kSmallK <= Kp) {
@@ -847,7 +855,7 @@ __global__ __launch_bounds__(kSmallThreads, 2) void gemm_w4a4_small_kernel(
     uint4 v[4];  // fragments A0, A1, B0, B1
     uint32_t sc[4];
   };
-  auto read_raw = [&](Raw& h, auto stage) {
+  auto read_raw = [&](Raw& h, auto stage) __attribute__((always_inline)) {
     constexpr int kBase = decltype(stage)::value * kSmallStage;
 #pragma unroll
     for (int f = 0; f < 4; ++f) {
@@ -869,7 +877,7 @@ __global__ __launch_bounds__(kSmallThreads, 2) void gemm_w4a4_small_kernel(
     for (int i = 0; i < 8; ++i) o[1][f][i] = (_Float16)0.0f;  // the first step's "previous sub-step" adds nothing
   // The four MFMAs of a sub-step with the decode of the next one between them, a fragment (eight instructions) behind
   // each; the scheduling barriers hold that order (left to itself the compiler pairs MFMAs that depend on each other).
-  auto mma_under = [&](half8v (&dst)[4], const Raw& h, const half2v (&s2)[4][2], int j, const half8v (&x)[4]) {
+  auto mma_under = [&](half8v (&dst)[4], const Raw& h, const half2v (&s2)[4][2], int j, const half8v (&x)[4]) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       acc[i >> 1][i & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[2 + (i >> 1)], x[i & 1], acc[i >> 1][i & 1], 0, 0, 0);
@@ -880,16 +888,71 @@ __global__ __launch_bounds__(kSmallThreads, 2) void gemm_w4a4_small_kernel(
     }
   };
   // The wave's five loads of the step that comes next have landed; those of the `behind` steps after it may be under way.
-  auto wait_loads = [&](int behind) {
+  auto wait_loads = [&](int behind) __attribute__((always_inline)) {
     if (behind >= 3) __builtin_amdgcn_s_waitcnt(0x0F7F);       // vmcnt(15)
     else if (behind == 2) __builtin_amdgcn_s_waitcnt(0x0F7A);  // vmcnt(10)
     else if (behind == 1) __builtin_amdgcn_s_waitcnt(0x0F75);  // vmcnt(5)
     else __builtin_amdgcn_s_waitcnt(0x0F70);
   };
+  // The MFMAs of the last sub-step, whose operands are decoded.
+  auto mma_last = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      acc[i >> 1][i & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(o[1][2 + (i >> 1)], o[1][i & 1], acc[i >> 1][i & 1], 0, 0, 0);
+  };
+  // The K quarters of the four waves meet: wave w adds up fragment (g, f) = (w / 2, w % 2), of which the others leave their
+  // parts in LDS.
+  float16v sum[1][1];
+  auto exchange_quarters = [&](float* exchange) __attribute__((always_inline)) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const float16v& a = acc[q >> 1][q & 1];
+      if (q == wave) {
+        sum[0][0] = a;
+      } else {
+        float* dst = exchange + (q * 3 + (wave < q ? wave : wave - 1)) * 1024 + lane * 4;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) *reinterpret_cast<float4*>(dst + i * 256) = make_float4(a[4 * i], a[4 * i + 1], a[4 * i + 2], a[4 * i + 3]);
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float* p = exchange + wave * 3 * 1024 + lane * 4 + i * 256;
+      const float4 x = *reinterpret_cast<const float4*>(p), y = *reinterpret_cast<const float4*>(p + 1024),
+                   z = *reinterpret_cast<const float4*>(p + 2048);
+      const float xs[4] = {x.x, x.y, x.z, x.w}, ys[4] = {y.x, y.y, y.z, y.w}, zs[4] = {z.x, z.y, z.z, z.w};
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {  // x, y, z: the three other waves in order; own part at its place
+        const float m = sum[0][0][4 * i + c];
+        const float s0 = wave == 0 ? m : xs[c], s1 = wave == 1 ? m : (wave == 0 ? xs[c] : ys[c]);
+        const float s2v = wave == 2 ? m : (wave == 3 ? zs[c] : ys[c]), s3 = wave == 3 ? m : zs[c];
+        sum[0][0][4 * i + c] = (s0 + s1) + (s2v + s3);
+      }
+    }
+    __syncthreads();  // the exchange may be written again
+  };
+  // WHOLE: behind the last step of a part.  What the accumulators hold is added to the parts before it, as the workgroup that
+  // arrives last adds them; the next part starts from zeros.
+  float16v all;
+  auto end_part = [&](int p) __attribute__((always_inline)) {
+    mma_last();
+    exchange_quarters(reinterpret_cast<float*>(smem + kSmallSmem));
+#pragma unroll
+    for (int i = 0; i < 16; ++i) all[i] = (p == 0 ? 0.0f : all[i]) + sum[0][0][i];
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[g >> 1][g & 1][i] = 0.0f;
+#pragma unroll
+    for (int f = 0; f < 4; ++f)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) o[1][f][i] = (_Float16)0.0f;
+  };
   // One K step from the packed words in h; the words of the step behind it are read into `next` half way through,
   // when every wave has its loads of that step in LDS and has read this step's stage for the last time (the stage is
   // then refilled with the step four further on), so that neither the barrier nor the LDS latency is waited out.
-  auto step = [&](int t, auto stage, const Raw& h, Raw& next) {
+  auto step = [&](int t, auto stage, const Raw& h, Raw& next) __attribute__((always_inline)) {
     constexpr int kStageNo = decltype(stage)::value;
     half2v s2[4][2];
 #pragma unroll
@@ -921,53 +984,50 @@ __global__ __launch_bounds__(kSmallThreads, 2) void gemm_w4a4_small_kernel(
   __syncthreads();
   Raw h0, h1;
   read_raw(h0, kS0);
-  int t = 0;
+  if constexpr (WHOLE) {
+    for (int t = 0, p = 0, end = first_step(1);;) {
+      switch (t & 3) {  // the stage of step t
+        case 0:
+          step(t, kS0, h0, h1);
+          if (++t == end) break;
+          [[fallthrough]];
+        case 1:
+          step(t, kS1, h1, h0);
+          if (++t == end) break;
+          [[fallthrough]];
+        case 2:
+          step(t, kS2, h0, h1);
+          if (++t == end) break;
+          [[fallthrough]];
+        default:
+          step(t, kS3, h1, h0);
+          if (++t != end) continue;
+      }
+      end_part(p);
+      if (++p == parts) break;
+      end = first_step(p + 1);
+    }
+  } else {
+    int t = 0;
 #pragma unroll 1
-  for (; t + 4 <= nk; t += 4) {
-    step(t, kS0, h0, h1);
-    step(t + 1, kS1, h1, h0);
-    step(t + 2, kS2, h0, h1);
-    step(t + 3, kS3, h1, h0);
-  }
-  if (t < nk) step(t, kS0, h0, h1);
-  if (t + 1 < nk) step(t + 1, kS1, h1, h0);
-  if (t + 2 < nk) step(t + 2, kS2, h0, h1);
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-    acc[i >> 1][i & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(o[1][2 + (i >> 1)], o[1][i & 1], acc[i >> 1][i & 1], 0, 0, 0);
-  __syncthreads();  // every wave has left the ring
-
-  // ---- wave w finishes fragment (g, f) = (w / 2, w % 2): the others leave their parts of it in LDS
-  float* exchange = reinterpret_cast<float*>(smem);
-  float16v sum[1][1];
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const float16v& a = acc[q >> 1][q & 1];
-    if (q == wave) {
-      sum[0][0] = a;
-    } else {
-      float* dst = exchange + (q * 3 + (wave < q ? wave : wave - 1)) * 1024 + lane * 4;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) *reinterpret_cast<float4*>(dst + i * 256) = make_float4(a[4 * i], a[4 * i + 1], a[4 * i + 2], a[4 * i + 3]);
+    for (; t + 4 <= nk; t += 4) {
+      step(t, kS0, h0, h1);
+      step(t + 1, kS1, h1, h0);
+      step(t + 2, kS2, h0, h1);
+      step(t + 3, kS3, h1, h0);
     }
+    if (t < nk) step(t, kS0, h0, h1);
+    if (t + 1 < nk) step(t + 1, kS1, h1, h0);
+    if (t + 2 < nk) step(t + 2, kS2, h0, h1);
   }
-  __syncthreads();
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const float* p = exchange + wave * 3 * 1024 + lane * 4 + i * 256;
-    const float4 x = *reinterpret_cast<const float4*>(p), y = *reinterpret_cast<const float4*>(p + 1024),
-                 z = *reinterpret_cast<const float4*>(p + 2048);
-    const float xs[4] = {x.x, x.y, x.z, x.w}, ys[4] = {y.x, y.y, y.z, y.w}, zs[4] = {z.x, z.y, z.z, z.w};
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {  // x, y, z: the three other waves in order; own part at its place
-      const float m = sum[0][0][4 * i + c];
-      const float s0 = wave == 0 ? m : xs[c], s1 = wave == 1 ? m : (wave == 0 ? xs[c] : ys[c]);
-      const float s2v = wave == 2 ? m : (wave == 3 ? zs[c] : ys[c]), s3 = wave == 3 ? m : zs[c];
-      sum[0][0][4 * i + c] = (s0 + s1) + (s2v + s3);
-    }
+  if constexpr (WHOLE) {
+    sum[0][0] = all;  // end_part has left the ring and the exchange behind a barrier
+  } else {
+    mma_last();
+    __syncthreads();  // every wave has left the ring, which the exchange and then the patches of the epilogue take
+    exchange_quarters(reinterpret_cast<float*>(smem));
   }
-  __syncthreads();  // the patches of the epilogue overlap the exchange
-  if (parts > 1) {
+  if (!WHOLE && parts > 1) {
     // Part of a tile: the workgroup that arrives last adds the parts up in the order of their K ranges, so the sum does
     // not depend on who that is; the others leave theirs in a record.  Same protocol as in the persistent kernel:
     // device-scope stores, every wave waits for its own, then the barrier, then thread 0 counts the arrival.
@@ -991,7 +1051,6 @@ __global__ __launch_bounds__(kSmallThreads, 2) void gemm_w4a4_small_kernel(
     }
     if (!last) return;
     if (tid == 0) __hip_atomic_store(arrivals + tile, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // ready for the next launch
-    float16v all;
 #pragma unroll
     for (int i = 0; i < 16; ++i) all[i] = 0.0f;
     for (int p0 = 0; p0 < parts; p0 += 4) {  // sixteen loads in flight
@@ -1446,7 +1505,6 @@ extern "C" int ll_nvfp4_gemm_tnt_fused(const uint8_t* A_values, const uint8_t* A
 
 namespace ll {
 
-inline size_t small_record_bytes(const SmallGemmPlan& p) { return (size_t)p.tiles * p.parts * 64 * 64 * sizeof(float); }
 inline size_t persistent_record_bytes(const GemmDivision& d) { return (size_t)2 * d.G * kPRecordFloats * sizeof(float); }
 
 // Launches the persistent kernel if the plan says so and its memory is at hand; *launched tells.
@@ -1528,22 +1586,24 @@ int dispatch_gemm(const uint8_t* A_values, const uint8_t* A_scales, const uint8_
     return LL_OK;
   }
   if (choice.kernel == LL_GEMM_KERNEL_64X64 && g_gemm_schedule.load(std::memory_order_relaxed) != LL_GEMM_TILES_COMPILED) {
-    SmallGemmPlan plan = plan_small_gemm(M, N, Kp, groups.n, cus);
-    StreamScratch w;
-    if (plan.parts > 1) {
-      bool missing = false;
-      if (int rc = stream_scratch(dev, s, small_record_bytes(plan), (size_t)plan.tiles, !stream_is_capturing(s), w, &missing,
-                                  "ll_nvfp4_gemm_tnt")) return rc;
-      if (missing) plan.parts = 1;  // a capturing stream without the memory: one workgroup per tile, which needs none
-    }
+    const SmallGemmPlan plan = plan_small_gemm(M, N, Kp, groups.n, cus);
     GemmGroups gr = groups;
     gr.tiles_n_each = plan.tiles_n_each;
-    static std::atomic<uint64_t> lds_allowed{0};
-    if (int rc = allow_dynamic_lds(reinterpret_cast<const void*>(&gemm_w4a4_small_kernel), kSmallSmem, lds_allowed, "ll_nvfp4_gemm_tnt")) return rc;
-    hipLaunchKernelGGL(gemm_w4a4_small_kernel, dim3((unsigned)((plan.tiles * plan.parts + 7) / 8 * 8)), dim3(kSmallThreads), kSmallSmem, s,
-                       A_values, A_scales, B_values, B_scales, alpha, amax_a, amax_b, 1.0f / denom_a, 1.0f / denom_b, (int)M, (int)N,
-                       (int)Mp, (int)Np, (int)Kp, static_cast<uint16_t*>(D), ldd, plan.tiles_m, plan.tiles_n_each * gr.n, epi, gr,
-                       plan.parts, reinterpret_cast<float*>(w.records), w.counters);
+#define LL_SMALL_LAUNCH(WHOLE, wgs, lds, records, arrivals)                                                                    \
+  hipLaunchKernelGGL(gemm_w4a4_small_kernel<WHOLE>, dim3((unsigned)(((wgs) + 7) / 8 * 8)), dim3(kSmallThreads), lds, s, A_values, A_scales, \
+                     B_values, B_scales, alpha, amax_a, amax_b, 1.0f / denom_a, 1.0f / denom_b, (int)M, (int)N, (int)Mp, (int)Np, (int)Kp, \
+                     static_cast<uint16_t*>(D), ldd, plan.tiles_m, plan.tiles_n_each * gr.n, epi, gr, plan.parts, records, arrivals)
+    StreamScratch w;
+    if (plan.parts > 1 && !small_product_scratch(dev, s, cus, w)) {
+      static std::atomic<uint64_t> lds_allowed{0};
+      if (int rc = allow_dynamic_lds(reinterpret_cast<const void*>(&gemm_w4a4_small_kernel<true>), kSmallWholeSmem, lds_allowed, "ll_nvfp4_gemm_tnt")) return rc;
+      LL_SMALL_LAUNCH(true, plan.tiles, kSmallWholeSmem, nullptr, nullptr);
+    } else {
+      static std::atomic<uint64_t> lds_allowed{0};
+      if (int rc = allow_dynamic_lds(reinterpret_cast<const void*>(&gemm_w4a4_small_kernel<false>), kSmallSmem, lds_allowed, "ll_nvfp4_gemm_tnt")) return rc;
+      LL_SMALL_LAUNCH(false, plan.tiles * plan.parts, kSmallSmem, reinterpret_cast<float*>(w.records), w.counters);
+    }
+#undef LL_SMALL_LAUNCH
     LL_CHECK_LAUNCH("gemm_w4a4_small_kernel");
     return LL_OK;
   }
@@ -1657,24 +1717,13 @@ extern "C" int ll_nvfp4_gemm_reserve(int64_t M, int64_t N, int64_t Kp, int n_pro
     return LL_ELAUNCH;
   }
   if (int rc = compute_units_of(dev, cus, "ll_nvfp4_gemm_reserve")) return rc;
-  const int schedule = g_gemm_schedule.load(std::memory_order_relaxed);
-  size_t bytes = 0, counters = 0;
-  if (const PersistentPlan plan = plan_persistent(M, N, Kp, n_products, cus, schedule); plan.use) {
-    bytes = persistent_record_bytes(plan.d);
-    counters = gemm_split_tiles(plan.d);
-  } else if (schedule != LL_GEMM_TILES_COMPILED && choose_tile_kernel(M, N, Kp, n_products, cus, schedule).kernel == LL_GEMM_KERNEL_64X64) {
-    const SmallGemmPlan small = plan_small_gemm(M, N, Kp, n_products, cus);
-    if (small.parts > 1) {
-      bytes = small_record_bytes(small);
-      counters = (size_t)small.tiles;
-    }
-  }
-  if (bytes == 0) return LL_OK;
+  const PersistentPlan plan = plan_persistent(M, N, Kp, n_products, cus, g_gemm_schedule.load(std::memory_order_relaxed));
+  if (!plan.use) return LL_OK;
   if (stream_is_capturing(static_cast<hipStream_t>(stream))) {
     set_error("ll_nvfp4_gemm_reserve: the stream is being captured; reserve before the recording starts");
     return LL_ENOSUP;
   }
   StreamScratch w;
-  return stream_scratch(dev, static_cast<hipStream_t>(stream), bytes, counters, true, w, nullptr,
+  return stream_scratch(dev, static_cast<hipStream_t>(stream), persistent_record_bytes(plan.d), gemm_split_tiles(plan.d), true, w, nullptr,
                         "ll_nvfp4_gemm_reserve");
 }

@@ -44,6 +44,9 @@ struct StreamScratch {
 // a graph): only a set that is already large enough is handed out, and *missing says that there is none.
 int stream_scratch(int dev, hipStream_t stream, size_t record_bytes, size_t counters, bool may_allocate, StreamScratch& out,
                    bool* missing, const char* what);
+// The records and counters of the small products of a stream; false where there is none to be had (the stream is being
+// captured, the allocation fails): no error, the launch then takes its way without memory.
+bool small_product_scratch(int dev, hipStream_t stream, int cus, StreamScratch& out);
 int release_stream_scratch(int dev, hipStream_t stream);
 // Whether work submitted to `stream` is being recorded into a graph instead of run.  A failing query (the legacy
 // stream while another stream of the thread captures) counts as recording: then nothing may be allocated either.

@@ -1,6 +1,6 @@
 // Device memory of the library's own: the records through which workgroups of one launch hand partial tiles to each
-// other (the split division of the attention kernel, the K-split shares of the persistent GEMM) and the arrival
-// counters that go with them.  One set per (device, stream): launches on one stream run one after the other and can
+// other (the split division of the attention kernel, the K-split shares of the persistent GEMM, the K ranges of small
+// products) and the arrival counters that go with them.  One set per (device, stream): launches on one stream run one after the other and can
 // share it, launches on different streams get different sets.  A set is created at the first launch that needs one,
 // grown when a later launch needs more, and kept until ll_release_stream_memory or the end of the process.  The
 // counters are zero whenever no launch is running: every kernel that uses them leaves them at zero.
@@ -9,6 +9,7 @@
 #include <vector>
 
 #include "ll_common.h"
+#include "gemm_split.h"
 
 namespace ll {
 
@@ -21,6 +22,11 @@ struct ScratchEntry {
 };
 static std::mutex g_scratch_mutex;
 static std::map<std::pair<int, hipStream_t>, ScratchEntry> g_scratch;
+
+// The memory of small products (gemm_w4a4_small_kernel) is a set of its own: launches of the other kernels that are
+// recorded keep using the set above at every replay, on whatever stream that is, and an ordinary linear layer beside
+// them must not meet them there.  No recorded launch uses this one.  One size holds every small product, so it never grows.
+static std::map<std::pair<int, hipStream_t>, StreamScratch> g_small_scratch;
 
 static void free_scratch(StreamScratch& w) {
   if (w.records) (void)hipFree(w.records);  // waits for the launches that still use it
@@ -72,8 +78,37 @@ int stream_scratch(int dev, hipStream_t stream, size_t record_bytes, size_t coun
   return LL_OK;
 }
 
+bool small_product_scratch(int dev, hipStream_t stream, int cus, StreamScratch& out) {
+  if (stream_is_capturing(stream)) return false;
+  std::lock_guard<std::mutex> lock(g_scratch_mutex);
+  StreamScratch& w = g_small_scratch[{dev, stream}];
+  if (!w.records) {
+    w.record_bytes = (size_t)small_product_units(cus) * kSmallRecordBytes;
+    w.n_counters = (size_t)small_product_units(cus);
+    // an allocation is refused, and a recording elsewhere spoilt, while another stream is captured in the global mode
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    const bool exchanged = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+    hipError_t e = hipMalloc(reinterpret_cast<void**>(&w.records), w.record_bytes);
+    if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void**>(&w.counters), w.n_counters * sizeof(int));
+    if (e == hipSuccess) e = hipMemsetAsync(w.counters, 0, w.n_counters * sizeof(int), stream);
+    if (e != hipSuccess) free_scratch(w);
+    if (exchanged) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (e != hipSuccess) {
+      (void)hipGetLastError();  // the caller has a way without the memory
+      g_small_scratch.erase({dev, stream});
+      return false;
+    }
+  }
+  out = w;
+  return true;
+}
+
 int release_stream_scratch(int dev, hipStream_t stream) {
   std::lock_guard<std::mutex> lock(g_scratch_mutex);
+  if (const auto small = g_small_scratch.find({dev, stream}); small != g_small_scratch.end()) {
+    free_scratch(small->second);
+    g_small_scratch.erase(small);
+  }
   const auto it = g_scratch.find({dev, stream});
   if (it == g_scratch.end()) return LL_OK;
   free_scratch(it->second.current);

@@ -703,7 +703,8 @@ def test_small_products_with_k_shared_between_waves_and_workgroups(gpu, M, N, K,
     """The small-product kernel (64 x 64 tiles, every wave a quarter of each K step, the K range of few tiles shared
     between workgroups) adds the exact products in another order than the compiled tile kernel: within one bf16 ulp of
     the fp32 sum of it (fp32 sums of up to 2^14 exact products of unit-scale data differ by far less than a bf16 step),
-    twice for identical bits, and recorded into a graph, with and without the memory its parts pass through."""
+    twice for identical bits, and recorded into a graph for the same bits, on a stream that has run it before and on one
+    that has not."""
     cfg = QuantizationConfig(scale_rule="mse")
     xq = quantize_to_fp4(activations((M, K), 25).to(gpu), cfg)
     ws = [quantize_to_fp4((weights((N, K), 26 + i) * (1 + i)).to(gpu), cfg) for i in range(groups)]
@@ -721,12 +722,12 @@ def test_small_products_with_k_shared_between_waves_and_workgroups(gpu, M, N, K,
     for a, b, c in zip(got, again, want):
         assert torch.equal(a, b)
         _ulp_close(a, c, frac=5e-3)
-    for reserve in (False, True):
+    for warm in (False, True):
         side = torch.cuda.Stream(device=gpu)
         side.wait_stream(torch.cuda.current_stream())
-        if reserve:
+        if warm:
             with torch.cuda.stream(side):
-                _native.gemm_reserve(M, N, xq.padded_shape[1], groups)
+                run()
             side.synchronize()
         graph = torch.cuda.CUDAGraph()
         with torch.cuda.graph(graph, stream=side):
@@ -736,11 +737,67 @@ def test_small_products_with_k_shared_between_waves_and_workgroups(gpu, M, N, K,
                 y.zero_()
             graph.replay()
             torch.cuda.synchronize()
-            for a, b in zip(out, got):
-                if reserve:
-                    assert torch.equal(a, b)
-                else:
-                    _ulp_close(a, b, frac=5e-3)
+            assert all(torch.equal(a, b) for a, b in zip(out, got))
             run()
         with torch.cuda.stream(side):
             _native.release_stream_memory()
+
+
+def test_recorded_small_products_replayed_at_the_same_time(gpu):
+    """Products whose K range several workgroups share, recorded twice on one stream that has run them before and replayed
+    on two streams beside the same work on the recording stream: every result has the bits of the launch by itself."""
+    cfg = QuantizationConfig(scale_rule="mse")
+    sizes = [(48, 512, 4096), (40, 256, 5888), (64, 3072, 3072)]
+    ops = [[quantize_to_fp4((activations if i == 0 else weights)(s, 61 + i).to(gpu), cfg) for i, s in enumerate(((M, K), (N, K)))]
+           for M, N, K in sizes]
+
+    def run():
+        return [fp4_matmul(x, w) for x, w in ops]
+
+    want = run()
+    side, others = torch.cuda.Stream(device=gpu), [torch.cuda.Stream(device=gpu) for _ in range(2)]
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        run()
+    side.synchronize()
+    graphs, outs = [], []
+    for _ in others:
+        graphs.append(torch.cuda.CUDAGraph())
+        with torch.cuda.graph(graphs[-1], stream=side):
+            outs.append(run())
+    for _ in range(20):
+        for y in outs[0] + outs[1]:
+            y.zero_()
+        torch.cuda.synchronize()
+        for graph, stream in zip(graphs, others):
+            with torch.cuda.stream(stream):
+                graph.replay()
+        with torch.cuda.stream(side):
+            eager = run()
+        torch.cuda.synchronize()
+        for got in (*outs, eager):
+            assert all(torch.equal(a, b) for a, b in zip(got, want))
+    with torch.cuda.stream(side):
+        _native.release_stream_memory()
+
+
+def test_small_product_while_another_stream_is_being_captured(gpu):
+    """A product whose parts need memory, run for the first time on its stream while another stream is captured in the
+    global mode (in which an allocation is refused and spoils the recording): same bits, and the recording goes on."""
+    cfg = QuantizationConfig(scale_rule="mse")
+    M, N, K = 40, 256, 5888
+    x, w = quantize_to_fp4(activations((M, K), 71).to(gpu), cfg), quantize_to_fp4(weights((N, K), 72).to(gpu), cfg)
+    want, got = fp4_matmul(x, w), torch.empty((M, N), dtype=torch.bfloat16, device=gpu)   # torch's allocator stays out of it
+    side, other, y = torch.cuda.Stream(device=gpu), torch.cuda.Stream(device=gpu), torch.zeros(8, device=gpu)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        y.add_(1.0)
+        with torch.cuda.stream(other):
+            _native.gemm(x.values, x.scale_factors, w.values, w.scale_factors, M, N, amax_a=x.amax, amax_b=w.amax, out=got)
+        y.add_(1.0)
+    graph.replay()
+    torch.cuda.synchronize()
+    assert torch.equal(got, want) and y.tolist() == [2.0] * 8
+    with torch.cuda.stream(other):
+        _native.release_stream_memory()

@@ -211,8 +211,9 @@ int ll_nvfp4_gemm_tnt_fused(const uint8_t* A_values, const uint8_t* A_scales, co
  * Several ll_nvfp4_gemm_tnt products with the same A operand and the same N and Kp in one launch: the q, k and v
  * projections of one activation (wan_5b/modules/causal_model.py:363-365) and the k, v projections of the text
  * (:234-235), three resp. two fp4_matmul calls in the reference.  Each product has its own weight, scales, tensor
- * scale, bias, output and amax sink (bias and sink optional, as in ll_gemm_epilogue); product i computes exactly
- * what ll_nvfp4_gemm_tnt_fused computes for it alone, bit for bit.  1 <= n_products <= 4.
+ * scale, bias, output and amax sink (bias and sink optional, as in ll_gemm_epilogue); product i computes
+ * what ll_nvfp4_gemm_tnt_fused computes for it alone up to the order of the fp32 additions (the number of products has a
+ * part in the choice of the kernel; ll_nvfp4_gemm_kernel), bit for bit under LL_GEMM_TILES_COMPILED.  1 <= n_products <= 4.
  */
 typedef struct ll_gemm_product {
   const uint8_t* B_values;

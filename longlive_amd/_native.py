@@ -521,7 +521,8 @@ def gemm_grouped(a_values, a_scales, amax_a, denom_a: float, M: int, N: int, pro
     """Several products ``A @ B_i^T`` with the same A operand and the same N and K in one launch
     (ll_nvfp4_gemm_tnt_grouped).  ``products``: one dict per product with ``values``, ``scales``, ``amax``,
     ``denom`` and optionally ``bias`` and ``amax_out`` (an :class:`AmaxTicket`).  Each output equals what
-    :func:`gemm` returns for that product alone, bit for bit."""
+    :func:`gemm` returns for that product alone up to the order of the fp32 additions (the number of products has a part
+    in the choice of the kernel), bit for bit under ``gemm_schedule("tiles_compiled")``."""
     Mp, Kb = a_values.shape
     sinks = [pr["amax_out"].parts.data_ptr() for pr in products if pr.get("amax_out") is not None]
     if len(set(sinks)) != len(sinks):

@@ -170,10 +170,23 @@ inline TileKernelChoice choose_tile_kernel(int64_t M, int64_t N, int64_t Kp, int
 }
 
 // How the small-product kernel divides a launch: 64 x 64 tiles, each by `parts` workgroups that share its K range (steps of
-// 256 elements).  Measured: a step takes 0.55 us with one workgroup on every compute unit and 0.85 with two; handing the
-// parts over and adding them up takes 3 us and 0.1 more per part (64 x 512 x 5888: 17.7 us whole, 10.7 in four parts,
-// 10.2 in eight; 128 x 3072 x 14336: 36.4 whole, 23.9 in two, 21.8 in four; 112 x 2944 x 8192: 23.0 whole, 15.6 in four,
-// 18.0 in five; 256 x 3072 x 3072: 11.9 whole, 13.6 in two).  More workgroups than two per unit would run one after the other.
+// 256 elements).  Measured: a step takes 0.55 us with one workgroup on every compute unit; handing two to four parts over
+// and adding them up takes 2.4 us (their records are read four at a time: five to eight 3.6); with more workgroups than
+// units a step takes 0.8 and the launch 2 us more.  us by parts:
+//                     tiles, steps    1     2     3     4     5     6     8    12
+//   40 x 256 x 5888       4, 23     17.6  13.9  11.8  10.7  11.0  10.9  10.0  10.6
+//   48 x 1024 x 4096     16, 16     13.7  12.0  10.8  10.2  11.8  10.3  10.8  11.9
+//   64 x 1536 x 6912     24, 27     19.6  15.2  12.9  11.5  12.0  11.7  13.9  16.0
+//   130 x 1024 x 4096    48, 16     13.7  12.3  11.1  10.8  11.9  12.7  15.7
+//   112 x 2944 x 8192    92, 32     22.8  17.1  17.0  15.3  17.7
+//   128 x 3072 x 14336   96, 56     35.9  24.1  24.8  21.8  21.7
+//   64 x 3072 x 3072     48, 12     11.5  11.2  10.5  10.1  10.5  12.8  13.3
+//   368 x 768 x 3456     72, 14     12.6  11.9  11.1  13.9  14.7  14.3
+//   300 x 1024 x 3072    80, 12     11.5  11.5  10.9  12.8  14.3  16.5
+//   256 x 3072 x 3072   192, 12     11.9  13.6
+// More than four parts gain half a microsecond at most, and below sixteen steps parts gain about one, which is less than what
+// they cost a recorded launch (gemm_w4a4_small_kernel<true>).
+constexpr int kSmallParts = 4, kSmallPartsSteps = 16;
 constexpr int kSmallRecordBytes = 64 * 64 * 4;                            // a part's fp32 sums of its tile
 inline int64_t small_product_units(int cus) { return 2 * (int64_t)cus; }  // most (tile, part) pairs of a launch with parts
 struct SmallGemmPlan {
@@ -185,10 +198,11 @@ inline SmallGemmPlan plan_small_gemm(int64_t M, int64_t N, int64_t Kp, int n_pro
   SmallGemmPlan p{1, (int)((M + 63) / 64), (int)((N + 63) / 64), 0};
   p.tiles = (int64_t)p.tiles_m * p.tiles_n_each * n_products;
   const int64_t steps = (Kp + 255) / 256;
+  if (steps < kSmallPartsSteps) return p;
   double best = 0.0;
-  for (int64_t s = 1; s <= 16 && s <= steps && (s == 1 || p.tiles * s <= small_product_units(cus)); ++s) {
-    const double beyond = p.tiles * s <= cus ? 0.0 : (double)(p.tiles * s - cus) / cus;
-    const double time = (double)((steps + s - 1) / s) * (0.55 + 0.3 * beyond) + (s > 1 ? 3.0 + 0.1 * (double)s : 0.0);
+  for (int64_t s = 1; s <= kSmallParts && (s == 1 || p.tiles * s <= small_product_units(cus)); ++s) {
+    const bool beyond = p.tiles * s > cus;
+    const double time = (double)((steps + s - 1) / s) * (beyond ? 0.8 : 0.55) + (s > 1 ? 2.4 : 0.0) + (beyond ? 2.0 : 0.0);
     if (s == 1 || time < best) {
       best = time;
       p.parts = (int)s;

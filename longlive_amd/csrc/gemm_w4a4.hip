@@ -763,7 +763,9 @@ __device__ __forceinline__ void load_to_lds_b128_at(const uint8_t* base, uint32_
 // WHOLE: one workgroup computes all parts of its tile one after the other and adds them up in their order, which gives the
 // bits of `parts` workgroups without the memory that these share.  That memory belongs to a stream, and a recorded launch
 // may be replayed on any stream beside others: two that counted their arrivals in the same words would add up each other's
-// parts.  The loads run on across the parts; what a part costs is its exchange through LDS.
+// parts.  The loads run on across the parts; what a part costs is its exchange through LDS, 2 us.  Four parts (the workgroups
+// that share them / one for all / the 64 x 64 tile kernel above): 64 x 512 x 5888 10.6 / 24.2 / 25.5 us, 112 x 2944 x 8192 15.3 /
+// 28.6 / 34.7, 128 x 3072 x 14336 21.8 / 41.8 / 58.3, 48 x 1024 x 4096 10.2 / 20.1 / 18.7.
 template <bool WHOLE>
 __global__ __launch_bounds__(kSmallThreads, WHOLE ? 1 : 2) void gemm_w4a4_small_kernel(
     const uint8_t* __restrict__ Av, const uint8_t* __restrict__ As, const uint8_t* __restrict__ Bv0,

@@ -129,3 +129,7 @@ extern "C" void ll_test_gemm_plan(int64_t M, int64_t N, int64_t Kp, int n_produc
   out[5] = (uint32_t)plan.tiles_m;
   out[6] = (uint32_t)plan.tiles_n_each;
 }
+// How a small product is divided: workgroups that share a tile's K range.
+extern "C" int ll_test_small_gemm_parts(int64_t M, int64_t N, int64_t Kp, int n_products, int cus) {
+  return ll::plan_small_gemm(M, N, Kp, n_products, cus).parts;
+}

@@ -180,9 +180,9 @@ class FourOverSixLinear(nn.Linear):
     @staticmethod
     def forward_quantized_together(layers, xq: QuantizedTensor, amax_outs=None) -> list[torch.Tensor]:
         """``[m.forward_quantized(xq) for m in layers]`` as one GEMM launch when the layers have the same shape
-        (the q / k / v projections of an attention layer): the products are computed exactly as they would be
-        alone, only the cost of two launches and of two half-empty rounds of workgroups is saved.  ``amax_outs``:
-        one amax ticket or ``None`` per layer."""
+        (the q / k / v projections of an attention layer): the products are those of the single launches up to the
+        order of the fp32 additions (:func:`_native.gemm_grouped`), only the cost of two launches and of two half-empty
+        rounds of workgroups is saved.  ``amax_outs``: one amax ticket or ``None`` per layer."""
         amax_outs = amax_outs or [None] * len(layers)
         weights = [m.quantized_weight() for m in layers]
         same = (1 < len(layers) <= 4 and all(isinstance(w, QuantizedTensor) for w in weights)

@@ -181,6 +181,16 @@ def gemm_plan(M: int, N: int, Kp: int, n_products: int = 1, cus: int = 256, sche
     return dict(use=bool(out[0]), G=out[1], tiles=out[2], nk=out[3], whole_rounds=out[4], tiles_m=out[5], tiles_n_each=out[6])
 
 
+def small_gemm_parts(M: int, N: int, Kp: int, n_products: int = 1, cus: int = 256) -> int:
+    """Workgroups that share the K range of a tile of a small product (longlive_amd/csrc/gemm_split.h)."""
+    import ctypes
+
+    lib = _test_hooks()
+    lib.ll_test_small_gemm_parts.restype = ctypes.c_int
+    lib.ll_test_small_gemm_parts.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, ctypes.c_int, ctypes.c_int]
+    return lib.ll_test_small_gemm_parts(M, N, Kp, n_products, cus)
+
+
 def gemm_segments(division: dict, g: int):
     """The (tile, begin, end) segments workgroup g of the persistent GEMM walks, in order."""
     import ctypes

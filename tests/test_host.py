@@ -1,5 +1,7 @@
 """CPU tests of the host side: the C-ABI library loads and exports every declared symbol, the
 configuration / front-end error behaviour mirrors the reference, module swap and cache policy."""
+import itertools
+
 import numpy as np
 import pytest
 import torch
@@ -504,3 +506,21 @@ def test_which_gemm_kernel_the_shapes_of_the_block_take():
     assert k(2640, 3072, 3072, compute_units=128)["kernel"] != "eight_waves"   # 252 tiles on 128 units
     with pytest.raises(Exception):
         k(0, 3072, 3072)
+
+
+@pytest.mark.parametrize("M,N,K,products,parts", [
+    (64, 512, 5888, 1, 4), (48, 1024, 4096, 1, 4), (128, 3072, 14336, 1, 4), (112, 2944, 8192, 1, 4),   # few tiles, long K
+    (300, 1024, 3072, 1, 1), (368, 768, 3456, 1, 1), (64, 3072, 3072, 1, 1), (48, 512, 2048, 1, 1),     # K too short
+    (512, 3072, 14336, 1, 1), (300, 1024, 4096, 2, 1), (130, 1024, 3841, 1, 4), (130, 1024, 3840, 1, 1),
+])
+def test_parts_of_small_products(M, N, K, products, parts):
+    """How many workgroups share a tile's K range (measured at each of the first eight shapes)."""
+    from helpers import small_gemm_parts
+    assert small_gemm_parts(M, N, K, products) == parts
+
+
+def test_parts_of_small_products_fit_their_memory():
+    from helpers import small_gemm_parts
+    for cus, M, N, K, products in itertools.product((1, 64, 256, 304), (1, 64, 65, 500), (8, 640, 3072), (64, 3840, 4096, 20000), (1, 3)):
+        parts, tiles = small_gemm_parts(M, N, K, products, cus), -(-M // 64) * -(-N // 64) * products
+        assert 1 <= parts <= 4 and parts <= -(-K // 256) and (parts == 1 or tiles * parts <= 2 * cus)

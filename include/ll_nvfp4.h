@@ -266,7 +266,7 @@ int ll_nvfp4_gemm_plan(int64_t M, int64_t N, int64_t Kp, int n_products, int com
  * only; a persistent launch on a capturing stream without memory falls back to the tile kernels, which this does not
  * see): *kernel = one of the codes below, *hand_scheduled = 1 if its main loop is the generated instruction sequence.
  * The 128- and 256-row four-wave tile kernels add the K steps in order, and so does every kernel under
- * LL_GEMM_TILES_COMPILED; LL_GEMM_KERNEL_64X64 (each wave a quarter of every K step; where there are few tiles and K is
+ * LL_GEMM_TILES_COMPILED; LL_GEMM_KERNEL_64X64 for Kp > 1024 (each wave a quarter of every K step; where there are few tiles and K is
  * long, K ranges that several workgroups share or, on a capturing stream or without memory, one runs through),
  * LL_GEMM_KERNEL_EIGHT_WAVES and LL_GEMM_KERNEL_PERSISTENT form partial sums over parts of K, added in a fixed order.  Output pointers may be NULL.  No counterpart in the reference. */
 #define LL_GEMM_KERNEL_64X64 0       /* four waves per workgroup, two workgroups per compute unit */

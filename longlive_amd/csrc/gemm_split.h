@@ -169,6 +169,15 @@ inline TileKernelChoice choose_tile_kernel(int64_t M, int64_t N, int64_t Kp, int
   return {best, generated_ok && best >= 2};
 }
 
+// Which kernel runs the 64 x 64 tiles (LL_GEMM_KERNEL_64X64): gemm_w4a4_small_kernel from five K steps of 256 on, else the tile
+// kernel, which has less to do before the first step and behind the last.  us, small kernel / tile kernel, by K:
+//   tiles       256          512          768          1024         1536         3072
+//     8     5.31 / 4.01  5.80 / 4.92  6.34 / 5.91  7.17 / 6.87  8.19 / 8.81  11.5 / 14.8
+//    72     5.43 / 3.92  5.90 / 4.82  6.45 / 5.78  7.29 / 6.74  8.28 / 8.68  11.7 / 14.6
+//   384     6.38 / 5.22  7.37 / 6.70  8.70 / 8.41  9.97 / 9.80  11.7 / 12.7  17.4 / 21.7
+// It addresses eight rows of Kp / 2 bytes with 32-bit offsets.
+inline bool small_kernel_takes(int64_t Kp, int schedule) { return Kp > 1024 && Kp < (1 << 28) && schedule != 2 /* LL_GEMM_TILES_COMPILED */; }
+
 // How the small-product kernel divides a launch: 64 x 64 tiles, each by `parts` workgroups that share its K range (steps of
 // 256 elements).  Measured: a step takes 0.55 us with one workgroup on every compute unit; handing two to four parts over
 // and adding them up takes 2.4 us (their records are read four at a time: five to eight 3.6); with more workgroups than

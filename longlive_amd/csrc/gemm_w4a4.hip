@@ -738,9 +738,8 @@ __global__ __launch_bounds__(256) void gemm_w4a4_persistent_kernel(PersistentPar
 // the other waves' parts of it, always in the order of the K quarters, from LDS.  Where there are few tiles and K is
 // long, several workgroups share the K range of a tile (plan_small_gemm).
 // Measured (this kernel / the 64 x 64 tile kernel above): 512 x 3072 x 3072 16.6 / 21.8 us, 128 x 3072 x 14336 21.8 / 58.1 us
-// (four parts), 64 x 512 x 5888 10.7 / 25.3 us (four parts), 736 x 1536 x 8960 35.2 / 56.2 us; a single K step (48 x 512 x
-// 256) 5.5 / 5.3 us, which is the launch.  The kernel above keeps this tile for LL_GEMM_TILES_COMPILED (one order of
-// summation for every shape).
+// (four parts), 64 x 512 x 5888 10.7 / 25.3 us (four parts), 736 x 1536 x 8960 35.2 / 56.2 us.  The kernel above keeps
+// short contractions (small_kernel_takes) and LL_GEMM_TILES_COMPILED (one order of summation for every shape).
 constexpr int kSmallThreads = 256;
 constexpr int kSmallStages = 4;
 constexpr int kSmallK = 256;                                  // K elements per step: 64 per wave
@@ -1587,7 +1586,7 @@ int dispatch_gemm(const uint8_t* A_values, const uint8_t* A_scales, const uint8_
     LL_CHECK_LAUNCH("gemm_w4a4_asm8_kernel");
     return LL_OK;
   }
-  if (choice.kernel == LL_GEMM_KERNEL_64X64 && g_gemm_schedule.load(std::memory_order_relaxed) != LL_GEMM_TILES_COMPILED) {
+  if (choice.kernel == LL_GEMM_KERNEL_64X64 && small_kernel_takes(Kp, g_gemm_schedule.load(std::memory_order_relaxed))) {
     const SmallGemmPlan plan = plan_small_gemm(M, N, Kp, groups.n, cus);
     GemmGroups gr = groups;
     gr.tiles_n_each = plan.tiles_n_each;

@@ -695,6 +695,9 @@ def test_native_linear_call_equals_the_separate_operations(gpu, view):
     (63, 65, 192, 1),         # ragged both ways, one partial K step
     (64, 64, 256, 2),         # one tile and one whole step per product
     (65, 200, 320, 1),        # a second row of tiles with one row, a step and a quarter
+    (64, 64, 1024, 2),        # the longest K that adds the steps in order
+    (63, 65, 1088, 1),        # ragged both ways, a step that is three quarters zeros
+    (64, 64, 1280, 2),        # one tile and five whole steps per product
     (130, 136, 1088, 3),      # five steps, the last a quarter; three products
     (40, 256, 5888, 1),       # few tiles, long K: several workgroups share a tile's K range
     (100, 72, 14400, 2),      # the same with a ragged last step and two products

@@ -228,6 +228,16 @@ def _device_key(device: torch.device):
     return (device.type, index)
 
 
+def recording(device: torch.device) -> bool:
+    """Whether launches on the device's current stream are being recorded into a graph."""
+    if device.type != "cuda":
+        return False
+    if device.index is None or device.index == torch.cuda.current_device():
+        return torch.cuda.is_current_stream_capturing()
+    with torch.cuda.device(device):
+        return torch.cuda.is_current_stream_capturing()
+
+
 class PrivateAmaxSink:
     """An amax sink buffer of its own for one producer / consumer pair whose two ends lie far apart in the launch
     sequence (the K and V of a chunk are produced early in a forward and quantized into the cache after it): the
@@ -242,7 +252,7 @@ class PrivateAmaxSink:
         all its producers, whose slots the next producer overwrites, and no place for a maximum that is consumed
         after the forward.  Without a ticket the producer leaves nothing behind and the consumer reduces the tensor
         itself."""
-        if _device_key(self.parts.device) in _active_graph_sinks:
+        if _device_key(self.parts.device) in _active_graph_sinks or recording(self.parts.device):
             return None
         if self.entry[1] >= 0xFFFFFFFE:
             self.parts.zero_()
@@ -292,8 +302,10 @@ class ReplayableAmaxSink:
         return AmaxTicket(self.parts, self.entry[1], self.entry, self.offset)
 
 
-def amax_ticket(device: torch.device) -> AmaxTicket:
-    """A fresh epoch on the device's amax sink buffer.  Epochs only grow, which is what lets the buffer go
+def amax_ticket(device: torch.device) -> AmaxTicket | None:
+    """A fresh epoch on the device's amax sink buffer, or None while launches are being recorded into a graph without a
+    :class:`ReplayableAmaxSink`: a recorded epoch would be the same in every replay, whose maxima the slots would then
+    hide.  Without a ticket the consumer reduces the tensor itself.  Epochs only grow, which is what lets the buffer go
     uncleared between uses.  All tickets of a device share the one buffer, so a ticket is good for exactly one
     producer launch followed by the quantization(s) of its output, on one stream, with no other producer launch
     in between: a later producer overwrites the slots.  The host side checks this (see ``_check_consumer``)."""
@@ -301,6 +313,8 @@ def amax_ticket(device: torch.device) -> AmaxTicket:
     key = _device_key(device)
     if key in _active_graph_sinks:
         return _active_graph_sinks[key].ticket()
+    if recording(device):
+        return None
     entry = _sinks.get(key)
     if entry is None or entry[1] >= 0xFFFFFFFE:
         entry = [torch.zeros(AMAX_PARTS, dtype=torch.int64, device=device), 0, None]
@@ -812,7 +826,8 @@ def _norm_quantize_result(code: int, what: str, values, scales, amax):
 
 def adaln_quantize(x, e_scale, e_shift, frame_seqlen, rule: str, eps=1e-6, add_one_to_scale=True, spin_limit=None):
     """``quantize(adaln_modulate(x, ...).reshape(-1, C), rule)`` as one launch that never writes the modulated
-    tensor: (values, scales, amax) with the same bytes, or None when the kernel does not take the shape."""
+    tensor: (values, scales, amax) with the same bytes, or None when the kernel does not take the shape or there is no
+    amax ticket to be had (:func:`amax_ticket`)."""
     _require_cuda(x, e_scale, e_shift)
     if x.ndim != 3 or x.dtype != torch.bfloat16 or not x.is_contiguous():
         raise ValueError("x must be a contiguous bfloat16 [B, L, C] tensor")
@@ -821,8 +836,11 @@ def adaln_quantize(x, e_scale, e_shift, frame_seqlen, rule: str, eps=1e-6, add_o
     for name, e in (("e_scale", e_scale), ("e_shift", e_shift)):
         if e.shape != (B, F, 1, C) or e.dtype != torch.bfloat16 or e.stride(3) != 1:
             raise ValueError(f"{name} must be bfloat16 [B, F, 1, C] = {(B, F, 1, C)}, got {tuple(e.shape)}")
+    ticket = amax_ticket(x.device)
+    if ticket is None:
+        return None
     values, scales, amax = _norm_quantize_outputs(B * L, C, x.device)
-    sink = _sink_struct(amax_ticket(x.device))
+    sink = _sink_struct(ticket)
     with torch.cuda.device(x.device):
         code = load().ll_adaln_quantize(x.data_ptr(), B, L, C, e_scale.data_ptr(), e_shift.data_ptr(),
                                         e_scale.stride(0), e_scale.stride(1), e_shift.stride(0), e_shift.stride(1),
@@ -843,8 +861,11 @@ def layer_norm_quantize(x, weight, bias, rule: str, eps=1e-6, spin_limit=None):
         x2 = x2.contiguous()
     w = None if weight is None else weight.contiguous()
     b = None if bias is None else bias.contiguous()
+    ticket = amax_ticket(x.device)
+    if ticket is None:
+        return None
     values, scales, amax = _norm_quantize_outputs(x2.shape[0], C, x.device)
-    sink = _sink_struct(amax_ticket(x.device))
+    sink = _sink_struct(ticket)
     with torch.cuda.device(x.device):
         code = load().ll_layer_norm_quantize(x2.data_ptr(), x2.shape[0], C, _ptr(w), _ptr(b), float(eps), RULE_IDS[rule],
                                              values.data_ptr(), scales.data_ptr(), amax.data_ptr(), ctypes.byref(sink),
@@ -856,7 +877,8 @@ def layer_norm_quantize(x, weight, bias, rule: str, eps=1e-6, spin_limit=None):
 def block_forward(x, e, layers, norms, cos, sin, window, text, rule: str, sizes, keys_only: bool, tickets):
     """One transformer block as one native call (``block_forward`` of csrc/host_ops.cpp, which documents the arguments):
     (out, roped K, V, text K, text V), or None when it does not take the call.  ``tickets``: of the producers of K and V.
-    The other tensor maxima go through a sink of the current stream, or through that of an active recording."""
+    The other tensor maxima go through a sink of the current stream, or through that of an active recording; a recording
+    without one is not taken."""
     lib, graph, graph_sink = host(), _active_graph_sinks.get(_device_key(x.device)), None
     if graph is not None:
         graph_sink = (graph.parts, graph.entry[1], graph.offset)

@@ -120,19 +120,32 @@ struct Epochs {
   uint32_t next;
   ll_amax_sink take() { return ll_amax_sink{parts, ++next, offset}; }
 };
-// parts is null where the sink would have to be made while the stream is being captured (its memory would belong to the
-// capture, its clearing to every replay).
+// A failing query (the legacy stream while another one is captured) counts as recording, and leaves no error behind.
+bool recording(void* stream) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(static_cast<hipStream_t>(stream), &status) != hipSuccess) {
+    (void)hipGetLastError();
+    return true;
+  }
+  return status != hipStreamCaptureStatusNone;
+}
+
+// parts is null while the stream is being captured: a recorded epoch would be the same in every replay, whose maxima the
+// slots, raised meanwhile by later epochs, would then hide.
 Epochs epochs_of_stream(int dev, void* stream) {
+  if (recording(stream)) return Epochs{nullptr, nullptr, 0};
   std::lock_guard<std::mutex> lock(g_sink_mutex);
   auto& sinks = stream_sinks();
   const std::pair<int, void*> key{dev, stream};
   auto found = sinks.find(key);
   if (found == sinks.end() || found->second.epoch > 0xFFFFFF00u) {
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(static_cast<hipStream_t>(stream), &capture) != hipSuccess || capture != hipStreamCaptureStatusNone)
-      return Epochs{nullptr, nullptr, 0};
     if (found == sinks.end()) found = sinks.emplace(key, StreamSink{empty({(int64_t)LL_AMAX_PARTS}, at::kLong, dev), 0}).first;
-    found->second.parts.zero_();
+    // not through torch's zero_: it may have a mode to report to, or refuse a tensor made in inference mode
+    if (hipMemsetAsync(found->second.parts.data_ptr(), 0, LL_AMAX_PARTS * sizeof(uint64_t), static_cast<hipStream_t>(stream)) != hipSuccess) {
+      (void)hipGetLastError();
+      sinks.erase(found);
+      return Epochs{nullptr, nullptr, 0};
+    }
     found->second.epoch = 0;
   }
   StreamSink& s = found->second;
@@ -141,20 +154,16 @@ Epochs epochs_of_stream(int dev, void* stream) {
   return e;
 }
 
-// The amax of x and its quantization: one launch for a small tensor, two otherwise and while the stream is being captured (a
-// recorded epoch would be the same in every replay).
+// The amax of x and its quantization: one launch for a small tensor, two otherwise and while the stream is being captured.
 constexpr int64_t kSpinLimit = 64;  // looks of one to two microseconds at the other workgroups' maxima
 int quantize_operand(const void* x, int64_t M, int64_t K, int64_t ldx, int rule, uint8_t* values, uint8_t* scales, float* amax, float* workspace,
                      int dev, void* stream) {
   if (K % 64 == 0 && ((M + 127) / 128) * (K / 64) <= 256) {
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(static_cast<hipStream_t>(stream), &capture) == hipSuccess && capture == hipStreamCaptureStatusNone) {
-      Epochs e = epochs_of_stream(dev, stream);
-      if (e.parts) {
-        const ll_amax_sink sink = e.take();
-        const int code = ll_nvfp4_quantize_once(x, M, K, ldx, rule, values, scales, amax, &sink, kSpinLimit, stream);
-        if (code != LL_ENOSUP) return code;
-      }
+    Epochs e = epochs_of_stream(dev, stream);
+    if (e.parts) {
+      const ll_amax_sink sink = e.take();
+      const int code = ll_nvfp4_quantize_once(x, M, K, ldx, rule, values, scales, amax, &sink, kSpinLimit, stream);
+      if (code != LL_ENOSUP) return code;
     }
   }
   return ll_nvfp4_quantize(x, M, K, ldx, rule, values, scales, amax, 0, workspace, stream);

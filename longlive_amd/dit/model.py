@@ -145,12 +145,15 @@ class CausalSelfAttention(nn.Module):
         self.use_relative_rope = False  # set on the module by the pipeline (pipeline/causal_diffusion_inference.py:316)
 
     @staticmethod
-    def amax_sinks(kv_cache: dict, device):
-        """The two sinks of a layer's cache in which the producers of K and V leave the maxima for the cache write."""
+    def amax_tickets(kv_cache: dict, device):
+        """Tickets of the two sinks of a layer's cache in which the producers of K and V leave the maxima for the cache
+        write.  None for both in a recording, which has no place for them (and whose memory a sink must not be made of)."""
+        if _native.recording(device):
+            return None, None
         sinks = kv_cache.get("_amax_sinks")
         if sinks is None:
             sinks = kv_cache["_amax_sinks"] = (_native.PrivateAmaxSink(device), _native.PrivateAmaxSink(device))
-        return sinks
+        return tuple(sink.ticket() for sink in sinks)
 
     def forward(self, x, cos, sin, kv_cache, current_start, sink_tokens, max_attention_size, *, input_amax=None,
                 residual=None, gate=None, gate_rows=0, global_sink_tokens=0, rope_fn=None, collect_kv_amax=True,
@@ -173,7 +176,7 @@ class CausalSelfAttention(nn.Module):
         fused_path = b == 1 and d == 128 and not self.use_relative_rope and self.norm_q.eps == self.norm_k.eps
         k_amax = v_amax = None
         if fused_path and collect_kv_amax and isinstance(kv_cache, dict):
-            k_amax, v_amax = (sink.ticket() for sink in self.amax_sinks(kv_cache, x.device))
+            k_amax, v_amax = self.amax_tickets(kv_cache, x.device)
         (q, k, v), v_amax_written = _project_shared(x, [self.q, self.k, self.v], amax=input_amax,
                                                     amax_outs=[None, None, v_amax])
         v = v.view(b, s, n, d)
@@ -357,7 +360,7 @@ class DiTBlock(nn.Module):
             window = kvc._window(kv_cache, slot_ids)
         tickets = (None, None)
         if collect_kv_amax:
-            tickets = tuple(sink.ticket() for sink in sa.amax_sinks(kv_cache, x.device))
+            tickets = sa.amax_tickets(kv_cache, x.device)
         out = _native.block_forward(
             x, e, tuple(layers), (norms[0].weight, norms[1].weight, norm3.weight, norm3.bias, norms[2].weight, norms[3].weight),
             cos, sin, window, text, rule.value, (sa.num_heads, self.eps, norms[0].eps, norm3.eps, norms[2].eps, norms[3].eps),

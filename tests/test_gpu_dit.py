@@ -761,6 +761,49 @@ def test_block_forward_recorded_into_a_graph_replays_bit_for_bit(gpu):
             torch.cuda.synchronize()
 
 
+def test_block_recorded_without_a_replayable_sink_replays_bit_for_bit(gpu):
+    """Recorded on a stream that has run the block before, with no ReplayableAmaxSink: the recording then carries no epochs
+    (the tensors are reduced by launches of their own), so that replays on falling and rising activations, with eager
+    forwards on both streams between them, equal the eager results; and no sink is made of the recording's memory."""
+    torch.manual_seed(0)
+    dim, heads, ffn, F, h, w, T = 256, 2, 512, 2, 8, 8, 16
+    L = F * h * w
+    block, _ = quantize_model_with_filter(DiTBlock(dim, ffn, heads).to(gpu), ModelQuantizationConfig(), use_default_filtered_modules=True,
+                                          materialize_for_inference=True, verbose=False)
+    cos, sin = rope_cos_sin(build_rope_angles(128), F, h, w, 0, gpu)
+    g = torch.Generator().manual_seed(6)
+
+    def run(x, e0, ctx, cache):
+        return block(x, e0, cos, sin, ctx, cache, 0, sink_tokens=L)[0]
+
+    with torch.no_grad():
+        cases = [((torch.randn(1, L, dim, generator=g) * s).bfloat16().to(gpu), torch.randn(1, F, 6, dim, generator=g).bfloat16().to(gpu),
+                  torch.randn(1, T, dim, generator=g).bfloat16().to(gpu)) for s in (8.0, 1.0, 0.05, 3.0)]
+        cache, fresh = (kvc.initialize_kv_cache(1, L, 3, heads, 128, KV, gpu)[0] for _ in range(2))
+        eager = [run(*case, cache).clone() for case in cases]
+        static = [t.clone() for t in cases[0]]
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            run(*static, cache)
+        torch.cuda.current_stream().wait_stream(side)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            recorded = run(*static, fresh)
+        assert "_amax_sinks" not in fresh
+        for i, case in enumerate(cases):
+            for dst, src in zip(static, case):
+                dst.copy_(src)
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(recorded, eager[i]), i
+            j = (i + 1) % 4
+            with torch.cuda.stream(side):
+                on_side = run(*cases[j], cache)
+            torch.cuda.synchronize()
+            assert torch.equal(on_side, eager[j]) and torch.equal(run(*cases[j], cache), eager[j])
+
+
 def test_cache_write_takes_the_k_and_v_maxima_from_their_producers(gpu):
     """The chunk's roped K and its V are quantized into the cache after the forward.  Their producers (the norm +
     RoPE kernel, the V projection's epilogue) leave the tensor maxima in the layer's own amax sinks, and the cache

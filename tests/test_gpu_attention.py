@@ -925,6 +925,7 @@ def test_native_cache_step_equals_the_separate_operations(gpu, relative, frames,
         assert torch.equal(a, b), i
 
 
+@pytest.mark.parametrize("peaked", [False, True])
 @pytest.mark.parametrize("Lq,H,T,cached,n_new", [
     (1, 1, 0, 0, 1),            # one query, one key: seven or three waves without a tile
     (64, 2, 0, 0, 128),         # four waves, four tiles
@@ -935,10 +936,11 @@ def test_native_cache_step_equals_the_separate_operations(gpu, relative, frames,
     (512, 16, 512, 2048, 512),  # as many workgroups as compute units, the longest range
     (520, 24, 0, 0, 1030),      # two workgroups of four waves per compute unit
 ])
-def test_short_launches_against_fp64(gpu, Lq, H, T, cached, n_new):
+def test_short_launches_against_fp64(gpu, Lq, H, T, cached, n_new, peaked):
     """The kernel with 32 queries per workgroup, over the edges of its tiles and of its rule, twice for
-    identical bits, its amax sink included.  Bound: bf16 probabilities and a bf16 result, 2^-9 relative each, with
-    sum p |v| <= max |v|, and as much again for the fp32 sums and scores."""
+    identical bits, its amax sink included.  ``peaked``: the queries are the keys' own directions, spread over all tiles, so
+    that every tile and wave holds most of some query's weight.  Bound, element by element: bf16 probabilities, 2^-9 of
+    sum p |v|, and a bf16 result, 2^-9 of its magnitude, and a quarter of the first for the fp32 sums and scores."""
     q, k, v = (_randn((n, H, 128), s).to(gpu) for n, s in ((Lq, 31), (max(n_new, 1), 32), (max(n_new, 1), 33)))
     slots, tables, K, V = -(-cached // T) if cached else 0, None, [], []
     if cached:
@@ -954,6 +956,11 @@ def test_short_launches_against_fp64(gpu, Lq, H, T, cached, n_new):
     new = (k[:n_new], v[:n_new]) if n_new else (None, None)
     if n_new:
         K.append(k), V.append(v)
+    K, V = torch.cat(K), torch.cat(V)
+    if peaked:
+        at = (torch.arange(Lq, device=gpu)[:, None] * len(K) // Lq + torch.arange(H, device=gpu) * 37) % len(K)
+        q = torch.gather(K, 0, at[:, :, None].expand(Lq, H, 128)).contiguous()
+    K, V = K.double(), V.double()
     outs = []
     for _ in range(2):
         ticket = _native.amax_ticket(gpu)
@@ -961,6 +968,21 @@ def test_short_launches_against_fp64(gpu, Lq, H, T, cached, n_new):
         xq = quantize_to_fp4(outs[-1].flatten(1), CFG, amax=ticket)
         assert float(xq.amax) == float(outs[-1].float().abs().max())
     assert torch.equal(*outs)
-    K, V = torch.cat(K).double(), torch.cat(V).double()
-    ref = torch.stack([torch.softmax(q[:, h].double() @ K[:, h].T.contiguous() * 128 ** -0.5, -1) @ V[:, h] for h in range(H)], 1)
-    assert (outs[0].double() - ref).abs().max().item() <= 2 ** -7 * V.abs().max().item()
+    p = [torch.softmax(q[:, h].double() @ K[:, h].T.contiguous() * 128 ** -0.5, -1) for h in range(H)]
+    ref, size = (torch.stack([ph @ v[:, h] for h, ph in enumerate(p)], 1) for v in (V, V.abs()))
+    error = (outs[0].double() - ref).abs()
+    assert (error <= 1.25 * 2 ** -9 * size + 2 ** -9 * ref.abs()).all()
+
+
+@pytest.mark.parametrize("Lq,H,keys", [(368, 16, 1472), (384, 2, 1152), (512, 16, 2560), (736, 12, 512)])
+def test_short_launches_are_no_further_from_fp64_than_the_tile_kernels(gpu, Lq, H, keys):
+    """Relative error (2-norm) of the kernel with 32 queries per workgroup against that of the divided 256-query tiles (the
+    closest of the others: every part has a softmax of its own) on the same inputs, over some hundred thousand results."""
+    q, k, v = (_randn((n, H, 128), s).to(gpu) for n, s in ((Lq, 51), (keys, 52), (keys, 53)))
+    assert _native.attention_plan(Lq, H, keys)["workgroups"] == H * -(-Lq // 32)
+    ref = torch.stack([torch.softmax(q[:, h].double() @ k[:, h].double().T.contiguous() * 128 ** -0.5, -1) @ v[:, h].double() for h in range(H)], 1)
+    errors = []
+    for policy in ("auto", "split"):
+        with _native.attention_policy(policy):
+            errors.append(((_native.attention_bf16(q, k, v, 128 ** -0.5).double() - ref).norm() / ref.norm()).item())
+    assert errors[0] <= errors[1]

@@ -873,6 +873,7 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) 
 #pragma unroll
     for (int i = 0; i < 16; ++i) o[dt][i] = 0.0f;
   float m_run = -INFINITY, l_run = 0.0f;
+  float neg = 0.0f;  // the reference point in the exponent of 2; 0 while no score above -inf has been met: all weigh nothing
   // The reference point follows the maximum in steps.  A probability close below its reference point loses least in bf16, and
   // the largest ones weigh most: with steps of 2^2, all queries of the wave raised as soon as one has to be, the result is
   // closer to fp64 than that of the divided tiles (368 queries x 16 heads over 1472 keys 0.00220 relative against 0.00224,
@@ -906,7 +907,8 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) 
     mx = max_over_wave_halves(mx);
     if (__builtin_amdgcn_ballot_w64((mx - m_run) * p.scale_log2 > kRescaleStep) != 0) {
       const float m_new = fmaxf(m_run, mx);
-      const float alpha = __builtin_amdgcn_exp2f((m_run - m_new) * p.scale_log2);
+      neg = m_new == -INFINITY ? 0.0f : -m_new * p.scale_log2;
+      const float alpha = __builtin_amdgcn_exp2f(fmaf(m_run, p.scale_log2, neg));
       m_run = m_new;
       l_run *= alpha;
 #pragma unroll
@@ -914,7 +916,6 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) 
 #pragma unroll
         for (int i = 0; i < 16; ++i) o[dt][i] *= alpha;
     }
-    const float neg = -m_run * p.scale_log2;
     read_v(1);
 #pragma unroll
     for (int step = 0; step < 2; ++step) {

@@ -986,3 +986,20 @@ def test_short_launches_are_no_further_from_fp64_than_the_tile_kernels(gpu, Lq, 
         with _native.attention_policy(policy):
             errors.append(((_native.attention_bf16(q, k, v, 128 ** -0.5).double() - ref).norm() / ref.norm()).item())
     assert errors[0] <= errors[1]
+
+
+@pytest.mark.parametrize("Lq,H,keys,gone", [(64, 2, 128, (0, 32)), (64, 2, 128, (96, 128)), (70, 4, 417, (0, 40)), (368, 16, 1472, (0, 288)),
+                                            (368, 16, 1472, (800, 1200))])
+def test_scores_of_minus_infinity_weigh_nothing(gpu, Lq, H, keys, gone):
+    """Keys whose scores overflow to -inf for every query, whole 32-key tiles of them (a wave's first, its only, all of a
+    wave's): the result is that of the other keys.  Bound as for the short launches."""
+    q, k, v = (_randn((n, H, 128), s).to(gpu) for n, s in ((Lq, 61), (keys, 62), (keys, 63)))
+    q[..., 0], k[..., 0] = 1e20, 0.0
+    k[gone[0]:gone[1], :, 0] = -1e20
+    assert _native.attention_plan(Lq, H, keys)["workgroups"] == H * -(-Lq // 32)
+    out = _native.attention_bf16(q, k, v, 128 ** -0.5)
+    left = [i for i in range(keys) if not gone[0] <= i < gone[1]]
+    K, V = k[left].double(), v[left].double()
+    p = [torch.softmax(q[:, h].double() @ K[:, h].T.contiguous() * 128 ** -0.5, -1) for h in range(H)]
+    ref, size = (torch.stack([ph @ x[:, h] for h, ph in enumerate(p)], 1) for x in (V, V.abs()))
+    assert ((out.double() - ref).abs() <= 1.25 * 2 ** -9 * size + 2 ** -9 * ref.abs()).all()

@@ -368,16 +368,20 @@ int ll_kv_attention_get_policy(void);
  * would need under the current policy (nothing when that launch would not take the split division), so that the
  * launch itself allocates nothing: call it ahead of a graph recording or a latency-critical loop.  May allocate,
  * and may free a smaller set (which waits for the device).  LL_ENOSUP while the stream is being captured.  No
- * counterpart in the reference. */
+ * counterpart in the reference.  Whether a launch of a few hundred queries needs memory depends on how many of its keys
+ * are cached: ll_kv_attention_reserve_window is told, ll_kv_attention_reserve provides for any division of the keys. */
+int ll_kv_attention_reserve_window(int64_t Lq, int num_heads, int64_t n_cached, int64_t n_new, void* stream);
 int ll_kv_attention_reserve(int64_t Lq, int num_heads, int64_t n_keys, void* stream);
 /* ll_release_stream_memory under its first name. */
 int ll_kv_attention_release(void* stream);
-/* What a launch of Lq queries x num_heads heads over n_keys keys would do on a device with `compute_units` CUs
- * under `policy` (pure host arithmetic, no GPU needed): the division taken (an LL_ATTENTION_SPLIT request falls
+/* What a launch of Lq queries x num_heads heads over n_cached cached and n_new bf16 keys would do on a device with
+ * `compute_units` CUs under `policy` (pure host arithmetic, no GPU needed): the division taken (an LL_ATTENTION_SPLIT request falls
  * back to WIDE when there is nothing to split), the number of workgroups, the whole rounds of tiles all of them
  * run first and the number of tiles cut into shares (tiles behind the whole rounds that are not counted here run
  * whole on workgroups that take no share).  Lets a caller know ahead of a launch whether it will
- * take the allocating division.  Output pointers may be NULL. */
+ * take the allocating division.  Output pointers may be NULL.  ll_kv_attention_plan: for a launch without cached keys. */
+int ll_kv_attention_plan_window(int64_t Lq, int num_heads, int64_t n_cached, int64_t n_new, int compute_units, int policy,
+                                int* division, uint32_t* workgroups, uint32_t* whole_rounds, int64_t* split_tiles);
 int ll_kv_attention_plan(int64_t Lq, int num_heads, int64_t n_keys, int compute_units, int policy,
                          int* division, uint32_t* workgroups, uint32_t* whole_rounds, int64_t* split_tiles);
 

@@ -68,6 +68,7 @@ _SIGNATURES = {
     "ll_kv_attention_set_policy": (c_int, [c_int]),
     "ll_kv_attention_get_policy": (c_int, []),
     "ll_kv_attention_plan": (c_int, [c_int64, c_int, c_int64, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p]),
+    "ll_kv_attention_plan_window": (c_int, [c_int64, c_int, c_int64, c_int64, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p]),
     "ll_rope_apply": (c_int, [c_void_p, c_int64, c_int, c_int, c_int64, c_int64, c_void_p, c_void_p, c_int64,
                               c_void_p, c_void_p]),
     "ll_adaln_modulate": (c_int, [c_void_p, c_int64, c_int64, c_int, c_void_p, c_void_p, c_int64, c_int64, c_int64,
@@ -104,6 +105,7 @@ _SIGNATURES = {
     "ll_nvfp4_gemm_plan": (c_int, [c_int64, c_int64, c_int64, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p]),
     "ll_nvfp4_gemm_kernel": (c_int, [c_int64, c_int64, c_int64, c_int, c_int, c_int, c_void_p, c_void_p]),
     "ll_kv_attention_reserve": (c_int, [c_int64, c_int, c_int64, c_void_p]),
+    "ll_kv_attention_reserve_window": (c_int, [c_int64, c_int, c_int64, c_int64, c_void_p]),
     "ll_kv_attention_release": (c_int, [c_void_p]),
     "ll_nvfp4_quantize_noalloc_max_elements": (c_int64, []),
     "ll_nvfp4_quantize_noalloc": (c_int, [c_void_p, c_int64, c_int64, c_int64, c_int, c_void_p, c_void_p, c_void_p,
@@ -667,26 +669,29 @@ def attention_bf16(q, k, v, softmax_scale, amax_out=None):
 ATTENTION_POLICIES = {"auto": -1, "narrow": 0, "wide": 1, "split": 2}
 
 
-def attention_plan(Lq: int, num_heads: int, n_keys: int, compute_units: int = 256, policy: str = "auto") -> dict:
-    """How an attention launch of these sizes would be divided between workgroups on a device with
-    ``compute_units`` CUs (host arithmetic only): division name, workgroups, whole tiles per workgroup and the
-    number of tiles cut into shares."""
+def attention_plan(Lq: int, num_heads: int, n_keys: int, compute_units: int = 256, policy: str = "auto", n_cached: int = 0) -> dict:
+    """How an attention launch of these sizes, ``n_cached`` of its keys in cache slots, would be divided between workgroups
+    on a device with ``compute_units`` CUs (host arithmetic only): division name, workgroups, whole tiles per workgroup and
+    the number of tiles cut into shares."""
     division, groups, rounds = c_int(), ctypes.c_uint32(), ctypes.c_uint32()
     split = c_int64()
-    _check(load().ll_kv_attention_plan(Lq, num_heads, n_keys, compute_units, ATTENTION_POLICIES[policy],
-                                       ctypes.byref(division), ctypes.byref(groups), ctypes.byref(rounds),
-                                       ctypes.byref(split)), "ll_kv_attention_plan")
+    _check(load().ll_kv_attention_plan_window(Lq, num_heads, n_cached, n_keys - n_cached, compute_units, ATTENTION_POLICIES[policy],
+                                              ctypes.byref(division), ctypes.byref(groups), ctypes.byref(rounds),
+                                              ctypes.byref(split)), "ll_kv_attention_plan")
     names = {v: k for k, v in ATTENTION_POLICIES.items()}
     return {"division": names[division.value], "workgroups": groups.value, "whole_rounds": rounds.value,
             "split_tiles": split.value}
 
 
-def attention_reserve(Lq: int, num_heads: int, n_keys: int, device=None) -> None:
+def attention_reserve(Lq: int, num_heads: int, n_keys: int, device=None, n_cached: int | None = None) -> None:
     """Set up, on the current stream, the memory an attention launch of these sizes would pass partial tiles
     through (nothing if it would not split), so that the launch itself - for instance inside a graph recording -
-    allocates nothing."""
+    allocates nothing.  ``n_cached``: how many of the keys are in cache slots; None provides for any number."""
     with torch.cuda.device(device if device is not None else torch.cuda.current_device()):
-        _check(load().ll_kv_attention_reserve(Lq, num_heads, n_keys, _stream()), "ll_kv_attention_reserve")
+        if n_cached is None:
+            _check(load().ll_kv_attention_reserve(Lq, num_heads, n_keys, _stream()), "ll_kv_attention_reserve")
+        else:
+            _check(load().ll_kv_attention_reserve_window(Lq, num_heads, n_cached, n_keys - n_cached, _stream()), "ll_kv_attention_reserve")
 
 
 def attention_release(device=None) -> None:

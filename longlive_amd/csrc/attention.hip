@@ -1108,7 +1108,7 @@ static int launch_attention(const AttnParams& p_in, hipStream_t stream) {
   const int64_t n_iter = (p.n_cached + p.n_new + kIterKeys - 1) / kIterKeys;
   LL_REQUIRE(p.H * ((p.Lq + kWgQueries - 1) / kWgQueries) * n_iter < (1ll << 32), "ll_kv_attention: too many (tile, iteration) units");
   const int policy = g_attention_policy.load(std::memory_order_relaxed);
-  if (const int waves = policy <= LL_ATTENTION_NARROW ? short_kernel_waves(p.Lq, p.H, p.n_cached, p.n_new, cus) : 0) {
+  if (const int waves = short_kernel_waves(p.Lq, p.H, p.n_cached, p.n_new, cus, policy)) {
     p.n_qtiles = (int)((p.Lq + kWaveQueries - 1) / kWaveQueries);
     p.d.G = (uint32_t)(p.H * p.n_qtiles);
     static std::atomic<uint64_t> lds_allowed4{0}, lds_allowed8{0};
@@ -1174,9 +1174,11 @@ extern "C" int ll_kv_attention_set_policy(int policy) {
 
 extern "C" int ll_kv_attention_get_policy(void) { return ll::g_attention_policy.load(); }
 
-extern "C" int ll_kv_attention_reserve(int64_t Lq, int num_heads, int64_t n_keys, void* stream) {
+extern "C" int ll_kv_attention_reserve_window(int64_t Lq, int num_heads, int64_t n_cached, int64_t n_new, void* stream) {
   using namespace ll;
-  LL_REQUIRE(Lq > 0 && num_heads > 0 && n_keys > 0 && Lq < (1ll << 30) && n_keys < (1ll << 30), "ll_kv_attention_reserve: bad sizes");
+  LL_REQUIRE(Lq > 0 && num_heads > 0 && n_cached >= 0 && n_new >= 0 && n_cached + n_new > 0 && Lq < (1ll << 30) && n_cached < (1ll << 30) &&
+                 n_new < (1ll << 30) && n_cached + n_new < (1ll << 30),
+             "ll_kv_attention_reserve: bad sizes");
   int dev = 0, cus = 0;
   if (hipGetDevice(&dev) != hipSuccess) {
     set_error("ll_kv_attention_reserve: hipGetDevice failed");
@@ -1184,10 +1186,8 @@ extern "C" int ll_kv_attention_reserve(int64_t Lq, int num_heads, int64_t n_keys
   }
   if (int rc = compute_units_of(dev, cus, "ll_kv_attention")) return rc;
   const int policy = g_attention_policy.load(std::memory_order_relaxed);
-  const AttentionPlan plan = plan_attention(Lq, num_heads, n_keys, cus, policy);
-  // (what is cached and what is the chunk's own decides between the short kernel and the tiles: only a launch that takes
-  // the short kernel either way needs no memory; + 32: a window of both has a partly filled tile more)
-  if (policy <= LL_ATTENTION_NARROW && short_kernel_waves(Lq, num_heads, n_keys + 32, 0, cus)) return LL_OK;
+  if (short_kernel_waves(Lq, num_heads, n_cached, n_new, cus, policy)) return LL_OK;
+  const AttentionPlan plan = plan_attention(Lq, num_heads, n_cached + n_new, cus, policy);
   if (plan.mode != LL_ATTENTION_SPLIT) return LL_OK;
   if (stream_is_capturing(static_cast<hipStream_t>(stream))) {
     set_error("ll_kv_attention_reserve: the stream is being captured; reserve before the recording starts");
@@ -1198,26 +1198,39 @@ extern "C" int ll_kv_attention_reserve(int64_t Lq, int num_heads, int64_t n_keys
                         (size_t)plan.split_tiles, true, w, nullptr, "ll_kv_attention_reserve");
 }
 
+// Cached keys are the longer way through the short kernel, and one fresh key may make a tile more: where these two need no
+// memory, no other division of the keys into cached and fresh ones does.
+extern "C" int ll_kv_attention_reserve(int64_t Lq, int num_heads, int64_t n_keys, void* stream) {
+  if (int rc = ll_kv_attention_reserve_window(Lq, num_heads, n_keys, 0, stream)) return rc;
+  return n_keys > 1 ? ll_kv_attention_reserve_window(Lq, num_heads, n_keys - 1, 1, stream) : LL_OK;
+}
+
 extern "C" int ll_kv_attention_release(void* stream) { return ll_release_stream_memory(stream); }
 
-extern "C" int ll_kv_attention_plan(int64_t Lq, int num_heads, int64_t n_keys, int compute_units, int policy,
-                                    int* division, uint32_t* workgroups, uint32_t* whole_rounds, int64_t* split_tiles) {
-  LL_REQUIRE(Lq > 0 && num_heads > 0 && n_keys > 0 && compute_units > 0 && Lq < (1ll << 30) && n_keys < (1ll << 30),
+extern "C" int ll_kv_attention_plan_window(int64_t Lq, int num_heads, int64_t n_cached, int64_t n_new, int compute_units, int policy,
+                                           int* division, uint32_t* workgroups, uint32_t* whole_rounds, int64_t* split_tiles) {
+  LL_REQUIRE(Lq > 0 && num_heads > 0 && n_cached >= 0 && n_new >= 0 && n_cached + n_new > 0 && compute_units > 0 && Lq < (1ll << 30) &&
+                 n_cached < (1ll << 30) && n_new < (1ll << 30) && n_cached + n_new < (1ll << 30),
              "ll_kv_attention_plan: bad sizes");
   LL_REQUIRE(policy >= LL_ATTENTION_AUTO && policy <= LL_ATTENTION_SPLIT, "ll_kv_attention_plan: unknown policy %d", policy);
-  if (policy <= LL_ATTENTION_NARROW && ll::short_kernel_waves(Lq, num_heads, n_keys + 32, 0, compute_units)) {
+  if (ll::short_kernel_waves(Lq, num_heads, n_cached, n_new, compute_units, policy)) {
     if (division) *division = LL_ATTENTION_NARROW;
     if (workgroups) *workgroups = (uint32_t)(num_heads * ((Lq + 31) / 32));
     if (whole_rounds) *whole_rounds = 1;
     if (split_tiles) *split_tiles = 0;
     return LL_OK;
   }
-  const ll::AttentionPlan plan = ll::plan_attention(Lq, num_heads, n_keys, compute_units, policy);
+  const ll::AttentionPlan plan = ll::plan_attention(Lq, num_heads, n_cached + n_new, compute_units, policy);
   if (division) *division = plan.mode;
   if (workgroups) *workgroups = plan.d.G;
   if (whole_rounds) *whole_rounds = plan.d.whole_rounds;
   if (split_tiles) *split_tiles = plan.split_tiles;
   return LL_OK;
+}
+
+extern "C" int ll_kv_attention_plan(int64_t Lq, int num_heads, int64_t n_keys, int compute_units, int policy,
+                                    int* division, uint32_t* workgroups, uint32_t* whole_rounds, int64_t* split_tiles) {
+  return ll_kv_attention_plan_window(Lq, num_heads, 0, n_keys, compute_units, policy, division, workgroups, whole_rounds, split_tiles);
 }
 
 extern "C" int ll_kv_attention(const void* q, int64_t Lq, int num_heads, const uint64_t* k_values_ptrs,

@@ -113,9 +113,13 @@ LL_SPLIT_FN uint32_t record_of_part(uint32_t g, uint32_t split_tile, const Divis
 //   G <= 2 CUs    736 x 12, 0 + 16: 16.3 / 18.4 / 13.7; 512 x 24, 32 + 16: 34.7 / 38.3 / 32.8, but 46 + 23 on 736 x 12:
 //                 38.7 / 49.9 / 43.5;   G > 2 CUs: 736 x 24, 0 + 16: 16.8 / 26.4 / 20.5
 // A cached tile costs about half as much again as one of the chunk (conversion).  Launches of more than 256 queries per
-// head for every head (700 queries of 2 heads: 27.8 / 12.9) stay with the divided tiles: programs that reserve their memory
-// ahead of a recording count on that division and its bits.
-inline int short_kernel_waves(int64_t Lq, int H, int64_t n_cached, int64_t n_new, int cus) {
+// head for every head stay with the divided tiles because the line ends where the measurements above do, not because the
+// tiles are ahead there: the one point taken beyond it (700 queries of 2 heads over 900 keys) is 27.8 us against 12.9 in this
+// kernel.  Moving it takes a sweep of 1 to 6 heads with 512 to 4096 queries.
+// `policy`: only the automatic choice (-1) and the division without shared tiles (0) take this kernel.  The launch, the
+// plan query and the reserve call all ask here.
+inline int short_kernel_waves(int64_t Lq, int H, int64_t n_cached, int64_t n_new, int cus, int policy) {
+  if (policy > 0) return 0;
   const int64_t groups = H * ((Lq + 31) / 32), cached = (n_cached + 31) / 32, fresh = (n_new + 31) / 32;
   const int64_t length = cached + cached / 2 + fresh;
   if (Lq > 256 * (int64_t)H) return 0;

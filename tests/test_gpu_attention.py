@@ -1003,3 +1003,25 @@ def test_scores_of_minus_infinity_weigh_nothing(gpu, Lq, H, keys, gone):
     p = [torch.softmax(q[:, h].double() @ K[:, h].T.contiguous() * 128 ** -0.5, -1) for h in range(H)]
     ref, size = (torch.stack([ph @ x[:, h] for h, ph in enumerate(p)], 1) for x in (V, V.abs()))
     assert ((out.double() - ref).abs() <= 1.25 * 2 ** -9 * size + 2 ** -9 * ref.abs()).all()
+
+
+@pytest.mark.parametrize("Lq,H,T,cached,n_new", [(512, 16, 512, 0, 4000), (512, 16, 512, 3584, 416), (520, 24, 480, 0, 1900),
+                                                (520, 24, 480, 1440, 460), (512, 16, 512, 2048, 512)])
+def test_the_plan_is_what_the_launch_does(gpu, Lq, H, T, cached, n_new):
+    """Shapes whose division depends on how many of the keys are cached: the automatic choice has the bits of the division
+    that the plan names, and not those of the other one."""
+    q, k, v = (_randn((n, H, 128), s).to(gpu) for n, s in ((Lq, 71), (n_new, 72), (n_new, 73)))
+    tables = None
+    if cached:
+        cache = kvc.initialize_kv_cache(1, T, cached // T, H, 128, CFG, gpu)[0]
+        for c in range(cached // T):
+            kv = [_randn((1, T, H, 128), 80 + 2 * c + i).to(gpu) for i in range(2)]
+            kvc.apply_cache_update(cache, *kvc.kv_cache_update_only(*kv, cache, c * T, T), CFG)
+        kt, vt = kvc._tables_for(cache, tuple(range(cached // T)))
+        tables = (kt.values, kt.scales, kt.amax, vt.values, vt.scales, vt.amax)
+    outs = {}
+    for policy in ("auto", "narrow", "split"):
+        with _native.attention_policy(policy):
+            outs[policy] = _native.kv_attention(q, tables, cached, T, 6.0, 256.0, k, v, 128 ** -0.5)
+    planned = _native.attention_plan(Lq, H, cached + n_new, n_cached=cached)["division"]
+    assert [torch.equal(outs["auto"], outs[p]) for p in ("narrow", "split")] == [planned == "narrow", planned == "split"]

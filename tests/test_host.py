@@ -304,6 +304,16 @@ def test_short_launches_take_32_queries_per_workgroup(Lq, H, keys, short):
     assert _native.attention_plan(Lq, H, keys, policy="wide")["division"] == "wide"
 
 
+@pytest.mark.parametrize("Lq,H,keys,fresh,cached", [(512, 16, 4000, "narrow", "split"), (520, 24, 1900, "narrow", "split"),
+                                                   (512, 16, 3200, "narrow", "narrow"), (512, 16, 6000, "split", "split")])
+def test_plan_weighs_cached_and_fresh_keys_as_the_launch_does(Lq, H, keys, fresh, cached):
+    """A cached key costs a short launch more than a fresh one, so that the division depends on how many there are."""
+    divisions = [_native.attention_plan(Lq, H, keys, n_cached=n)["division"] for n in (0, keys)]
+    assert divisions == [fresh, cached] and _native.attention_plan(Lq, H, keys)["division"] == fresh
+    with pytest.raises(ValueError):
+        _native.attention_plan(Lq, H, keys, n_cached=keys + 1)
+
+
 def _check_division(plan, tiles):
     """Every (tile, iteration) in exactly one segment; whole tiles first; the parts of a split tile held by exactly
     the workgroups parts_of_tile names, one part each, in records no two parts share; at most two partial tiles

@@ -1,0 +1,19 @@
+"""A native call that stands for several methods of an object is right only while these are the package's own: a subclass, an
+instance or a test may have put others in their place, which then have to run."""
+from __future__ import annotations
+
+
+class OwnMethods:
+    """The methods ``names`` of ``cls`` as the package defines them; to be made where the class is defined."""
+
+    def __init__(self, cls: type, *names: str) -> None:
+        self._methods = tuple((name, getattr(cls, name)) for name in names)
+        self._names = frozenset(names)
+
+    def of(self, obj) -> bool:
+        """Whether ``obj`` runs these very methods."""
+        cls = type(obj)
+        for name, method in self._methods:
+            if getattr(cls, name) is not method:
+                return False
+        return self._names.isdisjoint(obj.__dict__)

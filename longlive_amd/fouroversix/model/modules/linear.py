@@ -9,6 +9,7 @@ import torch
 import torch.nn as nn
 
 from .... import _native
+from ...._own_methods import OwnMethods
 from ...matmul import fp4_matmul
 from ...quantize import QuantizationConfig, QuantizedTensor, quantize_to_fp4
 from ...quantize.frontend import _unsupported
@@ -126,7 +127,7 @@ class FourOverSixLinear(nn.Linear):
 
     def _forward_2d(self, x2d: torch.Tensor) -> torch.Tensor:
         weight, config = self.quantized_weight(), self.config
-        if (isinstance(weight, QuantizedTensor) and config.output_dtype is DataType.bfloat16 and config.dtype is DataType.nvfp4
+        if (_OWN.of(self) and isinstance(weight, QuantizedTensor) and config.output_dtype is DataType.bfloat16 and config.dtype is DataType.nvfp4
                 and weight.original_shape[1] == x2d.shape[1]):
             # quantization and product as one native call; the operand between them has no other reader
             rule = config.activation_scale_rule._value_
@@ -139,9 +140,10 @@ class FourOverSixLinear(nn.Linear):
 
     def native_operand(self):
         """(values, scale factors, amax, bias or None, denominator, out_features) for the native calls that run this
-        layer among others; ``None`` when it has no quantized weight or another type than NVFP4 in, bf16 out."""
+        layer among others; ``None`` when it has no quantized weight, another type than NVFP4 in, bf16 out, or methods
+        of its own."""
         config, weight = self.config, self.quantized_weight()
-        if not isinstance(weight, QuantizedTensor) or config.output_dtype is not DataType.bfloat16 or config.dtype is not DataType.nvfp4:
+        if not _OWN.of(self) or not isinstance(weight, QuantizedTensor) or config.output_dtype is not DataType.bfloat16 or config.dtype is not DataType.nvfp4:
             return None
         return (weight.values, weight.scale_factors, weight.amax, self._parameters.get("bias"),
                 _native.DENOMINATORS[weight.scale_rule._value_], weight.original_shape[0])
@@ -213,3 +215,7 @@ class FourOverSixLinear(nn.Linear):
         return fp4_matmul(xq, weight, backend=self.config.matmul_backend, out_dtype=self.config.output_dtype,
                           bias=self.bias, activation=activation, residual=residual, gate=gate, gate_rows=gate_rows,
                           amax_out=amax_out)
+
+
+# what the native calls stand for
+_OWN = OwnMethods(FourOverSixLinear, "quantize_input", "quantize_normalized_input", "forward_quantized", "forward_quantized_together")

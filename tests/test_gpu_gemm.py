@@ -804,3 +804,31 @@ def test_small_product_while_another_stream_is_being_captured(gpu):
     assert torch.equal(got, want) and y.tolist() == [2.0] * 8
     with torch.cuda.stream(other):
         _native.release_stream_memory()
+
+
+@pytest.mark.parametrize("how", ["subclass", "instance", "class"])
+@pytest.mark.parametrize("method", ["quantize_input", "forward_quantized"])
+def test_linear_layer_calls_the_methods_put_in_place_of_its_own(gpu, monkeypatch, how, method):
+    """FourOverSixLinear.forward is one native call only while quantize_input and forward_quantized are the package's."""
+    from longlive_amd.fouroversix import FourOverSixLinear, ModelQuantizationConfig
+    from longlive_amd.utils.quant import quantize_model_with_filter
+
+    model, _ = quantize_model_with_filter(torch.nn.Sequential(torch.nn.Linear(256, 128)).to(gpu), ModelQuantizationConfig(),
+                                          materialize_for_inference=True, verbose=False)
+    layer, calls, original = model[0], [], getattr(FourOverSixLinear, method)
+
+    def replacement(self, *args, **kwargs):
+        calls.append(method)
+        return original(self, *args, **kwargs)
+
+    x = activations((48, 256), 5).to(gpu)
+    with torch.no_grad():
+        want = layer(x)
+        assert not calls
+        if how == "subclass":
+            layer.__class__ = type("Mine", (FourOverSixLinear,), {method: replacement})
+        elif how == "instance":
+            monkeypatch.setattr(layer, method, replacement.__get__(layer))
+        else:
+            monkeypatch.setattr(FourOverSixLinear, method, replacement)
+        assert torch.equal(layer(x), want) and calls == [method] and layer.native_operand() is None

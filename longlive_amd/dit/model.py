@@ -17,6 +17,7 @@ import torch
 import torch.nn as nn
 
 from .. import _native
+from .._own_methods import OwnMethods
 from ..fouroversix.model.modules.linear import FourOverSixLinear
 from ..utils import kv_cache as kvc
 from ..utils.adaln import adaln_modulate, gate_residual
@@ -263,6 +264,12 @@ def _has_hooks(*modules) -> bool:
         m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__ for m in modules)
 
 
+# what a native block call stands for besides the linear layers
+_OWN_RMS_NORM = OwnMethods(WanRMSNorm, "forward")
+_OWN_SELF_ATTENTION = OwnMethods(CausalSelfAttention, "forward", "amax_tickets")
+_OWN_CROSS_ATTENTION = OwnMethods(CrossAttention, "forward")
+
+
 class DiTBlock(nn.Module):
     # normalize and quantize in one launch where a quantized layer reads the result (the same bytes either way)
     fuse_norm_quantize = True
@@ -340,6 +347,8 @@ class DiTBlock(nn.Module):
         norms = (sm["norm_q"], sm["norm_k"], cm["norm_q"], cm["norm_k"])
         if norms[0].eps != norms[1].eps or any(type(n) is not WanRMSNorm for n in norms) or _has_hooks(sa, ca, norm3, *norms):
             return None
+        if not (_OWN_BLOCK.of(self) and _OWN_SELF_ATTENTION.of(sa) and _OWN_CROSS_ATTENTION.of(ca) and _OWN_RMS_NORM.of(norms[2])):
+            return None
         linears = (sm["q"], sm["k"], sm["v"], sm["o"], cm["q"], cm["k"], cm["v"], cm["o"], ffn[0], ffn[2])
         rule, layers = None, []
         for m in linears:
@@ -395,6 +404,9 @@ class DiTBlock(nn.Module):
         return norm(x, amax_out=ticket), ticket
 
 
+_OWN_BLOCK = OwnMethods(DiTBlock, "_normalized_for", "_feed_forward")
+
+
 class CausalHead(nn.Module):
     def __init__(self, dim: int, out_dim: int, patch_size, eps: float = 1e-6) -> None:
         super().__init__()
@@ -415,10 +427,13 @@ class CausalHead(nn.Module):
         """``unpatchify(forward(x, e))`` as one native call, the linear layer writing the latents in place of its rows; None
         where the modules have to run."""
         if not x.is_cuda or type(self.norm) is not WanLayerNorm or type(self.head) is not nn.Linear or self.norm.weight is not None \
-                or _has_hooks(self, self.norm, self.head):
+                or not _OWN_HEAD.of(self) or _has_hooks(self, self.norm, self.head):
             return None
         return _native.host().head(x, self.modulation.unsqueeze(1) + e, self.head.weight, self.head.bias, self.norm.eps, channels,
                                    tuple(grid), tuple(patch_size))
+
+
+_OWN_HEAD = OwnMethods(CausalHead, "forward")
 
 
 def sinusoidal_embedding_1d(dim: int, position: torch.Tensor) -> torch.Tensor:
@@ -573,9 +588,12 @@ class CausalDiT(nn.Module):
                 kvc.apply_cache_update(kv_cache[i], cur_end, loc_end, info, self.kv_quant_config)
         if cache_only:
             return None
-        if type(self.head) is CausalHead:
+        if type(self.head) is CausalHead and _OWN_MODEL.of(self):   # head and unpatchify in one
             latents = self.head.latents(x, e.unsqueeze(2), (f, h, w), cfg.patch_size, cfg.out_dim)
             if latents is not None:
                 return latents
         x = self.head(x, e.unsqueeze(2))
         return self.unpatchify(x[0].flatten(0, 1) if x.dim() == 4 else x[0], (f, h, w))
+
+
+_OWN_MODEL = OwnMethods(CausalDiT, "unpatchify")

@@ -1076,3 +1076,55 @@ def test_patch_embedding_and_head_against_their_modules(gpu, monkeypatch, dim, c
         assert got.shape == other.shape == ref.shape
         bound = ref.abs() * 2 ** -8 + size * (a.shape[1] + 2) * 2 ** -24
         assert ((got.double() - ref).abs() <= bound).all() and ((other.double() - ref).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("method", ["_normalized_for", "_feed_forward", "self_attn.forward", "cross_attn.forward"])
+def test_block_calls_the_methods_put_in_place_of_its_own(gpu, monkeypatch, method):
+    """A block is one native call only while the methods that the call stands for are the package's: a subclass's, an
+    instance's or a patched class's run instead, with the same bits here."""
+    dim, heads, F, L = 256, 2, 1, 64
+    block, _ = quantize_model_with_filter(DiTBlock(dim, 512, heads).to(gpu), ModelQuantizationConfig(), use_default_filtered_modules=True,
+                                          materialize_for_inference=True, verbose=False)
+    g = torch.Generator().manual_seed(8)
+    x, ctx = (torch.randn(1, n, dim, generator=g).bfloat16().to(gpu) for n in (L, 16))
+    e = torch.randn(1, F, 6, dim, generator=g).bfloat16().to(gpu)
+    cos, sin = rope_cos_sin(build_rope_angles(128), F, 8, 8, 0, gpu)
+
+    def run():
+        return block(x, e, cos, sin, ctx, kvc.initialize_kv_cache(1, L, 2, heads, 128, KV, gpu)[0], 0, sink_tokens=0)[0]
+
+    *path, name = method.split(".")
+    owner = block.get_submodule(".".join(path))
+    cls, calls, original = type(owner), [], getattr(type(owner), name)
+
+    def replacement(self, *args, **kwargs):
+        calls.append(name)
+        return original(self, *args, **kwargs)
+
+    with torch.no_grad():
+        want = run()
+        owner.__class__ = type("Mine", (cls,), {name: replacement})
+        assert torch.equal(run(), want) and calls
+        owner.__class__ = cls
+        for target, value in ((cls, replacement), (owner, replacement.__get__(owner))):
+            calls.clear()
+            with monkeypatch.context() as m:
+                m.setattr(target, name, value)
+                assert torch.equal(run(), want) and calls
+
+
+def test_model_calls_an_unpatchify_of_its_own(gpu):
+    class Mine(CausalDiT):
+        def unpatchify(self, x, grid):
+            return super().unpatchify(x, grid) + 1
+
+    cfg = DiTConfig(dim=256, ffn_dim=512, num_heads=2, num_layers=1, text_dim=64, text_len=16)
+    gen = StreamingGenerator(cfg, gpu)
+    gen.reset_cache(4 * 16)
+    x, ctx = torch.randn(cfg.in_dim, 3, 8, 32, device=gpu).bfloat16(), torch.randn(16, 64, device=gpu).bfloat16()
+    outs = []
+    for cls in (CausalDiT, Mine):
+        gen.model.__class__ = cls
+        outs.append(gen.model(x, torch.full((1, 3), 250.0, device=gpu), ctx, gen.kv_cache, 0, apply_cache_updates=False).float())
+    # both heads round one fp32 sum to bf16, the second rounds its sum with 1 once more: a step of either apart at most
+    assert ((outs[1] - 1 - outs[0]).abs() <= 2 ** -7 * (outs[0].abs() + 1)).all()

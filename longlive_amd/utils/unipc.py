@@ -28,6 +28,7 @@ import numpy as np
 import torch
 
 from .. import _native
+from .._own_methods import OwnMethods
 
 
 @dataclass
@@ -188,8 +189,8 @@ class FlowUniPCMultistepScheduler:
 
     def _fused_step(self, model_output, sample, correct: bool):
         """(x0 prediction, corrected sample, next sample) by one launch, or None where the tensor expressions have to run
-        (anything but bf16 CUDA tensors of one shape without gradients, a higher order)."""
-        if type(model_output) is not torch.Tensor or not model_output.is_cuda or model_output.dtype != torch.bfloat16 \
+        (anything but bf16 CUDA tensors of one shape without gradients, a higher order, methods of its own)."""
+        if not _OWN.of(self) or type(model_output) is not torch.Tensor or not model_output.is_cuda or model_output.dtype != torch.bfloat16 \
                 or torch.get_default_dtype() != torch.float32 or self.sigmas.dtype != torch.float32:
             return None
         order, corrector_order = self._predictor_order(), self.this_order if correct else 0
@@ -250,6 +251,10 @@ class FlowUniPCMultistepScheduler:
 
     def __len__(self) -> int:
         return self.num_train_timesteps
+
+
+# what the one launch stands for
+_OWN = OwnMethods(FlowUniPCMultistepScheduler, "convert_model_output", "_predict", "_correct", "_differences", "_lambda")
 
 
 def convert_flow_pred_to_x0(flow_pred: torch.Tensor, xt: torch.Tensor, sigma_t) -> torch.Tensor:

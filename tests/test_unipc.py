@@ -181,3 +181,25 @@ def test_one_launch_step_has_the_bits_of_the_tensor_expressions(gpu, monkeypatch
     sch.set_timesteps(2, device=gpu)
     flow = torch.ones(4, device=gpu, dtype=torch.bfloat16, requires_grad=True)
     assert sch.step(flow, sch.timesteps[0], torch.ones_like(flow), return_dict=False)[0].requires_grad
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("method", ["convert_model_output", "_predict", "_correct"])
+def test_step_calls_the_methods_put_in_place_of_its_own(gpu, method):
+    """A scheduler whose pieces of a step are a subclass's runs them instead of the one launch."""
+    calls = []
+
+    def replacement(self, *args):
+        calls.append(method)
+        return getattr(super(Mine, self), method)(*args) + 1
+
+    Mine = type("Mine", (FlowUniPCMultistepScheduler,), {method: replacement})
+    outs = []
+    for cls in (FlowUniPCMultistepScheduler, Mine):
+        sch = cls(shift=1)
+        sch.set_timesteps(3, device=gpu, shift=5.0)
+        x = torch.zeros(16, device=gpu, dtype=torch.bfloat16)
+        for t in sch.timesteps:
+            x = sch.step(torch.ones_like(x), t, x, return_dict=False)[0]
+        outs.append(x)
+    assert len(calls) == (2 if method == "_correct" else 3) and not torch.equal(*outs)

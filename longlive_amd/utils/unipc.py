@@ -64,15 +64,16 @@ def _step_scalars(sigma_t: float, sigma_s0: float, older: tuple, order: int, sol
     """(order, ratio, m0, b, rho, rk, rho_new) of ``ll_unipc_scalars`` for a step from sigma_s0 to sigma_t whose history
     reaches back to the sigmas ``older`` (order - 1 of them): the scalars of ``_predict`` / ``_correct``, formed by
     the same float32 operations."""
-    lam = FlowUniPCMultistepScheduler._lambda
-    s_t, s_0 = (torch.tensor(s, dtype=torch.float32) for s in (sigma_t, sigma_s0))
-    alpha_t, lambda_s0 = 1 - s_t, lam(s_0)
-    h = lam(s_t) - lambda_s0
-    rks = [(lam(torch.tensor(s, dtype=torch.float32)) - lambda_s0) / h for s in older] + [1.0]
-    R, b, h_phi_1, B_h = unipc_weights(order, torch.tensor(rks), -h, solver_type)
-    rhos = torch.linalg.solve(R, b) if corrector and order > 1 else torch.tensor([0.5])
-    rhos = rhos.to(torch.bfloat16).tolist()
-    return (order, (s_t / s_0).item(), (alpha_t * h_phi_1).item(), (alpha_t * B_h).item(), rhos[0], float(rks[0]), rhos[-1])
+    with torch.device("cpu"):   # what is kept is the same under whatever default device a step is first called
+        lam = FlowUniPCMultistepScheduler._lambda
+        s_t, s_0 = (torch.tensor(s, dtype=torch.float32) for s in (sigma_t, sigma_s0))
+        alpha_t, lambda_s0 = 1 - s_t, lam(s_0)
+        h = lam(s_t) - lambda_s0
+        rks = [(lam(torch.tensor(s, dtype=torch.float32)) - lambda_s0) / h for s in older] + [1.0]
+        R, b, h_phi_1, B_h = unipc_weights(order, torch.tensor(rks), -h, solver_type)
+        rhos = torch.linalg.solve(R, b) if corrector and order > 1 else torch.tensor([0.5])
+        rhos = rhos.to(torch.bfloat16).tolist()
+        return (order, (s_t / s_0).item(), (alpha_t * h_phi_1).item(), (alpha_t * B_h).item(), rhos[0], float(rks[0]), rhos[-1])
 
 
 class FlowUniPCMultistepScheduler:

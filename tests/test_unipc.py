@@ -8,6 +8,7 @@ import torch
 from scipy.integrate import quad
 
 import unipc_oracle as uo
+from longlive_amd.utils import unipc
 from longlive_amd.utils.unipc import FlowUniPCMultistepScheduler, convert_flow_pred_to_x0
 
 
@@ -203,3 +204,13 @@ def test_step_calls_the_methods_put_in_place_of_its_own(gpu, method):
             x = sch.step(torch.ones_like(x), t, x, return_dict=False)[0]
         outs.append(x)
     assert len(calls) == (2 if method == "_correct" else 3) and not torch.equal(*outs)
+
+
+def test_scalars_of_a_step_do_not_depend_on_the_default_device():
+    """They are kept per schedule, so the first call must not leave another device's arithmetic behind."""
+    args = (0.6, 0.8, (0.9,), 2, "bh2", True)
+    unipc._step_scalars.cache_clear()
+    want = unipc._step_scalars(*args)
+    unipc._step_scalars.cache_clear()
+    with torch.device("meta"):
+        assert unipc._step_scalars(*args) == want

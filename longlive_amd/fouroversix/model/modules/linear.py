@@ -133,7 +133,7 @@ class FourOverSixLinear(nn.Linear):
             rule = config.activation_scale_rule._value_
             out = _native.host().linear(x2d, _native.RULE_IDS[rule], _native.DENOMINATORS[rule], weight.values, weight.scale_factors,
                                         weight.amax, _native.DENOMINATORS[weight.scale_rule._value_], weight.original_shape[0],
-                                        self._parameters.get("bias"))
+                                        self.bias)
             if out is not None:
                 return out
         return self.forward_quantized(self.quantize_input(x2d))
@@ -145,7 +145,7 @@ class FourOverSixLinear(nn.Linear):
         config, weight = self.config, self.quantized_weight()
         if not _OWN.of(self) or not isinstance(weight, QuantizedTensor) or config.output_dtype is not DataType.bfloat16 or config.dtype is not DataType.nvfp4:
             return None
-        return (weight.values, weight.scale_factors, weight.amax, self._parameters.get("bias"),
+        return (weight.values, weight.scale_factors, weight.amax, self.bias,
                 _native.DENOMINATORS[weight.scale_rule._value_], weight.original_shape[0])
 
     def quantize_input(self, x2d: torch.Tensor, amax=None) -> QuantizedTensor:

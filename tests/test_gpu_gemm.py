@@ -832,3 +832,19 @@ def test_linear_layer_calls_the_methods_put_in_place_of_its_own(gpu, monkeypatch
         else:
             monkeypatch.setattr(FourOverSixLinear, method, replacement)
         assert torch.equal(layer(x), want) and calls == [method] and layer.native_operand() is None
+
+
+def test_linear_layer_whose_bias_is_no_parameter(gpu):
+    """A bias held as a buffer (or any attribute) is added as a parameter is."""
+    from longlive_amd.fouroversix import ModelQuantizationConfig
+    from longlive_amd.utils.quant import quantize_model_with_filter
+
+    model, _ = quantize_model_with_filter(torch.nn.Sequential(torch.nn.Linear(256, 128)).to(gpu), ModelQuantizationConfig(),
+                                          materialize_for_inference=True, verbose=False)
+    layer, x = model[0], activations((48, 256), 5).to(gpu)
+    with torch.no_grad():
+        layer.bias.normal_()
+        want, bias = layer(x), layer.bias.data
+        del layer.bias
+        layer.register_buffer("bias", bias)
+        assert torch.equal(layer(x), want) and layer.native_operand()[3] is bias

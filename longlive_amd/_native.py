@@ -9,6 +9,7 @@ from __future__ import annotations
 import ctypes
 import os
 import re
+import warnings
 from ctypes import c_char_p, c_float, c_int, c_int64, c_size_t, c_void_p
 
 import torch
@@ -142,17 +143,34 @@ def load():
 _host = None
 
 
+class _NoHostPath:
+    """In place of the native host path where that does not load: takes no call, so that every one goes through ctypes."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
+def load_host():
+    """The native host path (csrc/host_ops.cpp).  Raises ImportError unless it was built for this Python and this torch,
+    whose internals it is linked against."""
+    from . import _host_ops
+    if _host_ops.TORCH_VERSION != torch.__version__:
+        raise ImportError(f"built for torch {_host_ops.TORCH_VERSION}, running under {torch.__version__}")
+    return _host_ops
+
+
 def host():
-    """The native host path (csrc/host_ops.cpp): whole calls from tensors to launches.  Raises if it has not been built."""
+    """The native host path: whole calls from tensors to launches, each None for a call it does not take.  The library
+    alone does the same work through ctypes, call by call, so a host path that does not load is worth a warning only."""
     global _host
     if _host is None:
         load()
         try:
-            from . import _host_ops
+            _host = load_host()
         except ImportError as e:
-            raise RuntimeError(f"longlive_amd/_host_ops.so is missing or does not load ({e}): build it with "
-                               "`python -c 'import __graft_entry__ as g; g.build()'`") from e
-        _host = _host_ops
+            warnings.warn(f"longlive_amd._host_ops does not load ({e}): small calls will take several times their host time; build it "
+                          "with `python -c 'import __graft_entry__ as g; g.build()'`", RuntimeWarning, stacklevel=2)
+            _host = _NoHostPath()
     return _host
 
 
@@ -885,6 +903,8 @@ def block_forward(x, e, layers, norms, cos, sin, window, text, rule: str, sizes,
     The other tensor maxima go through a sink of the current stream, or through that of an active recording; a recording
     without one is not taken."""
     lib, graph, graph_sink = host(), _active_graph_sinks.get(_device_key(x.device)), None
+    if isinstance(lib, _NoHostPath):
+        return None
     if graph is not None:
         graph_sink = (graph.parts, graph.entry[1], graph.offset)
         graph.entry[1] += lib.EPOCHS_PER_CALL

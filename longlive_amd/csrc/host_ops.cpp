@@ -857,5 +857,6 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host_ops", nullptr, -1, methods, 
 PyMODINIT_FUNC PyInit__host_ops(void) {
   PyObject* m = PyModule_Create(&module);
   if (m) PyModule_AddIntConstant(m, "EPOCHS_PER_CALL", kEpochsPerCall);
+  if (m) PyModule_AddStringConstant(m, "TORCH_VERSION", LL_TORCH_VERSION);
   return m;
 }

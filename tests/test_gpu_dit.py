@@ -1128,3 +1128,29 @@ def test_model_calls_an_unpatchify_of_its_own(gpu):
         outs.append(gen.model(x, torch.full((1, 3), 250.0, device=gpu), ctx, gen.kv_cache, 0, apply_cache_updates=False).float())
     # both heads round one fp32 sum to bf16, the second rounds its sum with 1 once more: a step of either apart at most
     assert ((outs[1] - 1 - outs[0]).abs() <= 2 ** -7 * (outs[0].abs() + 1)).all()
+
+
+def test_without_the_native_host_path_the_same_bits(gpu, monkeypatch):
+    """Every call goes through ctypes where the host path does not load: a linear layer, a block with its cache write and a
+    dequantization give the same bits."""
+    from longlive_amd import _native
+
+    dim, heads, F, L = 256, 2, 1, 64
+    block, _ = quantize_model_with_filter(DiTBlock(dim, 512, heads).to(gpu), ModelQuantizationConfig(), use_default_filtered_modules=True,
+                                          materialize_for_inference=True, verbose=False)
+    g = torch.Generator().manual_seed(9)
+    x, ctx = (torch.randn(1, n, dim, generator=g).bfloat16().to(gpu) for n in (L, 16))
+    e = torch.randn(1, F, 6, dim, generator=g).bfloat16().to(gpu)
+    cos, sin = rope_cos_sin(build_rope_angles(128), F, 8, 8, 0, gpu)
+
+    def run():
+        cache = kvc.initialize_kv_cache(1, L, 2, heads, 128, KV, gpu)[0]
+        y, update = block(x, e, cos, sin, ctx, cache, 0, sink_tokens=0)
+        kvc.apply_cache_update(cache, *update, KV)
+        slots = [cache[n][0] for n in "kv"]
+        return [y, block.self_attn.q(x)] + [t for s in slots for t in (s.values, s.scale_factors.view(torch.uint8), s.amax, s.dequantize())]
+
+    with torch.no_grad():
+        want = run()
+        monkeypatch.setattr(_native, "_host", _native._NoHostPath())
+        assert all(torch.equal(a, b) for a, b in zip(run(), want))

@@ -534,3 +534,16 @@ def test_parts_of_small_products_fit_their_memory():
     for cus, M, N, K, products in itertools.product((1, 64, 256, 304), (1, 64, 65, 500), (8, 640, 3072), (64, 3840, 4096, 20000), (1, 3)):
         parts, tiles = small_gemm_parts(M, N, K, products, cus), -(-M // 64) * -(-N // 64) * products
         assert 1 <= parts <= 4 and parts <= -(-K // 256) and (parts == 1 or tiles * parts <= 2 * cus)
+
+
+def test_host_path_is_built_for_this_torch_and_optional(monkeypatch):
+    """The native host path loads here; where it does not (another torch, no file) calls fall to the general path with one
+    warning."""
+    assert _native.load_host().TORCH_VERSION == torch.__version__ and _native.host() is _native.load_host()
+    monkeypatch.setattr(_native, "_host", None)
+    monkeypatch.setattr(_native.load_host(), "TORCH_VERSION", "0.0")
+    with pytest.warns(RuntimeWarning, match="built for torch 0.0"):
+        assert _native.host().quantize(torch.zeros(1), 0) is None
+    with pytest.raises(ValueError, match="GPU only"):
+        quantize_to_fp4(torch.zeros(16, 16, dtype=torch.bfloat16))
+    assert _native.block_forward(torch.zeros(1), *[None] * 7, "mse", (), False, ()) is None

@@ -429,7 +429,10 @@ class CausalHead(nn.Module):
         if not x.is_cuda or type(self.norm) is not WanLayerNorm or type(self.head) is not nn.Linear or self.norm.weight is not None \
                 or not _OWN_HEAD.of(self) or _has_hooks(self, self.norm, self.head):
             return None
-        return _native.host().head(x, self.modulation.unsqueeze(1) + e, self.head.weight, self.head.bias, self.norm.eps, channels,
+        host = _native.host()
+        if not host.head_takes(x.shape[1], x.shape[2]):
+            return None
+        return host.head(x, self.modulation.unsqueeze(1) + e, self.head.weight, self.head.bias, self.norm.eps, channels,
                                    tuple(grid), tuple(patch_size))
 
 

@@ -1154,3 +1154,20 @@ def test_without_the_native_host_path_the_same_bits(gpu, monkeypatch):
         want = run()
         monkeypatch.setattr(_native, "_host", _native._NoHostPath())
         assert all(torch.equal(a, b) for a, b in zip(run(), want))
+
+
+@pytest.mark.parametrize("dim,grid,head,embedding", [
+    (256, (3, 4, 16), True, True), (1024, (1, 28, 32), True, True), (2304, (1, 12, 16), True, True),
+    (3072, (1, 12, 16), False, True), (2304, (1, 24, 16), False, True), (1536, (1, 24, 32), False, True),
+    (3072, (1, 28, 32), False, False), (256, (3, 22, 40), False, False),
+])
+def test_which_calls_the_ends_of_the_model_run_themselves(gpu, dim, grid, head, embedding):
+    """The lines of host_ops.cpp between the package's kernels and torch's products, on both sides of them."""
+    from longlive_amd import _native
+
+    f, h, w = grid
+    x, weight = torch.randn(48, f, 2 * h, 2 * w, device=gpu).bfloat16(), torch.randn(dim, 192, device=gpu).bfloat16()
+    y, e = torch.randn(1, f * h * w, dim, device=gpu).bfloat16(), torch.randn(1, f, 2, dim, device=gpu).bfloat16()
+    lib = _native.host()
+    assert (lib.patch_embed(x, weight, None, dim, 1, 2, 2) is not None) == embedding
+    assert (lib.head(y, e, weight.t().contiguous(), None, 1e-6, 48, grid, (1, 2, 2)) is not None) == head == lib.head_takes(f * h * w, dim)

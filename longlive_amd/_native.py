@@ -248,10 +248,16 @@ def _device_key(device: torch.device):
     return (device.type, index)
 
 
-def recording(device: torch.device) -> bool:
-    """Whether launches on the device's current stream are being recorded into a graph."""
+def recording(device: torch.device, replayable: bool = False) -> bool:
+    """Whether launches on the device's current stream are being recorded into a graph; ``replayable``: or a
+    :class:`ReplayableAmaxSink` of the device is active."""
     if device.type != "cuda":
         return False
+    if replayable and _active_graph_sinks and _device_key(device) in _active_graph_sinks:
+        return True
+    answer = host().recording(-1 if device.index is None else device.index)
+    if answer is not None:
+        return answer
     if device.index is None or device.index == torch.cuda.current_device():
         return torch.cuda.is_current_stream_capturing()
     with torch.cuda.device(device):
@@ -272,8 +278,10 @@ class PrivateAmaxSink:
         all its producers, whose slots the next producer overwrites, and no place for a maximum that is consumed
         after the forward.  Without a ticket the producer leaves nothing behind and the consumer reduces the tensor
         itself."""
-        if _device_key(self.parts.device) in _active_graph_sinks or recording(self.parts.device):
-            return None
+        return None if recording(self.parts.device, replayable=True) else self.next_ticket()
+
+    def next_ticket(self) -> "AmaxTicket":
+        """:meth:`ticket` for a caller that knows of no recording."""
         if self.entry[1] >= 0xFFFFFFFE:
             self.parts.zero_()
             self.entry[1] = 0

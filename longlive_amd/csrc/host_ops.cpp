@@ -840,6 +840,16 @@ PyObject* py_unipc_step(PyObject*, PyObject* const* args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// recording(device index, -1: the current one) -> whether launches on the device's current stream are being recorded
+PyObject* py_recording(PyObject*, PyObject* arg) {
+  HANDLE_TH_ERRORS
+  const int64_t dev = PyLong_AsLongLong(arg);
+  if (PyErr_Occurred()) return nullptr;
+  if (recording(stream_of(dev < 0 ? c10::hip::current_device() : (int)dev))) Py_RETURN_TRUE;
+  Py_RETURN_FALSE;
+  END_HANDLE_TH_ERRORS
+}
+
 // current_stream() -> the current HIP stream of the current device as an integer
 PyObject* py_current_stream(PyObject*, PyObject*) {
   HANDLE_TH_ERRORS
@@ -866,6 +876,7 @@ PyMethodDef methods[] = {
     {"head", (PyCFunction)(void (*)(void))py_head, METH_FASTCALL, nullptr},
     {"head_takes", (PyCFunction)(void (*)(void))py_head_takes, METH_FASTCALL, nullptr},
     {"unipc_step", (PyCFunction)(void (*)(void))py_unipc_step, METH_FASTCALL, nullptr},
+    {"recording", py_recording, METH_O, nullptr},
     {"current_stream", py_current_stream, METH_NOARGS, nullptr},
     {"release_stream_sink", py_release_stream_sink, METH_NOARGS, nullptr},
     {"quantize", (PyCFunction)(void (*)(void))py_quantize, METH_FASTCALL, nullptr},

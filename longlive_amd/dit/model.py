@@ -18,7 +18,7 @@ import torch.nn as nn
 
 from .. import _native
 from .._own_methods import OwnMethods
-from ..fouroversix.model.modules.linear import FourOverSixLinear
+from ..fouroversix.model.modules.linear import OWN as OWN_LINEAR, FourOverSixLinear
 from ..utils import kv_cache as kvc
 from ..utils.adaln import adaln_modulate, gate_residual
 from ..utils.rope import build_rope_angles, rope_apply, rope_cos_sin
@@ -149,12 +149,12 @@ class CausalSelfAttention(nn.Module):
     def amax_tickets(kv_cache: dict, device):
         """Tickets of the two sinks of a layer's cache in which the producers of K and V leave the maxima for the cache
         write.  None for both in a recording, which has no place for them (and whose memory a sink must not be made of)."""
-        if _native.recording(device):
+        if _native.recording(device, replayable=True):
             return None, None
         sinks = kv_cache.get("_amax_sinks")
         if sinks is None:
             sinks = kv_cache["_amax_sinks"] = (_native.PrivateAmaxSink(device), _native.PrivateAmaxSink(device))
-        return tuple(sink.ticket() for sink in sinks)
+        return sinks[0].next_ticket(), sinks[1].next_ticket()
 
     def forward(self, x, cos, sin, kv_cache, current_start, sink_tokens, max_attention_size, *, input_amax=None,
                 residual=None, gate=None, gate_rows=0, global_sink_tokens=0, rope_fn=None, collect_kv_amax=True,
@@ -347,7 +347,7 @@ class DiTBlock(nn.Module):
         norms = (sm["norm_q"], sm["norm_k"], cm["norm_q"], cm["norm_k"])
         if norms[0].eps != norms[1].eps or any(type(n) is not WanRMSNorm for n in norms) or _has_hooks(sa, ca, norm3, *norms):
             return None
-        if not (_OWN_BLOCK.of(self) and _OWN_SELF_ATTENTION.of(sa) and _OWN_CROSS_ATTENTION.of(ca) and _OWN_RMS_NORM.of(norms[2])):
+        if not (OWN_LINEAR.of_class(FourOverSixLinear) and _OWN_BLOCK.of(self) and _OWN_SELF_ATTENTION.of(sa) and _OWN_CROSS_ATTENTION.of(ca) and _OWN_RMS_NORM.of(norms[2])):
             return None
         linears = (sm["q"], sm["k"], sm["v"], sm["o"], cm["q"], cm["k"], cm["v"], cm["o"], ffn[0], ffn[2])
         rule, layers = None, []

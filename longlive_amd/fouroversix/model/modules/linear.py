@@ -127,25 +127,34 @@ class FourOverSixLinear(nn.Linear):
 
     def _forward_2d(self, x2d: torch.Tensor) -> torch.Tensor:
         weight, config = self.quantized_weight(), self.config
-        if (_OWN.of(self) and isinstance(weight, QuantizedTensor) and config.output_dtype is DataType.bfloat16 and config.dtype is DataType.nvfp4
+        if (OWN.of(self) and isinstance(weight, QuantizedTensor) and config.output_dtype is DataType.bfloat16 and config.dtype is DataType.nvfp4
                 and weight.original_shape[1] == x2d.shape[1]):
             # quantization and product as one native call; the operand between them has no other reader
             rule = config.activation_scale_rule._value_
             out = _native.host().linear(x2d, _native.RULE_IDS[rule], _native.DENOMINATORS[rule], weight.values, weight.scale_factors,
                                         weight.amax, _native.DENOMINATORS[weight.scale_rule._value_], weight.original_shape[0],
-                                        self.bias)
+                                        self._bias())
             if out is not None:
                 return out
         return self.forward_quantized(self.quantize_input(x2d))
 
+    def _bias(self):
+        """``self.bias`` without the module's attribute search for the common case of a parameter (or none)."""
+        parameters = self._parameters
+        return parameters["bias"] if "bias" in parameters else self.bias
+
     def native_operand(self):
         """(values, scale factors, amax, bias or None, denominator, out_features) for the native calls that run this
         layer among others; ``None`` when it has no quantized weight, another type than NVFP4 in, bf16 out, or methods
-        of its own."""
-        config, weight = self.config, self.quantized_weight()
-        if not _OWN.of(self) or not isinstance(weight, QuantizedTensor) or config.output_dtype is not DataType.bfloat16 or config.dtype is not DataType.nvfp4:
+        in place of those that such a call stands for.  Of those only the ones held by the layer itself are looked for:
+        the caller asks ``OWN.of_class`` once for all its layers."""
+        held = self.__dict__
+        if "quantize_input" in held or "quantize_normalized_input" in held or "forward_quantized" in held or "forward_quantized_together" in held:
             return None
-        return (weight.values, weight.scale_factors, weight.amax, self.bias,
+        config, weight = held["config"], held.get("_quantized_weight") or self.quantized_weight()
+        if not isinstance(weight, QuantizedTensor) or config.output_dtype is not DataType.bfloat16 or config.dtype is not DataType.nvfp4:
+            return None
+        return (weight.values, weight.scale_factors, weight.amax, self._bias(),
                 _native.DENOMINATORS[weight.scale_rule._value_], weight.original_shape[0])
 
     def quantize_input(self, x2d: torch.Tensor, amax=None) -> QuantizedTensor:
@@ -218,4 +227,4 @@ class FourOverSixLinear(nn.Linear):
 
 
 # what the native calls stand for
-_OWN = OwnMethods(FourOverSixLinear, "quantize_input", "quantize_normalized_input", "forward_quantized", "forward_quantized_together")
+OWN = OwnMethods(FourOverSixLinear, "quantize_input", "quantize_normalized_input", "forward_quantized", "forward_quantized_together")

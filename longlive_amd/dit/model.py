@@ -426,14 +426,15 @@ class CausalHead(nn.Module):
     def latents(self, x, e, grid, patch_size, channels: int):
         """``unpatchify(forward(x, e))`` as one native call, the linear layer writing the latents in place of its rows; None
         where the modules have to run."""
-        if not x.is_cuda or type(self.norm) is not WanLayerNorm or type(self.head) is not nn.Linear or self.norm.weight is not None \
-                or not _OWN_HEAD.of(self) or _has_hooks(self, self.norm, self.head):
+        norm, head = (self._modules[name] for name in ("norm", "head"))
+        if not x.is_cuda or type(norm) is not WanLayerNorm or type(head) is not nn.Linear or norm.weight is not None \
+                or not _OWN_HEAD.of(self) or _has_hooks(self, norm, head):
             return None
         host = _native.host()
         if not host.head_takes(x.shape[1], x.shape[2]):
             return None
-        return host.head(x, self.modulation.unsqueeze(1) + e, self.head.weight, self.head.bias, self.norm.eps, channels,
-                                   tuple(grid), tuple(patch_size))
+        return host.head(x, self.modulation.unsqueeze(1) + e, head.weight, head.bias, norm.eps, channels, tuple(grid),
+                         tuple(patch_size))
 
 
 _OWN_HEAD = OwnMethods(CausalHead, "forward")

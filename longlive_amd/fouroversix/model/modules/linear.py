@@ -126,8 +126,9 @@ class FourOverSixLinear(nn.Linear):
         return out.reshape(*input.shape[:-1], out.shape[-1])
 
     def _forward_2d(self, x2d: torch.Tensor) -> torch.Tensor:
-        weight, config = self.quantized_weight(), self.config
-        if (OWN.of(self) and isinstance(weight, QuantizedTensor) and config.output_dtype is DataType.bfloat16 and config.dtype is DataType.nvfp4
+        held = self.__dict__
+        weight, config = held.get("_quantized_weight") or self.quantized_weight(), held["config"]
+        if (_OWN_FORWARD.of(self) and isinstance(weight, QuantizedTensor) and config.output_dtype is DataType.bfloat16 and config.dtype is DataType.nvfp4
                 and weight.original_shape[1] == x2d.shape[1]):
             # quantization and product as one native call; the operand between them has no other reader
             rule = config.activation_scale_rule._value_
@@ -226,5 +227,6 @@ class FourOverSixLinear(nn.Linear):
                           amax_out=amax_out)
 
 
-# what the native calls stand for
+# what the native calls stand for: forward, the calls that run several layers
+_OWN_FORWARD = OwnMethods(FourOverSixLinear, "quantize_input", "forward_quantized")
 OWN = OwnMethods(FourOverSixLinear, "quantize_input", "quantize_normalized_input", "forward_quantized", "forward_quantized_together")

@@ -62,8 +62,14 @@ _MAX_TABLES = 16
 
 def _tables_for(cache: dict, slot_ids: tuple[int, ...]):
     # keyed by the buffers, not by the positions: a roll moves the buffers through the positions (apply_cache_update),
-    # and the handful of arrangements that a streaming run cycles through are each built once
-    key = tuple(cache["k"][i].values.data_ptr() for i in slot_ids)
+    # and the handful of arrangements that a streaming run cycles through are each built once.  By all of them: a table
+    # holds nothing but their addresses, so that one found here is right whatever has been put into the cache meanwhile.
+    key = []
+    for slots in (cache["k"], cache["v"]):
+        for i in slot_ids:
+            s = slots[i]
+            key += s.values.data_ptr(), s.scale_factors.data_ptr(), s.amax.data_ptr()
+    key = tuple(key)
     tables = cache["_tables"]
     entry = tables.pop(key, None)
     if entry is None:

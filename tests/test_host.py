@@ -547,3 +547,21 @@ def test_host_path_is_built_for_this_torch_and_optional(monkeypatch):
     with pytest.raises(ValueError, match="GPU only"):
         quantize_to_fp4(torch.zeros(16, 16, dtype=torch.bfloat16))
     assert _native.block_forward(torch.zeros(1), *[None] * 7, "mse", (), False, ()) is None
+
+
+def test_pointer_tables_follow_every_buffer_of_a_slot():
+    """The tables of the attended slots are kept between calls; a values, scale or amax buffer of K or V that has been
+    replaced gets a table of its own."""
+    def slot():
+        return QuantizedTensor(torch.zeros(128, 64, dtype=torch.uint8), torch.zeros(1024, dtype=torch.uint8).view(torch.float8_e4m3fn),
+                               torch.zeros(1), "nvfp4", (128, 128), "mse", (128, 128))
+
+    cache = {"k": [slot() for _ in range(3)], "v": [slot() for _ in range(3)], "_tables": {}}
+    first = kvc._tables_for(cache, (0, 2))
+    assert kvc._tables_for(cache, (0, 2)) is first
+    for name, attribute in itertools.product("kv", ("values", "scale_factors", "amax")):
+        old = getattr(cache[name][2], attribute)
+        setattr(cache[name][2], attribute, old.clone())
+        kt, vt = kvc._tables_for(cache, (0, 2))
+        for table, slots in ((kt, cache["k"]), (vt, cache["v"])):
+            assert table.table.tolist() == [[getattr(slots[i], a).data_ptr() for i in (0, 2)] for a in ("values", "scale_factors", "amax")]

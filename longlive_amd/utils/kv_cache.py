@@ -264,7 +264,8 @@ def kv_cache_attention_relative(q: torch.Tensor, k: torch.Tensor, v: torch.Tenso
                                                 global_sink_tokens)
     info["new_k"], info["new_v"] = k, v
     scale = D ** -0.5 if softmax_scale is None else softmax_scale
-    if slot_ids is not None and q.is_cuda:   # window, rotations and attention as one native call
+    # window, rotations and attention as one native call, which decodes K and V by one rule
+    if slot_ids is not None and q.is_cuda and cache["k"][0].scale_rule is cache["v"][0].scale_rule:
         frames, new_frames = (len(slot_ids) * cache["block_token_size"] + S) // frame_seqlen, S // frame_seqlen
         out = _native.host().kv_attention_relative(q, k, v, _window(cache, slot_ids), *rope_fn(frames, 0),
                                                    *rope_fn(new_frames, frames - new_frames), float(scale))

@@ -1025,3 +1025,19 @@ def test_the_plan_is_what_the_launch_does(gpu, Lq, H, T, cached, n_new):
             outs[policy] = _native.kv_attention(q, tables, cached, T, 6.0, 256.0, k, v, 128 ** -0.5)
     planned = _native.attention_plan(Lq, H, cached + n_new, n_cached=cached)["division"]
     assert [torch.equal(outs["auto"], outs[p]) for p in ("narrow", "split")] == [planned == "narrow", planned == "split"]
+
+
+def test_relative_rope_over_slots_of_two_scale_rules(gpu, monkeypatch):
+    """K slots under one scale rule and V slots under another: each is decoded by its own, as by the separate operations."""
+    H, T, D = 2, 128, 128
+    cache = kvc.initialize_kv_cache(1, T, 2, H, D, CFG, gpu)[0]
+    rows = [_randn((T * H, D), 90 + i).to(gpu) for i in range(2)]
+    cache["k"][0], cache["v"][0] = (quantize_to_fp4(r, QuantizationConfig(scale_rule=rule)) for r, rule in zip(rows, ("mse", "static_6")))
+    cache["_global_end"] = cache["_local_end"] = T
+    q, k, v = (_randn((1, T, H, D), 93 + i).to(gpu) for i in range(3))
+    angles = build_rope_angles(D)
+    rope_fn = lambda frames, first: rope_cos_sin(angles, frames, 8, 16, first, gpu)
+    run = lambda: kvc.kv_cache_attention_relative(q, k, v, cache, T, 0, rope_fn)[0]
+    got = run()
+    monkeypatch.setattr(_native, "_host", _native._NoHostPath())
+    assert torch.equal(got, run())

@@ -571,8 +571,8 @@ __global__ __launch_bounds__(kAttnThreads) void kv_attention_kernel(AttnParams p
   // The rows of a chunk tile reach LDS in pieces of 1 KB, one load of 64 x 16 bytes each: 34 of K, 36 of V, the rows' padding
   // included (its lanes fetch the row's last 16 bytes again).  Wave w takes pieces w, w + 8, w + 16, w + 24 of either and
   // one of the six behind them; here the source offsets of its lanes.  2640 queries x 24 heads over 13200 bf16 keys take
-  // 400 us; with 32 loads of 4 bytes per lane and iteration (one row each), which cost 100 vector instructions for their
-  // addresses, 446 us; with 10560 of the keys cached 432 instead of 449 us.
+  // 407 us; with 32 loads of 4 bytes per lane and iteration (one row each), which cost 100 vector instructions for their
+  // addresses, 437 us; with 10560 of the keys cached 422 instead of 429 us (one box, in turn).
   constexpr int kKPieces = 2 * kKTileBytes / 1024, kVPieces = 2 * kVTileBytes / 1024;
   static_assert(kKPieces * 1024 == 2 * kKTileBytes && kVPieces * 1024 == 2 * kVTileBytes && kKPieces + kVPieces <= 72, "nine pieces per wave at most");
   const int chunk_wave = __builtin_amdgcn_readfirstlane(wave);
@@ -826,9 +826,11 @@ __global__ __launch_bounds__(kAttnThreads) void kv_attention_kernel(AttnParams p
 // scale bytes of the lane's own, without LDS.  Rows of the chunk (bf16) are loaded four whole rows per instruction
 // and pass through LDS, as V always does (its operand needs the transposing read).
 //
-// Bound by vector instructions (per tile 16 MFMAs beside about 480 others where the keys are cached, 150 where not) and,
-// for the chunk's rows, by the 64 B per clock a CU takes from its L1.  368 queries x 16 heads over 1472 bf16 keys 16.9 us
-// (36.8 in the 256-query kernel), 192 x 12 over 768 cached + 192 keys 15.5 (27.3), 64 x 2 over 128 keys 5.6 (8.0).
+// Bound by the issue of vector instructions (per tile 16 MFMAs beside about 480 others where the keys are cached, 150 where
+// not; counters of the first shape below: a wave issues 36 % of its cycles and waits 26 % for an issue slot, the matrix pipe
+// is busy 15 %) and, for the chunk's rows, by the LDS they pass through (index unit active 32 %, waits for it 12 %).  us, here /
+// in the tile kernels: 368 queries x 16 heads over 1472 bf16 keys 17.9 / 31.5, over 1104 cached + 368 20.5 / 32.1, 192 x 12 over
+// 768 + 192 15.7 / 23.6, 64 x 2 over 128 keys 5.5 / 7.8.
 constexpr int kShortKeys = 32;                                                // keys per wave tile
 constexpr int kShortWaveBytes = kShortKeys * (kKPitch + kVPitch);             // a wave's K and V rows
 constexpr int kShortRecord = 66 * 64;                                         // floats of a wave's result in the merge

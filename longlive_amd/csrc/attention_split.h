@@ -106,7 +106,8 @@ LL_SPLIT_FN uint32_t record_of_part(uint32_t g, uint32_t split_tile, const Divis
 // ---- short launches (host): waves per workgroup with which kv_attention_short_kernel takes a launch, 0 for the tile
 // kernels.  It converts K and V once per 32 queries and fills a compute unit with one workgroup of eight or two of
 // four waves, so it is ahead while everything runs at once and the key range is short (us, tile kernels / 8 waves /
-// 4 waves; "a + b" = cached + chunk keys in tiles of 32):
+// 4 waves; "a + b" = cached + chunk keys in tiles of 32; taken when this kernel rescaled its sums in steps of 2^8, those of
+// 2^2 that it has now cost 1 to 2.5 % and move no line by a measured point):
 //   G <= CUs      368 queries x 16 heads, 0 + 46 tiles 36.8 / 16.9 / 20.3; 512 x 16, 64 + 16: 36.9 / 28.8 / 31.2;
 //                 1024 x 6, 64 + 32: 42.5 / 32.9 / 36.5, but 128 + 32: 48.5 / 50.1 / 57.7 (the divided tiles use all units)
 //   up to 12 tiles four waves have two or three tiles each and half the merge: 64 x 12, 0 + 4: 8.4 / 6.7 / 5.8

@@ -572,7 +572,7 @@ __global__ __launch_bounds__(kAttnThreads) void kv_attention_kernel(AttnParams p
   // included (its lanes fetch the row's last 16 bytes again).  Wave w takes pieces w, w + 8, w + 16, w + 24 of either and
   // one of the six behind them; here the source offsets of its lanes.  2640 queries x 24 heads over 13200 bf16 keys take
   // 407 us; with 32 loads of 4 bytes per lane and iteration (one row each), which cost 100 vector instructions for their
-  // addresses, 437 us; with 10560 of the keys cached 422 instead of 429 us (one box, in turn).
+  // addresses, 437 us; with 10560 of the keys cached 422 instead of 429 us (measured in turn).
   constexpr int kKPieces = 2 * kKTileBytes / 1024, kVPieces = 2 * kVTileBytes / 1024;
   static_assert(kKPieces * 1024 == 2 * kKTileBytes && kVPieces * 1024 == 2 * kVTileBytes && kKPieces + kVPieces <= 72, "nine pieces per wave at most");
   const int chunk_wave = __builtin_amdgcn_readfirstlane(wave);

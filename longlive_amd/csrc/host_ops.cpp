@@ -141,7 +141,8 @@ Epochs epochs_of_stream(int dev, void* stream) {
   if (found == sinks.end() || found->second.epoch > 0xFFFFFF00u) {
     if (found == sinks.end()) found = sinks.emplace(key, StreamSink{empty({(int64_t)LL_AMAX_PARTS}, at::kLong, dev), 0}).first;
     // not through torch's zero_: it may have a mode to report to, or refuse a tensor made in inference mode
-    if (hipMemsetAsync(found->second.parts.data_ptr(), 0, LL_AMAX_PARTS * sizeof(uint64_t), static_cast<hipStream_t>(stream)) != hipSuccess) {
+    if (hipMemsetAsync(found->second.parts.data_ptr(), 0, LL_AMAX_PARTS * sizeof(uint64_t),
+                       static_cast<hipStream_t>(stream)) != hipSuccess) {
       (void)hipGetLastError();
       sinks.erase(found);
       return Epochs{nullptr, nullptr, 0};
@@ -156,8 +157,8 @@ Epochs epochs_of_stream(int dev, void* stream) {
 
 // The amax of x and its quantization: one launch for a small tensor, two otherwise and while the stream is being captured.
 constexpr int64_t kSpinLimit = 64;  // looks of one to two microseconds at the other workgroups' maxima
-int quantize_operand(const void* x, int64_t M, int64_t K, int64_t ldx, int rule, uint8_t* values, uint8_t* scales, float* amax, float* workspace,
-                     int dev, void* stream) {
+int quantize_operand(const void* x, int64_t M, int64_t K, int64_t ldx, int rule, uint8_t* values, uint8_t* scales, float* amax,
+                     float* workspace, int dev, void* stream) {
   if (K % 64 == 0 && ((M + 127) / 128) * (K / 64) <= 256) {
     Epochs e = epochs_of_stream(dev, stream);
     if (e.parts) {
@@ -180,9 +181,9 @@ PyObject* py_quantize(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const int rule = (int)PyLong_AsLong(args[1]);
   const Tensor values = empty({Mp, Kp / 2}, at::kByte, dev), scales = empty({Mp * Kp / 16}, at::kFloat8_e4m3fn, dev),
                amax = empty({1}, at::kFloat, dev), ws = empty({(int64_t)LL_AMAX_PARTS}, at::kFloat, dev);
-  if (failed(quantize_operand(x.data_ptr(), M, K, x.stride(0), rule, values.data_ptr<uint8_t>(), static_cast<uint8_t*>(scales.data_ptr()),
-                              amax.data_ptr<float>(), ws.data_ptr<float>(), dev, stream_of(dev)),
-             "ll_nvfp4_quantize"))
+  if (failed(quantize_operand(x.data_ptr(), M, K, x.stride(0), rule, values.data_ptr<uint8_t>(),
+                              static_cast<uint8_t*>(scales.data_ptr()), amax.data_ptr<float>(), ws.data_ptr<float>(), dev,
+                              stream_of(dev)), "ll_nvfp4_quantize"))
     return nullptr;
   return tuple3(values, scales, amax);
   END_HANDLE_TH_ERRORS
@@ -203,7 +204,8 @@ PyObject* py_linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const int rule = (int)PyLong_AsLong(args[1]);
   const double denom_a = PyFloat_AsDouble(args[2]), denom_b = PyFloat_AsDouble(args[6]);
   if (PyErr_Occurred()) return nullptr;
-  if (wv->size(1) * 2 != round_up(K, 64) || wv->size(0) != round_up(N, 128) || !wv->is_contiguous() || !ws->is_contiguous()) Py_RETURN_NONE;
+  if (wv->size(1) * 2 != round_up(K, 64) || wv->size(0) != round_up(N, 128) || !wv->is_contiguous() || !ws->is_contiguous())
+    Py_RETURN_NONE;
   if (bias && (!is_bf16(*bias, dev) || bias->numel() != N || !bias->is_contiguous())) Py_RETURN_NONE;
   void* stream = stream_of(dev);
   const TempOperand a = temp_operand(M, K, dev);
@@ -256,7 +258,9 @@ bool parse_layer(PyObject* t, int dev, Layer& l) {
   PyObject* b = PyTuple_GET_ITEM(t, 3);
   const Tensor* bias = as_tensor(b);
   if (!v || !s || !a || (!bias && b != Py_None)) return false;
-  if (!on_device(*v, dev) || !on_device(*s, dev) || !on_device(*a, dev) || v->dim() != 2 || !v->is_contiguous() || !s->is_contiguous()) return false;
+  if (!on_device(*v, dev) || !on_device(*s, dev) || !on_device(*a, dev) || v->dim() != 2 || !v->is_contiguous() ||
+      !s->is_contiguous())
+    return false;
   l.n = PyLong_AsLongLong(PyTuple_GET_ITEM(t, 5));
   l.np = v->size(0);
   l.kp = v->size(1) * 2;
@@ -281,7 +285,8 @@ bool parse_window(PyObject* o, int dev, Window& w) {
   if (!PyTuple_CheckExact(o) || PyTuple_GET_SIZE(o) != 6) return false;
   for (int i = 0; i < 2; ++i) {
     const Tensor* t = as_tensor(PyTuple_GET_ITEM(o, i));
-    if (!t || !on_device(*t, dev) || t->scalar_type() != at::kLong || t->dim() != 2 || t->size(0) != 3 || !t->is_contiguous()) return false;
+    if (!t || !on_device(*t, dev) || t->scalar_type() != at::kLong || t->dim() != 2 || t->size(0) != 3 || !t->is_contiguous())
+      return false;
     for (int j = 0; j < 3; ++j) w.p[3 * i + j] = reinterpret_cast<const uint64_t*>(t->data_ptr<int64_t>()) + j * t->size(1);
   }
   w.n_cached = PyLong_AsLongLong(PyTuple_GET_ITEM(o, 2));
@@ -295,7 +300,8 @@ bool parse_window(PyObject* o, int dev, Window& w) {
 bool parse_sink(PyObject* t, int dev, ll_amax_sink& s) {
   const Tensor* parts = PyTuple_CheckExact(t) && PyTuple_GET_SIZE(t) == 2 ? as_tensor(PyTuple_GET_ITEM(t, 0)) : nullptr;
   if (!parts || !on_device(*parts, dev)) return false;
-  s = ll_amax_sink{reinterpret_cast<uint64_t*>(parts->data_ptr<int64_t>()), (uint32_t)PyLong_AsUnsignedLong(PyTuple_GET_ITEM(t, 1)), nullptr};
+  s = ll_amax_sink{reinterpret_cast<uint64_t*>(parts->data_ptr<int64_t>()),
+                   (uint32_t)PyLong_AsUnsignedLong(PyTuple_GET_ITEM(t, 1)), nullptr};
   return !PyErr_Occurred();
 }
 
@@ -310,8 +316,8 @@ struct BlockCall {
   // out = epilogue(a @ layer^T)
   int gemm(const TempOperand& a, const Layer& w, int64_t M, void* out, ll_gemm_epilogue e) const {
     e.bias = w.bias;
-    return ll_nvfp4_gemm_tnt_fused(a.values, a.scales, w.values, w.scales, nullptr, a.amax, w.amax, denom_a, w.denom, M, w.n, a.mp, w.np,
-                                   a.kp, out, w.n, &e, stream);
+    return ll_nvfp4_gemm_tnt_fused(a.values, a.scales, w.values, w.scales, nullptr, a.amax, w.amax, denom_a, w.denom, M, w.n,
+                                   a.mp, w.np, a.kp, out, w.n, &e, stream);
   }
   int grouped(const TempOperand& a, const Layer* const* w, int n, int64_t M, void* const* outs, const ll_amax_sink* sinks) const {
     ll_gemm_product p[4];
@@ -329,9 +335,9 @@ struct BlockCall {
 // block_forward(x, e, layers, norms, cos, sin, kv, text, options, k_sink, v_sink, graph_sink) ->
 //   (x_out or None, roped K [1, L, H, 128], V [1, L, H, 128], text K, text V) or None
 //   e: the six modulation vectors per frame [1, F, 6, C];  layers: q, k, v, o, cross q, k, v, o, FFN up, down;  norms: weights of
-//   norm_q, norm_k, norm3, norm3's bias, cross norm_q, cross norm_k;  kv: the window (see Window);  text: the context [1, T, C] or (K, V) [1, T, H, 128];  options: (rule,
-//   denominator, heads, eps, eps of q/k norm, of norm3, of cross norm_q, of cross norm_k, spin limit, keys_only);  k_sink,
-//   v_sink: (parts, epoch) or None;  graph_sink: (parts, last epoch, offset) or None.
+//   norm_q, norm_k, norm3, norm3's bias, cross norm_q, cross norm_k;  kv: the window (see Window);  text: the context [1, T, C]
+//   or (K, V) [1, T, H, 128];  options: (rule, denominator, heads, eps, eps of q/k norm, of norm3, of cross norm_q, of cross
+//   norm_k, spin limit, keys_only);  k_sink, v_sink: (parts, epoch) or None;  graph_sink: (parts, last epoch, offset) or None.
 // The launches and their order are those of DiTBlock.forward (longlive_amd/dit/model.py), which documents them.
 PyObject* py_block_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
@@ -347,10 +353,12 @@ PyObject* py_block_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
   c.L = x.size(1);
   c.C = x.size(2);
   const int64_t L = c.L, C = c.C, F = e.size(1);
-  if (L == 0 || F == 0 || L % F || C % 128 || e.stride(1) % 8 || e.stride(2) % 8 || !aligned16(e.data_ptr()) || !aligned16(x.data_ptr())) Py_RETURN_NONE;
+  if (L == 0 || F == 0 || L % F || C % 128 || e.stride(1) % 8 || e.stride(2) % 8 || !aligned16(e.data_ptr()) ||
+      !aligned16(x.data_ptr()))
+    Py_RETURN_NONE;
   const int64_t frame_rows = L / F;
-  if (!PyTuple_CheckExact(args[2]) || PyTuple_GET_SIZE(args[2]) != 10 || !PyTuple_CheckExact(args[3]) || PyTuple_GET_SIZE(args[3]) != 6 ||
-      !PyTuple_CheckExact(args[8]) || PyTuple_GET_SIZE(args[8]) != 10)
+  if (!PyTuple_CheckExact(args[2]) || PyTuple_GET_SIZE(args[2]) != 10 || !PyTuple_CheckExact(args[3]) ||
+      PyTuple_GET_SIZE(args[3]) != 6 || !PyTuple_CheckExact(args[8]) || PyTuple_GET_SIZE(args[8]) != 10)
     Py_RETURN_NONE;
   Layer w[10];
   for (int i = 0; i < 10; ++i)
@@ -365,8 +373,9 @@ PyObject* py_block_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
     norm[i] = t->data_ptr();
   }
   const Tensor *cos = as_tensor(args[4]), *sin = as_tensor(args[5]);
-  if (!cos || !sin || !on_device(*cos, dev) || !on_device(*sin, dev) || cos->scalar_type() != at::kFloat || sin->scalar_type() != at::kFloat ||
-      !cos->is_contiguous() || !sin->is_contiguous() || cos->numel() != L * 64 || sin->numel() != L * 64)
+  if (!cos || !sin || !on_device(*cos, dev) || !on_device(*sin, dev) || cos->scalar_type() != at::kFloat ||
+      sin->scalar_type() != at::kFloat || !cos->is_contiguous() || !sin->is_contiguous() || cos->numel() != L * 64 ||
+      sin->numel() != L * 64)
     Py_RETURN_NONE;
   PyObject* const o = args[8];
   c.rule = (int)PyLong_AsLong(PyTuple_GET_ITEM(o, 0));
@@ -469,9 +478,9 @@ PyObject* py_block_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
     }
     attended = empty({L, C}, at::kBFloat16, dev);
     const ll_amax_sink sink = ep.take();
-    LL_TRY(ll_kv_attention_amax(roped_q.data_ptr(), L, H, kv.p[0], kv.p[1], kv.p[2], kv.p[3], kv.p[4], kv.p[5], kv.n_cached, kv.bts, kv.e2,
-                                kv.e4,                                smooth_k.data_ptr(), value.data_ptr(), L, 0.08838834764831845f, attended.data_ptr(), &sink, c.stream),
-           "self-attention");
+    LL_TRY(ll_kv_attention_amax(roped_q.data_ptr(), L, H, kv.p[0], kv.p[1], kv.p[2], kv.p[3], kv.p[4], kv.p[5], kv.n_cached,
+                                kv.bts, kv.e2, kv.e4, smooth_k.data_ptr(), value.data_ptr(), L, 0.08838834764831845f,
+                                attended.data_ptr(), &sink, c.stream), "self-attention");
     LL_TRY(c.quantize_from(attended, L, C, xq, sink), "quantization");
   }
   const Tensor x1 = empty({1, L, C}, at::kBFloat16, dev);
@@ -486,8 +495,8 @@ PyObject* py_block_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
   // ---- cross-attention
   {
     const ll_amax_sink sink = ep.take();
-    int code = ll_layer_norm_quantize(x1.data_ptr(), L, (int)C, norm[2], norm[3], eps[2], c.rule, xq.values, xq.scales, xq.amax, &sink, spin,
-                                      c.stream);
+    int code = ll_layer_norm_quantize(x1.data_ptr(), L, (int)C, norm[2], norm[3], eps[2], c.rule, xq.values, xq.scales,
+                                      xq.amax, &sink, spin, c.stream);
     if (code == LL_ENOSUP) {
       const ll_amax_sink again = ep.take();
       const Tensor y = empty({L, C}, at::kBFloat16, dev);
@@ -502,7 +511,8 @@ PyObject* py_block_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
     LL_TRY(ll_rms_norm(q.data_ptr(), L, (int)C, norm[4], eps[3], qn.data_ptr(), c.stream), "cross-attention norm_q");
     if (context) {
       const TempOperand tq = c.operand(T, C);
-      LL_TRY(ll_nvfp4_quantize(context->data_ptr(), T, C, C, c.rule, tq.values, tq.scales, tq.amax, 0, tq.workspace, c.stream), "text quantization");
+      LL_TRY(ll_nvfp4_quantize(context->data_ptr(), T, C, C, c.rule, tq.values, tq.scales, tq.amax, 0, tq.workspace, c.stream),
+             "text quantization");
       const Tensor k = empty({T, C}, at::kBFloat16, dev);
       text_k = empty({1, T, H, 128}, at::kBFloat16, dev);
       text_v = empty({1, T, H, 128}, at::kBFloat16, dev);
@@ -554,8 +564,9 @@ PyObject* py_block_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
 const Tensor* as_chunk(PyObject* o, int dev) {
   if (!plain(o)) return nullptr;
   const Tensor& t = THPVariable_Unpack(o);
-  return is_bf16(t, dev) && t.dim() == 4 && t.size(0) == 1 && t.size(3) == 128 && t.numel() > 0 && t.is_contiguous() && aligned16(t.data_ptr()) ? &t
-                                                                                                                                                : nullptr;
+  const bool ok = is_bf16(t, dev) && t.dim() == 4 && t.size(0) == 1 && t.size(3) == 128 && t.numel() > 0 && t.is_contiguous() &&
+                  aligned16(t.data_ptr());
+  return ok ? &t : nullptr;
 }
 
 // kv_attention(q, k, v, smoothed K or None, window, scale) -> [1, S, H, 128]
@@ -586,8 +597,8 @@ PyObject* py_kv_attention(PyObject*, PyObject* const* args, Py_ssize_t n) {
     if (failed(ll_kv_smooth(k->data_ptr(), k->size(1), H, smooth.data_ptr(), stream), "ll_kv_smooth")) return nullptr;
   }
   const Tensor out = empty(q->sizes(), at::kBFloat16, dev);
-  if (failed(ll_kv_attention(q->data_ptr(), q->size(1), H, w.p[0], w.p[1], w.p[2], w.p[3], w.p[4], w.p[5], w.n_cached, w.bts, w.e2, w.e4,
-                             smooth.data_ptr(), v->data_ptr(), k->size(1), scale, out.data_ptr(), stream),
+  if (failed(ll_kv_attention(q->data_ptr(), q->size(1), H, w.p[0], w.p[1], w.p[2], w.p[3], w.p[4], w.p[5], w.n_cached, w.bts,
+                             w.e2, w.e4, smooth.data_ptr(), v->data_ptr(), k->size(1), scale, out.data_ptr(), stream),
              "ll_kv_attention"))
     return nullptr;
   return THPVariable_Wrap(out);
@@ -623,10 +634,9 @@ PyObject* py_kv_attention_relative(PyObject*, PyObject* const* args, Py_ssize_t 
   void* stream = stream_of(dev);
   const Tensor wk = empty({keys, H, 128}, at::kBFloat16, dev), wv = empty({keys, H, 128}, at::kBFloat16, dev);
   const Tensor rq = empty(q->sizes(), at::kBFloat16, dev), out = empty(q->sizes(), at::kBFloat16, dev);
-  if (failed(ll_kv_window_rope(q->data_ptr(), S, H, w.p[0], w.p[1], w.p[2], w.p[3], w.p[4], w.p[5], w.n_cached, w.bts, w.e2, w.e4,
-                               k->data_ptr(), v->data_ptr(), S, tables[0], tables[1], tables[2], tables[3], rq.data_ptr(), wk.data_ptr(),
-                               wv.data_ptr(), stream),
-             "ll_kv_window_rope"))
+  if (failed(ll_kv_window_rope(q->data_ptr(), S, H, w.p[0], w.p[1], w.p[2], w.p[3], w.p[4], w.p[5], w.n_cached, w.bts, w.e2,
+                               w.e4, k->data_ptr(), v->data_ptr(), S, tables[0], tables[1], tables[2], tables[3],
+                               rq.data_ptr(), wk.data_ptr(), wv.data_ptr(), stream), "ll_kv_window_rope"))
     return nullptr;
   if (failed(ll_kv_attention(rq.data_ptr(), S, H, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0, 6.f, 256.f, wk.data_ptr(),
                              wv.data_ptr(), keys, scale, out.data_ptr(), stream),
@@ -654,10 +664,12 @@ PyObject* py_cache_write(PyObject*, PyObject* const* args, Py_ssize_t n) {
   for (int i = 0; i < 2; ++i) {
     PyObject* t = args[5 + i];
     if (!PyTuple_CheckExact(t) || PyTuple_GET_SIZE(t) != 3) Py_RETURN_NONE;
-    const Tensor *values = as_tensor(PyTuple_GET_ITEM(t, 0)), *scales = as_tensor(PyTuple_GET_ITEM(t, 1)), *a = as_tensor(PyTuple_GET_ITEM(t, 2));
+    const Tensor *values = as_tensor(PyTuple_GET_ITEM(t, 0)), *scales = as_tensor(PyTuple_GET_ITEM(t, 1)),
+        *a = as_tensor(PyTuple_GET_ITEM(t, 2));
     if (!values || !scales || !a || !on_device(*values, dev) || !on_device(*scales, dev) || !on_device(*a, dev) ||
-        values->scalar_type() != at::kByte || values->dim() != 2 || values->size(0) != Mp || values->size(1) != 64 || scales->numel() != Mp * 8 ||
-        scales->element_size() != 1 || a->numel() != 1 || a->scalar_type() != at::kFloat || !values->is_contiguous() || !scales->is_contiguous())
+        values->scalar_type() != at::kByte || values->dim() != 2 || values->size(0) != Mp || values->size(1) != 64 ||
+        scales->numel() != Mp * 8 || scales->element_size() != 1 || a->numel() != 1 || a->scalar_type() != at::kFloat ||
+        !values->is_contiguous() || !scales->is_contiguous())
       Py_RETURN_NONE;
     out[i][0] = values->data_ptr<uint8_t>();
     out[i][1] = static_cast<uint8_t*>(scales->data_ptr());
@@ -674,12 +686,12 @@ PyObject* py_cache_write(PyObject*, PyObject* const* args, Py_ssize_t n) {
       if (PyErr_Occurred()) return nullptr;
       Py_RETURN_NONE;
     }
-    code = ll_nvfp4_quantize_pair_from_sinks(kx, vx, M, 128, 128, rule, out[0][0], out[1][0], out[0][1], out[1][1], amax[0], amax[1], &sinks[0],
-                                             &sinks[1], stream);
+    code = ll_nvfp4_quantize_pair_from_sinks(kx, vx, M, 128, 128, rule, out[0][0], out[1][0], out[0][1], out[1][1], amax[0],
+                                             amax[1], &sinks[0], &sinks[1], stream);
   } else {
     const Tensor ws = empty({2 * (int64_t)LL_AMAX_PARTS}, at::kFloat, dev);
-    code = ll_nvfp4_quantize_pair(kx, vx, M, 128, 128, rule, out[0][0], out[1][0], out[0][1], out[1][1], amax[0], amax[1], ws.data_ptr<float>(),
-                                  stream);
+    code = ll_nvfp4_quantize_pair(kx, vx, M, 128, 128, rule, out[0][0], out[1][0], out[0][1], out[1][1], amax[0], amax[1],
+                                  ws.data_ptr<float>(), stream);
   }
   if (failed(code, "cache write")) return nullptr;
   Py_RETURN_TRUE;
@@ -689,8 +701,8 @@ PyObject* py_cache_write(PyObject*, PyObject* const* args, Py_ssize_t n) {
 // Calls that took torch's own operations before stay with them where Python code or torch itself has to see each one, or
 // where a gradient is wanted.
 inline bool traced() {
-  return c10::impl::TorchDispatchModeTLS::any_modes_set() || at::impl::torch_function_mode_enabled() || torch::jit::tracer::isTracing() ||
-         at::autocast::is_autocast_enabled(c10::kCUDA);
+  return c10::impl::TorchDispatchModeTLS::any_modes_set() || at::impl::torch_function_mode_enabled() ||
+         torch::jit::tracer::isTracing() || at::autocast::is_autocast_enabled(c10::kCUDA);
 }
 inline bool needs_torch(const Tensor& t) {
   // batched and functional wrappers have no storage
@@ -701,7 +713,9 @@ inline bool needs_torch(const Tensor& t) {
 inline const Tensor* as_weight(PyObject* o, int dev, int64_t rows, int64_t cols) {
   if (!plain(o)) return nullptr;
   const Tensor& t = THPVariable_Unpack(o);
-  if (needs_torch(t) || !is_bf16(t, dev) || !t.is_contiguous() || t.numel() != (rows < 0 ? cols : rows * cols) || !aligned16(t.data_ptr())) return nullptr;
+  if (needs_torch(t) || !is_bf16(t, dev) || !t.is_contiguous() || t.numel() != (rows < 0 ? cols : rows * cols) ||
+      !aligned16(t.data_ptr()))
+    return nullptr;
   return &t;
 }
 
@@ -729,8 +743,10 @@ PyObject* py_patch_embed(PyObject*, PyObject* const* args, Py_ssize_t n) {
   if (n != 7 || !plain(args[0]) || traced()) Py_RETURN_NONE;
   const Tensor& x = THPVariable_Unpack(args[0]);
   const int dev = current_device_of(x);
-  if (needs_torch(x) || !is_bf16(x, dev) || x.dim() != 4 || !x.is_contiguous() || x.numel() == 0 || x.numel() >= (1ll << 31)) Py_RETURN_NONE;
-  const int64_t N = PyLong_AsLongLong(args[3]), pt = PyLong_AsLongLong(args[4]), ph = PyLong_AsLongLong(args[5]), pw = PyLong_AsLongLong(args[6]);
+  if (needs_torch(x) || !is_bf16(x, dev) || x.dim() != 4 || !x.is_contiguous() || x.numel() == 0 || x.numel() >= (1ll << 31))
+    Py_RETURN_NONE;
+  const int64_t N = PyLong_AsLongLong(args[3]), pt = PyLong_AsLongLong(args[4]), ph = PyLong_AsLongLong(args[5]),
+      pw = PyLong_AsLongLong(args[6]);
   if (PyErr_Occurred()) return nullptr;
   if (pt < 1 || ph < 1 || pw < 1 || x.size(1) < pt || x.size(2) < ph || x.size(3) < pw || N < 1 || N > (1 << 20)) Py_RETURN_NONE;
   if (!embedding_takes((x.size(1) / pt) * (x.size(2) / ph) * (x.size(3) / pw), N)) Py_RETURN_NONE;
@@ -738,8 +754,9 @@ PyObject* py_patch_embed(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const Tensor* b = args[2] == Py_None ? nullptr : as_weight(args[2], dev, -1, N);
   if (!w || (!b && args[2] != Py_None)) Py_RETURN_NONE;
   const Tensor out = empty({1, (x.size(1) / pt) * (x.size(2) / ph) * (x.size(3) / pw), N}, at::kBFloat16, dev);
-  const int code = ll_patch_embed(x.data_ptr(), (int)x.size(0), (int)x.size(1), (int)x.size(2), (int)x.size(3), (int)pt, (int)ph, (int)pw,
-                                  w->data_ptr(), b ? b->data_ptr() : nullptr, (int)N, out.data_ptr(), stream_of(dev));
+  const int code = ll_patch_embed(x.data_ptr(), (int)x.size(0), (int)x.size(1), (int)x.size(2), (int)x.size(3), (int)pt,
+                                  (int)ph, (int)pw, w->data_ptr(), b ? b->data_ptr() : nullptr, (int)N, out.data_ptr(),
+                                  stream_of(dev));
   if (code == LL_ENOSUP) Py_RETURN_NONE;
   if (failed(code, "ll_patch_embed")) return nullptr;
   return THPVariable_Wrap(out);
@@ -753,8 +770,9 @@ PyObject* py_head(PyObject*, PyObject* const* args, Py_ssize_t n) {
   if (n != 8 || !plain(args[0]) || !plain(args[1]) || traced()) Py_RETURN_NONE;
   const Tensor &x = THPVariable_Unpack(args[0]), &e = THPVariable_Unpack(args[1]);
   const int dev = current_device_of(x);
-  if (needs_torch(x) || needs_torch(e) || !is_bf16(x, dev) || !is_bf16(e, dev) || x.dim() != 3 || x.size(0) != 1 || !x.is_contiguous() ||
-      e.dim() != 4 || e.size(0) != 1 || e.size(2) != 2 || e.size(3) != x.size(2) || !e.is_contiguous() || x.numel() == 0)
+  if (needs_torch(x) || needs_torch(e) || !is_bf16(x, dev) || !is_bf16(e, dev) || x.dim() != 3 || x.size(0) != 1 ||
+      !x.is_contiguous() || e.dim() != 4 || e.size(0) != 1 || e.size(2) != 2 || e.size(3) != x.size(2) || !e.is_contiguous() ||
+      x.numel() == 0)
     Py_RETURN_NONE;
   const int64_t L = x.size(1), C = x.size(2), F = e.size(1);
   int64_t grid[3], patch[3];
@@ -768,7 +786,9 @@ PyObject* py_head(PyObject*, PyObject* const* args, Py_ssize_t n) {
   if (PyErr_Occurred()) return nullptr;
   for (int j = 0; j < 3; ++j)
     if (grid[j] < 1 || patch[j] < 1) Py_RETURN_NONE;
-  if (F < 1 || L % F || !head_takes(L, C) || grid[0] * grid[1] * grid[2] != L || C % 16 || channels < 1 || !aligned16(x.data_ptr()) || !aligned16(e.data_ptr())) Py_RETURN_NONE;
+  if (F < 1 || L % F || !head_takes(L, C) || grid[0] * grid[1] * grid[2] != L || C % 16 || channels < 1 ||
+      !aligned16(x.data_ptr())
+    || !aligned16(e.data_ptr())) Py_RETURN_NONE;
   const int64_t N = channels * patch[0] * patch[1] * patch[2];
   if (N >= (1 << 20) || N * L >= (1ll << 31)) Py_RETURN_NONE;
   const Tensor* w = as_weight(args[2], dev, N, C);
@@ -777,14 +797,13 @@ PyObject* py_head(PyObject*, PyObject* const* args, Py_ssize_t n) {
   void* stream = stream_of(dev);
   const Tensor y = empty({L, C}, at::kBFloat16, dev);
   const uint16_t* shift = static_cast<const uint16_t*>(e.data_ptr());
-  if (failed(ll_adaln_modulate_amax(x.data_ptr(), 1, L, (int)C, shift + C, shift, e.stride(0), e.stride(1), e.stride(0), e.stride(1), L / F,
-                                    (float)eps, 1, y.data_ptr(), nullptr, stream),
-             "ll_adaln_modulate"))
+  if (failed(ll_adaln_modulate_amax(x.data_ptr(), 1, L, (int)C, shift + C, shift, e.stride(0), e.stride(1), e.stride(0),
+                                    e.stride(1), L / F, (float)eps, 1, y.data_ptr(), nullptr, stream), "ll_adaln_modulate"))
     return nullptr;
   const Tensor out = empty({channels, grid[0] * patch[0], grid[1] * patch[1], grid[2] * patch[2]}, at::kBFloat16, dev);
-  if (failed(ll_patch_head(y.data_ptr(), (int)C, w->data_ptr(), b ? b->data_ptr() : nullptr, (int)channels, (int)out.size(1), (int)out.size(2),
-                           (int)out.size(3), (int)patch[0], (int)patch[1], (int)patch[2], out.data_ptr(), stream),
-             "ll_patch_head"))
+  if (failed(ll_patch_head(y.data_ptr(), (int)C, w->data_ptr(), b ? b->data_ptr() : nullptr, (int)channels, (int)out.size(1),
+                           (int)out.size(2), (int)out.size(3), (int)patch[0], (int)patch[1], (int)patch[2], out.data_ptr(),
+                           stream), "ll_patch_head"))
     return nullptr;
   return THPVariable_Wrap(out);
   END_HANDLE_TH_ERRORS

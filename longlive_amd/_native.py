@@ -146,6 +146,8 @@ _host = None
 class _NoHostPath:
     """In place of the native host path where that does not load: takes no call, so that every one goes through ctypes."""
 
+    PATCH_TOKENS = 0
+
     def __getattr__(self, name):
         return lambda *args: None
 

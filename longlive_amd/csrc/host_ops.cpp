@@ -12,7 +12,9 @@
 // Nothing is kept between calls but one amax sink (8 KB) per device and stream, which release_stream_memory gives back.
 #include <Python.h>
 
+#include <ATen/core/LegacyTypeDispatch.h>
 #include <ATen/hip/EmptyTensor.h>
+#include <ATen/ops/linear.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <ATen/PythonTorchFunctionTLS.h>
@@ -719,22 +721,23 @@ inline const Tensor* as_weight(PyObject* o, int dev, int64_t rows, int64_t cols)
   return &t;
 }
 
-// Up to here the ends of the model run on the kernels of patch_linear.hip, beyond on torch's matrix products and permuted
-// copies.  The kernels save the host 25 us (embedding) and 50 us (head) a call; on the GPU alone they are level with torch at
-// small sizes and behind at large ones.
-//   GPU alone, us, here / torch:  embedding, tokens                          head without its normalization
-//       width                     368          720          1012             368          720          1012
-//       512                       8.9 / 8.6    9.1 / 8.8    9.1 / 8.7        9.1 / 9.2    9.2 / 9.6    9.2 / 9.9
-//       1536                      9.1 / 9.3    10.7 / 10.6  10.9 / 10.7      14.5 / 9.8   14.6 / 10.5  14.6 / 10.8
-//       2304                      9.2 / 9.3    11.0 / 10.5  14.8 / 12.3      19.5 / 10.2  19.7 / 11.7  19.7 / 12.0
-//       3072                      10.8 / 10.8  14.3 / 12.4  14.9 / 13.0      22.1 / 11.0  22.3 / 12.6  22.0 / 13.1
-// The embedding's line is where it falls behind on the GPU.  The head's is where the blocks, whose products grow with tokens x
-// width^2, keep the GPU so busy that the host's time is hidden: a forward of two layers, us, head here / by torch, with tokens x
-// width^2 in 10^9: 1024 x 896 (0.94) 529 / 552, 1536 x 384 (0.91) 496 / 539, 2304 x 192 (1.0) 555 / 562, 1536 x 768 (1.8) 632 / 635,
-// 3072 x 192 (1.8) 610 / 607, 2304 x 384 (2.0) 614 / 614, 3072 x 384 (3.6) 764 / 752, 2304 x 768 (4.1) 774 / 767.
+// The ends of the model: calls of up to kPatchTokens tokens are taken here, larger ones are left to the Python path.  us, kernels of
+// patch_linear.hip / torch's matrix product and permuted copy, on the GPU alone:
+//                   embedding, tokens                          head without its normalization
+//       width       368          720          1012             368          720          1012
+//       512         8.9 / 8.6    9.1 / 8.8    9.1 / 8.7        9.1 / 9.2    9.2 / 9.6    9.2 / 9.9
+//       1536        9.1 / 9.3    10.7 / 10.6  10.9 / 10.7      14.5 / 9.8   14.6 / 10.5  14.6 / 10.8
+//       2304        9.2 / 9.3    11.0 / 10.5  14.8 / 12.3      19.5 / 10.2  19.7 / 11.7  19.7 / 12.0
+//       3072        10.8 / 10.8  14.3 / 12.4  14.9 / 13.0      22.1 / 11.0  22.3 / 12.6  22.0 / 13.1
+// and on the host: embedding 7 / 30 (35 in Python), head 21 / 43 (75).  The embedding comes first in a forward: where the GPU has
+// waited for the host (at every chunk, whose time steps are read back) its host time is all waited for, so the kernel takes every
+// call.  The head comes last: its host time matters only while the blocks, whose products grow with tokens x width^2, keep the
+// GPU less busy than the host.  A forward of two layers, us, head by the kernel / in Python, with tokens x width^2 in 10^9: 1024 x
+// 896 (0.94) 529 / 552, 1536 x 384 (0.91) 496 / 539, 2304 x 192 (1.0) 555 / 562, 1536 x 768 (1.8) 632 / 635, 3072 x 192 (1.8)
+// 610 / 607, 2304 x 384 (2.0) 614 / 614, 3072 x 384 (3.6) 764 / 752, 2304 x 768 (4.1) 774 / 767.  Beyond the line the head runs
+// on torch's operations, the same bits as in Python, without Python between them.
 constexpr int64_t kPatchTokens = 1024;
-inline bool embedding_takes(int64_t tokens, int64_t width) { return tokens <= kPatchTokens && tokens * width <= kPatchTokens * 1536; }
-inline bool head_takes(int64_t tokens, int64_t width) { return tokens <= kPatchTokens && tokens * width * width <= 3ll << 29; }
+inline bool head_kernel_takes(int64_t tokens, int64_t width) { return tokens * width * width <= 3ll << 29; }
 
 // patch_embed(x [C, F, H, W], weight, bias or None, outputs, pt, ph, pw) -> tokens [1, f h w, outputs], or None when it does not
 // take the call.
@@ -749,11 +752,12 @@ PyObject* py_patch_embed(PyObject*, PyObject* const* args, Py_ssize_t n) {
       pw = PyLong_AsLongLong(args[6]);
   if (PyErr_Occurred()) return nullptr;
   if (pt < 1 || ph < 1 || pw < 1 || x.size(1) < pt || x.size(2) < ph || x.size(3) < pw || N < 1 || N > (1 << 20)) Py_RETURN_NONE;
-  if (!embedding_takes((x.size(1) / pt) * (x.size(2) / ph) * (x.size(3) / pw), N)) Py_RETURN_NONE;
+  const int64_t f = x.size(1) / pt, h = x.size(2) / ph, wd = x.size(3) / pw;
+  if (f * h * wd > kPatchTokens) Py_RETURN_NONE;
   const Tensor* w = as_weight(args[1], dev, N, x.size(0) * pt * ph * pw);
   const Tensor* b = args[2] == Py_None ? nullptr : as_weight(args[2], dev, -1, N);
   if (!w || (!b && args[2] != Py_None)) Py_RETURN_NONE;
-  const Tensor out = empty({1, (x.size(1) / pt) * (x.size(2) / ph) * (x.size(3) / pw), N}, at::kBFloat16, dev);
+  const Tensor out = empty({1, f * h * wd, N}, at::kBFloat16, dev);
   const int code = ll_patch_embed(x.data_ptr(), (int)x.size(0), (int)x.size(1), (int)x.size(2), (int)x.size(3), (int)pt,
                                   (int)ph, (int)pw, w->data_ptr(), b ? b->data_ptr() : nullptr, (int)N, out.data_ptr(),
                                   stream_of(dev));
@@ -786,9 +790,9 @@ PyObject* py_head(PyObject*, PyObject* const* args, Py_ssize_t n) {
   if (PyErr_Occurred()) return nullptr;
   for (int j = 0; j < 3; ++j)
     if (grid[j] < 1 || patch[j] < 1) Py_RETURN_NONE;
-  if (F < 1 || L % F || !head_takes(L, C) || grid[0] * grid[1] * grid[2] != L || C % 16 || channels < 1 ||
-      !aligned16(x.data_ptr())
-    || !aligned16(e.data_ptr())) Py_RETURN_NONE;
+  if (F < 1 || L % F || L > kPatchTokens || grid[0] * grid[1] * grid[2] != L || C % 16 || channels < 1 ||
+      !aligned16(x.data_ptr()) || !aligned16(e.data_ptr()))
+    Py_RETURN_NONE;
   const int64_t N = channels * patch[0] * patch[1] * patch[2];
   if (N >= (1 << 20) || N * L >= (1ll << 31)) Py_RETURN_NONE;
   const Tensor* w = as_weight(args[2], dev, N, C);
@@ -800,23 +804,19 @@ PyObject* py_head(PyObject*, PyObject* const* args, Py_ssize_t n) {
   if (failed(ll_adaln_modulate_amax(x.data_ptr(), 1, L, (int)C, shift + C, shift, e.stride(0), e.stride(1), e.stride(0),
                                     e.stride(1), L / F, (float)eps, 1, y.data_ptr(), nullptr, stream), "ll_adaln_modulate"))
     return nullptr;
-  const Tensor out = empty({channels, grid[0] * patch[0], grid[1] * patch[1], grid[2] * patch[2]}, at::kBFloat16, dev);
+  const int64_t extent[4] = {channels, grid[0] * patch[0], grid[1] * patch[1], grid[2] * patch[2]};
+  if (!head_kernel_takes(L, C)) {
+    at::AutoDispatchBelowADInplaceOrView no_autograd;
+    const Tensor rows = at::linear(y, *w, b ? std::optional<Tensor>(*b) : std::nullopt);
+    return THPVariable_Wrap(rows.view({grid[0], grid[1], grid[2], patch[0], patch[1], patch[2], channels})
+                                .permute({6, 0, 3, 1, 4, 2, 5}).reshape(extent));
+  }
+  const Tensor out = empty(extent, at::kBFloat16, dev);
   if (failed(ll_patch_head(y.data_ptr(), (int)C, w->data_ptr(), b ? b->data_ptr() : nullptr, (int)channels, (int)out.size(1),
                            (int)out.size(2), (int)out.size(3), (int)patch[0], (int)patch[1], (int)patch[2], out.data_ptr(),
                            stream), "ll_patch_head"))
     return nullptr;
   return THPVariable_Wrap(out);
-  END_HANDLE_TH_ERRORS
-}
-
-// head_takes(tokens, width) -> whether head() takes a call of these sizes, for a caller with work to do ahead of it
-PyObject* py_head_takes(PyObject*, PyObject* const* args, Py_ssize_t n) {
-  HANDLE_TH_ERRORS
-  if (n != 2) Py_RETURN_NONE;
-  const int64_t tokens = PyLong_AsLongLong(args[0]), width = PyLong_AsLongLong(args[1]);
-  if (PyErr_Occurred()) return nullptr;
-  if (head_takes(tokens, width)) Py_RETURN_TRUE;
-  Py_RETURN_FALSE;
   END_HANDLE_TH_ERRORS
 }
 
@@ -893,7 +893,6 @@ PyMethodDef methods[] = {
     {"cache_write", (PyCFunction)(void (*)(void))py_cache_write, METH_FASTCALL, nullptr},
     {"patch_embed", (PyCFunction)(void (*)(void))py_patch_embed, METH_FASTCALL, nullptr},
     {"head", (PyCFunction)(void (*)(void))py_head, METH_FASTCALL, nullptr},
-    {"head_takes", (PyCFunction)(void (*)(void))py_head_takes, METH_FASTCALL, nullptr},
     {"unipc_step", (PyCFunction)(void (*)(void))py_unipc_step, METH_FASTCALL, nullptr},
     {"recording", py_recording, METH_O, nullptr},
     {"current_stream", py_current_stream, METH_NOARGS, nullptr},
@@ -910,6 +909,7 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host_ops", nullptr, -1, methods, 
 PyMODINIT_FUNC PyInit__host_ops(void) {
   PyObject* m = PyModule_Create(&module);
   if (m) PyModule_AddIntConstant(m, "EPOCHS_PER_CALL", kEpochsPerCall);
+  if (m) PyModule_AddIntConstant(m, "PATCH_TOKENS", kPatchTokens);
   if (m) PyModule_AddStringConstant(m, "TORCH_VERSION", LL_TORCH_VERSION);
   return m;
 }

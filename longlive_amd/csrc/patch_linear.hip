@@ -21,7 +21,7 @@ __device__ __forceinline__ bf16x8 load_bf16x8(const uint16_t* p) { return __buil
 // out[m][n] = sum_k patch(m)[k] weight[n][k] + bias[n], k = ((c pt + dt) ph + dh) pw + dw (the order of the convolution
 // weight).  A workgroup takes 32 tokens x 128 outputs, a wave 32 x 32: the tokens' patches are gathered into LDS once
 // (32 x K, neighbouring threads take neighbouring tokens of a row), the weight (1.2 MB at full width) comes from L2 straight
-// into registers, and the result leaves through LDS in whole rows.  Meant for small calls (embedding_takes in host_ops.cpp), where it is bound
+// into registers, and the result leaves through LDS in whole rows.  Meant for up to about a thousand tokens, where it is bound
 // by its launch and one pass of latencies (192 x 256 9.3 us, 736 x 1536 11.5 us; with a copy of the patches ahead of a library
 // product 11.5 and 13.1); every workgroup gathers its patches anew, which costs more than that copy at 2640 x 3072 (28.5 / 20 us).
 constexpr int kEmbedTokens = 32, kEmbedOutputs = 128, kEmbedMaxK = 896;  // 32 x (896 + 8) x 2 bytes of LDS

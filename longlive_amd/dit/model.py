@@ -431,7 +431,7 @@ class CausalHead(nn.Module):
                 or not _OWN_HEAD.of(self) or _has_hooks(self, norm, head):
             return None
         host = _native.host()
-        if not host.head_takes(x.shape[1], x.shape[2]):
+        if x.shape[1] > host.PATCH_TOKENS:   # ahead of the sum below, which forward forms too
             return None
         return host.head(x, self.modulation.unsqueeze(1) + e, head.weight, head.bias, norm.eps, channels, tuple(grid),
                          tuple(patch_size))

@@ -1156,18 +1156,42 @@ def test_without_the_native_host_path_the_same_bits(gpu, monkeypatch):
         assert all(torch.equal(a, b) for a, b in zip(run(), want))
 
 
-@pytest.mark.parametrize("dim,grid,head,embedding", [
-    (256, (3, 4, 16), True, True), (1024, (1, 28, 32), True, True), (2304, (1, 12, 16), True, True),
-    (3072, (1, 12, 16), False, True), (2304, (1, 24, 16), False, True), (1536, (1, 24, 32), False, True),
-    (3072, (1, 28, 32), False, False), (256, (3, 22, 40), False, False),
+@pytest.mark.parametrize("dim,grid,head", [
+    (256, (3, 4, 16), True), (1024, (1, 28, 32), True), (2304, (1, 12, 16), True), (3072, (1, 12, 16), False), (2304, (1, 24, 16), False),
+    (1536, (1, 24, 32), False), (3072, (1, 28, 32), False),
 ])
-def test_which_calls_the_ends_of_the_model_run_themselves(gpu, dim, grid, head, embedding):
-    """The lines of host_ops.cpp between the package's kernels and torch's products, on both sides of them."""
+def test_which_calls_the_ends_of_the_model_run_on_their_kernels(gpu, monkeypatch, dim, grid, head):
+    """Both sides of the head's line of host_ops.cpp: beyond it the native call has the bits of torch's operations, before it
+    those of the kernel, with and without bias; the embedding, here with a row that no patch covers, always the kernel's."""
     from longlive_amd import _native
 
     f, h, w = grid
-    x, weight = torch.randn(48, f, 2 * h, 2 * w, device=gpu).bfloat16(), torch.randn(dim, 192, device=gpu).bfloat16()
-    y, e = torch.randn(1, f * h * w, dim, device=gpu).bfloat16(), torch.randn(1, f, 2, dim, device=gpu).bfloat16()
-    lib = _native.host()
-    assert (lib.patch_embed(x, weight, None, dim, 1, 2, 2) is not None) == embedding
-    assert (lib.head(y, e, weight.t().contiguous(), None, 1e-6, 48, grid, (1, 2, 2)) is not None) == head == lib.head_takes(f * h * w, dim)
+    cfg = DiTConfig(dim=dim, ffn_dim=dim, num_heads=dim // 128, num_layers=0, text_dim=64, text_len=4)
+    torch.manual_seed(11)
+    with torch.device(gpu):
+        model = CausalDiT(cfg).bfloat16()
+        x = torch.randn(48, f, 2 * h + 1, 2 * w).bfloat16()
+        y, e = torch.randn(1, f * h * w, dim).bfloat16(), torch.randn(1, f, 1, dim).bfloat16()
+    lib = _native.load()
+    with torch.no_grad():
+        for bias in (True, False):
+            if not bias:
+                model.patch_embedding.bias = model.head.head.bias = None
+            else:
+                model.patch_embedding.bias.normal_(), model.head.head.bias.normal_()
+            tokens, latents = model.patch_embed(x)[0], model.head.latents(y, e, grid, (1, 2, 2), 48)
+            with monkeypatch.context() as m:
+                m.setattr(_native, "_host", _native._NoHostPath())
+                plain = model.unpatchify(model.head(y, e)[0].flatten(0, 1), grid)
+            conv, linear, stream = model.patch_embedding, model.head.head, torch.cuda.current_stream().cuda_stream
+            kernel_tokens, kernel = torch.empty_like(tokens), torch.empty_like(latents)
+            assert lib.ll_patch_embed(x.data_ptr(), 48, f, 2 * h + 1, 2 * w, 1, 2, 2, conv.weight.data_ptr(), _native._ptr(conv.bias), dim,
+                                      kernel_tokens.data_ptr(), stream) == 0
+            rows = _native.adaln_modulate(y, *[(model.head.modulation.unsqueeze(1) + e)[:, :, i:i + 1] for i in (1, 0)], h * w)
+            assert lib.ll_patch_head(rows.data_ptr(), dim, linear.weight.data_ptr(), _native._ptr(linear.bias), 48, f, 2 * h, 2 * w, 1, 2, 2,
+                                     kernel.data_ptr(), stream) == 0
+            assert torch.equal(tokens, kernel_tokens)
+            assert torch.equal(latents, kernel if head else plain)
+        too_many = torch.randn(1, 1025, 128, device=gpu).bfloat16()
+        small = CausalDiT(DiTConfig(dim=128, ffn_dim=128, num_heads=1, num_layers=0)).to(gpu).bfloat16()
+        assert small.head.latents(too_many, torch.randn(1, 1, 1, 128, device=gpu).bfloat16(), (1, 1, 1025), (1, 2, 2), 48) is None

@@ -571,6 +571,41 @@ const Tensor* as_chunk(PyObject* o, int dev) {
   return ok ? &t : nullptr;
 }
 
+// slot_addresses(K slots, V slots, ids) -> the addresses of the values, scale_factors and amax buffers of those slots of either
+// list, packed: what a pointer table of the window is found by (24 buffers for four slots, 3 us in Python).
+PyObject* py_slot_addresses(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  static PyObject* const names[3] = {PyUnicode_InternFromString("values"), PyUnicode_InternFromString("scale_factors"),
+                                     PyUnicode_InternFromString("amax")};
+  if (n != 3 || !PyList_CheckExact(args[0]) || !PyList_CheckExact(args[1]) || !PyTuple_CheckExact(args[2])) Py_RETURN_NONE;
+  const Py_ssize_t ids = PyTuple_GET_SIZE(args[2]);
+  PyObject* key = PyBytes_FromStringAndSize(nullptr, ids * 2 * 3 * (Py_ssize_t)sizeof(void*));
+  if (!key) return nullptr;
+  void** out = reinterpret_cast<void**>(PyBytes_AS_STRING(key));
+  for (int side = 0; side < 2; ++side)
+    for (Py_ssize_t i = 0; i < ids; ++i) {
+      const Py_ssize_t at = PyLong_AsSsize_t(PyTuple_GET_ITEM(args[2], i));
+      if (at < 0 || at >= PyList_GET_SIZE(args[side])) {
+        Py_DECREF(key);
+        if (PyErr_Occurred()) return nullptr;
+        Py_RETURN_NONE;
+      }
+      for (PyObject* name : names) {
+        PyObject* t = PyObject_GetAttr(PyList_GET_ITEM(args[side], at), name);
+        const bool tensor = t && THPVariable_Check(t) && THPVariable_Unpack(t).has_storage();
+        if (tensor) *out++ = THPVariable_Unpack(t).data_ptr();
+        Py_XDECREF(t);
+        if (!tensor) {
+          Py_DECREF(key);
+          if (PyErr_Occurred()) return nullptr;
+          Py_RETURN_NONE;
+        }
+      }
+    }
+  return key;
+  END_HANDLE_TH_ERRORS
+}
+
 // kv_attention(q, k, v, smoothed K or None, window, scale) -> [1, S, H, 128]
 PyObject* py_kv_attention(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
@@ -888,6 +923,7 @@ PyObject* py_release_stream_sink(PyObject*, PyObject*) {
 
 PyMethodDef methods[] = {
     {"block_forward", (PyCFunction)(void (*)(void))py_block_forward, METH_FASTCALL, nullptr},
+    {"slot_addresses", (PyCFunction)(void (*)(void))py_slot_addresses, METH_FASTCALL, nullptr},
     {"kv_attention", (PyCFunction)(void (*)(void))py_kv_attention, METH_FASTCALL, nullptr},
     {"kv_attention_relative", (PyCFunction)(void (*)(void))py_kv_attention_relative, METH_FASTCALL, nullptr},
     {"cache_write", (PyCFunction)(void (*)(void))py_cache_write, METH_FASTCALL, nullptr},

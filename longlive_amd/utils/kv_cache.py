@@ -13,7 +13,7 @@ from __future__ import annotations
 import torch
 
 from .. import _native
-from ..fouroversix import QuantizationConfig, QuantizedTensor, quantize_to_fp4
+from ..fouroversix import QuantizationConfig, QuantizedTensor, ScaleRule, quantize_to_fp4
 from .quant import SlotPointerTable, clone_quantized_tensor, copy_quantized_into, dequantize_kv_cache, k_smooth
 
 
@@ -58,18 +58,18 @@ def initialize_kv_cache(num_layers: int, block_token_size: int, max_blocks: int,
 
 
 _MAX_TABLES = 16
+# largest e2m1 and e4m3 magnitude of a scale rule
+_RULE_LIMITS = {rule.value: (rule.max_allowed_e2m1_value(), rule.max_allowed_e4m3_value()) for rule in ScaleRule}
 
 
 def _tables_for(cache: dict, slot_ids: tuple[int, ...]):
     # keyed by the buffers, not by the positions: a roll moves the buffers through the positions (apply_cache_update),
     # and the handful of arrangements that a streaming run cycles through are each built once.  By all of them: a table
     # holds nothing but their addresses, so that one found here is right whatever has been put into the cache meanwhile.
-    key = []
-    for slots in (cache["k"], cache["v"]):
-        for i in slot_ids:
-            s = slots[i]
-            key += s.values.data_ptr(), s.scale_factors.data_ptr(), s.amax.data_ptr()
-    key = tuple(key)
+    key = _native.host().slot_addresses(cache["k"], cache["v"], slot_ids)
+    if key is None:
+        slots = [cache[name][i] for name in ("k", "v") for i in slot_ids]
+        key = tuple(t.data_ptr() for s in slots for t in (s.values, s.scale_factors, s.amax))
     tables = cache["_tables"]
     entry = tables.pop(key, None)
     if entry is None:
@@ -87,8 +87,8 @@ def _window(cache: dict, slot_ids):
     if not slot_ids:
         return None
     kt, vt = _tables_for(cache, slot_ids)
-    rule, blk = cache["k"][0].scale_rule, cache["block_token_size"]
-    return kt.table, vt.table, len(slot_ids) * blk, blk, rule.max_allowed_e2m1_value(), rule.max_allowed_e4m3_value()
+    blk = cache["block_token_size"]
+    return kt.table, vt.table, len(slot_ids) * blk, blk, *_RULE_LIMITS[cache["k"][0].scale_rule._value_]
 
 
 def plan_cache_step(cache: dict, current_start: int, num_new_tokens: int, sink_tokens: int,

@@ -549,9 +549,13 @@ def test_host_path_is_built_for_this_torch_and_optional(monkeypatch):
     assert _native.block_forward(torch.zeros(1), *[None] * 7, "mse", (), False, ()) is None
 
 
-def test_pointer_tables_follow_every_buffer_of_a_slot():
+@pytest.mark.parametrize("native", [True, False])
+def test_pointer_tables_follow_every_buffer_of_a_slot(monkeypatch, native):
     """The tables of the attended slots are kept between calls; a values, scale or amax buffer of K or V that has been
     replaced gets a table of its own."""
+    if not native:
+        monkeypatch.setattr(_native, "_host", _native._NoHostPath())
+
     def slot():
         return QuantizedTensor(torch.zeros(128, 64, dtype=torch.uint8), torch.zeros(1024, dtype=torch.uint8).view(torch.float8_e4m3fn),
                                torch.zeros(1), "nvfp4", (128, 128), "mse", (128, 128))

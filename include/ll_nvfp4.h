@@ -349,7 +349,10 @@ int ll_kv_attention_amax(const void* q, int64_t Lq, int num_heads,
  *   LL_ATTENTION_WIDE    one workgroup per (head, 256 queries): every decoded K/V tile serves twice as many MFMAs;
  *   LL_ATTENTION_SPLIT   256-query tiles; what does not fill whole rounds of one tile per compute unit is cut
  *                        along the key range into shares of equal cost (a head's last, partly filled group of
- *                        queries counts for less), so that no compute unit waits for another.  Tiles shared by two
+ *                        queries counts for less), so that no compute unit waits for another.  Launches with at most
+ *                        half a 128-query tile per compute unit take those instead where that is cheapest, the key range
+ *                        of each in equal parts (while a stream is being captured only if this division is asked for:
+ *                        the automatic choice then takes one of the others).  Tiles shared by two
  *                        workgroups pass through device memory that the library allocates on the first such
  *                        launch on a (device, stream) pair and keeps (69 MB on a 256-CU device); launches that
  *                        use it must not overlap on one stream's memory, which same-stream order guarantees.

@@ -6,7 +6,8 @@
 //
 // A workgroup is 8 waves = two per SIMD, in one of two shapes (template parameter WIDE):
 //   * one head x 128 queries: wave w owns 32 queries (w & 3) and every second 64-key tile (w >> 2); the two
-//     halves of the key range are merged at the end;
+//     halves of the key range are merged at the end.  Where tiles are few, several workgroups share the key range of each
+//     (plan_narrow_split, attention_split.h);
 //   * one head x 256 queries: wave w owns 32 queries and walks both 64-key tiles of an iteration, so a decoded
 //     tile serves twice as many MFMAs.  A launch of this shape may hand a workgroup whole tiles, parts of the
 //     key range of tiles (combined through device memory), or both: attention_split.h.  Where a head's last
@@ -25,6 +26,7 @@
 #include "ll_common.h"
 #include "attention_split.h"
 
+#include <algorithm>
 #include <map>
 #include <mutex>
 #include <utility>
@@ -46,7 +48,9 @@ constexpr int kVTileBytes = kTileKeys * kVPitch;
 constexpr int kStageBytes = 2 * kKTileBytes + 2 * kVTileBytes;
 constexpr int kMaxSlots = 64;
 constexpr int kAttnThreads = 512;
-constexpr int kPartialFloats = 8 * 66 * 64;    // a workgroup's partial result: per wave 64 O^T registers, reference point and row sum, per lane
+// A workgroup's partial result: per wave 64 (256-query tiles) or 32 (128) O^T registers, reference point and row sum, per lane.
+inline size_t partial_records(const AttentionPlan& plan) { return (plan.queries == 128 ? 1 : 2) * (size_t)plan.d.G; }
+constexpr size_t partial_bytes(int queries) { return (size_t)8 * (queries / 4 + 2) * 64 * sizeof(float); }
 
 struct AttnParams {
   const uint16_t* q;
@@ -64,9 +68,10 @@ struct AttnParams {
   int full_qtiles;  // tile t < H * full_qtiles is (head t / full_qtiles, group t % full_qtiles); the tiles behind are
                     // the heads' last groups, (head t - H * full_qtiles, group full_qtiles)
   // Division of the launch between its d.G workgroups (attention_split.h).  One workgroup per tile is
-  // whole_rounds = 1, extra = 0, units = 0; `partials` / `arrivals` serve the split part (256-query kernel only).
+  // whole_rounds = 1, extra = 0, units = 0; `partials` / `arrivals` serve the split part.
   Division d;
-  float* partials;  // [2 G] records of kPartialFloats floats
+  uint32_t parts;   // 128-query tiles: workgroups that share a tile's key range; p.d.G = tiles * parts
+  float* partials;  // [2 G] (256-query tiles) or [G] records of partial_bytes
   int* arrivals;    // [tiles] counters, zero between launches
 };
 
@@ -144,6 +149,7 @@ __device__ __forceinline__ T load_global(const void* ptr) {
   return *(const __attribute__((address_space(1))) T*)ptr;
 }
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ uint4 load_global_b128(const void* ptr) {
   const u32x4 v = load_global<u32x4>(ptr);
   return make_uint4(v[0], v[1], v[2], v[3]);
@@ -226,6 +232,21 @@ __device__ __forceinline__ void store_shared_f32(float* ptr, float v) {
 __device__ __forceinline__ float load_shared_f32(const float* ptr) {
   return __uint_as_float(__hip_atomic_load(reinterpret_cast<const uint32_t*>(ptr), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
 }
+// The same, sixteen or eight bytes per lane (buffer accesses with the sc1 bit: device scope).
+typedef float float4v __attribute__((ext_vector_type(4)));
+constexpr int kDeviceScope = 1 << 4;
+__device__ __forceinline__ void store_shared_b128(__amdgpu_buffer_rsrc_t mem, uint32_t offset, uint32_t base, float4v x) {
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, x), mem, offset, base, kDeviceScope);
+}
+__device__ __forceinline__ void store_shared_b64(__amdgpu_buffer_rsrc_t mem, uint32_t offset, uint32_t base, float2v x) {
+  __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, x), mem, offset, base, kDeviceScope);
+}
+__device__ __forceinline__ float4v load_shared_b128(__amdgpu_buffer_rsrc_t mem, uint32_t offset, uint32_t base) {
+  return __builtin_bit_cast(float4v, __builtin_amdgcn_raw_buffer_load_b128(mem, offset, base, kDeviceScope));
+}
+__device__ __forceinline__ float2v load_shared_b64(__amdgpu_buffer_rsrc_t mem, uint32_t offset, uint32_t base) {
+  return __builtin_bit_cast(float2v, __builtin_amdgcn_raw_buffer_load_b64(mem, offset, base, kDeviceScope));
+}
 // This workgroup's number in the order in which the work is handed out: consecutive hardware workgroup numbers go
 // to different XCDs; every XCD gets a contiguous range of the work instead, so that workgroups that share an L2
 // read the same heads.
@@ -243,8 +264,10 @@ __global__ __launch_bounds__(kAttnThreads) void kv_attention_kernel(AttnParams p
   SlotTable& tab = *reinterpret_cast<SlotTable*>(smem + 2 * kStageBytes);
 
   const int n_iter = (int)((p.n_cached + p.n_new + kIterKeys - 1) / kIterKeys);
-  WorkCursor at;  // where this workgroup is in its work (attention_split.h)
-  {
+  // 256-query tiles: where this workgroup is in its work (attention_split.h).  With 128 queries it has one segment: its part
+  // of the key range of one tile.
+  WorkCursor at{};
+  if constexpr (WIDE) {
     const auto& c = reread_params();
     at = start_of_work(group_number(c.d.G), division_of(c));
   }
@@ -271,13 +294,18 @@ __global__ __launch_bounds__(kAttnThreads) void kv_attention_kernel(AttnParams p
   for (;;) {
   int tile_id, seg_begin, seg_end;
   bf16x8 qf[8];
-  {
+  if constexpr (WIDE) {
     const auto& c = reread_params();
     Segment seg;
     if (!next_segment(at, group_number(c.d.G), division_of(c), seg)) break;
     tile_id = (int)seg.tile;
     seg_begin = seg.begin;
     seg_end = seg.end;
+  } else {
+    const uint32_t g = group_number(p.d.G), part = g % p.parts;
+    tile_id = (int)(g / p.parts);
+    seg_begin = first_iteration_of_part(part, p.parts, n_iter);
+    seg_end = first_iteration_of_part(part + 1, p.parts, n_iter);
   }
   int head, qtile;
   if (const int n_full = p.H * p.full_qtiles; tile_id < n_full) {
@@ -378,7 +406,10 @@ __global__ __launch_bounds__(kAttnThreads) void kv_attention_kernel(AttnParams p
   // reach 2^kRescaleStep instead of 1 (harmless in fp32 / bf16) and the 64 accumulator registers per lane
   // are rescaled a handful of times per kernel instead of at almost every tile.  The final division by
   // the row sum, which is accumulated against the same reference, makes the result independent of it.
-  constexpr float kRescaleStep = 8.0f;
+  // Where workgroups share the key range of a 128-query tile the step is 2^2, as for the short launches: the result is then no
+  // further from fp64 than that of the 256-query tiles' shares, which it replaced (736 queries x 12 heads over 2208 keys 0.002287
+  // relative, 2-norm, against 0.002302; with 2^8 0.002318).
+  const float kRescaleStep = !WIDE && p.parts > 1 ? 2.0f : 8.0f;
 
   // Second half of an iteration: reference point of the exponentials over the wave's 64 keys (S^T in sc:
   // register r of tile kt <-> key 32 kt + 8 (r / 4) + 4 lh + r % 4), then the PV phase in four steps of 16
@@ -685,7 +716,7 @@ __global__ __launch_bounds__(kAttnThreads) void kv_attention_kernel(AttnParams p
       const uint32_t wg = group_number(c.d.G);
       const uint32_t split_tile = (uint32_t)tile_id - c.d.whole_rounds * c.d.G - c.d.extra;  // the tile's number among the split ones
       auto record_of = [&](uint32_t g) {
-        return c.partials + (size_t)record_of_part(g, split_tile, division_of(c)) * kPartialFloats + wave * (66 * 64) + lane;
+        return c.partials + (size_t)record_of_part(g, split_tile, division_of(c)) * (partial_bytes(kQueries) / sizeof(float)) + wave * (66 * 64) + lane;
       };
       uint32_t g_first, g_last;
       parts_of_tile(split_tile, division_of(c), g_first, g_last);
@@ -763,53 +794,133 @@ __global__ __launch_bounds__(kAttnThreads) void kv_attention_kernel(AttnParams p
       }
     }
   } else {
-    // ---- merge the two key-parity halves through LDS and write out.
-    float* xo = reinterpret_cast<float*>(smem);   // [qq][64 regs][64 lanes]
-    float* xm = xo + 4 * 64 * 64;                  // [qq][64]
-    float* xl = xm + 4 * 64;
-    if (kp == 1 && !wave_idle) {
+    // ---- The two waves of a group of queries leave each other two of their four 32-column groups in LDS; wave kp keeps
+    // groups 2 kp and 2 kp + 1.
+    float4* xo = reinterpret_cast<float4*>(smem);                     // [wave][8][64 lanes]
+    float2* xml = reinterpret_cast<float2*>(smem + 8 * 8 * 64 * 16);  // [wave][64]
 #pragma unroll
-      for (int dt = 0; dt < 4; ++dt)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) xo[(qq * 64 + dt * 16 + i) * 64 + lane] = o[dt][i];
-      xm[qq * 64 + lane] = m_run;
-      xl[qq * 64 + lane] = l_run;
+    for (int i = 0; i < 8; ++i) {
+      const float16v give = kp == 0 ? o[2 + (i >> 2)] : o[i >> 2];
+      xo[(wave * 8 + i) * 64 + lane] = make_float4(give[4 * (i & 3)], give[4 * (i & 3) + 1], give[4 * (i & 3) + 2], give[4 * (i & 3) + 3]);
     }
+    xml[wave * 64 + lane] = make_float2(m_run, l_run);
     __syncthreads();
-    if (kp == 0 && !wave_idle) {
-      float out_max = 0.0f;
-      const float m1 = xm[qq * 64 + lane], l1 = xl[qq * 64 + lane];
-      const float m = fmaxf(m_run, m1);
-      const float a0 = __builtin_amdgcn_exp2f((m_run - m) * p.scale_log2);
+    float16v own[2];
+    {
+      const float2 other = xml[(wave ^ 4) * 64 + lane];
+      const float m0 = kp == 0 ? m_run : other.x, m1 = kp == 0 ? other.x : m_run;  // first and second half of the key range
+      const float m = fmaxf(m0, m1);
+      const float a0 = __builtin_amdgcn_exp2f((m0 - m) * p.scale_log2);
       const float a1 = (m1 == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f((m1 - m) * p.scale_log2);
-      const float inv_l = 1.0f / (l_run * a0 + l1 * a1);
-      const int64_t query = (int64_t)qtile * kQueries + qq * kWaveQueries + l32;
-      if (query < c.Lq) {
-        uint16_t* dst = c.out + (query * p.H + head) * kHeadDim;
+      const float mine = kp == 0 ? a0 : a1, theirs = kp == 0 ? a1 : a0;
+      l_run = (kp == 0 ? l_run : other.y) * a0 + (kp == 0 ? other.y : l_run) * a1;
+      m_run = m;
 #pragma unroll
-        for (int dt = 0; dt < 4; ++dt)
+      for (int i = 0; i < 8; ++i) {
+        const float4 x = xo[((wave ^ 4) * 8 + i) * 64 + lane];
+        const float xs[4] = {x.x, x.y, x.z, x.w};
+        const float16v keep = kp == 0 ? o[i >> 2] : o[2 + (i >> 2)];
 #pragma unroll
-          for (int rg = 0; rg < 4; ++rg) {
-            float v[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              const float o1 = xo[(qq * 64 + dt * 16 + 4 * rg + i) * 64 + lane];
-              v[i] = (o[dt][4 * rg + i] * a0 + o1 * a1) * inv_l;
-            }
-            const int d = dt * 32 + 8 * rg + 4 * lh;
-            const uint2 packed = make_uint2(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]));
-            *reinterpret_cast<uint2*>(dst + d) = packed;
-            out_max = abs_max_bf16x8(make_uint4(packed.x, packed.y, 0u, 0u), out_max);
-          }
+        for (int j = 0; j < 4; ++j) own[i >> 2][4 * (i & 3) + j] = keep[4 * (i & 3) + j] * mine + xs[j] * theirs;
       }
-      if (c.sink.parts) {
-        out_max = wave_max(out_max);
-        if (lane == 0) amax_sink_update(AmaxSink{c.sink.parts, c.sink.epoch, c.sink.epoch_offset}, (uint32_t)tile_id * 4 + qq, out_max);
+    }
+    if (c.parts > 1) {
+      // Part of a tile.  The workgroups of a tile each leave (O^T, reference point, row sum) in a record of their own and count
+      // their arrival; the last to arrive adds the parts up, from the first to the last, four at a time, its own from its
+      // registers at its place in that order - so the result does not depend on the order of arrival.  Stores and count are
+      // ordered as above.  Bound by the latency of the exchange past the L2 (store, count, load: about 8 us of a launch in
+      // all), hence 16-byte accesses with all of four parts in flight and no look at the counter ahead of the stores.
+      constexpr uint32_t kRecordBytes = (uint32_t)partial_bytes(kQueries), kWaveBytes = kRecordBytes / 8;
+      constexpr int kInFlight = 4;
+      const int parts = (int)c.parts, part = (int)(group_number(c.d.G) - (uint32_t)tile_id * c.parts);
+      const auto records = __builtin_amdgcn_make_buffer_rsrc(c.partials, 0, 0xFFFFFFFFu, 0x00027000u);
+      const uint32_t first_record = (uint32_t)tile_id * c.parts * kRecordBytes;
+      const uint32_t at_o = wave * kWaveBytes + lane * 16, at_ml = wave * kWaveBytes + 8 * 1024 + lane * 8;
+      {
+        const uint32_t rec = first_record + part * kRecordBytes;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const float16v& v = own[i >> 2];
+          store_shared_b128(records, at_o + i * 1024, rec, float4v{v[4 * (i & 3)], v[4 * (i & 3) + 1], v[4 * (i & 3) + 2], v[4 * (i & 3) + 3]});
+        }
+        store_shared_b64(records, at_ml, rec, float2v{m_run, l_run});
       }
+      __builtin_amdgcn_s_waitcnt(0x0F70);
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+      __syncthreads();
+      if (tid == 0)
+        tab.last_arrival = __hip_atomic_fetch_add(c.arrivals + tile_id, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == parts - 1;
+      __syncthreads();
+      if (tab.last_arrival == 0) break;
+      if (tid == 0) __hip_atomic_store(c.arrivals + tile_id, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // ready for the next launch
+      float16v sum[2];
+#pragma unroll
+      for (int d = 0; d < 2; ++d)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) sum[d][i] = 0.0f;
+      float m = -INFINITY, l = 0.0f;
+      for (int q0 = 0; q0 < parts; q0 += kInFlight) {
+        float4v v[kInFlight][8];
+        float2v ml[kInFlight];
+#pragma unroll
+        for (int j = 0; j < kInFlight; ++j) {  // behind the last part: the last again, which is not used
+          const uint32_t rec = first_record + min(q0 + j, parts - 1) * kRecordBytes;
+          ml[j] = load_shared_b64(records, at_ml, rec);
+#pragma unroll
+          for (int i = 0; i < 8; ++i) v[j][i] = load_shared_b128(records, at_o + i * 1024, rec);
+        }
+        float mj[kInFlight], m_new = m;
+#pragma unroll
+        for (int j = 0; j < kInFlight; ++j) {
+          mj[j] = q0 + j >= parts ? -INFINITY : q0 + j == part ? m_run : ml[j][0];
+          m_new = fmaxf(m_new, mj[j]);
+        }
+        const float a = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((m - m_new) * p.scale_log2);
+        m = m_new;
+        l *= a;
+#pragma unroll
+        for (int d = 0; d < 2; ++d)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) sum[d][i] *= a;
+#pragma unroll
+        for (int j = 0; j < kInFlight; ++j) {
+          if (q0 + j >= parts) break;
+          const bool mine = q0 + j == part;
+          const float w = mj[j] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((mj[j] - m_new) * p.scale_log2);
+          l += (mine ? l_run : ml[j][1]) * w;
+#pragma unroll
+          for (int d = 0; d < 2; ++d)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) sum[d][i] += (mine ? own[d][i] : v[j][4 * d + (i >> 2)][i & 3]) * w;
+        }
+      }
+      l_run = l;
+#pragma unroll
+      for (int d = 0; d < 2; ++d) own[d] = sum[d];
+    }
+    float out_max = 0.0f;
+    const float inv_l = 1.0f / l_run;
+    const int64_t query = (int64_t)qtile * kQueries + qq * kWaveQueries + l32;
+    if (query < c.Lq) {
+      uint16_t* dst = c.out + (query * p.H + head) * kHeadDim + 64 * kp;
+#pragma unroll
+      for (int d = 0; d < 2; ++d)
+#pragma unroll
+        for (int rg = 0; rg < 4; ++rg) {
+          const uint2 packed = make_uint2(pack_bf16(own[d][4 * rg] * inv_l, own[d][4 * rg + 1] * inv_l),
+                                          pack_bf16(own[d][4 * rg + 2] * inv_l, own[d][4 * rg + 3] * inv_l));
+          *reinterpret_cast<uint2*>(dst + d * 32 + 8 * rg + 4 * lh) = packed;
+          out_max = abs_max_bf16x8(make_uint4(packed.x, packed.y, 0u, 0u), out_max);
+        }
+    }
+    if (c.sink.parts) {
+      out_max = wave_max(out_max);
+      if (lane == 0) amax_sink_update(AmaxSink{c.sink.parts, c.sink.epoch, c.sink.epoch_offset}, (uint32_t)tile_id * 8 + wave, out_max);
     }
   }
   }
-  __syncthreads();  // the stages (and the merge area) are free for the next segment
+  if constexpr (!WIDE) break;
+  __syncthreads();  // the stages are free for the next segment
   }  // segments
 }
 
@@ -1125,17 +1236,20 @@ static int launch_attention(const AttnParams& p_in, hipStream_t stream) {
     LL_CHECK_LAUNCH("kv_attention_short_kernel");
     return LL_OK;
   }
-  AttentionPlan plan = plan_attention(p.Lq, p.H, p.n_cached + p.n_new, cus, policy);
+  AttentionPlan plan = plan_division(p.Lq, p.H, p.n_cached, p.n_new, cus, policy);
   StreamScratch w;
+  const bool capturing = plan.mode == LL_ATTENTION_SPLIT && stream_is_capturing(stream);
+  // A recorded launch takes 128-query tiles with shared key ranges only where the split division is asked for: replays on
+  // several streams may meet in the memory that these use, and what they take the place of mostly uses none.
+  if (capturing && policy == LL_ATTENTION_AUTO && plan.queries == kWgQueries) plan = plan_attention(p.Lq, p.H, p.n_cached + p.n_new, cus, policy);
   if (plan.mode == LL_ATTENTION_SPLIT) {
     // The split division passes partial tiles through device memory of the library's own.  While the stream is
     // being captured nothing may be allocated (and the clearing of a new set must not become a graph node): a set
     // that an earlier launch or ll_kv_attention_reserve left on this stream is used as it is; without one the
     // automatic choice falls back to the cheaper of the two divisions that need no memory, and an explicit
     // request for the split division is refused.
-    const bool capturing = stream_is_capturing(stream);
     bool missing = false;
-    if (int rc = stream_scratch(dev, stream, (size_t)2 * plan.d.G * kPartialFloats * sizeof(float), (size_t)plan.split_tiles, !capturing, w,
+    if (int rc = stream_scratch(dev, stream, partial_records(plan) * partial_bytes(plan.queries), (size_t)plan.split_tiles, !capturing, w,
                                 &missing, "ll_kv_attention")) return rc;
     if (missing) {
       if (policy == LL_ATTENTION_SPLIT) {
@@ -1149,15 +1263,16 @@ static int launch_attention(const AttnParams& p_in, hipStream_t stream) {
   p.n_qtiles = plan.n_qtiles;
   p.full_qtiles = plan.full_qtiles;
   p.d = plan.d;
-  if (plan.mode == LL_ATTENTION_NARROW) {
+  p.parts = (uint32_t)plan.parts;
+  if (plan.mode == LL_ATTENTION_SPLIT) {
+    p.partials = reinterpret_cast<float*>(w.records);
+    p.arrivals = w.counters;
+  }
+  if (plan.queries == kWgQueries) {
     static std::atomic<uint64_t> lds_allowed{0};
     if (int rc = allow_dynamic_lds(reinterpret_cast<const void*>(&kv_attention_kernel<false>), smem, lds_allowed, "ll_kv_attention")) return rc;
     hipLaunchKernelGGL(kv_attention_kernel<false>, dim3(p.d.G), dim3(kAttnThreads), smem, stream, p);
   } else {
-    if (plan.mode == LL_ATTENTION_SPLIT) {
-      p.partials = reinterpret_cast<float*>(w.records);
-      p.arrivals = w.counters;
-    }
     static std::atomic<uint64_t> lds_allowed_w{0};
     if (int rc = allow_dynamic_lds(reinterpret_cast<const void*>(&kv_attention_kernel<true>), smem, lds_allowed_w, "ll_kv_attention")) return rc;
     hipLaunchKernelGGL(kv_attention_kernel<true>, dim3(p.d.G), dim3(kAttnThreads), smem, stream, p);
@@ -1189,15 +1304,21 @@ extern "C" int ll_kv_attention_reserve_window(int64_t Lq, int num_heads, int64_t
   if (int rc = compute_units_of(dev, cus, "ll_kv_attention")) return rc;
   const int policy = g_attention_policy.load(std::memory_order_relaxed);
   if (short_kernel_waves(Lq, num_heads, n_cached, n_new, cus, policy)) return LL_OK;
-  const AttentionPlan plan = plan_attention(Lq, num_heads, n_cached + n_new, cus, policy);
-  if (plan.mode != LL_ATTENTION_SPLIT) return LL_OK;
+  // what the launch takes, and what it takes while the stream is being captured
+  const AttentionPlan plans[2] = {plan_division(Lq, num_heads, n_cached, n_new, cus, policy), plan_attention(Lq, num_heads, n_cached + n_new, cus, policy)};
+  size_t record_bytes = 0, counters = 0;
+  for (const AttentionPlan& plan : plans) {
+    if (plan.mode != LL_ATTENTION_SPLIT) continue;
+    record_bytes = std::max(record_bytes, partial_records(plan) * partial_bytes(plan.queries));
+    counters = std::max(counters, (size_t)plan.split_tiles);
+  }
+  if (record_bytes == 0) return LL_OK;
   if (stream_is_capturing(static_cast<hipStream_t>(stream))) {
     set_error("ll_kv_attention_reserve: the stream is being captured; reserve before the recording starts");
     return LL_ENOSUP;
   }
   StreamScratch w;
-  return stream_scratch(dev, static_cast<hipStream_t>(stream), (size_t)2 * plan.d.G * kPartialFloats * sizeof(float),
-                        (size_t)plan.split_tiles, true, w, nullptr, "ll_kv_attention_reserve");
+  return stream_scratch(dev, static_cast<hipStream_t>(stream), record_bytes, counters, true, w, nullptr, "ll_kv_attention_reserve");
 }
 
 // Cached keys are the longer way through the short kernel, and one fresh key may make a tile more: where these two need no
@@ -1222,7 +1343,7 @@ extern "C" int ll_kv_attention_plan_window(int64_t Lq, int num_heads, int64_t n_
     if (split_tiles) *split_tiles = 0;
     return LL_OK;
   }
-  const ll::AttentionPlan plan = ll::plan_attention(Lq, num_heads, n_cached + n_new, compute_units, policy);
+  const ll::AttentionPlan plan = ll::plan_division(Lq, num_heads, n_cached, n_new, compute_units, policy);
   if (division) *division = plan.mode;
   if (workgroups) *workgroups = plan.d.G;
   if (whole_rounds) *whole_rounds = plan.d.whole_rounds;

@@ -103,6 +103,9 @@ LL_SPLIT_FN uint32_t record_of_part(uint32_t g, uint32_t split_tile, const Divis
   return 2 * g + (first_tile == split_tile ? 0u : 1u);
 }
 
+// First iteration of part `part` of a tile of n_iter iterations in `parts` parts (part = parts: one past the last).
+LL_SPLIT_FN int first_iteration_of_part(uint32_t part, uint32_t parts, int n_iter) { return (int)(part * (uint32_t)n_iter / parts); }
+
 // ---- short launches (host): waves per workgroup with which kv_attention_short_kernel takes a launch, 0 for the tile
 // kernels.  It converts K and V once per 32 queries and fills a compute unit with one workgroup of eight or two of
 // four waves, so it is ahead while everything runs at once and the key range is short (us, tile kernels / 8 waves /
@@ -123,7 +126,7 @@ inline int short_kernel_waves(int64_t Lq, int H, int64_t n_cached, int64_t n_new
   if (policy > 0) return 0;
   const int64_t groups = H * ((Lq + 31) / 32), cached = (n_cached + 31) / 32, fresh = (n_new + 31) / 32;
   const int64_t length = cached + cached / 2 + fresh;
-  if (Lq > 256 * (int64_t)H) return 0;
+  if (Lq > 256 * (int64_t)H && length > 16) return 0;
   if (groups <= cus) return length > 176 ? 0 : (cached + fresh <= 12 ? 4 : 8);
   return groups <= 2 * (int64_t)cus && length <= 64 ? 4 : 0;
 }
@@ -132,15 +135,19 @@ inline int short_kernel_waves(int64_t Lq, int H, int64_t n_cached, int64_t n_new
 // count in full.
 struct AttentionPlan {
   int mode;             // LL_ATTENTION_NARROW / WIDE / SPLIT
+  int queries;          // per tile: 128 (NARROW, and SPLIT where plan_narrow_split is taken) or 256
+  int parts;            // 128-query tiles: workgroups that share the key range of each
   int n_qtiles;         // query tiles per head
   int full_qtiles;      // of which this many come first in the tile numbering (all of them unless mode is SPLIT)
   Division d;           // G = workgroups of the launch; units = 0 unless mode is SPLIT
   int64_t split_tiles;  // tiles of the split part
 };
 
+// The cost of a plan for the automatic choice, in the same unit, goes to `cost` (if asked for).
 // `allow_split` false leaves the split division out of the automatic choice (a launch that may not use the memory
 // partial tiles pass through).
-inline AttentionPlan plan_attention(int64_t Lq, int H, int64_t n_keys, int cus, int policy, bool allow_split = true) {
+inline AttentionPlan plan_attention(int64_t Lq, int H, int64_t n_keys, int cus, int policy, bool allow_split = true,
+                                    double* cost = nullptr) {
   constexpr double kWideIteration = 1.64;  // an iteration of the 256-query kernel takes this much longer for twice the work
   constexpr double kCombine = 6.0;         // partial results when every workgroup shares: writing, counting, combining
   constexpr double kCombineFew = 1.5;      // the same when only the workgroups without a whole extra tile share
@@ -193,6 +200,7 @@ inline AttentionPlan plan_attention(int64_t Lq, int H, int64_t n_keys, int cus, 
   const double cost_narrow = (double)((tiles_narrow + cus - 1) / cus) * ((double)n_iter + kRound);
   const double cost_wide = (double)((tiles_wide + cus - 1) / cus) * (kWideIteration * (double)n_iter + kRound);
   int mode = cost_narrow <= cost_wide && cost_narrow <= best.cost ? 0 : (cost_wide <= best.cost ? 1 : 2);
+  if (cost) *cost = mode == 0 ? cost_narrow : mode == 1 ? cost_wide : best.cost;
   if (policy >= 0) mode = policy;
   if (tiles_wide * n_iter >= (1ll << 31)) mode = 0;  // units are counted in 32 bits (costs in 64)
   if (mode == 2 && best.cost >= 1e300) mode = 1;     // nothing that could be split
@@ -201,6 +209,8 @@ inline AttentionPlan plan_attention(int64_t Lq, int H, int64_t n_keys, int cus, 
   plan.d.whole_rounds = 1;
   plan.d.n_iter = (uint32_t)n_iter;
   plan.d.light = kFullUnitCost;
+  plan.queries = mode == 0 ? 128 : 256;
+  plan.parts = 1;
   if (mode == 0) {
     plan.n_qtiles = plan.full_qtiles = (int)((Lq + 127) / 128);
     plan.d.G = (uint32_t)tiles_narrow;
@@ -223,6 +233,56 @@ inline AttentionPlan plan_attention(int64_t Lq, int H, int64_t n_keys, int cus, 
     }
   }
   return plan;
+}
+
+// Split division with tiles of 128 queries: the key range of every tile shared by the same number of workgroups (`parts`), all
+// in one round, each with one run of iterations.  Returns its cost in iterations of the 128-query kernel, 2 us each.  us, by
+// parts (in brackets: whole 128-query tiles / shares of 256-query tiles, which cross tiles and then pay for two prologues,
+// two exchanges and the 64-bit arithmetic of the shares):
+//    736 queries x 12, 1472 cached + 736 keys   31.6 (2) 27.4 (3)                   [44.3 / 40.4]
+//   1408 x 4, 2816 + 1408                       46.1 (2) 37.7 (3) 31.3 (4) 31.5 (5) [75.3 / 46.8]
+//   1760 x 8, 3520 + 1760                       58.2 (2)                            [91.8 / 63.2]
+//   2000 x 6, 0 + 2000                          29.7 (2)                            [39.4 / 38.7]
+//   3520 x 2, 7040 + 3520                       96.1 (2) 70.4 (3) 58.2 (4)          [172 / 70.3]
+//    512 x 4, 1024 + 512                        24.5 (2) 21.1 (3) 19.3 (4) 20.9 (5) 19.6 (6) 19.5 (8) 22.1 (12)
+//    736 x 12, 0 + 512                          17.6 (2) 18.0 (3)                   [15.6 / 25.1]
+// Two rounds of parts (880 x 24, 0.88 k + 880: 47.5 with three parts) lose against whole tiles (38.2).
+inline double plan_narrow_split(int64_t Lq, int H, int64_t n_keys, int cus, AttentionPlan& plan) {
+  constexpr double kRound = 4.0, kExchange = 2.5, kPerPart = 0.5;
+  const int64_t n_iter = (n_keys + 127) / 128, nq = (Lq + 127) / 128, tiles = H * nq;
+  int64_t parts = 0;
+  double best = 1e300;
+  for (int64_t s = 2; s * tiles <= cus && s <= n_iter; ++s) {
+    const double cost = (double)((n_iter + s - 1) / s) + kRound + kExchange + kPerPart * (double)s;
+    if (cost < best) {
+      best = cost;
+      parts = s;
+    }
+  }
+  if (parts < 2) return 1e300;
+  plan = AttentionPlan{};
+  plan.mode = 2;
+  plan.queries = 128;
+  plan.parts = (int)parts;
+  plan.n_qtiles = plan.full_qtiles = (int)nq;
+  plan.d.G = (uint32_t)(tiles * parts);
+  plan.d.n_iter = (uint32_t)n_iter;
+  plan.split_tiles = tiles;
+  return best;
+}
+
+// The division of a launch that the short kernel does not take, under `policy`.  The split division has tiles of 128 queries
+// where these are the cheapest division of all under the automatic choice.
+inline AttentionPlan plan_division(int64_t Lq, int H, int64_t n_cached, int64_t n_new, int cus, int policy, bool allow_split = true) {
+  constexpr double kCrossing = 5.0;  // what shares that cross 256-query tiles cost beyond plan_attention's estimate (40 instead of 30 us on the first shape above)
+  double cost = 0.0;
+  const AttentionPlan plan = plan_attention(Lq, H, n_cached + n_new, cus, policy == 2 ? -1 : policy, allow_split, &cost);
+  const bool may_split = policy == 2 /* LL_ATTENTION_SPLIT */ || (policy == -1 /* LL_ATTENTION_AUTO */ && allow_split);
+  if (may_split && !short_kernel_waves(Lq, H, n_cached, n_new, cus, -1)) {
+    AttentionPlan narrow;
+    if (plan_narrow_split(Lq, H, n_cached + n_new, cus, narrow) < cost + (plan.mode == 2 ? kCrossing : 0.0)) return narrow;
+  }
+  return policy == 2 ? plan_attention(Lq, H, n_cached + n_new, cus, policy, allow_split) : plan;
 }
 
 }  // namespace ll

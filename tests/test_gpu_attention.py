@@ -974,6 +974,21 @@ def test_short_launches_against_fp64(gpu, Lq, H, T, cached, n_new, peaked):
     assert (error <= 1.25 * 2 ** -9 * size + 2 ** -9 * ref.abs()).all()
 
 
+@pytest.mark.parametrize("peaked", [False, True])
+@pytest.mark.parametrize("Lq,H,T,cached,n_new,parts", [
+    (600, 2, 0, 0, 771, 4),         # seven iterations in four parts, three keys in the last one; queries behind a group of 32
+    (700, 2, 64, 865, 35, 4),       # the last slot attended in part; cached keys up to the last part, the chunk behind them
+    (513, 2, 64, 1024, 0, 4),       # nothing but cached keys
+    (1665, 6, 0, 0, 1281, 3),       # 84 tiles of 11 iterations in three parts: 3, 4 and 4
+    (1300, 1, 256, 4352, 1300, 9),  # more parts than are read at a time
+])
+def test_key_ranges_shared_by_workgroups_against_fp64(gpu, Lq, H, T, cached, n_new, parts, peaked):
+    """128-query tiles whose key ranges several workgroups share, under the checks and the bound of the short launches."""
+    plan = _native.attention_plan(Lq, H, cached + n_new, n_cached=cached)
+    assert plan == {"division": "split", "workgroups": parts * H * -(-Lq // 128), "whole_rounds": 0, "split_tiles": H * -(-Lq // 128)}
+    test_short_launches_against_fp64(gpu, Lq, H, T, cached, n_new, peaked)
+
+
 @pytest.mark.parametrize("Lq,H,keys", [(368, 16, 1472), (384, 2, 1152), (512, 16, 2560), (736, 12, 512)])
 def test_short_launches_are_no_further_from_fp64_than_the_tile_kernels(gpu, Lq, H, keys):
     """Relative error (2-norm) of the kernel with 32 queries per workgroup against that of the divided 256-query tiles (the

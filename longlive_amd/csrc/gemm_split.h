@@ -119,6 +119,15 @@ inline PersistentPlan plan_persistent(int64_t M, int64_t N, int64_t Kp, int n_pr
   return plan;
 }
 
+// Which kernel runs the 64 x 64 tiles (LL_GEMM_KERNEL_64X64): gemm_w4a4_small_kernel from three K steps of 256 on, else the tile
+// kernel, which has less to do before the first step and behind the last.  us, small kernel / tile kernel, by K:
+//   tiles       64           256          512          768          1024         1536
+//     8     4.4 / 3.6    4.3 / 4.1    4.9 / 5.0    5.4 / 6.0    6.1 / 7.0    7.2 / 8.9
+//    72     4.5 / 3.5    4.4 / 4.0    5.0 / 4.9    5.5 / 5.9    6.2 / 6.9    7.3 / 8.8
+//   384     5.4 / 4.5    5.3 / 5.4    6.5 / 6.7    7.3 / 8.2    8.2 / 9.7    10.0 / 12.7
+// It addresses eight rows of Kp / 2 bytes with 32-bit offsets.
+inline bool small_kernel_takes(int64_t Kp, int schedule) { return Kp > 512 && Kp < (1 << 28) && schedule != 2 /* LL_GEMM_TILES_COMPILED */; }
+
 // ---- which one-workgroup-per-tile kernel a launch takes (host arithmetic; the values are the header's
 // LL_GEMM_KERNEL_* codes)
 struct TileKernelChoice {
@@ -127,23 +136,28 @@ struct TileKernelChoice {
 };
 inline TileKernelChoice choose_tile_kernel(int64_t M, int64_t N, int64_t Kp, int n_products, int cus, int schedule) {
   // the generated loops address a row band with 32-bit offsets: 16 rows of Kp / 2 bytes
+  const int64_t tiles_64 = ((M + 63) / 64) * ((N + 63) / 64) * n_products;
   const bool generated_ok = Kp % 128 == 0 && Kp < (1 << 28) && schedule != 2 /* LL_GEMM_TILES_COMPILED */;
   // At most one 128 x 256 tile per compute unit, and more than half of the units busy: one workgroup of eight waves
   // per tile, the K range of every step split between its two halves.
   if (generated_ok && Kp >= 512) {
     const int64_t tiles = ((M + 127) / 128) * ((N + 255) / 256) * n_products;
-    if (tiles <= cus && 2 * tiles > cus) return {4, true};
+    // ... unless the 64 x 64 tiles of the small-product kernel are no more than four and a half per unit: 1320 x 3072 x 3072, 1008
+    // of them: 28.5 against 36.8 us; x 768 12.8 / 14.9, x 14336 116 / 139; 1400 x 3072 x 3072, 1056: 34.8 / 36.7; 1760 x 2560 x 2560,
+    // 1120: 30.0 / 32.3; but 736 x 8960 x 1536, 1680: 28.6 / 23.9.
+    if (tiles <= cus && 2 * tiles > cus) {
+      if (small_kernel_takes(Kp, schedule) && 2 * tiles_64 <= 9 * (int64_t)cus) return {0, false};
+      return {4, true};
+    }
   }
   // Small problems: when even 128 x 128 tiles would occupy at most half of the compute units, 64 x 64 tiles (more
-  // decode work per MFMA, but four times the workgroups) finish sooner.  Up to three of them per unit they still do where K is
-  // long, since each 128 x 128 tile then has a unit to itself with one wave per SIMD (880 x 3072 x 3072, 672 small tiles:
-  // 24.8 against 27.7 us; 1173 x 2048 x 8192, 608: 52.6 against 65.4; 1173 x 2304 x 9216, 684: 59.9 against 72.8; 1173 x 2560 x
-  // 10240, 760: 68 against 81; 368 x 8192 x 2048, 768: 22.0 against 22.2; but
-  // 1760 x 2048 x 8192, 896: 68.3 against 65.8, and 256 x 14336 x 3072, 896: 32.5 against
-  // 28.4; with K = 1536, 335 x 5888, 552: 16.4 against 16.0).
+  // decode work per MFMA, but four times the workgroups) finish sooner.  Up to three of them per unit they still do in the
+  // small-product kernel, since each 128 x 128 tile then has a unit to itself or shares it with one other (us, that kernel /
+  // tiles of 128 x 128): 1320 x 1536 x 1536, 504 small tiles: 10.4 / 16.1; x 640 7.5 / 9.2; 335 x 5888 x 1536, 552: 14.7 / 15.9; 1500 x
+  // 2048 x 1536, 768: 15.0 / 16.4; 1760 x 1536 x 768, 672: 10.3 / 10.3; but 2640 x 1024 x 640, 672: 10.4 / 9.6; 736 x 4608 x 1536,
+  // 864: 18.2 / 16.5; 2048 x 2048 x 8192, 1024: 72.9 / 69.6.
   const int64_t tiles_128 = ((M + 127) / 128) * ((N * n_products + 127) / 128);
-  const int64_t tiles_64 = ((M + 63) / 64) * ((N + 63) / 64) * n_products;
-  if (tiles_128 <= cus / 2 || (schedule != 2 && Kp >= 2048 && tiles_64 <= 3 * (int64_t)cus)) return {0, false};
+  if (tiles_128 <= cus / 2 || (small_kernel_takes(Kp, schedule) && tiles_64 <= (Kp >= 768 ? 3 : 2) * (int64_t)cus)) return {0, false};
   // Two workgroups of four waves are resident per compute unit.  The 256 x 128 / 128 x 256 tiles need 6 decode
   // instructions per MFMA, the 128 x 128 tile 8, so the larger tiles win unless they fill the slots much worse.  A last
   // round of at most one workgroup per unit is cheap: alone on its unit a workgroup runs in 0.56 of the time it takes
@@ -169,17 +183,8 @@ inline TileKernelChoice choose_tile_kernel(int64_t M, int64_t N, int64_t Kp, int
   return {best, generated_ok && best >= 2};
 }
 
-// Which kernel runs the 64 x 64 tiles (LL_GEMM_KERNEL_64X64): gemm_w4a4_small_kernel from five K steps of 256 on, else the tile
-// kernel, which has less to do before the first step and behind the last.  us, small kernel / tile kernel, by K:
-//   tiles       256          512          768          1024         1536         3072
-//     8     5.31 / 4.01  5.80 / 4.92  6.34 / 5.91  7.17 / 6.87  8.19 / 8.81  11.5 / 14.8
-//    72     5.43 / 3.92  5.90 / 4.82  6.45 / 5.78  7.29 / 6.74  8.28 / 8.68  11.7 / 14.6
-//   384     6.38 / 5.22  7.37 / 6.70  8.70 / 8.41  9.97 / 9.80  11.7 / 12.7  17.4 / 21.7
-// It addresses eight rows of Kp / 2 bytes with 32-bit offsets.
-inline bool small_kernel_takes(int64_t Kp, int schedule) { return Kp > 1024 && Kp < (1 << 28) && schedule != 2 /* LL_GEMM_TILES_COMPILED */; }
-
 // How the small-product kernel divides a launch: 64 x 64 tiles, each by `parts` workgroups that share its K range (steps of
-// 256 elements).  Measured: a step takes 0.55 us with one workgroup on every compute unit; handing two to four parts over
+// 256 elements).  Measured when a step took 0.55 us (0.47 now) with one workgroup on every compute unit; handing two to four parts over
 // and adding them up takes 2.4 us (their records are read four at a time: five to eight 3.6); with more workgroups than
 // units a step takes 0.8 and the launch 2 us more.  us by parts:
 //                     tiles, steps    1     2     3     4     5     6     8    12
@@ -198,14 +203,25 @@ inline bool small_kernel_takes(int64_t Kp, int schedule) { return Kp > 1024 && K
 constexpr int kSmallParts = 4, kSmallPartsSteps = 16;
 constexpr int kSmallRecordBytes = 64 * 64 * 4;                            // a part's fp32 sums of its tile
 inline int64_t small_product_units(int cus) { return 2 * (int64_t)cus; }  // most (tile, part) pairs of a launch with parts
+// Tiles of 64 x 96 where those of 64 x 64 would be more than one per unit and these are not: a step takes 0.71 us against 0.9 us
+// for two of the smaller ones (us, 64 x 64 / 64 x 96: 512 x 3072 x 3072 15.2 / 13.7, 736 x 1536 x 1536 9.9 / 9.4, x 8960 33.3 / 30.5,
+// 440 x 3072 x 14336 50.4 / 45.2).  Larger ones were measured too: 64 x 128 and 96 x 128 were never ahead of both, 128 x 128 by 6 % on
+// 2048 x 2048 x 3072.
 struct SmallGemmPlan {
+  int fb;  // tiles of 64 rows by 32 fb columns
   int parts;
   int tiles_m, tiles_n_each;
   int64_t tiles;
 };
 inline SmallGemmPlan plan_small_gemm(int64_t M, int64_t N, int64_t Kp, int n_products, int cus) {
-  SmallGemmPlan p{1, (int)((M + 63) / 64), (int)((N + 63) / 64), 0};
+  SmallGemmPlan p{2, 1, (int)((M + 63) / 64), (int)((N + 63) / 64), 0};
   p.tiles = (int64_t)p.tiles_m * p.tiles_n_each * n_products;
+  if (const int64_t each = (N + 95) / 96, wide = p.tiles_m * each * n_products; Kp >= 1024 && p.tiles > cus && wide <= cus) {
+    p.fb = 3;
+    p.tiles_n_each = (int)each;
+    p.tiles = wide;
+    return p;
+  }
   const int64_t steps = (Kp + 255) / 256;
   if (steps < kSmallPartsSteps) return p;
   double best = 0.0;

@@ -729,28 +729,40 @@ __global__ __launch_bounds__(256) void gemm_w4a4_persistent_kernel(PersistentPar
 
 
 // ============================================================================ small products
-// 64 x 64 tiles for products that give at most half a 128 x 128 tile per compute unit.  A workgroup is four waves; each
-// holds the whole 64 x 64 tile (2 x 2 fragments) and multiplies one quarter of every K step of 256 elements, so a
-// decoded fragment serves two MFMAs (8 decode instructions per MFMA; the tile kernel above, whose four waves share the
-// tile out as 32 x 32 each, decodes 16).  With one or two waves per SIMD the kernel is bound by the instructions a wave
-// issues, one per four cycles whatever their kind: the stages of the ring are unrolled so that LDS addresses are
-// immediates, and the loads take a scalar base.  Behind the loop each wave finishes one of the four fragments: it adds
-// the other waves' parts of it, always in the order of the K quarters, from LDS.  Where there are few tiles and K is
-// long, several workgroups share the K range of a tile (plan_small_gemm).
-// Measured (this kernel / the 64 x 64 tile kernel above): 512 x 3072 x 3072 16.6 / 21.8 us, 128 x 3072 x 14336 21.8 / 58.1 us
-// (four parts), 64 x 512 x 5888 10.7 / 25.3 us (four parts), 736 x 1536 x 8960 35.2 / 56.2 us.  The kernel above keeps
-// short contractions (small_kernel_takes) and LL_GEMM_TILES_COMPILED (one order of summation for every shape).
+// 64 x 64 tiles, or 64 x 96, for products that give a compute unit no more than three or four of them (choose_tile_kernel,
+// plan_small_gemm).  A workgroup is four waves; each holds the whole tile (2 x 2 or 2 x 3 fragments) and multiplies one quarter
+// of every K step of 256 elements, so a decoded fragment serves two MFMAs or more (8 or 6.7 decode instructions per MFMA; the
+// tile kernel above, whose four waves share a 64 x 64 tile out as 32 x 32 each, decodes 16).  With one or two waves per SIMD the
+// kernel is bound by the instructions a wave issues, one per four to five cycles whatever their kind: the stages of the ring
+// are unrolled so that LDS addresses are immediates, the loads take a scalar base, and a step that is followed by four more
+// has two branches.  Behind the loop the waves' parts are added in two steps, which move three quarters of the tile through
+// LDS and leave every wave with a quarter of it (exchange_quarters), always in the order of the K quarters.  Where there are
+// few tiles and K is long, several workgroups share the K range of a tile (plan_small_gemm).
+// Measured (this kernel / with one exchange in which a wave gathered its fragment from three others, and four branches around
+// the waits of a step / the 64 x 64 tile kernel above): 512 x 3072 x 3072 13.7 / 16.2 / 21.8 us, 736 x 1536 x 1536 9.4 / 11.0, 368 x 2048
+// x 2048 8.2 / 9.6, 736 x 1536 x 8960 30.5 / 35.5 / 56.2, 40 x 2048 x 2048 8.1 / 9.5.  The kernel above keeps short contractions
+// (small_kernel_takes) and LL_GEMM_TILES_COMPILED (one order of summation for every shape).
 constexpr int kSmallThreads = 256;
 constexpr int kSmallStages = 4;
 constexpr int kSmallK = 256;                                  // K elements per step: 64 per wave
 constexpr int kSmallRow = kSmallK / 2;                        // bytes per row and stage; pieces stored at piece ^ (row % 8)
-constexpr int kSmallVals = 64 * kSmallRow;                    // one operand's values of a stage
-constexpr int kSmallScales = 4 * 512;                         // one operand's scales: four 128 x 4 tiles
-constexpr int kSmallStage = 2 * (kSmallVals + kSmallScales);
-constexpr int kSmallSmem = kSmallStages * kSmallStage;
-constexpr int kSmallFlag = 4 * 3 * 4096;                      // behind the exchange
-static_assert(kSmallFlag + 16 <= kSmallSmem && 2 * kSmallSmem <= 160 * 1024, "the exchange fits the ring, two workgroups fit a unit");
-constexpr int kSmallWholeSmem = kSmallSmem + kSmallFlag;      // WHOLE: the exchange lies behind the ring, which stays full
+constexpr int kSmallFragment = 32 * kSmallRow;                // the values of 32 rows of a stage
+constexpr int kSmallScales = 4 * 512;                         // the scales of 128 rows of a stage: four 128 x 4 tiles
+constexpr int kSmallFA = 2;                                   // fragments of 32 rows of A in a tile
+// A tile of 64 rows of A by 32 FB rows of B.  96 rows may lie in two of the 128-row blocks of the scales.
+template <int FB>
+struct SmallTile {
+  static constexpr int kBlocks = 1 + (FB == 3 ? 2 : 1);       // of scales: A's, B's
+  static constexpr int kValues = (kSmallFA + FB) * kSmallFragment;
+  static constexpr int kStage = kValues + kBlocks * kSmallScales;
+  static constexpr int kScaleLoads = (2 * kBlocks + 3) / 4;   // per wave and step, 1 KB each
+  static constexpr int kLoads = kSmallFA + FB + kScaleLoads;
+  static constexpr int kRing = kSmallStages * kStage;
+  static constexpr int kExchange = FB * 4 * 4096;             // half of each wave's sums
+  static_assert(kExchange + 16 <= kRing && kRing <= 160 * 1024, "the exchange and a flag fit the ring");
+};
+static_assert(2 * SmallTile<2>::kRing <= 160 * 1024, "two workgroups fit a unit");
+constexpr int kSmallWholeSmem = SmallTile<2>::kRing + SmallTile<2>::kExchange;  // WHOLE: the exchange lies behind the ring, which stays full
 
 // 16 bytes per lane from base + offset straight into LDS at lds_base + IMM + 16 * lane (see load_to_lds_b128).
 template <int IMM>
@@ -759,13 +771,20 @@ __device__ __forceinline__ void load_to_lds_b128_at(const uint8_t* base, uint32_
                : "memory", "scc");
 }
 
+// One such load of every fragment's rows, each kSmallFragment behind the one before it.
+template <int IMM, int F = 0, int N>
+__device__ __forceinline__ void load_fragments_to_lds(const uint8_t* const (&base)[N], uint32_t offset, uint32_t lds_base) {
+  load_to_lds_b128_at<IMM + F * kSmallFragment>(base[F], offset, lds_base);
+  if constexpr (F + 1 < N) load_fragments_to_lds<IMM, F + 1>(base, offset, lds_base);
+}
+
 // WHOLE: one workgroup computes all parts of its tile one after the other and adds them up in their order, which gives the
 // bits of `parts` workgroups without the memory that these share.  That memory belongs to a stream, and a recorded launch
 // may be replayed on any stream beside others: two that counted their arrivals in the same words would add up each other's
 // parts.  The loads run on across the parts; what a part costs is its exchange through LDS, 2 us.  Four parts (the workgroups
 // that share them / one for all / the 64 x 64 tile kernel above): 64 x 512 x 5888 10.6 / 24.2 / 25.5 us, 112 x 2944 x 8192 15.3 /
 // 28.6 / 34.7, 128 x 3072 x 14336 21.8 / 41.8 / 58.3, 48 x 1024 x 4096 10.2 / 20.1 / 18.7.
-template <bool WHOLE>
+template <bool WHOLE, int FB>
 __global__ __launch_bounds__(kSmallThreads, WHOLE ? 1 : 2) void gemm_w4a4_small_kernel(
     const uint8_t* __restrict__ Av, const uint8_t* __restrict__ As, const uint8_t* __restrict__ Bv0,
     const uint8_t* __restrict__ Bs0, const float* __restrict__ alpha_ptr0, const float* __restrict__ amax_a,
@@ -807,7 +826,10 @@ __global__ __launch_bounds__(kSmallThreads, WHOLE ? 1 : 2) void gemm_w4a4_small_
       epi.sink = gg.sink;
     }
   }
-  const int row0 = tile_m * 64, col0 = tile_n * 64;
+  using S = SmallTile<FB>;
+  constexpr int FA = kSmallFA;
+  constexpr int kFragments = FA + FB;  // A first
+  const int row0 = tile_m * (32 * FA), col0 = tile_n * (32 * FB);
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, lh = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int all_steps = (Kp + kSmallK - 1) / kSmallK;
@@ -815,122 +837,154 @@ __global__ __launch_bounds__(kSmallThreads, WHOLE ? 1 : 2) void gemm_w4a4_small_
   const int t0 = WHOLE ? 0 : first_step(part);
   const int nk = WHOLE ? all_steps : first_step(part + 1) - t0;
 
-  // ---- global -> LDS: a load instruction covers 1 KB = 8 rows of 128 bytes.  Wave w brings rows 8 w .. and 32 + 8 w .. of
-  // A and of B and 1 KB of scales (waves 0, 1: A, tiles 0-1 and 2-3 of the step; waves 2, 3: B).  The tiles of a matrix
-  // padded to 128 rows have all their rows.
+  // ---- global -> LDS: a load instruction covers 1 KB = 8 rows of 128 bytes.  Wave w brings rows 8 w .. 8 w + 7 of every
+  // fragment and one or two KB of scales.  The matrices are padded to 128 rows; a fragment of B behind them is the last one again.
   const int64_t row_bytes = Kp >> 1;
   const int piece = (lane & 7) ^ (lane >> 3);      // the row's piece that belongs at this lane's position
-  const uint8_t* a_src = Av + (int64_t)(row0 + 8 * wave) * row_bytes + (int64_t)t0 * kSmallRow;
-  const uint8_t* b_src = Bv + (int64_t)(col0 + 8 * wave) * row_bytes + (int64_t)t0 * kSmallRow;
-  const uint8_t* s_src = (wave < 2 ? As + (int64_t)(row0 >> 7) * (Kp >> 6) * 512 : Bs + (int64_t)(col0 >> 7) * (Kp >> 6) * 512) +
-                         (wave & 1) * 1024 + (int64_t)t0 * 2048;
-  const uint8_t* src[4] = {a_src, a_src + 32 * row_bytes, b_src, b_src + 32 * row_bytes};
+  const uint8_t* src[kFragments];
+#pragma unroll
+  for (int f = 0; f < kFragments; ++f)
+    src[f] = (f < FA ? Av + (int64_t)(row0 + 32 * f + 8 * wave) * row_bytes
+                     : Bv + (int64_t)(min(col0 + 32 * (f - FA), Np - 32) + 8 * wave) * row_bytes) + (int64_t)t0 * kSmallRow;
+  const uint8_t* s_src[S::kScaleLoads];
+  uint32_t s_dst[S::kScaleLoads];
+#pragma unroll
+  for (int i = 0; i < S::kScaleLoads; ++i) {
+    const int at = min(wave + 4 * i, 2 * S::kBlocks - 1), block = at >> 1;  // behind the last: the last again
+    const int64_t first = block == 0 ? row0 >> 7 : min((col0 >> 7) + block - 1, (Np >> 7) - 1);
+    s_src[i] = (block == 0 ? As : Bs) + first * (Kp >> 6) * 512 + (at & 1) * 1024 + (int64_t)t0 * 2048;
+    s_dst[i] = lds_address(smem) + S::kValues + at * 1024;
+  }
   uint32_t voff = (uint32_t)(lane >> 3) * (uint32_t)row_bytes + (uint32_t)piece * 16u, soff = (uint32_t)lane * 16u;
   const uint32_t v_dst = lds_address(smem) + wave * 1024;
   auto load_step = [&](int step, auto stage) __attribute__((always_inline)) {  // called for the steps in order
-    constexpr int kBase = decltype(stage)::value * kSmallStage;
+    constexpr int kBase = decltype(stage)::value * S::kStage;
     const int k0 = (t0 + step) * kSmallK;
     if (k0 + kSmallK <= Kp) {
-      load_to_lds_b128_at<kBase>(src[0], voff, v_dst);
-      load_to_lds_b128_at<kBase + 4096>(src[1], voff, v_dst);
-      load_to_lds_b128_at<kBase + 8192>(src[2], voff, v_dst);
-      load_to_lds_b128_at<kBase + 12288>(src[3], voff, v_dst);
-      load_to_lds_b128_at<kBase + 16384>(s_src, soff, v_dst);
+      load_fragments_to_lds<kBase>(src, voff, v_dst);
+#pragma unroll
+      for (int i = 0; i < S::kScaleLoads; ++i) load_to_lds_b128_at<kBase>(s_src[i], soff, s_dst[i]);
     } else {  // the rows end inside this step: zeros behind their end
       const uint8_t* zero16 = reinterpret_cast<const uint8_t*>(&g_gemm_zero16);
-      const bool have = k0 + piece * 32 < Kp, have_scales = k0 + 64 * (2 * (wave & 1) + (lane >> 5)) < Kp;
+      const bool have = k0 + piece * 32 < Kp;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) load_to_lds_b128(have ? src[i] + voff : zero16, v_dst + kBase + i * 4096);
-      load_to_lds_b128(have_scales ? s_src + soff : zero16, v_dst + kBase + 16384);
+      for (int f = 0; f < kFragments; ++f) load_to_lds_b128(have ? src[f] + voff : zero16, v_dst + kBase + f * kSmallFragment);
+#pragma unroll
+      for (int i = 0; i < S::kScaleLoads; ++i) {
+        const int half = min(wave + 4 * i, 2 * S::kBlocks - 1) & 1;
+        load_to_lds_b128(k0 + 64 * (2 * half + (lane >> 5)) < Kp ? s_src[i] + soff : zero16, s_dst[i] + kBase);
+      }
     }
     voff += kSmallRow;
     soff += 2048;
   };
 
-  // ---- the lane's LDS reads: row 32 f + l32, piece 2 wave + lh; the scale bytes of the piece's two blocks
-  const uint8_t* v_rd = smem + l32 * kSmallRow + 16 * ((2 * wave + lh) ^ (l32 & 7));
-  const uint8_t* s_rd = smem + 2 * kSmallVals + 512 * wave + l32 * 16 + 2 * lh;
-  const uint8_t* sa_rd = s_rd + ((row0 & 127) >> 5) * 4;
-  const uint8_t* sb_rd = s_rd + kSmallScales + ((col0 & 127) >> 5) * 4;
+  // ---- the lane's LDS reads: row l32 of a fragment, piece 2 wave + lh; the scale bytes of the piece's two blocks.  A wave
+  // takes its fragments in an order in which those whose sums it will keep (exchange_quarters) come first: of A the first in
+  // waves 0 and 2 and the second in waves 1 and 3, of B the first kKeepB in waves 0 and 1 and the others in 2 and 3.
+  constexpr int kKeepB = (FB + 1) / 2;
+  const bool odd = wave & 1, upper = wave & 2;
+  const uint8_t *v_rd[kFragments], *s_rd[kFragments];
+#pragma unroll
+  for (int f = 0; f < kFragments; ++f) {
+    const int own = f < FA ? (odd ? 1 - f : f) : FA + (upper ? (f - FA + kKeepB) % FB : f - FA);
+    v_rd[f] = smem + l32 * kSmallRow + 16 * ((2 * wave + lh) ^ (l32 & 7)) + own * kSmallFragment;
+    const int first = f < FA ? row0 : col0, at = first + 32 * (f < FA ? own : own - FA);  // of the operand's rows
+    const int block = (at >> 7) - (first >> 7) + (f < FA ? 0 : 1);
+    s_rd[f] = smem + S::kValues + block * kSmallScales + 512 * wave + l32 * 16 + 2 * lh + ((at & 127) >> 5) * 4;
+  }
   struct Raw {
-    uint4 v[4];  // fragments A0, A1, B0, B1
-    uint32_t sc[4];
+    uint4 v[kFragments];
+    uint32_t sc[kFragments];
   };
   auto read_raw = [&](Raw& h, auto stage) __attribute__((always_inline)) {
-    constexpr int kBase = decltype(stage)::value * kSmallStage;
+    constexpr int kBase = decltype(stage)::value * S::kStage;
 #pragma unroll
-    for (int f = 0; f < 4; ++f) {
-      h.v[f] = *reinterpret_cast<const uint4*>(v_rd + kBase + f * 4096);
-      h.sc[f] = *reinterpret_cast<const uint16_t*>((f < 2 ? sa_rd : sb_rd) + kBase + 4 * (f & 1));
+    for (int f = 0; f < kFragments; ++f) {
+      h.v[f] = *reinterpret_cast<const uint4*>(v_rd[f] + kBase);
+      h.sc[f] = *reinterpret_cast<const uint16_t*>(s_rd[f] + kBase);
     }
   };
-  float16v acc[2][2];
+  constexpr int kProducts = FA * FB;
+  float16v acc[FB][FA];
+  auto clear_sums = [&]() __attribute__((always_inline)) {
 #pragma unroll
-  for (int g = 0; g < 2; ++g)
+    for (int q = 0; q < kProducts; ++q)
 #pragma unroll
-    for (int f = 0; f < 2; ++f)
+      for (int i = 0; i < 16; ++i) acc[q / FA][q % FA][i] = 0.0f;
+  };
+  clear_sums();
+  half8v o[2][kFragments];
 #pragma unroll
-      for (int i = 0; i < 16; ++i) acc[g][f][i] = 0.0f;
-  half8v o[2][4];
-#pragma unroll
-  for (int f = 0; f < 4; ++f)
+  for (int f = 0; f < kFragments; ++f)
 #pragma unroll
     for (int i = 0; i < 8; ++i) o[1][f][i] = (_Float16)0.0f;  // the first step's "previous sub-step" adds nothing
-  // The four MFMAs of a sub-step with the decode of the next one between them, a fragment (eight instructions) behind
-  // each; the scheduling barriers hold that order (left to itself the compiler pairs MFMAs that depend on each other).
-  auto mma_under = [&](half8v (&dst)[4], const Raw& h, const half2v (&s2)[4][2], int j, const half8v (&x)[4]) __attribute__((always_inline)) {
+  // The MFMAs of a sub-step with the decode of the next one between them, a fragment (eight instructions) behind every first,
+  // or every first or second; the scheduling barriers hold that order (left to itself the compiler pairs MFMAs that depend
+  // on each other).
+  auto mma_under = [&](half8v (&dst)[kFragments], const Raw& h, const half2v (&s2)[kFragments][2], int j, const half8v (&x)[kFragments]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      acc[i >> 1][i & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[2 + (i >> 1)], x[i & 1], acc[i >> 1][i & 1], 0, 0, 0);
-      const uint32_t w = j == 0 ? h.v[i].x : j == 1 ? h.v[i].y : j == 2 ? h.v[i].z : h.v[i].w;
-      dst[i] = decode8(w, s2[i][j >> 1]);
-      asm volatile("" : "+v"(dst[i]));  // here, and not sunk behind the branches to the MFMA that reads it
+    for (int q = 0; q < kProducts; ++q) {
+      acc[q / FA][q % FA] = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[FA + q / FA], x[q % FA], acc[q / FA][q % FA], 0, 0, 0);
+#pragma unroll
+      for (int i = q * kFragments / kProducts; i < (q + 1) * kFragments / kProducts; ++i) {
+        const uint32_t w = j == 0 ? h.v[i].x : j == 1 ? h.v[i].y : j == 2 ? h.v[i].z : h.v[i].w;
+        dst[i] = decode8(w, s2[i][j >> 1]);
+      }
       __builtin_amdgcn_sched_barrier(0);
     }
+#pragma unroll
+    for (int i = 0; i < kFragments; ++i) asm volatile("" : "+v"(dst[i]));  // here, and not sunk behind the branches to the MFMA that reads it
   };
-  // The wave's five loads of the step that comes next have landed; those of the `behind` steps after it may be under way.
-  auto wait_loads = [&](int behind) __attribute__((always_inline)) {
-    if (behind >= 3) __builtin_amdgcn_s_waitcnt(0x0F7F);       // vmcnt(15)
-    else if (behind == 2) __builtin_amdgcn_s_waitcnt(0x0F7A);  // vmcnt(10)
-    else if (behind == 1) __builtin_amdgcn_s_waitcnt(0x0F75);  // vmcnt(5)
-    else __builtin_amdgcn_s_waitcnt(0x0F70);
+  constexpr std::integral_constant<int, 0> kS0{};
+  constexpr std::integral_constant<int, 1> kS1{};
+  constexpr std::integral_constant<int, 2> kS2{};
+  constexpr std::integral_constant<int, 3> kS3{};
+  // The wave's loads of the step that comes next have landed; those of the `behind` steps after it may be under way.
+  auto wait_loads = [&](auto behind) __attribute__((always_inline)) {
+    constexpr int n = decltype(behind)::value * S::kLoads;
+    __builtin_amdgcn_s_waitcnt(0x0F70 | (n & 15) | ((n >> 4) << 14));  // vmcnt(n)
   };
   // The MFMAs of the last sub-step, whose operands are decoded.
   auto mma_last = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      acc[i >> 1][i & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(o[1][2 + (i >> 1)], o[1][i & 1], acc[i >> 1][i & 1], 0, 0, 0);
+    for (int q = 0; q < kProducts; ++q)
+      acc[q / FA][q % FA] = __builtin_amdgcn_mfma_f32_32x32x16_f16(o[1][FA + q / FA], o[1][q % FA], acc[q / FA][q % FA], 0, 0, 0);
   };
-  // The K quarters of the four waves meet: wave w adds up fragment (g, f) = (w / 2, w % 2), of which the others leave their
-  // parts in LDS.
-  float16v sum[1][1];
+  // The K quarters of the four waves meet in two steps: waves w and w ^ 1 leave each other the sums of the A fragment that
+  // the other one keeps in LDS and add, then waves w and w ^ 2 those of the B fragments.  Every result is (0 + 1) + (2 + 3),
+  // whatever the tile.  Of three B fragments the second in the wave's order is kept in waves 0 and 1 and left in 2 and 3.
   auto exchange_quarters = [&](float* exchange) __attribute__((always_inline)) {
+    auto give = [&](const float16v& a, int slot) __attribute__((always_inline)) {
+      float* dst = exchange + (wave * FB + slot) * 1024 + lane * 4;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const float16v& a = acc[q >> 1][q & 1];
-      if (q == wave) {
-        sum[0][0] = a;
-      } else {
-        float* dst = exchange + (q * 3 + (wave < q ? wave : wave - 1)) * 1024 + lane * 4;
+      for (int i = 0; i < 4; ++i) *reinterpret_cast<float4*>(dst + i * 256) = make_float4(a[4 * i], a[4 * i + 1], a[4 * i + 2], a[4 * i + 3]);
+    };
+    auto take = [&](float16v& a, int from, int slot) __attribute__((always_inline)) {
+      const float* p = exchange + (from * FB + slot) * 1024 + lane * 4;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) *reinterpret_cast<float4*>(dst + i * 256) = make_float4(a[4 * i], a[4 * i + 1], a[4 * i + 2], a[4 * i + 3]);
+      for (int i = 0; i < 4; ++i) {
+        const float4 x = *reinterpret_cast<const float4*>(p + i * 256);
+        a[4 * i] += x.x;
+        a[4 * i + 1] += x.y;
+        a[4 * i + 2] += x.z;
+        a[4 * i + 3] += x.w;
       }
-    }
+    };
+#pragma unroll
+    for (int g = 0; g < FB; ++g) give(acc[g][1], g);
     __syncthreads();
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float* p = exchange + wave * 3 * 1024 + lane * 4 + i * 256;
-      const float4 x = *reinterpret_cast<const float4*>(p), y = *reinterpret_cast<const float4*>(p + 1024),
-                   z = *reinterpret_cast<const float4*>(p + 2048);
-      const float xs[4] = {x.x, x.y, x.z, x.w}, ys[4] = {y.x, y.y, y.z, y.w}, zs[4] = {z.x, z.y, z.z, z.w};
+    for (int g = 0; g < FB; ++g) take(acc[g][0], wave ^ 1, g);
+    __syncthreads();
+    // the slot is the fragment's place in the other wave's order
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {  // x, y, z: the three other waves in order; own part at its place
-        const float m = sum[0][0][4 * i + c];
-        const float s0 = wave == 0 ? m : xs[c], s1 = wave == 1 ? m : (wave == 0 ? xs[c] : ys[c]);
-        const float s2v = wave == 2 ? m : (wave == 3 ? zs[c] : ys[c]), s3 = wave == 3 ? m : zs[c];
-        sum[0][0][4 * i + c] = (s0 + s1) + (s2v + s3);
-      }
-    }
+    for (int g = FB - kKeepB; g < FB; ++g)
+      if (g >= kKeepB || upper) give(acc[g][0], g - (g >= kKeepB && !upper ? kKeepB : FB - kKeepB));
+    __syncthreads();
+#pragma unroll
+    for (int g = 0; g < kKeepB; ++g)
+      if (g < FB - kKeepB || !upper) take(acc[g][0], wave ^ 2, g);
     __syncthreads();  // the exchange may be written again
   };
   // WHOLE: behind the last step of a part.  What the accumulators hold is added to the parts before it, as the workgroup that
@@ -938,50 +992,54 @@ __global__ __launch_bounds__(kSmallThreads, WHOLE ? 1 : 2) void gemm_w4a4_small_
   float16v all;
   auto end_part = [&](int p) __attribute__((always_inline)) {
     mma_last();
-    exchange_quarters(reinterpret_cast<float*>(smem + kSmallSmem));
+    exchange_quarters(reinterpret_cast<float*>(smem + S::kRing));
 #pragma unroll
-    for (int i = 0; i < 16; ++i) all[i] = (p == 0 ? 0.0f : all[i]) + sum[0][0][i];
+    for (int i = 0; i < 16; ++i) all[i] = (p == 0 ? 0.0f : all[i]) + acc[0][0][i];
+    clear_sums();
 #pragma unroll
-    for (int g = 0; g < 4; ++g)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) acc[g >> 1][g & 1][i] = 0.0f;
-#pragma unroll
-    for (int f = 0; f < 4; ++f)
+    for (int f = 0; f < kFragments; ++f)
 #pragma unroll
       for (int i = 0; i < 8; ++i) o[1][f][i] = (_Float16)0.0f;
   };
   // One K step from the packed words in h; the words of the step behind it are read into `next` half way through,
   // when every wave has its loads of that step in LDS and has read this step's stage for the last time (the stage is
   // then refilled with the step four further on), so that neither the barrier nor the LDS latency is waited out.
-  auto step = [&](int t, auto stage, const Raw& h, Raw& next) __attribute__((always_inline)) {
+  auto step = [&](int t, auto stage, Raw& h, Raw& next) __attribute__((always_inline)) {
     constexpr int kStageNo = decltype(stage)::value;
-    half2v s2[4][2];
+    half2v s2[kFragments][2];
 #pragma unroll
-    for (int f = 0; f < 4; ++f) {
+    for (int f = 0; f < kFragments; ++f) {
+      asm volatile("" : "+v"(h.sc[f]));  // not ahead of the last step's MFMAs, where its read would be waited out
       const half2v sc = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(h.sc[f], 1.0f, false);
       s2[f][0] = half2v{sc[0], sc[0]};
       s2[f][1] = half2v{sc[1], sc[1]};
     }
     mma_under(o[0], h, s2, 0, o[1]);
     mma_under(o[1], h, s2, 1, o[0]);
-    if (t + 1 < nk) {
-      wait_loads(nk - 2 - t < 2 ? nk - 2 - t : 2);
+    constexpr std::integral_constant<int, (kStageNo + 1) % kSmallStages> kNext{};
+    if (const int behind = nk - 2 - t; behind >= 3) {
+      wait_loads(kS2);
       __syncthreads();
-      if (t + kSmallStages < nk) load_step(t + kSmallStages, stage);
-      read_raw(next, std::integral_constant<int, (kStageNo + 1) % kSmallStages>{});
+      load_step(t + kSmallStages, stage);
+      read_raw(next, kNext);
+    } else if (behind >= 0) {
+      if (behind == 2) wait_loads(kS2);
+      else if (behind == 1) wait_loads(kS1);
+      else wait_loads(kS0);
+      __syncthreads();
+      read_raw(next, kNext);
     }
     mma_under(o[0], h, s2, 2, o[1]);
     mma_under(o[1], h, s2, 3, o[0]);
   };
-  constexpr std::integral_constant<int, 0> kS0{};
-  constexpr std::integral_constant<int, 1> kS1{};
-  constexpr std::integral_constant<int, 2> kS2{};
-  constexpr std::integral_constant<int, 3> kS3{};
   load_step(0, kS0);
   if (1 < nk) load_step(1, kS1);
   if (2 < nk) load_step(2, kS2);
   if (3 < nk) load_step(3, kS3);
-  wait_loads(nk - 1);
+  if (nk > 3) wait_loads(kS3);
+  else if (nk == 3) wait_loads(kS2);
+  else if (nk == 2) wait_loads(kS1);
+  else wait_loads(kS0);
   __syncthreads();
   Raw h0, h1;
   read_raw(h0, kS0);
@@ -1022,19 +1080,19 @@ __global__ __launch_bounds__(kSmallThreads, WHOLE ? 1 : 2) void gemm_w4a4_small_
     if (t + 2 < nk) step(t + 2, kS2, h0, h1);
   }
   if constexpr (WHOLE) {
-    sum[0][0] = all;  // end_part has left the ring and the exchange behind a barrier
+    acc[0][0] = all;  // end_part has left the ring and the exchange behind a barrier
   } else {
     mma_last();
     __syncthreads();  // every wave has left the ring, which the exchange and then the patches of the epilogue take
     exchange_quarters(reinterpret_cast<float*>(smem));
   }
-  if (!WHOLE && parts > 1) {
+  if (FB == 2 && !WHOLE && parts > 1) {
     // Part of a tile: the workgroup that arrives last adds the parts up in the order of their K ranges, so the sum does
     // not depend on who that is; the others leave theirs in a record.  Same protocol as in the persistent kernel:
     // device-scope stores, every wave waits for its own, then the barrier, then thread 0 counts the arrival.
-    int* flag = reinterpret_cast<int*>(smem + kSmallFlag);
+    int* flag = reinterpret_cast<int*>(smem + S::kExchange);
     float* tile_records = records + (size_t)tile * parts * 4096 + wave * 1024 + lane * 4;
-    float16v& own = sum[0][0];
+    float16v& own = acc[0][0];
     if (tid == 0) *flag = __hip_atomic_load(arrivals + tile, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == parts - 1;
     __syncthreads();
     bool last = *flag != 0;
@@ -1081,8 +1139,17 @@ __global__ __launch_bounds__(kSmallThreads, WHOLE ? 1 : 2) void gemm_w4a4_small_
     own = all;
   }
   const float alpha = alpha_ptr ? alpha_ptr[0] : (amax_a[0] * amax_b[0]) * (inv_denom_a * inv_denom_b);
-  gemm_epilogue<1, 1>(sum, alpha, smem, wave, lane, row0 + 32 * (wave & 1), col0 + 32 * (wave >> 1), M, N, D, ldd, bias, act, epi,
-                      (uint32_t)blockIdx.x * 4 + wave);
+  // one fragment of A by kKeepB or the rest of B
+  auto write_out = [&](auto fragments, uint8_t* patches) __attribute__((always_inline)) {
+    constexpr int n = decltype(fragments)::value;
+    float16v kept[n][1];
+#pragma unroll
+    for (int g = 0; g < n; ++g) kept[g][0] = acc[g][0];
+    gemm_epilogue<1, n>(kept, alpha, patches, wave, lane, row0 + (odd ? 32 : 0), col0 + (upper ? 32 * kKeepB : 0), M, N, D, ldd, bias, act, epi,
+                        (uint32_t)blockIdx.x * 4 + wave);
+  };
+  if (FB == 3 && !upper) write_out(std::integral_constant<int, kKeepB>{}, smem);
+  else write_out(kS1, FB == 3 ? smem + 32768 : smem);  // patches of another pitch
 }
 
 // ============================================================================ tile kernel, hand-scheduled loop
@@ -1590,19 +1657,21 @@ int dispatch_gemm(const uint8_t* A_values, const uint8_t* A_scales, const uint8_
     const SmallGemmPlan plan = plan_small_gemm(M, N, Kp, groups.n, cus);
     GemmGroups gr = groups;
     gr.tiles_n_each = plan.tiles_n_each;
-#define LL_SMALL_LAUNCH(WHOLE, wgs, lds, records, arrivals)                                                                    \
-  hipLaunchKernelGGL(gemm_w4a4_small_kernel<WHOLE>, dim3((unsigned)(((wgs) + 7) / 8 * 8)), dim3(kSmallThreads), lds, s, A_values, A_scales, \
-                     B_values, B_scales, alpha, amax_a, amax_b, 1.0f / denom_a, 1.0f / denom_b, (int)M, (int)N, (int)Mp, (int)Np, (int)Kp, \
-                     static_cast<uint16_t*>(D), ldd, plan.tiles_m, plan.tiles_n_each * gr.n, epi, gr, plan.parts, records, arrivals)
+#define LL_SMALL_LAUNCH(WHOLE, FB, wgs, lds, records, arrivals)                                                            \
+  do {                                                                                                                       \
+    static std::atomic<uint64_t> lds_allowed{0};                                                                              \
+    if (int rc = allow_dynamic_lds(reinterpret_cast<const void*>(&gemm_w4a4_small_kernel<WHOLE, FB>), lds, lds_allowed, "ll_nvfp4_gemm_tnt")) return rc; \
+    hipLaunchKernelGGL((gemm_w4a4_small_kernel<WHOLE, FB>), dim3((unsigned)(((wgs) + 7) / 8 * 8)), dim3(kSmallThreads), lds, s, A_values, A_scales, \
+                       B_values, B_scales, alpha, amax_a, amax_b, 1.0f / denom_a, 1.0f / denom_b, (int)M, (int)N, (int)Mp, (int)Np, (int)Kp, \
+                       static_cast<uint16_t*>(D), ldd, plan.tiles_m, plan.tiles_n_each * gr.n, epi, gr, plan.parts, records, arrivals);   \
+  } while (0)
     StreamScratch w;
-    if (plan.parts > 1 && !small_product_scratch(dev, s, cus, w)) {
-      static std::atomic<uint64_t> lds_allowed{0};
-      if (int rc = allow_dynamic_lds(reinterpret_cast<const void*>(&gemm_w4a4_small_kernel<true>), kSmallWholeSmem, lds_allowed, "ll_nvfp4_gemm_tnt")) return rc;
-      LL_SMALL_LAUNCH(true, plan.tiles, kSmallWholeSmem, nullptr, nullptr);
+    if (plan.fb == 3) {
+      LL_SMALL_LAUNCH(false, 3, plan.tiles, SmallTile<3>::kRing, nullptr, nullptr);
+    } else if (plan.parts > 1 && !small_product_scratch(dev, s, cus, w)) {
+      LL_SMALL_LAUNCH(true, 2, plan.tiles, kSmallWholeSmem, nullptr, nullptr);
     } else {
-      static std::atomic<uint64_t> lds_allowed{0};
-      if (int rc = allow_dynamic_lds(reinterpret_cast<const void*>(&gemm_w4a4_small_kernel<false>), kSmallSmem, lds_allowed, "ll_nvfp4_gemm_tnt")) return rc;
-      LL_SMALL_LAUNCH(false, plan.tiles * plan.parts, kSmallSmem, reinterpret_cast<float*>(w.records), w.counters);
+      LL_SMALL_LAUNCH(false, 2, plan.tiles * plan.parts, SmallTile<2>::kRing, reinterpret_cast<float*>(w.records), w.counters);
     }
 #undef LL_SMALL_LAUNCH
     LL_CHECK_LAUNCH("gemm_w4a4_small_kernel");

@@ -746,6 +746,17 @@ def test_small_products_with_k_shared_between_waves_and_workgroups(gpu, M, N, K,
             _native.release_stream_memory()
 
 
+@pytest.mark.parametrize("M,N,K,groups", [
+    (700, 1100, 576, 1),      # the shortest K that the kernel takes: a third step of a quarter
+    (1320, 1544, 832, 1),     # three tiles on some compute units
+    (1030, 1000, 1088, 1),    # 64 x 96 tiles: the last one reaches behind the padded matrix, tiles across 128-row scale blocks
+    (1100, 930, 1024, 1),     # the same where it ends inside, N no multiple of 8
+    (500, 700, 1344, 3),      # three products, a ragged last step
+])
+def test_small_products_of_more_tiles_than_compute_units(gpu, M, N, K, groups):
+    test_small_products_with_k_shared_between_waves_and_workgroups(gpu, M, N, K, groups)
+
+
 def test_recorded_small_products_replayed_at_the_same_time(gpu):
     """Products whose K range several workgroups share, recorded twice on one stream that has run them before and replayed
     on two streams beside the same work on the recording stream: every result has the bits of the launch by itself."""

@@ -125,6 +125,13 @@ int ll_amax_epoch_advance(uint32_t* epoch_offset, uint32_t step, uint64_t* parts
 int ll_nvfp4_quantize_once(const void* x, int64_t M, int64_t K, int64_t ldx, int rule, uint8_t* values, uint8_t* scales, float* amax,
                            const ll_amax_sink* amax_sink, int64_t spin_limit, void* stream);
 
+/* The same for one tensor (x1 NULL) or two of one shape, leading dimension and rule (the K and V of a chunk), of up to 512
+ * tiles of 128 x 64 (or two per compute unit) each. */
+int ll_nvfp4_quantize_one_pass(const void* x0, const void* x1, int64_t M, int64_t K, int64_t ldx, int rule,
+                               uint8_t* values0, uint8_t* values1, uint8_t* scales0, uint8_t* scales1,
+                               float* amax0, float* amax1, const ll_amax_sink* amax_sink, int64_t spin_limit,
+                               void* stream);
+
 /* ll_nvfp4_quantize whose tensor amax comes from an amax sink that the producer of x has filled with the
  * same epoch; amax (f32[1]) is written.  The bytes equal those of ll_nvfp4_quantize with amax_given == 0. */
 int ll_nvfp4_quantize_from_sink(const void* x, int64_t M, int64_t K, int64_t ldx, int rule,

@@ -82,6 +82,8 @@ _SIGNATURES = {
                                      c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p]),
     "ll_qk_norm_rope_pair_amax": (c_int, [c_void_p, c_void_p, c_int64, c_int, c_void_p, c_void_p, c_float, c_void_p,
                                      c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
+    "ll_nvfp4_quantize_one_pass": (c_int, [c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int, c_void_p, c_void_p, c_void_p,
+                                           c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_void_p]),
     "ll_nvfp4_quantize_once": (c_int, [c_void_p, c_int64, c_int64, c_int64, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_int64,
                                        c_void_p]),
     "ll_patch_embed": (c_int, [c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_int, c_void_p,

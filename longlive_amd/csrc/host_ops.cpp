@@ -159,13 +159,15 @@ Epochs epochs_of_stream(int dev, void* stream) {
 
 // The amax of x and its quantization: one launch for a small tensor, two otherwise and while the stream is being captured.
 constexpr int64_t kSpinLimit = 64;  // looks of one to two microseconds at the other workgroups' maxima
+inline bool one_pass_tiles(int64_t M, int64_t K) { return K % 64 == 0 && ((M + 127) / 128) * (K / 64) <= 512; }
 int quantize_operand(const void* x, int64_t M, int64_t K, int64_t ldx, int rule, uint8_t* values, uint8_t* scales, float* amax,
                      float* workspace, int dev, void* stream) {
-  if (K % 64 == 0 && ((M + 127) / 128) * (K / 64) <= 256) {
+  if (one_pass_tiles(M, K)) {
     Epochs e = epochs_of_stream(dev, stream);
     if (e.parts) {
       const ll_amax_sink sink = e.take();
-      const int code = ll_nvfp4_quantize_once(x, M, K, ldx, rule, values, scales, amax, &sink, kSpinLimit, stream);
+      const int code = ll_nvfp4_quantize_one_pass(x, nullptr, M, K, ldx, rule, values, nullptr, scales, nullptr, amax, nullptr, &sink,
+                                                  kSpinLimit, stream);
       if (code != LL_ENOSUP) return code;
     }
   }
@@ -726,9 +728,20 @@ PyObject* py_cache_write(PyObject*, PyObject* const* args, Py_ssize_t n) {
     code = ll_nvfp4_quantize_pair_from_sinks(kx, vx, M, 128, 128, rule, out[0][0], out[1][0], out[0][1], out[1][1], amax[0],
                                              amax[1], &sinks[0], &sinks[1], stream);
   } else {
-    const Tensor ws = empty({2 * (int64_t)LL_AMAX_PARTS}, at::kFloat, dev);
-    code = ll_nvfp4_quantize_pair(kx, vx, M, 128, 128, rule, out[0][0], out[1][0], out[0][1], out[1][1], amax[0], amax[1],
-                                  ws.data_ptr<float>(), stream);
+    code = LL_ENOSUP;
+    if (one_pass_tiles(M, 128)) {
+      Epochs e = epochs_of_stream(dev, stream);
+      if (e.parts) {
+        const ll_amax_sink sink = e.take();
+        code = ll_nvfp4_quantize_one_pass(kx, vx, M, 128, 128, rule, out[0][0], out[1][0], out[0][1], out[1][1], amax[0], amax[1], &sink,
+                                          kSpinLimit, stream);
+      }
+    }
+    if (code == LL_ENOSUP) {
+      const Tensor ws = empty({2 * (int64_t)LL_AMAX_PARTS}, at::kFloat, dev);
+      code = ll_nvfp4_quantize_pair(kx, vx, M, 128, 128, rule, out[0][0], out[1][0], out[0][1], out[1][1], amax[0], amax[1],
+                                    ws.data_ptr<float>(), stream);
+    }
   }
   if (failed(code, "cache write")) return nullptr;
   Py_RETURN_TRUE;

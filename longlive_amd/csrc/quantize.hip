@@ -254,44 +254,84 @@ __global__ __launch_bounds__(kThreads) void quantize_kernel(QuantJobs jobs, int6
 }
 
 // ----------------------------------------------------------------------------- small tensors: both passes in one launch
-// One workgroup = one 128 x 64 tile, one block of 16 per thread, kept in registers between its two halves: the maximum of
-// the tile, exchanged with the other workgroups through the sink (amax_exchange.h), and the quantization.  What a small
-// tensor costs is launches and one trip to memory each: 48 x 256 7.8 instead of 9.6 us a call, 512 x 3072 8.2 instead of 9.3.
-template <int RULE>
-__global__ __launch_bounds__(512) void quantize_once_kernel(const uint16_t* __restrict__ x, uint8_t* __restrict__ values,
-                                                            uint8_t* __restrict__ scales, float* __restrict__ amax_out, int64_t M, int64_t K,
-                                                            int64_t ldx, AmaxSink sink, uint32_t spin_limit, int recompute) {
+// One workgroup = T neighbouring tiles of 128 x 64, a block of 16 of each per thread, kept packed in registers between the two
+// halves of the kernel: the maximum of the tiles, exchanged with the tensor's other workgroups through the sink
+// (amax_exchange.h), and the quantization.  Two tensors of one shape (the K and V of a chunk) take half of the workgroups and
+// half of the slots each.  Bound by the latency of a launch, of a trip to memory and of the exchange: what a small tensor costs
+// is launches and one trip to memory each, and not its bytes (figures: quantize_one_pass).  128 registers at most, so that
+// two workgroups are resident per compute unit.
+struct OnceJob {
+  const uint16_t* x;
+  uint8_t* values;
+  uint8_t* scales;
+  float* amax;
+};
+struct OnceJobs {
+  OnceJob j[2];
+  int n;
+};
+constexpr uint32_t kOnceSlots = kAmaxParts / 2;  // of a tensor
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+template <int RULE, int T>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void quantize_once_kernel(OnceJobs jobs, int64_t M, int64_t K, int64_t ldx, uint32_t tiles, AmaxSink sink,
+                                                            uint32_t spin_limit, int recompute) {
   __shared__ AmaxExchangeSmem s_exchange;
   __shared__ ScaleEntry s_tab[128];
-  __shared__ uint32_t s_scales[128];  // the tile's 128 x 4 scale bytes in blocked order
-  const uint32_t tiles_x = (uint32_t)(K >> 6), tile = blockIdx.x;
+  __shared__ uint32_t s_scales[2][128];  // a tile's 128 x 4 scale bytes in blocked order
+  const uint32_t G = jobs.n == 2 ? gridDim.x >> 1 : gridDim.x;
+  const bool other = blockIdx.x >= G;
+  const uint32_t wg = other ? blockIdx.x - G : blockIdx.x;
+  const OnceJob job = other ? jobs.j[1] : jobs.j[0];
+  if (other) sink.parts += kOnceSlots;
+  const uint32_t tiles_x = (uint32_t)(K >> 6);
   const int row_in_tile = threadIdx.x >> 2, cb = threadIdx.x & 3;
-  auto load = [&](uint32_t t, float (&X)[16]) __attribute__((always_inline)) {
-    const uint32_t ty = t / tiles_x, tx = t - ty * tiles_x;
-    const int64_t row = (int64_t)ty * 128 + row_in_tile;
-    uint4 lo = make_uint4(0u, 0u, 0u, 0u), hi = lo;
-    if (row < M) {
-      const uint4* p = reinterpret_cast<const uint4*>(x + row * ldx + (int64_t)tx * 64 + cb * 16);
+  struct Place {
+    uint32_t tile, ty, tx;
+  };
+  auto first_of = [&](uint32_t g) { return Place{g * T, g * T / tiles_x, g * T % tiles_x}; };  // of workgroup g
+  auto next_of = [&](const Place& p) {
+    const bool wrap = p.tx + 1 == tiles_x;
+    return Place{p.tile + 1, p.ty + (wrap ? 1 : 0), wrap ? 0 : p.tx + 1};
+  };
+  // The thread's block of a tile as it lies in memory; zeros behind the last row and the last tile.
+  auto load = [&](const Place& at, u32x4& lo, u32x4& hi) __attribute__((always_inline)) {
+    const int64_t row = (int64_t)at.ty * 128 + row_in_tile;
+    lo = hi = u32x4{0u, 0u, 0u, 0u};
+    if (row < M && at.tile < tiles) {
+      const u32x4* p = reinterpret_cast<const u32x4*>(job.x + row * ldx + (int64_t)at.tx * 64 + cb * 16);
       lo = p[0];
       hi = p[1];
     }
-    const uint32_t w[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-    float m = 0.0f;
+  };
+  auto abs_max = [&](const u32x4& lo, const u32x4& hi, float m) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      X[2 * i] = __uint_as_float(w[i] << 16);
-      X[2 * i + 1] = __uint_as_float(w[i] & 0xFFFF0000u);
-      m = fmaxf(m, fmaxf(fabsf(X[2 * i]), fabsf(X[2 * i + 1])));
+      const uint32_t w = i < 4 ? lo[i] : hi[i - 4];
+      m = fmaxf(m, fmaxf(fabsf(__uint_as_float(w << 16)), fabsf(__uint_as_float(w & 0xFFFF0000u))));
     }
     return m;
   };
-  float X[16];
-  const float part = load(tile, X);
-  const float amax = exchange_amax(sink, gridDim.x, tile, part, spin_limit, recompute != 0, s_exchange, [&](uint32_t s) {
-    float unused[16];
-    return load(s, unused);
+  static_assert(T == 1 || T == 2, "one or two tiles");
+  const Place first = first_of(wg), second = next_of(first);
+  u32x4 lo[T], hi[T];
+  float part = 0.0f;
+  load(first, lo[0], hi[0]);
+  if constexpr (T == 2) load(second, lo[1], hi[1]);
+#pragma unroll
+  for (int t = 0; t < T; ++t) part = abs_max(lo[t], hi[t], part);
+  const float amax = exchange_amax(sink, G, wg, part, spin_limit, recompute != 0, s_exchange, [&](uint32_t s) {
+    float m = 0.0f;
+    Place at = first_of(s);
+#pragma unroll 1
+    for (int t = 0; t < T; ++t, at = next_of(at)) {
+      u32x4 l, h;
+      load(at, l, h);
+      m = abs_max(l, h, m);
+    }
+    return m;
   });
-  if (tile == 0 && threadIdx.x == 0) amax_out[0] = amax;
+  if (wg == 0 && threadIdx.x == 0) job.amax[0] = amax;
 
   constexpr bool kStaticRule = (RULE == LL_RULE_STATIC_6 || RULE == LL_RULE_STATIC_4);
   constexpr float kE2 = (RULE == LL_RULE_STATIC_4) ? 4.0f : 6.0f;
@@ -302,13 +342,26 @@ __global__ __launch_bounds__(512) void quantize_once_kernel(const uint16_t* __re
   const float dec = 1.0f / enc;
   if (fast) fill_scale_table<RULE>(s_tab, amax, dec);
   __syncthreads();
-  uint32_t lo, hi, sb;
-  if (!fast || !quantize_block_fast<RULE>(X, enc, s_tab, approx_ok, __builtin_inff(), lo, hi, sb)) quantize_block<RULE>(X, amax, enc, dec, lo, hi, sb);
-  const uint32_t ty = tile / tiles_x, tx = tile - ty * tiles_x;
-  *reinterpret_cast<uint2*>(values + ((int64_t)ty * 128 + row_in_tile) * (K >> 1) + (int64_t)tx * 32 + cb * 8) = make_uint2(lo, hi);
-  reinterpret_cast<uint8_t*>(s_scales)[(row_in_tile & 31) * 16 + (row_in_tile >> 5) * 4 + cb] = (uint8_t)sb;
-  __syncthreads();
-  if (threadIdx.x < 128) reinterpret_cast<uint32_t*>(scales)[(int64_t)tile * 128 + threadIdx.x] = s_scales[threadIdx.x];
+#pragma unroll 1
+  for (int t = 0; t < T; ++t) {
+    const Place at = t == 0 ? first : second;
+    if (T > 1 && at.tile >= tiles) break;
+    const u32x4 l = t == 0 ? lo[0] : lo[T - 1], h = t == 0 ? hi[0] : hi[T - 1];
+    float X[16];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const uint32_t w = i < 4 ? l[i] : h[i - 4];
+      X[2 * i] = __uint_as_float(w << 16);
+      X[2 * i + 1] = __uint_as_float(w & 0xFFFF0000u);
+    }
+    uint32_t out_lo, out_hi, sb;
+    if (!fast || !quantize_block_fast<RULE>(X, enc, s_tab, approx_ok, __builtin_inff(), out_lo, out_hi, sb))
+      quantize_block<RULE>(X, amax, enc, dec, out_lo, out_hi, sb);
+    *reinterpret_cast<uint2*>(job.values + ((int64_t)at.ty * 128 + row_in_tile) * (K >> 1) + (int64_t)at.tx * 32 + cb * 8) = make_uint2(out_lo, out_hi);
+    reinterpret_cast<uint8_t*>(s_scales[t & 1])[(row_in_tile & 31) * 16 + (row_in_tile >> 5) * 4 + cb] = (uint8_t)sb;
+    __syncthreads();  // the buffer is written again two tiles, and a barrier, later
+    if (threadIdx.x < 128) reinterpret_cast<uint32_t*>(job.scales)[(int64_t)at.tile * 128 + threadIdx.x] = s_scales[t & 1][threadIdx.x];
+  }
 }
 
 }  // namespace ll
@@ -442,42 +495,55 @@ extern "C" int ll_nvfp4_quantize(const void* x, int64_t M, int64_t K, int64_t ld
   return quantize_impl(&r, 1, M, K, ldx, rule, amax_given, stream);
 }
 
-// The line: one workgroup per compute unit.  The exchange grows with the workgroups (each reads all slots): 192 tiles 8.2 us
-// against 9.3 in two launches, 224 8.4 against 9.2, but 320 9.5 against 9.3, 384 9.9 against 9.3, 504 11.2 against 9.6.
-static constexpr int64_t kOnceTiles = 256;
-extern "C" int ll_nvfp4_quantize_once(const void* x, int64_t M, int64_t K, int64_t ldx, int rule, uint8_t* values, uint8_t* scales, float* amax,
-                                      const ll_amax_sink* amax_sink, int64_t spin_limit, void* stream) {
+// The line: one workgroup per compute unit and tensor.  The exchange grows with a tensor's workgroups, each of which reads all
+// their slots, and a workgroup of four tiles has a chain of its own.  us, mse, here / in two launches:
+//   one tensor    4 tiles 5.3 / 8.2, 192 6.2 / 9.1, two tiles per workgroup: 320 8.9 / 9.6, 384 8.4 / 9.9; beyond the line, with two
+//                 workgroups per unit: 576 11.5 / 10.8, 1008 12.5 / 12.5; with four tiles per workgroup: 576 12.7 / 10.7, 1008 13.7 / 12.4
+//   two tensors   2 x 92 tiles 6.3 / 9.3, 2 x 166 8.3 / 10.0, 2 x 220 8.4 / 10.3, 2 x 496 (512 workgroups) 10.9 / 12.8
+static constexpr int64_t kOnceTiles = 256;      // ll_nvfp4_quantize_once
+static constexpr int64_t kOnePassTiles = 512;   // of a tensor, ll_nvfp4_quantize_one_pass
+
+static int quantize_one_pass(const ll::OnceJobs& jobs, int64_t M, int64_t K, int64_t ldx, int rule, const ll_amax_sink* amax_sink,
+                             int64_t spin_limit, int64_t most_tiles, void* stream, const char* what) {
   using namespace ll;
-  LL_REQUIRE(x && values && scales && amax, "ll_nvfp4_quantize_once: null pointer");
-  LL_REQUIRE(M > 0 && K > 0 && ldx >= K, "ll_nvfp4_quantize_once: bad shape M=%lld K=%lld ldx=%lld", (long long)M, (long long)K, (long long)ldx);
-  LL_REQUIRE(rule >= 0 && rule <= 4, "ll_nvfp4_quantize_once: unknown scale rule %d", rule);
-  LL_REQUIRE(amax_sink && amax_sink->parts && sink_is_valid(amax_sink),
-             "ll_nvfp4_quantize_once: an amax sink (8-byte aligned buffer, non-zero epoch) is required");
-  LL_REQUIRE((reinterpret_cast<uintptr_t>(values) & 7) == 0 && (reinterpret_cast<uintptr_t>(scales) & 3) == 0,
-             "ll_nvfp4_quantize_once: outputs must be 8-byte (values) / 4-byte (scales) aligned");
+  LL_REQUIRE(M > 0 && K > 0 && ldx >= K, "%s: bad shape M=%lld K=%lld ldx=%lld", what, (long long)M, (long long)K, (long long)ldx);
+  LL_REQUIRE(rule >= 0 && rule <= 4, "%s: unknown scale rule %d", what, rule);
+  LL_REQUIRE(amax_sink && amax_sink->parts && sink_is_valid(amax_sink), "%s: an amax sink (8-byte aligned buffer, non-zero epoch) is required", what);
   const int64_t groups_m = (M + 127) / 128, groups_k = K / 64;
-  if (K % 64 != 0 || ldx % 8 != 0 || (reinterpret_cast<uintptr_t>(x) & 15) != 0 || groups_m > kOnceTiles || groups_k > kOnceTiles ||
-      groups_m * groups_k > kOnceTiles) {
-    set_error("ll_nvfp4_quantize_once: takes up to %lld tiles of 128 x 64 in whole 16-byte pieces", (long long)kOnceTiles);
+  bool whole = K % 64 == 0 && ldx % 8 == 0 && groups_m <= most_tiles && groups_k <= most_tiles && groups_m * groups_k <= most_tiles;
+  for (int i = 0; i < jobs.n; ++i) {
+    const OnceJob& j = jobs.j[i];
+    LL_REQUIRE(j.x && j.values && j.scales && j.amax, "%s: null pointer", what);
+    LL_REQUIRE((reinterpret_cast<uintptr_t>(j.values) & 7) == 0 && (reinterpret_cast<uintptr_t>(j.scales) & 3) == 0,
+               "%s: outputs must be 8-byte (values) / 4-byte (scales) aligned", what);
+    whole = whole && (reinterpret_cast<uintptr_t>(j.x) & 15) == 0;
+  }
+  if (!whole) {
+    set_error("%s: takes up to %lld tiles of 128 x 64 in whole 16-byte pieces", what, (long long)most_tiles);
     return LL_ENOSUP;
   }
   const int64_t tiles = groups_m * groups_k;
   int dev = 0, cus = 0;
   if (hipGetDevice(&dev) != hipSuccess) {
-    set_error("ll_nvfp4_quantize_once: hipGetDevice failed");
+    set_error("%s: hipGetDevice failed", what);
     return LL_ELAUNCH;
   }
-  if (int rc = compute_units_of(dev, cus, "ll_nvfp4_quantize_once")) return rc;
-  if (tiles > cus) {
-    set_error("ll_nvfp4_quantize_once: %lld tiles are more than the device holds at once", (long long)tiles);
+  if (int rc = compute_units_of(dev, cus, what)) return rc;
+  const int per_wg = tiles * jobs.n <= cus ? 1 : 2;
+  const int64_t wgs = (tiles + per_wg - 1) / per_wg;
+  if (wgs > cus || wgs > (int64_t)kOnceSlots) {
+    set_error("%s: %lld tiles are more than the device holds at once", what, (long long)(tiles * jobs.n));
     return LL_ENOSUP;
   }
   const AmaxSink sink = make_sink(amax_sink);
   const uint32_t spin = spin_limit < 0 ? 0u : (spin_limit > 0x7FFFFFFF ? 0x7FFFFFFFu : (uint32_t)spin_limit);
   hipStream_t s = static_cast<hipStream_t>(stream);
-#define LL_LAUNCH_ONCE(R)                                                                                                       \
-  hipLaunchKernelGGL(quantize_once_kernel<R>, dim3((unsigned)tiles), dim3(512), 0, s, static_cast<const uint16_t*>(x), values, scales, amax, M, \
-                     K, ldx, sink, spin, spin_limit < 0 ? 1 : 0)
+  const dim3 grid((unsigned)(wgs * jobs.n));
+#define LL_LAUNCH_ONCE(R)                                                                                                          \
+  do {                                                                                                                             \
+    if (per_wg == 1) hipLaunchKernelGGL((quantize_once_kernel<R, 1>), grid, dim3(512), 0, s, jobs, M, K, ldx, (uint32_t)tiles, sink, spin, spin_limit < 0 ? 1 : 0); \
+    else hipLaunchKernelGGL((quantize_once_kernel<R, 2>), grid, dim3(512), 0, s, jobs, M, K, ldx, (uint32_t)tiles, sink, spin, spin_limit < 0 ? 1 : 0); \
+  } while (0)
   switch (rule) {
     case LL_RULE_STATIC_6: LL_LAUNCH_ONCE(LL_RULE_STATIC_6); break;
     case LL_RULE_STATIC_4: LL_LAUNCH_ONCE(LL_RULE_STATIC_4); break;
@@ -488,6 +554,21 @@ extern "C" int ll_nvfp4_quantize_once(const void* x, int64_t M, int64_t K, int64
 #undef LL_LAUNCH_ONCE
   LL_CHECK_LAUNCH("quantize_once_kernel");
   return LL_OK;
+}
+
+extern "C" int ll_nvfp4_quantize_once(const void* x, int64_t M, int64_t K, int64_t ldx, int rule, uint8_t* values, uint8_t* scales, float* amax,
+                                      const ll_amax_sink* amax_sink, int64_t spin_limit, void* stream) {
+  const ll::OnceJobs jobs{{{static_cast<const uint16_t*>(x), values, scales, amax}, {}}, 1};
+  return quantize_one_pass(jobs, M, K, ldx, rule, amax_sink, spin_limit, kOnceTiles, stream, "ll_nvfp4_quantize_once");
+}
+
+extern "C" int ll_nvfp4_quantize_one_pass(const void* x0, const void* x1, int64_t M, int64_t K, int64_t ldx, int rule, uint8_t* values0,
+                                          uint8_t* values1, uint8_t* scales0, uint8_t* scales1, float* amax0, float* amax1,
+                                          const ll_amax_sink* amax_sink, int64_t spin_limit, void* stream) {
+  using namespace ll;
+  LL_REQUIRE(!x1 || (values0 != values1 && scales0 != scales1 && amax0 != amax1), "ll_nvfp4_quantize_one_pass: the two tensors need outputs of their own");
+  const OnceJobs jobs{{{static_cast<const uint16_t*>(x0), values0, scales0, amax0}, {static_cast<const uint16_t*>(x1), values1, scales1, amax1}}, x1 ? 2 : 1};
+  return quantize_one_pass(jobs, M, K, ldx, rule, amax_sink, spin_limit, kOnePassTiles, stream, "ll_nvfp4_quantize_one_pass");
 }
 
 // One workgroup of kAmaxParts threads.  Every thread reads the word before anyone writes it, so all agree on

@@ -260,6 +260,37 @@ def test_small_tensors_in_one_launch_have_the_bytes_of_the_two_launches(gpu, rul
     assert lib.ll_nvfp4_quantize_once(x.data_ptr(), 128 * 257, 64, 64, *args[4:], ctypes.byref(sink), 64, stream) == -3   # refused on the host
 
 
+@pytest.mark.parametrize("rule", ["mse", "static_4", "abs_max"])
+@pytest.mark.parametrize("M,K,pad,tensors", [(1, 64, 0, 2), (1173, 2112, 8, 1), (16384, 256, 0, 1), (5888, 128, 0, 2), (16321, 128, 8, 2), (32768, 128, 0, 2)])
+def test_one_pass_has_the_bytes_of_the_two_launches(gpu, rule, M, K, pad, tensors):
+    """One or two tensors of up to 512 tiles, one or two tiles per workgroup: an odd number of them, as many as the rule takes,
+    ragged rows and rows with a stride; several calls on one sink with the maxima falling, with the wait's way out, and with
+    zeros and maxima outside the fast path.  The two tensors differ in scale, so that neither may see the other's maximum."""
+    lib, stream, code = _native.load(), torch.cuda.current_stream().cuda_stream, _native.RULE_IDS[rule]
+    g = torch.Generator(device=gpu).manual_seed(M + K)
+    Mp = -(-M // 128) * 128
+    parts = torch.zeros(1024, dtype=torch.int64, device=gpu)
+    ws = torch.empty(1024, dtype=torch.float32, device=gpu)
+
+    def buffers():
+        return [torch.full((n,), 7, dtype=t, device=gpu) for n, t in ((Mp * K // 2, torch.uint8), (Mp * K // 16, torch.uint8), (1, torch.float32))]
+
+    for i, (scale, spin) in enumerate([(1e3, 64), (1.0, 64), (0.01, -1), (0.0, 64), (1e35, 64), (1.0, 0)]):
+        xs = [(torch.randn((M, K + pad), generator=g, device=gpu) * scale * f).bfloat16()[:, :K] for f in (1.0, 0.3, 5.0)[i % 2:][:tensors]]
+        xs[0][0, -1] *= 30
+        got, want = [buffers() for _ in xs], [buffers() for _ in xs]
+        sink = _native.AmaxSinkStruct(parts.data_ptr(), i + 1, None)
+        two = [(x, o) for x, o in zip(xs, got)] if tensors == 2 else [(xs[0], got[0]), (None, [None] * 3)]
+        ptr = lambda t: t.data_ptr() if t is not None else None
+        args = [v for j in range(3) for v in (ptr(two[0][1][j]), ptr(two[1][1][j]))]
+        assert lib.ll_nvfp4_quantize_one_pass(xs[0].data_ptr(), ptr(two[1][0]), M, K, xs[0].stride(0), code, *args, ctypes.byref(sink), spin,
+                                              stream) == 0, lib.ll_last_error()
+        for x, (v, s, a) in zip(xs, want):
+            assert lib.ll_nvfp4_quantize(x.data_ptr(), M, K, x.stride(0), code, v.data_ptr(), s.data_ptr(), a.data_ptr(), 0, ws.data_ptr(), stream) == 0
+        assert all(torch.equal(p, q) for a, b in zip(got, want) for p, q in zip(a, b)), (i, scale, spin)
+    assert lib.ll_nvfp4_quantize_one_pass(xs[0].data_ptr(), None, 128 * 513, 64, 64, code, *args, ctypes.byref(sink), 64, stream) == -3   # refused on the host
+
+
 def test_small_quantization_recorded_into_a_graph(gpu):
     """While a stream is being captured the two launches are recorded: replays on a falling maximum equal the eager bytes."""
     cfg = QuantizationConfig(scale_rule="mse")

@@ -137,6 +137,9 @@ __global__ __launch_bounds__(kRowThreads) void rmsnorm_kernel(const uint16_t* __
 // above; optionally also k - mean(k over the head dimension) (utils/quant.py:797-798) as a second output,
 // mean and difference rounded to bf16 like the two eager operations.  One wave = one token row; a head is
 // held by 16 consecutive lanes.  blockIdx.y selects the tensor (q or k), so that both go in one launch.
+// Bound by the chain of a wave (loads, one reduction, some 25 instructions per element, one or two waves per SIMD up to
+// 1000 rows) and by memory above.  With weights and angles asked for where they are used, a head's sum through LDS and one
+// conversion per rounded value: 736 x 1536 5.6 us, now 4.9; 880 x 3072 9.6 / 8.2; 2640 x 3072 19.6 / 17.4.
 struct QkProblem {  // one tensor of the q / k pair
   const uint16_t* x;
   const uint16_t* w;
@@ -162,39 +165,54 @@ __global__ __launch_bounds__(kRowThreads) void qk_norm_rope_kernel(QkProblems pr
   if (row >= rows) return;
   const uint16_t* xr = x + row * (int64_t)C;
   const int nchunks = C >> 3;
+  const bool rotate = row < seq_len;
+  // The weights and the row's angles are requested up front: their latency runs under the reduction.  A lane's place in a
+  // head, and so its four rotation pairs, is the same in all of its groups.
+  const int pair0 = (lane & 15) * 4;
+  float4 cs = make_float4(1.0f, 1.0f, 1.0f, 1.0f), sn = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  if (rotate) {
+    cs = *reinterpret_cast<const float4*>(cosp + row * 64 + pair0);
+    sn = *reinterpret_cast<const float4*>(sinp + row * 64 + pair0);
+  }
+  const float cc[4] = {cs.x, cs.y, cs.z, cs.w}, ss[4] = {sn.x, sn.y, sn.z, sn.w};
   float v[NCH][8];
+  uint4 wraw[NCH];
   float sq = 0.0f;
 #pragma unroll
   for (int i = 0; i < NCH; ++i) {
     const int c = lane + i * 64;
     if (c < nchunks) {
       unpack8(*reinterpret_cast<const uint4*>(xr + c * 8), v[i]);
+      wraw[i] = *reinterpret_cast<const uint4*>(w + c * 8);
 #pragma unroll
       for (int j = 0; j < 8; ++j) sq += v[i][j] * v[i][j];
     }
   }
   const float ms = wave_sum_dpp(sq) / (float)C;
   const float r = 1.0f / sqrtf(ms + eps);
-  const bool rotate = row < seq_len;
   float out_max = 0.0f;
 #pragma unroll
   for (int i = 0; i < NCH; ++i) {
     const int c = lane + i * 64;  // uniform over each group of 16 threads: c < nchunks or not
     if (c < nchunks) {
       float w8[8], y[8], o8[8];
-      unpack8(*reinterpret_cast<const uint4*>(w + c * 8), w8);
+      unpack8(wraw[i], w8);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) y[j] = round_to_bf16(round_to_bf16(v[i][j] * r) * w8[j]);
+      for (int j = 0; j < 8; j += 2) {
+        y[j] = v[i][j] * r;
+        y[j + 1] = v[i][j + 1] * r;
+        round_to_bf16(y[j], y[j + 1]);
+        y[j] *= w8[j];
+        y[j + 1] *= w8[j + 1];
+        round_to_bf16(y[j], y[j + 1]);
+      }
       if (rotate) {
-        const int pair0 = (c & 15) * 4;  // first rotation pair of this chunk inside its head
-        const float4 cs = *reinterpret_cast<const float4*>(cosp + row * 64 + pair0);
-        const float4 sn = *reinterpret_cast<const float4*>(sinp + row * 64 + pair0);
-        const float cc[4] = {cs.x, cs.y, cs.z, cs.w}, ss[4] = {sn.x, sn.y, sn.z, sn.w};
 #pragma unroll
         for (int p = 0; p < 4; ++p) {
           const float a = y[2 * p], b = y[2 * p + 1];
-          o8[2 * p] = round_to_bf16(a * cc[p] - b * ss[p]);
-          o8[2 * p + 1] = round_to_bf16(a * ss[p] + b * cc[p]);
+          o8[2 * p] = a * cc[p] - b * ss[p];
+          o8[2 * p + 1] = a * ss[p] + b * cc[p];
+          round_to_bf16(o8[2 * p], o8[2 * p + 1]);
         }
       } else {
 #pragma unroll
@@ -207,9 +225,7 @@ __global__ __launch_bounds__(kRowThreads) void qk_norm_rope_kernel(QkProblems pr
         float part = 0.0f;
 #pragma unroll
         for (int j = 0; j < 8; ++j) part += o8[j];
-#pragma unroll
-        for (int m = 1; m < 16; m <<= 1) part += __shfl_xor(part, m, 64);
-        const float mean = round_to_bf16(part * (1.0f / 128.0f));
+        const float mean = round_to_bf16(sum_over_16_lanes(part) * (1.0f / 128.0f));
         float s8[8];
 #pragma unroll
         for (int j = 0; j < 8; ++j) s8[j] = o8[j] - mean;

@@ -19,11 +19,7 @@ namespace ll {
 
 // The sum over the 16 lanes that hold a head, in the order of qk_norm_rope_kernel.  torch's mean adds in another order: where a
 // mean lies at the edge between two bf16 values the two may round apart (none of 8 million values drawn from N(0, 1) did).
-__device__ __forceinline__ float head_sum(float v) {
-#pragma unroll
-  for (int m = 1; m < 16; m <<= 1) v += __shfl_xor(v, m, 64);
-  return v;
-}
+__device__ __forceinline__ float head_sum(float v) { return sum_over_16_lanes(v); }
 
 // v - mean(v) of a head, with the roundings of the two eager bf16 operations.
 __device__ __forceinline__ void smooth8(float (&v)[8]) {

@@ -89,6 +89,12 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
   const f32x2_hw v = {lo, hi};
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2_hw));
 }
+// Two at once: one conversion for both.
+__device__ __forceinline__ void round_to_bf16(float& a, float& b) {
+  const uint32_t w = pack_bf16x2(a, b);
+  a = __uint_as_float(w << 16);
+  b = __uint_as_float(w & 0xFFFF0000u);
+}
 __device__ __forceinline__ float round_to_bf16(float f) { return __uint_as_float(f32_to_bf16_bits(f) << 16); }
 
 // e4m3fn byte -> fp32 (exact). 0x7F / 0xFF decode to NaN.
@@ -173,6 +179,15 @@ __device__ __forceinline__ float wave_sum_dpp(float v) {
   LL_DPP_ADD(v, 0x142, 0xA, 0xF);  // row_bcast:15 into rows 1 and 3
   LL_DPP_ADD(v, 0x143, 0xC, 0xF);  // row_bcast:31 into rows 2 and 3
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
+}
+// Sum over 16 neighbouring lanes, in every one of them: over lanes 1, 2, 4 and 8 apart in turn.  (When the lanes of a quad agree, the
+// mirrored lane of the other quad stands for the one 4 apart, and likewise for 8.)
+__device__ __forceinline__ float sum_over_16_lanes(float v) {
+  LL_DPP_ADD(v, 0xB1, 0xF, 0xF);   // quad_perm [1, 0, 3, 2]
+  LL_DPP_ADD(v, 0x4E, 0xF, 0xF);   // quad_perm [2, 3, 0, 1]
+  LL_DPP_ADD(v, 0x141, 0xF, 0xF);  // row_half_mirror
+  LL_DPP_ADD(v, 0x140, 0xF, 0xF);  // row_mirror
+  return v;
 }
 #undef LL_DPP_ADD
 

@@ -33,7 +33,8 @@ constexpr int kMaxRowLength = 64 * kMaxChunks * 8;
 
 // adaLN modulation of one row, utils/adaln_triton.py:36-86: LayerNorm without affine in fp32, rounded to bf16,
 // times (1 + scale) rounded, plus shift rounded.  `packed[i]` receives the 8 results of group lane + 64 i; the
-// return value is the lane's share of the row's absolute maximum.
+// return value is the lane's share of the row's absolute maximum.  Two values share a rounding's conversion: adaln_kernel takes
+// 9.6 us for 2640 x 3072, with one each 10.2.
 template <int NCH>
 __device__ __forceinline__ float adaln_row(const uint16_t* __restrict__ xr, const uint16_t* __restrict__ scr,
                                            const uint16_t* __restrict__ shr, int C, float eps, int add_one, int lane,
@@ -79,11 +80,19 @@ __device__ __forceinline__ float adaln_row(const uint16_t* __restrict__ xr, cons
       unpack8(sraw[i], s8);
       unpack8(hraw[i], h8);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const float xn = round_to_bf16(v[i][j] * rstd);
-        const float s = add_one ? round_to_bf16(s8[j] + 1.0f) : s8[j];
-        const float prod = round_to_bf16(xn * s);
-        y[j] = prod + h8[j];
+      for (int j = 0; j < 8; j += 2) {
+        float x0 = v[i][j] * rstd, x1 = v[i][j + 1] * rstd, s0 = s8[j], s1 = s8[j + 1];
+        round_to_bf16(x0, x1);
+        if (add_one) {
+          s0 += 1.0f;
+          s1 += 1.0f;
+          round_to_bf16(s0, s1);
+        }
+        x0 *= s0;
+        x1 *= s1;
+        round_to_bf16(x0, x1);
+        y[j] = x0 + h8[j];
+        y[j + 1] = x1 + h8[j + 1];
       }
       packed[i] = pack8(y);
       out_max = abs_max_bf16x8(packed[i], out_max);

@@ -256,6 +256,35 @@ __device__ __forceinline__ uint32_t group_number(uint32_t G) {
   return G % 8 == 0 ? (b & 7) * (G / 8) + (b >> 3) : b;
 }
 
+// The wave's results O^T * inv_l (register r of o[d]: column 32 d + 8 (r / 4) + 4 lh + r % 4 of query l32), as bf16, to the first
+// `queries` of its 32 rows of 32 N columns at dst (rows H heads apart), through an LDS patch of the wave's own: whole rows per
+// store.  Straight from the registers a store reaches 16 bytes of each of 32 rows: 7040 queries x 24 heads over 512 keys 71.5 us, so
+// 63.1; 3520 x 24 46.7 / 41.2; 1760 x 12 16.3 / 15.1.  out_max: raised to the largest magnitude.
+template <int N>
+__device__ __forceinline__ void write_rows(const float16v (&o)[N], float inv_l, uint8_t* patch, int lane, uint16_t* dst, int H, int queries,
+                                           float& out_max) {
+  constexpr int kPitch = 64 * N + 16, kLanes = 4 * N, kRows = 64 / kLanes;  // lanes per row of 16 bytes each, rows per store
+  const int l32 = lane & 31, lh = lane >> 5;
+#pragma unroll
+  for (int d = 0; d < N; ++d)
+#pragma unroll
+    for (int rg = 0; rg < 4; ++rg)
+      *reinterpret_cast<uint2*>(patch + l32 * kPitch + (32 * d + 8 * rg + 4 * lh) * 2) =
+          make_uint2(pack_bf16(o[d][4 * rg] * inv_l, o[d][4 * rg + 1] * inv_l), pack_bf16(o[d][4 * rg + 2] * inv_l, o[d][4 * rg + 3] * inv_l));
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  const int at = (lane % kLanes) * 16;
+#pragma unroll
+  for (int it = 0; it < 32 / kRows; ++it) {
+    const int row = it * kRows + lane / kLanes;
+    const uint4 v = *reinterpret_cast<const uint4*>(patch + row * kPitch + at);
+    if (row < queries) {
+      *reinterpret_cast<uint4*>(reinterpret_cast<uint8_t*>(dst + (int64_t)row * H * kHeadDim) + at) = v;
+      out_max = abs_max_bf16x8(v, out_max);
+    }
+  }
+}
+
 template <bool WIDE>
 __global__ __launch_bounds__(kAttnThreads) void kv_attention_kernel(AttnParams p) {
   constexpr int kQueries = WIDE ? 2 * kWgQueries : kWgQueries;  // queries per workgroup
@@ -331,13 +360,26 @@ __global__ __launch_bounds__(kAttnThreads) void kv_attention_kernel(AttnParams p
     const int64_t first = (int64_t)qtile * kQueries;
     wave_idle = __builtin_amdgcn_readfirstlane((int)(c.Lq - first <= 128 && first + qq * kWaveQueries >= c.Lq)) != 0;
   }
-  {
+  if constexpr (WIDE) {
     const auto& c = reread_params();
     int64_t query = (int64_t)qtile * kQueries + qq * kWaveQueries + l32;
     if (query >= c.Lq) query = c.Lq - 1;
     const uint16_t* src = c.q + (query * p.H + head) * kHeadDim + 8 * lh;
 #pragma unroll
     for (int ks = 0; ks < 8; ++ks) qf[ks] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(src + 16 * ks));
+  } else {
+    // Four whole rows per load, into a patch of the stage that the first iteration leaves alone; the fragments are read from
+    // there behind the loads of the first tile.  Straight into the fragments a load reaches 32 bytes of each of 32 rows: 1760
+    // queries x 12 heads over 512 keys 15.1 us, so 13.9.  (256-query tiles: 2640 x 24 over 512 27.8 and 28.4, 3520 x 24 41.1 and 40.5.)
+    const auto& c = reread_params();
+    const int64_t first_query = (int64_t)qtile * kQueries + qq * kWaveQueries;
+    uint8_t* patch = smem + ((seg_begin & 1) ^ 1) * kStageBytes + wave * kWaveQueries * kKPitch;
+#pragma unroll
+    for (int it = 0; it < 8; ++it) {
+      const int row = it * 4 + (lane >> 4);
+      const uint4 v = *reinterpret_cast<const uint4*>(c.q + (min(first_query + row, c.Lq - 1) * p.H + head) * kHeadDim + (lane & 15) * 8);
+      *reinterpret_cast<uint4*>(patch + row * kKPitch + (lane & 15) * 16) = v;
+    }
   }
 
   float16v o[4];
@@ -499,6 +541,13 @@ __global__ __launch_bounds__(kAttnThreads) void kv_attention_kernel(AttnParams p
 
   // prologue: the segment's first iteration into its stage, raw registers <- the second one
   fetch_next();
+  if constexpr (!WIDE) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    const uint8_t* patch = smem + ((seg_begin & 1) ^ 1) * kStageBytes + wave * kWaveQueries * kKPitch + l32 * kKPitch + lh * 16;
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks) qf[ks] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(patch + 32 * ks));
+  }
   decode_any(seg_begin & 1);
   advance();
   if (seg_begin + 1 < seg_end) fetch_next();
@@ -775,19 +824,9 @@ __global__ __launch_bounds__(kAttnThreads) void kv_attention_kernel(AttnParams p
     if (write_out) {
       float out_max = 0.0f;
       const float inv_l = 1.0f / l_run;
-      const int64_t query = (int64_t)qtile * kQueries + qq * kWaveQueries + l32;
-      if (query < c.Lq) {
-        uint16_t* dst = c.out + (query * p.H + head) * kHeadDim;
-#pragma unroll
-        for (int dt = 0; dt < 4; ++dt)
-#pragma unroll
-          for (int rg = 0; rg < 4; ++rg) {
-            const uint2 packed = make_uint2(pack_bf16(o[dt][4 * rg] * inv_l, o[dt][4 * rg + 1] * inv_l),
-                                            pack_bf16(o[dt][4 * rg + 2] * inv_l, o[dt][4 * rg + 3] * inv_l));
-            *reinterpret_cast<uint2*>(dst + dt * 32 + 8 * rg + 4 * lh) = packed;
-            out_max = abs_max_bf16x8(make_uint4(packed.x, packed.y, 0u, 0u), out_max);
-          }
-      }
+      const int64_t first_query = (int64_t)qtile * kQueries + qq * kWaveQueries;
+      write_rows<4>(o, inv_l, smem + wave * kWaveQueries * kKPitch, lane, c.out + (first_query * p.H + head) * kHeadDim, p.H,
+                    (int)min(c.Lq - first_query, (int64_t)kWaveQueries), out_max);
       if (c.sink.parts) {
         out_max = wave_max(out_max);
         if (lane == 0) amax_sink_update(AmaxSink{c.sink.parts, c.sink.epoch, c.sink.epoch_offset}, (uint32_t)tile_id * 8 + wave, out_max);
@@ -798,6 +837,7 @@ __global__ __launch_bounds__(kAttnThreads) void kv_attention_kernel(AttnParams p
     // groups 2 kp and 2 kp + 1.
     float4* xo = reinterpret_cast<float4*>(smem);                     // [wave][8][64 lanes]
     float2* xml = reinterpret_cast<float2*>(smem + 8 * 8 * 64 * 16);  // [wave][64]
+    constexpr int kMergeBytes = 8 * 8 * 64 * 16 + 8 * 64 * 8;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const float16v give = kp == 0 ? o[2 + (i >> 2)] : o[i >> 2];
@@ -900,19 +940,9 @@ __global__ __launch_bounds__(kAttnThreads) void kv_attention_kernel(AttnParams p
     }
     float out_max = 0.0f;
     const float inv_l = 1.0f / l_run;
-    const int64_t query = (int64_t)qtile * kQueries + qq * kWaveQueries + l32;
-    if (query < c.Lq) {
-      uint16_t* dst = c.out + (query * p.H + head) * kHeadDim + 64 * kp;
-#pragma unroll
-      for (int d = 0; d < 2; ++d)
-#pragma unroll
-        for (int rg = 0; rg < 4; ++rg) {
-          const uint2 packed = make_uint2(pack_bf16(own[d][4 * rg] * inv_l, own[d][4 * rg + 1] * inv_l),
-                                          pack_bf16(own[d][4 * rg + 2] * inv_l, own[d][4 * rg + 3] * inv_l));
-          *reinterpret_cast<uint2*>(dst + d * 32 + 8 * rg + 4 * lh) = packed;
-          out_max = abs_max_bf16x8(make_uint4(packed.x, packed.y, 0u, 0u), out_max);
-        }
-    }
+    const int64_t first_query = (int64_t)qtile * kQueries + qq * kWaveQueries;
+    write_rows<2>(own, inv_l, smem + kMergeBytes + wave * kWaveQueries * kKPitch, lane, c.out + (first_query * p.H + head) * kHeadDim + 64 * kp, p.H,
+                  (int)min(c.Lq - first_query, (int64_t)kWaveQueries), out_max);
     if (c.sink.parts) {
       out_max = wave_max(out_max);
       if (lane == 0) amax_sink_update(AmaxSink{c.sink.parts, c.sink.epoch, c.sink.epoch_offset}, (uint32_t)tile_id * 8 + wave, out_max);
@@ -940,14 +970,15 @@ __global__ __launch_bounds__(kAttnThreads) void kv_attention_kernel(AttnParams p
 // Bound by the issue of vector instructions (per tile 16 MFMAs beside about 480 others where the keys are cached, 150 where
 // not; counters of the first shape below: a wave issues 36 % of its cycles and waits 26 % for an issue slot, the matrix pipe
 // is busy 15 %) and, for the chunk's rows, by the LDS they pass through (index unit active 32 %, waits for it 12 %).  us, here /
-// in the tile kernels: 368 queries x 16 heads over 1472 bf16 keys 17.9 / 31.5, over 1104 cached + 368 20.5 / 32.1, 192 x 12 over
-// 768 + 192 15.7 / 23.6, 64 x 2 over 128 keys 5.5 / 7.8.
+// in the tile kernels: 368 queries x 16 heads over 1472 bf16 keys 16.1 / 31.5, over 1104 cached + 368 18.7 / 32.1.  Each wave
+// loading Q for itself, 16 bytes of each of 32 rows at a time, and a merge in 4-byte accesses took 17.3 and 20.1 there, 5.5
+// instead of 4.9 for 192 x 2 over 16 keys.
 constexpr int kShortKeys = 32;                                                // keys per wave tile
 constexpr int kShortWaveBytes = kShortKeys * (kKPitch + kVPitch);             // a wave's K and V rows
-constexpr int kShortRecord = 66 * 64;                                         // floats of a wave's result in the merge
+constexpr int kShortRecord = 66 * 64;                                         // floats of a wave's result in the merge, 16-byte aligned
 template <int W>
 constexpr size_t kShortLds = (size_t)W * kShortWaveBytes + sizeof(SlotTable);
-static_assert(kShortRecord * 4 <= kShortWaveBytes, "the merge reuses the waves' rows");
+static_assert(kShortRecord * 4 <= kShortWaveBytes && kShortWaveBytes % 16 == 0, "the merge reuses the waves' rows");
 
 // amdgpu_waves_per_eu: 256 registers per lane, two waves per SIMD (one workgroup of eight or two of four per CU)
 template <int W>
@@ -974,11 +1005,20 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) 
   const int64_t query = (int64_t)qtile * kWaveQueries + l32;
   bf16x8 qf[8];
   {
-    const uint16_t* src = p.q + ((query < p.Lq ? query : p.Lq - 1) * p.H + head) * kHeadDim + 64 * lh;
+    // The waves bring the queries into LDS together, 32 / W rows each, four rows per load, and all read the same fragments.
 #pragma unroll
-    for (int ks = 0; ks < 8; ++ks) qf[ks] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(src + 8 * ks));
+    for (int it = 0; it < 8 / W; ++it) {
+      const int row = (wave * (8 / W) + it) * 4 + (lane >> 4);
+      const int64_t at = min((int64_t)qtile * kWaveQueries + row, p.Lq - 1);
+      *reinterpret_cast<uint4*>(smem + row * kKPitch + (lane & 15) * 16) =
+          *reinterpret_cast<const uint4*>(p.q + (at * p.H + head) * kHeadDim + (lane & 15) * 8);
+    }
+    __syncthreads();  // and the slot table
+    const uint8_t* src = smem + l32 * kKPitch + lh * 128;
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks) qf[ks] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(src + 16 * ks));
   }
-  __syncthreads();  // the slot table
+  __syncthreads();  // the first wave writes its rows there
 
   float16v o[4];
 #pragma unroll
@@ -1147,44 +1187,50 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) 
     }
   }
 
-  // ---- merge: every wave leaves (O^T, reference point, row sum) in LDS, wave w combines registers 64 w / W .. of all
+  // ---- merge: every wave leaves (O^T, reference point, row sum) where its rows were, wave w combines registers 64 w / W .. of
+  // all.  Four registers per access: register 4 g + i of a lane is element i of its g-th group.
   l_run += __shfl_xor(l_run, 32, 64);
-  __syncthreads();  // all waves are through with their rows
-  float* const records = reinterpret_cast<float*>(smem);
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  auto record = [&](int w) { return reinterpret_cast<float*>(smem + w * kShortWaveBytes) + lane * 4; };
   {
-    float* mine = records + wave * kShortRecord + lane;
+    float* mine = record(wave);
 #pragma unroll
     for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) mine[(dt * 16 + i) * 64] = o[dt][i];
-    mine[64 * 64] = m_run;
-    mine[65 * 64] = l_run;
+      for (int g = 0; g < 4; ++g)
+        *reinterpret_cast<float4*>(mine + (dt * 4 + g) * 256) = make_float4(o[dt][4 * g], o[dt][4 * g + 1], o[dt][4 * g + 2], o[dt][4 * g + 3]);
+    *reinterpret_cast<float2*>(mine + 64 * 64 - 2 * lane) = make_float2(m_run, l_run);
   }
   __syncthreads();
   float a[W], m = -INFINITY, l = 0.0f;
+  float2 ml[W];
 #pragma unroll
   for (int w = 0; w < W; ++w) {
-    a[w] = records[w * kShortRecord + 64 * 64 + lane];
-    m = fmaxf(m, a[w]);
+    ml[w] = *reinterpret_cast<const float2*>(record(w) + 64 * 64 - 2 * lane);
+    m = fmaxf(m, ml[w].x);
   }
 #pragma unroll
   for (int w = 0; w < W; ++w) {
-    a[w] = a[w] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((a[w] - m) * p.scale_log2);  // a wave without a tile: -inf
-    l += a[w] * records[w * kShortRecord + 65 * 64 + lane];
+    a[w] = ml[w].x == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((ml[w].x - m) * p.scale_log2);  // a wave without a tile: -inf
+    l += a[w] * ml[w].y;
   }
   const float inv_l = 1.0f / l;
   float out_max = 0.0f;
 #pragma unroll
   for (int g = 0; g < 16 / W; ++g) {
     const int reg = wave * (64 / W) + 4 * g;  // four registers = four neighbouring elements of the head dimension
-    float v[4];
+    float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      v[i] = 0.0f;
-#pragma unroll
-      for (int w = 0; w < W; ++w) v[i] += a[w] * records[w * kShortRecord + (reg + i) * 64 + lane];
-      v[i] *= inv_l;
+    for (int w = 0; w < W; ++w) {
+      const float4 x = *reinterpret_cast<const float4*>(record(w) + (reg >> 2) * 256);
+      v[0] += a[w] * x.x;
+      v[1] += a[w] * x.y;
+      v[2] += a[w] * x.z;
+      v[3] += a[w] * x.w;
     }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] *= inv_l;
     if (query < p.Lq) {
       const uint2 packed = make_uint2(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]));
       const int d = 32 * (reg >> 4) + 8 * ((reg & 15) >> 2) + 4 * lh;

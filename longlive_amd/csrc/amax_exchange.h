@@ -16,7 +16,7 @@ struct AmaxExchangeSmem {
   unsigned long long missing[kAmaxParts / 64];      // one bit per slot that did not carry the epoch at the last look
 };
 
-// Called by every thread of the workgroup (at most 16 waves).  `thread_part`: the thread's share of the maximum of
+// Called once, by every thread of the workgroup (at most 16 whole waves).  `thread_part`: the thread's share of the maximum of
 // this workgroup's share; `slot` < G <= kAmaxParts: this workgroup's slot; `share_max(s)`: the calling thread's
 // part of the maximum of the share of workgroup s, evaluated by all threads of the workgroup together (uniform
 // control flow) when s is missing.  spin_limit + 1 looks at most; `everything`: skip the wait and compute all
@@ -27,21 +27,22 @@ __device__ __forceinline__ float exchange_amax(const AmaxSink& sink, uint32_t G,
                                                ShareMax&& share_max) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n_waves = (blockDim.x + 63) >> 6;
   const uint32_t epoch = amax_sink_epoch(sink.epoch, sink.epoch_offset);
-  auto over_waves = [&](float v) {  // maximum over the workgroup; the value is valid in every thread
+  // Maximum over the workgroup, in every thread.  A launch uses sm for one exchange, and between the two uses of sm.red here is
+  // the barrier behind the looks.
+  auto over_waves = [&](float v) {
     v = wave_max(v);
-    __syncthreads();  // the previous use of sm.red is over
     if (lane == 0) sm.red[wave] = v;
     __syncthreads();
-    float r = sm.red[0];
-    for (int w = 1; w < n_waves; ++w) r = fmaxf(r, sm.red[w]);
-    return r;
+    return max_over_16_lanes(sm.red[min(lane & 15, n_waves - 1)]);
   };
   const float mine = over_waves(thread_part);
   if (threadIdx.x == 0) amax_sink_update(sink, slot, mine);
 
   // Wave 0 looks at the G slots until all carry this launch's epoch.  Bound by the latency of a trip past the L2, hence eight
   // loads of 64 slots under way at a time and no second look at slots that have all arrived: LayerNorm and quantization of
-  // 736 x 1536 (192 slots) 8.4 us, with one load under way 9.7; 2640 x 3072 (672 slots) 16.2 against 18.3.
+  // 736 x 1536 (192 slots) 8.4 us, with one load under way 9.7; 2640 x 3072 (672 slots) 16.2 against 18.3.  Every step around the
+  // looks is a part of that latency too: with maxima over lanes and waves by LDS permutes and a read per wave the same 736 x
+  // 1536 took 8.4 instead of 7.6 us, the one-pass quantization of 48 x 256 4.5 instead of 3.9, of 736 x 1536 5.6 instead of 4.95.
   if (wave == 0) {
     constexpr uint32_t kAtOnce = 8;
     const uint32_t n_words = (G + 63) >> 6;

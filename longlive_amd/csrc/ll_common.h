@@ -155,16 +155,25 @@ inline float kv_inverse_denominator(float e2m1_max, float e4m3_max) {
 }
 
 // ----------------------------------------------------------------------------- wave helpers
+// Maxima by data-parallel-primitive moves instead of LDS permutes, which are a trip to LDS each, one behind the other.  A lane
+// that a move does not reach keeps its own value.  All 64 lanes are active.
+#define LL_DPP_MAX(v, ctrl, row_mask)                                                                                \
+  v = fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, v), __builtin_bit_cast(int, v), ctrl, row_mask, 0xF, false)))
+// Over 16 neighbouring lanes, in every one of them; see sum_over_16_lanes.
+__device__ __forceinline__ float max_over_16_lanes(float v) {
+  LL_DPP_MAX(v, 0xB1, 0xF);   // quad_perm [1, 0, 3, 2]
+  LL_DPP_MAX(v, 0x4E, 0xF);   // quad_perm [2, 3, 0, 1]
+  LL_DPP_MAX(v, 0x141, 0xF);  // row_half_mirror
+  LL_DPP_MAX(v, 0x140, 0xF);  // row_mirror
+  return v;
+}
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-  return v;
+  v = max_over_16_lanes(v);
+  LL_DPP_MAX(v, 0x142, 0xA);  // row_bcast:15 into rows 1 and 3
+  LL_DPP_MAX(v, 0x143, 0xC);  // row_bcast:31 into rows 2 and 3
+  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
 }
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
-}
+#undef LL_DPP_MAX
 // Sum over the wave with data-parallel-primitive moves instead of LDS permutes: partial sums travel down
 // each row of 16 lanes (row_shr 1, 2, 3, then 4 and 8 under bank masks), then across the rows (row_bcast 15
 // and 31), which leaves the total in lane 63; every lane returns that value.  Lanes that a move does not

@@ -141,14 +141,6 @@ struct KRaw {         // K or V of one key, one quarter of the head dimension (3
   uint32_t scales;    // 2 e4m3 block scales (low 16 bits)
 };
 
-// Load through a pointer that is known to address global memory.  Slot pointers come out of a table, so
-// the compiler would otherwise emit flat loads, whose completion also counts as an LDS event and stalls
-// the first LDS wait that follows.
-template <typename T>
-__device__ __forceinline__ T load_global(const void* ptr) {
-  return *(const __attribute__((address_space(1))) T*)ptr;
-}
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ uint4 load_global_b128(const void* ptr) {
   const u32x4 v = load_global<u32x4>(ptr);

@@ -15,9 +15,9 @@ namespace ll {
 template <int DT>
 __device__ __forceinline__ void store8(void* out, int64_t off, const float (&v)[8]) {
   if (DT == LL_DTYPE_F32) {
-    float4* p = reinterpret_cast<float4*>(static_cast<float*>(out) + off);
-    p[0] = make_float4(v[0], v[1], v[2], v[3]);
-    p[1] = make_float4(v[4], v[5], v[6], v[7]);
+    float* p = static_cast<float*>(out) + off;
+    store_b128(p, __builtin_bit_cast(u32x4, make_float4(v[0], v[1], v[2], v[3])));
+    store_b128(p + 4, __builtin_bit_cast(u32x4, make_float4(v[4], v[5], v[6], v[7])));
   } else {
     uint32_t w[4];
 #pragma unroll
@@ -29,7 +29,7 @@ __device__ __forceinline__ void store8(void* out, int64_t off, const float (&v)[
         w[i] = *reinterpret_cast<const uint32_t*>(&h);
       }
     }
-    *reinterpret_cast<uint4*>(static_cast<uint16_t*>(out) + off) = make_uint4(w[0], w[1], w[2], w[3]);
+    store_b128(static_cast<uint16_t*>(out) + off, u32x4{w[0], w[1], w[2], w[3]});
   }
 }
 
@@ -51,7 +51,7 @@ __device__ __forceinline__ void store1(void* out, int64_t off, float v) {
 // columns: 32 lanes read the 128 packed bytes of a row and write 512 bytes (bf16 / f16), whole lines both ways, and
 // a thread's rows differ by constants.  With a division per element and a thread per 8 elements the kernel was bound
 // by vector instructions: 14336 x 3072 -> bf16 in 30.2 us (3.7 TB/s), now 18.5 us (6.1 TB/s, what a copy reaches while
-// it stays in the last-level cache).
+// it stays in the last-level cache).  To f32 32.2 us; 44.3 while the compiler split the second of a thread's two stores.
 constexpr int kDeqRows = 32;
 constexpr int kDeqCols = 256;
 template <int DT>
@@ -127,9 +127,9 @@ __global__ __launch_bounds__(256) void kv_dequantize_kernel(const uint64_t* __re
   const int64_t r = grow - slot * rows_per_slot;
   const uint8_t* values = reinterpret_cast<const uint8_t*>(values_ptrs[slot]);
   const uint8_t* scales = reinterpret_cast<const uint8_t*>(scales_ptrs[slot]);
-  const float amax = *reinterpret_cast<const float*>(amax_ptrs[slot]);
-  const uint32_t packed = *reinterpret_cast<const uint32_t*>(values + r * 64 + (c >> 1));
-  const float s = e4m3_to_f32(scales[blocked_scale_offset(r, c >> 4, 8)]);
+  const float amax = load_global<float>(reinterpret_cast<const void*>(amax_ptrs[slot]));
+  const uint32_t packed = load_global<uint32_t>(values + r * 64 + (c >> 1));
+  const float s = e4m3_to_f32(load_global<uint8_t>(scales + blocked_scale_offset(r, c >> 4, 8)));
   // The slot scale as the reference's fused path forms it: amax * f32(1 / (e2m1_max * e4m3_max))
   // (utils/kernel/kv_dequant_cuda.cu:95, 216), then (code * scale) * gs left to right (:97-106): the first product
   // is exact, so every value carries one fp32 rounding.  kv_attention_kernel decodes with the same expression.

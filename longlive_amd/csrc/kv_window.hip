@@ -5,7 +5,9 @@
 //  * ll_kv_window_rope   relative RoPE (wan_5b/modules/causal_model.py:486-487, 716-771): the attended window as bf16 K
 //                        and V, [cached slots | chunk], K rotated by the window's own positions, and the rotated queries
 //
-// Both are bound by the latency of memory (ll_kv_window_rope moves 18 MB in 10 us, its waves waiting 70 % of their cycles).  As separate operations (pointer tables copied to the device, two dequantizations, mean,
+// Both are bound by the latency of memory and, for large windows, by its bandwidth: 368 queries x 16 heads over 1104 cached + 368
+// keys, 21 MB, 5.7 us, 2640 x 24 over 10560 + 2640, 260 MB, 55 us.  (6.3 and 63 with flat loads from the slots, the angles loaded behind
+// them, and stores split in two.)  As separate operations (pointer tables copied to the device, two dequantizations, mean,
 // difference, two concatenations, two rotations) the window moved every byte four times in 13 launches and synchronised
 // the host for the tables: 368 tokens of 16 heads behind 1104 cached ones took 230 us, 62 us of them on the GPU.  Here each
 // value is read once and written once; a workgroup's 256 threads hold 16 (token, head) rows, 16 lanes a row, so that the
@@ -31,8 +33,7 @@ __device__ __forceinline__ void smooth8(float (&v)[8]) {
   for (int j = 0; j < 8; ++j) v[j] = round_to_bf16(v[j] - mean);
 }
 
-__device__ __forceinline__ void rotate8(float (&v)[8], const float* __restrict__ cosr, const float* __restrict__ sinr) {
-  const float4 cs = *reinterpret_cast<const float4*>(cosr), sn = *reinterpret_cast<const float4*>(sinr);
+__device__ __forceinline__ void rotate8(float (&v)[8], const float4& cs, const float4& sn) {
   const float cc[4] = {cs.x, cs.y, cs.z, cs.w}, ss[4] = {sn.x, sn.y, sn.z, sn.w};
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -79,34 +80,47 @@ __global__ __launch_bounds__(256) void kv_window_rope_kernel(WindowParams p) {
     const uint32_t t = row / p.H;
     float v[8];
     unpack8(*reinterpret_cast<const uint4*>(p.q + (int64_t)row * 128 + c), v);
-    rotate8(v, p.cos_q + (int64_t)t * 64 + (c >> 1), p.sin_q + (int64_t)t * 64 + (c >> 1));
-    *reinterpret_cast<uint4*>(p.q_out + (int64_t)row * 128 + c) = pack8(v);
+    rotate8(v, *reinterpret_cast<const float4*>(p.cos_q + (int64_t)t * 64 + (c >> 1)), *reinterpret_cast<const float4*>(p.sin_q + (int64_t)t * 64 + (c >> 1)));
+    store_b128(p.q_out + (int64_t)row * 128 + c, __builtin_bit_cast(u32x4, pack8(v)));
     return;
   }
   const bool is_v = wg >= p.wgs_window;
   if (is_v) wg -= p.wgs_window;
-  const WindowSide& side = is_v ? p.v : p.k;
+  const WindowSide side = is_v ? p.v : p.k;
   const uint32_t row = wg * kRowsPerWindowWg + (threadIdx.x >> 4);
   if (row >= (p.n_cached + p.n_new) * p.H) return;
   const uint32_t t = row / p.H;
-  float v[8];
-  if (t < p.n_cached) {
+  const bool cached = t < p.n_cached;
+  const uint8_t *values = nullptr, *scales = nullptr, *amax = nullptr;
+  uint32_t r = 0;  // row of the slot
+  if (cached) {
     const uint32_t slot = t / p.slot_tokens;
-    const uint32_t r = row - slot * p.slot_tokens * p.H;  // row of the slot
-    const uint8_t* values = reinterpret_cast<const uint8_t*>(side.values[slot]);
-    const uint8_t* scales = reinterpret_cast<const uint8_t*>(side.scales[slot]);
-    const float gs = *reinterpret_cast<const float*>(side.amax[slot]) * p.inv_denom;
-    const float s = e4m3_to_f32(scales[blocked_scale_offset(r, c >> 4, 8)]);
+    r = row - slot * p.slot_tokens * p.H;
+    values = reinterpret_cast<const uint8_t*>(side.values[slot]);
+    scales = reinterpret_cast<const uint8_t*>(side.scales[slot]);
+    amax = reinterpret_cast<const uint8_t*>(side.amax[slot]);
+  }
+  float4 cs{}, sn{};  // on their way while the slot's pointers and then its bytes are
+  if (!is_v) {
+    cs = *reinterpret_cast<const float4*>(p.cos_k + (int64_t)t * 64 + (c >> 1));
+    sn = *reinterpret_cast<const float4*>(p.sin_k + (int64_t)t * 64 + (c >> 1));
+  }
+  float v[8];
+  if (cached) {
+    const uint32_t w = load_global<uint32_t>(values + (int64_t)r * 64 + (c >> 1));
+    const uint32_t sb = load_global<uint8_t>(scales + blocked_scale_offset(r, c >> 4, 8));
+    const float gs = load_global<float>(amax) * p.inv_denom;
+    const float s = e4m3_to_f32(sb);
     float q[8];
-    fp4x8_values(*reinterpret_cast<const uint32_t*>(values + (int64_t)r * 64 + (c >> 1)), q);
+    fp4x8_values(w, q);
 #pragma unroll
     for (int i = 0; i < 8; ++i) v[i] = round_to_bf16((q[i] * s) * gs);  // kv_dequantize_kernel's value
   } else {
     unpack8(*reinterpret_cast<const uint4*>(side.fresh + (int64_t)(row - p.n_cached * p.H) * 128 + c), v);
     if (!is_v) smooth8(v);
   }
-  if (!is_v) rotate8(v, p.cos_k + (int64_t)t * 64 + (c >> 1), p.sin_k + (int64_t)t * 64 + (c >> 1));
-  *reinterpret_cast<uint4*>(side.out + (int64_t)row * 128 + c) = pack8(v);
+  if (!is_v) rotate8(v, cs, sn);
+  store_b128(side.out + (int64_t)row * 128 + c, __builtin_bit_cast(u32x4, pack8(v)));
 }
 
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }

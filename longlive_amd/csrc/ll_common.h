@@ -200,6 +200,20 @@ __device__ __forceinline__ float sum_over_16_lanes(float v) {
 }
 #undef LL_DPP_ADD
 
+// Load through a pointer that is known to address global memory.  Slot pointers come out of a table, so
+// the compiler would otherwise emit flat loads, whose completion also counts as an LDS event and stalls
+// the first LDS wait that follows.
+template <typename T>
+__device__ __forceinline__ T load_global(const void* ptr) {
+  return *(const __attribute__((address_space(1))) T*)ptr;
+}
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+// One store of 16 bytes.  Left to itself the compiler merges the ends of a kernel's branches and stores 12 and 4, or 4 and 12.
+__device__ __forceinline__ void store_b128(void* dst, u32x4 v) {
+  asm volatile("" : "+v"(v));
+  *reinterpret_cast<u32x4*>(dst) = v;
+}
+
 // max(m, |v|) over the 8 bf16 values of a packed 16-byte group
 __device__ __forceinline__ float abs_max_bf16x8(const uint4& v, float m) {
   const uint32_t w[4] = {v.x, v.y, v.z, v.w};

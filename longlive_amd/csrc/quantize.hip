@@ -271,7 +271,6 @@ struct OnceJobs {
   int n;
 };
 constexpr uint32_t kOnceSlots = kAmaxParts / 2;  // of a tensor
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 template <int RULE, int T>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void quantize_once_kernel(OnceJobs jobs, int64_t M, int64_t K, int64_t ldx, uint32_t tiles, AmaxSink sink,

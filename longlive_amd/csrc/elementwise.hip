@@ -49,9 +49,9 @@ __global__ __launch_bounds__(kRowThreads) void adaln_kernel(const uint16_t* __re
                                                             int64_t frame_seqlen, float eps, int add_one,
                                                             uint16_t* __restrict__ out, AmaxSink sink) {
   const int lane = threadIdx.x & 63;
-  const int64_t row = (int64_t)blockIdx.x * kRowsPerWg + (threadIdx.x >> 6);
+  const int64_t row = (int64_t)blockIdx.x * kRowsPerWg + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (row >= rows) return;
-  const int64_t b = row / L, l = row - b * L, f = l / frame_seqlen;
+  const uint32_t b = (uint32_t)row / (uint32_t)L, f = ((uint32_t)row - b * (uint32_t)L) / (uint32_t)frame_seqlen;  // the host: all below 2^31
   uint4 packed[NCH];
   float out_max = adaln_row<NCH>(x + row * (int64_t)C, scale + b * sc_sb + f * sc_sf, shift + b * sh_sb + f * sh_sf, C, eps,
                                  add_one, lane, packed);
@@ -76,7 +76,7 @@ __global__ __launch_bounds__(kRowThreads) void layernorm_kernel(const uint16_t* 
                                                                 const uint16_t* __restrict__ b, float eps,
                                                                 uint16_t* __restrict__ out, AmaxSink sink) {
   const int lane = threadIdx.x & 63;
-  const int64_t row = (int64_t)blockIdx.x * kRowsPerWg + (threadIdx.x >> 6);
+  const int64_t row = (int64_t)blockIdx.x * kRowsPerWg + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (row >= rows) return;
   uint4 packed[NCH];
   float out_max = layernorm_row<NCH>(x + row * (int64_t)C, w, b, C, eps, lane, packed);
@@ -99,17 +99,20 @@ __global__ __launch_bounds__(kRowThreads) void rmsnorm_kernel(const uint16_t* __
                                                               const uint16_t* __restrict__ w, float eps,
                                                               uint16_t* __restrict__ out) {
   const int lane = threadIdx.x & 63;
-  const int64_t row = (int64_t)blockIdx.x * kRowsPerWg + (threadIdx.x >> 6);
+  const int64_t row = (int64_t)blockIdx.x * kRowsPerWg + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (row >= rows) return;
   const uint16_t* xr = x + row * (int64_t)C;
   const int nchunks = C >> 3;
   float v[NCH][8];
+  uint4 xraw[NCH], wraw[NCH];
+  load_row<NCH>(xr, nchunks, lane, xraw);
+  load_row<NCH>(w, nchunks, lane, wraw);
+  __builtin_amdgcn_sched_barrier(0);  // all loads are under way
+  unpack_row<NCH>(xraw, nchunks, lane, v);
   float sq = 0.0f;
 #pragma unroll
   for (int i = 0; i < NCH; ++i) {
-    const int c = lane + i * 64;
-    if (c < nchunks) {
-      unpack8(*reinterpret_cast<const uint4*>(xr + c * 8), v[i]);
+    if (i * 64 < nchunks) {
 #pragma unroll
       for (int j = 0; j < 8; ++j) sq += v[i][j] * v[i][j];
     }
@@ -122,7 +125,7 @@ __global__ __launch_bounds__(kRowThreads) void rmsnorm_kernel(const uint16_t* __
     const int c = lane + i * 64;
     if (c < nchunks) {
       float w8[8], y[8];
-      unpack8(*reinterpret_cast<const uint4*>(w + c * 8), w8);
+      unpack8(wraw[i], w8);
 #pragma unroll
       for (int j = 0; j < 8; ++j) y[j] = round_to_bf16(v[i][j] * r) * w8[j];
       *reinterpret_cast<uint4*>(orow + c * 8) = pack8(y);
@@ -139,7 +142,7 @@ __global__ __launch_bounds__(kRowThreads) void rmsnorm_kernel(const uint16_t* __
 // held by 16 consecutive lanes.  blockIdx.y selects the tensor (q or k), so that both go in one launch.
 // Bound by the chain of a wave (loads, one reduction, some 25 instructions per element, one or two waves per SIMD up to
 // 1000 rows) and by memory above.  With weights and angles asked for where they are used, a head's sum through LDS and one
-// conversion per rounded value: 736 x 1536 5.6 us, now 4.9; 880 x 3072 9.6 / 8.2; 2640 x 3072 19.6 / 17.4.
+// conversion per rounded value: 736 x 1536 5.6 us, now 4.7; 880 x 3072 9.6 / 7.5; 2640 x 3072 19.6 / 14.6.
 struct QkProblem {  // one tensor of the q / k pair
   const uint16_t* x;
   const uint16_t* w;
@@ -161,7 +164,7 @@ __global__ __launch_bounds__(kRowThreads) void qk_norm_rope_kernel(QkProblems pr
   uint16_t* __restrict__ out = pr.out;
   uint16_t* __restrict__ out_smooth = pr.out_smooth;
   const int lane = threadIdx.x & 63;
-  const int64_t row = (int64_t)blockIdx.x * kRowsPerWg + (threadIdx.x >> 6);
+  const int64_t row = (int64_t)blockIdx.x * kRowsPerWg + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (row >= rows) return;
   const uint16_t* xr = x + row * (int64_t)C;
   const int nchunks = C >> 3;
@@ -176,14 +179,15 @@ __global__ __launch_bounds__(kRowThreads) void qk_norm_rope_kernel(QkProblems pr
   }
   const float cc[4] = {cs.x, cs.y, cs.z, cs.w}, ss[4] = {sn.x, sn.y, sn.z, sn.w};
   float v[NCH][8];
-  uint4 wraw[NCH];
+  uint4 xraw[NCH], wraw[NCH];
+  load_row<NCH>(xr, nchunks, lane, xraw);
+  load_row<NCH>(w, nchunks, lane, wraw);
+  __builtin_amdgcn_sched_barrier(0);  // all loads are under way
+  unpack_row<NCH>(xraw, nchunks, lane, v);
   float sq = 0.0f;
 #pragma unroll
   for (int i = 0; i < NCH; ++i) {
-    const int c = lane + i * 64;
-    if (c < nchunks) {
-      unpack8(*reinterpret_cast<const uint4*>(xr + c * 8), v[i]);
-      wraw[i] = *reinterpret_cast<const uint4*>(w + c * 8);
+    if (i * 64 < nchunks) {
 #pragma unroll
       for (int j = 0; j < 8; ++j) sq += v[i][j] * v[i][j];
     }
@@ -316,11 +320,7 @@ extern "C" int ll_adaln_modulate_amax(const void* x, int64_t B, int64_t L, int C
                      static_cast<const uint16_t*>(x), B * L, L, C, static_cast<const uint16_t*>(scale),         \
                      static_cast<const uint16_t*>(shift), scale_stride_b, scale_stride_f, shift_stride_b,       \
                      shift_stride_f, frame_seqlen, eps, add_one_to_scale, static_cast<uint16_t*>(out), sink)
-  if (C <= 64 * 6 * 8) {
-    LL_LAUNCH_ADALN(6);
-  } else {
-    LL_LAUNCH_ADALN(kMaxChunks);
-  }
+  LL_BY_ROW_LENGTH(C, LL_LAUNCH_ADALN)
 #undef LL_LAUNCH_ADALN
   LL_CHECK_LAUNCH("adaln_kernel");
   return LL_OK;
@@ -342,11 +342,7 @@ extern "C" int ll_layer_norm(const void* x, int64_t rows, int C, const void* wei
   hipLaunchKernelGGL(layernorm_kernel<NCH>, grid, dim3(kRowThreads), 0, static_cast<hipStream_t>(stream),        \
                      static_cast<const uint16_t*>(x), rows, C, static_cast<const uint16_t*>(weight),             \
                      static_cast<const uint16_t*>(bias), eps, static_cast<uint16_t*>(out), sink)
-  if (C <= 64 * 6 * 8) {
-    LL_LAUNCH_LN(6);
-  } else {
-    LL_LAUNCH_LN(kMaxChunks);
-  }
+  LL_BY_ROW_LENGTH(C, LL_LAUNCH_LN)
 #undef LL_LAUNCH_LN
   LL_CHECK_LAUNCH("layernorm_kernel");
   return LL_OK;
@@ -366,11 +362,7 @@ extern "C" int ll_rms_norm(const void* x, int64_t rows, int C, const void* weigh
   hipLaunchKernelGGL(rmsnorm_kernel<NCH>, grid, dim3(kRowThreads), 0, static_cast<hipStream_t>(stream),          \
                      static_cast<const uint16_t*>(x), rows, C, static_cast<const uint16_t*>(weight), eps,        \
                      static_cast<uint16_t*>(out))
-  if (C <= 64 * 6 * 8) {
-    LL_LAUNCH_RMS(6);
-  } else {
-    LL_LAUNCH_RMS(kMaxChunks);
-  }
+  LL_BY_ROW_LENGTH(C, LL_LAUNCH_RMS)
 #undef LL_LAUNCH_RMS
   LL_CHECK_LAUNCH("rmsnorm_kernel");
   return LL_OK;
@@ -416,11 +408,7 @@ static int launch_qk_norm_rope(const ll::QkProblems& problems, int n_problems, i
 #define LL_LAUNCH_QK(NCH)                                                                                       \
   hipLaunchKernelGGL(qk_norm_rope_kernel<NCH>, grid, dim3(kRowThreads), 0, static_cast<hipStream_t>(stream),    \
                      problems, rows, (int)C, eps, cos, sin, seq_len)
-  if (C <= 64 * 6 * 8) {
-    LL_LAUNCH_QK(6);
-  } else {
-    LL_LAUNCH_QK(kMaxChunks);
-  }
+  LL_BY_ROW_LENGTH(C, LL_LAUNCH_QK)
 #undef LL_LAUNCH_QK
   LL_CHECK_LAUNCH("qk_norm_rope_kernel");
   return LL_OK;

@@ -23,6 +23,7 @@ namespace ll {
 
 constexpr int kNqThreads = 256;
 constexpr int kNqChunks = 6;  // 16-byte groups per lane: rows of up to 64 * 6 * 8 = 3072 elements
+constexpr int kNqPerCu = 3;   // workgroups per compute unit
 constexpr int kNqMaxRowLength = 64 * kNqChunks * 8;
 constexpr int kNqAdaln = 0, kNqLayerNorm = 1;
 
@@ -43,15 +44,15 @@ struct NormQuantParams {
   int recompute;  // every workgroup takes the bounded wait's way out (tests)
 };
 
-template <int MODE>
-__device__ __forceinline__ float norm_row(const NormQuantParams& p, int64_t row, int lane, uint4 (&packed)[kNqChunks]) {
+template <int MODE, int NCH>
+__device__ __forceinline__ float norm_row(const NormQuantParams& p, int64_t row, int lane, uint4 (&packed)[NCH]) {
   const uint16_t* xr = p.x + row * (int64_t)p.C;
   if (MODE == kNqAdaln) {
-    const int64_t b = row / p.L, l = row - b * p.L, f = l / p.frame_seqlen;
-    return adaln_row<kNqChunks>(xr, p.a + b * p.a_sb + f * p.a_sf, p.b + b * p.b_sb + f * p.b_sf, p.C, p.eps, p.add_one,
+    const uint32_t b = (uint32_t)row / (uint32_t)p.L, f = ((uint32_t)row - b * (uint32_t)p.L) / (uint32_t)p.frame_seqlen;  // the host: all below 2^31
+    return adaln_row<NCH>(xr, p.a + b * p.a_sb + f * p.a_sf, p.b + b * p.b_sb + f * p.b_sf, p.C, p.eps, p.add_one,
                                 lane, packed);
   }
-  return layernorm_row<kNqChunks>(xr, p.a, p.b, p.C, p.eps, lane, packed);
+  return layernorm_row<NCH>(xr, p.a, p.b, p.C, p.eps, lane, packed);
 }
 
 // The value of the neighbouring lane (lane ^ 1): quad_perm [1, 0, 3, 2].
@@ -59,43 +60,32 @@ __device__ __forceinline__ uint32_t from_pair_lane(uint32_t v) {
   return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xF, 0xF, false);
 }
 
-// One workgroup = four waves, one wave = one row at a time, R rows per wave over the launch: row
-// (r * gridDim.x + blockIdx.x) * 4 + wave.  Rows [M, Mp) are the zero padding of the quantized operand.
-// Only R = 1 is launched (see launch_rule).
-template <int RULE, int MODE, int R>
-__global__ __launch_bounds__(kNqThreads) __attribute__((amdgpu_waves_per_eu(R == 1 ? 3 : 2)))
+// One workgroup = four waves, one wave = one row, blockIdx.x * 4 + wave.  Rows [M, Mp) are the zero padding of the quantized
+// operand.  NCH: 16-byte groups per lane, even (see the second half).
+template <int RULE, int MODE, int NCH>
+__global__ __launch_bounds__(kNqThreads) __attribute__((amdgpu_waves_per_eu(kNqPerCu)))
 void norm_quantize_kernel(NormQuantParams p) {
   __shared__ AmaxExchangeSmem s_exchange;
   __shared__ ScaleEntry s_tab[128];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t G = gridDim.x;
 
   // ---- first half: the rows, kept as packed bf16, and their maximum
-  uint4 kept[R][kNqChunks];
+  uint4 kept[NCH];
   float wave_part = 0.0f;
+  const int64_t row = (int64_t)blockIdx.x * 4 + wave;
+  if (row < p.M) {
+    wave_part = norm_row<MODE, NCH>(p, row, lane, kept);
+  } else {
 #pragma unroll
-  for (int r = 0; r < R; ++r) {
-    const int64_t row = ((int64_t)r * G + blockIdx.x) * 4 + wave;
-    if (row < p.M) {
-      wave_part = fmaxf(wave_part, norm_row<MODE>(p, row, lane, kept[r]));
-    } else {
-#pragma unroll
-      for (int i = 0; i < kNqChunks; ++i) kept[r][i] = make_uint4(0u, 0u, 0u, 0u);
-    }
+    for (int i = 0; i < NCH; ++i) kept[i] = make_uint4(0u, 0u, 0u, 0u);
   }
   // ---- the maximum of the whole tensor: exchanged with the other workgroups through the sink; a missing
   // workgroup's rows are normalized here, wave w taking the row its wave w has
   const float amax = exchange_amax(p.sink, G, blockIdx.x, wave_part, p.spin_limit, p.recompute != 0, s_exchange, [&](uint32_t s) {
-    float part = 0.0f;
-#pragma unroll 1
-    for (int r = 0; r < R; ++r) {
-      const int64_t row = ((int64_t)r * G + s) * 4 + wave;
-      if (row < p.M) {
-        uint4 unused[kNqChunks];
-        part = fmaxf(part, norm_row<MODE>(p, row, lane, unused));
-      }
-    }
-    return part;
+    const int64_t theirs = (int64_t)s * 4 + wave;
+    uint4 unused[NCH];
+    return theirs < p.M ? norm_row<MODE, NCH>(p, theirs, lane, unused) : 0.0f;
   });
   if (blockIdx.x == 0 && threadIdx.x == 0) p.amax_out[0] = amax;
 
@@ -117,43 +107,40 @@ void norm_quantize_kernel(NormQuantParams p) {
   const int64_t vrow = p.C >> 1;           // bytes per row of packed values
   const uint32_t tiles_x = (uint32_t)(p.C >> 6);
   const bool odd = (lane & 1) != 0;
+  if (row >= p.Mp) return;  // uniform over the wave
+  uint8_t* vdst = p.values + row * vrow;
+  uint8_t* sdst = p.scales + (row >> 7) * (int64_t)tiles_x * 512 + (row & 31) * 16 + ((row >> 5) & 3) * 4;
 #pragma unroll
-  for (int r = 0; r < R; ++r) {
-    const int64_t row = ((int64_t)r * G + blockIdx.x) * 4 + wave;
-    if (row >= p.Mp) continue;  // uniform over the wave
-    uint8_t* vdst = p.values + row * vrow;
-    uint8_t* sdst = p.scales + (row >> 7) * (int64_t)tiles_x * 512 + (row & 31) * 16 + ((row >> 5) & 3) * 4;
+  for (int k = 0; k < NCH / 2; ++k) {
+    const uint4 even_piece = kept[2 * k], odd_piece = kept[2 * k + 1];
+    const uint4 send = odd ? even_piece : odd_piece;
+    uint4 recv;
+    recv.x = from_pair_lane(send.x);
+    recv.y = from_pair_lane(send.y);
+    recv.z = from_pair_lane(send.z);
+    recv.w = from_pair_lane(send.w);
+    const uint4 lo4 = odd ? recv : even_piece, hi4 = odd ? odd_piece : recv;
+    const int c = lane + 64 * (2 * k + (odd ? 1 : 0));  // this lane's own group of the block
+    if (c >= nchunks) continue;
+    const int blk = c >> 1;
+    const uint32_t w[8] = {lo4.x, lo4.y, lo4.z, lo4.w, hi4.x, hi4.y, hi4.z, hi4.w};
+    float X[16];
 #pragma unroll
-    for (int k = 0; k < kNqChunks / 2; ++k) {
-      const uint4 even_piece = kept[r][2 * k], odd_piece = kept[r][2 * k + 1];
-      const uint4 send = odd ? even_piece : odd_piece;
-      uint4 recv;
-      recv.x = from_pair_lane(send.x);
-      recv.y = from_pair_lane(send.y);
-      recv.z = from_pair_lane(send.z);
-      recv.w = from_pair_lane(send.w);
-      const uint4 lo4 = odd ? recv : even_piece, hi4 = odd ? odd_piece : recv;
-      const int c = lane + 64 * (2 * k + (odd ? 1 : 0));  // this lane's own group of the block
-      if (c >= nchunks) continue;
-      const int blk = c >> 1;
-      const uint32_t w[8] = {lo4.x, lo4.y, lo4.z, lo4.w, hi4.x, hi4.y, hi4.z, hi4.w};
-      float X[16];
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        X[2 * i] = __uint_as_float(w[i] << 16);
-        X[2 * i + 1] = __uint_as_float(w[i] & 0xFFFF0000u);
-      }
-      uint32_t lo, hi, sb;
-      if (!fast || !quantize_block_fast<RULE>(X, enc, s_tab, approx_ok, __builtin_inff(), lo, hi, sb))
-        quantize_block<RULE>(X, amax, enc, dec, lo, hi, sb);
-      *reinterpret_cast<uint2*>(vdst + blk * 8) = make_uint2(lo, hi);
-      sdst[(int64_t)(blk >> 2) * 512 + (blk & 3)] = (uint8_t)sb;
+    for (int i = 0; i < 8; ++i) {
+      X[2 * i] = __uint_as_float(w[i] << 16);
+      X[2 * i + 1] = __uint_as_float(w[i] & 0xFFFF0000u);
     }
+    uint32_t lo, hi, sb;
+    if (!fast || !quantize_block_fast<RULE>(X, enc, s_tab, approx_ok, __builtin_inff(), lo, hi, sb))
+      quantize_block<RULE>(X, amax, enc, dec, lo, hi, sb);
+    *reinterpret_cast<uint2*>(vdst + blk * 8) = make_uint2(lo, hi);
+    sdst[(int64_t)(blk >> 2) * 512 + (blk & 3)] = (uint8_t)sb;
   }
 }
 
-// Workgroups of norm_quantize_kernel<rule, mode, R> that the current device holds at once.
-template <int RULE, int MODE, int R>
+// Workgroups of norm_quantize_kernel<rule, mode, NCH> that the current device holds at once.  Those for short rows would fit more
+// often; a unit counts for kNqPerCu of any, so that the rows of a launch do not depend on their length.
+template <int RULE, int MODE, int NCH>
 static int resident_of(int* out) {
   static std::atomic<int> cache[64];
   int dev = 0;
@@ -166,29 +153,29 @@ static int resident_of(int* out) {
   int n = slot ? slot->load(std::memory_order_relaxed) : 0;
   if (n == 0) {
     int per_cu = 0, cus = 0;
-    e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, norm_quantize_kernel<RULE, MODE, R>, kNqThreads, 0);
+    e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, norm_quantize_kernel<RULE, MODE, NCH>, kNqThreads, 0);
     if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
     if (e != hipSuccess || per_cu <= 0 || cus <= 0) {
       set_error("norm_quantize: occupancy query failed: %s", hipGetErrorString(e));
       return LL_ELAUNCH;
     }
-    n = per_cu * cus;
+    n = (per_cu < kNqPerCu ? per_cu : kNqPerCu) * cus;
     if (slot) slot->store(n, std::memory_order_relaxed);
   }
   *out = n;
   return LL_OK;
 }
 
-template <int RULE, int MODE, int R>
+template <int RULE, int MODE, int NCH>
 static int launch_with(NormQuantParams& p, hipStream_t stream, bool* fits) {
   int resident = 0;
-  if (int rc = resident_of<RULE, MODE, R>(&resident)) return rc;
+  if (int rc = resident_of<RULE, MODE, NCH>(&resident)) return rc;
   const int64_t groups = p.Mp / 4;  // Mp is a multiple of 128
   int64_t grid = resident < kAmaxParts ? resident : kAmaxParts;
   if (grid > groups) grid = groups;
-  *fits = grid * R >= groups;
+  *fits = grid >= groups;
   if (!*fits) return LL_OK;
-  hipLaunchKernelGGL((norm_quantize_kernel<RULE, MODE, R>), dim3((unsigned)grid), dim3(kNqThreads), 0, stream, p);
+  hipLaunchKernelGGL((norm_quantize_kernel<RULE, MODE, NCH>), dim3((unsigned)grid), dim3(kNqThreads), 0, stream, p);
   return LL_OK;
 }
 
@@ -197,7 +184,9 @@ static int launch_rule(NormQuantParams& p, hipStream_t stream, bool* fits) {
   // One row per wave, three waves per SIMD.  Variants that keep two or four rows per wave (and so take more rows
   // than the device holds waves) were measured: at 7040 rows the kernel then takes as long as the two separate
   // kernels (36 us), at two waves per SIMD, so those shapes are left to the separate operations.
-  return launch_with<RULE, MODE, 1>(p, stream, fits);
+  if (p.C <= 64 * 2 * 8) return launch_with<RULE, MODE, 2>(p, stream, fits);
+  if (p.C <= 64 * 4 * 8) return launch_with<RULE, MODE, 4>(p, stream, fits);
+  return launch_with<RULE, MODE, kNqChunks>(p, stream, fits);
 }
 
 template <int MODE>

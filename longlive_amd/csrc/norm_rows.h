@@ -25,46 +25,76 @@ __device__ __forceinline__ uint4 pack8(const float (&f)[8]) {
 }
 
 // Row kernels: one wave per row (no workgroup barrier; a row's sums are wave reductions), four rows per
-// workgroup.  A lane holds NCH groups of 8 elements: NCH = 6 covers C = 3072 exactly, 16 anything up to 8192.
+// workgroup.  A lane holds NCH groups of 8 elements: NCH = 6 covers C = 3072 exactly, 16 anything up to 8192; groups that a row
+// does not have cost their loads and the sum all the same, hence kernels for shorter rows.
 constexpr int kRowThreads = 256;
 constexpr int kRowsPerWg = kRowThreads / 64;
 constexpr int kMaxChunks = 16;  // 8 elements each: C <= 64 * 16 * 8 = 8192
 constexpr int kMaxRowLength = 64 * kMaxChunks * 8;
+#define LL_BY_ROW_LENGTH(C, LAUNCH) \
+  if ((C) <= 64 * 1 * 8) {          \
+    LAUNCH(1);                      \
+  } else if ((C) <= 64 * 3 * 8) {   \
+    LAUNCH(3);                      \
+  } else if ((C) <= 64 * 6 * 8) {   \
+    LAUNCH(6);                      \
+  } else if ((C) <= 64 * 10 * 8) {  \
+    LAUNCH(10);                     \
+  } else {                          \
+    LAUNCH(kMaxChunks);             \
+  }
+
+// The lane's groups of a row, all requested before the first is waited for; behind the row's end its last group once more.
+// (With the load of a group under a branch of its own, and its use there, the compiler waits for every group before it asks
+// for the next: a row of 3072 was six trips to memory.  us so / now, with kernels for shorter rows: RMSNorm 880 x 3072 4.8 / 3.9, LayerNorm
+// 2640 x 3072 8.5 / 7.8, adaLN 736 x 1536 4.0 / 3.6, 4096 x 5120 34.3 / 20.3, q and k 2640 x 3072 17.4 / 14.6, 4096 x 5120 42.8 / 33.5,
+// adaLN and quantization 736 x 1536 8.6 / 7.75.)
+template <int NCH>
+__device__ __forceinline__ void load_row(const uint16_t* __restrict__ row, int nchunks, int lane, uint4 (&raw)[NCH]) {
+#pragma unroll
+  for (int i = 0; i < NCH; ++i) raw[i] = *reinterpret_cast<const uint4*>(row + min(lane + i * 64, nchunks - 1) * 8);
+}
+// As floats, zeros behind the row's end; the lane's sum of them.  No branch and no choice here, into which a load would sink.
+template <int NCH>
+__device__ __forceinline__ float unpack_row(const uint4 (&raw)[NCH], int nchunks, int lane, float (&v)[NCH][8]) {
+  float sum = 0.0f;
+#pragma unroll
+  for (int i = 0; i < NCH; ++i) {
+    const uint32_t keep = lane + i * 64 < nchunks ? 0xFFFFFFFFu : 0u;
+    unpack8(make_uint4(raw[i].x & keep, raw[i].y & keep, raw[i].z & keep, raw[i].w & keep), v[i]);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) sum += v[i][j];
+  }
+  return sum;
+}
 
 // adaLN modulation of one row, utils/adaln_triton.py:36-86: LayerNorm without affine in fp32, rounded to bf16,
 // times (1 + scale) rounded, plus shift rounded.  `packed[i]` receives the 8 results of group lane + 64 i; the
-// return value is the lane's share of the row's absolute maximum.  Two values share a rounding's conversion: adaln_kernel takes
-// 9.6 us for 2640 x 3072, with one each 10.2.
+// return value is the lane's share of the row's absolute maximum.  Two values share a rounding's conversion: adaln_kernel took
+// 9.6 us for 2640 x 3072 so (before load_row), with one each 10.2.
 template <int NCH>
 __device__ __forceinline__ float adaln_row(const uint16_t* __restrict__ xr, const uint16_t* __restrict__ scr,
                                            const uint16_t* __restrict__ shr, int C, float eps, int add_one, int lane,
                                            uint4 (&packed)[NCH]) {
   const int nchunks = C >> 3;
   float v[NCH][8];
-  uint4 sraw[NCH], hraw[NCH];  // requested up front: their latency runs under the two reductions
-  float sum = 0.0f;
-#pragma unroll
-  for (int i = 0; i < NCH; ++i) {
-    const int c = lane + i * 64;
-    if (c < nchunks) {
-      unpack8(*reinterpret_cast<const uint4*>(xr + c * 8), v[i]);
-      sraw[i] = *reinterpret_cast<const uint4*>(scr + c * 8);
-      hraw[i] = *reinterpret_cast<const uint4*>(shr + c * 8);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) sum += v[i][j];
-    }
-  }
+  uint4 xraw[NCH], sraw[NCH], hraw[NCH];
+  load_row<NCH>(xr, nchunks, lane, xraw);
+  load_row<NCH>(scr, nchunks, lane, sraw);
+  load_row<NCH>(shr, nchunks, lane, hraw);
+  __builtin_amdgcn_sched_barrier(0);  // all loads are under way
+  const float sum = unpack_row<NCH>(xraw, nchunks, lane, v);
   const float inv_c = 1.0f / (float)C;
   const float mean = wave_sum_dpp(sum) * inv_c;
   float sq = 0.0f;
 #pragma unroll
   for (int i = 0; i < NCH; ++i) {
-    const int c = lane + i * 64;
-    if (c < nchunks) {
+    if (i * 64 < nchunks) {
+      const bool in = lane + i * 64 < nchunks;
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         v[i][j] -= mean;
-        sq += v[i][j] * v[i][j];
+        sq += in ? v[i][j] * v[i][j] : 0.0f;
       }
     }
   }
@@ -73,28 +103,30 @@ __device__ __forceinline__ float adaln_row(const uint16_t* __restrict__ xr, cons
   float out_max = 0.0f;
 #pragma unroll
   for (int i = 0; i < NCH; ++i) {
-    const int c = lane + i * 64;
     packed[i] = make_uint4(0u, 0u, 0u, 0u);
-    if (c < nchunks) {
+    if (i * 64 < nchunks) {
       float s8[8], h8[8], y[8];
       unpack8(sraw[i], s8);
       unpack8(hraw[i], h8);
+      if (add_one) {
+#pragma unroll
+        for (int j = 0; j < 8; j += 2) {
+          s8[j] += 1.0f;
+          s8[j + 1] += 1.0f;
+          round_to_bf16(s8[j], s8[j + 1]);
+        }
+      }
 #pragma unroll
       for (int j = 0; j < 8; j += 2) {
-        float x0 = v[i][j] * rstd, x1 = v[i][j + 1] * rstd, s0 = s8[j], s1 = s8[j + 1];
+        float x0 = v[i][j] * rstd, x1 = v[i][j + 1] * rstd;
         round_to_bf16(x0, x1);
-        if (add_one) {
-          s0 += 1.0f;
-          s1 += 1.0f;
-          round_to_bf16(s0, s1);
-        }
-        x0 *= s0;
-        x1 *= s1;
+        x0 *= s8[j];
+        x1 *= s8[j + 1];
         round_to_bf16(x0, x1);
         y[j] = x0 + h8[j];
         y[j + 1] = x1 + h8[j + 1];
       }
-      packed[i] = pack8(y);
+      if (lane + i * 64 < nchunks) packed[i] = pack8(y);
       out_max = abs_max_bf16x8(packed[i], out_max);
     }
   }
@@ -109,30 +141,28 @@ __device__ __forceinline__ float layernorm_row(const uint16_t* __restrict__ xr, 
                                                uint4 (&packed)[NCH]) {
   const int nchunks = C >> 3;
   float v[NCH][8];
-  uint4 wraw[NCH], braw[NCH];  // requested up front: their latency runs under the two reductions
-  float sum = 0.0f;
+  uint4 xraw[NCH], wraw[NCH], braw[NCH];
 #pragma unroll
   for (int i = 0; i < NCH; ++i) {
-    const int c = lane + i * 64;
-    if (c < nchunks) {
-      unpack8(*reinterpret_cast<const uint4*>(xr + c * 8), v[i]);
-      wraw[i] = w ? *reinterpret_cast<const uint4*>(w + c * 8) : make_uint4(0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u);
-      braw[i] = b ? *reinterpret_cast<const uint4*>(b + c * 8) : make_uint4(0, 0, 0, 0);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) sum += v[i][j];
-    }
+    wraw[i] = make_uint4(0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u);
+    braw[i] = make_uint4(0u, 0u, 0u, 0u);
   }
+  load_row<NCH>(xr, nchunks, lane, xraw);
+  if (w) load_row<NCH>(w, nchunks, lane, wraw);
+  if (b) load_row<NCH>(b, nchunks, lane, braw);
+  __builtin_amdgcn_sched_barrier(0);  // all loads are under way
+  const float sum = unpack_row<NCH>(xraw, nchunks, lane, v);
   const float inv_c = 1.0f / (float)C;
   const float mean = wave_sum_dpp(sum) * inv_c;
   float sq = 0.0f;
 #pragma unroll
   for (int i = 0; i < NCH; ++i) {
-    const int c = lane + i * 64;
-    if (c < nchunks) {
+    if (i * 64 < nchunks) {
+      const bool in = lane + i * 64 < nchunks;
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         v[i][j] -= mean;
-        sq += v[i][j] * v[i][j];
+        sq += in ? v[i][j] * v[i][j] : 0.0f;
       }
     }
   }
@@ -141,15 +171,14 @@ __device__ __forceinline__ float layernorm_row(const uint16_t* __restrict__ xr, 
   float out_max = 0.0f;
 #pragma unroll
   for (int i = 0; i < NCH; ++i) {
-    const int c = lane + i * 64;
     packed[i] = make_uint4(0u, 0u, 0u, 0u);
-    if (c < nchunks) {
+    if (i * 64 < nchunks) {
       float w8[8], b8[8], y[8];
       unpack8(wraw[i], w8);
       unpack8(braw[i], b8);
 #pragma unroll
       for (int j = 0; j < 8; ++j) y[j] = (v[i][j] * rstd) * w8[j] + b8[j];
-      packed[i] = pack8(y);
+      if (lane + i * 64 < nchunks) packed[i] = pack8(y);
       out_max = abs_max_bf16x8(packed[i], out_max);
     }
   }

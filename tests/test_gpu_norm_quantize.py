@@ -165,3 +165,44 @@ def test_batches_of_two_with_strided_scale_and_shift(gpu):
     y = _native.adaln_modulate(x, scale, shift, L // frames, amax_out=t)
     want = _native.quantize(y.reshape(-1, C), "mse", amax=t)
     _same(_native.adaln_quantize(x, scale, shift, L // frames, "mse"), want, "B = 2")
+
+
+@pytest.mark.parametrize("C", [64, 512, 576, 1024, 1088, 1536, 1544, 1600, 2048, 2112, 3072, 3080, 3136, 5120, 5128, 8192])
+def test_rows_at_the_edges_of_the_row_kernels(gpu, C):
+    """Lengths around those at which the row kernels hold more groups per lane, with a number of rows that leaves waves of
+    the last workgroup without one, against fp64.  Each bound is the roundings to bf16 on the way (half a step of eight bits,
+    2^-8 of the value at most, each) on the magnitudes that pass through them, and 2^-18 for the fp32 statistics of at most 8192 terms."""
+    L, frames = 21, 3
+    x, scale, shift = _inputs(gpu, L, C, frames, seed=C, outliers=False)
+    w, b = scale[0, 0, 0], shift[0, 0, 0]
+    x64, eps, half = x[0].double(), 2.0 ** -8, 2.0 ** -18
+    sc = scale[0, :, 0].double().repeat_interleave(L // frames, 0)
+    sh = shift[0, :, 0].double().repeat_interleave(L // frames, 0)
+    mean = x64.mean(-1, keepdim=True)
+    n = (x64 - mean) / ((x64 - mean).square().mean(-1, keepdim=True) + 1e-6).sqrt()
+
+    y = _native.adaln_modulate(x, scale, shift, L // frames)[0].double()
+    want, product = n * (1 + sc) + sh, (n * (1 + sc)).abs()
+    # the norm, 1 + scale (whose error the norm scales) and the product are rounded before the sum, then the sum
+    bound = (3 * eps + half) * 1.02 * product + half * (1 + sc).abs() + eps * want.abs() * 1.02
+    assert bool(((y - want).abs() <= bound).all())
+
+    y = _native.layer_norm(x, w, b, 1e-6)[0].double()
+    want, product = n * w.double() + b.double(), (n * w.double()).abs()
+    assert bool(((y - want).abs() <= eps * want.abs() + half * (product + b.double().abs() + w.double().abs())).all())
+
+    r = x64 / (x64.square().mean(-1, keepdim=True) + 1e-6).sqrt()
+    want = r * w.double()
+    y = _native.rms_norm(x[0], w, 1e-6).double()
+    assert bool(((y - want).abs() <= (2 * eps * 1.02 + half) * want.abs()).all())
+
+    if C % 128 == 0:
+        H, rms = C // 128, _native.rms_norm(x[0], w, 1e-6)
+        angle = torch.randn(L, 64, generator=torch.Generator().manual_seed(C)).to(gpu)
+        cos, sin = angle.cos(), angle.sin()
+        got = _native.qk_norm_rope(x[0], w, 1e-6, cos, sin, H)
+        assert torch.equal(got, _native.rope_apply(rms.view(L, H, 128), cos, sin).view_as(got))
+    if C % 64 == 0 and C <= 3072:
+        _same(_native.adaln_quantize(x, scale, shift, L // frames, "mse"), _separate_adaln(x, scale, shift, L // frames, "mse")[1], f"adaLN {L}x{C}")
+        want = _native.quantize(_native.layer_norm(x, w, b, 1e-6).reshape(-1, C), "mse")
+        _same(_native.layer_norm_quantize(x, w, b, "mse"), want, f"LayerNorm {L}x{C}")

@@ -1195,3 +1195,40 @@ def test_which_calls_the_ends_of_the_model_run_on_their_kernels(gpu, monkeypatch
         too_many = torch.randn(1, 1025, 128, device=gpu).bfloat16()
         small = CausalDiT(DiTConfig(dim=128, ffn_dim=128, num_heads=1, num_layers=0)).to(gpu).bfloat16()
         assert small.head.latents(too_many, torch.randn(1, 1, 1, 128, device=gpu).bfloat16(), (1, 1, 1025), (1, 2, 2), 48) is None
+
+
+@pytest.mark.parametrize("channels,patch,latent,k", [
+    (16, (1, 2, 2), (2, 6, 10), 16),      # one step of 16: seven of the head's eight waves have none
+    (56, (1, 4, 4), (1, 8, 12), 528),     # the longest patch the embedding takes, 896 elements; steps dealt unevenly
+    (16, (1, 3, 3), (2, 9, 12), 1088),    # no pairs; more than eight steps per wave
+    (8, (2, 1, 5), (4, 3, 15), 1552),     # 80 elements: less than a round of the gathering; twelve steps and a half per wave
+])
+def test_patches_land_where_they_belong(gpu, channels, patch, latent, k):
+    """The embedding with the unit matrix for a weight gives back every patch element exactly, with and without a bias of whole
+    numbers; the head against fp64 over contractions of uneven lengths (half a bf16 step, 2^-8, plus the fp32 sum's K 2^-24)."""
+    from longlive_amd import _native
+
+    lib, stream = _native.load(), torch.cuda.current_stream().cuda_stream
+    grid, K = tuple(a // b for a, b in zip(latent, patch)), channels * math.prod(patch)
+    g = torch.Generator().manual_seed(K)
+    x = torch.randint(-100, 100, (channels, *latent), generator=g).to(gpu).bfloat16()
+    (f, h, w), (pt, ph, pw) = grid, patch
+    patches = x.reshape(channels, f, pt, h, ph, w, pw).permute(1, 3, 5, 0, 2, 4, 6).reshape(-1, K)
+    unit, bias = torch.eye(K, device=gpu).bfloat16(), torch.randint(-20, 20, (K,), generator=g).to(gpu).bfloat16()
+    for b in (None, bias):
+        out = torch.empty(patches.shape, dtype=torch.bfloat16, device=gpu)
+        assert lib.ll_patch_embed(x.data_ptr(), channels, *latent, *patch, unit.data_ptr(), None if b is None else b.data_ptr(), K,
+                                  out.data_ptr(), stream) == 0, lib.ll_last_error()
+        assert torch.equal(out, patches if b is None else patches + b)
+
+    M = f * h * w
+    y, weight = torch.randn(M, k, generator=g).to(gpu).bfloat16(), torch.randn(K, k, generator=g).to(gpu).bfloat16()
+    for b in (None, bias):
+        out = torch.empty_like(x)
+        assert lib.ll_patch_head(y.data_ptr(), k, weight.data_ptr(), None if b is None else b.data_ptr(), channels, *latent, *patch,
+                                 out.data_ptr(), stream) == 0, lib.ll_last_error()
+        add = torch.zeros(K, dtype=torch.float64, device=gpu) if b is None else b.double()
+        back = lambda t: t.reshape(f, h, w, pt, ph, pw, channels).permute(6, 0, 3, 1, 4, 2, 5).reshape(x.shape)
+        ref = back(y.double() @ weight.double().T + add)
+        size = back(y.double().abs() @ weight.double().abs().T + add.abs())
+        assert bool(((out.double() - ref).abs() <= ref.abs() * 2 ** -8 + size * (k + 2) * 2 ** -24).all())

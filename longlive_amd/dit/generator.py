@@ -149,7 +149,9 @@ class StreamingGenerator:
             is_scene_cut = self.multi_shot_sink and cfg.sink_size > 0 and ci > 0 and ci in scene_cuts
             if self.sampler == "unipc":
                 scheduler = FlowUniPCMultistepScheduler(num_train_timesteps=1000, shift=1)
-                scheduler.set_timesteps(len(self.timesteps), device=self.device, shift=self.sample_shift)
+                # On the host, where the timesteps are looked at: on the device every chunk waited three times for all
+                # work before it (the list, and the place of the first timestep in it).
+                scheduler.set_timesteps(len(self.timesteps), shift=self.sample_shift)
                 steps = scheduler.timesteps.tolist()
             else:
                 scheduler, steps = None, self.timesteps

@@ -117,9 +117,9 @@ LL_SPLIT_FN int first_iteration_of_part(uint32_t part, uint32_t parts, int n_ite
 //   G <= 2 CUs    736 x 12, 0 + 16: 16.3 / 18.4 / 13.7; 512 x 24, 32 + 16: 34.7 / 38.3 / 32.8, but 46 + 23 on 736 x 12:
 //                 38.7 / 49.9 / 43.5;   G > 2 CUs: 736 x 24, 0 + 16: 16.8 / 26.4 / 20.5
 // A cached tile costs about half as much again as one of the chunk (conversion).  Launches of more than 256 queries per
-// head for every head stay with the divided tiles because the line ends where the measurements above do, not because the
-// tiles are ahead there: the one point taken beyond it (700 queries of 2 heads over 900 keys) is 27.8 us against 12.9 in this
-// kernel.  Moving it takes a sweep of 1 to 6 heads with 512 to 4096 queries.
+// head for every head take it over up to 16 tiles; over more the measurements end at one point (700 queries of 2 heads over
+// 900 keys: 12.9 us here, 27.8 in 256-query tiles), and 128-query tiles that share their key ranges (plan_narrow_split) have taken
+// most of what there was to gain.
 // `policy`: only the automatic choice (-1) and the division without shared tiles (0) take this kernel.  The launch, the
 // plan query and the reserve call all ask here.
 inline int short_kernel_waves(int64_t Lq, int H, int64_t n_cached, int64_t n_new, int cus, int policy) {

@@ -117,7 +117,7 @@ LL_SPLIT_FN int first_iteration_of_part(uint32_t part, uint32_t parts, int n_ite
 //   G <= 2 CUs    736 x 12, 0 + 16: 16.3 / 18.4 / 13.7; 512 x 24, 32 + 16: 34.7 / 38.3 / 32.8, but 46 + 23 on 736 x 12:
 //                 38.7 / 49.9 / 43.5;   G > 2 CUs: 736 x 24, 0 + 16: 16.8 / 26.4 / 20.5
 // A cached tile costs about half as much again as one of the chunk (conversion).  Launches of more than 256 queries per
-// head for every head take it over up to 16 tiles; over more the measurements end at one point (700 queries of 2 heads over
+// head for every head take it over up to 16 tiles (3520 x 2, 0 + 16: 15.4 / 10.4 / 10.5); over more the measurements end at one point (700 queries of 2 heads over
 // 900 keys: 12.9 us here, 27.8 in 256-query tiles), and 128-query tiles that share their key ranges (plan_narrow_split) have taken
 // most of what there was to gain.
 // `policy`: only the automatic choice (-1) and the division without shared tiles (0) take this kernel.  The launch, the

@@ -742,7 +742,7 @@ __global__ __launch_bounds__(kAttnThreads) void kv_attention_kernel(AttnParams p
   l_run += __shfl_xor(l_run, 32, 64);  // row sums were per wave half so far
   {  // epilogue of the segment, with its own copies of the thread's coordinates (see fresh_thread_index)
   const auto& c = reread_params();
-  const int tid = fresh_thread_index(), lane = tid & 63, wave = tid >> 6, l32 = lane & 31, lh = lane >> 5;
+  const int tid = fresh_thread_index(), lane = tid & 63, wave = tid >> 6;
   const int qq = WIDE ? wave : (wave & 3), kp = WIDE ? 0 : (wave >> 2);
   if constexpr (WIDE) {
     // Every wave has seen its segment of the key range for its 32 queries.
@@ -962,8 +962,8 @@ __global__ __launch_bounds__(kAttnThreads) void kv_attention_kernel(AttnParams p
 // Bound by the issue of vector instructions (per tile 16 MFMAs beside about 480 others where the keys are cached, 150 where
 // not; counters of the first shape below: a wave issues 36 % of its cycles and waits 26 % for an issue slot, the matrix pipe
 // is busy 15 %) and, for the chunk's rows, by the LDS they pass through (index unit active 32 %, waits for it 12 %).  us, here /
-// in the tile kernels: 368 queries x 16 heads over 1472 bf16 keys 16.1 / 31.5, over 1104 cached + 368 18.7 / 32.1.  Each wave
-// loading Q for itself, 16 bytes of each of 32 rows at a time, and a merge in 4-byte accesses took 17.3 and 20.1 there, 5.5
+// in the tile kernels: 368 queries x 16 heads over 1472 bf16 keys 14.8 / 31.5, over 1104 cached + 368 18.0 / 32.1.  Each wave
+// loading Q for itself, 16 bytes of each of 32 rows at a time, and a merge in 4-byte accesses cost 1.2 and 1.4 more there, 5.5
 // instead of 4.9 for 192 x 2 over 16 keys.
 constexpr int kShortKeys = 32;                                                // keys per wave tile
 constexpr int kShortWaveBytes = kShortKeys * (kKPitch + kVPitch);             // a wave's K and V rows
@@ -973,44 +973,87 @@ constexpr size_t kShortLds = (size_t)W * kShortWaveBytes + sizeof(SlotTable);
 static_assert(kShortRecord * 4 <= kShortWaveBytes && kShortWaveBytes % 16 == 0, "the merge reuses the waves' rows");
 
 // amdgpu_waves_per_eu: 256 registers per lane, two waves per SIMD (one workgroup of eight or two of four per CU)
-template <int W>
+// CACHED: there are cached keys.  The first tile's bytes are asked for with the queries (without cached keys) or as soon as the
+// slot pointers are there (with them, the slots' scales still on their way), and a tile's rows without conditions, which the
+// compiler turns into sixteen branches per tile.  us, before that / now: 368 x 16 over 1472 16.1 / 14.8, over 1104 + 368 18.7 / 18.0, 520 x
+// 24 over 1030 21.6 / 19.9, 736 x 12 over 512 12.9 / 12.0, 192 x 2 over 768 + 192 14.0 / 13.2.
+template <int W, bool CACHED>
 __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void kv_attention_short_kernel(AttnParams p) {
   static_assert(W == 4 || W == 8, "the merge gives every wave 64 / W of the 64 output registers");
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   SlotTable& tab = *reinterpret_cast<SlotTable*>(smem + W * kShortWaveBytes);
-  if (const int t = threadIdx.x; t < p.n_slots) {
+  float ka = 0.0f, va = 0.0f;
+  if (const int t = threadIdx.x; CACHED && t < p.n_slots) {
     tab.kv[t] = reinterpret_cast<const uint8_t*>(p.kv_ptrs[t]);
     tab.ks[t] = reinterpret_cast<const uint8_t*>(p.ks_ptrs[t]);
     tab.vv[t] = reinterpret_cast<const uint8_t*>(p.vv_ptrs[t]);
     tab.vs[t] = reinterpret_cast<const uint8_t*>(p.vs_ptrs[t]);
-    tab.kg[t] = load_global<float>(reinterpret_cast<const void*>(p.ka_ptrs[t])) * p.inv_denom;
-    tab.vg[t] = load_global<float>(reinterpret_cast<const void*>(p.va_ptrs[t])) * p.inv_denom;
+    ka = load_global<float>(reinterpret_cast<const void*>(p.ka_ptrs[t]));
+    va = load_global<float>(reinterpret_cast<const void*>(p.va_ptrs[t]));
   }
   const uint32_t tile_id = group_number(p.d.G);
   const int head = (int)(tile_id / (uint32_t)p.n_qtiles), qtile = (int)(tile_id - (uint32_t)head * (uint32_t)p.n_qtiles);
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l32 = lane & 31, lh = lane >> 5;
-  const int n_cached = (int)p.n_cached, n_new = (int)p.n_new;
+  const int n_cached = CACHED ? (int)p.n_cached : 0, n_new = (int)p.n_new;
   const int cached_tiles = (n_cached + kShortKeys - 1) / kShortKeys, n_tiles = cached_tiles + (n_new + kShortKeys - 1) / kShortKeys;
   uint8_t* const krows = smem + wave * kShortWaveBytes;
   uint8_t* const vrows = krows + kShortKeys * kKPitch;
+  int t = wave;
+
+  // The chunk's own keys: piece j of a tile is rows 4 j + lane / 16, 16 bytes per lane.
+  uint4 kb[8], vb[8];
+  const int64_t row_step = (int64_t)p.H * kHeadDim;
+  auto fetch_new = [&](int tile, const uint16_t* src, uint4 (&dst)[8]) __attribute__((always_inline)) {
+    const int key0 = (tile - cached_tiles) * kShortKeys + (lane >> 4);
+#pragma unroll
+    for (int j = 0; j < 8; ++j)  // behind the last key: the last again, zeros when it is written to LDS
+      dst[j] = load_global_b128(src + min(key0 + 4 * j, n_new - 1) * row_step + head * kHeadDim + (lane & 15) * 8);
+  };
+  // Cached keys: lane = (key l32, half lh of the head dimension) for K and V alike.
+  struct { uint4 v[2]; uint32_t scales; } kf, vf;
+  uint32_t slot = 0;
+  auto fetch_cached = [&](int tile) __attribute__((always_inline)) {
+    const uint32_t key = (uint32_t)min(tile * kShortKeys + l32, n_cached - 1);
+    slot = key / (uint32_t)p.bts;
+    const int64_t row = (int64_t)(key - slot * (uint32_t)p.bts) * p.H + head;
+    const uint32_t vo = (uint32_t)row * 64u + lh * 32u, so = (uint32_t)blocked_scale_offset(row, lh * 4, 8);
+    kf.v[0] = load_global_b128(tab.kv[slot] + vo);
+    kf.v[1] = load_global_b128(tab.kv[slot] + vo + 16);
+    kf.scales = load_global<uint32_t>(tab.ks[slot] + so);
+    vf.v[0] = load_global_b128(tab.vv[slot] + vo);
+    vf.v[1] = load_global_b128(tab.vv[slot] + vo + 16);
+    vf.scales = load_global<uint32_t>(tab.vs[slot] + so);
+  };
 
   const int64_t query = (int64_t)qtile * kWaveQueries + l32;
   bf16x8 qf[8];
   {
     // The waves bring the queries into LDS together, 32 / W rows each, four rows per load, and all read the same fragments.
+    uint4 q[8 / W];
 #pragma unroll
     for (int it = 0; it < 8 / W; ++it) {
       const int row = (wave * (8 / W) + it) * 4 + (lane >> 4);
       const int64_t at = min((int64_t)qtile * kWaveQueries + row, p.Lq - 1);
-      *reinterpret_cast<uint4*>(smem + row * kKPitch + (lane & 15) * 16) =
-          *reinterpret_cast<const uint4*>(p.q + (at * p.H + head) * kHeadDim + (lane & 15) * 8);
+      q[it] = load_global_b128(p.q + (at * p.H + head) * kHeadDim + (lane & 15) * 8);
     }
-    __syncthreads();  // and the slot table
+    if (!CACHED) {  // a wave without a tile loads the last: under a condition these loads would be waited for with the queries
+      fetch_new(min(t, n_tiles - 1), p.k_new, kb);
+      fetch_new(min(t, n_tiles - 1), p.v_new, vb);
+    }
+#pragma unroll
+    for (int it = 0; it < 8 / W; ++it)
+      *reinterpret_cast<uint4*>(smem + ((wave * (8 / W) + it) * 4 + (lane >> 4)) * kKPitch + (lane & 15) * 16) = q[it];
+    __syncthreads();  // and the slot pointers
+    if (CACHED && (int)threadIdx.x < p.n_slots) {
+      tab.kg[threadIdx.x] = ka * p.inv_denom;
+      tab.vg[threadIdx.x] = va * p.inv_denom;
+    }
+    if (CACHED && t < cached_tiles) fetch_cached(t);
     const uint8_t* src = smem + l32 * kKPitch + lh * 128;
 #pragma unroll
     for (int ks = 0; ks < 8; ++ks) qf[ks] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(src + 16 * ks));
   }
-  __syncthreads();  // the first wave writes its rows there
+  __syncthreads();  // the first wave writes its rows there; the slots' scales
 
   float16v o[4];
 #pragma unroll
@@ -1088,26 +1131,9 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) 
     __builtin_amdgcn_wave_barrier();
   };
 
-  // ---- cached keys: lane = (key l32, half lh of the head dimension) for K and V alike
-  int t = wave;
-  {
-    struct { uint4 v[2]; uint32_t scales; } kf, vf;
-    float kg = 0.0f, vg = 0.0f;
-    auto fetch = [&](int tile) __attribute__((always_inline)) {
-      const uint32_t key = (uint32_t)min(tile * kShortKeys + l32, n_cached - 1);
-      const uint32_t slot = key / (uint32_t)p.bts;
-      const int64_t row = (int64_t)(key - slot * (uint32_t)p.bts) * p.H + head;
-      const uint32_t vo = (uint32_t)row * 64u + lh * 32u, so = (uint32_t)blocked_scale_offset(row, lh * 4, 8);
-      kf.v[0] = load_global_b128(tab.kv[slot] + vo);
-      kf.v[1] = load_global_b128(tab.kv[slot] + vo + 16);
-      kf.scales = load_global<uint32_t>(tab.ks[slot] + so);
-      vf.v[0] = load_global_b128(tab.vv[slot] + vo);
-      vf.v[1] = load_global_b128(tab.vv[slot] + vo + 16);
-      vf.scales = load_global<uint32_t>(tab.vs[slot] + so);
-      kg = tab.kg[slot];
-      vg = tab.vg[slot];
-    };
-    if (t < cached_tiles) fetch(t);
+  // ---- cached keys
+  if constexpr (CACHED) {
+    float kg = tab.kg[slot], vg = tab.vg[slot];
     for (; t < cached_tiles; t += W) {
       const int valid = n_cached - t * kShortKeys;
       float16v sc;
@@ -1125,7 +1151,11 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) 
       block_scales_f16(vsc, *reinterpret_cast<half2v(*)[2]>(&vs2[0]));
       block_scales_f16(vsc >> 16, *reinterpret_cast<half2v(*)[2]>(&vs2[2]));
       const float kgt = kg, vgt = live ? vg : 0.0f;
-      if (t + W < cached_tiles) fetch(t + W);
+      if (t + W < cached_tiles) {
+        fetch_cached(t + W);
+        kg = tab.kg[slot];
+        vg = tab.vg[slot];
+      }
       uint4* vdst = reinterpret_cast<uint4*>(vrows + l32 * kVPitch + lh * 128);
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
@@ -1141,23 +1171,19 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) 
       softmax_pv(sc, valid);
     }
   }
-  // ---- the chunk's own keys: piece j of a tile is rows 4 j + lane / 16, 16 bytes per lane
+  // ---- the chunk's own keys
   if (t < n_tiles) {
-    uint4 kb[8], vb[8];
-    const int64_t row_step = (int64_t)p.H * kHeadDim;
-    auto fetch = [&](int tile, const uint16_t* src, uint4 (&dst)[8]) __attribute__((always_inline)) {
-      const int key0 = (tile - cached_tiles) * kShortKeys + (lane >> 4);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const int key = key0 + 4 * j;
-        dst[j] = make_uint4(0u, 0u, 0u, 0u);
-        if (key < n_new) dst[j] = load_global_b128(src + key * row_step + head * kHeadDim + (lane & 15) * 8);
-      }
-    };
-    fetch(t, p.k_new, kb);
-    fetch(t, p.v_new, vb);
+    if (CACHED) {
+      fetch_new(t, p.k_new, kb);
+      fetch_new(t, p.v_new, vb);
+    }
     for (; t < n_tiles; t += W) {
       const int valid = n_new - (t - cached_tiles) * kShortKeys;
+      if (valid < kShortKeys) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          if (4 * j + (lane >> 4) >= valid) kb[j] = vb[j] = make_uint4(0u, 0u, 0u, 0u);
+      }
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         *reinterpret_cast<uint4*>(krows + (4 * j + (lane >> 4)) * kKPitch + (lane & 15) * 16) = kb[j];
@@ -1165,8 +1191,8 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) 
       }
       rows_written();
       if (t + W < n_tiles) {
-        fetch(t + W, p.k_new, kb);
-        fetch(t + W, p.v_new, vb);
+        fetch_new(t + W, p.k_new, kb);
+        fetch_new(t + W, p.v_new, vb);
       }
       float16v sc;
 #pragma unroll
@@ -1262,15 +1288,21 @@ static int launch_attention(const AttnParams& p_in, hipStream_t stream) {
   if (const int waves = short_kernel_waves(p.Lq, p.H, p.n_cached, p.n_new, cus, policy)) {
     p.n_qtiles = (int)((p.Lq + kWaveQueries - 1) / kWaveQueries);
     p.d.G = (uint32_t)(p.H * p.n_qtiles);
-    static std::atomic<uint64_t> lds_allowed4{0}, lds_allowed8{0};
-    const void* kernel = waves == 8 ? reinterpret_cast<const void*>(&kv_attention_short_kernel<8>) : reinterpret_cast<const void*>(&kv_attention_short_kernel<4>);
-    const size_t lds = waves == 8 ? kShortLds<8> : kShortLds<4>;
-    if (int rc = allow_dynamic_lds(kernel, lds, waves == 8 ? lds_allowed8 : lds_allowed4, "ll_kv_attention")) return rc;
-    if (waves == 8) {
-      hipLaunchKernelGGL(kv_attention_short_kernel<8>, dim3(p.d.G), dim3(512), lds, stream, p);
+    static std::atomic<uint64_t> lds_allowed[4] = {};
+#define LL_LAUNCH_SHORT(W, CACHED, i)                                                                                                            \
+  if (int rc = allow_dynamic_lds(reinterpret_cast<const void*>(&kv_attention_short_kernel<W, CACHED>), kShortLds<W>, lds_allowed[i], "ll_kv_attention")) \
+    return rc;                                                                                                                                   \
+  hipLaunchKernelGGL((kv_attention_short_kernel<W, CACHED>), dim3(p.d.G), dim3(W * 64), kShortLds<W>, stream, p)
+    if (waves == 8 && p.n_cached > 0) {
+      LL_LAUNCH_SHORT(8, true, 0);
+    } else if (waves == 8) {
+      LL_LAUNCH_SHORT(8, false, 1);
+    } else if (p.n_cached > 0) {
+      LL_LAUNCH_SHORT(4, true, 2);
     } else {
-      hipLaunchKernelGGL(kv_attention_short_kernel<4>, dim3(p.d.G), dim3(256), lds, stream, p);
+      LL_LAUNCH_SHORT(4, false, 3);
     }
+#undef LL_LAUNCH_SHORT
     LL_CHECK_LAUNCH("kv_attention_short_kernel");
     return LL_OK;
   }

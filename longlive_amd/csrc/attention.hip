@@ -27,6 +27,7 @@
 #include "attention_split.h"
 
 #include <algorithm>
+#include <cfloat>
 #include <map>
 #include <mutex>
 #include <utility>
@@ -379,7 +380,9 @@ __global__ __launch_bounds__(kAttnThreads) void kv_attention_kernel(AttnParams p
   for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
     for (int i = 0; i < 16; ++i) o[dt][i] = 0.0f;
-  float m_run = -INFINITY, l_run = 0.0f;
+  // The reference point starts below every finite score and not at -inf: a tile whose scores are all -inf leaves it there and
+  // weighs exp2(-inf) = 0, where -inf - -inf is NaN.
+  float m_run = -FLT_MAX, l_run = 0.0f;
 
   // ---- decode plan.  Thread = (key_local = tid / 4, quarter of the head dim = tid % 4), the same for K and V.
   // Schedule of iteration `it`: the MFMAs work on LDS stage it & 1 while the raw FP4 bytes of iteration

@@ -1020,6 +1020,25 @@ def test_scores_of_minus_infinity_weigh_nothing(gpu, Lq, H, keys, gone):
     assert ((out.double() - ref).abs() <= 1.25 * 2 ** -9 * size + 2 ** -9 * ref.abs()).all()
 
 
+@pytest.mark.parametrize("policy", POLICIES)
+@pytest.mark.parametrize("gone", [(0, 128), (256, 512), (600, 900)])
+def test_tiles_whose_scores_are_all_minus_infinity_weigh_nothing(gpu, policy, gone):
+    """The same under every division, where the keys that are gone are a wave's first tile, all tiles of a part (128-query tiles
+    in four parts under the automatic choice) or a part's last ones."""
+    Lq, H, keys = 700, 2, 900
+    q, k, v = (_randn((n, H, 128), s).to(gpu) for n, s in ((Lq, 61), (keys, 62), (keys, 63)))
+    q[..., 0], k[..., 0] = 1e20, 0.0
+    k[gone[0]:gone[1], :, 0] = -1e20
+    assert _native.attention_plan(Lq, H, keys)["workgroups"] == 4 * H * -(-Lq // 128)
+    with _native.attention_policy(policy):
+        out = _native.attention_bf16(q, k, v, 128 ** -0.5)
+    left = [i for i in range(keys) if not gone[0] <= i < gone[1]]
+    K, V = k[left].double(), v[left].double()
+    p = [torch.softmax(q[:, h].double() @ K[:, h].T.contiguous() * 128 ** -0.5, -1) for h in range(H)]
+    ref, size = (torch.stack([ph @ x[:, h] for h, ph in enumerate(p)], 1) for x in (V, V.abs()))
+    assert ((out.double() - ref).abs() <= 1.25 * 2 ** -9 * size + 2 ** -9 * ref.abs()).all()
+
+
 @pytest.mark.parametrize("Lq,H,T,cached,n_new", [(512, 16, 512, 0, 4000), (512, 16, 512, 3584, 416), (520, 24, 480, 0, 1900),
                                                 (520, 24, 480, 1440, 460), (512, 16, 512, 2048, 512)])
 def test_the_plan_is_what_the_launch_does(gpu, Lq, H, T, cached, n_new):

@@ -51,11 +51,13 @@ int ll_version(void);
  * recorded launch uses: on a capturing stream, or where the memory cannot be had, one workgroup computes the parts of a
  * tile one after the other, with the same bits.  ll_release_stream_memory frees the sets of (current device, stream), if
  * any, after waiting for the launches that still use them - for callers that create streams as they go.  Launches of the
- * first two kernels on a stream that is being captured into a graph never allocate: they use the set a
+ * first two kernels on a stream that is being captured into a graph never allocate: they take the set a
  * reserve call or an earlier launch left on that stream, or fall back to a division of the work that needs none.
- * A set that a captured launch has used belongs to the recorded graph as well: it is not freed when the stream
- * later needs a larger one (the old set is kept aside), only by ll_release_stream_memory, which must therefore not
- * be called while such a graph may still be replayed.  No counterpart in the reference.
+ * A set that a captured launch has taken belongs to the recordings of that stream from then on: later recordings use it too,
+ * ordinary launches set up another one, so a graph may be replayed on any stream beside ordinary work on the stream it was
+ * recorded on.  Graphs recorded on one stream share the set: their replays must not overlap one another.  It is freed by
+ * ll_release_stream_memory only, which must therefore not be called while such a graph may still be replayed; where a
+ * recording needs a larger set, the old one is kept aside.  No counterpart in the reference.
  */
 int ll_release_stream_memory(void* stream);
 
@@ -362,7 +364,8 @@ int ll_kv_attention_amax(const void* q, int64_t Lq, int num_heads,
  *                        the automatic choice then takes one of the others).  Tiles shared by two
  *                        workgroups pass through device memory that the library allocates on the first such
  *                        launch on a (device, stream) pair and keeps (69 MB on a 256-CU device); launches that
- *                        use it must not overlap on one stream's memory, which same-stream order guarantees.
+ *                        use it must not overlap on one stream's memory, which same-stream order guarantees for
+ *                        ordinary launches (for recorded ones see ll_release_stream_memory).
  * All give the same result up to the order of fp32 additions (each is deterministic).  The setting is
  * process-wide.  A launch on a stream that is being captured into a graph never allocates: it uses the memory an
  * earlier launch or ll_kv_attention_reserve left on that stream, and without such memory the automatic choice

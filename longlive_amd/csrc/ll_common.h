@@ -7,6 +7,7 @@
 #include <atomic>
 
 #include "../../include/ll_nvfp4.h"
+#include "scratch_sets.h"
 
 namespace ll {
 
@@ -33,15 +34,8 @@ void set_error(const char* fmt, ...);
 inline int64_t round_up(int64_t x, int64_t m) { return (x + m - 1) / m * m; }
 
 // ----------------------------------------------------------------------------- memory of the library's own (stream_scratch.hip)
-// Records for partial tiles and arrival counters, one set per (device, stream).
-struct StreamScratch {
-  uint8_t* records = nullptr;
-  size_t record_bytes = 0;
-  int* counters = nullptr;  // zero whenever no launch is running
-  size_t n_counters = 0;
-};
-// A set with at least record_bytes and `counters` counters.  may_allocate false (the stream is being captured into
-// a graph): only a set that is already large enough is handed out, and *missing says that there is none.
+// A set with at least record_bytes and `counters` counters (scratch_sets.h).  may_allocate false (the stream is being
+// captured into a graph): only a set that is already large enough is handed out, and *missing says that there is none.
 int stream_scratch(int dev, hipStream_t stream, size_t record_bytes, size_t counters, bool may_allocate, StreamScratch& out,
                    bool* missing, const char* what);
 // The records and counters of the small products of a stream; false where there is none to be had (the stream is being

@@ -1,27 +1,20 @@
 // Device memory of the library's own: the records through which workgroups of one launch hand partial tiles to each
 // other (the split division of the attention kernel, the K-split shares of the persistent GEMM, the K ranges of small
-// products) and the arrival counters that go with them.  One set per (device, stream): launches on one stream run one after the other and can
-// share it, launches on different streams get different sets.  A set is created at the first launch that needs one,
-// grown when a later launch needs more, and kept until ll_release_stream_memory or the end of the process.  The
-// counters are zero whenever no launch is running: every kernel that uses them leaves them at zero.
+// products) and the arrival counters that go with them.  One set per (device, stream): launches on one stream run one after
+// the other and can share it, launches on different streams get different sets, and so do the launches that were recorded on a
+// stream (scratch_sets.h).  A set is created at the first launch that needs one, grown when a later launch needs more, and kept
+// until ll_release_stream_memory or the end of the process.  The counters are zero whenever no launch is running: every kernel
+// that uses them leaves them at zero.
 #include <map>
 #include <mutex>
-#include <vector>
 
 #include "ll_common.h"
 #include "gemm_split.h"
 
 namespace ll {
 
-// A set that a capturing stream has used is part of a recorded graph, which will use the same addresses at every
-// replay: such a set is never freed when a later launch needs a larger one (it is kept aside until the release call).
-struct ScratchEntry {
-  StreamScratch current{};
-  bool recorded = false;
-  std::vector<StreamScratch> retired;
-};
 static std::mutex g_scratch_mutex;
-static std::map<std::pair<int, hipStream_t>, ScratchEntry> g_scratch;
+static std::map<std::pair<int, hipStream_t>, ScratchSets> g_scratch;
 
 // The memory of small products (gemm_w4a4_small_kernel) is a set of its own: launches of the other kernels that are
 // recorded keep using the set above at every replay, on whatever stream that is, and an ordinary linear layer beside
@@ -34,47 +27,43 @@ static void free_scratch(StreamScratch& w) {
   w = StreamScratch{};
 }
 
+// Records and counters of the sizes in w, the counters zero for the work that follows on `stream`.
+static hipError_t allocate_scratch(StreamScratch& w, hipStream_t stream) {
+  // an allocation is refused, and a recording elsewhere spoilt, while another stream is captured in the global mode
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  const bool exchanged = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+  hipError_t e = hipMalloc(reinterpret_cast<void**>(&w.records), w.record_bytes);
+  if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void**>(&w.counters), w.n_counters * sizeof(int));
+  if (e == hipSuccess) e = hipMemsetAsync(w.counters, 0, w.n_counters * sizeof(int), stream);
+  if (e != hipSuccess) free_scratch(w);
+  if (exchanged) (void)hipThreadExchangeStreamCaptureMode(&mode);
+  return e;
+}
+
 int stream_scratch(int dev, hipStream_t stream, size_t record_bytes, size_t counters, bool may_allocate, StreamScratch& out,
                    bool* missing, const char* what) {
   std::lock_guard<std::mutex> lock(g_scratch_mutex);
   if (missing) *missing = false;
   if (!may_allocate) {  // the stream is being captured
     const auto it = g_scratch.find({dev, stream});
-    if (it == g_scratch.end() || it->second.current.record_bytes < record_bytes ||
-        it->second.current.n_counters < counters) {
-      if (missing) *missing = true;
-      return LL_OK;
-    }
-    it->second.recorded = true;
-    out = it->second.current;
+    const StreamScratch* w = it == g_scratch.end() ? nullptr : it->second.for_recording(record_bytes, counters);
+    if (w) out = *w;
+    else if (missing) *missing = true;
     return LL_OK;
   }
-  ScratchEntry& entry = g_scratch[{dev, stream}];
-  StreamScratch& w = entry.current;
-  if (w.record_bytes < record_bytes || w.n_counters < counters) {
-    const size_t want_bytes = record_bytes > w.record_bytes ? record_bytes : w.record_bytes;
-    size_t want_counters = counters > w.n_counters ? counters : w.n_counters;
-    if (want_counters < 4096) want_counters = 4096;
-    if (entry.recorded && w.records) {
-      entry.retired.push_back(w);
-      w = StreamScratch{};
-      entry.recorded = false;
-    } else {
-      free_scratch(w);
-    }
-    hipError_t e = hipMalloc(reinterpret_cast<void**>(&w.records), want_bytes);
-    if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void**>(&w.counters), want_counters * sizeof(int));
-    if (e == hipSuccess) e = hipMemsetAsync(w.counters, 0, want_counters * sizeof(int), stream);
-    if (e != hipSuccess) {
+  ScratchSets& sets = g_scratch[{dev, stream}];
+  StreamScratch grown;
+  if (!sets.for_launch(record_bytes, counters, grown)) {
+    free_scratch(sets.ordinary);
+    const size_t want_bytes = grown.record_bytes;
+    if (const hipError_t e = allocate_scratch(grown, stream); e != hipSuccess) {
       set_error("%s: cannot set up %zu bytes for partial results: %s", what, want_bytes, hipGetErrorString(e));
-      free_scratch(w);
-      if (entry.retired.empty()) g_scratch.erase({dev, stream});
+      if (sets.empty()) g_scratch.erase({dev, stream});
       return LL_ELAUNCH;
     }
-    w.record_bytes = want_bytes;
-    w.n_counters = want_counters;
+    sets.ordinary = grown;
   }
-  out = w;
+  out = sets.ordinary;
   return LL_OK;
 }
 
@@ -85,14 +74,7 @@ bool small_product_scratch(int dev, hipStream_t stream, int cus, StreamScratch& 
   if (!w.records) {
     w.record_bytes = (size_t)small_product_units(cus) * kSmallRecordBytes;
     w.n_counters = (size_t)small_product_units(cus);
-    // an allocation is refused, and a recording elsewhere spoilt, while another stream is captured in the global mode
-    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-    const bool exchanged = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
-    hipError_t e = hipMalloc(reinterpret_cast<void**>(&w.records), w.record_bytes);
-    if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void**>(&w.counters), w.n_counters * sizeof(int));
-    if (e == hipSuccess) e = hipMemsetAsync(w.counters, 0, w.n_counters * sizeof(int), stream);
-    if (e != hipSuccess) free_scratch(w);
-    if (exchanged) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    const hipError_t e = allocate_scratch(w, stream);
     if (e != hipSuccess) {
       (void)hipGetLastError();  // the caller has a way without the memory
       g_small_scratch.erase({dev, stream});
@@ -111,7 +93,8 @@ int release_stream_scratch(int dev, hipStream_t stream) {
   }
   const auto it = g_scratch.find({dev, stream});
   if (it == g_scratch.end()) return LL_OK;
-  free_scratch(it->second.current);
+  free_scratch(it->second.ordinary);
+  free_scratch(it->second.recorded);
   for (StreamScratch& old : it->second.retired) free_scratch(old);
   g_scratch.erase(it);
   return LL_OK;

@@ -3,12 +3,13 @@
 // software e4m3 / e2m1 codecs value by value; and runs the attention kernel's work-division arithmetic
 // (attention_split.h, the very functions the kernel calls) on the host, so that the CPU tests can check that every
 // (tile, iteration) of a launch is covered exactly once - and on the device, so that the GPU tests can check that both
-// sides compute the same numbers.
+// sides compute the same numbers; and likewise the bookkeeping of the streams' memory (scratch_sets.h).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
 #include "attention_split.h"
 #include "gemm_split.h"
+#include "scratch_sets.h"
 
 __global__ void convert_kernel(const float* __restrict__ in, int64_t n, int mode, uint8_t* __restrict__ out) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -132,4 +133,30 @@ extern "C" void ll_test_gemm_plan(int64_t M, int64_t N, int64_t Kp, int n_produc
 // How a small product is divided: workgroups that share a tile's K range.
 extern "C" int ll_test_small_gemm_parts(int64_t M, int64_t N, int64_t Kp, int n_products, int cus) {
   return ll::plan_small_gemm(M, N, Kp, n_products, cus).parts;
+}
+
+// A sequence of launches on one stream through the bookkeeping of its memory (scratch_sets.h).  ops: triples (0 ordinary launch,
+// 1 recorded launch; record bytes; counters).  set[i] = number of the set that launch i gets, in the order of their allocation
+// from 1 on, or 0 for none; freed[s] = whether set s + 1 was freed on the way.  Returns the number of sets allocated.
+extern "C" int ll_test_scratch_sets(const int64_t* ops, int n, int32_t* set, int32_t* freed) {
+  ll::ScratchSets sets;
+  intptr_t allocated = 0;
+  auto number = [](const ll::StreamScratch& w) { return (int32_t)reinterpret_cast<intptr_t>(w.records); };
+  for (int i = 0; i < n; ++i) {
+    const size_t bytes = (size_t)ops[3 * i + 1], counters = (size_t)ops[3 * i + 2];
+    if (ops[3 * i]) {
+      const ll::StreamScratch* w = sets.for_recording(bytes, counters);
+      set[i] = w ? number(*w) : 0;
+      continue;
+    }
+    ll::StreamScratch grown;
+    if (!sets.for_launch(bytes, counters, grown)) {
+      if (sets.ordinary.records) freed[number(sets.ordinary) - 1] = 1;
+      grown.records = reinterpret_cast<uint8_t*>(++allocated);
+      freed[allocated - 1] = 0;
+      sets.ordinary = grown;
+    }
+    set[i] = number(sets.ordinary);
+  }
+  return (int)allocated;
 }

@@ -139,6 +139,20 @@ def attention_full_plan(Lq: int, H: int, n_keys: int, cus: int = 256, policy: in
     return plan
 
 
+def scratch_sets(ops):
+    """[(recorded, record bytes, counters), ...] of one stream through the library's bookkeeping of its memory: the number of the
+    set each launch gets (0: none), and the numbers of the sets that were freed."""
+    import ctypes
+
+    lib = _test_hooks()
+    lib.ll_test_scratch_sets.restype = ctypes.c_int
+    lib.ll_test_scratch_sets.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p]
+    flat = (ctypes.c_int64 * (3 * len(ops)))(*[int(x) for op in ops for x in op])
+    sets, freed = (ctypes.c_int32 * len(ops))(), (ctypes.c_int32 * len(ops))()
+    n = lib.ll_test_scratch_sets(flat, len(ops), sets, freed)
+    return list(sets), [i + 1 for i in range(n) if freed[i]]
+
+
 def attention_division_on_device(division: dict, split_tiles: int, device):
     """first_unit_of(g) for g = 0 .. G and (first, last) holder of every split tile, computed by a kernel that calls the
     same functions as the attention kernel; and the host's values for the same division."""

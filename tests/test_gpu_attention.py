@@ -840,6 +840,31 @@ def test_launch_on_a_capturing_stream_never_allocates(gpu):
     _native.attention_release()   # a stream without memory: nothing to do
 
 
+@pytest.mark.parametrize("Lq,H,Lk", [(700, 2, 900), (3000, 24, 640)])   # shared 128-query and 256-query tiles
+def test_a_graph_replays_beside_ordinary_launches_of_the_stream_it_was_recorded_on(gpu, Lq, H, Lk):
+    """Recorded launches have memory of their own: replays on one stream and ordinary launches on the recording's stream, at
+    the same time, all give the bits of a launch by itself."""
+    q, k, v = (_randn((n, H, 128), s).to(gpu) for n, s in ((Lq, 91), (Lk, 92), (Lk, 93)))
+    side, other, graph = torch.cuda.Stream(device=gpu), torch.cuda.Stream(device=gpu), torch.cuda.CUDAGraph()
+    side.wait_stream(torch.cuda.current_stream())
+    with _native.attention_policy("split"):
+        with torch.cuda.stream(side):
+            alone = _native.attention_bf16(q, k, v, 128 ** -0.5)
+        side.synchronize()
+        with torch.cuda.graph(graph, stream=side):
+            recorded = [_native.attention_bf16(q, k, v, 128 ** -0.5) for _ in range(8)]
+        for _ in range(4):
+            with torch.cuda.stream(other):
+                graph.replay()
+            with torch.cuda.stream(side):
+                ordinary = [_native.attention_bf16(q, k, v, 128 ** -0.5) for _ in range(8)]
+            torch.cuda.synchronize()
+            assert all(torch.equal(out, alone) for out in recorded + ordinary)
+    del graph
+    with torch.cuda.stream(side):
+        _native.attention_release()
+
+
 @pytest.mark.parametrize("window_tokens,sink_blocks", [(2 * 128 + 40, 1), (3 * 128 - 1, 0), (128 + 64, 0)])
 def test_windows_that_end_inside_a_block_against_the_policy_oracle(gpu, window_tokens, sink_blocks):
     """max_attention_size that is not a multiple of the block size (wan_5b/modules/causal_model.py:673-724 slices token

@@ -397,6 +397,28 @@ def test_attention_work_division_covers_every_iteration_exactly_once():
         _check_division(plan, rounds * G + extra + full_split + light_split)
 
 
+def test_recorded_and_ordinary_launches_never_share_memory():
+    """A graph may be replayed on another stream beside ordinary launches of the stream it was recorded on."""
+    from helpers import scratch_sets
+
+    run, rec = 0, 1
+    #                     warm-up       recording     ordinary work  a smaller recording
+    assert scratch_sets([(run, 100, 9), (rec, 100, 9), (run, 100, 9), (rec, 50, 2), (run, 60, 3)]) == ([1, 1, 2, 1, 2], [])
+    # a recording without memory has none; what it finds too small stays with the graphs that use it, and only an ordinary
+    # launch's set is freed for a larger one
+    assert scratch_sets([(rec, 10, 1), (run, 100, 9), (rec, 200, 9), (rec, 100, 9), (run, 100, 9), (run, 200, 9), (rec, 200, 9), (rec, 100, 5),
+                         (run, 50, 1)]) == ([0, 1, 0, 1, 2, 3, 3, 3, 4], [2])
+    assert scratch_sets([(run, 100, 9), (rec, 100, 5000), (run, 100, 5000), (rec, 100, 5000)]) == ([1, 0, 2, 2], [1])
+    rng = np.random.default_rng(5)
+    for _ in range(200):
+        ops = [(int(rng.integers(2)), int(rng.integers(1, 500)), int(rng.integers(1, 9000))) for _ in range(30)]
+        sets, freed = scratch_sets(ops)
+        seen = [{s for s, op in zip(sets, ops) if op[0] == kind and s} for kind in (run, rec)]
+        assert not seen[rec] & set(freed)
+        for i, (s, op) in enumerate(zip(sets, ops)):   # once recorded, never an ordinary launch's again
+            assert op[0] == run or s == 0 or s not in [t for t, later in zip(sets[i:], ops[i:]) if later[0] == run]
+
+
 def test_persistent_gemm_division_covers_every_k_step_exactly_once():
     """The persistent GEMM's division of a launch between workgroups (longlive_amd/csrc/gemm_split.h, the functions
     the kernel calls, compiled for the host): over the launcher's plans for the benchmark shapes, the released

@@ -360,16 +360,15 @@ int ll_kv_attention_amax(const void* q, int64_t Lq, int num_heads,
  *                        along the key range into shares of equal cost (a head's last, partly filled group of
  *                        queries counts for less), so that no compute unit waits for another.  Launches with at most
  *                        half a 128-query tile per compute unit take those instead where that is cheapest, the key range
- *                        of each in equal parts (while a stream is being captured only if this division is asked for:
- *                        the automatic choice then takes one of the others).  Tiles shared by two
+ *                        of each in equal parts.  Tiles shared by several
  *                        workgroups pass through device memory that the library allocates on the first such
  *                        launch on a (device, stream) pair and keeps (69 MB on a 256-CU device); launches that
  *                        use it must not overlap on one stream's memory, which same-stream order guarantees for
  *                        ordinary launches (for recorded ones see ll_release_stream_memory).
  * All give the same result up to the order of fp32 additions (each is deterministic).  The setting is
- * process-wide.  A launch on a stream that is being captured into a graph never allocates: it uses the memory an
- * earlier launch or ll_kv_attention_reserve left on that stream, and without such memory the automatic choice
- * takes the cheaper of NARROW and WIDE while an explicit LL_ATTENTION_SPLIT returns LL_ENOSUP.
+ * process-wide.  A launch on a stream that is being captured into a graph is divided as any other, and has its bits, but never
+ * allocates: it uses the memory an earlier launch of the shape or ll_kv_attention_reserve left on that stream, and without
+ * such memory the automatic choice takes the cheaper of NARROW and WIDE while an explicit LL_ATTENTION_SPLIT returns LL_ENOSUP.
  */
 #define LL_ATTENTION_AUTO (-1)
 #define LL_ATTENTION_NARROW 0

@@ -26,7 +26,6 @@
 #include "ll_common.h"
 #include "attention_split.h"
 
-#include <algorithm>
 #include <cfloat>
 #include <map>
 #include <mutex>
@@ -1311,10 +1310,6 @@ static int launch_attention(const AttnParams& p_in, hipStream_t stream) {
   }
   AttentionPlan plan = plan_division(p.Lq, p.H, p.n_cached, p.n_new, cus, policy);
   StreamScratch w;
-  const bool capturing = plan.mode == LL_ATTENTION_SPLIT && stream_is_capturing(stream);
-  // A recorded launch takes 128-query tiles with shared key ranges only where the split division is asked for: replays on
-  // several streams may meet in the memory that these use, and what they take the place of mostly uses none.
-  if (capturing && policy == LL_ATTENTION_AUTO && plan.queries == kWgQueries) plan = plan_attention(p.Lq, p.H, p.n_cached + p.n_new, cus, policy);
   if (plan.mode == LL_ATTENTION_SPLIT) {
     // The split division passes partial tiles through device memory of the library's own.  While the stream is
     // being captured nothing may be allocated (and the clearing of a new set must not become a graph node): a set
@@ -1322,8 +1317,8 @@ static int launch_attention(const AttnParams& p_in, hipStream_t stream) {
     // automatic choice falls back to the cheaper of the two divisions that need no memory, and an explicit
     // request for the split division is refused.
     bool missing = false;
-    if (int rc = stream_scratch(dev, stream, partial_records(plan) * partial_bytes(plan.queries), (size_t)plan.split_tiles, !capturing, w,
-                                &missing, "ll_kv_attention")) return rc;
+    if (int rc = stream_scratch(dev, stream, partial_records(plan) * partial_bytes(plan.queries), (size_t)plan.split_tiles,
+                                !stream_is_capturing(stream), w, &missing, "ll_kv_attention")) return rc;
     if (missing) {
       if (policy == LL_ATTENTION_SPLIT) {
         set_error("ll_kv_attention: the split division needs device memory that cannot be allocated while the stream "
@@ -1377,21 +1372,15 @@ extern "C" int ll_kv_attention_reserve_window(int64_t Lq, int num_heads, int64_t
   if (int rc = compute_units_of(dev, cus, "ll_kv_attention")) return rc;
   const int policy = g_attention_policy.load(std::memory_order_relaxed);
   if (short_kernel_waves(Lq, num_heads, n_cached, n_new, cus, policy)) return LL_OK;
-  // what the launch takes, and what it takes while the stream is being captured
-  const AttentionPlan plans[2] = {plan_division(Lq, num_heads, n_cached, n_new, cus, policy), plan_attention(Lq, num_heads, n_cached + n_new, cus, policy)};
-  size_t record_bytes = 0, counters = 0;
-  for (const AttentionPlan& plan : plans) {
-    if (plan.mode != LL_ATTENTION_SPLIT) continue;
-    record_bytes = std::max(record_bytes, partial_records(plan) * partial_bytes(plan.queries));
-    counters = std::max(counters, (size_t)plan.split_tiles);
-  }
-  if (record_bytes == 0) return LL_OK;
+  const AttentionPlan plan = plan_division(Lq, num_heads, n_cached, n_new, cus, policy);
+  if (plan.mode != LL_ATTENTION_SPLIT) return LL_OK;
   if (stream_is_capturing(static_cast<hipStream_t>(stream))) {
     set_error("ll_kv_attention_reserve: the stream is being captured; reserve before the recording starts");
     return LL_ENOSUP;
   }
   StreamScratch w;
-  return stream_scratch(dev, static_cast<hipStream_t>(stream), record_bytes, counters, true, w, nullptr, "ll_kv_attention_reserve");
+  return stream_scratch(dev, static_cast<hipStream_t>(stream), partial_records(plan) * partial_bytes(plan.queries), (size_t)plan.split_tiles, true, w,
+                        nullptr, "ll_kv_attention_reserve");
 }
 
 // Cached keys are the longer way through the short kernel, and one fresh key may make a tile more: where these two need no

@@ -840,6 +840,33 @@ def test_launch_on_a_capturing_stream_never_allocates(gpu):
     _native.attention_release()   # a stream without memory: nothing to do
 
 
+@pytest.mark.parametrize("reserved", [False, True])
+@pytest.mark.parametrize("Lq,H,Lk", [(736, 12, 2208), (1408, 4, 4224), (3000, 24, 640)])   # 128-query tiles in three and four parts; shares
+def test_a_recorded_launch_is_divided_as_an_ordinary_one(gpu, Lq, H, Lk, reserved):
+    """Under the automatic choice, after a warm-up or a reserve call on the stream: the eager bits, at every replay."""
+    assert _native.attention_plan(Lq, H, Lk)["division"] == "split"
+    q, k, v = (_randn((n, H, 128), s).to(gpu) for n, s in ((Lq, 94), (Lk, 95), (Lk, 96)))
+    eager = _native.attention_bf16(q, k, v, 128 ** -0.5)
+    with _native.attention_policy("narrow"):
+        assert not torch.equal(_native.attention_bf16(q, k, v, 128 ** -0.5), eager)   # whole tiles add up in another order
+    side, graph = torch.cuda.Stream(device=gpu), torch.cuda.CUDAGraph()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        _native.attention_reserve(Lq, H, Lk) if reserved else _native.attention_bf16(q, k, v, 128 ** -0.5)
+    side.synchronize()
+    with torch.cuda.graph(graph, stream=side):
+        out = _native.attention_bf16(q, k, v, 128 ** -0.5)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager)
+        _native.attention_bf16(q, k, v, 128 ** -0.5)   # ordinary work between the replays
+    del graph
+    with torch.cuda.stream(side):
+        _native.attention_release()
+
+
 @pytest.mark.parametrize("Lq,H,Lk", [(700, 2, 900), (3000, 24, 640)])   # shared 128-query and 256-query tiles
 def test_a_graph_replays_beside_ordinary_launches_of_the_stream_it_was_recorded_on(gpu, Lq, H, Lk):
     """Recorded launches have memory of their own: replays on one stream and ordinary launches on the recording's stream, at

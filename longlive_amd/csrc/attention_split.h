@@ -247,8 +247,12 @@ inline AttentionPlan plan_attention(int64_t Lq, int H, int64_t n_keys, int cus, 
 //    512 x 4, 1024 + 512                        24.5 (2) 21.1 (3) 19.3 (4) 20.9 (5) 19.6 (6) 19.5 (8) 22.1 (12)
 //    736 x 12, 0 + 512                          17.6 (2) 18.0 (3)                   [15.6 / 25.1]
 // Two rounds of parts (880 x 24, 0.88 k + 880: 47.5 with three parts) lose against whole tiles (38.2).
+// Iterations take longer as the last tenth of the compute units joins in, which decides over long ranges; there shares of
+// 256-query tiles are ahead, most of all where four of them make up a tile and none crosses to the next (us, two parts / shares):
+// 2624 x 6 over 10496 107.4 / 103.1, 3200 x 5 over 9600 99.4 / 96.7, 1936 x 8 over 7744 84.1 / 80.8, 2000 x 8 over 8946 90.8 / 88.8,
+// but 2624 x 6 over 6471 71.6 / 73.1, 1000 x 16 over 5000 58.8 / 60.4.
 inline double plan_narrow_split(int64_t Lq, int H, int64_t n_keys, int cus, AttentionPlan& plan) {
-  constexpr double kRound = 4.0, kExchange = 2.5, kPerPart = 0.5;
+  constexpr double kRound = 4.0, kExchange = 2.5, kPerPart = 0.5, kFullChip = 0.8, kSpared = 1.0;
   const int64_t n_iter = (n_keys + 127) / 128, nq = (Lq + 127) / 128, tiles = H * nq;
   int64_t parts = 0;
   double best = 1e300;
@@ -268,19 +272,24 @@ inline double plan_narrow_split(int64_t Lq, int H, int64_t n_keys, int cus, Atte
   plan.d.G = (uint32_t)(tiles * parts);
   plan.d.n_iter = (uint32_t)n_iter;
   plan.split_tiles = tiles;
-  return best;
+  const double longer = kFullChip * ((double)(tiles * parts) / cus - 0.9) * (double)((n_iter + parts - 1) / parts);
+  return best + (longer > kSpared ? longer - kSpared : 0.0);
 }
 
 // The division of a launch that the short kernel does not take, under `policy`.  The split division has tiles of 128 queries
 // where these are the cheapest division of all under the automatic choice.
 inline AttentionPlan plan_division(int64_t Lq, int H, int64_t n_cached, int64_t n_new, int cus, int policy, bool allow_split = true) {
-  constexpr double kCrossing = 5.0;  // what shares that cross 256-query tiles cost beyond plan_attention's estimate (40 instead of 30 us on the first shape above)
+  // What shares of 256-query tiles cost beyond plan_attention's estimate: where they cross tiles (40 instead of 30 us on the
+  // first shape above), and where up to four of them make up each tile.
+  constexpr double kCrossing = 5.0, kWhole = 4.5;
   double cost = 0.0;
   const AttentionPlan plan = plan_attention(Lq, H, n_cached + n_new, cus, policy == 2 ? -1 : policy, allow_split, &cost);
   const bool may_split = policy == 2 /* LL_ATTENTION_SPLIT */ || (policy == -1 /* LL_ATTENTION_AUTO */ && allow_split);
   if (may_split && !short_kernel_waves(Lq, H, n_cached, n_new, cus, -1)) {
     AttentionPlan narrow;
-    if (plan_narrow_split(Lq, H, n_cached + n_new, cus, narrow) < cost + (plan.mode == 2 ? kCrossing : 0.0)) return narrow;
+    const bool whole = plan.mode == 2 && plan.d.whole_rounds == 0 && plan.d.extra == 0 && plan.d.full_units == plan.d.units &&
+                       plan.d.G % plan.split_tiles == 0 && plan.d.G <= 4 * plan.split_tiles;
+    if (plan_narrow_split(Lq, H, n_cached + n_new, cus, narrow) < cost + (plan.mode != 2 ? 0.0 : whole ? kWhole : kCrossing)) return narrow;
   }
   return policy == 2 ? plan_attention(Lq, H, n_cached + n_new, cus, policy, allow_split) : plan;
 }

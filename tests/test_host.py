@@ -314,6 +314,15 @@ def test_plan_weighs_cached_and_fresh_keys_as_the_launch_does(Lq, H, keys, fresh
         _native.attention_plan(Lq, H, keys, n_cached=keys + 1)
 
 
+@pytest.mark.parametrize("Lq,H,keys,tiles", [
+    (1968, 8, 9840, 64), (1936, 8, 7744, 64), (2624, 6, 10496, 66), (3200, 5, 9600, 65),     # long ranges over the whole chip: 256 queries
+    (736, 12, 2208, 72), (2624, 6, 6471, 126), (1000, 16, 5000, 128), (3520, 2, 10560, 56),  # 128 queries
+    (256, 5, 6294, 10), (1280, 1, 6400, 10)])                                                # a few 256-query tiles would be cut into dozens of parts
+def test_line_between_shared_tiles_of_128_and_256_queries(Lq, H, keys, tiles):
+    plan = _native.attention_plan(Lq, H, keys)
+    assert plan["division"] == "split" and plan["whole_rounds"] == 0 and plan["split_tiles"] == tiles
+
+
 def _check_division(plan, tiles):
     """Every (tile, iteration) in exactly one segment; whole tiles first; the parts of a split tile held by exactly
     the workgroups parts_of_tile names, one part each, in records no two parts share; at most two partial tiles

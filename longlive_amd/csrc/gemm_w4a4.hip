@@ -117,8 +117,10 @@ struct GemmGroups {
 // Epilogue of one wave: acc[g][f][r] holds output row m = row_base + 32 f + lane % 32 and output column
 // n = col_base + 32 g + 8 (r / 4) + 4 (lane / 32) + r % 4.  The wave transposes one 32-row slab at a time through its
 // own LDS patch (the stages of the main loop are free by now) and writes rows with coalesced 16-byte stores.  BATCH: rows of
-// the residual and the gate under way, as many as the kernel has registers for: with 4 the hand-scheduled tiles spill 12 to 19
-// registers and lose 0.5 to 2.5 us (asm8: 2640 x 3072 x 3072 47 / 50).
+// the residual and the gate under way, as many as are measured to pay: with 4 the hand-scheduled tiles spill 12 to 19
+// registers and lose 0.5 to 2.5 us (asm8: 2640 x 3072 x 3072 47 / 50).  The persistent kernel, whose 4 x 4 fragments leave none
+// to spare (253 spilled), takes 2: 2640 x 3072 x 3072 89 us, with gate and residual 97.5 (with 4 96 and 110.5; 7040 x 3072 x 14336
+// 568 and 676, with 4 607 and 785).
 template <int FA, int FB, int BATCH>
 __device__ __forceinline__ void gemm_epilogue(float16v (&acc)[FB][FA], float alpha, uint8_t* smem, int wave, int lane, int row_base,
                                               int col_base, int M, int N, uint16_t* __restrict__ D, int64_t ldd,
@@ -223,7 +225,12 @@ __device__ __forceinline__ void gemm_epilogue(float16v (&acc)[FB][FA], float alp
     __builtin_amdgcn_wave_barrier();
   }
   if (epi.sink.parts) {  // one atomic per wave
-    out_max = wave_max(out_max);
+    if constexpr (FA * FB == 16) {  // by permutes: the moves of wave_max cost that kernel 70 more spilled registers and 6 to 10 %
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) out_max = fmaxf(out_max, __shfl_xor(out_max, o, 64));
+    } else {
+      out_max = wave_max(out_max);
+    }
     if (lane == 0) amax_sink_update(epi.sink, sink_slot, out_max);
   }
 }
@@ -743,7 +750,7 @@ __global__ __launch_bounds__(256) void gemm_w4a4_persistent_kernel(PersistentPar
       const float alpha = pr.alpha ? pr.alpha[0] : (p.amax_a[0] * pr.amax_b[0]) * (p.inv_denom_a * pr.inv_denom_b);
       GemmEpilogue epi = p.epi;
       epi.sink = pr.sink;
-      gemm_epilogue<4, 4, 4>(acc, alpha, smem, wave, lane, row0, col0 + 128 * wave, p.M, p.N, pr.D, pr.ldd, pr.bias, epi.act, epi,
+      gemm_epilogue<4, 4, 2>(acc, alpha, smem, wave, lane, row0, col0 + 128 * wave, p.M, p.N, pr.D, pr.ldd, pr.bias, epi.act, epi,
                           seg.tile * 4 + wave);
     }
   }

@@ -183,7 +183,8 @@ template <int RULE, int MODE>
 static int launch_rule(NormQuantParams& p, hipStream_t stream, bool* fits) {
   // One row per wave, three waves per SIMD.  Variants that keep two or four rows per wave (and so take more rows
   // than the device holds waves) were measured: at 7040 rows the kernel then takes as long as the two separate
-  // kernels (36 us), at two waves per SIMD, so those shapes are left to the separate operations.
+  // kernels (36 us), at two waves per SIMD, so those shapes are left to the separate operations.  Of the steps of
+  // LL_BY_ROW_LENGTH the even ones: the second half of the kernel takes a lane's groups in pairs.
   if (p.C <= 64 * 2 * 8) return launch_with<RULE, MODE, 2>(p, stream, fits);
   if (p.C <= 64 * 4 * 8) return launch_with<RULE, MODE, 4>(p, stream, fits);
   return launch_with<RULE, MODE, kNqChunks>(p, stream, fits);

@@ -26,7 +26,10 @@ __device__ __forceinline__ uint4 pack8(const float (&f)[8]) {
 
 // Row kernels: one wave per row (no workgroup barrier; a row's sums are wave reductions), four rows per
 // workgroup.  A lane holds NCH groups of 8 elements: NCH = 6 covers C = 3072 exactly, 16 anything up to 8192; groups that a row
-// does not have cost their loads and the sum all the same, hence kernels for shorter rows.
+// does not have cost their loads and the sum all the same, and their registers waves per SIMD, hence kernels for shorter rows in
+// steps of a third or less.  us, with kernels of 1, 3, 6, 10 and 16 groups / with these: LayerNorm 7040 x 1024 7.25 / 6.9, 7040 x 2048
+// 12.1 / 11.3, 7040 x 4096 24.0 / 20.7, 7040 x 6144 50.4 / 31.6; adaLN 736 x 2048 4.7 / 4.4, 736 x 6144 10.25 / 9.0; RMSNorm 2640 x 6144
+// 14.0 / 11.8.
 constexpr int kRowThreads = 256;
 constexpr int kRowsPerWg = kRowThreads / 64;
 constexpr int kMaxChunks = 16;  // 8 elements each: C <= 64 * 16 * 8 = 8192
@@ -34,12 +37,22 @@ constexpr int kMaxRowLength = 64 * kMaxChunks * 8;
 #define LL_BY_ROW_LENGTH(C, LAUNCH) \
   if ((C) <= 64 * 1 * 8) {          \
     LAUNCH(1);                      \
+  } else if ((C) <= 64 * 2 * 8) {   \
+    LAUNCH(2);                      \
   } else if ((C) <= 64 * 3 * 8) {   \
     LAUNCH(3);                      \
+  } else if ((C) <= 64 * 4 * 8) {   \
+    LAUNCH(4);                      \
   } else if ((C) <= 64 * 6 * 8) {   \
     LAUNCH(6);                      \
+  } else if ((C) <= 64 * 8 * 8) {   \
+    LAUNCH(8);                      \
   } else if ((C) <= 64 * 10 * 8) {  \
     LAUNCH(10);                     \
+  } else if ((C) <= 64 * 12 * 8) {  \
+    LAUNCH(12);                     \
+  } else if ((C) <= 64 * 14 * 8) {  \
+    LAUNCH(14);                     \
   } else {                          \
     LAUNCH(kMaxChunks);             \
   }
@@ -54,6 +67,18 @@ __device__ __forceinline__ void load_row(const uint16_t* __restrict__ row, int n
 #pragma unroll
   for (int i = 0; i < NCH; ++i) raw[i] = *reinterpret_cast<const uint4*>(row + min(lane + i * 64, nchunks - 1) * 8);
 }
+// The operands of a row (weight and bias, scale and shift) are asked for with it where that leaves two waves per SIMD or more, and
+// else kLateGroups groups at a time where they are used (us, all ahead in one wave per SIMD / so: adaLN 2640 x 7168 32.8 / 22.1, 7040 x
+// 7168 67.5 / 42.0).
+template <int NCH>
+constexpr bool kOperandsAhead = NCH <= 12;
+constexpr int kLateGroups = 4;
+template <int NCH>
+__device__ __forceinline__ void load_late(const uint16_t* __restrict__ row, int nchunks, int lane, int group, uint4 (&raw)[NCH]) {
+  if (kOperandsAhead<NCH> || group % kLateGroups != 0) return;
+#pragma unroll
+  for (int i = group; i < min(group + kLateGroups, NCH); ++i) raw[i] = *reinterpret_cast<const uint4*>(row + min(lane + i * 64, nchunks - 1) * 8);
+}
 // As floats, zeros behind the row's end; the lane's sum of them.  No branch and no choice here, into which a load would sink.
 template <int NCH>
 __device__ __forceinline__ float unpack_row(const uint4 (&raw)[NCH], int nchunks, int lane, float (&v)[NCH][8]) {
@@ -67,7 +92,6 @@ __device__ __forceinline__ float unpack_row(const uint4 (&raw)[NCH], int nchunks
   }
   return sum;
 }
-
 // adaLN modulation of one row, utils/adaln_triton.py:36-86: LayerNorm without affine in fp32, rounded to bf16,
 // times (1 + scale) rounded, plus shift rounded.  `packed[i]` receives the 8 results of group lane + 64 i; the
 // return value is the lane's share of the row's absolute maximum.  Two values share a rounding's conversion: adaln_kernel took
@@ -80,8 +104,10 @@ __device__ __forceinline__ float adaln_row(const uint16_t* __restrict__ xr, cons
   float v[NCH][8];
   uint4 xraw[NCH], sraw[NCH], hraw[NCH];
   load_row<NCH>(xr, nchunks, lane, xraw);
-  load_row<NCH>(scr, nchunks, lane, sraw);
-  load_row<NCH>(shr, nchunks, lane, hraw);
+  if (kOperandsAhead<NCH>) {
+    load_row<NCH>(scr, nchunks, lane, sraw);
+    load_row<NCH>(shr, nchunks, lane, hraw);
+  }
   __builtin_amdgcn_sched_barrier(0);  // all loads are under way
   const float sum = unpack_row<NCH>(xraw, nchunks, lane, v);
   const float inv_c = 1.0f / (float)C;
@@ -104,6 +130,8 @@ __device__ __forceinline__ float adaln_row(const uint16_t* __restrict__ xr, cons
 #pragma unroll
   for (int i = 0; i < NCH; ++i) {
     packed[i] = make_uint4(0u, 0u, 0u, 0u);
+    load_late<NCH>(scr, nchunks, lane, i, sraw);
+    load_late<NCH>(shr, nchunks, lane, i, hraw);
     if (i * 64 < nchunks) {
       float s8[8], h8[8], y[8];
       unpack8(sraw[i], s8);
@@ -148,8 +176,8 @@ __device__ __forceinline__ float layernorm_row(const uint16_t* __restrict__ xr, 
     braw[i] = make_uint4(0u, 0u, 0u, 0u);
   }
   load_row<NCH>(xr, nchunks, lane, xraw);
-  if (w) load_row<NCH>(w, nchunks, lane, wraw);
-  if (b) load_row<NCH>(b, nchunks, lane, braw);
+  if (kOperandsAhead<NCH> && w) load_row<NCH>(w, nchunks, lane, wraw);
+  if (kOperandsAhead<NCH> && b) load_row<NCH>(b, nchunks, lane, braw);
   __builtin_amdgcn_sched_barrier(0);  // all loads are under way
   const float sum = unpack_row<NCH>(xraw, nchunks, lane, v);
   const float inv_c = 1.0f / (float)C;
@@ -172,6 +200,8 @@ __device__ __forceinline__ float layernorm_row(const uint16_t* __restrict__ xr, 
 #pragma unroll
   for (int i = 0; i < NCH; ++i) {
     packed[i] = make_uint4(0u, 0u, 0u, 0u);
+    if (w) load_late<NCH>(w, nchunks, lane, i, wraw);
+    if (b) load_late<NCH>(b, nchunks, lane, i, braw);
     if (i * 64 < nchunks) {
       float w8[8], b8[8], y[8];
       unpack8(wraw[i], w8);

@@ -301,6 +301,34 @@ def test_layer_norm_against_oracle_and_torch(gpu, L, C, affine):
     assert torch.equal(xq_sink.values, xq_pass.values)
 
 
+@pytest.mark.parametrize("groups", [1, 2, 3, 4, 6, 8, 10, 12, 14, 16])
+def test_row_kernels_at_the_ends_of_their_row_lengths(gpu, groups):
+    """The longest row of each row kernel and, where there is one, the shortest of the next: RMSNorm, LayerNorm and adaLN
+    against fp64 with the bounds above, and q's norm and rotation against the separate kernels bit for bit."""
+    import dit_oracle
+
+    L = 6
+    for C in {512 * groups, min(512 * groups + 8, 8192)}:
+        x, w = _randn((1, L, C), C, 3.0) + 0.5, _randn((C,), C + 1, 0.2) + 1.0
+        b, sc, sh = _randn((C,), C + 2, 0.3), _randn((1, 2, 1, C), C + 3), _randn((1, 2, 1, C), C + 4)
+        f = lambda t: t.float().cpu().numpy()
+        got = f(_native.layer_norm(x.to(gpu), w.to(gpu), b.to(gpu), 1e-6))[0]
+        ref = dit_oracle.layer_norm_affine(f(x)[0], f(w), f(b), 1e-6)
+        assert (np.abs(got - ref) <= np.abs(ref) * 2.0 ** -7 + 4e-6 * (np.abs(f(b)) + 6.0 * np.abs(f(w)))[None, :]).all()
+        got = f(adaln_modulate(x.to(gpu), sc.to(gpu), sh.to(gpu), L // 2))[0]
+        ref, shift = o.adaln_modulate(f(x)[0], f(sc)[0, :, 0], f(sh)[0, :, 0], L // 2), np.abs(f(sh)[0, :, 0]).repeat(L // 2, 0)
+        # a step of bf16 in the normalized value, in its product and in the result
+        diff = np.abs(got - ref)
+        assert (diff <= 2.0 ** -7 * (3 * np.abs(ref) + 2 * shift)).all() and (diff != 0).mean() < 5e-3
+        normed = _native.rms_norm(x[0].to(gpu), w.to(gpu), 1e-6)
+        diff = np.abs(f(normed) - o.rms_norm(f(x)[0], f(w)))
+        assert diff.max() <= 2 ** -5 and (diff != 0).mean() < 5e-3
+        if C % 128 == 0:
+            cos, sin = rope_cos_sin(build_rope_angles(128), 1, 2, 3, 0, gpu)
+            want = rope_apply(normed.view(L, C // 128, 128), cos, sin)
+            assert torch.equal(_native.qk_norm_rope(x[0].to(gpu), w.to(gpu), 1e-6, cos, sin, C // 128), want)
+
+
 def _tile_samples(Lq, H, n_keys):
     """(kind, head, query rows) samples chosen from the launcher's own plan for a shape: a tile that one workgroup
     runs whole, a tile whose parts two or more workgroups compute and one of them combines, and a head's last,

@@ -36,6 +36,7 @@ enum {
 
 enum { LL_RULE_STATIC_6 = 0, LL_RULE_STATIC_4 = 1, LL_RULE_MAE = 2, LL_RULE_MSE = 3, LL_RULE_ABS_MAX = 4 };
 enum { LL_ACT_NONE = 0, LL_ACT_GELU_TANH = 1 };
+#define LL_EXCHANGE_LOOKS 320 /* spin_limit of launches whose workgroups exchange their maxima: 110 to 260 us */
 #define LL_AMAX_PARTS 1024 /* partial maxima per tensor: size of the quantizer's scratch and of an amax sink */
 enum { LL_DTYPE_BF16 = 0, LL_DTYPE_F16 = 1, LL_DTYPE_F32 = 2 }; /* utils/kernel/kv_dequant.py:18-25 */
 
@@ -447,9 +448,9 @@ int ll_layer_norm(const void* x, int64_t rows, int C, const void* weight, const 
  * byte for byte what the two calls give (M = B * L rows, Mp = M rounded up to 128).  The launch is one resident
  * grid whose workgroups exchange their maxima through amax_sink (required: a buffer of LL_AMAX_PARTS slots and a
  * fresh epoch, as for ll_adaln_modulate_amax; nothing has to read it afterwards).  A workgroup waits for the others
- * at most spin_limit + 1 looks at the slots (one to two microseconds each; with the device to itself a launch's
- * workgroups arrive within ~10 us of each other, and 64 is plenty) and then computes the maxima of the rows of the
- * workgroups it has not seen itself, so the launch ends whatever else occupies the device (another stream may hold
+ * at most spin_limit + 1 looks at the slots (0.35 us each with up to 64 workgroups, 0.55 with 256, 0.8 with 512; with
+ * the device to itself a launch's workgroups arrive within ~10 us of each other, and LL_EXCHANGE_LOOKS is plenty) and
+ * then computes the maxima of the rows of the workgroups it has not seen itself, so the launch ends whatever else occupies the device (another stream may hold
  * compute units for milliseconds) and costs at most one extra pass over the rows; spin_limit < 0 makes every
  * workgroup do that (tests of that path).  LL_ENOSUP when C is not a multiple of 64 or exceeds 3072, or when the
  * device does not hold one wave per row of Mp at once (3072 rows on 256 compute units; with more rows per wave the

@@ -21,8 +21,8 @@ HEADER_PATH = os.path.join(os.path.dirname(_HERE), "include", "ll_nvfp4.h")
 RULE_IDS = {"static_6": 0, "static_4": 1, "mae": 2, "mse": 3, "abs_max": 4}
 # e2m1_max * e4m3_max of a scale rule: what the tensor amax is divided by
 DENOMINATORS = {"static_6": 2688.0, "static_4": 1792.0, "mae": 1536.0, "mse": 1536.0, "abs_max": 1536.0}
-# looks (1-2 us each) a workgroup of a launch whose workgroups exchange their maxima waits for the others
-NORM_QUANTIZE_SPIN_LIMIT = 64
+# LL_EXCHANGE_LOOKS: looks a workgroup of a launch whose workgroups exchange their maxima waits for the others
+NORM_QUANTIZE_SPIN_LIMIT = 320
 DTYPE_CODES = {torch.bfloat16: 0, torch.float16: 1, torch.float32: 2}
 ACTIVATION_IDS = {"gelu_tanh": 1}
 

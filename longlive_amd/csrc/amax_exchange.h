@@ -20,7 +20,8 @@ struct AmaxExchangeSmem {
 // this workgroup's share; `slot` < G <= kAmaxParts: this workgroup's slot; `share_max(s)`: the calling thread's
 // part of the maximum of the share of workgroup s, evaluated by all threads of the workgroup together (uniform
 // control flow) when s is missing.  spin_limit + 1 looks at most; `everything`: skip the wait and compute all
-// shares (tests of that path).  Returns the tensor maximum.
+// shares (tests of that path).  Returns the tensor maximum.  us a look, by slots: up to 64 0.35, 192 0.48, 256 0.55,
+// 512 0.81, 672 0.51, 768 0.59 (words of slots that have all arrived are not looked at again).
 template <class ShareMax>
 __device__ __forceinline__ float exchange_amax(const AmaxSink& sink, uint32_t G, uint32_t slot, float thread_part,
                                                uint32_t spin_limit, bool everything, AmaxExchangeSmem& sm,

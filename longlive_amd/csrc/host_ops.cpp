@@ -158,7 +158,6 @@ Epochs epochs_of_stream(int dev, void* stream) {
 }
 
 // The amax of x and its quantization: one launch for a small tensor, two otherwise and while the stream is being captured.
-constexpr int64_t kSpinLimit = 64;  // looks of one to two microseconds at the other workgroups' maxima
 inline bool one_pass_tiles(int64_t M, int64_t K) { return K % 64 == 0 && ((M + 127) / 128) * (K / 64) <= 512; }
 int quantize_operand(const void* x, int64_t M, int64_t K, int64_t ldx, int rule, uint8_t* values, uint8_t* scales, float* amax,
                      float* workspace, int dev, void* stream) {
@@ -167,7 +166,7 @@ int quantize_operand(const void* x, int64_t M, int64_t K, int64_t ldx, int rule,
     if (e.parts) {
       const ll_amax_sink sink = e.take();
       const int code = ll_nvfp4_quantize_one_pass(x, nullptr, M, K, ldx, rule, values, nullptr, scales, nullptr, amax, nullptr, &sink,
-                                                  kSpinLimit, stream);
+                                                  LL_EXCHANGE_LOOKS, stream);
       if (code != LL_ENOSUP) return code;
     }
   }
@@ -734,7 +733,7 @@ PyObject* py_cache_write(PyObject*, PyObject* const* args, Py_ssize_t n) {
       if (e.parts) {
         const ll_amax_sink sink = e.take();
         code = ll_nvfp4_quantize_one_pass(kx, vx, M, 128, 128, rule, out[0][0], out[1][0], out[0][1], out[1][1], amax[0], amax[1], &sink,
-                                          kSpinLimit, stream);
+                                          LL_EXCHANGE_LOOKS, stream);
       }
     }
     if (code == LL_ENOSUP) {

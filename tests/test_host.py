@@ -25,6 +25,16 @@ def test_library_loads_and_exports_every_declared_symbol():
     assert lib.ll_nvfp4_quantize_workspace_floats() == 1024
 
 
+def test_both_host_paths_wait_for_as_many_looks():
+    """The bounded wait of launches whose workgroups exchange their maxima: a look has taken 0.35 us or more, and the wait
+    is to outlast the 170 us that 64 looks at 768 slots, one load after the other, once took (0.59 us each now)."""
+    import re
+    with open(_native.HEADER_PATH) as f:
+        looks = int(re.search(r"#define LL_EXCHANGE_LOOKS (\d+)", f.read()).group(1))
+    assert _native.NORM_QUANTIZE_SPIN_LIMIT == looks
+    assert looks * 0.35 >= 64 * 0.46 and looks * 0.55 >= 64 * 1.02 and looks * 0.81 >= 64 * 1.76 and looks * 0.59 >= 64 * 2.52
+
+
 def test_c_abi_rejects_bad_arguments_without_touching_the_gpu():
     lib = _native.load()
     assert lib.ll_nvfp4_quantize(None, 1, 1, 1, 3, None, None, None, 0, None, None) == -1

@@ -48,9 +48,6 @@ constexpr int kVTileBytes = kTileKeys * kVPitch;
 constexpr int kStageBytes = 2 * kKTileBytes + 2 * kVTileBytes;
 constexpr int kMaxSlots = 64;
 constexpr int kAttnThreads = 512;
-// A workgroup's partial result: per wave 64 (256-query tiles) or 32 (128) O^T registers, reference point and row sum, per lane.
-inline size_t partial_records(const AttentionPlan& plan) { return (plan.queries == 128 ? 1 : 2) * (size_t)plan.d.G; }
-constexpr size_t partial_bytes(int queries) { return (size_t)8 * (queries / 4 + 2) * 64 * sizeof(float); }
 
 struct AttnParams {
   const uint16_t* q;

@@ -235,6 +235,11 @@ inline AttentionPlan plan_attention(int64_t Lq, int H, int64_t n_keys, int cus, 
   return plan;
 }
 
+// The memory of a split division.  A workgroup's partial result: per wave 64 (256-query tiles) or 32 (128) O^T registers, reference
+// point and row sum, per lane; a share of 256-query tiles may end one tile and begin another.
+constexpr size_t partial_bytes(int queries) { return (size_t)8 * (queries / 4 + 2) * 64 * sizeof(float); }
+inline size_t partial_records(const AttentionPlan& plan) { return (plan.queries == 128 ? 1 : 2) * (size_t)plan.d.G; }
+
 // Split division with tiles of 128 queries: the key range of every tile shared by the same number of workgroups (`parts`), all
 // in one round, each with one run of iterations.  Returns its cost in iterations of the 128-query kernel, 2 us each.  us, by
 // parts (in brackets: whole 128-query tiles / shares of 256-query tiles, which cross tiles and then pay for two prologues,

@@ -60,8 +60,8 @@ extern "C" uint32_t ll_test_attention_record(uint32_t g, uint32_t split_tile, co
   return ll::record_of_part(g, split_tile, division_of(division));
 }
 
-// The launcher's whole choice for a shape: out = mode, n_qtiles, full_qtiles, split_tiles, then the division's
-// seven numbers.
+// The divisions with 256-query tiles and the whole 128-query tiles (plan_attention), of which the launcher's choice is one unless
+// it shares 128-query tiles: out = mode, n_qtiles, full_qtiles, split_tiles, then the division's seven numbers.
 extern "C" void ll_test_attention_full_plan(int64_t Lq, int H, int64_t n_keys, int cus, int policy, uint32_t* out) {
   const ll::AttentionPlan plan = ll::plan_attention(Lq, H, n_keys, cus, policy);
   out[0] = (uint32_t)plan.mode;
@@ -71,6 +71,22 @@ extern "C" void ll_test_attention_full_plan(int64_t Lq, int H, int64_t n_keys, i
   const uint32_t d[7] = {plan.d.G, plan.d.whole_rounds, plan.d.extra, plan.d.n_iter, plan.d.units, plan.d.full_units, plan.d.light};
   for (int i = 0; i < 7; ++i) out[4 + i] = d[i];
 }
+
+// The launcher's whole choice for a shape: out = waves of the short kernel (then the rest is 0), mode, queries per tile, parts per
+// tile, workgroups, iterations, tiles in parts or shares, records and bytes of each.
+extern "C" void ll_test_attention_launch(int64_t Lq, int H, int64_t n_cached, int64_t n_new, int cus, int policy, int64_t* out) {
+  for (int i = 0; i < 9; ++i) out[i] = 0;
+  out[0] = ll::short_kernel_waves(Lq, H, n_cached, n_new, cus, policy);
+  if (out[0]) return;
+  const ll::AttentionPlan plan = ll::plan_division(Lq, H, n_cached, n_new, cus, policy);
+  const int64_t v[8] = {plan.mode, plan.queries, plan.parts, plan.d.G, plan.d.n_iter, plan.split_tiles, 0, 0};
+  for (int i = 0; i < 8; ++i) out[1 + i] = v[i];
+  if (plan.mode == 2) {
+    out[7] = (int64_t)ll::partial_records(plan);
+    out[8] = (int64_t)ll::partial_bytes(plan.queries);
+  }
+}
+extern "C" int ll_test_attention_part(uint32_t part, uint32_t parts, int n_iter) { return ll::first_iteration_of_part(part, parts, n_iter); }
 
 // The same arithmetic evaluated on the device: out[g] = first_unit_of(g) for g = 0 .. G, then for every split tile
 // its first and last holder (2 * split_tiles numbers).  Returns 0, -2 when the launch fails.

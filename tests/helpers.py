@@ -124,7 +124,7 @@ def attention_record(g: int, split_tile: int, division: dict) -> int:
 
 
 def attention_full_plan(Lq: int, H: int, n_keys: int, cus: int = 256, policy: int = -1) -> dict:
-    """The launcher's choice for a shape, division included: mode (0 narrow, 1 wide, 2 split), n_qtiles,
+    """The division of a shape into 256-query tiles or whole 128-query tiles: mode (0 narrow, 1 wide, 2 split), n_qtiles,
     full_qtiles, split_tiles and the keys of DIVISION_FIELDS."""
     import ctypes
 
@@ -137,6 +137,30 @@ def attention_full_plan(Lq: int, H: int, n_keys: int, cus: int = 256, policy: in
     plan = dict(mode=out[0], n_qtiles=out[1], full_qtiles=out[2], split_tiles=out[3])
     plan.update({k: out[4 + i] for i, k in enumerate(DIVISION_FIELDS)})
     return plan
+
+
+def attention_launch(Lq: int, H: int, n_cached: int, n_new: int, cus: int = 256, policy: int = -1) -> dict:
+    """The launcher's whole choice for a shape: short (waves of the short kernel, or 0 and the rest), mode, queries and parts per
+    tile, G, n_iter, split_tiles, records, record_bytes."""
+    import ctypes
+
+    lib = _test_hooks()
+    lib.ll_test_attention_launch.restype = None
+    lib.ll_test_attention_launch.argtypes = [ctypes.c_int64, ctypes.c_int, ctypes.c_int64, ctypes.c_int64, ctypes.c_int, ctypes.c_int,
+                                             ctypes.c_void_p]
+    out = (ctypes.c_int64 * 9)()
+    lib.ll_test_attention_launch(Lq, H, n_cached, n_new, cus, policy, out)
+    return dict(zip(("short", "mode", "queries", "parts", "G", "n_iter", "split_tiles", "records", "record_bytes"), out))
+
+
+def attention_part(part: int, parts: int, n_iter: int) -> int:
+    """First iteration of a part of a 128-query tile's key range."""
+    import ctypes
+
+    lib = _test_hooks()
+    lib.ll_test_attention_part.restype = ctypes.c_int
+    lib.ll_test_attention_part.argtypes = [ctypes.c_uint32, ctypes.c_uint32, ctypes.c_int]
+    return lib.ll_test_attention_part(part, parts, n_iter)
 
 
 def scratch_sets(ops):

@@ -416,6 +416,38 @@ def test_attention_work_division_covers_every_iteration_exactly_once():
         _check_division(plan, rounds * G + extra + full_split + light_split)
 
 
+def test_shared_128_query_tiles_cover_every_iteration_exactly_once():
+    """The launcher's choice where it shares the key ranges of 128-query tiles, for shapes known to take it and a spread of others:
+    one round of workgroups, parts that are not empty and follow each other without a gap, records that 32-bit offsets
+    reach; and the plan query tells the same division."""
+    from helpers import attention_launch, attention_part
+
+    cases = [(736, 12, 1472, 736, 256), (2000, 6, 0, 2000, 256), (700, 2, 0, 900, 256), (3520, 2, 7040, 3520, 256), (1408, 4, 2816, 1408, 256)]
+    known, rng = len(cases), np.random.default_rng(12)
+    for _ in range(400):
+        Lq, H = int(np.exp(rng.uniform(0, 9))), int(rng.integers(1, 48))
+        cases.append((Lq, H, int(rng.choice([0, 0, 3 * Lq, rng.integers(1, 30000)])), int(rng.choice([0, 16, Lq, 5000])) + 1, int(rng.choice([8, 64, 256, 304]))))
+    seen, policies = 0, {-1: "auto", 2: "split"}
+    for i, (Lq, H, cached, fresh, cus) in enumerate(cases):
+        for policy, name in policies.items():
+            plan = attention_launch(Lq, H, cached, fresh, cus, policy)
+            if plan["short"] or plan["mode"] != 2 or plan["queries"] != 128:
+                assert i >= known
+                continue
+            seen += 1
+            tiles, parts, n_iter = H * -(-Lq // 128), plan["parts"], -(-(cached + fresh) // 128)
+            assert (plan["split_tiles"], plan["n_iter"], plan["G"]) == (tiles, n_iter, tiles * parts)
+            assert 2 <= parts <= n_iter and plan["G"] <= cus
+            at = [attention_part(p, parts, n_iter) for p in range(parts + 1)]
+            assert at[0] == 0 and at[-1] == n_iter and all(a < b for a, b in zip(at, at[1:]))
+            # workgroup (tile, part) writes record tile * parts + part: 8 waves of 32 + 2 registers of 64 lanes
+            assert plan["records"] == plan["G"] and plan["record_bytes"] == 8 * 34 * 64 * 4
+            assert plan["records"] * plan["record_bytes"] < 1 << 32
+            told = _native.attention_plan(Lq, H, cached + fresh, cus, name, n_cached=cached)
+            assert told == {"division": "split", "workgroups": plan["G"], "whole_rounds": 0, "split_tiles": tiles}
+    assert seen > 60
+
+
 def test_recorded_and_ordinary_launches_never_share_memory():
     """A graph may be replayed on another stream beside ordinary launches of the stream it was recorded on."""
     from helpers import scratch_sets

@@ -276,10 +276,13 @@ int ll_nvfp4_gemm_plan(int64_t M, int64_t N, int64_t Kp, int n_products, int com
  * only; a persistent launch on a capturing stream without memory falls back to the tile kernels, which this does not
  * see): *kernel = one of the codes below, *hand_scheduled = 1 if its main loop is the generated instruction sequence.
  * The 128- and 256-row four-wave tile kernels add the K steps in order, and so does every kernel under
- * LL_GEMM_TILES_COMPILED; LL_GEMM_KERNEL_64X64 for Kp > 1024 (each wave a quarter of every K step; where there are few tiles and K is
- * long, K ranges that several workgroups share or, on a capturing stream or without memory, one runs through),
- * LL_GEMM_KERNEL_EIGHT_WAVES and LL_GEMM_KERNEL_PERSISTENT form partial sums over parts of K, added in a fixed order.  Output pointers may be NULL.  No counterpart in the reference. */
-#define LL_GEMM_KERNEL_64X64 0       /* four waves per workgroup, two workgroups per compute unit */
+ * LL_GEMM_TILES_COMPILED and LL_GEMM_KERNEL_64X64 for Kp <= 512.  For Kp > 512 that kernel (each wave a quarter of every
+ * K step; where there are few tiles and K is long, K ranges that several workgroups share or, on a capturing stream or
+ * without memory, one runs through), LL_GEMM_KERNEL_EIGHT_WAVES and LL_GEMM_KERNEL_PERSISTENT form partial sums over
+ * parts of K, added in a fixed order.  Output pointers may be NULL.  No counterpart in the reference. */
+#define LL_GEMM_KERNEL_64X64 0       /* four waves per workgroup, two workgroups per compute unit; for Kp >= 1024, where its
+                                        tiles are more than the units, 64 x 96 tiles if these are not, one workgroup per
+                                        unit, with the same sums */
 #define LL_GEMM_KERNEL_128X128 1
 #define LL_GEMM_KERNEL_128X256 2
 #define LL_GEMM_KERNEL_256X128 3
@@ -445,17 +448,17 @@ int ll_layer_norm(const void* x, int64_t rows, int C, const void* weight, const 
  * ll_adaln_modulate_amax followed by ll_nvfp4_quantize_from_sink of its result (the pairs at
  * wan_5b/modules/causal_model.py:869-878 and :909-918 with a quantized linear layer behind them) as one launch that
  * never writes the modulated tensor: values [Mp, C/2], scales [Mp * C / 16] in the blocked layout and amax [1] are
- * byte for byte what the two calls give (M = B * L rows, Mp = M rounded up to 128).  The launch is one resident
- * grid whose workgroups exchange their maxima through amax_sink (required: a buffer of LL_AMAX_PARTS slots and a
- * fresh epoch, as for ll_adaln_modulate_amax; nothing has to read it afterwards).  A workgroup waits for the others
- * at most spin_limit + 1 looks at the slots (0.35 us each with up to 64 workgroups, 0.55 with 256, 0.8 with 512; with
- * the device to itself a launch's workgroups arrive within ~10 us of each other, and LL_EXCHANGE_LOOKS is plenty) and
- * then computes the maxima of the rows of the workgroups it has not seen itself, so the launch ends whatever else occupies the device (another stream may hold
- * compute units for milliseconds) and costs at most one extra pass over the rows; spin_limit < 0 makes every
- * workgroup do that (tests of that path).  LL_ENOSUP when C is not a multiple of 64 or exceeds 3072, or when the
- * device does not hold one wave per row of Mp at once (3072 rows on 256 compute units; with more rows per wave the
- * launch was measured no faster than the two kernels): call the two separate entry points then.  No allocation, safe
- * under stream capture.
+ * byte for byte what the two calls give (M = B * L rows, Mp = M rounded up to 128).  The launch is one resident grid whose
+ * workgroups exchange their maxima through amax_sink (required: a buffer of LL_AMAX_PARTS slots and a fresh epoch, as for
+ * ll_adaln_modulate_amax; nothing has to read it afterwards).  A workgroup waits for the others at most spin_limit + 1
+ * looks at the slots (0.35 us each with up to 64 workgroups, 0.55 with 256, 0.8 with 512; with the device to itself a
+ * launch's workgroups arrive within ~10 us of each other, and LL_EXCHANGE_LOOKS is plenty) and then computes the maxima of
+ * the rows of the workgroups it has not seen itself, so the launch ends whatever else occupies the device (another stream
+ * may hold compute units for milliseconds) and costs at most one extra pass over the rows; spin_limit < 0 makes every
+ * workgroup do that (tests of that path).  LL_ENOSUP when C is not a multiple of 64 or exceeds 3072, or when the device
+ * does not hold one wave per row of Mp at once (3072 rows on 256 compute units; with more rows per wave the launch was
+ * measured no faster than the two kernels): call the two separate entry points then.  No allocation, safe under stream
+ * capture.
  */
 int ll_adaln_quantize(const void* x, int64_t B, int64_t L, int C, const void* scale, const void* shift,
                       int64_t scale_stride_b, int64_t scale_stride_f, int64_t shift_stride_b, int64_t shift_stride_f,

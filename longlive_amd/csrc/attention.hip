@@ -245,10 +245,10 @@ __device__ __forceinline__ uint32_t group_number(uint32_t G) {
   return G % 8 == 0 ? (b & 7) * (G / 8) + (b >> 3) : b;
 }
 
-// The wave's results O^T * inv_l (register r of o[d]: column 32 d + 8 (r / 4) + 4 lh + r % 4 of query l32), as bf16, to the first
-// `queries` of its 32 rows of 32 N columns at dst (rows H heads apart), through an LDS patch of the wave's own: whole rows per
-// store.  Straight from the registers a store reaches 16 bytes of each of 32 rows: 7040 queries x 24 heads over 512 keys 71.5 us, so
-// 63.1; 3520 x 24 46.7 / 41.2; 1760 x 12 16.3 / 15.1.  out_max: raised to the largest magnitude.
+// The wave's results O^T * inv_l (register r of o[d]: column 32 d + 8 (r / 4) + 4 lh + r % 4 of query l32), as bf16, to the
+// first `queries` of its 32 rows of 32 N columns at dst (rows H heads apart), through an LDS patch of the wave's own: whole
+// rows per store.  Straight from the registers a store reaches 16 bytes of each of 32 rows: 7040 queries x 24 heads over
+// 512 keys 71.5 us, so 63.1; 3520 x 24 46.7 / 41.2; 1760 x 12 16.3 / 15.1.  out_max: raised to the largest magnitude.
 template <int N>
 __device__ __forceinline__ void write_rows(const float16v (&o)[N], float inv_l, uint8_t* patch, int lane, uint16_t* dst, int H, int queries,
                                            float& out_max) {
@@ -357,9 +357,10 @@ __global__ __launch_bounds__(kAttnThreads) void kv_attention_kernel(AttnParams p
 #pragma unroll
     for (int ks = 0; ks < 8; ++ks) qf[ks] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(src + 16 * ks));
   } else {
-    // Four whole rows per load, into a patch of the stage that the first iteration leaves alone; the fragments are read from
-    // there behind the loads of the first tile.  Straight into the fragments a load reaches 32 bytes of each of 32 rows: 1760
-    // queries x 12 heads over 512 keys 15.1 us, so 13.9.  (256-query tiles: 2640 x 24 over 512 27.8 and 28.4, 3520 x 24 41.1 and 40.5.)
+    // Four whole rows per load, into a patch of the stage that the first iteration leaves alone; the fragments are read
+    // from there behind the loads of the first tile.  Straight into the fragments a load reaches 32 bytes of each of 32
+    // rows: 1760 queries x 12 heads over 512 keys 15.1 us, so 13.9.  (256-query tiles: 2640 x 24 over 512 27.8 and 28.4,
+    // 3520 x 24 41.1 and 40.5.)
     const auto& c = reread_params();
     const int64_t first_query = (int64_t)qtile * kQueries + qq * kWaveQueries;
     uint8_t* patch = smem + ((seg_begin & 1) ^ 1) * kStageBytes + wave * kWaveQueries * kKPitch;
@@ -762,7 +763,8 @@ __global__ __launch_bounds__(kAttnThreads) void kv_attention_kernel(AttnParams p
       const uint32_t wg = group_number(c.d.G);
       const uint32_t split_tile = (uint32_t)tile_id - c.d.whole_rounds * c.d.G - c.d.extra;  // the tile's number among the split ones
       auto record_of = [&](uint32_t g) {
-        return c.partials + (size_t)record_of_part(g, split_tile, division_of(c)) * (partial_bytes(kQueries) / sizeof(float)) + wave * (66 * 64) + lane;
+        return c.partials + (size_t)record_of_part(g, split_tile, division_of(c)) * (partial_bytes(kQueries) / sizeof(float)) +
+               wave * (66 * 64) + lane;
       };
       uint32_t g_first, g_last;
       parts_of_tile(split_tile, division_of(c), g_first, g_last);
@@ -978,10 +980,11 @@ constexpr size_t kShortLds = (size_t)W * kShortWaveBytes + sizeof(SlotTable);
 static_assert(kShortRecord * 4 <= kShortWaveBytes && kShortWaveBytes % 16 == 0, "the merge reuses the waves' rows");
 
 // amdgpu_waves_per_eu: 256 registers per lane, two waves per SIMD (one workgroup of eight or two of four per CU)
-// CACHED: there are cached keys.  The first tile's bytes are asked for with the queries (without cached keys) or as soon as the
-// slot pointers are there (with them, the slots' scales still on their way), and a tile's rows without conditions, which the
-// compiler turns into sixteen branches per tile.  us, before that / now: 368 x 16 over 1472 16.1 / 14.8, over 1104 + 368 18.7 / 18.0, 520 x
-// 24 over 1030 21.6 / 19.9, 736 x 12 over 512 12.9 / 12.0, 192 x 2 over 768 + 192 14.0 / 13.2.
+// CACHED: there are cached keys.  The first tile's bytes are asked for with the queries (without cached keys) or as soon as
+// the slot pointers are there (with them, the slots' scales still on their way), and a tile's rows without conditions,
+// which the compiler turns into sixteen branches per tile.  us, before that / now: 368 x 16 over 1472 16.1 / 14.8, over
+// 1104 + 368 18.7 / 18.0, 520 x 24 over 1030 21.6 / 19.9, 736 x 12 over 512 12.9 / 12.0, 192 x 2 over 768 + 192 14.0 /
+// 13.2.
 template <int W, bool CACHED>
 __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void kv_attention_short_kernel(AttnParams p) {
   static_assert(W == 4 || W == 8, "the merge gives every wave 64 / W of the 64 output registers");
@@ -1270,14 +1273,17 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) 
 static std::atomic<int> g_attention_policy{LL_ATTENTION_AUTO};
 
 // Short launches take kv_attention_short_kernel, under the automatic choice and where the division without shared tiles and
-// with few queries per workgroup (LL_ATTENTION_NARROW) is asked for.  For the others there are three ways, all one workgroup per compute unit at a time (LDS):
+// with few queries per workgroup (LL_ATTENTION_NARROW) is asked for.  For the others there are four ways, all one workgroup
+// per compute unit at a time (LDS):
 //  * 128 queries per workgroup, the key range halved between two sets of waves; one workgroup per tile;
 //  * 256 queries per workgroup (every decoded K/V tile serves twice as many MFMAs: an iteration takes about 1.64
 //    times as long for twice the work), one workgroup per tile;
 //  * 256 queries per workgroup, whole rounds of tiles first and the (tile, iteration) sequence of the tiles behind
 //    them cut into one equal share per compute unit; tiles that straddle two shares are combined by the workgroup
-//    that finishes last.
-// plan_attention (attention_split.h) chooses.
+//    that finishes last;
+//  * 128 queries per workgroup where there are few tiles: the same number of workgroups share the key range of each, all
+//    of them in one round, combined likewise.
+// plan_division (attention_split.h) chooses: plan_attention among the first three, then between that and the fourth.
 static int launch_attention(const AttnParams& p_in, hipStream_t stream) {
   AttnParams p = p_in;
   const size_t smem = 2 * kStageBytes + sizeof(SlotTable);
@@ -1294,9 +1300,9 @@ static int launch_attention(const AttnParams& p_in, hipStream_t stream) {
     p.n_qtiles = (int)((p.Lq + kWaveQueries - 1) / kWaveQueries);
     p.d.G = (uint32_t)(p.H * p.n_qtiles);
     static std::atomic<uint64_t> lds_allowed[4] = {};
-#define LL_LAUNCH_SHORT(W, CACHED, i)                                                                                                            \
-  if (int rc = allow_dynamic_lds(reinterpret_cast<const void*>(&kv_attention_short_kernel<W, CACHED>), kShortLds<W>, lds_allowed[i], "ll_kv_attention")) \
-    return rc;                                                                                                                                   \
+#define LL_LAUNCH_SHORT(W, CACHED, i)                                                                                      \
+  const void* kernel = reinterpret_cast<const void*>(&kv_attention_short_kernel<W, CACHED>);                               \
+  if (int rc = allow_dynamic_lds(kernel, kShortLds<W>, lds_allowed[i], "ll_kv_attention")) return rc;                      \
   hipLaunchKernelGGL((kv_attention_short_kernel<W, CACHED>), dim3(p.d.G), dim3(W * 64), kShortLds<W>, stream, p)
     if (waves == 8 && p.n_cached > 0) {
       LL_LAUNCH_SHORT(8, true, 0);
@@ -1382,8 +1388,8 @@ extern "C" int ll_kv_attention_reserve_window(int64_t Lq, int num_heads, int64_t
     return LL_ENOSUP;
   }
   StreamScratch w;
-  return stream_scratch(dev, static_cast<hipStream_t>(stream), partial_records(plan) * partial_bytes(plan.queries), (size_t)plan.split_tiles, true, w,
-                        nullptr, "ll_kv_attention_reserve");
+  return stream_scratch(dev, static_cast<hipStream_t>(stream), partial_records(plan) * partial_bytes(plan.queries),
+                        (size_t)plan.split_tiles, true, w, nullptr, "ll_kv_attention_reserve");
 }
 
 // Cached keys are the longer way through the short kernel, and one fresh key may make a tile more: where these two need no

@@ -2,14 +2,13 @@
 // launcher (host) and the host-side checks of the test suite.  Everything here is integer arithmetic on a few
 // launch-wide numbers, identical on both sides.
 //
-// A launch has tiles (head x group of queries) of n_iter iterations (128 keys each) and G workgroups.  Tiles whose
-// group of queries is full come first in the numbering, the heads' last, partly filled groups behind them: the
-// waves of such a tile that have no queries skip the matrix work, so an iteration of it costs less (`light`
-// sixteenths of a full one) when the busy waves are few enough to have a SIMD each.  Workgroup g first runs `whole_rounds` whole tiles (tile j * G + g in round j);
-// workgroups [0, extra) then run one more whole tile each (tile whole_rounds * G + g) and are done.  The tiles
-// behind those, numbered from 0 as "split tiles", are cut into units = split tiles x n_iter, and the workgroups
-// [extra, G) divide them into shares of equal cost, each cut at tile boundaries into segments and walked from the
-// end backwards.
+// A launch has tiles (head x group of queries) of n_iter iterations (128 keys each) and G workgroups.  Tiles whose group of
+// queries is full come first in the numbering, the heads' last, partly filled groups behind them: the waves of such a tile
+// that have no queries skip the matrix work, so an iteration of it costs less (`light` sixteenths of a full one) when the
+// busy waves are few enough to have a SIMD each.  Workgroup g first runs `whole_rounds` whole tiles (tile j * G + g in
+// round j); workgroups [0, extra) then run one more whole tile each (tile whole_rounds * G + g) and are done.  The tiles
+// behind those, numbered from 0 as "split tiles", are cut into units = split tiles x n_iter, and the workgroups [extra, G)
+// divide them into shares of equal cost, each cut at tile boundaries into segments and walked from the end backwards.
 #pragma once
 #include <stdint.h>
 
@@ -117,9 +116,9 @@ LL_SPLIT_FN int first_iteration_of_part(uint32_t part, uint32_t parts, int n_ite
 //   G <= 2 CUs    736 x 12, 0 + 16: 16.3 / 18.4 / 13.7; 512 x 24, 32 + 16: 34.7 / 38.3 / 32.8, but 46 + 23 on 736 x 12:
 //                 38.7 / 49.9 / 43.5;   G > 2 CUs: 736 x 24, 0 + 16: 16.8 / 26.4 / 20.5
 // A cached tile costs about half as much again as one of the chunk (conversion).  Launches of more than 256 queries per
-// head for every head take it over up to 16 tiles (3520 x 2, 0 + 16: 15.4 / 10.4 / 10.5); over more the measurements end at one point (700 queries of 2 heads over
-// 900 keys: 12.9 us here, 27.8 in 256-query tiles), and 128-query tiles that share their key ranges (plan_narrow_split) have taken
-// most of what there was to gain.
+// head for every head take it over up to 16 tiles (3520 x 2, 0 + 16: 15.4 / 10.4 / 10.5); over more the measurements end at
+// one point (700 queries of 2 heads over 900 keys: 12.9 us here, 27.8 in 256-query tiles), and 128-query tiles that share
+// their key ranges (plan_narrow_split) have taken most of what there was to gain.
 // `policy`: only the automatic choice (-1) and the division without shared tiles (0) take this kernel.  The launch, the
 // plan query and the reserve call all ask here.
 inline int short_kernel_waves(int64_t Lq, int H, int64_t n_cached, int64_t n_new, int cus, int policy) {
@@ -253,9 +252,9 @@ inline size_t partial_records(const AttentionPlan& plan) { return (plan.queries 
 //    736 x 12, 0 + 512                          17.6 (2) 18.0 (3)                   [15.6 / 25.1]
 // Two rounds of parts (880 x 24, 0.88 k + 880: 47.5 with three parts) lose against whole tiles (38.2).
 // Iterations take longer as the last tenth of the compute units joins in, which decides over long ranges; there shares of
-// 256-query tiles are ahead, most of all where four of them make up a tile and none crosses to the next (us, two parts / shares):
-// 2624 x 6 over 10496 107.4 / 103.1, 3200 x 5 over 9600 99.4 / 96.7, 1936 x 8 over 7744 84.1 / 80.8, 2000 x 8 over 8946 90.8 / 88.8,
-// but 2624 x 6 over 6471 71.6 / 73.1, 1000 x 16 over 5000 58.8 / 60.4.
+// 256-query tiles are ahead, most of all where four of them make up a tile and none crosses to the next (us, two parts /
+// shares): 2624 x 6 over 10496 107.4 / 103.1, 3200 x 5 over 9600 99.4 / 96.7, 1936 x 8 over 7744 84.1 / 80.8, 2000 x 8 over
+// 8946 90.8 / 88.8, but 2624 x 6 over 6471 71.6 / 73.1, 1000 x 16 over 5000 58.8 / 60.4.
 inline double plan_narrow_split(int64_t Lq, int H, int64_t n_keys, int cus, AttentionPlan& plan) {
   constexpr double kRound = 4.0, kExchange = 2.5, kPerPart = 0.5, kFullChip = 0.8, kSpared = 1.0;
   const int64_t n_iter = (n_keys + 127) / 128, nq = (Lq + 127) / 128, tiles = H * nq;

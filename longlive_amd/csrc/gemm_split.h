@@ -142,20 +142,20 @@ inline TileKernelChoice choose_tile_kernel(int64_t M, int64_t N, int64_t Kp, int
   // per tile, the K range of every step split between its two halves.
   if (generated_ok && Kp >= 512) {
     const int64_t tiles = ((M + 127) / 128) * ((N + 255) / 256) * n_products;
-    // ... unless the 64 x 64 tiles of the small-product kernel are no more than four and a half per unit: 1320 x 3072 x 3072, 1008
-    // of them: 28.5 against 36.8 us; x 768 12.8 / 14.9, x 14336 116 / 139; 1400 x 3072 x 3072, 1056: 34.8 / 36.7; 1760 x 2560 x 2560,
-    // 1120: 30.0 / 32.3; but 736 x 8960 x 1536, 1680: 28.6 / 23.9.
+    // ... unless the 64 x 64 tiles of the small-product kernel are no more than four and a half per unit: 1320 x 3072 x
+    // 3072, 1008 of them: 28.5 against 36.8 us; x 768 12.8 / 14.9, x 14336 116 / 139; 1400 x 3072 x 3072, 1056: 34.8 /
+    // 36.7; 1760 x 2560 x 2560, 1120: 30.0 / 32.3; but 736 x 8960 x 1536, 1680: 28.6 / 23.9.
     if (tiles <= cus && 2 * tiles > cus) {
       if (small_kernel_takes(Kp, schedule) && 2 * tiles_64 <= 9 * (int64_t)cus) return {0, false};
       return {4, true};
     }
   }
-  // Small problems: when even 128 x 128 tiles would occupy at most half of the compute units, 64 x 64 tiles (more
-  // decode work per MFMA, but four times the workgroups) finish sooner.  Up to three of them per unit they still do in the
-  // small-product kernel, since each 128 x 128 tile then has a unit to itself or shares it with one other (us, that kernel /
-  // tiles of 128 x 128): 1320 x 1536 x 1536, 504 small tiles: 10.4 / 16.1; x 640 7.5 / 9.2; 335 x 5888 x 1536, 552: 14.7 / 15.9; 1500 x
-  // 2048 x 1536, 768: 15.0 / 16.4; 1760 x 1536 x 768, 672: 10.3 / 10.3; but 2640 x 1024 x 640, 672: 10.4 / 9.6; 736 x 4608 x 1536,
-  // 864: 18.2 / 16.5; 2048 x 2048 x 8192, 1024: 72.9 / 69.6.
+  // Small problems: when even 128 x 128 tiles would occupy at most half of the compute units, 64 x 64 tiles (more decode
+  // work per MFMA, but four times the workgroups) finish sooner.  Up to three of them per unit they still do in the
+  // small-product kernel, since each 128 x 128 tile then has a unit to itself or shares it with one other (us, that kernel
+  // / tiles of 128 x 128): 1320 x 1536 x 1536, 504 small tiles: 10.4 / 16.1; x 640 7.5 / 9.2; 335 x 5888 x 1536, 552: 14.7
+  // / 15.9; 1500 x 2048 x 1536, 768: 15.0 / 16.4; 1760 x 1536 x 768, 672: 10.3 / 10.3; but 2640 x 1024 x 640, 672: 10.4 /
+  // 9.6; 736 x 4608 x 1536, 864: 18.2 / 16.5; 2048 x 2048 x 8192, 1024: 72.9 / 69.6.
   const int64_t tiles_128 = ((M + 127) / 128) * ((N * n_products + 127) / 128);
   if (tiles_128 <= cus / 2 || (small_kernel_takes(Kp, schedule) && tiles_64 <= (Kp >= 768 ? 3 : 2) * (int64_t)cus)) return {0, false};
   // Two workgroups of four waves are resident per compute unit.  The 256 x 128 / 128 x 256 tiles need 6 decode
@@ -184,9 +184,9 @@ inline TileKernelChoice choose_tile_kernel(int64_t M, int64_t N, int64_t Kp, int
 }
 
 // How the small-product kernel divides a launch: 64 x 64 tiles, each by `parts` workgroups that share its K range (steps of
-// 256 elements).  Measured when a step took 0.55 us (0.47 now) with one workgroup on every compute unit; handing two to four parts over
-// and adding them up takes 2.4 us (their records are read four at a time: five to eight 3.6); with more workgroups than
-// units a step takes 0.8 and the launch 2 us more.  us by parts:
+// 256 elements).  Measured when a step took 0.55 us (0.47 now) with one workgroup on every compute unit; handing two to
+// four parts over and adding them up takes 2.4 us (their records are read four at a time: five to eight 3.6); with more
+// workgroups than units a step takes 0.8 and the launch 2 us more.  us by parts:
 //                     tiles, steps    1     2     3     4     5     6     8    12
 //   40 x 256 x 5888       4, 23     17.6  13.9  11.8  10.7  11.0  10.9  10.0  10.6
 //   48 x 1024 x 4096     16, 16     13.7  12.0  10.8  10.2  11.8  10.3  10.8  11.9
@@ -203,10 +203,10 @@ inline TileKernelChoice choose_tile_kernel(int64_t M, int64_t N, int64_t Kp, int
 constexpr int kSmallParts = 4, kSmallPartsSteps = 16;
 constexpr int kSmallRecordBytes = 64 * 64 * 4;                            // a part's fp32 sums of its tile
 inline int64_t small_product_units(int cus) { return 2 * (int64_t)cus; }  // most (tile, part) pairs of a launch with parts
-// Tiles of 64 x 96 where those of 64 x 64 would be more than one per unit and these are not: a step takes 0.71 us against 0.9 us
-// for two of the smaller ones (us, 64 x 64 / 64 x 96: 512 x 3072 x 3072 15.2 / 13.7, 736 x 1536 x 1536 9.9 / 9.4, x 8960 33.3 / 30.5,
-// 440 x 3072 x 14336 50.4 / 45.2).  Larger ones were measured too: 64 x 128 and 96 x 128 were never ahead of both, 128 x 128 by 6 % on
-// 2048 x 2048 x 3072.
+// Tiles of 64 x 96 where those of 64 x 64 would be more than one per unit and these are not: a step takes 0.71 us against
+// 0.9 us for two of the smaller ones (us, 64 x 64 / 64 x 96: 512 x 3072 x 3072 15.2 / 13.7, 736 x 1536 x 1536 9.9 / 9.4, x
+// 8960 33.3 / 30.5, 440 x 3072 x 14336 50.4 / 45.2).  Larger ones were measured too: 64 x 128 and 96 x 128 were never ahead
+// of both, 128 x 128 by 6 % on 2048 x 2048 x 3072.
 struct SmallGemmPlan {
   int fb;  // tiles of 64 rows by 32 fb columns
   int parts;

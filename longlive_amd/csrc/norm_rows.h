@@ -24,12 +24,12 @@ __device__ __forceinline__ uint4 pack8(const float (&f)[8]) {
   return make_uint4(w[0], w[1], w[2], w[3]);
 }
 
-// Row kernels: one wave per row (no workgroup barrier; a row's sums are wave reductions), four rows per
-// workgroup.  A lane holds NCH groups of 8 elements: NCH = 6 covers C = 3072 exactly, 16 anything up to 8192; groups that a row
-// does not have cost their loads and the sum all the same, and their registers waves per SIMD, hence kernels for shorter rows in
-// steps of a third or less.  us, with kernels of 1, 3, 6, 10 and 16 groups / with these: LayerNorm 7040 x 1024 7.25 / 6.9, 7040 x 2048
-// 12.1 / 11.3, 7040 x 4096 24.0 / 20.7, 7040 x 6144 50.4 / 31.6; adaLN 736 x 2048 4.7 / 4.4, 736 x 6144 10.25 / 9.0; RMSNorm 2640 x 6144
-// 14.0 / 11.8.
+// Row kernels: one wave per row (no workgroup barrier; a row's sums are wave reductions), four rows per workgroup.  A lane
+// holds NCH groups of 8 elements: NCH = 6 covers C = 3072 exactly, 16 anything up to 8192; groups that a row does not have
+// cost their loads and the sum all the same, and their registers waves per SIMD, hence kernels for shorter rows in steps of
+// a third or less.  us, with kernels of 1, 3, 6, 10 and 16 groups / with these: LayerNorm 7040 x 1024 7.25 / 6.9, 7040 x
+// 2048 12.1 / 11.3, 7040 x 4096 24.0 / 20.7, 7040 x 6144 50.4 / 31.6; adaLN 736 x 2048 4.7 / 4.4, 736 x 6144 10.25 / 9.0;
+// RMSNorm 2640 x 6144 14.0 / 11.8.
 constexpr int kRowThreads = 256;
 constexpr int kRowsPerWg = kRowThreads / 64;
 constexpr int kMaxChunks = 16;  // 8 elements each: C <= 64 * 16 * 8 = 8192
@@ -59,17 +59,17 @@ constexpr int kMaxRowLength = 64 * kMaxChunks * 8;
 
 // The lane's groups of a row, all requested before the first is waited for; behind the row's end its last group once more.
 // (With the load of a group under a branch of its own, and its use there, the compiler waits for every group before it asks
-// for the next: a row of 3072 was six trips to memory.  us so / now, with kernels for shorter rows: RMSNorm 880 x 3072 4.8 / 3.9, LayerNorm
-// 2640 x 3072 8.5 / 7.8, adaLN 736 x 1536 4.0 / 3.6, 4096 x 5120 34.3 / 20.3, q and k 2640 x 3072 17.4 / 14.6, 4096 x 5120 42.8 / 33.5,
-// adaLN and quantization 736 x 1536 8.6 / 7.75.)
+// for the next: a row of 3072 was six trips to memory.  us so / now, with kernels for shorter rows: RMSNorm 880 x 3072 4.8
+// / 3.9, LayerNorm 2640 x 3072 8.5 / 7.8, adaLN 736 x 1536 4.0 / 3.6, 4096 x 5120 34.3 / 20.3, q and k 2640 x 3072 17.4 /
+// 14.6, 4096 x 5120 42.8 / 33.5, adaLN and quantization 736 x 1536 8.6 / 7.75.)
 template <int NCH>
 __device__ __forceinline__ void load_row(const uint16_t* __restrict__ row, int nchunks, int lane, uint4 (&raw)[NCH]) {
 #pragma unroll
   for (int i = 0; i < NCH; ++i) raw[i] = *reinterpret_cast<const uint4*>(row + min(lane + i * 64, nchunks - 1) * 8);
 }
-// The operands of a row (weight and bias, scale and shift) are asked for with it where that leaves two waves per SIMD or more, and
-// else kLateGroups groups at a time where they are used (us, all ahead in one wave per SIMD / so: adaLN 2640 x 7168 32.8 / 22.1, 7040 x
-// 7168 67.5 / 42.0).
+// The operands of a row (weight and bias, scale and shift) are asked for with it where that leaves two waves per SIMD or
+// more, and else kLateGroups groups at a time where they are used (us, all ahead in one wave per SIMD / so: adaLN 2640 x
+// 7168 32.8 / 22.1, 7040 x 7168 67.5 / 42.0).
 template <int NCH>
 constexpr bool kOperandsAhead = NCH <= 12;
 constexpr int kLateGroups = 4;

@@ -273,8 +273,9 @@ struct OnceJobs {
 constexpr uint32_t kOnceSlots = kAmaxParts / 2;  // of a tensor
 
 template <int RULE, int T>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void quantize_once_kernel(OnceJobs jobs, int64_t M, int64_t K, int64_t ldx, uint32_t tiles, AmaxSink sink,
-                                                            uint32_t spin_limit, int recompute) {
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4)))
+void quantize_once_kernel(OnceJobs jobs, int64_t M, int64_t K, int64_t ldx, uint32_t tiles, AmaxSink sink, uint32_t spin_limit,
+                          int recompute) {
   __shared__ AmaxExchangeSmem s_exchange;
   __shared__ ScaleEntry s_tab[128];
   __shared__ uint32_t s_scales[2][128];  // a tile's 128 x 4 scale bytes in blocked order
@@ -356,7 +357,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void q
     uint32_t out_lo, out_hi, sb;
     if (!fast || !quantize_block_fast<RULE>(X, enc, s_tab, approx_ok, __builtin_inff(), out_lo, out_hi, sb))
       quantize_block<RULE>(X, amax, enc, dec, out_lo, out_hi, sb);
-    *reinterpret_cast<uint2*>(job.values + ((int64_t)at.ty * 128 + row_in_tile) * (K >> 1) + (int64_t)at.tx * 32 + cb * 8) = make_uint2(out_lo, out_hi);
+    uint8_t* const vdst = job.values + ((int64_t)at.ty * 128 + row_in_tile) * (K >> 1) + (int64_t)at.tx * 32 + cb * 8;
+    *reinterpret_cast<uint2*>(vdst) = make_uint2(out_lo, out_hi);
     reinterpret_cast<uint8_t*>(s_scales[t & 1])[(row_in_tile & 31) * 16 + (row_in_tile >> 5) * 4 + cb] = (uint8_t)sb;
     __syncthreads();  // the buffer is written again two tiles, and a barrier, later
     if (threadIdx.x < 128) reinterpret_cast<uint32_t*>(job.scales)[(int64_t)at.tile * 128 + threadIdx.x] = s_scales[t & 1][threadIdx.x];
@@ -497,8 +499,9 @@ extern "C" int ll_nvfp4_quantize(const void* x, int64_t M, int64_t K, int64_t ld
 // The line: one workgroup per compute unit and tensor.  The exchange grows with a tensor's workgroups, each of which reads all
 // their slots, and a workgroup of four tiles has a chain of its own.  us, mse, here / in two launches (taken when the exchange
 // cost 0.5 us more, 0.7 at 96 workgroups):
-//   one tensor    4 tiles 5.3 / 8.2, 192 6.2 / 9.1, two tiles per workgroup: 320 8.9 / 9.6, 384 8.4 / 9.9; beyond the line, with two
-//                 workgroups per unit: 576 11.5 / 10.8, 1008 12.5 / 12.5; with four tiles per workgroup: 576 12.7 / 10.7, 1008 13.7 / 12.4
+//   one tensor    4 tiles 5.3 / 8.2, 192 6.2 / 9.1, two tiles per workgroup: 320 8.9 / 9.6, 384 8.4 / 9.9; beyond the
+//                 line, with two workgroups per unit: 576 11.5 / 10.8, 1008 12.5 / 12.5; with four tiles per workgroup:
+//                 576 12.7 / 10.7, 1008 13.7 / 12.4
 //   two tensors   2 x 92 tiles 6.3 / 9.3, 2 x 166 8.3 / 10.0, 2 x 220 8.4 / 10.3, 2 x 496 (512 workgroups) 10.9 / 12.8
 static constexpr int64_t kOnceTiles = 256;      // ll_nvfp4_quantize_once
 static constexpr int64_t kOnePassTiles = 512;   // of a tensor, ll_nvfp4_quantize_one_pass
@@ -508,7 +511,8 @@ static int quantize_one_pass(const ll::OnceJobs& jobs, int64_t M, int64_t K, int
   using namespace ll;
   LL_REQUIRE(M > 0 && K > 0 && ldx >= K, "%s: bad shape M=%lld K=%lld ldx=%lld", what, (long long)M, (long long)K, (long long)ldx);
   LL_REQUIRE(rule >= 0 && rule <= 4, "%s: unknown scale rule %d", what, rule);
-  LL_REQUIRE(amax_sink && amax_sink->parts && sink_is_valid(amax_sink), "%s: an amax sink (8-byte aligned buffer, non-zero epoch) is required", what);
+  LL_REQUIRE(amax_sink && amax_sink->parts && sink_is_valid(amax_sink),
+             "%s: an amax sink (8-byte aligned buffer, non-zero epoch) is required", what);
   const int64_t groups_m = (M + 127) / 128, groups_k = K / 64;
   bool whole = K % 64 == 0 && ldx % 8 == 0 && groups_m <= most_tiles && groups_k <= most_tiles && groups_m * groups_k <= most_tiles;
   for (int i = 0; i < jobs.n; ++i) {
@@ -539,11 +543,10 @@ static int quantize_one_pass(const ll::OnceJobs& jobs, int64_t M, int64_t K, int
   const uint32_t spin = spin_limit < 0 ? 0u : (spin_limit > 0x7FFFFFFF ? 0x7FFFFFFFu : (uint32_t)spin_limit);
   hipStream_t s = static_cast<hipStream_t>(stream);
   const dim3 grid((unsigned)(wgs * jobs.n));
-#define LL_LAUNCH_ONCE(R)                                                                                                          \
-  do {                                                                                                                             \
-    if (per_wg == 1) hipLaunchKernelGGL((quantize_once_kernel<R, 1>), grid, dim3(512), 0, s, jobs, M, K, ldx, (uint32_t)tiles, sink, spin, spin_limit < 0 ? 1 : 0); \
-    else hipLaunchKernelGGL((quantize_once_kernel<R, 2>), grid, dim3(512), 0, s, jobs, M, K, ldx, (uint32_t)tiles, sink, spin, spin_limit < 0 ? 1 : 0); \
-  } while (0)
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(512), 0, s, jobs, M, K, ldx, (uint32_t)tiles, sink, spin, spin_limit < 0 ? 1 : 0);
+  };
+#define LL_LAUNCH_ONCE(R) per_wg == 1 ? launch(&quantize_once_kernel<R, 1>) : launch(&quantize_once_kernel<R, 2>)
   switch (rule) {
     case LL_RULE_STATIC_6: LL_LAUNCH_ONCE(LL_RULE_STATIC_6); break;
     case LL_RULE_STATIC_4: LL_LAUNCH_ONCE(LL_RULE_STATIC_4); break;
@@ -566,8 +569,10 @@ extern "C" int ll_nvfp4_quantize_one_pass(const void* x0, const void* x1, int64_
                                           uint8_t* values1, uint8_t* scales0, uint8_t* scales1, float* amax0, float* amax1,
                                           const ll_amax_sink* amax_sink, int64_t spin_limit, void* stream) {
   using namespace ll;
-  LL_REQUIRE(!x1 || (values0 != values1 && scales0 != scales1 && amax0 != amax1), "ll_nvfp4_quantize_one_pass: the two tensors need outputs of their own");
-  const OnceJobs jobs{{{static_cast<const uint16_t*>(x0), values0, scales0, amax0}, {static_cast<const uint16_t*>(x1), values1, scales1, amax1}}, x1 ? 2 : 1};
+  LL_REQUIRE(!x1 || (values0 != values1 && scales0 != scales1 && amax0 != amax1),
+             "ll_nvfp4_quantize_one_pass: the two tensors need outputs of their own");
+  const OnceJobs jobs{{{static_cast<const uint16_t*>(x0), values0, scales0, amax0},
+                       {static_cast<const uint16_t*>(x1), values1, scales1, amax1}}, x1 ? 2 : 1};
   return quantize_one_pass(jobs, M, K, ldx, rule, amax_sink, spin_limit, kOnePassTiles, stream, "ll_nvfp4_quantize_one_pass");
 }
 

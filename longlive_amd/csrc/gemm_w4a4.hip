@@ -119,8 +119,8 @@ struct GemmGroups {
 // own LDS patch (the stages of the main loop are free by now) and writes rows with coalesced 16-byte stores.  BATCH: rows of
 // the residual and the gate under way, as many as are measured to pay: with 4 the hand-scheduled tiles spill 12 to 19
 // registers and lose 0.5 to 2.5 us (asm8: 2640 x 3072 x 3072 47 / 50).  The persistent kernel, whose 4 x 4 fragments leave none
-// to spare (253 spilled), takes 2: 2640 x 3072 x 3072 89 us, with gate and residual 97.5 (with 4 96 and 110.5; 7040 x 3072 x 14336
-// 568 and 676, with 4 607 and 785).
+// to spare (253 spilled), takes 2: 2640 x 3072 x 3072 89 us, with gate and residual 97.5 (with 4 96 and 110.5; 7040 x 14336 x
+// 3072 568 and 676, with 4 607 and 785).
 template <int FA, int FB, int BATCH>
 __device__ __forceinline__ void gemm_epilogue(float16v (&acc)[FB][FA], float alpha, uint8_t* smem, int wave, int lane, int row_base,
                                               int col_base, int M, int N, uint16_t* __restrict__ D, int64_t ldd,

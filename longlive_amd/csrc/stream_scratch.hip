@@ -21,7 +21,18 @@ static std::map<std::pair<int, hipStream_t>, ScratchSets> g_scratch;
 // them must not meet them there.  No recorded launch uses this one.  One size holds every small product, so it never grows.
 static std::map<std::pair<int, hipStream_t>, StreamScratch> g_small_scratch;
 
+// Memory is set up and freed as if no stream were being captured: while one is, in the global mode, either call is refused and
+// spoils the recording, on whatever stream it is made.
+struct RelaxedCapture {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  const bool exchanged = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+  ~RelaxedCapture() {
+    if (exchanged) (void)hipThreadExchangeStreamCaptureMode(&mode);
+  }
+};
+
 static void free_scratch(StreamScratch& w) {
+  const RelaxedCapture relaxed;
   if (w.records) (void)hipFree(w.records);  // waits for the launches that still use it
   if (w.counters) (void)hipFree(w.counters);
   w = StreamScratch{};
@@ -29,14 +40,11 @@ static void free_scratch(StreamScratch& w) {
 
 // Records and counters of the sizes in w, the counters zero for the work that follows on `stream`.
 static hipError_t allocate_scratch(StreamScratch& w, hipStream_t stream) {
-  // an allocation is refused, and a recording elsewhere spoilt, while another stream is captured in the global mode
-  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-  const bool exchanged = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+  const RelaxedCapture relaxed;
   hipError_t e = hipMalloc(reinterpret_cast<void**>(&w.records), w.record_bytes);
   if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void**>(&w.counters), w.n_counters * sizeof(int));
   if (e == hipSuccess) e = hipMemsetAsync(w.counters, 0, w.n_counters * sizeof(int), stream);
   if (e != hipSuccess) free_scratch(w);
-  if (exchanged) (void)hipThreadExchangeStreamCaptureMode(&mode);
   return e;
 }
 

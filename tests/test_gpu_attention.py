@@ -920,6 +920,34 @@ def test_a_graph_replays_beside_ordinary_launches_of_the_stream_it_was_recorded_
         _native.attention_release()
 
 
+def test_memory_grows_beside_a_recording_on_another_stream(gpu):
+    """Ordinary launches on one stream set up their memory, and replace it by more, while another stream is being captured in
+    the mode that refuses allocations everywhere: neither they nor the recording notice."""
+    small, large = ([_randn((n, H, 128), s).to(gpu) for n, s in ((Lq, 97), (Lk, 98), (Lk, 99))] for Lq, H, Lk in ((700, 2, 900), (3000, 24, 640)))
+    want = [_native.attention_bf16(*t, 128 ** -0.5) for t in (small, large)]
+    torch.cuda.synchronize()
+    side, busy, graph, x = torch.cuda.Stream(device=gpu), torch.cuda.Stream(device=gpu), torch.cuda.CUDAGraph(), torch.zeros(64, device=gpu)
+    with torch.cuda.stream(busy), _native.attention_policy("narrow"):
+        outputs = [_native.attention_bf16(*t, 128 ** -0.5) for t in (small, large, small)]   # torch keeps their memory for below
+    torch.cuda.synchronize()
+    del outputs
+    with torch.cuda.stream(side):   # torch.cuda.graph would give that memory back
+        graph.capture_begin(capture_error_mode="global")
+        x += 1
+        with torch.cuda.stream(busy):
+            got = [_native.attention_bf16(*t, 128 ** -0.5) for t in (small, large, small)]
+        x += 1
+        graph.capture_end()
+    for n in range(1, 4):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert bool((x == 2 * n).all())
+    assert all(torch.equal(g, w) for g, w in zip(got, want + want[:1]))
+    del graph
+    with torch.cuda.stream(busy):
+        _native.attention_release()
+
+
 @pytest.mark.parametrize("window_tokens,sink_blocks", [(2 * 128 + 40, 1), (3 * 128 - 1, 0), (128 + 64, 0)])
 def test_windows_that_end_inside_a_block_against_the_policy_oracle(gpu, window_tokens, sink_blocks):
     """max_attention_size that is not a multiple of the block size (wan_5b/modules/causal_model.py:673-724 slices token

@@ -158,10 +158,14 @@ Epochs epochs_of_stream(int dev, void* stream) {
 }
 
 // The amax of x and its quantization: one launch for a small tensor, two otherwise and while the stream is being captured.
-inline bool one_pass_tiles(int64_t M, int64_t K) { return K % 64 == 0 && ((M + 127) / 128) * (K / 64) <= 512; }
+// The line: two tiles per workgroup and one workgroup per unit for all tensors together.  With two workgroups per unit the
+// launch is ahead only where it is repeated by itself (2 x 408 tiles 10.7 against 12.3 us).  Behind an attention launch, as in
+// a KV step, it is not; us, two launches / one, by tiles of K and of V: 192 (768 queries x 16 heads) 28.4 / 27.9, 256 (1024 x 16)
+// 33.5 / 32.3, 288 (1152 x 16) 38.5 / 39.8, 384 (1536 x 16) 46.8 / 49.4, 288 (768 x 24, 1536 cached) 55.1 / 57.8.
+inline bool one_pass_tiles(int64_t M, int64_t K, int tensors) { return K % 64 == 0 && tensors * ((M + 127) / 128) * (K / 64) <= 512; }
 int quantize_operand(const void* x, int64_t M, int64_t K, int64_t ldx, int rule, uint8_t* values, uint8_t* scales, float* amax,
                      float* workspace, int dev, void* stream) {
-  if (one_pass_tiles(M, K)) {
+  if (one_pass_tiles(M, K, 1)) {
     Epochs e = epochs_of_stream(dev, stream);
     if (e.parts) {
       const ll_amax_sink sink = e.take();
@@ -728,7 +732,7 @@ PyObject* py_cache_write(PyObject*, PyObject* const* args, Py_ssize_t n) {
                                              amax[1], &sinks[0], &sinks[1], stream);
   } else {
     code = LL_ENOSUP;
-    if (one_pass_tiles(M, 128)) {
+    if (one_pass_tiles(M, 128, 2)) {
       Epochs e = epochs_of_stream(dev, stream);
       if (e.parts) {
         const ll_amax_sink sink = e.take();

@@ -502,7 +502,9 @@ extern "C" int ll_nvfp4_quantize(const void* x, int64_t M, int64_t K, int64_t ld
 //   one tensor    4 tiles 5.3 / 8.2, 192 6.2 / 9.1, two tiles per workgroup: 320 8.9 / 9.6, 384 8.4 / 9.9; beyond the
 //                 line, with two workgroups per unit: 576 11.5 / 10.8, 1008 12.5 / 12.5; with four tiles per workgroup:
 //                 576 12.7 / 10.7, 1008 13.7 / 12.4
-//   two tensors   2 x 92 tiles 6.3 / 9.3, 2 x 166 8.3 / 10.0, 2 x 220 8.4 / 10.3, 2 x 496 (512 workgroups) 10.9 / 12.8
+//   two tensors   2 x 92 tiles 6.3 / 9.3, 2 x 166 8.3 / 10.0, 2 x 220 8.4 / 10.3, 2 x 496 (512 workgroups) 10.9 / 12.8; with
+//                 more than one workgroup per unit that holds only for a launch by itself, and a KV step does not ask for
+//                 it (host_ops.cpp)
 static constexpr int64_t kOnceTiles = 256;      // ll_nvfp4_quantize_once
 static constexpr int64_t kOnePassTiles = 512;   // of a tensor, ll_nvfp4_quantize_one_pass
 

@@ -1147,6 +1147,37 @@ def test_tiles_whose_scores_are_all_minus_infinity_weigh_nothing(gpu, policy, go
     assert ((out.double() - ref).abs() <= 1.25 * 2 ** -9 * size + 2 ** -9 * ref.abs()).all()
 
 
+@pytest.mark.parametrize("policy", ["wide", "split"])
+@pytest.mark.parametrize("high,far", [(60.0, (40,)), (60.0, (200, 700, 1190)), (150.0, (40,)), (150.0, (700,)), (150.0, (1100,)), (150.0, (1190,)),
+                                      (400.0, (0, 500, 1150))])
+def test_scores_far_above_those_of_the_first_keys(gpu, policy, high, far):
+    """256-query tiles keep the reference point of a segment's first 32 keys and run the segment again where that is too low: keys
+    whose scores lie `high` above the others', within what fp32 holds and beyond, behind the first 32 keys, in later cached tiles, in
+    the chunk and in its ragged last tile; a full and a light group of queries, half of the queries without such keys.  Bound,
+    element by element: half a step of bf16 is at most 2^-8 of a number, of every probability and of the result."""
+    Lq, H, T, cached, n_new = 300, 2, 384, 1000, 200
+    q, k, v = (_randn((n, H, 128), s).to(gpu) for n, s in ((Lq, 71), (cached + n_new, 72), (cached + n_new, 73)))
+    q[..., 0], k[..., 0] = 0.0, 0.0
+    q[::2, :, 0] = 16.0
+    k[list(far), :, 0] = high / (16.0 * 128 ** -0.5)
+    kq, vq, K, V = [], [], [], []
+    for x, slots, rows in ((k, kq, K), (v, vq, V)):
+        padded = torch.cat([x[:cached], x.new_zeros(-cached % T, H, 128)])
+        for i in range(0, len(padded), T):
+            slots.append(quantize_to_fp4(padded[i:i + T].reshape(-1, 128), CFG))
+        rows.append(dequantize_kv_cache(slots, len(slots), H, T, torch.bfloat16, gpu)[0][:cached])
+        rows.append(x[cached:])
+    from longlive_amd.utils.quant import SlotPointerTable
+    kt, vt = SlotPointerTable(kq), SlotPointerTable(vq)
+    with _native.attention_policy(policy):
+        out = _native.kv_attention(q, (kt.values, kt.scales, kt.amax, vt.values, vt.scales, vt.amax), cached, T, 6.0, 256.0,
+                                   k[cached:].contiguous(), v[cached:].contiguous(), 128 ** -0.5)
+    K, V = torch.cat(K).double(), torch.cat(V).double()
+    p = [torch.softmax(q[:, h].double() @ K[:, h].T.contiguous() * 128 ** -0.5, -1) for h in range(H)]
+    ref, size = (torch.stack([ph @ x[:, h] for h, ph in enumerate(p)], 1) for x in (V, V.abs()))
+    assert ((out.double() - ref).abs() <= 2 ** -8 * (size + ref.abs())).all()
+
+
 @pytest.mark.parametrize("Lq,H,T,cached,n_new", [(512, 16, 512, 0, 4000), (512, 16, 512, 3584, 416), (520, 24, 480, 0, 1900),
                                                 (520, 24, 480, 1440, 460), (512, 16, 512, 2048, 512)])
 def test_the_plan_is_what_the_launch_does(gpu, Lq, H, T, cached, n_new):

@@ -218,6 +218,17 @@ int ll_nvfp4_gemm_tnt_fused(const uint8_t* A_values, const uint8_t* A_scales, co
                             void* D, int64_t ldd, const ll_gemm_epilogue* epilogue, void* stream);
 
 /*
+ * ll_nvfp4_quantize (x_sink NULL) or ll_nvfp4_quantize_from_sink of x [M, K] and ll_nvfp4_gemm_tnt_fused of the result, in one
+ * launch and with the same bits.  For small activations: LL_ENOSUP, and nothing is launched, unless K is a multiple of 64 up to
+ * 512, ldx a multiple of 8, x 16-byte aligned, the product one that ll_nvfp4_gemm_tnt computes in plain 64 x 64 tiles, for K
+ * beyond 256 of no more tiles of 32 x 128 than compute units, and, without x_sink, M * K <= 65536.  B [Np, K], Np a multiple of 128.
+ */
+int ll_nvfp4_quantize_gemm(const void* x, int64_t M, int64_t K, int64_t ldx, int rule, const ll_amax_sink* x_sink,
+                           float denom_a, const uint8_t* B_values, const uint8_t* B_scales, const float* amax_b,
+                           float denom_b, int64_t N, int64_t Np, void* D, int64_t ldd,
+                           const ll_gemm_epilogue* epilogue, void* stream);
+
+/*
  * Several ll_nvfp4_gemm_tnt products with the same A operand and the same N and Kp in one launch: the q, k and v
  * projections of one activation (wan_5b/modules/causal_model.py:363-365) and the k, v projections of the text
  * (:234-235), three resp. two fp4_matmul calls in the reference.  Each product has its own weight, scales, tensor

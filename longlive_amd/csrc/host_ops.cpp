@@ -215,8 +215,17 @@ PyObject* py_linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
     Py_RETURN_NONE;
   if (bias && (!is_bf16(*bias, dev) || bias->numel() != N || !bias->is_contiguous())) Py_RETURN_NONE;
   void* stream = stream_of(dev);
-  const TempOperand a = temp_operand(M, K, dev);
   const Tensor out = empty({M, N}, at::kBFloat16, dev);
+  ll_gemm_epilogue epilogue{};
+  epilogue.bias = bias ? bias->data_ptr() : nullptr;
+  const int code = ll_nvfp4_quantize_gemm(x.data_ptr(), M, K, x.stride(0), rule, nullptr, (float)denom_a, wv->data_ptr<uint8_t>(),
+                                          static_cast<const uint8_t*>(ws->data_ptr()), wa->data_ptr<float>(), (float)denom_b, N,
+                                          wv->size(0), out.data_ptr(), N, &epilogue, stream);
+  if (code != LL_ENOSUP) {
+    if (failed(code, "ll_nvfp4_quantize_gemm")) return nullptr;
+    return THPVariable_Wrap(out);
+  }
+  const TempOperand a = temp_operand(M, K, dev);
   if (failed(quantize_operand(x.data_ptr(), M, K, x.stride(0), rule, a.values, a.scales, a.amax, a.workspace, dev, stream),
              "ll_nvfp4_quantize"))
     return nullptr;
@@ -325,6 +334,16 @@ struct BlockCall {
     e.bias = w.bias;
     return ll_nvfp4_gemm_tnt_fused(a.values, a.scales, w.values, w.scales, nullptr, a.amax, w.amax, denom_a, w.denom, M, w.n,
                                    a.mp, w.np, a.kp, out, w.n, &e, stream);
+  }
+  // out = epilogue(x @ layer^T), the maximum of x in `sink`: one launch for small activations, else quantization into q and product
+  int linear(const void* x, int64_t K, const ll_amax_sink& sink, const Layer& w, int64_t M, void* out, ll_gemm_epilogue e, TempOperand& q) const {
+    e.bias = w.bias;
+    const int code = ll_nvfp4_quantize_gemm(x, M, K, K, rule, &sink, denom_a, w.values, w.scales, w.amax, w.denom, w.n, w.np, out, w.n, &e,
+                                            stream);
+    if (code != LL_ENOSUP) return code;
+    if (!q.values) q = operand(M, K);
+    const int quantized = ll_nvfp4_quantize_from_sink(x, M, K, K, rule, q.values, q.scales, q.amax, &sink, stream);
+    return quantized ? quantized : gemm(q, w, M, out, e);
   }
   int grouped(const TempOperand& a, const Layer* const* w, int n, int64_t M, void* const* outs, const ll_amax_sink* sinks) const {
     ll_gemm_product p[4];
@@ -455,12 +474,13 @@ PyObject* py_block_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
                                   y.data_ptr(), &again, c.stream);
     return code ? code : c.quantize_from(y, L, C, q, again);
   };
-  const TempOperand xq = c.operand(L, C);
+  TempOperand xq = c.operand(L, C);
   LL_TRY(adaln_operand(x.data_ptr(), 1, 0, xq), "adaLN");
 
   // ---- self-attention
   const Tensor value = empty({1, L, H, 128}, at::kBFloat16, dev), key = empty({1, L, H, 128}, at::kBFloat16, dev);
   Tensor attended;  // [L, C]
+  ll_amax_sink attended_sink;
   {
     const Tensor q = empty({L, C}, at::kBFloat16, dev), k = empty({L, C}, at::kBFloat16, dev);
     const Layer* const layers[3] = {&w[Q], &w[K], &w[V]};
@@ -484,11 +504,10 @@ PyObject* py_block_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
       return r;
     }
     attended = empty({L, C}, at::kBFloat16, dev);
-    const ll_amax_sink sink = ep.take();
+    attended_sink = ep.take();
     LL_TRY(ll_kv_attention_amax(roped_q.data_ptr(), L, H, kv.p[0], kv.p[1], kv.p[2], kv.p[3], kv.p[4], kv.p[5], kv.n_cached,
                                 kv.bts, kv.e2, kv.e4, smooth_k.data_ptr(), value.data_ptr(), L, 0.08838834764831845f,
-                                attended.data_ptr(), &sink, c.stream), "self-attention");
-    LL_TRY(c.quantize_from(attended, L, C, xq, sink), "quantization");
+                                attended.data_ptr(), &attended_sink, c.stream), "self-attention");
   }
   const Tensor x1 = empty({1, L, C}, at::kBFloat16, dev);
   ll_gemm_epilogue plain_epilogue{}, gated{};
@@ -497,7 +516,7 @@ PyObject* py_block_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
   gated.ldr = C;
   gated.gate = modulation(2);
   gated.residual = x.data_ptr();
-  LL_TRY(c.gemm(xq, w[O], L, x1.data_ptr(), gated), "output projection");
+  LL_TRY(c.linear(attended.data_ptr(), C, attended_sink, w[O], L, x1.data_ptr(), gated, xq), "output projection");
 
   // ---- cross-attention
   {
@@ -528,17 +547,17 @@ PyObject* py_block_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
       LL_TRY(c.grouped(tq, layers, 2, T, outs, nullptr), "text projections");
       LL_TRY(ll_rms_norm(k.data_ptr(), T, (int)C, norm[5], eps[4], text_k.data_ptr(), c.stream), "cross-attention norm_k");
     }
-    const ll_amax_sink sink = ep.take();
+    attended_sink = ep.take();
     LL_TRY(ll_kv_attention_amax(qn.data_ptr(), L, H, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0, 6.f, 256.f,
-                                text_k.data_ptr(), text_v.data_ptr(), T, 0.08838834764831845f, attended.data_ptr(), &sink, c.stream),
+                                text_k.data_ptr(), text_v.data_ptr(), T, 0.08838834764831845f, attended.data_ptr(), &attended_sink,
+                                c.stream),
            "cross-attention");
-    LL_TRY(c.quantize_from(attended, L, C, xq, sink), "quantization");
   }
   const Tensor x2 = empty({1, L, C}, at::kBFloat16, dev);
   ll_gemm_epilogue residual{};
   residual.ldr = C;
   residual.residual = x1.data_ptr();
-  LL_TRY(c.gemm(xq, w[CO], L, x2.data_ptr(), residual), "cross-attention output projection");
+  LL_TRY(c.linear(attended.data_ptr(), C, attended_sink, w[CO], L, x2.data_ptr(), residual, xq), "cross-attention output projection");
 
   // ---- feed-forward
   LL_TRY(adaln_operand(x2.data_ptr(), 4, 3, xq), "adaLN");
@@ -547,12 +566,11 @@ PyObject* py_block_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
   gelu.activation = LL_ACT_GELU_TANH;
   gelu.amax_sink = ep.take();
   LL_TRY(c.gemm(xq, w[UP], L, hidden.data_ptr(), gelu), "FFN up");
-  const TempOperand hq = c.operand(L, w[UP].n);
-  LL_TRY(c.quantize_from(hidden, L, w[UP].n, hq, gelu.amax_sink), "quantization");
+  TempOperand hq{};
   const Tensor& out = attended;  // its memory is free by now
   gated.gate = modulation(5);
   gated.residual = x2.data_ptr();
-  LL_TRY(c.gemm(hq, w[DOWN], L, out.data_ptr(), gated), "FFN down");
+  LL_TRY(c.linear(hidden.data_ptr(), w[UP].n, gelu.amax_sink, w[DOWN], L, out.data_ptr(), gated, hq), "FFN down");
 #undef LL_TRY
 
   PyObject* r = PyTuple_New(5);

@@ -1,0 +1,237 @@
+// A W4A4 linear layer of a small activation in one launch: tensor amax, quantization to NVFP4 and the product.
+//
+// What a product of 48 x 256 x 512 costs is launches and trips to memory: quantization and GEMM are two of either, 4 to 5 us
+// each, for a microsecond of work.  Here a workgroup quantizes the 32 rows of its own tile, into LDS, and multiplies them;
+// the column tiles of a row quantize it again, which costs nothing while compute units are idle.  The tensor amax comes
+// from the sink in which the producer of x left it, or every workgroup forms it from the whole tensor.
+//
+// Measured, us on the GPU, two launches / one.  Maximum in a sink: 48 x 256 x 512 8.1 / 6.0, 1024 x 256 x 256 8.8 / 6.6, 368 x 384 x 384
+// 9.0 / 7.9, 192 x 512 x 512 9.9 / 9.3.  Maximum of its own: 48 x 256 x 512 8.3 / 6.1, 192 x 256 x 256 8.4 / 7.6; a call with its host time
+// 12.2 / 7.6 and 12.3 / 7.6.
+#include "ll_common.h"
+#include "gemm_epilogue.h"
+#include "quantize_block.h"  // from here on without floating-point contraction
+
+namespace ll {
+
+constexpr int kFusedThreads = 256;  // eight waves: 48 x 256 x 512 7.2 instead of 6.1 us, 64 x 512 x 512 11.2 instead of 9.5
+constexpr int kFusedRows = 32, kFusedCols = 32 * (kFusedThreads / 64);  // of a workgroup's tile: a wave multiplies all rows and 32 columns
+constexpr int kFusedMaxK = 512;
+constexpr int kFusedPatch = 32 * (64 + 16);       // bytes of a wave's patch in the epilogue
+
+struct FusedParams {
+  const uint16_t* x;
+  int64_t ldx;
+  const unsigned long long* sink_parts;  // null: the maximum of x itself
+  uint32_t sink_epoch;
+  const uint32_t* sink_epoch_offset;
+  const uint8_t *Bv, *Bs;
+  const float* amax_b;
+  float inv_denom_a, inv_denom_b;
+  int M, N, K, Np, tiles_m;
+  uint16_t* D;
+  int64_t ldd;
+  GemmEpilogue epi;
+};
+
+// T: 64 elements of K at most, a wave's weights in registers.  Quantization is the arithmetic of quantize_kernel, the product
+// the order of gemm_w4a4_kernel<1, 1> (64 elements of K after 64, dword after dword of the lanes' pieces): the same bits.
+// Bound by the chain: one trip to memory for x, weights and maximum together, the scale table, a few hundred instructions per
+// block of 16 (229 a block and lane), the products, the store.
+template <int RULE, int T>
+__global__ __launch_bounds__(kFusedThreads) void quantize_gemm_kernel(FusedParams p) {
+  constexpr int kPitch = 32 * T + 16, kScalePitch = 4 * T + 2;
+  constexpr int kRowBlocks = 4 * T, kBlocks = kFusedRows * kRowBlocks / kFusedThreads;  // per row; per thread, at most
+  __shared__ float s_red[kFusedThreads / 64];
+  __shared__ ScaleEntry s_tab[128];
+  __shared__ __attribute__((aligned(16))) uint8_t s_values[kFusedRows * kPitch];
+  __shared__ __attribute__((aligned(16))) uint8_t s_scales[kFusedRows * kScalePitch];
+  __shared__ __attribute__((aligned(16))) uint8_t s_patch[kFusedThreads / 64 * kFusedPatch];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l32 = lane & 31, lh = lane >> 5;
+  const int tile_n = blockIdx.x / p.tiles_m, tile_m = blockIdx.x - tile_n * p.tiles_m;
+  const int row0 = tile_m * kFusedRows, col0 = tile_n * kFusedCols + 32 * wave;
+  const int steps = p.K >> 6, row_blocks = p.K >> 4;
+
+  // ---- everything the workgroup reads, asked for at once and without branches
+  // the thread's blocks of x: block tid + 256 i of the tile's 32 rows
+  u32x4 lo[kBlocks], hi[kBlocks];
+  int block_row[kBlocks], block_col[kBlocks];
+#pragma unroll
+  for (int i = 0; i < kBlocks; ++i) {
+    const int b = tid + i * kFusedThreads;
+    block_row[i] = b / row_blocks;
+    block_col[i] = b - block_row[i] * row_blocks;
+    const int row = min(row0 + block_row[i], p.M - 1);
+    const u32x4* src = reinterpret_cast<const u32x4*>(p.x + (int64_t)row * p.ldx + block_col[i] * 16);
+    lo[i] = src[0];
+    hi[i] = src[1];
+  }
+  // the wave's weights: row l32 of its 32, pieces 2 t + lh of 16 bytes and the scales of their two blocks
+  uint4 bv[T];
+  uint32_t bs[T];
+  {
+    const int n = min(col0 + l32, p.Np - 1);
+    const uint8_t* values = p.Bv + (int64_t)n * (p.K >> 1) + 16 * lh;
+    const uint8_t* scales = p.Bs + (int64_t)(n >> 7) * (p.K >> 6) * 512 + (n & 31) * 16 + ((n & 127) >> 5) * 4 + 2 * lh;
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      const int at = min(t, steps - 1);
+      bv[t] = *reinterpret_cast<const uint4*>(values + 32 * at);
+      bs[t] = *reinterpret_cast<const uint16_t*>(scales + 512 * at);
+    }
+  }
+  float part = 0.0f;
+  if (p.sink_parts) {
+    const uint32_t epoch = amax_sink_epoch(p.sink_epoch, p.sink_epoch_offset);
+#pragma unroll
+    for (int i = 0; i < kAmaxParts / kFusedThreads; ++i) part = fmaxf(part, amax_sink_read(p.sink_parts, epoch, i * kFusedThreads + tid));
+  } else {
+    // eight pieces of 16 bytes under way; behind the end the last one again
+    const uint32_t row_pieces = (uint32_t)p.K >> 3, pieces = (uint32_t)p.M * row_pieces;
+    for (uint32_t c0 = tid; c0 < pieces; c0 += 8 * kFusedThreads) {
+      uint4 v[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const uint32_t c = min(c0 + i * kFusedThreads, pieces - 1), r = c / row_pieces;
+        v[i] = *reinterpret_cast<const uint4*>(p.x + (int64_t)r * p.ldx + (c - r * row_pieces) * 8);
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) part = abs_max_bf16x8(v[i], part);
+    }
+  }
+  part = wave_max(part);
+  if (lane == 0) s_red[wave] = part;
+  __syncthreads();
+  float amax = s_red[0];
+#pragma unroll
+  for (int i = 1; i < kFusedThreads / 64; ++i) amax = fmaxf(amax, s_red[i]);
+
+  // ---- quantization of the 32 rows into LDS (the prologue and the paths of quantize_kernel)
+  constexpr bool kStaticRule = (RULE == LL_RULE_STATIC_6 || RULE == LL_RULE_STATIC_4);
+  constexpr float kE2 = (RULE == LL_RULE_STATIC_4) ? 4.0f : 6.0f;
+  constexpr float kE4 = kStaticRule ? 448.0f : 256.0f;
+  const bool fast = amax >= 0x1p-100f && amax <= 0x1p100f;
+  const bool approx_ok = amax >= 0x1p-30f && amax <= 0x1p30f;
+  const float enc = (kE2 * kE4) / amax;
+  const float dec = 1.0f / enc;
+  if (fast) fill_scale_table<RULE>(s_tab, amax, dec);
+  __syncthreads();
+#pragma unroll 1
+  for (int i = 0; i < kBlocks; ++i) {
+    u32x4 l = lo[0], h = hi[0];
+    int row = block_row[0], col = block_col[0];
+#pragma unroll
+    for (int j = 1; j < kBlocks; ++j)
+      if (i == j) l = lo[j], h = hi[j], row = block_row[j], col = block_col[j];
+    if (row >= kFusedRows) break;
+    float X[16];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const uint32_t w = j < 4 ? l[j] : h[j - 4];
+      X[2 * j] = __uint_as_float(w << 16);
+      X[2 * j + 1] = __uint_as_float(w & 0xFFFF0000u);
+    }
+    uint32_t out_lo, out_hi, sb;
+    if (!fast || !quantize_block_fast<RULE>(X, enc, s_tab, approx_ok, __builtin_inff(), out_lo, out_hi, sb))
+      quantize_block<RULE>(X, amax, enc, dec, out_lo, out_hi, sb);
+    *reinterpret_cast<uint2*>(s_values + row * kPitch + col * 8) = make_uint2(out_lo, out_hi);
+    s_scales[row * kScalePitch + col] = (uint8_t)sb;
+  }
+  __syncthreads();
+  if (col0 >= p.N) return;
+
+  // ---- product: 32 x 32 per wave
+  float16v acc[1][1];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) acc[0][0][i] = 0.0f;
+  const uint8_t* a_values = s_values + l32 * kPitch + 16 * lh;
+  const uint8_t* a_scales = s_scales + l32 * kScalePitch + 2 * lh;
+#pragma unroll
+  for (int t = 0; t < T; ++t) {
+    if (t >= steps) break;
+    const uint4 av = *reinterpret_cast<const uint4*>(a_values + 32 * t);
+    const half2v as = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(*reinterpret_cast<const uint16_t*>(a_scales + 4 * t), 1.0f, false);
+    const half2v ws = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(bs[t], 1.0f, false);
+    const uint32_t a[4] = {av.x, av.y, av.z, av.w}, b[4] = {bv[t].x, bv[t].y, bv[t].z, bv[t].w};
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(decode8(b[j], half2v{ws[j >> 1], ws[j >> 1]}),
+                                                         decode8(a[j], half2v{as[j >> 1], as[j >> 1]}), acc[0][0], 0, 0, 0);
+  }
+  const float alpha = (amax * p.amax_b[0]) * (p.inv_denom_a * p.inv_denom_b);
+  gemm_epilogue<1, 1, 4>(acc, alpha, s_patch, wave, lane, row0, col0, p.M, p.N, p.D, p.ldd, p.epi.bias, p.epi.act, p.epi,
+                         (uint32_t)blockIdx.x * (kFusedThreads / 64) + wave);
+}
+
+template <int RULE>
+void launch_quantize_gemm(const FusedParams& p, unsigned grid, hipStream_t s) {
+  if (p.K <= 256)
+    hipLaunchKernelGGL((quantize_gemm_kernel<RULE, 4>), dim3(grid), dim3(kFusedThreads), 0, s, p);
+  else
+    hipLaunchKernelGGL((quantize_gemm_kernel<RULE, 8>), dim3(grid), dim3(kFusedThreads), 0, s, p);
+}
+
+}  // namespace ll
+
+extern "C" int ll_nvfp4_quantize_gemm(const void* x, int64_t M, int64_t K, int64_t ldx, int rule, const ll_amax_sink* x_sink, float denom_a,
+                                      const uint8_t* B_values, const uint8_t* B_scales, const float* amax_b, float denom_b, int64_t N,
+                                      int64_t Np, void* D, int64_t ldd, const ll_gemm_epilogue* epilogue, void* stream) {
+  using namespace ll;
+  LL_REQUIRE(x && B_values && B_scales && amax_b && D && epilogue, "ll_nvfp4_quantize_gemm: null pointer");
+  LL_REQUIRE(M > 0 && K > 0 && N > 0 && ldx >= K && Np % 128 == 0 && N <= Np && ldd >= N && denom_a > 0.f && denom_b > 0.f,
+             "ll_nvfp4_quantize_gemm: bad shape M=%lld N=%lld Np=%lld K=%lld ldx=%lld ldd=%lld", (long long)M, (long long)N, (long long)Np,
+             (long long)K, (long long)ldx, (long long)ldd);
+  LL_REQUIRE(rule >= 0 && rule <= 4, "ll_nvfp4_quantize_gemm: unknown scale rule %d", rule);
+  LL_REQUIRE(!x_sink || (x_sink->parts && sink_is_valid(x_sink)), "ll_nvfp4_quantize_gemm: amax sink needs an 8-byte aligned buffer and a non-zero epoch");
+  LL_REQUIRE(((reinterpret_cast<uintptr_t>(B_values) | reinterpret_cast<uintptr_t>(B_scales)) & 15) == 0 &&
+                 (reinterpret_cast<uintptr_t>(D) & 1) == 0 && (reinterpret_cast<uintptr_t>(epilogue->bias) & 1) == 0,
+             "ll_nvfp4_quantize_gemm: operands must be 16-byte, D and bias 2-byte aligned");
+  FusedParams p{};
+  if (int rc = make_epilogue(*epilogue, N, p.epi)) return rc;
+  // Where the launch is ahead of quantization and product of their own.  A workgroup that reads the whole tensor for its maximum: up
+  // to 65536 elements (a call with its host time, two launches / one, us: 64 x 512 x 512 12.4 / 9.9, 128 x 512 x 256 12.4 / 11.3; 192 x 512
+  // x 512, beyond the line, 12.6 / 12.5 and on the GPU 9.9 / 12.2).
+  if (K % 64 != 0 || K > kFusedMaxK || ldx % 8 != 0 || (reinterpret_cast<uintptr_t>(x) & 15) != 0 || M > (1 << 20) || N > (1 << 20) ||
+      (!x_sink && M * K > 65536))
+    return LL_ENOSUP;
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess) {
+    set_error("ll_nvfp4_quantize_gemm: hipGetDevice failed");
+    return LL_ELAUNCH;
+  }
+  if (int rc = compute_units_of(dev, cus, "ll_nvfp4_quantize_gemm")) return rc;
+  if (!product_takes_plain_64x64_tiles(M, N, K, cus)) return LL_ENOSUP;
+  // More than one workgroup per unit of the longer rows, whose quantization is then repeated in turn: 1760 x 512 x 512, 220
+  // workgroups, 10.6 / 10.1, 2640 x 512 x 512, 332, 12.0 / 13.1; but 5280 x 256 x 256, 330, 10.3 / 8.7.
+  const int64_t grid = ((M + kFusedRows - 1) / kFusedRows) * ((N + kFusedCols - 1) / kFusedCols);
+  if (K > 256 && grid > cus) return LL_ENOSUP;
+  p.x = static_cast<const uint16_t*>(x);
+  p.ldx = ldx;
+  if (x_sink) {
+    p.sink_parts = reinterpret_cast<const unsigned long long*>(x_sink->parts);
+    p.sink_epoch = x_sink->epoch;
+    p.sink_epoch_offset = x_sink->epoch_offset;
+  }
+  p.Bv = B_values;
+  p.Bs = B_scales;
+  p.amax_b = amax_b;
+  p.inv_denom_a = 1.0f / denom_a;
+  p.inv_denom_b = 1.0f / denom_b;
+  p.M = (int)M;
+  p.N = (int)N;
+  p.K = (int)K;
+  p.Np = (int)Np;
+  p.tiles_m = (int)((M + kFusedRows - 1) / kFusedRows);
+  p.D = static_cast<uint16_t*>(D);
+  p.ldd = ldd;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  switch (rule) {
+    case LL_RULE_STATIC_6: launch_quantize_gemm<LL_RULE_STATIC_6>(p, (unsigned)grid, s); break;
+    case LL_RULE_STATIC_4: launch_quantize_gemm<LL_RULE_STATIC_4>(p, (unsigned)grid, s); break;
+    case LL_RULE_MAE: launch_quantize_gemm<LL_RULE_MAE>(p, (unsigned)grid, s); break;
+    case LL_RULE_MSE: launch_quantize_gemm<LL_RULE_MSE>(p, (unsigned)grid, s); break;
+    default: launch_quantize_gemm<LL_RULE_ABS_MAX>(p, (unsigned)grid, s); break;
+  }
+  LL_CHECK_LAUNCH("quantize_gemm_kernel");
+  return LL_OK;
+}

@@ -1,5 +1,6 @@
 """GPU parity: W4A4 GEMM and the quantized Linear against the oracle's dequantize-then-fp32-matmul.
 Bar (floating point): relative Frobenius error <= 1e-3."""
+import ctypes
 import os
 
 import numpy as np
@@ -688,6 +689,47 @@ def test_native_linear_call_equals_the_separate_operations(gpu, view):
         with torch.no_grad():
             want = fp4_matmul(quantize_to_fp4(x, QuantizationConfig()), model[0].quantized_weight(), bias=model[0].bias)
             assert torch.equal(model(x), want)
+
+
+@pytest.mark.parametrize("rule", ["mse", "mae", "abs_max", "static_6", "static_4"])
+@pytest.mark.parametrize("M,K,N,bias", [(1, 64, 8, False), (31, 128, 128, True), (33, 192, 100, True), (48, 256, 512, True), (192, 320, 256, False),
+                                        (128, 512, 264, True), (65, 448, 129, False)])
+def test_small_layer_in_one_launch_equals_quantization_and_product(gpu, M, K, N, bias, rule):
+    """The launch in which every workgroup quantizes the rows of its tile, over the ends of its tiles and of K, against the two
+    launches: the maximum of its own, strided rows, values at the ends of the ranges; the maximum from a sink, with gate and
+    residual."""
+    torch.manual_seed(M + K)
+    layer = quantize_model_with_filter(nn.Sequential(nn.Linear(K, N, bias=bias).to(gpu)), ModelQuantizationConfig(scale_rule=rule),
+                                       materialize_for_inference=True, verbose=False)[0][0]
+    w = layer.quantized_weight()
+    x = activations((M, K), M + K).to(gpu)
+    wide = torch.zeros(M, K + 8, dtype=torch.bfloat16, device=gpu)
+    infinite = x.clone()
+    infinite[M // 2, K - 1] = float("inf")
+    for values in (x, torch.zeros_like(x), x * 1e-36, x * 1e33, infinite):
+        wide[:, :K] = values
+        with torch.no_grad():
+            want = layer.forward_quantized(layer.quantize_input(values))
+            assert all(torch.equal(layer(v).view(torch.int16), want.view(torch.int16)) for v in (values, wide[:, :K]))
+    if N % 8:
+        return
+    nothing = torch.zeros(1, 1, 1, K, dtype=torch.bfloat16, device=gpu)
+    ticket = _native.amax_ticket(gpu)
+    y = _native.adaln_modulate(x[None], nothing, nothing, M, amax_out=ticket)[0]
+    residual, gate = activations((M, N), 5).to(gpu), activations((1, N), 6).to(gpu)
+    denominators = [_native.DENOMINATORS[rule], _native.DENOMINATORS[w.scale_rule.value]]
+    got = torch.empty(M, N, dtype=torch.bfloat16, device=gpu)
+    sink = ticket.struct()
+    epilogue = _native.GemmEpilogue(None if layer.bias is None else layer.bias.data_ptr(), 0, gate.data_ptr(), M, N, residual.data_ptr(), N,
+                                    _native.AmaxSinkStruct())
+    code = _native.load().ll_nvfp4_quantize_gemm(
+        y.data_ptr(), M, K, K, _native.RULE_IDS[rule], ctypes.byref(sink), denominators[0], w.values.data_ptr(), w.scale_factors.data_ptr(),
+        w.amax.data_ptr(), denominators[1], N, w.values.shape[0], got.data_ptr(), N, ctypes.byref(epilogue), torch.cuda.current_stream().cuda_stream)
+    assert code == 0
+    q = quantize_to_fp4(y, QuantizationConfig(scale_rule=rule))
+    want = _native.gemm(q.values, q.scale_factors, w.values, w.scale_factors, M, N, amax_a=q.amax, amax_b=w.amax, denom_a=denominators[0],
+                        denom_b=denominators[1], bias=layer.bias, residual=residual, gate=gate, gate_rows=M)
+    assert torch.equal(got, want)
 
 
 @pytest.mark.parametrize("M,N,K,groups", [

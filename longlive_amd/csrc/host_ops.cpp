@@ -158,6 +158,7 @@ Epochs epochs_of_stream(int dev, void* stream) {
 }
 
 // The amax of x and its quantization: one launch for a small tensor, two otherwise and while the stream is being captured.
+// workspace: LL_AMAX_PARTS floats, or null: allocated where two launches need them (1173 x 2048 in one launch: 8.9, so 8.4 us of host time a call).
 // The line: two tiles per workgroup and one workgroup per unit for all tensors together.  With two workgroups per unit the
 // launch is ahead only where it is repeated by itself (2 x 408 tiles 10.7 against 12.3 us).  Behind an attention launch, as in
 // a KV step, it is not; us, two launches / one, by tiles of K and of V: 192 (768 queries x 16 heads) 28.4 / 27.9, 256 (1024 x 16)
@@ -174,6 +175,11 @@ int quantize_operand(const void* x, int64_t M, int64_t K, int64_t ldx, int rule,
       if (code != LL_ENOSUP) return code;
     }
   }
+  Tensor own;  // freed for work behind this launch on the stream
+  if (!workspace) {
+    own = empty({(int64_t)LL_AMAX_PARTS}, at::kFloat, dev);
+    workspace = own.data_ptr<float>();
+  }
   return ll_nvfp4_quantize(x, M, K, ldx, rule, values, scales, amax, 0, workspace, stream);
 }
 
@@ -187,10 +193,10 @@ PyObject* py_quantize(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const int64_t M = x.size(0), K = x.size(1), Mp = round_up(M, 128), Kp = round_up(K, 64);
   const int rule = (int)PyLong_AsLong(args[1]);
   const Tensor values = empty({Mp, Kp / 2}, at::kByte, dev), scales = empty({Mp * Kp / 16}, at::kFloat8_e4m3fn, dev),
-               amax = empty({1}, at::kFloat, dev), ws = empty({(int64_t)LL_AMAX_PARTS}, at::kFloat, dev);
+               amax = empty({1}, at::kFloat, dev);
   if (failed(quantize_operand(x.data_ptr(), M, K, x.stride(0), rule, values.data_ptr<uint8_t>(),
-                              static_cast<uint8_t*>(scales.data_ptr()), amax.data_ptr<float>(), ws.data_ptr<float>(), dev,
-                              stream_of(dev)), "ll_nvfp4_quantize"))
+                              static_cast<uint8_t*>(scales.data_ptr()), amax.data_ptr<float>(), nullptr, dev, stream_of(dev)),
+             "ll_nvfp4_quantize"))
     return nullptr;
   return tuple3(values, scales, amax);
   END_HANDLE_TH_ERRORS

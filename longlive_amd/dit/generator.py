@@ -132,6 +132,13 @@ class StreamingGenerator:
         shot_index = 0
         self.model.rope_temporal_offset = 0.0
         sigmas = [t / 1000.0 for t in self.timesteps] + [0.0]
+        scheduler, levels = None, {}   # levels: the timestep tensors, (t, frames) -> [1, frames]
+
+        def level(t: float, frames: int) -> torch.Tensor:
+            if (t, frames) not in levels:
+                levels[t, frames] = torch.full((1, frames), t, device=self.device, dtype=torch.float32)
+            return levels[t, frames]
+
         decoded, previous_decode = [], None
         if decode_chunk is not None and decode_stream is None:
             decode_stream = torch.cuda.Stream(device=self.device)
@@ -148,15 +155,16 @@ class StreamingGenerator:
                 self.model.rope_temporal_offset = shot_index * self.multi_shot_rope_offset
             is_scene_cut = self.multi_shot_sink and cfg.sink_size > 0 and ci > 0 and ci in scene_cuts
             if self.sampler == "unipc":
-                scheduler = FlowUniPCMultistepScheduler(num_train_timesteps=1000, shift=1)
+                if scheduler is None:
+                    scheduler = FlowUniPCMultistepScheduler(num_train_timesteps=1000, shift=1)
                 # On the host, where the timesteps are looked at: on the device every chunk waited three times for all
                 # work before it (the list, and the place of the first timestep in it).
                 scheduler.set_timesteps(len(self.timesteps), shift=self.sample_shift)
                 steps = scheduler.timesteps.tolist()
             else:
-                scheduler, steps = None, self.timesteps
+                steps = self.timesteps
             for si, t in enumerate(steps):
-                tt = torch.full((1, f), float(t), device=self.device, dtype=torch.float32)
+                tt = level(float(t), f)
                 # The K / V a denoising forward would write into the chunk's slot are overwritten by the next
                 # forward before anything reads them (the chunk attends its own K / V in bf16), so only the
                 # clean-context pass below writes; the cache after the chunk is the same either way.
@@ -187,7 +195,7 @@ class StreamingGenerator:
             for cache, text, xc in zip(caches, (context, negative_context), (xcache, xcache_neg)):
                 if is_scene_cut and self.shot_clean_recache:
                     kvc.zero_kv_data(cache, start * fs, self.global_sink_size * fs)
-                self.model(x, torch.zeros((1, f), device=self.device), text, cache, start * fs, crossattn_cache=xc,
+                self.model(x, level(0.0, f), text, cache, start * fs, crossattn_cache=xc,
                            timestep_key=(0.0, f), cache_only=self.skip_dead_recache_tail)
                 if is_scene_cut:
                     kvc.pin_current_chunk(cache, f * fs, cfg.sink_size * fs)

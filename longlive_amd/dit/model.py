@@ -340,7 +340,7 @@ class DiTBlock(nn.Module):
         is not the common one; :meth:`forward` then runs the operations one by one."""
         sa, ca, norm3, ffn = (self._modules[name] for name in ("self_attn", "cross_attn", "norm3", "ffn"))
         if (not x.is_cuda or type(sa) is not CausalSelfAttention or type(ca) is not CrossAttention or sa.use_relative_rope
-                or type(norm3) is not WanLayerNorm or norm3.weight is None or sa.head_dim != 128 or not self.fuse_norm_quantize
+                or type(norm3) is not WanLayerNorm or sa.head_dim != 128 or not self.fuse_norm_quantize
                 or not isinstance(kv_cache, dict) or len(ffn) != 3 or getattr(ffn[1], "approximate", None) != "tanh"):
             return None
         sm, cm = sa._modules, ca._modules
@@ -348,6 +348,11 @@ class DiTBlock(nn.Module):
         if norms[0].eps != norms[1].eps or any(type(n) is not WanRMSNorm for n in norms) or _has_hooks(sa, ca, norm3, *norms):
             return None
         if not (OWN_LINEAR.of_class(FourOverSixLinear) and _OWN_BLOCK.of(self) and _OWN_SELF_ATTENTION.of(sa) and _OWN_CROSS_ATTENTION.of(ca) and _OWN_RMS_NORM.of(norms[2])):
+            return None
+        # parameters past the modules' attribute search; a weight that is none takes the general path
+        weights = (*(n._parameters.get("weight") for n in norms[:2]), norm3._parameters.get("weight"), norm3._parameters.get("bias"),
+                   *(n._parameters.get("weight") for n in norms[2:]))
+        if weights[2] is None:
             return None
         linears = (sm["q"], sm["k"], sm["v"], sm["o"], cm["q"], cm["k"], cm["v"], cm["o"], ffn[0], ffn[2])
         rule, layers = None, []
@@ -371,8 +376,7 @@ class DiTBlock(nn.Module):
         if collect_kv_amax:
             tickets = sa.amax_tickets(kv_cache, x.device)
         out = _native.block_forward(
-            x, e, tuple(layers), (norms[0].weight, norms[1].weight, norm3.weight, norm3.bias, norms[2].weight, norms[3].weight),
-            cos, sin, window, text, rule.value, (sa.num_heads, self.eps, norms[0].eps, norm3.eps, norms[2].eps, norms[3].eps),
+            x, e, tuple(layers), weights, cos, sin, window, text, rule.value, (sa.num_heads, self.eps, norms[0].eps, norm3.eps, norms[2].eps, norms[3].eps),
             keys_only, tickets)
         if out is None:
             return None
@@ -535,9 +539,9 @@ class CausalDiT(nn.Module):
         for instance ``(250.0, 3)``) the three tensors are computed once per value and kept until a parameter they
         depend on is replaced or written."""
         cfg = self.cfg
-        params = [p for seq in (self.time_embedding, self.time_projection) for p in seq.parameters()] + \
-                 [b.modulation for b in self.blocks]
-        version = tuple((p.data_ptr(), p._version) for p in params)
+        # every parameter that parameters() would yield, without its search for names and duplicates (10 us a forward)
+        params = [p for seq in (self.time_embedding, self.time_projection) for m in seq.modules() for p in m._parameters.values() if p is not None]
+        version = tuple((p.data_ptr(), p._version) for p in (*params, *(b.modulation for b in self.blocks)))
         if self._time_cache.get("version") != version:
             self._time_cache = {"version": version}
         key = None if timestep_key is None else (timestep_key, tuple(t.shape), like.dtype, str(like.device))

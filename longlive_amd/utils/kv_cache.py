@@ -14,7 +14,7 @@ import torch
 
 from .. import _native
 from ..fouroversix import QuantizationConfig, QuantizedTensor, ScaleRule, quantize_to_fp4
-from .quant import SlotPointerTable, clone_quantized_tensor, copy_quantized_into, dequantize_kv_cache, k_smooth
+from .quant import SlotPointerTable, copy_quantized_into, dequantize_kv_cache, k_smooth
 
 
 def initialize_kv_cache(num_layers: int, block_token_size: int, max_blocks: int, num_heads: int, head_dim: int,
@@ -25,11 +25,19 @@ def initialize_kv_cache(num_layers: int, block_token_size: int, max_blocks: int,
         raise ValueError("the KV-cache kernels are built for head_dim 128")
     zero = quantize_to_fp4(torch.zeros(block_token_size * num_heads, head_dim, dtype=dtype, device=device),
                            kv_quant_config)
+    # Every buffer an allocation of its own (slots side by side in one: a KV step of 368 tokens x 16 heads 28.1 -> 30.1 us), all of
+    # them written by a launch or two (one each: 0.4 ms of host time for two layers of five blocks).
+    parts = (zero.values, zero.scale_factors.view(torch.uint8), zero.amax)
+    buffers = [[torch.empty_like(t) for _ in range(num_layers * 2 * max_blocks)] for t in parts]
+    for t, copies in zip(parts, buffers):
+        torch._foreach_copy_(copies, [t] * len(copies))
+    made = iter([QuantizedTensor(v, s.view(zero.scale_factors.dtype), a, zero.dtype, zero.original_shape, zero.scale_rule, zero.padded_shape)
+                 for v, s, a in zip(*buffers)])
     cache = []
     for _ in range(num_layers):
         cache.append({
-            "k": [clone_quantized_tensor(zero) for _ in range(max_blocks)],
-            "v": [clone_quantized_tensor(zero) for _ in range(max_blocks)],
+            "k": [next(made) for _ in range(max_blocks)],
+            "v": [next(made) for _ in range(max_blocks)],
             "quantized": True,
             "block_token_size": block_token_size,
             "max_blocks": max_blocks,

@@ -51,6 +51,8 @@ _SIGNATURES = {
                                         c_void_p, c_void_p]),
     "ll_nvfp4_quantize_gemm": (c_int, [c_void_p, c_int64, c_int64, c_int64, c_int, c_void_p, c_float, c_void_p, c_void_p, c_void_p,
                                        c_float, c_int64, c_int64, c_void_p, c_int64, c_void_p, c_void_p]),
+    "ll_nvfp4_norm_gemm": (c_int, [c_void_p, c_int64, c_int, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int, c_void_p, c_void_p, c_float,
+                                   c_int, c_void_p, c_int64, c_float, c_int64, c_int64, c_int, c_void_p, c_int, c_void_p]),
     "ll_nvfp4_gemm_tnt_grouped": (c_int, [c_void_p, c_void_p, c_void_p, c_float, c_int64, c_int64, c_int64, c_int64,
                                           c_int64, c_int, c_void_p, c_void_p]),
     "ll_nvfp4_quantize_pair": (c_int, [c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int, c_void_p, c_void_p, c_void_p,

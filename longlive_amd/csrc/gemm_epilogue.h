@@ -189,7 +189,29 @@ inline int make_epilogue(const ll_gemm_epilogue& e, int64_t N, GemmEpilogue& epi
   }
   return LL_OK;
 }
-// Whether ll_nvfp4_gemm_tnt computes a product of these sizes in 64 x 64 tiles, K in ascending order (gemm_w4a4.hip).
-bool product_takes_plain_64x64_tiles(int64_t M, int64_t N, int64_t Kp, int cus);
+// Whether ll_nvfp4_gemm_tnt(_grouped) computes products of these sizes in 64 x 64 tiles, K in ascending order (gemm_w4a4.hip).
+bool product_takes_plain_64x64_tiles(int64_t M, int64_t N, int64_t Kp, int n_products, int cus);
+
+// Several products with the same A operand and the same N and K in one launch (the q / k / v projections of one
+// activation): the weight, its scales and tensor scale, the bias, the output and the amax sink of the products
+// behind the first one.  The column tiles of all products form one row of tiles_n tiles, tiles_n_each per product.
+constexpr int kMaxGemmGroups = 4;
+struct GemmGroup {
+  const uint8_t* Bv;
+  const uint8_t* Bs;
+  const float* alpha;
+  const float* amax_b;
+  float inv_denom_b;
+  uint16_t* D;
+  int64_t ldd;
+  const uint16_t* bias;
+  AmaxSink sink;
+};
+struct GemmGroups {
+  int n;             // number of products (1: the plain call, `more` unused)
+  int tiles_n_each;  // column tiles per product
+  GemmGroup more[kMaxGemmGroups - 1];
+};
+
 
 }  // namespace ll

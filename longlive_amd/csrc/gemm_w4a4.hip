@@ -56,27 +56,6 @@ struct GemmSmem {
   static constexpr int kStage = kAVals + kBVals + kAScales + kBScales;
 };
 
-// Several products with the same A operand and the same N and K in one launch (the q / k / v projections of one
-// activation): the weight, its scales and tensor scale, the bias, the output and the amax sink of the products
-// behind the first one.  The column tiles of all products form one row of tiles_n tiles, tiles_n_each per product.
-constexpr int kMaxGemmGroups = 4;
-struct GemmGroup {
-  const uint8_t* Bv;
-  const uint8_t* Bs;
-  const float* alpha;
-  const float* amax_b;
-  float inv_denom_b;
-  uint16_t* D;
-  int64_t ldd;
-  const uint16_t* bias;
-  AmaxSink sink;
-};
-struct GemmGroups {
-  int n;             // number of products (1: the plain call, `more` unused)
-  int tiles_n_each;  // column tiles per product
-  GemmGroup more[kMaxGemmGroups - 1];
-};
-
 template <int FA, int FB>
 __global__ __launch_bounds__(kGemmThreads, 2) void gemm_w4a4_kernel(
     const uint8_t* __restrict__ Av, const uint8_t* __restrict__ As, const uint8_t* __restrict__ Bv0,
@@ -1471,10 +1450,10 @@ static int try_persistent(const uint8_t* A_values, const uint8_t* A_scales, cons
   return LL_OK;
 }
 
-bool product_takes_plain_64x64_tiles(int64_t M, int64_t N, int64_t Kp, int cus) {
+bool product_takes_plain_64x64_tiles(int64_t M, int64_t N, int64_t Kp, int n_products, int cus) {
   const int schedule = g_gemm_schedule.load(std::memory_order_relaxed);
-  return !plan_persistent(M, N, Kp, 1, cus, schedule).use && !small_kernel_takes(Kp, schedule) &&
-         choose_tile_kernel(M, N, Kp, 1, cus, schedule).kernel == LL_GEMM_KERNEL_64X64;
+  return !plan_persistent(M, N, Kp, n_products, cus, schedule).use && !small_kernel_takes(Kp, schedule) &&
+         choose_tile_kernel(M, N, Kp, n_products, cus, schedule).kernel == LL_GEMM_KERNEL_64X64;
 }
 
 // Tile choice and launch; `groups.n` products side by side count as one product of groups.n * N columns.

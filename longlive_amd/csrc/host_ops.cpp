@@ -351,11 +351,14 @@ struct BlockCall {
     const int quantized = ll_nvfp4_quantize_from_sink(x, M, K, K, rule, q.values, q.scales, q.amax, &sink, stream);
     return quantized ? quantized : gemm(q, w, M, out, e);
   }
-  int grouped(const TempOperand& a, const Layer* const* w, int n, int64_t M, void* const* outs, const ll_amax_sink* sinks) const {
-    ll_gemm_product p[4];
+  static void products(const Layer* const* w, int n, void* const* outs, const ll_amax_sink* sinks, ll_gemm_product* p) {
     for (int i = 0; i < n; ++i)
       p[i] = ll_gemm_product{w[i]->values, w[i]->scales, nullptr, w[i]->amax, w[i]->denom, outs[i], w[i]->n, w[i]->bias,
                              sinks ? sinks[i] : ll_amax_sink{nullptr, 0, nullptr}};
+  }
+  int grouped(const TempOperand& a, const Layer* const* w, int n, int64_t M, void* const* outs, const ll_amax_sink* sinks) const {
+    ll_gemm_product p[4];
+    products(w, n, outs, sinks, p);
     return ll_nvfp4_gemm_tnt_grouped(a.values, a.scales, a.amax, denom_a, M, w[0]->n, a.mp, w[0]->np, a.kp, n, p, stream);
   }
   TempOperand operand(int64_t m, int64_t k) const { return temp_operand(m, k, dev); }
@@ -469,8 +472,7 @@ PyObject* py_block_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const int64_t sb = e.stride(0), sf = e.stride(1);
   auto modulation = [&](int i) { return mod + i * e.stride(2); };
   // LayerNorm(h) * (1 + e[scale]) + e[shift] as an NVFP4 operand: one launch, or two where the rows do not fit one
-  auto adaln_operand = [&](const void* h, int scale, int shift, const TempOperand& q) -> int {
-    const ll_amax_sink sink = ep.take();
+  auto adaln_operand = [&](const void* h, int scale, int shift, const TempOperand& q, const ll_amax_sink& sink) -> int {
     int code = ll_adaln_quantize(h, 1, L, (int)C, modulation(scale), modulation(shift), sb, sf, sb, sf, frame_rows, eps[0], 1, c.rule,
                                  q.values, q.scales, q.amax, &sink, spin, c.stream);
     if (code != LL_ENOSUP) return code;
@@ -480,8 +482,26 @@ PyObject* py_block_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
                                   y.data_ptr(), &again, c.stream);
     return code ? code : c.quantize_from(y, L, C, q, again);
   };
-  TempOperand xq = c.operand(L, C);
-  LL_TRY(adaln_operand(x.data_ptr(), 1, 0, xq), "adaLN");
+  // The layers behind a normalization of h [L, C] (adaLN with the modulation vectors `scale` and `shift`, or norm3 where scale is
+  // negative): one launch for small activations, else `operand(exchange)` and `product()`.  result_sink: the sink of the first
+  // product where it is to have a fresh epoch, which has to be newer than those of the launches before it.
+  TempOperand xq{};  // allocated by the first that needs it
+  auto normed_layers = [&](const void* h, int scale, int shift, const Layer* const* layers, int n, void* const* outs, const ll_amax_sink* sinks,
+                           ll_amax_sink* result_sink, int activation, auto operand, auto product) -> int {
+    const ll_amax_sink exchange = ep.take();
+    if (result_sink) *result_sink = ep.take();
+    ll_gemm_product p[4];
+    BlockCall::products(layers, n, outs, sinks ? sinks : result_sink, p);
+    const bool adaln = scale >= 0;
+    int code = ll_nvfp4_norm_gemm(h, L, (int)C, adaln ? modulation(scale) : nullptr, adaln ? modulation(shift) : nullptr, sf, sf, frame_rows, 1,
+                                  adaln ? nullptr : norm[2], adaln ? nullptr : norm[3], adaln ? eps[0] : eps[2], c.rule, &exchange, spin,
+                                  c.denom_a, layers[0]->n, layers[0]->np, n, p, activation, c.stream);
+    if (code != LL_ENOSUP) return code;
+    if (!xq.values) xq = c.operand(L, C);
+    if ((code = operand(exchange))) return code;
+    if (result_sink) *result_sink = ep.take();
+    return product();
+  };
 
   // ---- self-attention
   const Tensor value = empty({1, L, H, 128}, at::kBFloat16, dev), key = empty({1, L, H, 128}, at::kBFloat16, dev);
@@ -492,7 +512,10 @@ PyObject* py_block_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
     const Layer* const layers[3] = {&w[Q], &w[K], &w[V]};
     void* const outs[3] = {q.data_ptr(), k.data_ptr(), value.data_ptr()};
     const ll_amax_sink sinks[3] = {{nullptr, 0, nullptr}, {nullptr, 0, nullptr}, kv_sink[1]};
-    LL_TRY(c.grouped(xq, layers, 3, L, outs, sinks), "q / k / v projections");
+    LL_TRY(normed_layers(x.data_ptr(), 1, 0, layers, 3, outs, sinks, nullptr, LL_ACT_NONE,
+                         [&](const ll_amax_sink& sink) { return adaln_operand(x.data_ptr(), 1, 0, xq, sink); },
+                         [&] { return c.grouped(xq, layers, 3, L, outs, sinks); }),
+           "adaLN and q / k / v projections");
     const Tensor roped_q = empty({L, C}, at::kBFloat16, dev), smooth_k = empty({L, C}, at::kBFloat16, dev);
     LL_TRY(ll_qk_norm_rope_pair_amax(q.data_ptr(), k.data_ptr(), L, H, norm[0], norm[1], eps[1], cos->data_ptr<float>(),
                                      sin->data_ptr<float>(), L, roped_q.data_ptr(), key.data_ptr(), smooth_k.data_ptr(), &kv_sink[0],
@@ -525,21 +548,22 @@ PyObject* py_block_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
   LL_TRY(c.linear(attended.data_ptr(), C, attended_sink, w[O], L, x1.data_ptr(), gated, xq), "output projection");
 
   // ---- cross-attention
-  {
-    const ll_amax_sink sink = ep.take();
-    int code = ll_layer_norm_quantize(x1.data_ptr(), L, (int)C, norm[2], norm[3], eps[2], c.rule, xq.values, xq.scales,
-                                      xq.amax, &sink, spin, c.stream);
-    if (code == LL_ENOSUP) {
-      const ll_amax_sink again = ep.take();
-      const Tensor y = empty({L, C}, at::kBFloat16, dev);
-      code = ll_layer_norm(x1.data_ptr(), L, (int)C, norm[2], norm[3], eps[2], y.data_ptr(), &again, c.stream);
-      if (!code) code = c.quantize_from(y, L, C, xq, again);
-    }
-    LL_TRY(code, "norm3");
-  }
+  auto norm3_operand = [&](const ll_amax_sink& sink) -> int {
+    int code = ll_layer_norm_quantize(x1.data_ptr(), L, (int)C, norm[2], norm[3], eps[2], c.rule, xq.values, xq.scales, xq.amax, &sink, spin,
+                                      c.stream);
+    if (code != LL_ENOSUP) return code;
+    const ll_amax_sink again = ep.take();
+    const Tensor y = empty({L, C}, at::kBFloat16, dev);
+    code = ll_layer_norm(x1.data_ptr(), L, (int)C, norm[2], norm[3], eps[2], y.data_ptr(), &again, c.stream);
+    return code ? code : c.quantize_from(y, L, C, xq, again);
+  };
   {
     const Tensor q = empty({L, C}, at::kBFloat16, dev), qn = empty({L, C}, at::kBFloat16, dev);
-    LL_TRY(c.gemm(xq, w[CQ], L, q.data_ptr(), plain_epilogue), "cross-attention q");
+    const Layer* const layers[1] = {&w[CQ]};
+    void* const outs[1] = {q.data_ptr()};
+    LL_TRY(normed_layers(x1.data_ptr(), -1, -1, layers, 1, outs, nullptr, nullptr, LL_ACT_NONE, norm3_operand,
+                         [&] { return c.gemm(xq, w[CQ], L, q.data_ptr(), plain_epilogue); }),
+           "norm3 and cross-attention q");
     LL_TRY(ll_rms_norm(q.data_ptr(), L, (int)C, norm[4], eps[3], qn.data_ptr(), c.stream), "cross-attention norm_q");
     if (context) {
       const TempOperand tq = c.operand(T, C);
@@ -566,12 +590,17 @@ PyObject* py_block_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
   LL_TRY(c.linear(attended.data_ptr(), C, attended_sink, w[CO], L, x2.data_ptr(), residual, xq), "cross-attention output projection");
 
   // ---- feed-forward
-  LL_TRY(adaln_operand(x2.data_ptr(), 4, 3, xq), "adaLN");
   const Tensor hidden = empty({L, w[UP].n}, at::kBFloat16, dev);
   ll_gemm_epilogue gelu{};
   gelu.activation = LL_ACT_GELU_TANH;
-  gelu.amax_sink = ep.take();
-  LL_TRY(c.gemm(xq, w[UP], L, hidden.data_ptr(), gelu), "FFN up");
+  {
+    const Layer* const layers[1] = {&w[UP]};
+    void* const outs[1] = {hidden.data_ptr()};
+    LL_TRY(normed_layers(x2.data_ptr(), 4, 3, layers, 1, outs, nullptr, &gelu.amax_sink, LL_ACT_GELU_TANH,
+                         [&](const ll_amax_sink& sink) { return adaln_operand(x2.data_ptr(), 4, 3, xq, sink); },
+                         [&] { return c.gemm(xq, w[UP], L, hidden.data_ptr(), gelu); }),
+           "adaLN and FFN up");
+  }
   TempOperand hq{};
   const Tensor& out = attended;  // its memory is free by now
   gated.gate = modulation(5);

@@ -183,6 +183,16 @@ __device__ __forceinline__ float wave_sum_dpp(float v) {
   LL_DPP_ADD(v, 0x143, 0xC, 0xF);  // row_bcast:31 into rows 2 and 3
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
 }
+// The same over each half of the wave, in all lanes of it: the bits that wave_sum_dpp has for 32 values and zeros behind them.
+__device__ __forceinline__ float half_wave_sum_dpp(float v) {
+  LL_DPP_ADD(v, 0x111, 0xF, 0xF);
+  LL_DPP_ADD(v, 0x112, 0xF, 0xF);
+  LL_DPP_ADD(v, 0x114, 0xF, 0xE);
+  LL_DPP_ADD(v, 0x118, 0xF, 0xC);
+  LL_DPP_ADD(v, 0x142, 0xA, 0xF);
+  const int lower = __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 31), upper = __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63);
+  return __builtin_bit_cast(float, (threadIdx.x & 32) ? upper : lower);
+}
 // Sum over 16 neighbouring lanes, in every one of them: over lanes 1, 2, 4 and 8 apart in turn.  (When the lanes of a quad agree, the
 // mirrored lane of the other quad stands for the one 4 apart, and likewise for 8.)
 __device__ __forceinline__ float sum_over_16_lanes(float v) {

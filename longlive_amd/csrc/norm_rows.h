@@ -92,26 +92,24 @@ __device__ __forceinline__ float unpack_row(const uint4 (&raw)[NCH], int nchunks
   }
   return sum;
 }
+template <bool HALF>
+__device__ __forceinline__ float row_sum(float v) {
+  return HALF ? half_wave_sum_dpp(v) : wave_sum_dpp(v);
+}
 // adaLN modulation of one row, utils/adaln_triton.py:36-86: LayerNorm without affine in fp32, rounded to bf16,
 // times (1 + scale) rounded, plus shift rounded.  `packed[i]` receives the 8 results of group lane + 64 i; the
 // return value is the lane's share of the row's absolute maximum.  Two values share a rounding's conversion: adaln_kernel took
 // 9.6 us for 2640 x 3072 so (before load_row), with one each 10.2.
-template <int NCH>
-__device__ __forceinline__ float adaln_row(const uint16_t* __restrict__ xr, const uint16_t* __restrict__ scr,
-                                           const uint16_t* __restrict__ shr, int C, float eps, int add_one, int lane,
-                                           uint4 (&packed)[NCH]) {
+// HALF: a row per half of the wave, lane 0 .. 31 of it, NCH = 1: rows of up to 256 elements, the same bits.
+template <int NCH, bool HALF = false>
+__device__ __forceinline__ float adaln_loaded_row(const uint4 (&xraw)[NCH], uint4 (&sraw)[NCH], uint4 (&hraw)[NCH],
+                                                  const uint16_t* __restrict__ scr, const uint16_t* __restrict__ shr, int C, float eps,
+                                                  int add_one, int lane, uint4 (&packed)[NCH]) {
   const int nchunks = C >> 3;
   float v[NCH][8];
-  uint4 xraw[NCH], sraw[NCH], hraw[NCH];
-  load_row<NCH>(xr, nchunks, lane, xraw);
-  if (kOperandsAhead<NCH>) {
-    load_row<NCH>(scr, nchunks, lane, sraw);
-    load_row<NCH>(shr, nchunks, lane, hraw);
-  }
-  __builtin_amdgcn_sched_barrier(0);  // all loads are under way
   const float sum = unpack_row<NCH>(xraw, nchunks, lane, v);
   const float inv_c = 1.0f / (float)C;
-  const float mean = wave_sum_dpp(sum) * inv_c;
+  const float mean = row_sum<HALF>(sum) * inv_c;
   float sq = 0.0f;
 #pragma unroll
   for (int i = 0; i < NCH; ++i) {
@@ -124,7 +122,7 @@ __device__ __forceinline__ float adaln_row(const uint16_t* __restrict__ xr, cons
       }
     }
   }
-  const float var = wave_sum_dpp(sq) * inv_c;
+  const float var = row_sum<HALF>(sq) * inv_c;
   const float rstd = 1.0f / sqrtf(var + eps);
   float out_max = 0.0f;
 #pragma unroll
@@ -161,27 +159,32 @@ __device__ __forceinline__ float adaln_row(const uint16_t* __restrict__ xr, cons
   return out_max;
 }
 
+template <int NCH>
+__device__ __forceinline__ float adaln_row(const uint16_t* __restrict__ xr, const uint16_t* __restrict__ scr,
+                                           const uint16_t* __restrict__ shr, int C, float eps, int add_one, int lane,
+                                           uint4 (&packed)[NCH]) {
+  const int nchunks = C >> 3;
+  uint4 xraw[NCH], sraw[NCH], hraw[NCH];
+  load_row<NCH>(xr, nchunks, lane, xraw);
+  if (kOperandsAhead<NCH>) {
+    load_row<NCH>(scr, nchunks, lane, sraw);
+    load_row<NCH>(shr, nchunks, lane, hraw);
+  }
+  __builtin_amdgcn_sched_barrier(0);  // all loads are under way
+  return adaln_loaded_row<NCH>(xraw, sraw, hraw, scr, shr, C, eps, add_one, lane, packed);
+}
+
 // LayerNorm with optional weight and bias of one row, wan_5b/modules/model.py:101-111 (nn.LayerNorm on bf16
 // tensors: statistics and the affine map in fp32, one rounding to bf16 at the end).
-template <int NCH>
-__device__ __forceinline__ float layernorm_row(const uint16_t* __restrict__ xr, const uint16_t* __restrict__ w,
-                                               const uint16_t* __restrict__ b, int C, float eps, int lane,
-                                               uint4 (&packed)[NCH]) {
+template <int NCH, bool HALF = false>
+__device__ __forceinline__ float layernorm_loaded_row(const uint4 (&xraw)[NCH], uint4 (&wraw)[NCH], uint4 (&braw)[NCH],
+                                                      const uint16_t* __restrict__ w, const uint16_t* __restrict__ b, int C, float eps,
+                                                      int lane, uint4 (&packed)[NCH]) {
   const int nchunks = C >> 3;
   float v[NCH][8];
-  uint4 xraw[NCH], wraw[NCH], braw[NCH];
-#pragma unroll
-  for (int i = 0; i < NCH; ++i) {
-    wraw[i] = make_uint4(0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u);
-    braw[i] = make_uint4(0u, 0u, 0u, 0u);
-  }
-  load_row<NCH>(xr, nchunks, lane, xraw);
-  if (kOperandsAhead<NCH> && w) load_row<NCH>(w, nchunks, lane, wraw);
-  if (kOperandsAhead<NCH> && b) load_row<NCH>(b, nchunks, lane, braw);
-  __builtin_amdgcn_sched_barrier(0);  // all loads are under way
   const float sum = unpack_row<NCH>(xraw, nchunks, lane, v);
   const float inv_c = 1.0f / (float)C;
-  const float mean = wave_sum_dpp(sum) * inv_c;
+  const float mean = row_sum<HALF>(sum) * inv_c;
   float sq = 0.0f;
 #pragma unroll
   for (int i = 0; i < NCH; ++i) {
@@ -194,7 +197,7 @@ __device__ __forceinline__ float layernorm_row(const uint16_t* __restrict__ xr, 
       }
     }
   }
-  const float var = wave_sum_dpp(sq) * inv_c;
+  const float var = row_sum<HALF>(sq) * inv_c;
   const float rstd = 1.0f / sqrtf(var + eps);
   float out_max = 0.0f;
 #pragma unroll
@@ -213,6 +216,30 @@ __device__ __forceinline__ float layernorm_row(const uint16_t* __restrict__ xr, 
     }
   }
   return out_max;
+}
+
+// The weight and bias of a LayerNorm for the lane's groups: ones and zeros where there is none.
+template <int NCH>
+__device__ __forceinline__ void load_affine(const uint16_t* __restrict__ w, const uint16_t* __restrict__ b, int nchunks, int lane,
+                                            uint4 (&wraw)[NCH], uint4 (&braw)[NCH]) {
+#pragma unroll
+  for (int i = 0; i < NCH; ++i) {
+    wraw[i] = make_uint4(0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u);
+    braw[i] = make_uint4(0u, 0u, 0u, 0u);
+  }
+  if (kOperandsAhead<NCH> && w) load_row<NCH>(w, nchunks, lane, wraw);
+  if (kOperandsAhead<NCH> && b) load_row<NCH>(b, nchunks, lane, braw);
+}
+template <int NCH>
+__device__ __forceinline__ float layernorm_row(const uint16_t* __restrict__ xr, const uint16_t* __restrict__ w,
+                                               const uint16_t* __restrict__ b, int C, float eps, int lane,
+                                               uint4 (&packed)[NCH]) {
+  const int nchunks = C >> 3;
+  uint4 xraw[NCH], wraw[NCH], braw[NCH];
+  load_row<NCH>(xr, nchunks, lane, xraw);
+  load_affine<NCH>(w, b, nchunks, lane, wraw, braw);
+  __builtin_amdgcn_sched_barrier(0);  // all loads are under way
+  return layernorm_loaded_row<NCH>(xraw, wraw, braw, w, b, C, eps, lane, packed);
 }
 
 }  // namespace ll

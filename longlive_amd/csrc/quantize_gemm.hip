@@ -10,13 +10,15 @@
 // 12.2 / 7.6 and 12.3 / 7.6.
 #include "ll_common.h"
 #include "gemm_epilogue.h"
-#include "quantize_block.h"  // from here on without floating-point contraction
+#include "amax_exchange.h"
+#include "norm_rows.h"       // from here on without floating-point contraction
+#include "quantize_block.h"
 
 namespace ll {
 
 constexpr int kFusedThreads = 256;  // eight waves: 48 x 256 x 512 7.2 instead of 6.1 us, 64 x 512 x 512 11.2 instead of 9.5
 constexpr int kFusedRows = 32, kFusedCols = 32 * (kFusedThreads / 64);  // of a workgroup's tile: a wave multiplies all rows and 32 columns
-constexpr int kFusedMaxK = 512;
+constexpr int kFusedMaxK = 512, kNormMaxK = 256;
 constexpr int kFusedPatch = 32 * (64 + 16);       // bytes of a wave's patch in the epilogue
 
 struct FusedParams {
@@ -33,22 +35,65 @@ struct FusedParams {
   int64_t ldd;
   GemmEpilogue epi;
 };
+// The rows are normalized first: adaLN modulation (a, b: scale and shift, a row per frame) or LayerNorm (weight and bias, or null),
+// for up to kMaxGemmGroups products of tiles_n_each column tiles each.
+struct NormFusedParams : FusedParams {
+  const uint16_t *a, *b;
+  int64_t a_stride, b_stride;
+  int frame_rows, add_one;
+  float eps;
+  AmaxSink exchange;
+  uint32_t spin_limit;
+  int recompute;
+  int tiles_n_each;
+  GemmGroup more[kMaxGemmGroups - 1];
+};
+enum { kPlainRows, kAdalnRows, kLayerNormRows };
+template <int ROWS>
+struct FusedParamsOf {
+  typedef NormFusedParams type;
+};
+template <>
+struct FusedParamsOf<kPlainRows> {
+  typedef FusedParams type;
+};
+constexpr int fused_threads(int rows) { return rows == kPlainRows ? kFusedThreads : 2 * kFusedThreads; }
+constexpr int fused_waves(int rows) { return rows == kPlainRows ? 1 : 4; }  // per SIMD: two workgroups with an exchange are resident
+constexpr int kExchangeSlots = kAmaxParts / 2;  // of a sink: a launch whose workgroups exchange maxima leaves its results' in the others
 
 // T: 64 elements of K at most, a wave's weights in registers.  Quantization is the arithmetic of quantize_kernel, the product
 // the order of gemm_w4a4_kernel<1, 1> (64 elements of K after 64, dword after dword of the lanes' pieces): the same bits.
 // Bound by the chain: one trip to memory for x, weights and maximum together, the scale table, a few hundred instructions per
 // block of 16 (229 a block and lane), the products, the store.
-template <int RULE, int T>
-__global__ __launch_bounds__(kFusedThreads) void quantize_gemm_kernel(FusedParams p) {
+//
+// ROWS other than kPlainRows: the rows are normalized here too, and the tensor maximum is exchanged between the row tiles
+// (amax_exchange.h); for the pairs adaLN - q / k / v or FFN up and norm3 - cross-attention q of a small model's block, a launch of 5 to 6 us
+// each.  Every column tile normalizes its rows again, 32 rows on one compute unit, so the instructions of a row count: rows
+// of up to 256 elements lie two to a wave (norm_rows.h, the same bits), four more waves join in up to the products.  A
+// block of 192 rows, dim 256, in two launches each 90.2 us, with a wave per row and four waves 92, with eight 85, so 80.1; of 768
+// rows 104.3 / 97.2.  Of 192 rows, dim 512 (a wave per row, eight waves): 108 / 115, hence kNormMaxK.
+template <int RULE, int T, int ROWS>
+__global__ __launch_bounds__(fused_threads(ROWS), fused_waves(ROWS)) void quantize_gemm_kernel(typename FusedParamsOf<ROWS>::type p) {
+  constexpr bool kNorm = ROWS != kPlainRows;
+  constexpr int kThreads = fused_threads(ROWS), kRowPitch = 128 * T + 16, kWaveRows = kFusedRows / (kThreads / 64);
+  __shared__ __attribute__((aligned(16))) uint8_t s_rows[kNorm ? kFusedRows * kRowPitch : 16];  // normalized, bf16
+  __shared__ AmaxExchangeSmem s_exchange;
   constexpr int kPitch = 32 * T + 16, kScalePitch = 4 * T + 2;
-  constexpr int kRowBlocks = 4 * T, kBlocks = kFusedRows * kRowBlocks / kFusedThreads;  // per row; per thread, at most
+  constexpr int kRowBlocks = 4 * T, kBlocks = kFusedRows * kRowBlocks / kThreads;  // per row; per thread, at most
   __shared__ float s_red[kFusedThreads / 64];
   __shared__ ScaleEntry s_tab[128];
   __shared__ __attribute__((aligned(16))) uint8_t s_values[kFusedRows * kPitch];
   __shared__ __attribute__((aligned(16))) uint8_t s_scales[kFusedRows * kScalePitch];
   __shared__ __attribute__((aligned(16))) uint8_t s_patch[kFusedThreads / 64 * kFusedPatch];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l32 = lane & 31, lh = lane >> 5;
-  const int tile_n = blockIdx.x / p.tiles_m, tile_m = blockIdx.x - tile_n * p.tiles_m;
+  GemmGroup pr{p.Bv, p.Bs, nullptr, p.amax_b, p.inv_denom_b, p.D, p.ldd, p.epi.bias, p.epi.sink};
+  int tile_n = blockIdx.x / p.tiles_m;
+  const int tile_m = blockIdx.x - tile_n * p.tiles_m;
+  if constexpr (kNorm) {
+    const int g = tile_n / p.tiles_n_each;
+    tile_n -= g * p.tiles_n_each;
+    if (g > 0) pr = p.more[g - 1];
+  }
   const int row0 = tile_m * kFusedRows, col0 = tile_n * kFusedCols + 32 * wave;
   const int steps = p.K >> 6, row_blocks = p.K >> 4;
 
@@ -58,21 +103,39 @@ __global__ __launch_bounds__(kFusedThreads) void quantize_gemm_kernel(FusedParam
   int block_row[kBlocks], block_col[kBlocks];
 #pragma unroll
   for (int i = 0; i < kBlocks; ++i) {
-    const int b = tid + i * kFusedThreads;
+    const int b = tid + i * kThreads;
     block_row[i] = b / row_blocks;
     block_col[i] = b - block_row[i] * row_blocks;
+    if constexpr (kNorm) continue;
     const int row = min(row0 + block_row[i], p.M - 1);
     const u32x4* src = reinterpret_cast<const u32x4*>(p.x + (int64_t)row * p.ldx + block_col[i] * 16);
     lo[i] = src[0];
     hi[i] = src[1];
   }
+  // normalized rows: the wave's eight rows of the tile (behind the last row: the last again), with their operands
+  constexpr int kPairs = kWaveRows / 2;
+  uint4 xraw[kPairs][1], araw[kPairs][1], braw[kPairs][1];
+  if constexpr (kNorm) {
+    const int nchunks = p.K >> 3;
+#pragma unroll
+    for (int i = 0; i < kPairs; ++i) {
+      const int row = min(row0 + wave * kWaveRows + 2 * i + lh, p.M - 1);
+      load_row<1>(p.x + (int64_t)row * p.ldx, nchunks, l32, xraw[i]);
+      if constexpr (ROWS == kAdalnRows) {
+        const int f = row / p.frame_rows;
+        load_row<1>(p.a + f * p.a_stride, nchunks, l32, araw[i]);
+        load_row<1>(p.b + f * p.b_stride, nchunks, l32, braw[i]);
+      }
+    }
+    if constexpr (ROWS == kLayerNormRows) load_affine<1>(p.a, p.b, nchunks, l32, araw[0], braw[0]);
+  }
   // the wave's weights: row l32 of its 32, pieces 2 t + lh of 16 bytes and the scales of their two blocks
   uint4 bv[T];
   uint32_t bs[T];
-  {
+  if (!kNorm || wave < kFusedThreads / 64) {
     const int n = min(col0 + l32, p.Np - 1);
-    const uint8_t* values = p.Bv + (int64_t)n * (p.K >> 1) + 16 * lh;
-    const uint8_t* scales = p.Bs + (int64_t)(n >> 7) * (p.K >> 6) * 512 + (n & 31) * 16 + ((n & 127) >> 5) * 4 + 2 * lh;
+    const uint8_t* values = pr.Bv + (int64_t)n * (p.K >> 1) + 16 * lh;
+    const uint8_t* scales = pr.Bs + (int64_t)(n >> 7) * (p.K >> 6) * 512 + (n & 31) * 16 + ((n & 127) >> 5) * 4 + 2 * lh;
 #pragma unroll
     for (int t = 0; t < T; ++t) {
       const int at = min(t, steps - 1);
@@ -80,8 +143,35 @@ __global__ __launch_bounds__(kFusedThreads) void quantize_gemm_kernel(FusedParam
       bs[t] = *reinterpret_cast<const uint16_t*>(scales + 512 * at);
     }
   }
-  float part = 0.0f;
-  if (p.sink_parts) {
+  float part = 0.0f, amax;
+  if constexpr (kNorm) {
+    __builtin_amdgcn_sched_barrier(0);  // all loads are under way
+#pragma unroll
+    for (int i = 0; i < kPairs; ++i) {
+      uint4 packed[1];
+      if constexpr (ROWS == kAdalnRows)
+        part = fmaxf(part, adaln_loaded_row<1, true>(xraw[i], araw[i], braw[i], nullptr, nullptr, p.K, p.eps, p.add_one, l32, packed));
+      else
+        part = fmaxf(part, layernorm_loaded_row<1, true>(xraw[i], araw[0], braw[0], nullptr, nullptr, p.K, p.eps, l32, packed));
+      if (l32 < p.K >> 3) *reinterpret_cast<uint4*>(s_rows + (wave * kWaveRows + 2 * i + lh) * kRowPitch + 16 * l32) = packed[0];
+    }
+    // The column tiles of a row have the same maximum and share its slot.
+    amax = exchange_amax(p.exchange, (uint32_t)p.tiles_m, (uint32_t)tile_m, part, p.spin_limit, p.recompute != 0, s_exchange, [&](uint32_t s) {
+      float m = 0.0f;
+#pragma unroll 1
+      for (int i = 0; i < kWaveRows; ++i) {
+        const int row = min((int)s * kFusedRows + wave * kWaveRows + i, p.M - 1);
+        uint4 packed[1];
+        if constexpr (ROWS == kAdalnRows) {
+          const int f = row / p.frame_rows;
+          m = fmaxf(m, adaln_row<1>(p.x + (int64_t)row * p.ldx, p.a + f * p.a_stride, p.b + f * p.b_stride, p.K, p.eps, p.add_one, lane, packed));
+        } else {
+          m = fmaxf(m, layernorm_row<1>(p.x + (int64_t)row * p.ldx, p.a, p.b, p.K, p.eps, lane, packed));
+        }
+      }
+      return m;
+    });
+  } else if (p.sink_parts) {
     const uint32_t epoch = amax_sink_epoch(p.sink_epoch, p.sink_epoch_offset);
 #pragma unroll
     for (int i = 0; i < kAmaxParts / kFusedThreads; ++i) part = fmaxf(part, amax_sink_read(p.sink_parts, epoch, i * kFusedThreads + tid));
@@ -99,12 +189,14 @@ __global__ __launch_bounds__(kFusedThreads) void quantize_gemm_kernel(FusedParam
       for (int i = 0; i < 8; ++i) part = abs_max_bf16x8(v[i], part);
     }
   }
-  part = wave_max(part);
-  if (lane == 0) s_red[wave] = part;
-  __syncthreads();
-  float amax = s_red[0];
+  if constexpr (!kNorm) {
+    part = wave_max(part);
+    if (lane == 0) s_red[wave] = part;
+    __syncthreads();
+    amax = s_red[0];
 #pragma unroll
-  for (int i = 1; i < kFusedThreads / 64; ++i) amax = fmaxf(amax, s_red[i]);
+    for (int i = 1; i < kFusedThreads / 64; ++i) amax = fmaxf(amax, s_red[i]);
+  }
 
   // ---- quantization of the 32 rows into LDS (the prologue and the paths of quantize_kernel)
   constexpr bool kStaticRule = (RULE == LL_RULE_STATIC_6 || RULE == LL_RULE_STATIC_4);
@@ -124,6 +216,11 @@ __global__ __launch_bounds__(kFusedThreads) void quantize_gemm_kernel(FusedParam
     for (int j = 1; j < kBlocks; ++j)
       if (i == j) l = lo[j], h = hi[j], row = block_row[j], col = block_col[j];
     if (row >= kFusedRows) break;
+    if constexpr (kNorm) {
+      const u32x4* src = reinterpret_cast<const u32x4*>(s_rows + row * kRowPitch + col * 32);
+      l = src[0];
+      h = src[1];
+    }
     float X[16];
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
@@ -138,7 +235,7 @@ __global__ __launch_bounds__(kFusedThreads) void quantize_gemm_kernel(FusedParam
     s_scales[row * kScalePitch + col] = (uint8_t)sb;
   }
   __syncthreads();
-  if (col0 >= p.N) return;
+  if ((kNorm && wave >= kFusedThreads / 64) || col0 >= p.N) return;
 
   // ---- product: 32 x 32 per wave
   float16v acc[1][1];
@@ -158,17 +255,30 @@ __global__ __launch_bounds__(kFusedThreads) void quantize_gemm_kernel(FusedParam
       acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(decode8(b[j], half2v{ws[j >> 1], ws[j >> 1]}),
                                                          decode8(a[j], half2v{as[j >> 1], as[j >> 1]}), acc[0][0], 0, 0, 0);
   }
-  const float alpha = (amax * p.amax_b[0]) * (p.inv_denom_a * p.inv_denom_b);
-  gemm_epilogue<1, 1, 4>(acc, alpha, s_patch, wave, lane, row0, col0, p.M, p.N, p.D, p.ldd, p.epi.bias, p.epi.act, p.epi,
-                         (uint32_t)blockIdx.x * (kFusedThreads / 64) + wave);
+  const float alpha = (amax * pr.amax_b[0]) * (p.inv_denom_a * pr.inv_denom_b);
+  GemmEpilogue epi = p.epi;
+  epi.sink = pr.sink;
+  const uint32_t slot = (uint32_t)blockIdx.x * (kFusedThreads / 64) + wave;
+  gemm_epilogue<1, 1, 4>(acc, alpha, s_patch, wave, lane, row0, col0, p.M, p.N, pr.D, pr.ldd, pr.bias, p.epi.act, epi,
+                         kNorm ? kExchangeSlots + slot % (kAmaxParts - kExchangeSlots) : slot);
 }
 
-template <int RULE>
-void launch_quantize_gemm(const FusedParams& p, unsigned grid, hipStream_t s) {
-  if (p.K <= 256)
-    hipLaunchKernelGGL((quantize_gemm_kernel<RULE, 4>), dim3(grid), dim3(kFusedThreads), 0, s, p);
-  else
-    hipLaunchKernelGGL((quantize_gemm_kernel<RULE, 8>), dim3(grid), dim3(kFusedThreads), 0, s, p);
+template <int RULE, int ROWS>
+void launch_rows(const typename FusedParamsOf<ROWS>::type& p, unsigned grid, hipStream_t s) {
+  if (ROWS != kPlainRows || p.K <= kNormMaxK)
+    hipLaunchKernelGGL((quantize_gemm_kernel<RULE, kNormMaxK / 64, ROWS>), dim3(grid), dim3(fused_threads(ROWS)), 0, s, p);
+  else if constexpr (ROWS == kPlainRows)
+    hipLaunchKernelGGL((quantize_gemm_kernel<RULE, kFusedMaxK / 64, ROWS>), dim3(grid), dim3(fused_threads(ROWS)), 0, s, p);
+}
+template <int ROWS>
+void launch_quantize_gemm(const typename FusedParamsOf<ROWS>::type& p, int rule, unsigned grid, hipStream_t s) {
+  switch (rule) {
+    case LL_RULE_STATIC_6: launch_rows<LL_RULE_STATIC_6, ROWS>(p, grid, s); break;
+    case LL_RULE_STATIC_4: launch_rows<LL_RULE_STATIC_4, ROWS>(p, grid, s); break;
+    case LL_RULE_MAE: launch_rows<LL_RULE_MAE, ROWS>(p, grid, s); break;
+    case LL_RULE_MSE: launch_rows<LL_RULE_MSE, ROWS>(p, grid, s); break;
+    default: launch_rows<LL_RULE_ABS_MAX, ROWS>(p, grid, s); break;
+  }
 }
 
 }  // namespace ll
@@ -200,7 +310,7 @@ extern "C" int ll_nvfp4_quantize_gemm(const void* x, int64_t M, int64_t K, int64
     return LL_ELAUNCH;
   }
   if (int rc = compute_units_of(dev, cus, "ll_nvfp4_quantize_gemm")) return rc;
-  if (!product_takes_plain_64x64_tiles(M, N, K, cus)) return LL_ENOSUP;
+  if (!product_takes_plain_64x64_tiles(M, N, K, 1, cus)) return LL_ENOSUP;
   // More than one workgroup per unit of the longer rows, whose quantization is then repeated in turn: 1760 x 512 x 512, 220
   // workgroups, 10.6 / 10.1, 2640 x 512 x 512, 332, 12.0 / 13.1; but 5280 x 256 x 256, 330, 10.3 / 8.7.
   const int64_t grid = ((M + kFusedRows - 1) / kFusedRows) * ((N + kFusedCols - 1) / kFusedCols);
@@ -224,14 +334,87 @@ extern "C" int ll_nvfp4_quantize_gemm(const void* x, int64_t M, int64_t K, int64
   p.tiles_m = (int)((M + kFusedRows - 1) / kFusedRows);
   p.D = static_cast<uint16_t*>(D);
   p.ldd = ldd;
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  switch (rule) {
-    case LL_RULE_STATIC_6: launch_quantize_gemm<LL_RULE_STATIC_6>(p, (unsigned)grid, s); break;
-    case LL_RULE_STATIC_4: launch_quantize_gemm<LL_RULE_STATIC_4>(p, (unsigned)grid, s); break;
-    case LL_RULE_MAE: launch_quantize_gemm<LL_RULE_MAE>(p, (unsigned)grid, s); break;
-    case LL_RULE_MSE: launch_quantize_gemm<LL_RULE_MSE>(p, (unsigned)grid, s); break;
-    default: launch_quantize_gemm<LL_RULE_ABS_MAX>(p, (unsigned)grid, s); break;
+  launch_quantize_gemm<kPlainRows>(p, rule, (unsigned)grid, static_cast<hipStream_t>(stream));
+  LL_CHECK_LAUNCH("quantize_gemm_kernel");
+  return LL_OK;
+}
+
+extern "C" int ll_nvfp4_norm_gemm(const void* x, int64_t M, int C, const void* scale, const void* shift, int64_t scale_stride,
+                                  int64_t shift_stride, int64_t frame_rows, int add_one_to_scale, const void* weight, const void* bias, float eps,
+                                  int rule, const ll_amax_sink* exchange, int64_t spin_limit, float denom_a, int64_t N, int64_t Np,
+                                  int n_products, const ll_gemm_product* products, int activation, void* stream) {
+  using namespace ll;
+  const char* what = "ll_nvfp4_norm_gemm";
+  LL_REQUIRE(x && products && (scale != nullptr) == (shift != nullptr) && !(scale && (weight || bias)), "%s: null pointer, or both kinds of normalization", what);
+  LL_REQUIRE(M > 0 && C > 0 && N > 0 && Np % 128 == 0 && N <= Np && denom_a > 0.f && n_products >= 1 && n_products <= kMaxGemmGroups &&
+                 (!scale || (frame_rows > 0 && M % frame_rows == 0)),
+             "%s: bad shape M=%lld C=%d N=%lld Np=%lld frame_rows=%lld, %d products", what, (long long)M, C, (long long)N, (long long)Np,
+             (long long)frame_rows, n_products);
+  LL_REQUIRE(rule >= 0 && rule <= 4, "%s: unknown scale rule %d", what, rule);
+  LL_REQUIRE(exchange && exchange->parts && sink_is_valid(exchange), "%s: an amax sink (8-byte aligned buffer, non-zero epoch) is required", what);
+  LL_REQUIRE(((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(scale) | reinterpret_cast<uintptr_t>(shift) |
+               reinterpret_cast<uintptr_t>(weight) | reinterpret_cast<uintptr_t>(bias)) & 15) == 0 && scale_stride % 8 == 0 && shift_stride % 8 == 0,
+             "%s: inputs must be 16-byte aligned, strides multiples of 8 elements", what);
+  NormFusedParams p{};
+  for (int i = 0; i < n_products; ++i) {
+    const ll_gemm_product& pr = products[i];
+    LL_REQUIRE(pr.B_values && pr.B_scales && pr.amax_b && pr.D && pr.ldd >= N && pr.denom_b > 0.f && !pr.alpha,
+               "%s: product %d: null pointer, ldd < N or an alpha", what, i);
+    LL_REQUIRE(((reinterpret_cast<uintptr_t>(pr.B_values) | reinterpret_cast<uintptr_t>(pr.B_scales)) & 15) == 0 &&
+                   (reinterpret_cast<uintptr_t>(pr.D) & 1) == 0 && (reinterpret_cast<uintptr_t>(pr.bias) & 1) == 0,
+               "%s: product %d: operands must be 16-byte, D and bias 2-byte aligned", what, i);
+    ll_gemm_epilogue e{};
+    e.bias = pr.bias;
+    e.activation = activation;
+    e.amax_sink = pr.amax_sink;
+    GemmEpilogue epi;
+    if (int rc = make_epilogue(e, N, epi)) return rc;
+    if (i == 0) {
+      p.epi = epi;
+      p.Bv = pr.B_values;
+      p.Bs = pr.B_scales;
+      p.amax_b = pr.amax_b;
+      p.inv_denom_b = 1.0f / pr.denom_b;
+      p.D = static_cast<uint16_t*>(pr.D);
+      p.ldd = pr.ldd;
+    } else {
+      p.more[i - 1] = GemmGroup{pr.B_values, pr.B_scales, nullptr, pr.amax_b, 1.0f / pr.denom_b, static_cast<uint16_t*>(pr.D), pr.ldd, epi.bias, epi.sink};
+    }
   }
+  if (C % 64 != 0 || C > kNormMaxK || M > (1 << 20) || N > (1 << 20)) return LL_ENOSUP;
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess) {
+    set_error("%s: hipGetDevice failed", what);
+    return LL_ELAUNCH;
+  }
+  if (int rc = compute_units_of(dev, cus, what)) return rc;
+  if (!product_takes_plain_64x64_tiles(M, N, C, n_products, cus)) return LL_ENOSUP;
+  const int64_t tiles_m = (M + kFusedRows - 1) / kFusedRows, tiles_n = (N + kFusedCols - 1) / kFusedCols;
+  const int64_t grid = tiles_m * tiles_n * n_products;
+  // Where the launch is ahead of two: while all its workgroups are resident, two per unit (a block of 2688 rows, dim 256, with one per
+  // unit 146.6 us, so 142.5, in two launches each 153; of 1536 rows 110.9, 106.3).
+  if (grid > 2 * (int64_t)cus || tiles_m > kExchangeSlots) return LL_ENOSUP;
+  p.x = static_cast<const uint16_t*>(x);
+  p.ldx = C;
+  p.inv_denom_a = 1.0f / denom_a;
+  p.M = (int)M;
+  p.N = (int)N;
+  p.K = C;
+  p.Np = (int)Np;
+  p.tiles_m = (int)tiles_m;
+  p.tiles_n_each = (int)tiles_n;
+  p.a = static_cast<const uint16_t*>(scale ? scale : weight);
+  p.b = static_cast<const uint16_t*>(scale ? shift : bias);
+  p.a_stride = scale_stride;
+  p.b_stride = shift_stride;
+  p.frame_rows = (int)frame_rows;
+  p.add_one = add_one_to_scale;
+  p.eps = eps;
+  p.exchange = make_sink(exchange);
+  p.spin_limit = spin_limit < 0 ? 0u : (spin_limit > 0x7FFFFFFF ? 0x7FFFFFFFu : (uint32_t)spin_limit);
+  p.recompute = spin_limit < 0 ? 1 : 0;
+  if (scale) launch_quantize_gemm<kAdalnRows>(p, rule, (unsigned)grid, static_cast<hipStream_t>(stream));
+  else launch_quantize_gemm<kLayerNormRows>(p, rule, (unsigned)grid, static_cast<hipStream_t>(stream));
   LL_CHECK_LAUNCH("quantize_gemm_kernel");
   return LL_OK;
 }

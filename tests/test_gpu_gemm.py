@@ -732,6 +732,55 @@ def test_small_layer_in_one_launch_equals_quantization_and_product(gpu, M, K, N,
     assert torch.equal(got, want)
 
 
+@pytest.mark.parametrize("rule,spin_limit", [("mse", None), ("mse", 0), ("mse", -1), ("mae", None), ("abs_max", None), ("static_6", None), ("static_4", -1)])
+@pytest.mark.parametrize("M,C,N,groups,frames,act", [
+    (1, 64, 8, 1, 1, 0),        # one row, the shortest
+    (33, 128, 136, 1, 3, 1),    # a second row of tiles with one row, ragged columns, GELU, a frame's rows across tiles
+    (192, 256, 256, 3, 3, 0),   # three products
+    (70, 192, 264, 2, 1, 0),    # the K range not full, two products
+    (2001, 256, 256, 3, 3, 0),  # two workgroups on some compute units
+])
+def test_normalization_and_small_layers_in_one_launch_equal_the_separate_launches(gpu, M, C, N, groups, frames, act, rule, spin_limit):
+    """Bit for bit, adaLN and LayerNorm with and without weight, over the ends of tiles, rows and K; results' maxima in a later epoch
+    of the buffer through which the workgroups exchange theirs; with workgroups that do not wait for the others."""
+    x = activations((M, C), M + C).to(gpu)
+    modulation = [activations((1, frames, 1, C), 50 + i).to(gpu) * 0.3 for i in range(2)]
+    affine = [activations((C,), 60 + i).to(gpu) for i in range(2)]
+    ws = [quantize_to_fp4((weights((N, C), 26 + i) * (1 + i)).to(gpu), QuantizationConfig(scale_rule="mse")) for i in range(groups)]
+    bias = (torch.randn(N, generator=torch.Generator().manual_seed(27)) * 0.1).to(gpu).bfloat16()
+    denom_a = _native.DENOMINATORS[rule]
+    spin = _native.NORM_QUANTIZE_SPIN_LIMIT if spin_limit is None else spin_limit
+    slots = torch.zeros(_native.AMAX_PARTS, dtype=torch.int64, device=gpu)
+    epoch = 0
+    while M % frames:
+        frames -= 1
+        modulation = [m[:, :frames].contiguous() for m in modulation]
+    for kind in ("adaln", "affine", "plain"):
+        if kind == "adaln":
+            values, scales, amax = _native.adaln_quantize(x[None], *modulation, M // frames, rule)
+            pointers = (modulation[0].data_ptr(), modulation[1].data_ptr(), C, C, M // frames, 1, None, None)
+        else:
+            w, b = affine if kind == "affine" else (None, None)
+            values, scales, amax = _native.layer_norm_quantize(x[None], w, b, rule)
+            pointers = (None, None, 0, 0, 1, 0, *(None if t is None else t.data_ptr() for t in (w, b)))
+        want = [_native.gemm(values, scales, w.values, w.scale_factors, M, N, amax_a=amax, amax_b=w.amax, denom_a=denom_a, denom_b=1536.0,
+                             bias=None if i == 1 else bias, activation="gelu_tanh" if act else None) for i, w in enumerate(ws)]
+        got = [torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=gpu) for _ in ws]
+        products = (_native.GemmProduct * groups)(*[
+            _native.GemmProduct(w.values.data_ptr(), w.scale_factors.data_ptr(), None, w.amax.data_ptr(), 1536.0, y.data_ptr(), N,
+                                None if i == 1 else bias.data_ptr(), _native.AmaxSinkStruct(slots.data_ptr(), epoch + 2 + i, None))
+            for i, (w, y) in enumerate(zip(ws, got))])
+        exchange = _native.AmaxSinkStruct(slots.data_ptr(), epoch + 1, None)
+        code = _native.load().ll_nvfp4_norm_gemm(
+            x.data_ptr(), M, C, *pointers, 1e-6, _native.RULE_IDS[rule], ctypes.byref(exchange), spin, denom_a, N, ws[0].values.shape[0], groups,
+            products, act, torch.cuda.current_stream().cuda_stream)
+        assert code == 0
+        epoch += 1 + groups
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
+        last = slots[(slots >> 32) == epoch] & 0xFFFFFFFF
+        assert last.max().to(torch.int32).view(torch.float32) == want[-1].abs().max().float()
+
+
 @pytest.mark.parametrize("M,N,K,groups", [
     (1, 8, 64, 1),            # one row, a K step that is three quarters zeros
     (63, 65, 192, 1),         # ragged both ways, one partial K step

@@ -1154,10 +1154,12 @@ __global__ __launch_bounds__(kAttnThreads) void kv_attention_kernel(AttnParams p
 // scale bytes of the lane's own, without LDS.  Rows of the chunk (bf16) are loaded four whole rows per instruction
 // and pass through LDS, as V always does (its operand needs the transposing read).
 //
-// Bound by the issue of vector instructions (per tile 16 MFMAs beside about 480 others where the keys are cached, 150 where
-// not; counters of the first shape below: a wave issues 36 % of its cycles and waits 26 % for an issue slot, the matrix pipe
-// is busy 15 %) and, for the chunk's rows, by the LDS they pass through (index unit active 32 %, waits for it 12 %).  us, here /
-// in the tile kernels: 368 queries x 16 heads over 1472 bf16 keys 14.8 / 31.5, over 1104 cached + 368 18.0 / 32.1.  Each wave
+// Bound by the issue of instructions (per tile 16 MFMAs beside about 640 others where the keys are cached, 250 where not, of
+// which a row's address is two: with a clamp, a product and a 64-bit sum for each of a tile's sixteen loads, and a division per
+// cached key, 368 queries x 16 heads over 1472 bf16 keys took 15.6 us, so 14.3, 736 x 12 over 512 12.35 / 11.4, over 736 cached +
+// 736 30.2 / 28.8, 368 x 16 over 1104 + 368 19.3 / 18.8; counters of the first shape before that: a wave issues 36 % of its
+// cycles and waits 26 % for an issue slot, the matrix pipe is busy 15 %) and, for the chunk's rows, by the LDS they pass
+// through (index unit active 32 %, waits for it 12 %).  The tile kernels take 31.5 and 32.1 us for the first and the last.  Each wave
 // loading Q for itself, 16 bytes of each of 32 rows at a time, and a merge in 4-byte accesses cost 1.2 and 1.4 more there, 5.5
 // instead of 4.9 for 192 x 2 over 16 keys.
 constexpr int kShortKeys = 32;                                                // keys per wave tile
@@ -1196,21 +1198,30 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) 
   uint8_t* const vrows = krows + kShortKeys * kKPitch;
   int t = wave;
 
-  // The chunk's own keys: piece j of a tile is rows 4 j + lane / 16, 16 bytes per lane.
+  // The chunk's own keys: piece j of a tile is rows 4 j + lane / 16, 16 bytes per lane.  Offsets of 32 bits for K and V alike: the
+  // chunk has a few thousand keys (short_kernel_waves), and there are no more heads than twice the compute units.
   uint4 kb[8], vb[8];
-  const int64_t row_step = (int64_t)p.H * kHeadDim;
-  auto fetch_new = [&](int tile, const uint16_t* src, uint4 (&dst)[8]) __attribute__((always_inline)) {
-    const int key0 = (tile - cached_tiles) * kShortKeys + (lane >> 4);
+  const uint32_t row_bytes = (uint32_t)p.H * kHeadDim * 2, column = (uint32_t)head * kHeadDim * 2 + (lane & 15) * 16;
+  const uint32_t last_row = (uint32_t)(n_new - 1) * row_bytes + column;
+  auto fetch_new = [&](int tile) __attribute__((always_inline)) {
+    uint32_t first_row = (uint32_t)((tile - cached_tiles) * kShortKeys + (lane >> 4)) * row_bytes + column;
+    asm volatile("" : "+v"(first_row));  // one running offset and not eight
+    uint32_t at[8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j)  // behind the last key: the last again, zeros when it is written to LDS
-      dst[j] = load_global_b128(src + min(key0 + 4 * j, n_new - 1) * row_step + head * kHeadDim + (lane & 15) * 8);
+    for (int j = 0; j < 8; ++j) at[j] = min(first_row + 4 * j * row_bytes, last_row);  // behind the last key: the last again, zeros when it is written to LDS
+#pragma unroll
+    for (int j = 0; j < 8; ++j) kb[j] = load_global_b128(reinterpret_cast<const uint8_t*>(p.k_new) + at[j]);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) vb[j] = load_global_b128(reinterpret_cast<const uint8_t*>(p.v_new) + at[j]);
   };
   // Cached keys: lane = (key l32, half lh of the head dimension) for K and V alike.
   struct { uint4 v[2]; uint32_t scales; } kf, vf;
   uint32_t slot = 0;
+  // key / bts by a product: exact while key * bts < 2^31, and here both are a few thousand (short_kernel_waves)
+  const uint32_t per_slot = CACHED ? (0x80000000u + (uint32_t)p.bts - 1u) / (uint32_t)p.bts : 0u;
   auto fetch_cached = [&](int tile) __attribute__((always_inline)) {
     const uint32_t key = (uint32_t)min(tile * kShortKeys + l32, n_cached - 1);
-    slot = key / (uint32_t)p.bts;
+    slot = __umulhi(2u * key, per_slot);
     const int64_t row = (int64_t)(key - slot * (uint32_t)p.bts) * p.H + head;
     const uint32_t vo = (uint32_t)row * 64u + lh * 32u, so = (uint32_t)blocked_scale_offset(row, lh * 4, 8);
     kf.v[0] = load_global_b128(tab.kv[slot] + vo);
@@ -1233,8 +1244,7 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) 
       q[it] = load_global_b128(p.q + (at * p.H + head) * kHeadDim + (lane & 15) * 8);
     }
     if (!CACHED) {  // a wave without a tile loads the last: under a condition these loads would be waited for with the queries
-      fetch_new(min(t, n_tiles - 1), p.k_new, kb);
-      fetch_new(min(t, n_tiles - 1), p.v_new, vb);
+      fetch_new(min(t, n_tiles - 1));
     }
 #pragma unroll
     for (int it = 0; it < 8 / W; ++it)
@@ -1369,10 +1379,7 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) 
   }
   // ---- the chunk's own keys
   if (t < n_tiles) {
-    if (CACHED) {
-      fetch_new(t, p.k_new, kb);
-      fetch_new(t, p.v_new, vb);
-    }
+    if (CACHED) fetch_new(t);
     for (; t < n_tiles; t += W) {
       const int valid = n_new - (t - cached_tiles) * kShortKeys;
       if (valid < kShortKeys) {
@@ -1386,10 +1393,7 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) 
         *reinterpret_cast<uint4*>(vrows + (4 * j + (lane >> 4)) * kVPitch + (lane & 15) * 16) = vb[j];
       }
       rows_written();
-      if (t + W < n_tiles) {
-        fetch_new(t + W, p.k_new, kb);
-        fetch_new(t + W, p.v_new, vb);
-      }
+      if (t + W < n_tiles) fetch_new(t + W);
       float16v sc;
 #pragma unroll
       for (int i = 0; i < 16; ++i) sc[i] = 0.0f;

@@ -6,7 +6,7 @@
 //                        and V, [cached slots | chunk], K rotated by the window's own positions, and the rotated queries
 //
 // Both are bound by the latency of memory and, for large windows, by its bandwidth: 368 queries x 16 heads over 1104 cached + 368
-// keys, 21 MB, 5.7 us, 2640 x 24 over 10560 + 2640, 260 MB, 55 us.  (6.3 and 63 with flat loads from the slots, the angles loaded behind
+// keys, 21 MB, 5.4 us, 2640 x 24 over 10560 + 2640, 260 MB, 60 us.  (6.3 and 63 with flat loads from the slots, the angles loaded behind
 // them, and stores split in two.)  As separate operations (pointer tables copied to the device, two dequantizations, mean,
 // difference, two concatenations, two rotations) the window moved every byte four times in 13 launches and synchronised
 // the host for the tables: 368 tokens of 16 heads behind 1104 cached ones took 230 us, 62 us of them on the GPU.  Here each
@@ -60,42 +60,60 @@ struct WindowSide {  // K or V of the window
   const uint16_t* fresh;                   // the chunk's, [n_new, H, 128]
   uint16_t* out;                           // [n_cached + n_new, H, 128]
 };
+// n / d for any 32-bit n in five instructions (Granlund and Montgomery, Division by invariant integers using multiplication).
+struct Divisor {
+  uint32_t d, m, s1, s2;
+};
+static Divisor divisor(uint32_t d) {
+  uint32_t l = 0;
+  while (l < 32 && (1ull << l) < d) ++l;
+  return Divisor{d, (uint32_t)(((1ull << 32) * ((1ull << l) - d)) / d + 1), l < 1 ? l : 1, l > 1 ? l - 1 : 0};
+}
+__device__ __forceinline__ uint32_t operator/(uint32_t n, const Divisor& by) {
+  const uint32_t t = __umulhi(by.m, n);
+  return (t + ((n - t) >> by.s1)) >> by.s2;
+}
 struct WindowParams {
   WindowSide k, v;
   const uint16_t* q;
   uint16_t* q_out;
   const float *cos_k, *sin_k, *cos_q, *sin_q;  // rows of 64: one per key, one per query
-  uint32_t H, Lq, n_cached, n_new, slot_tokens;
+  Divisor H, slot_tokens;
+  uint32_t Lq, n_cached, n_new;
   float inv_denom;
   uint32_t wgs_window, wgs_q;  // workgroups of one side of the window, of the queries
 };
 
-// Workgroups [0, wgs_window): K, then wgs_window for V, then wgs_q for the queries.
+// Workgroups [0, wgs_window): K, then wgs_window for V, then wgs_q for the queries.  Windows of a few thousand tokens are bound by
+// the chain (slot pointers, bytes, store) and by the instructions of a thread, about 200 for its eight values: a division is a
+// product and a scale byte one conversion.  us, with divisions and the scale taken apart / so: 368 queries x 16 heads over 1104 +
+// 368 keys 5.8 / 5.4, 880 x 12 over 3520 + 880 10.9 / 10.4, 2640 x 24 over 10560 + 2640 61.7 / 60.  Two rows a thread, their loads
+// under way together: 6.0, 11.4 and 57.9, but 2.6 instead of 2.15 for 64 x 2 over 128 + 64.
 __global__ __launch_bounds__(256) void kv_window_rope_kernel(WindowParams p) {
   const int c = (threadIdx.x & 15) * 8;  // element of the head
   uint32_t wg = blockIdx.x;
   if (wg >= 2 * p.wgs_window) {
     const uint32_t row = (wg - 2 * p.wgs_window) * kRowsPerWindowWg + (threadIdx.x >> 4);
-    if (row >= p.Lq * p.H) return;
-    const uint32_t t = row / p.H;
+    if (row >= p.Lq * p.H.d) return;
+    const int64_t angles = (int64_t)(row / p.H) * 64 + (c >> 1);
     float v[8];
     unpack8(*reinterpret_cast<const uint4*>(p.q + (int64_t)row * 128 + c), v);
-    rotate8(v, *reinterpret_cast<const float4*>(p.cos_q + (int64_t)t * 64 + (c >> 1)), *reinterpret_cast<const float4*>(p.sin_q + (int64_t)t * 64 + (c >> 1)));
+    rotate8(v, *reinterpret_cast<const float4*>(p.cos_q + angles), *reinterpret_cast<const float4*>(p.sin_q + angles));
     store_b128(p.q_out + (int64_t)row * 128 + c, __builtin_bit_cast(u32x4, pack8(v)));
     return;
   }
   const bool is_v = wg >= p.wgs_window;
   if (is_v) wg -= p.wgs_window;
   const WindowSide side = is_v ? p.v : p.k;
-  const uint32_t row = wg * kRowsPerWindowWg + (threadIdx.x >> 4);
-  if (row >= (p.n_cached + p.n_new) * p.H) return;
+  const uint32_t cached_rows = p.n_cached * p.H.d, row = wg * kRowsPerWindowWg + (threadIdx.x >> 4);
+  if (row >= cached_rows + p.n_new * p.H.d) return;
   const uint32_t t = row / p.H;
-  const bool cached = t < p.n_cached;
+  const bool cached = row < cached_rows;
   const uint8_t *values = nullptr, *scales = nullptr, *amax = nullptr;
   uint32_t r = 0;  // row of the slot
   if (cached) {
     const uint32_t slot = t / p.slot_tokens;
-    r = row - slot * p.slot_tokens * p.H;
+    r = row - slot * p.slot_tokens.d * p.H.d;
     values = reinterpret_cast<const uint8_t*>(side.values[slot]);
     scales = reinterpret_cast<const uint8_t*>(side.scales[slot]);
     amax = reinterpret_cast<const uint8_t*>(side.amax[slot]);
@@ -110,13 +128,15 @@ __global__ __launch_bounds__(256) void kv_window_rope_kernel(WindowParams p) {
     const uint32_t w = load_global<uint32_t>(values + (int64_t)r * 64 + (c >> 1));
     const uint32_t sb = load_global<uint8_t>(scales + blocked_scale_offset(r, c >> 4, 8));
     const float gs = load_global<float>(amax) * p.inv_denom;
-    const float s = e4m3_to_f32(sb);
+    const float s = __builtin_amdgcn_cvt_f32_fp8((int)sb, 0);
     float q[8];
     fp4x8_values(w, q);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] = round_to_bf16((q[i] * s) * gs);  // kv_dequantize_kernel's value
+    for (int j = 0; j < 8; ++j) v[j] = (q[j] * s) * gs;  // kv_dequantize_kernel's value, rounded to bf16
+#pragma unroll
+    for (int j = 0; j < 8; j += 2) round_to_bf16(v[j], v[j + 1]);
   } else {
-    unpack8(*reinterpret_cast<const uint4*>(side.fresh + (int64_t)(row - p.n_cached * p.H) * 128 + c), v);
+    unpack8(*reinterpret_cast<const uint4*>(side.fresh + (int64_t)(row - cached_rows) * 128 + c), v);
     if (!is_v) smooth8(v);
   }
   if (!is_v) rotate8(v, cs, sn);
@@ -164,11 +184,11 @@ extern "C" int ll_kv_window_rope(const void* q, int64_t Lq, int num_heads, const
   p.sin_k = sin_k;
   p.cos_q = cos_q;
   p.sin_q = sin_q;
-  p.H = (uint32_t)num_heads;
+  p.H = divisor((uint32_t)num_heads);
   p.Lq = (uint32_t)Lq;
   p.n_cached = (uint32_t)n_cached;
   p.n_new = (uint32_t)n_new;
-  p.slot_tokens = n_cached ? (uint32_t)block_token_size : 1u;
+  p.slot_tokens = divisor(n_cached ? (uint32_t)block_token_size : 1u);
   p.inv_denom = kv_inverse_denominator(e2m1_max, e4m3_max);
   p.wgs_window = (uint32_t)(((n_cached + n_new) * num_heads + kRowsPerWindowWg - 1) / kRowsPerWindowWg);
   p.wgs_q = (uint32_t)((Lq * num_heads + kRowsPerWindowWg - 1) / kRowsPerWindowWg);

@@ -1152,34 +1152,39 @@ __global__ __launch_bounds__(kAttnThreads) void kv_attention_kernel(AttnParams p
 // The contraction over the head dimension may run in any order as long as Q and K agree: step ks of lane half lh
 // covers elements 64 lh + 8 ks .. + 7, so the K operand of a cached row comes straight out of 32 packed bytes and four
 // scale bytes of the lane's own, without LDS.  Rows of the chunk (bf16) are loaded four whole rows per instruction
-// and pass through LDS, as V always does (its operand needs the transposing read).
+// straight into LDS, as V always passes through it (its operand needs the transposing read).
 //
-// Bound by the issue of instructions (per tile 16 MFMAs beside about 640 others where the keys are cached, 250 where not, of
-// which a row's address is two: with a clamp, a product and a 64-bit sum for each of a tile's sixteen loads, and a division per
-// cached key, 368 queries x 16 heads over 1472 bf16 keys took 15.6 us, so 14.3, 736 x 12 over 512 12.35 / 11.4, over 736 cached +
-// 736 30.2 / 28.8, 368 x 16 over 1104 + 368 19.3 / 18.8; counters of the first shape before that: a wave issues 36 % of its
-// cycles and waits 26 % for an issue slot, the matrix pipe is busy 15 %) and, for the chunk's rows, by the LDS they pass
-// through (index unit active 32 %, waits for it 12 %).  The tile kernels take 31.5 and 32.1 us for the first and the last.  Each wave
-// loading Q for itself, 16 bytes of each of 32 rows at a time, and a merge in 4-byte accesses cost 1.2 and 1.4 more there, 5.5
-// instead of 4.9 for 192 x 2 over 16 keys.
+// Bound by the issue of instructions: per tile 16 MFMAs beside about 600 others where the keys are cached and 230 where not,
+// and by the LDS that the chunk's rows pass through.  us, with a 64-bit product per loaded row and a division per cached key /
+// with 32-bit offsets that K and V share / with loads that need no registers and no stores to LDS: 368 queries x 16 heads over
+// 1472 bf16 keys 15.6 / 14.4 / 12.6, 736 x 12 over 512 12.35 / 11.4 / 9.8, 192 x 2 over 2048 17.4 / 16.3 / 12.9, 736 x 12 over 736
+// cached + 736 30.2 / 29.0 / 28.1, 368 x 16 over 1104 + 368 19.3 / 18.9 / 18.7 (the chunk's first K rows asked for ahead of
+// the cached tiles: 19.1).  The tile kernels take 31.5 and 32.1 us for the first and the last.  Each wave loading Q for
+// itself, 16 bytes of each of 32 rows at a time, and a merge in 4-byte accesses cost 1.2 and 1.4 more there, 5.5 instead of
+// 4.9 for 192 x 2 over 16 keys (now 4.4).
 constexpr int kShortKeys = 32;                                                // keys per wave tile
-constexpr int kShortWaveBytes = kShortKeys * (kKPitch + kVPitch);             // a wave's K and V rows
+// A wave's K rows and V rows lie unpadded, as loads from memory straight into LDS write them: piece c of 16 bytes of row r at
+// position c ^ swizzle(r), which spreads the 16 rows of a K read and the 4 of a transposing V read over all banks.
+constexpr int kShortRow = 256, kShortRows = kShortKeys * kShortRow;
+__device__ __forceinline__ int swizzle(int row) { return (row & 3) << 2 | ((row >> 2) & 3); }
 constexpr int kShortRecord = 66 * 64;                                         // floats of a wave's result in the merge, 16-byte aligned
+constexpr int kShortWaveBytes = kShortRecord * 4;                             // its K and V rows before that
+constexpr int kShortQueries = kWaveQueries * kShortRow;                       // the queries, behind the waves' rows
 template <int W>
-constexpr size_t kShortLds = (size_t)W * kShortWaveBytes + sizeof(SlotTable);
-static_assert(kShortRecord * 4 <= kShortWaveBytes && kShortWaveBytes % 16 == 0, "the merge reuses the waves' rows");
+constexpr size_t kShortLds = (size_t)W * kShortWaveBytes + kShortQueries + sizeof(SlotTable);
+static_assert(2 * kShortRows <= kShortWaveBytes && kShortWaveBytes % 16 == 0, "the merge reuses the waves' rows");
+static_assert(kShortLds<8> <= 160 * 1024 && 2 * kShortLds<4> <= 160 * 1024, "one workgroup of eight waves or two of four fit a unit");
 
 // amdgpu_waves_per_eu: 256 registers per lane, two waves per SIMD (one workgroup of eight or two of four per CU)
 // CACHED: there are cached keys.  The first tile's bytes are asked for with the queries (without cached keys) or as soon as
 // the slot pointers are there (with them, the slots' scales still on their way), and a tile's rows without conditions,
-// which the compiler turns into sixteen branches per tile.  us, before that / now: 368 x 16 over 1472 16.1 / 14.8, over
-// 1104 + 368 18.7 / 18.0, 520 x 24 over 1030 21.6 / 19.9, 736 x 12 over 512 12.9 / 12.0, 192 x 2 over 768 + 192 14.0 /
-// 13.2.
+// which the compiler turns into sixteen branches per tile (368 x 16 over 1472 16.1 instead of 14.8 us when that was found).
 template <int W, bool CACHED>
 __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void kv_attention_short_kernel(AttnParams p) {
   static_assert(W == 4 || W == 8, "the merge gives every wave 64 / W of the 64 output registers");
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  SlotTable& tab = *reinterpret_cast<SlotTable*>(smem + W * kShortWaveBytes);
+  uint8_t* const queries = smem + W * kShortWaveBytes;
+  SlotTable& tab = *reinterpret_cast<SlotTable*>(queries + kShortQueries);
   float ka = 0.0f, va = 0.0f;
   if (const int t = threadIdx.x; CACHED && t < p.n_slots) {
     tab.kv[t] = reinterpret_cast<const uint8_t*>(p.kv_ptrs[t]);
@@ -1195,25 +1200,28 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) 
   const int n_cached = CACHED ? (int)p.n_cached : 0, n_new = (int)p.n_new;
   const int cached_tiles = (n_cached + kShortKeys - 1) / kShortKeys, n_tiles = cached_tiles + (n_new + kShortKeys - 1) / kShortKeys;
   uint8_t* const krows = smem + wave * kShortWaveBytes;
-  uint8_t* const vrows = krows + kShortKeys * kKPitch;
+  uint8_t* const vrows = krows + kShortRows;
   int t = wave;
 
   // The chunk's own keys: piece j of a tile is rows 4 j + lane / 16, 16 bytes per lane.  Offsets of 32 bits for K and V alike: the
   // chunk has a few thousand keys (short_kernel_waves), and there are no more heads than twice the compute units.
-  uint4 kb[8], vb[8];
-  const uint32_t row_bytes = (uint32_t)p.H * kHeadDim * 2, column = (uint32_t)head * kHeadDim * 2 + (lane & 15) * 16;
-  const uint32_t last_row = (uint32_t)(n_new - 1) * row_bytes + column;
-  auto fetch_new = [&](int tile) __attribute__((always_inline)) {
-    uint32_t first_row = (uint32_t)((tile - cached_tiles) * kShortKeys + (lane >> 4)) * row_bytes + column;
-    asm volatile("" : "+v"(first_row));  // one running offset and not eight
-    uint32_t at[8];
+  const uint32_t row_bytes = (uint32_t)p.H * kHeadDim * 2, last_row = (uint32_t)(n_new - 1) * row_bytes;
+  const uint32_t krows_lds = lds_address(krows);
+  const uint32_t piece = (uint32_t)((lane & 15) ^ (lane >> 4) << 2), column = (uint32_t)head * kHeadDim * 2;
+  uint32_t at[8];
+  auto fetch = [&](const uint16_t* src, uint32_t lds) __attribute__((always_inline)) {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) at[j] = min(first_row + 4 * j * row_bytes, last_row);  // behind the last key: the last again, zeros when it is written to LDS
-#pragma unroll
-    for (int j = 0; j < 8; ++j) kb[j] = load_global_b128(reinterpret_cast<const uint8_t*>(p.k_new) + at[j]);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) vb[j] = load_global_b128(reinterpret_cast<const uint8_t*>(p.v_new) + at[j]);
+    for (int j = 0; j < 8; ++j) load_to_lds_b128(at[j], src, lds + j * 1024);
   };
+  auto fetch_k = [&](int tile) __attribute__((always_inline)) {
+    uint32_t first_row = (uint32_t)((tile - cached_tiles) * kShortKeys + (lane >> 4)) * row_bytes;
+    asm volatile("" : "+v"(first_row));  // one running offset and not eight
+#pragma unroll
+    for (int j = 0; j < 8; ++j)  // behind the last key: the last again (V: zeros in LDS)
+      at[j] = min(first_row + 4 * j * row_bytes, last_row) + ((piece ^ (j & 3)) * 16 + column);
+    fetch(p.k_new, krows_lds);
+  };
+  auto fetch_v = [&]() __attribute__((always_inline)) { fetch(p.v_new, krows_lds + kShortRows); };  // of the tile of the last fetch_k
   // Cached keys: lane = (key l32, half lh of the head dimension) for K and V alike.
   struct { uint4 v[2]; uint32_t scales; } kf, vf;
   uint32_t slot = 0;
@@ -1232,34 +1240,35 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) 
     vf.scales = load_global<uint32_t>(tab.vs[slot] + so);
   };
 
+  // piece 8 lh + i of row l32
+  const uint32_t own_row0 = (uint32_t)(l32 * kShortRow + ((8 * lh) ^ swizzle(l32)) * 16);
+  auto own_row = [&](int i) { return own_row0 ^ (uint32_t)(16 * i); };
   const int64_t query = (int64_t)qtile * kWaveQueries + l32;
   bf16x8 qf[8];
   {
     // The waves bring the queries into LDS together, 32 / W rows each, four rows per load, and all read the same fragments.
-    uint4 q[8 / W];
 #pragma unroll
     for (int it = 0; it < 8 / W; ++it) {
-      const int row = (wave * (8 / W) + it) * 4 + (lane >> 4);
-      const int64_t at = min((int64_t)qtile * kWaveQueries + row, p.Lq - 1);
-      q[it] = load_global_b128(p.q + (at * p.H + head) * kHeadDim + (lane & 15) * 8);
+      const int group = wave * (8 / W) + it;
+      const uint32_t row = (uint32_t)min((int64_t)qtile * kWaveQueries + group * 4 + (lane >> 4), p.Lq - 1);
+      load_to_lds_b128(row * row_bytes + (piece ^ (uint32_t)(group & 3)) * 16 + column, p.q, lds_address(queries) + group * 1024);
     }
-    if (!CACHED) {  // a wave without a tile loads the last: under a condition these loads would be waited for with the queries
-      fetch_new(min(t, n_tiles - 1));
+    if (!CACHED) {  // a wave without a tile loads the last
+      fetch_k(min(t, n_tiles - 1));
+      fetch_v();
     }
-#pragma unroll
-    for (int it = 0; it < 8 / W; ++it)
-      *reinterpret_cast<uint4*>(smem + ((wave * (8 / W) + it) * 4 + (lane >> 4)) * kKPitch + (lane & 15) * 16) = q[it];
+    if (CACHED) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    else asm volatile("s_waitcnt vmcnt(16)" ::: "memory");  // K and V of the first tile
     __syncthreads();  // and the slot pointers
     if (CACHED && (int)threadIdx.x < p.n_slots) {
       tab.kg[threadIdx.x] = ka * p.inv_denom;
       tab.vg[threadIdx.x] = va * p.inv_denom;
     }
     if (CACHED && t < cached_tiles) fetch_cached(t);
-    const uint8_t* src = smem + l32 * kKPitch + lh * 128;
 #pragma unroll
-    for (int ks = 0; ks < 8; ++ks) qf[ks] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(src + 16 * ks));
+    for (int ks = 0; ks < 8; ++ks) qf[ks] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(queries + own_row(ks)));
   }
-  __syncthreads();  // the first wave writes its rows there; the slots' scales
+  if (CACHED) __syncthreads();  // the slots' scales
 
   float16v o[4];
 #pragma unroll
@@ -1277,19 +1286,22 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) 
 
   // Softmax of the wave's 32 scores per query (register r of sc: key 8 (r / 4) + 4 lh + r % 4 of the tile, `valid` keys
   // exist) and O^T += V^T P^T from the V rows in LDS.
-  auto softmax_pv = [&](float16v& sc, int valid) __attribute__((always_inline)) {
+  // `v_there()`: the V rows are in LDS.
+  // Row 4 lh + (lane / 4) % 4 + 8 j + 16 step of V, elements 32 dt + 16 (lane / 16 % 2) + 4 (lane % 4) .. + 3: with j, 16 step and dt.
+  const uint32_t v_row0 = (uint32_t)((4 * lh + ((lane >> 2) & 3)) * kShortRow + (lane & 1) * 8);
+  const uint32_t v_piece = (uint32_t)(((lane >> 2) & 3) << 2 | ((2 * ((lane >> 4) & 1) + ((lane & 3) >> 1)) ^ lh));
+  auto softmax_pv = [&](float16v& sc, int valid, auto v_there) __attribute__((always_inline)) {
     typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
     typedef __attribute__((address_space(3))) bf16x4* lds_bf16x4_t;
-    const uint8_t* vt_lane = vrows + (4 * lh + ((lane & 15) >> 2)) * kVPitch + (16 * ((lane >> 4) & 1) + 4 * (lane & 3)) * 2;
     bf16x4 vfr[2][4][2];
     auto read_v = [&](int step) __attribute__((always_inline)) {
 #pragma unroll
       for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
         for (int j = 0; j < 2; ++j)
-          vfr[step][dt][j] = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4_t)(vt_lane + (16 * step + 8 * j) * kVPitch + dt * 64));
+          vfr[step][dt][j] = __builtin_amdgcn_ds_read_tr16_b64_v4bf16(
+              (lds_bf16x4_t)(vrows + v_row0 + (16 * step + 8 * j) * kShortRow + (v_piece ^ (uint32_t)(4 * dt + 2 * j)) * 16));
     };
-    read_v(0);
     if (valid < kShortKeys) {
 #pragma unroll
       for (int r = 0; r < 16; ++r)
@@ -1310,6 +1322,8 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) 
 #pragma unroll
         for (int i = 0; i < 16; ++i) o[dt][i] *= alpha;
     }
+    v_there();
+    read_v(0);
     read_v(1);
 #pragma unroll
     for (int step = 0; step < 2; ++step) {
@@ -1362,7 +1376,6 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) 
         kg = tab.kg[slot];
         vg = tab.vg[slot];
       }
-      uint4* vdst = reinterpret_cast<uint4*>(vrows + l32 * kVPitch + lh * 128);
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         float v8[8];
@@ -1371,43 +1384,51 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) 
                                                                 pack_bf16(v8[4], v8[5]), pack_bf16(v8[6], v8[7])));
         sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa, qf[j], sc, 0, 0, 0);
         fp4x8_to_f32(wv[j], vs2[j >> 1], vgt, v8);
-        vdst[j] = make_uint4(pack_bf16(v8[0], v8[1]), pack_bf16(v8[2], v8[3]), pack_bf16(v8[4], v8[5]), pack_bf16(v8[6], v8[7]));
+        *reinterpret_cast<uint4*>(vrows + own_row(j)) =
+            make_uint4(pack_bf16(v8[0], v8[1]), pack_bf16(v8[2], v8[3]), pack_bf16(v8[4], v8[5]), pack_bf16(v8[6], v8[7]));
       }
       rows_written();
-      softmax_pv(sc, valid);
+      softmax_pv(sc, valid, [] {});
     }
   }
-  // ---- the chunk's own keys
+  // ---- the chunk's own keys.  A tile's K rows are replaced by the next one's when they have been read, likewise its V rows, so
+  // that either is under way while the other is worked on.
   if (t < n_tiles) {
-    if (CACHED) fetch_new(t);
+    if (CACHED) {
+      fetch_k(t);
+      fetch_v();
+    }
     for (; t < n_tiles; t += W) {
       const int valid = n_new - (t - cached_tiles) * kShortKeys;
-      if (valid < kShortKeys) {
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-          if (4 * j + (lane >> 4) >= valid) kb[j] = vb[j] = make_uint4(0u, 0u, 0u, 0u);
-      }
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        *reinterpret_cast<uint4*>(krows + (4 * j + (lane >> 4)) * kKPitch + (lane & 15) * 16) = kb[j];
-        *reinterpret_cast<uint4*>(vrows + (4 * j + (lane >> 4)) * kVPitch + (lane & 15) * 16) = vb[j];
-      }
-      rows_written();
-      if (t + W < n_tiles) fetch_new(t + W);
+      const bool more = t + W < n_tiles;
+      asm volatile("s_waitcnt vmcnt(8)" ::: "memory");  // K; V behind it
       float16v sc;
 #pragma unroll
       for (int i = 0; i < 16; ++i) sc[i] = 0.0f;
-      const uint8_t* krow = krows + l32 * kKPitch + lh * 128;
 #pragma unroll
       for (int ks = 0; ks < 8; ++ks)
-        sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(krow + 16 * ks)), qf[ks], sc, 0, 0, 0);
-      softmax_pv(sc, valid);
+        sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(krows + own_row(ks))), qf[ks], sc, 0, 0, 0);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // all read
+      if (more) fetch_k(t + W);
+      softmax_pv(sc, valid, [&] {
+        if (more) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        if (valid < kShortKeys) {  // nothing but zeros weighed with zero
+#pragma unroll
+          for (int j = 0; j < 8; ++j)
+            if (4 * j + (lane >> 4) >= valid) *reinterpret_cast<uint4*>(vrows + j * 1024 + lane * 16) = make_uint4(0u, 0u, 0u, 0u);
+          rows_written();
+        }
+      });
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      if (more) fetch_v();
     }
   }
 
   // ---- merge: every wave leaves (O^T, reference point, row sum) where its rows were, wave w combines registers 64 w / W .. of
   // all.  Four registers per access: register 4 g + i of a lane is element i of its g-th group.
   l_run += __shfl_xor(l_run, 32, 64);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // a wave without a tile has loaded one all the same
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   __builtin_amdgcn_wave_barrier();
   auto record = [&](int w) { return reinterpret_cast<float*>(smem + w * kShortWaveBytes) + lane * 4; };

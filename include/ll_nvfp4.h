@@ -482,18 +482,28 @@ int ll_layer_norm_quantize(const void* x, int64_t rows, int C, const void* weigh
                            int rule, uint8_t* values, uint8_t* scales, float* amax, const ll_amax_sink* amax_sink,
                            int64_t spin_limit, void* stream);
 
+/* What ll_nvfp4_norm_gemm does with whole rows of a product, as ll_rms_norm and ll_qk_norm_rope_pair_amax do with them. */
+typedef struct ll_row_norm {
+  const void* weight; /* bf16 [N] of WanRMSNorm; NULL: the rows stay as they are */
+  void* smooth;       /* bf16 [M, N], rows as D's: the result minus its mean over each head, or NULL */
+  int rope;           /* rotate by cos / sin [seq_len, 64] behind the norm */
+} ll_row_norm;
+
 /*
  * ll_adaln_quantize (scale and shift given: bf16 rows scale_stride and shift_stride elements apart, one per frame_rows rows of x) or
  * ll_layer_norm_quantize (weight and bias, either may be NULL) of x bf16 [M, C], contiguous, and ll_nvfp4_gemm_tnt_grouped of
  * the result with `activation` on every product (alpha NULL), in one launch and with the same bits.  For small activations:
  * LL_ENOSUP, and nothing is launched, unless C is a multiple of 64 up to 256, the products ones that ll_nvfp4_gemm_tnt_grouped
- * computes in plain 64 x 64 tiles, and their tiles of 32 x 128 no more than two per compute unit.  exchange and spin_limit as
+ * computes in plain 64 x 64 tiles, and their tiles of 32 x 256 no more than two per compute unit.  row_norms (NULL or n_products, N <= 256):
+ * D receives the rows after WanRMSNorm with row_eps and, where asked for, RoPE; the product's sink their maximum.  exchange and spin_limit as
  * amax_sink and spin_limit of ll_adaln_quantize; the products' own sinks may be later epochs of the same buffer.
  */
 int ll_nvfp4_norm_gemm(const void* x, int64_t M, int C, const void* scale, const void* shift, int64_t scale_stride,
                        int64_t shift_stride, int64_t frame_rows, int add_one_to_scale, const void* weight, const void* bias,
                        float eps, int rule, const ll_amax_sink* exchange, int64_t spin_limit, float denom_a, int64_t N,
-                       int64_t Np, int n_products, const ll_gemm_product* products, int activation, void* stream);
+                       int64_t Np, int n_products, const ll_gemm_product* products, int activation,
+                       const ll_row_norm* row_norms, float row_eps, const float* cos, const float* sin, int64_t seq_len,
+                       void* stream);
 
 /* WanRMSNorm (wan_5b/modules/model.py:82-98): y = bf16(bf16(x * rsqrt(mean(x^2) + eps)) * w) over the
  * last dim C of x bf16 [rows, C]; w bf16 [C]. */

@@ -52,7 +52,8 @@ _SIGNATURES = {
     "ll_nvfp4_quantize_gemm": (c_int, [c_void_p, c_int64, c_int64, c_int64, c_int, c_void_p, c_float, c_void_p, c_void_p, c_void_p,
                                        c_float, c_int64, c_int64, c_void_p, c_int64, c_void_p, c_void_p]),
     "ll_nvfp4_norm_gemm": (c_int, [c_void_p, c_int64, c_int, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int, c_void_p, c_void_p, c_float,
-                                   c_int, c_void_p, c_int64, c_float, c_int64, c_int64, c_int, c_void_p, c_int, c_void_p]),
+                                   c_int, c_void_p, c_int64, c_float, c_int64, c_int64, c_int, c_void_p, c_int, c_void_p, c_float, c_void_p,
+                                   c_void_p, c_int64, c_void_p]),
     "ll_nvfp4_gemm_tnt_grouped": (c_int, [c_void_p, c_void_p, c_void_p, c_float, c_int64, c_int64, c_int64, c_int64,
                                           c_int64, c_int, c_void_p, c_void_p]),
     "ll_nvfp4_quantize_pair": (c_int, [c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int, c_void_p, c_void_p, c_void_p,
@@ -565,6 +566,11 @@ class GemmProduct(ctypes.Structure):
     _fields_ = [("B_values", c_void_p), ("B_scales", c_void_p), ("alpha", c_void_p), ("amax_b", c_void_p),
                 ("denom_b", ctypes.c_float), ("D", c_void_p), ("ldd", c_int64), ("bias", c_void_p),
                 ("amax_sink", AmaxSinkStruct)]
+
+
+class RowNorm(ctypes.Structure):
+    """struct ll_row_norm of include/ll_nvfp4.h."""
+    _fields_ = [("weight", c_void_p), ("smooth", c_void_p), ("rope", c_int)]
 
 
 def gemm_grouped(a_values, a_scales, amax_a, denom_a: float, M: int, N: int, products) -> list[torch.Tensor]:

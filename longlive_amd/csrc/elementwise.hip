@@ -109,16 +109,7 @@ __global__ __launch_bounds__(kRowThreads) void rmsnorm_kernel(const uint16_t* __
   load_row<NCH>(w, nchunks, lane, wraw);
   __builtin_amdgcn_sched_barrier(0);  // all loads are under way
   unpack_row<NCH>(xraw, nchunks, lane, v);
-  float sq = 0.0f;
-#pragma unroll
-  for (int i = 0; i < NCH; ++i) {
-    if (i * 64 < nchunks) {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) sq += v[i][j] * v[i][j];
-    }
-  }
-  const float ms = wave_sum_dpp(sq) / (float)C;
-  const float r = 1.0f / sqrtf(ms + eps);
+  const float r = rms_scale<NCH>(v, nchunks, C, eps);
   // The row once more from its packed groups: with the floats kept a SIMD holds two waves instead of three (2640 x 7168: 15.8 us, so 14.1).
   if constexpr (NCH > 12) {
 #pragma unroll
@@ -183,64 +174,24 @@ __global__ __launch_bounds__(kRowThreads) void qk_norm_rope_kernel(QkProblems pr
     cs = *reinterpret_cast<const float4*>(cosp + row * 64 + pair0);
     sn = *reinterpret_cast<const float4*>(sinp + row * 64 + pair0);
   }
-  const float cc[4] = {cs.x, cs.y, cs.z, cs.w}, ss[4] = {sn.x, sn.y, sn.z, sn.w};
   float v[NCH][8];
   uint4 xraw[NCH], wraw[NCH];
   load_row<NCH>(xr, nchunks, lane, xraw);
   load_row<NCH>(w, nchunks, lane, wraw);
   __builtin_amdgcn_sched_barrier(0);  // all loads are under way
   unpack_row<NCH>(xraw, nchunks, lane, v);
-  float sq = 0.0f;
-#pragma unroll
-  for (int i = 0; i < NCH; ++i) {
-    if (i * 64 < nchunks) {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) sq += v[i][j] * v[i][j];
-    }
-  }
-  const float ms = wave_sum_dpp(sq) / (float)C;
-  const float r = 1.0f / sqrtf(ms + eps);
+  const float r = rms_scale<NCH>(v, nchunks, C, eps);
   float out_max = 0.0f;
 #pragma unroll
   for (int i = 0; i < NCH; ++i) {
     const int c = lane + i * 64;  // uniform over each group of 16 threads: c < nchunks or not
     if (c < nchunks) {
-      float w8[8], y[8], o8[8];
-      unpack8(wraw[i], w8);
-#pragma unroll
-      for (int j = 0; j < 8; j += 2) {
-        y[j] = v[i][j] * r;
-        y[j + 1] = v[i][j + 1] * r;
-        round_to_bf16(y[j], y[j + 1]);
-        y[j] *= w8[j];
-        y[j + 1] *= w8[j + 1];
-        round_to_bf16(y[j], y[j + 1]);
-      }
-      if (rotate) {
-#pragma unroll
-        for (int p = 0; p < 4; ++p) {
-          const float a = y[2 * p], b = y[2 * p + 1];
-          o8[2 * p] = a * cc[p] - b * ss[p];
-          o8[2 * p + 1] = a * ss[p] + b * cc[p];
-          round_to_bf16(o8[2 * p], o8[2 * p + 1]);
-        }
-      } else {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) o8[j] = y[j];
-      }
+      float o8[8];
+      norm_rope8(v[i], r, wraw[i], rotate, cs, sn, o8);
       const uint4 packed = pack8(o8);
       *reinterpret_cast<uint4*>(out + row * (int64_t)C + c * 8) = packed;
       out_max = abs_max_bf16x8(packed, out_max);
-      if (out_smooth) {
-        float part = 0.0f;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) part += o8[j];
-        const float mean = round_to_bf16(sum_over_16_lanes(part) * (1.0f / 128.0f));
-        float s8[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) s8[j] = o8[j] - mean;
-        *reinterpret_cast<uint4*>(out_smooth + row * (int64_t)C + c * 8) = pack8(s8);
-      }
+      if (out_smooth) *reinterpret_cast<uint4*>(out_smooth + row * (int64_t)C + c * 8) = smooth_head8(o8);
     }
   }
   if (pr.sink.parts) {

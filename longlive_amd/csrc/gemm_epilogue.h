@@ -50,11 +50,32 @@ struct GemmEpilogue {
 // registers and lose 0.5 to 2.5 us (asm8: 2640 x 3072 x 3072 47 / 50).  The persistent kernel, whose 4 x 4 fragments leave none
 // to spare (253 spilled), takes 2: 2640 x 3072 x 3072 89 us, with gate and residual 97.5 (with 4 96 and 110.5; 7040 x 14336 x
 // 3072 568 and 676, with 4 607 and 785).
+//
+// The bias, which epilogue_bias asks for: ahead of the epilogue where the registers are there and something is left to wait for.
+struct EpilogueBias {
+  uint32_t w[4];  // of the lane's eight columns
+};
+template <int FB>
+__device__ __forceinline__ EpilogueBias epilogue_bias(const uint16_t* __restrict__ bias, int lane, int col_base, int N) {
+  const int n_lane = col_base + 8 * (lane % (4 * FB));
+  EpilogueBias b;
+  if (!bias || ((N & 7) == 0 && (reinterpret_cast<uintptr_t>(bias) & 15) == 0)) {
+    const uint4 v = *reinterpret_cast<const uint4*>(bias ? bias + min(n_lane, N - 8) : reinterpret_cast<const uint16_t*>(&g_gemm_zero16));
+    b.w[0] = v.x, b.w[1] = v.y, b.w[2] = v.z, b.w[3] = v.w;
+  } else {
+    uint32_t bits[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) bits[i] = bias[min(n_lane + i, N - 1)];  // behind the last column: not used
+#pragma unroll
+    for (int i = 0; i < 4; ++i) b.w[i] = bits[2 * i] | bits[2 * i + 1] << 16;
+  }
+  return b;
+}
 template <int FA, int FB, int BATCH>
 __device__ __forceinline__ void gemm_epilogue(float16v (&acc)[FB][FA], float alpha, uint8_t* smem, int wave, int lane, int row_base,
                                               int col_base, int M, int N, uint16_t* __restrict__ D, int64_t ldd,
                                               const uint16_t* __restrict__ bias, int act, const GemmEpilogue& epi,
-                                              uint32_t sink_slot) {
+                                              uint32_t sink_slot, const EpilogueBias& bias_bits) {
   const int l32 = lane & 31, lh = lane >> 5;
   constexpr int kEpiPitch = 64 * FB + 16;  // bytes per slab row: 32*FB bf16 + pad
   uint8_t* ebuf = smem + wave * (32 * kEpiPitch);
@@ -67,13 +88,10 @@ __device__ __forceinline__ void gemm_epilogue(float16v (&acc)[FB][FA], float alp
   // for before the next is issued.  us, so / now: 48 x 512 x 256 with bias 4.7 / 4.3, with bias, gate and residual 5.3 / 4.7, 368 x 2048 x
   // 2048 with bias 9.1 / 8.7, 880 x 3072 x 3072 with all 25.1 / 24.1, 7040 x 3072 x 3072 with all 132.5 / 129.5.
   float bias_f[8];
-  {
-    const uint16_t* from = bias ? bias : reinterpret_cast<const uint16_t*>(&g_gemm_zero16);
-    uint32_t bits[8];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) bits[i] = from[bias ? min(n_lane + i, N - 1) : i];  // behind the last column: not used
-#pragma unroll
-    for (int i = 0; i < 8; ++i) bias_f[i] = bf16_bits_to_f32((uint16_t)bits[i]);
+  for (int i = 0; i < 4; ++i) {
+    bias_f[2 * i] = __uint_as_float(bias_bits.w[i] << 16);
+    bias_f[2 * i + 1] = __uint_as_float(bias_bits.w[i] & 0xFFFF0000u);
   }
   constexpr int kPasses = (32 * kChunksPerRow) / 64, kBatch = kPasses < BATCH ? kPasses : BATCH;
   constexpr bool kAhead = FA == 1 || BATCH >= 4;  // the first batch of a slab is asked for before its results go to LDS
@@ -162,6 +180,15 @@ __device__ __forceinline__ void gemm_epilogue(float16v (&acc)[FB][FA], float alp
     }
     if (lane == 0) amax_sink_update(epi.sink, sink_slot, out_max);
   }
+}
+
+template <int FA, int FB, int BATCH>
+__device__ __forceinline__ void gemm_epilogue(float16v (&acc)[FB][FA], float alpha, uint8_t* smem, int wave, int lane, int row_base,
+                                              int col_base, int M, int N, uint16_t* __restrict__ D, int64_t ldd,
+                                              const uint16_t* __restrict__ bias, int act, const GemmEpilogue& epi,
+                                              uint32_t sink_slot) {
+  gemm_epilogue<FA, FB, BATCH>(acc, alpha, smem, wave, lane, row_base, col_base, M, N, D, ldd, bias, act, epi, sink_slot,
+                               epilogue_bias<FB>(bias, lane, col_base, N));
 }
 
 // The kernel-side epilogue of a caller's ll_gemm_epilogue for a product of N columns.

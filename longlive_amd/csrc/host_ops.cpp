@@ -486,16 +486,22 @@ PyObject* py_block_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
   // negative): one launch for small activations, else `operand(exchange)` and `product()`.  result_sink: the sink of the first
   // product where it is to have a fresh epoch, which has to be newer than those of the launches before it.
   TempOperand xq{};  // allocated by the first that needs it
+  const bool whole_rows = C <= 256;  // a workgroup of ll_nvfp4_norm_gemm has them: the norms and RoPE of q and k are part of it
+  auto norm_gemm = [&](const void* h, int scale, int shift, const ll_amax_sink& exchange, const Layer* const* layers, int n, void* const* outs,
+                       const ll_amax_sink* sinks, int activation, const ll_row_norm* row_norms, float row_eps) -> int {
+    ll_gemm_product p[4];
+    BlockCall::products(layers, n, outs, sinks, p);
+    const bool adaln = scale >= 0;
+    return ll_nvfp4_norm_gemm(h, L, (int)C, adaln ? modulation(scale) : nullptr, adaln ? modulation(shift) : nullptr, sf, sf, frame_rows, 1,
+                              adaln ? nullptr : norm[2], adaln ? nullptr : norm[3], adaln ? eps[0] : eps[2], c.rule, &exchange, spin,
+                              c.denom_a, layers[0]->n, layers[0]->np, n, p, activation, row_norms, row_eps, cos->data_ptr<float>(),
+                              sin->data_ptr<float>(), L, c.stream);
+  };
   auto normed_layers = [&](const void* h, int scale, int shift, const Layer* const* layers, int n, void* const* outs, const ll_amax_sink* sinks,
                            ll_amax_sink* result_sink, int activation, auto operand, auto product) -> int {
     const ll_amax_sink exchange = ep.take();
     if (result_sink) *result_sink = ep.take();
-    ll_gemm_product p[4];
-    BlockCall::products(layers, n, outs, sinks ? sinks : result_sink, p);
-    const bool adaln = scale >= 0;
-    int code = ll_nvfp4_norm_gemm(h, L, (int)C, adaln ? modulation(scale) : nullptr, adaln ? modulation(shift) : nullptr, sf, sf, frame_rows, 1,
-                                  adaln ? nullptr : norm[2], adaln ? nullptr : norm[3], adaln ? eps[0] : eps[2], c.rule, &exchange, spin,
-                                  c.denom_a, layers[0]->n, layers[0]->np, n, p, activation, c.stream);
+    int code = norm_gemm(h, scale, shift, exchange, layers, n, outs, sinks ? sinks : result_sink, activation, nullptr, 0.f);
     if (code != LL_ENOSUP) return code;
     if (!xq.values) xq = c.operand(L, C);
     if ((code = operand(exchange))) return code;
@@ -508,19 +514,27 @@ PyObject* py_block_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
   Tensor attended;  // [L, C]
   ll_amax_sink attended_sink;
   {
-    const Tensor q = empty({L, C}, at::kBFloat16, dev), k = empty({L, C}, at::kBFloat16, dev);
-    const Layer* const layers[3] = {&w[Q], &w[K], &w[V]};
-    void* const outs[3] = {q.data_ptr(), k.data_ptr(), value.data_ptr()};
-    const ll_amax_sink sinks[3] = {{nullptr, 0, nullptr}, {nullptr, 0, nullptr}, kv_sink[1]};
-    LL_TRY(normed_layers(x.data_ptr(), 1, 0, layers, 3, outs, sinks, nullptr, LL_ACT_NONE,
-                         [&](const ll_amax_sink& sink) { return adaln_operand(x.data_ptr(), 1, 0, xq, sink); },
-                         [&] { return c.grouped(xq, layers, 3, L, outs, sinks); }),
-           "adaLN and q / k / v projections");
     const Tensor roped_q = empty({L, C}, at::kBFloat16, dev), smooth_k = empty({L, C}, at::kBFloat16, dev);
-    LL_TRY(ll_qk_norm_rope_pair_amax(q.data_ptr(), k.data_ptr(), L, H, norm[0], norm[1], eps[1], cos->data_ptr<float>(),
-                                     sin->data_ptr<float>(), L, roped_q.data_ptr(), key.data_ptr(), smooth_k.data_ptr(), &kv_sink[0],
-                                     c.stream),
-           "norm and RoPE");
+    const Layer* const layers[3] = {&w[Q], &w[K], &w[V]};
+    int code = LL_ENOSUP;
+    if (whole_rows) {
+      void* const outs[3] = {roped_q.data_ptr(), key.data_ptr(), value.data_ptr()};
+      const ll_row_norm row_norms[3] = {{norm[0], nullptr, 1}, {norm[1], smooth_k.data_ptr(), 1}, {nullptr, nullptr, 0}};
+      const ll_amax_sink sinks[3] = {{nullptr, 0, nullptr}, kv_sink[0], kv_sink[1]};
+      code = norm_gemm(x.data_ptr(), 1, 0, ep.take(), layers, 3, outs, sinks, LL_ACT_NONE, row_norms, eps[1]);
+    }
+    if (code == LL_ENOSUP) {
+      const Tensor q = empty({L, C}, at::kBFloat16, dev), k = empty({L, C}, at::kBFloat16, dev);
+      void* const outs[3] = {q.data_ptr(), k.data_ptr(), value.data_ptr()};
+      const ll_amax_sink sinks[3] = {{nullptr, 0, nullptr}, {nullptr, 0, nullptr}, kv_sink[1]};
+      LL_TRY(normed_layers(x.data_ptr(), 1, 0, layers, 3, outs, sinks, nullptr, LL_ACT_NONE,
+                           [&](const ll_amax_sink& sink) { return adaln_operand(x.data_ptr(), 1, 0, xq, sink); },
+                           [&] { return c.grouped(xq, layers, 3, L, outs, sinks); }),
+             "adaLN and q / k / v projections");
+      code = ll_qk_norm_rope_pair_amax(q.data_ptr(), k.data_ptr(), L, H, norm[0], norm[1], eps[1], cos->data_ptr<float>(), sin->data_ptr<float>(),
+                                       L, roped_q.data_ptr(), key.data_ptr(), smooth_k.data_ptr(), &kv_sink[0], c.stream);
+    }
+    LL_TRY(code, "q / k / v projections, norm and RoPE");
     if (keys_only) {
       PyObject* r = PyTuple_New(5);
       if (!r) return nullptr;
@@ -558,16 +572,26 @@ PyObject* py_block_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
     return code ? code : c.quantize_from(y, L, C, xq, again);
   };
   {
-    const Tensor q = empty({L, C}, at::kBFloat16, dev), qn = empty({L, C}, at::kBFloat16, dev);
+    const Tensor qn = empty({L, C}, at::kBFloat16, dev);
     const Layer* const layers[1] = {&w[CQ]};
-    void* const outs[1] = {q.data_ptr()};
-    LL_TRY(normed_layers(x1.data_ptr(), -1, -1, layers, 1, outs, nullptr, nullptr, LL_ACT_NONE, norm3_operand,
-                         [&] { return c.gemm(xq, w[CQ], L, q.data_ptr(), plain_epilogue); }),
-           "norm3 and cross-attention q");
-    LL_TRY(ll_rms_norm(q.data_ptr(), L, (int)C, norm[4], eps[3], qn.data_ptr(), c.stream), "cross-attention norm_q");
+    int code = LL_ENOSUP;
+    if (whole_rows) {
+      void* const outs[1] = {qn.data_ptr()};
+      const ll_row_norm row_norms[1] = {{norm[4], nullptr, 0}};
+      code = norm_gemm(x1.data_ptr(), -1, -1, ep.take(), layers, 1, outs, nullptr, LL_ACT_NONE, row_norms, eps[3]);
+    }
+    if (code == LL_ENOSUP) {
+      const Tensor q = empty({L, C}, at::kBFloat16, dev);
+      void* const outs[1] = {q.data_ptr()};
+      LL_TRY(normed_layers(x1.data_ptr(), -1, -1, layers, 1, outs, nullptr, nullptr, LL_ACT_NONE, norm3_operand,
+                           [&] { return c.gemm(xq, w[CQ], L, q.data_ptr(), plain_epilogue); }),
+             "norm3 and cross-attention q");
+      code = ll_rms_norm(q.data_ptr(), L, (int)C, norm[4], eps[3], qn.data_ptr(), c.stream);
+    }
+    LL_TRY(code, "cross-attention q");
     if (context) {
       const TempOperand tq = c.operand(T, C);
-      int code = LL_ENOSUP;
+      code = LL_ENOSUP;
       if (one_pass_tiles(T, C, 1)) {  // a block of 736 rows, text of 512 x 1536: in two launches 237.2 us, so 234.4
         const ll_amax_sink sink = ep.take();
         code = ll_nvfp4_quantize_one_pass(context->data_ptr(), nullptr, T, C, C, c.rule, tq.values, nullptr, tq.scales, nullptr, tq.amax, nullptr,

@@ -60,19 +60,6 @@ struct WindowSide {  // K or V of the window
   const uint16_t* fresh;                   // the chunk's, [n_new, H, 128]
   uint16_t* out;                           // [n_cached + n_new, H, 128]
 };
-// n / d for any 32-bit n in five instructions (Granlund and Montgomery, Division by invariant integers using multiplication).
-struct Divisor {
-  uint32_t d, m, s1, s2;
-};
-static Divisor divisor(uint32_t d) {
-  uint32_t l = 0;
-  while (l < 32 && (1ull << l) < d) ++l;
-  return Divisor{d, (uint32_t)(((1ull << 32) * ((1ull << l) - d)) / d + 1), l < 1 ? l : 1, l > 1 ? l - 1 : 0};
-}
-__device__ __forceinline__ uint32_t operator/(uint32_t n, const Divisor& by) {
-  const uint32_t t = __umulhi(by.m, n);
-  return (t + ((n - t) >> by.s1)) >> by.s2;
-}
 struct WindowParams {
   WindowSide k, v;
   const uint16_t* q;

@@ -204,6 +204,20 @@ __device__ __forceinline__ float sum_over_16_lanes(float v) {
 }
 #undef LL_DPP_ADD
 
+// n / d for any 32-bit n in five instructions (Granlund and Montgomery, Division by invariant integers using multiplication).
+struct Divisor {
+  uint32_t d, m, s1, s2;
+};
+inline Divisor divisor(uint32_t d) {
+  uint32_t l = 0;
+  while (l < 32 && (1ull << l) < d) ++l;
+  return Divisor{d, (uint32_t)(((1ull << 32) * ((1ull << l) - d)) / d + 1), l < 1 ? l : 1, l > 1 ? l - 1 : 0};
+}
+__device__ __forceinline__ uint32_t operator/(uint32_t n, const Divisor& by) {
+  const uint32_t t = __umulhi(by.m, n);
+  return (t + ((n - t) >> by.s1)) >> by.s2;
+}
+
 // Load through a pointer that is known to address global memory.  Slot pointers come out of a table, so
 // the compiler would otherwise emit flat loads, whose completion also counts as an LDS event and stalls
 // the first LDS wait that follows.

@@ -242,4 +242,58 @@ __device__ __forceinline__ float layernorm_row(const uint16_t* __restrict__ xr, 
   return layernorm_loaded_row<NCH>(xraw, wraw, braw, w, b, C, eps, lane, packed);
 }
 
+// 1 / sqrt(mean of squares + eps) of a row (WanRMSNorm, wan_5b/modules/model.py:82-98).
+template <int NCH, bool HALF = false>
+__device__ __forceinline__ float rms_scale(const float (&v)[NCH][8], int nchunks, int C, float eps) {
+  float sq = 0.0f;
+#pragma unroll
+  for (int i = 0; i < NCH; ++i) {
+    if (i * 64 < nchunks) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) sq += v[i][j] * v[i][j];
+    }
+  }
+  const float ms = row_sum<HALF>(sq) / (float)C;
+  return 1.0f / sqrtf(ms + eps);
+}
+// A group of a row normalized with scale r and weights w, then rotated by the group's four angles, each step rounded to bf16.
+__device__ __forceinline__ void norm_rope8(const float (&v)[8], float r, const uint4& w, bool rotate, const float4& cs, const float4& sn,
+                                           float (&o8)[8]) {
+  const float cc[4] = {cs.x, cs.y, cs.z, cs.w}, ss[4] = {sn.x, sn.y, sn.z, sn.w};
+  float w8[8], y[8];
+  unpack8(w, w8);
+#pragma unroll
+  for (int j = 0; j < 8; j += 2) {
+    y[j] = v[j] * r;
+    y[j + 1] = v[j + 1] * r;
+    round_to_bf16(y[j], y[j + 1]);
+    y[j] *= w8[j];
+    y[j + 1] *= w8[j + 1];
+    round_to_bf16(y[j], y[j + 1]);
+  }
+  if (rotate) {
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      const float a = y[2 * p], b = y[2 * p + 1];
+      o8[2 * p] = a * cc[p] - b * ss[p];
+      o8[2 * p + 1] = a * ss[p] + b * cc[p];
+      round_to_bf16(o8[2 * p], o8[2 * p + 1]);
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) o8[j] = y[j];
+  }
+}
+// o8 - its mean over the head, which lies in sixteen neighbouring lanes (utils/quant.py:797-798): mean and difference rounded to bf16.
+__device__ __forceinline__ uint4 smooth_head8(const float (&o8)[8]) {
+  float part = 0.0f;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) part += o8[j];
+  const float mean = round_to_bf16(sum_over_16_lanes(part) * (1.0f / 128.0f));
+  float s8[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) s8[j] = o8[j] - mean;
+  return pack8(s8);
+}
+
 }  // namespace ll

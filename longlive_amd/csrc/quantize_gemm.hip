@@ -7,7 +7,8 @@
 //
 // Measured, us on the GPU, two launches / one.  Maximum in a sink: 48 x 256 x 512 8.1 / 6.0, 1024 x 256 x 256 8.8 / 6.6, 368 x 384 x 384
 // 9.0 / 7.9, 192 x 512 x 512 9.9 / 9.3.  Maximum of its own: 48 x 256 x 512 8.3 / 6.1, 192 x 256 x 256 8.4 / 7.6; a call with its host time
-// 12.2 / 7.6 and 12.3 / 7.6.
+// 12.2 / 7.6 and 12.3 / 7.6.  (Four waves in all, bias and tensor scale loaded behind the product, divisions in the addresses.  In
+// a block of 192 rows, dim 256, the output projection took 7.5 us so, now 6.1, FFN down with its 512 columns 10.2, now 8.4.)
 #include "ll_common.h"
 #include "gemm_epilogue.h"
 #include "amax_exchange.h"
@@ -16,8 +17,10 @@
 
 namespace ll {
 
-constexpr int kFusedThreads = 256;  // eight waves: 48 x 256 x 512 7.2 instead of 6.1 us, 64 x 512 x 512 11.2 instead of 9.5
-constexpr int kFusedRows = 32, kFusedCols = 32 * (kFusedThreads / 64);  // of a workgroup's tile: a wave multiplies all rows and 32 columns
+// Eight waves normalize and quantize; all of them multiply where rows are normalized, four of them otherwise: with more columns per
+// workgroup fewer compute units are busy (48 x 256 x 512 7.2 instead of 6.1 us).
+constexpr int kFusedThreads = 512;
+constexpr int kFusedRows = 32;  // of a workgroup's tile: a wave multiplies all rows and 32 columns
 constexpr int kFusedMaxK = 512, kNormMaxK = 256;
 constexpr int kFusedPatch = 32 * (64 + 16);       // bytes of a wave's patch in the epilogue
 
@@ -30,7 +33,8 @@ struct FusedParams {
   const uint8_t *Bv, *Bs;
   const float* amax_b;
   float inv_denom_a, inv_denom_b;
-  int M, N, K, Np, tiles_m;
+  int M, N, K, Np;
+  Divisor tiles_m, row_blocks;  // blocks of 16 of a row
   uint16_t* D;
   int64_t ldd;
   GemmEpilogue epi;
@@ -40,13 +44,18 @@ struct FusedParams {
 struct NormFusedParams : FusedParams {
   const uint16_t *a, *b;
   int64_t a_stride, b_stride;
-  int frame_rows, add_one;
+  Divisor frame_rows, tiles_n_each;
+  int add_one;
   float eps;
   AmaxSink exchange;
   uint32_t spin_limit;
   int recompute;
-  int tiles_n_each;
   GemmGroup more[kMaxGemmGroups - 1];
+  // of whole rows of up to kNormMaxK results, see ll_row_norm
+  ll_row_norm row_norm[kMaxGemmGroups];
+  float row_eps;
+  const float *cosp, *sinp;
+  int seq_len;
 };
 enum { kPlainRows, kAdalnRows, kLayerNormRows };
 template <int ROWS>
@@ -57,8 +66,8 @@ template <>
 struct FusedParamsOf<kPlainRows> {
   typedef FusedParams type;
 };
-constexpr int fused_threads(int rows) { return rows == kPlainRows ? kFusedThreads : 2 * kFusedThreads; }
-constexpr int fused_waves(int rows) { return rows == kPlainRows ? 1 : 4; }  // per SIMD: two workgroups with an exchange are resident
+constexpr int fused_cols(int rows) { return rows == kPlainRows ? 128 : 256; }      // of a workgroup: 32 per wave
+constexpr int fused_waves(int rows) { return rows == kPlainRows ? 2 : 4; }  // per SIMD: two workgroups with an exchange are resident
 constexpr int kExchangeSlots = kAmaxParts / 2;  // of a sink: a launch whose workgroups exchange maxima leaves its results' in the others
 
 // T: 64 elements of K at most, a wave's weights in registers.  Quantization is the arithmetic of quantize_kernel, the product
@@ -72,30 +81,36 @@ constexpr int kExchangeSlots = kAmaxParts / 2;  // of a sink: a launch whose wor
 // of up to 256 elements lie two to a wave (norm_rows.h, the same bits), four more waves join in up to the products.  A
 // block of 192 rows, dim 256, in two launches each 90.2 us, with a wave per row and four waves 92, with eight 85, so 80.1; of 768
 // rows 104.3 / 97.2.  Of 192 rows, dim 512 (a wave per row, eight waves): 108 / 115, hence kNormMaxK.
+// Where a workgroup has whole rows of a product, WanRMSNorm and RoPE of q and k follow in the launch (row_norm): that block issues
+// two launches less, 8 us of its host time, and takes 79 instead of 82 us, one of 2688 rows 136 instead of 145.  Its 12 us by
+// phase: arguments and addresses 1.0, loads 0.9, norm 1.1, exchange 2.1, scale table 0.4, quantization 1.1, product 1.2, rows to LDS
+// 1.0, their norm 1.0, and the launch.
 template <int RULE, int T, int ROWS>
-__global__ __launch_bounds__(fused_threads(ROWS), fused_waves(ROWS)) void quantize_gemm_kernel(typename FusedParamsOf<ROWS>::type p) {
+__global__ __launch_bounds__(kFusedThreads, fused_waves(ROWS)) void quantize_gemm_kernel(typename FusedParamsOf<ROWS>::type p) {
   constexpr bool kNorm = ROWS != kPlainRows;
-  constexpr int kThreads = fused_threads(ROWS), kRowPitch = 128 * T + 16, kWaveRows = kFusedRows / (kThreads / 64);
+  constexpr int kRowPitch = 128 * T + 16, kWaveRows = kFusedRows / (kFusedThreads / 64);
   __shared__ __attribute__((aligned(16))) uint8_t s_rows[kNorm ? kFusedRows * kRowPitch : 16];  // normalized, bf16
   __shared__ AmaxExchangeSmem s_exchange;
   constexpr int kPitch = 32 * T + 16, kScalePitch = 4 * T + 2;
-  constexpr int kRowBlocks = 4 * T, kBlocks = kFusedRows * kRowBlocks / kThreads;  // per row; per thread, at most
+  constexpr int kRowBlocks = 4 * T, kBlocks = (kFusedRows * kRowBlocks + kFusedThreads - 1) / kFusedThreads;  // per row; per thread, at most
   __shared__ float s_red[kFusedThreads / 64];
   __shared__ ScaleEntry s_tab[128];
   __shared__ __attribute__((aligned(16))) uint8_t s_values[kFusedRows * kPitch];
   __shared__ __attribute__((aligned(16))) uint8_t s_scales[kFusedRows * kScalePitch];
-  __shared__ __attribute__((aligned(16))) uint8_t s_patch[kFusedThreads / 64 * kFusedPatch];
+  __shared__ __attribute__((aligned(16))) uint8_t s_patch[fused_cols(ROWS) / 32 * kFusedPatch];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l32 = lane & 31, lh = lane >> 5;
   GemmGroup pr{p.Bv, p.Bs, nullptr, p.amax_b, p.inv_denom_b, p.D, p.ldd, p.epi.bias, p.epi.sink};
   int tile_n = blockIdx.x / p.tiles_m;
-  const int tile_m = blockIdx.x - tile_n * p.tiles_m;
+  const int tile_m = blockIdx.x - tile_n * p.tiles_m.d;
+  ll_row_norm row_norm{};
   if constexpr (kNorm) {
-    const int g = tile_n / p.tiles_n_each;
-    tile_n -= g * p.tiles_n_each;
+    const int g = (uint32_t)tile_n / p.tiles_n_each;
+    tile_n -= g * p.tiles_n_each.d;
     if (g > 0) pr = p.more[g - 1];
+    row_norm = p.row_norm[g];
   }
-  const int row0 = tile_m * kFusedRows, col0 = tile_n * kFusedCols + 32 * wave;
-  const int steps = p.K >> 6, row_blocks = p.K >> 4;
+  const int row0 = tile_m * kFusedRows, col0 = tile_n * fused_cols(ROWS) + 32 * wave;
+  const int steps = p.K >> 6;
 
   // ---- everything the workgroup reads, asked for at once and without branches
   // the thread's blocks of x: block tid + 256 i of the tile's 32 rows
@@ -103,9 +118,9 @@ __global__ __launch_bounds__(fused_threads(ROWS), fused_waves(ROWS)) void quanti
   int block_row[kBlocks], block_col[kBlocks];
 #pragma unroll
   for (int i = 0; i < kBlocks; ++i) {
-    const int b = tid + i * kThreads;
-    block_row[i] = b / row_blocks;
-    block_col[i] = b - block_row[i] * row_blocks;
+    const int b = tid + i * kFusedThreads;
+    block_row[i] = (uint32_t)b / p.row_blocks;
+    block_col[i] = b - block_row[i] * p.row_blocks.d;
     if constexpr (kNorm) continue;
     const int row = min(row0 + block_row[i], p.M - 1);
     const u32x4* src = reinterpret_cast<const u32x4*>(p.x + (int64_t)row * p.ldx + block_col[i] * 16);
@@ -122,7 +137,7 @@ __global__ __launch_bounds__(fused_threads(ROWS), fused_waves(ROWS)) void quanti
       const int row = min(row0 + wave * kWaveRows + 2 * i + lh, p.M - 1);
       load_row<1>(p.x + (int64_t)row * p.ldx, nchunks, l32, xraw[i]);
       if constexpr (ROWS == kAdalnRows) {
-        const int f = row / p.frame_rows;
+        const int f = (uint32_t)row / p.frame_rows;
         load_row<1>(p.a + f * p.a_stride, nchunks, l32, araw[i]);
         load_row<1>(p.b + f * p.b_stride, nchunks, l32, braw[i]);
       }
@@ -132,7 +147,7 @@ __global__ __launch_bounds__(fused_threads(ROWS), fused_waves(ROWS)) void quanti
   // the wave's weights: row l32 of its 32, pieces 2 t + lh of 16 bytes and the scales of their two blocks
   uint4 bv[T];
   uint32_t bs[T];
-  if (!kNorm || wave < kFusedThreads / 64) {
+  if (wave < fused_cols(ROWS) / 32) {
     const int n = min(col0 + l32, p.Np - 1);
     const uint8_t* values = pr.Bv + (int64_t)n * (p.K >> 1) + 16 * lh;
     const uint8_t* scales = pr.Bs + (int64_t)(n >> 7) * (p.K >> 6) * 512 + (n & 31) * 16 + ((n & 127) >> 5) * 4 + 2 * lh;
@@ -143,6 +158,10 @@ __global__ __launch_bounds__(fused_threads(ROWS), fused_waves(ROWS)) void quanti
       bs[t] = *reinterpret_cast<const uint16_t*>(scales + 512 * at);
     }
   }
+  // and what the epilogue needs
+  const float amax_b = pr.amax_b[0];
+  EpilogueBias bias_bits;
+  if (ROWS == kPlainRows) bias_bits = epilogue_bias<1>(pr.bias, lane, col0, p.N);
   float part = 0.0f, amax;
   if constexpr (kNorm) {
     __builtin_amdgcn_sched_barrier(0);  // all loads are under way
@@ -156,14 +175,14 @@ __global__ __launch_bounds__(fused_threads(ROWS), fused_waves(ROWS)) void quanti
       if (l32 < p.K >> 3) *reinterpret_cast<uint4*>(s_rows + (wave * kWaveRows + 2 * i + lh) * kRowPitch + 16 * l32) = packed[0];
     }
     // The column tiles of a row have the same maximum and share its slot.
-    amax = exchange_amax(p.exchange, (uint32_t)p.tiles_m, (uint32_t)tile_m, part, p.spin_limit, p.recompute != 0, s_exchange, [&](uint32_t s) {
+    amax = exchange_amax(p.exchange, p.tiles_m.d, (uint32_t)tile_m, part, p.spin_limit, p.recompute != 0, s_exchange, [&](uint32_t s) {
       float m = 0.0f;
 #pragma unroll 1
       for (int i = 0; i < kWaveRows; ++i) {
         const int row = min((int)s * kFusedRows + wave * kWaveRows + i, p.M - 1);
         uint4 packed[1];
         if constexpr (ROWS == kAdalnRows) {
-          const int f = row / p.frame_rows;
+          const int f = (uint32_t)row / p.frame_rows;
           m = fmaxf(m, adaln_row<1>(p.x + (int64_t)row * p.ldx, p.a + f * p.a_stride, p.b + f * p.b_stride, p.K, p.eps, p.add_one, lane, packed));
         } else {
           m = fmaxf(m, layernorm_row<1>(p.x + (int64_t)row * p.ldx, p.a, p.b, p.K, p.eps, lane, packed));
@@ -235,8 +254,33 @@ __global__ __launch_bounds__(fused_threads(ROWS), fused_waves(ROWS)) void quanti
     s_scales[row * kScalePitch + col] = (uint8_t)sb;
   }
   __syncthreads();
-  if ((kNorm && wave >= kFusedThreads / 64) || col0 >= p.N) return;
+  if ((wave >= fused_cols(ROWS) / 32 || col0 >= p.N) && !row_norm.weight) return;
 
+  // what the rows need behind the product, on its way under it
+  uint4 row_weight[1];
+  uint2 row_bias[4];
+  if constexpr (kNorm) {
+    if (!row_norm.weight) bias_bits = epilogue_bias<1>(pr.bias, lane, col0, p.N);
+  }
+  float4 row_cos[kPairs], row_sin[kPairs];
+  if constexpr (kNorm) {
+    if (row_norm.weight) {
+      load_row<1>(static_cast<const uint16_t*>(row_norm.weight), p.N >> 3, l32, row_weight);
+#pragma unroll
+      for (int rg = 0; rg < 4; ++rg)  // N is a multiple of 8
+        row_bias[rg] = *reinterpret_cast<const uint2*>(pr.bias ? pr.bias + min(col0 + 8 * rg + 4 * lh, p.N - 4) : reinterpret_cast<const uint16_t*>(&g_gemm_zero16));
+#pragma unroll
+      for (int i = 0; i < kPairs; ++i) {
+        const int row = row0 + wave * kWaveRows + 2 * i + lh;
+        row_cos[i] = make_float4(1.0f, 1.0f, 1.0f, 1.0f);
+        row_sin[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (row_norm.rope && row < p.seq_len) {
+          row_cos[i] = *reinterpret_cast<const float4*>(p.cosp + (int64_t)row * 64 + (l32 & 15) * 4);
+          row_sin[i] = *reinterpret_cast<const float4*>(p.sinp + (int64_t)row * 64 + (l32 & 15) * 4);
+        }
+      }
+    }
+  }
   // ---- product: 32 x 32 per wave
   float16v acc[1][1];
 #pragma unroll
@@ -255,20 +299,63 @@ __global__ __launch_bounds__(fused_threads(ROWS), fused_waves(ROWS)) void quanti
       acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(decode8(b[j], half2v{ws[j >> 1], ws[j >> 1]}),
                                                          decode8(a[j], half2v{as[j >> 1], as[j >> 1]}), acc[0][0], 0, 0, 0);
   }
-  const float alpha = (amax * pr.amax_b[0]) * (p.inv_denom_a * pr.inv_denom_b);
+  const float alpha = (amax * amax_b) * (p.inv_denom_a * pr.inv_denom_b);
   GemmEpilogue epi = p.epi;
   epi.sink = pr.sink;
-  const uint32_t slot = (uint32_t)blockIdx.x * (kFusedThreads / 64) + wave;
-  gemm_epilogue<1, 1, 4>(acc, alpha, s_patch, wave, lane, row0, col0, p.M, p.N, pr.D, pr.ldd, pr.bias, p.epi.act, epi,
-                         kNorm ? kExchangeSlots + slot % (kAmaxParts - kExchangeSlots) : slot);
+  uint32_t slot = (uint32_t)blockIdx.x * (kFusedThreads / 64) + wave;
+  if (kNorm) slot = kExchangeSlots + slot % (kAmaxParts - kExchangeSlots);
+  if constexpr (kNorm) {
+    if (row_norm.weight) {
+      // The workgroup has whole rows of results: they meet in LDS where the normalized rows were, and every wave takes the rows that
+      // it normalized.
+      if (col0 < p.N) {
+#pragma unroll
+        for (int rg = 0; rg < 4; ++rg) {
+          const int col = col0 + 8 * rg + 4 * lh;
+          uint32_t w[2] = {pack_bf16x2(acc[0][0][4 * rg] * alpha, acc[0][0][4 * rg + 1] * alpha),
+                           pack_bf16x2(acc[0][0][4 * rg + 2] * alpha, acc[0][0][4 * rg + 3] * alpha)};
+          if (pr.bias) {
+            const uint2 b = row_bias[rg];
+            w[0] = pack_bf16x2(__uint_as_float(w[0] << 16) + __uint_as_float(b.x << 16), __uint_as_float(w[0] & 0xFFFF0000u) + __uint_as_float(b.x & 0xFFFF0000u));
+            w[1] = pack_bf16x2(__uint_as_float(w[1] << 16) + __uint_as_float(b.y << 16), __uint_as_float(w[1] & 0xFFFF0000u) + __uint_as_float(b.y & 0xFFFF0000u));
+          }
+          *reinterpret_cast<uint2*>(s_rows + l32 * kRowPitch + col * 2) = make_uint2(w[0], w[1]);
+        }
+      }
+      __syncthreads();
+      const int nchunks = p.N >> 3;
+      float out_max = 0.0f;
+#pragma unroll
+      for (int i = 0; i < kPairs; ++i) {
+        const int r = wave * kWaveRows + 2 * i + lh, row = row0 + r;
+        const uint4 x[1] = {*reinterpret_cast<const uint4*>(s_rows + r * kRowPitch + min(l32, nchunks - 1) * 16)};
+        float v[1][8], o8[8];
+        unpack_row<1>(x, nchunks, l32, v);
+        const float scale = rms_scale<1, true>(v, nchunks, p.N, p.row_eps);
+        norm_rope8(v[0], scale, row_weight[0], row_norm.rope && row < p.seq_len, row_cos[i], row_sin[i], o8);
+        const uint4 packed = pack8(o8), smooth = smooth_head8(o8);
+        if (row < p.M && l32 < nchunks) {
+          *reinterpret_cast<uint4*>(pr.D + (int64_t)row * pr.ldd + 8 * l32) = packed;
+          out_max = abs_max_bf16x8(packed, out_max);
+          if (row_norm.smooth) *reinterpret_cast<uint4*>(static_cast<uint16_t*>(row_norm.smooth) + (int64_t)row * pr.ldd + 8 * l32) = smooth;
+        }
+      }
+      if (pr.sink.parts) {
+        out_max = wave_max(out_max);
+        if (lane == 0) amax_sink_update(pr.sink, slot, out_max);
+      }
+      return;
+    }
+  }
+  gemm_epilogue<1, 1, 4>(acc, alpha, s_patch, wave, lane, row0, col0, p.M, p.N, pr.D, pr.ldd, pr.bias, p.epi.act, epi, slot, bias_bits);
 }
 
 template <int RULE, int ROWS>
 void launch_rows(const typename FusedParamsOf<ROWS>::type& p, unsigned grid, hipStream_t s) {
   if (ROWS != kPlainRows || p.K <= kNormMaxK)
-    hipLaunchKernelGGL((quantize_gemm_kernel<RULE, kNormMaxK / 64, ROWS>), dim3(grid), dim3(fused_threads(ROWS)), 0, s, p);
+    hipLaunchKernelGGL((quantize_gemm_kernel<RULE, kNormMaxK / 64, ROWS>), dim3(grid), dim3(kFusedThreads), 0, s, p);
   else if constexpr (ROWS == kPlainRows)
-    hipLaunchKernelGGL((quantize_gemm_kernel<RULE, kFusedMaxK / 64, ROWS>), dim3(grid), dim3(fused_threads(ROWS)), 0, s, p);
+    hipLaunchKernelGGL((quantize_gemm_kernel<RULE, kFusedMaxK / 64, ROWS>), dim3(grid), dim3(kFusedThreads), 0, s, p);
 }
 template <int ROWS>
 void launch_quantize_gemm(const typename FusedParamsOf<ROWS>::type& p, int rule, unsigned grid, hipStream_t s) {
@@ -313,7 +400,8 @@ extern "C" int ll_nvfp4_quantize_gemm(const void* x, int64_t M, int64_t K, int64
   if (!product_takes_plain_64x64_tiles(M, N, K, 1, cus)) return LL_ENOSUP;
   // More than one workgroup per unit of the longer rows, whose quantization is then repeated in turn: 1760 x 512 x 512, 220
   // workgroups, 10.6 / 10.1, 2640 x 512 x 512, 332, 12.0 / 13.1; but 5280 x 256 x 256, 330, 10.3 / 8.7.
-  const int64_t grid = ((M + kFusedRows - 1) / kFusedRows) * ((N + kFusedCols - 1) / kFusedCols);
+  constexpr int cols = fused_cols(kPlainRows);
+  const int64_t grid = ((M + kFusedRows - 1) / kFusedRows) * ((N + cols - 1) / cols);
   if (K > 256 && grid > cus) return LL_ENOSUP;
   p.x = static_cast<const uint16_t*>(x);
   p.ldx = ldx;
@@ -331,7 +419,8 @@ extern "C" int ll_nvfp4_quantize_gemm(const void* x, int64_t M, int64_t K, int64
   p.N = (int)N;
   p.K = (int)K;
   p.Np = (int)Np;
-  p.tiles_m = (int)((M + kFusedRows - 1) / kFusedRows);
+  p.tiles_m = divisor((uint32_t)((M + kFusedRows - 1) / kFusedRows));
+  p.row_blocks = divisor((uint32_t)K >> 4);
   p.D = static_cast<uint16_t*>(D);
   p.ldd = ldd;
   launch_quantize_gemm<kPlainRows>(p, rule, (unsigned)grid, static_cast<hipStream_t>(stream));
@@ -342,7 +431,8 @@ extern "C" int ll_nvfp4_quantize_gemm(const void* x, int64_t M, int64_t K, int64
 extern "C" int ll_nvfp4_norm_gemm(const void* x, int64_t M, int C, const void* scale, const void* shift, int64_t scale_stride,
                                   int64_t shift_stride, int64_t frame_rows, int add_one_to_scale, const void* weight, const void* bias, float eps,
                                   int rule, const ll_amax_sink* exchange, int64_t spin_limit, float denom_a, int64_t N, int64_t Np,
-                                  int n_products, const ll_gemm_product* products, int activation, void* stream) {
+                                  int n_products, const ll_gemm_product* products, int activation, const ll_row_norm* row_norms, float row_eps,
+                                  const float* cos, const float* sin, int64_t seq_len, void* stream) {
   using namespace ll;
   const char* what = "ll_nvfp4_norm_gemm";
   LL_REQUIRE(x && products && (scale != nullptr) == (shift != nullptr) && !(scale && (weight || bias)), "%s: null pointer, or both kinds of normalization", what);
@@ -381,6 +471,24 @@ extern "C" int ll_nvfp4_norm_gemm(const void* x, int64_t M, int C, const void* s
       p.more[i - 1] = GemmGroup{pr.B_values, pr.B_scales, nullptr, pr.amax_b, 1.0f / pr.denom_b, static_cast<uint16_t*>(pr.D), pr.ldd, epi.bias, epi.sink};
     }
   }
+  if (row_norms) {
+    for (int i = 0; i < n_products; ++i) {
+      const ll_row_norm& rn = row_norms[i];
+      if (!rn.weight) continue;
+      LL_REQUIRE(N % 8 == 0 && products[i].ldd % 8 == 0 && activation == LL_ACT_NONE && (!(rn.rope || rn.smooth) || N % 128 == 0) &&
+                     (!rn.rope || (cos && sin && seq_len >= 0)),
+                 "%s: product %d: a row norm needs N and ldd of whole 16-byte pieces, no activation, heads of 128 and angles for RoPE", what, i);
+      LL_REQUIRE(((reinterpret_cast<uintptr_t>(rn.weight) | reinterpret_cast<uintptr_t>(rn.smooth) | reinterpret_cast<uintptr_t>(products[i].D) |
+                   reinterpret_cast<uintptr_t>(cos) | reinterpret_cast<uintptr_t>(sin)) & 15) == 0 && (reinterpret_cast<uintptr_t>(products[i].bias) & 7) == 0,
+                 "%s: product %d: row norm operands must be 16-byte aligned (bias 8-byte)", what, i);
+      if (N > fused_cols(kAdalnRows)) return LL_ENOSUP;
+      p.row_norm[i] = rn;
+    }
+    p.row_eps = row_eps;
+    p.cosp = cos;
+    p.sinp = sin;
+    p.seq_len = (int)(seq_len < M ? seq_len : M);
+  }
   if (C % 64 != 0 || C > kNormMaxK || M > (1 << 20) || N > (1 << 20)) return LL_ENOSUP;
   int dev = 0, cus = 0;
   if (hipGetDevice(&dev) != hipSuccess) {
@@ -389,7 +497,7 @@ extern "C" int ll_nvfp4_norm_gemm(const void* x, int64_t M, int C, const void* s
   }
   if (int rc = compute_units_of(dev, cus, what)) return rc;
   if (!product_takes_plain_64x64_tiles(M, N, C, n_products, cus)) return LL_ENOSUP;
-  const int64_t tiles_m = (M + kFusedRows - 1) / kFusedRows, tiles_n = (N + kFusedCols - 1) / kFusedCols;
+  const int64_t tiles_m = (M + kFusedRows - 1) / kFusedRows, tiles_n = (N + fused_cols(kAdalnRows) - 1) / fused_cols(kAdalnRows);
   const int64_t grid = tiles_m * tiles_n * n_products;
   // Where the launch is ahead of two: while all its workgroups are resident, two per unit (a block of 2688 rows, dim 256, with one per
   // unit 146.6 us, so 142.5, in two launches each 153; of 1536 rows 110.9, 106.3).
@@ -401,13 +509,14 @@ extern "C" int ll_nvfp4_norm_gemm(const void* x, int64_t M, int C, const void* s
   p.N = (int)N;
   p.K = C;
   p.Np = (int)Np;
-  p.tiles_m = (int)tiles_m;
-  p.tiles_n_each = (int)tiles_n;
+  p.tiles_m = divisor((uint32_t)tiles_m);
+  p.tiles_n_each = divisor((uint32_t)tiles_n);
+  p.row_blocks = divisor((uint32_t)C >> 4);
   p.a = static_cast<const uint16_t*>(scale ? scale : weight);
   p.b = static_cast<const uint16_t*>(scale ? shift : bias);
   p.a_stride = scale_stride;
   p.b_stride = shift_stride;
-  p.frame_rows = (int)frame_rows;
+  p.frame_rows = divisor(scale ? (uint32_t)frame_rows : 1u);
   p.add_one = add_one_to_scale;
   p.eps = eps;
   p.exchange = make_sink(exchange);

@@ -773,12 +773,54 @@ def test_normalization_and_small_layers_in_one_launch_equal_the_separate_launche
         exchange = _native.AmaxSinkStruct(slots.data_ptr(), epoch + 1, None)
         code = _native.load().ll_nvfp4_norm_gemm(
             x.data_ptr(), M, C, *pointers, 1e-6, _native.RULE_IDS[rule], ctypes.byref(exchange), spin, denom_a, N, ws[0].values.shape[0], groups,
-            products, act, torch.cuda.current_stream().cuda_stream)
+            products, act, None, 0.0, None, None, 0, torch.cuda.current_stream().cuda_stream)
         assert code == 0
         epoch += 1 + groups
         assert all(torch.equal(a, b) for a, b in zip(got, want))
         last = slots[(slots >> 32) == epoch] & 0xFFFFFFFF
         assert last.max().to(torch.int32).view(torch.float32) == want[-1].abs().max().float()
+
+
+@pytest.mark.parametrize("M,C,H,rotated", [
+    (1, 64, 1, 1),       # one row
+    (33, 128, 2, 20),    # a second row of tiles with one row, rows behind the angles, more results than inputs
+    (192, 256, 2, 192),
+    (2001, 256, 1, 2001),
+])
+def test_row_norms_in_the_launch_of_the_projections_equal_the_separate_kernels(gpu, M, C, H, rotated):
+    """WanRMSNorm, RoPE and the smoothed K of whole rows of the products, bit for bit, next to a product that keeps its rows; the
+    maximum of K."""
+    N = H * 128
+    x = activations((M, C), M + C).to(gpu)
+    ws = [quantize_to_fp4((weights((N, C), 26 + i) * (1 + i)).to(gpu), QuantizationConfig(scale_rule="mse")) for i in range(4)]
+    bias = (torch.randn(N, generator=torch.Generator().manual_seed(27)) * 0.1).to(gpu).bfloat16()
+    norms = [(1 + 0.1 * torch.randn(N, generator=torch.Generator().manual_seed(28 + i))).to(gpu).bfloat16() for i in range(3)]
+    angles = torch.rand(rotated, 64, generator=torch.Generator().manual_seed(31)).to(gpu) * 6
+    cos, sin = angles.cos(), angles.sin()
+    values, scales, amax = _native.layer_norm_quantize(x[None], None, None, "mse")
+    plain = [_native.gemm(values, scales, w.values, w.scale_factors, M, N, amax_a=amax, amax_b=w.amax, bias=None if i == 1 else bias)
+             for i, w in enumerate(ws)]
+    q = _native.qk_norm_rope(plain[0], norms[0], 1e-6, cos, sin, H, seq_len=rotated)
+    k, smooth = _native.qk_norm_rope(plain[1], norms[1], 1e-6, cos, sin, H, seq_len=rotated, smooth=True)
+    lib, stream = _native.load(), torch.cuda.current_stream().cuda_stream
+    want = [q, k, plain[2], _native.rms_norm(plain[3], norms[2], 1e-6)]
+    got = [torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=gpu) for _ in range(5)]
+    slots = torch.zeros(_native.AMAX_PARTS, dtype=torch.int64, device=gpu)
+    products = (_native.GemmProduct * 4)(*[
+        _native.GemmProduct(w.values.data_ptr(), w.scale_factors.data_ptr(), None, w.amax.data_ptr(), 1536.0, y.data_ptr(), N,
+                            None if i == 1 else bias.data_ptr(), _native.AmaxSinkStruct(slots.data_ptr(), 2, None) if i == 1 else _native.AmaxSinkStruct())
+        for i, (w, y) in enumerate(zip(ws, got))])
+    row_norms = (_native.RowNorm * 4)(_native.RowNorm(norms[0].data_ptr(), None, 1), _native.RowNorm(norms[1].data_ptr(), got[4].data_ptr(), 1),
+                                      _native.RowNorm(), _native.RowNorm(norms[2].data_ptr(), None, 0))
+    exchange = _native.AmaxSinkStruct(slots.data_ptr(), 1, None)
+    code = lib.ll_nvfp4_norm_gemm(
+        x.data_ptr(), M, C, None, None, 0, 0, 1, 0, None, None, 1e-6, _native.RULE_IDS["mse"], ctypes.byref(exchange), _native.NORM_QUANTIZE_SPIN_LIMIT,
+        1536.0, N, ws[0].values.shape[0], 4, products, 0, row_norms, 1e-6, cos.data_ptr(), sin.data_ptr(), rotated, stream)
+    assert code == 0
+    for i, (a, b) in enumerate(zip(got, [*want, smooth])):
+        assert torch.equal(a, b.reshape(M, N)), i
+    last = slots[(slots >> 32) == 2] & 0xFFFFFFFF
+    assert last.max().to(torch.int32).view(torch.float32) == k.abs().max().float()
 
 
 @pytest.mark.parametrize("M,N,K,groups", [

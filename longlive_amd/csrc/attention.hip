@@ -95,7 +95,6 @@ __device__ __forceinline__ float max_over_wave_halves(float v) {
 }
 
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
-typedef short short4v __attribute__((ext_vector_type(4)));
 
 // The two e4m3 block scales in the low 16 bits of `word`, as f16 pairs (s, s) ready for a packed multiply.
 __device__ __forceinline__ void block_scales_f16(uint32_t word, half2v (&s2)[2]) {
@@ -553,9 +552,9 @@ __global__ __launch_bounds__(kAttnThreads) void kv_attention_kernel(AttnParams p
   // What bounds the loop is the power limit: the MFMA pipe is busy 55 % of the cycles at 1.93 GHz, and with zeros for operands the same
   // cycles take 15 % less time, so what counts is what is not executed.  160 vector instructions per wave and iteration convert,
   // 160 are the softmax.  The iteration is 64 slots of one MFMA with what is to run beside it, held in place by scheduling barriers,
-  // in which no instruction waits for another.  Row sums are taken of the probabilities as the bf16 that multiply V, four to an
-  // MFMA of 4 x 4 x 4: 1 % faster than additions in fp32 ahead of the rounding (v_dot2c_f32_bf16 keeps the MFMA pipe for 7.5
-  // cycles: 4 % slower), and a probability that outweighs all others leaves no error of its rounding.  Raw bytes are asked for
+  // in which no instruction waits for another.  Row sums are added up in fp32, of the probabilities ahead of their rounding to bf16:
+  // of the rounded ones, four to an MFMA of 4 x 4 x 4, they cost 0.6 % less (a chunk step of 2640 x 24 418.9 us, so 421.9), but where one
+  // probability outweighs the others its rounding would scale what the others add by up to 2^-8.  Raw bytes are asked for
   // without branches, behind which the compiler waits for every load under way (one busy wave per SIMD: 247 us, so 202).
   // With the maximum followed per tile (as softmax_pv does) / so, us: 7040 queries x 24 heads over 21120 cached + 7040 keys 2276 /
   // 2135, 2560 x 24 over 10560 + 2640 452 / 425, one tile of 80 queries per unit over 13200 keys 226 / 202.
@@ -579,7 +578,7 @@ __global__ __launch_bounds__(kAttnThreads) void kv_attention_kernel(AttnParams p
     uint32_t pw[16];
     half2v s2[2], t[4];
     float v8[8], x[2][2], e[2][2];
-    float4v sums = {0.0f, 0.0f, 0.0f, 0.0f};
+    float sums[2] = {0.0f, 0.0f};
     const float gs_k = k_gs, gs_v = v_gs;
     const uint8_t *values, *scales;  // where the raw registers are filled from next
     uint32_t vo, so;
@@ -628,11 +627,8 @@ __global__ __launch_bounds__(kAttnThreads) void kv_attention_kernel(AttnParams p
       if constexpr (i >= 11 && i < 27) {
         constexpr int pair = i - 11;
         pw[pair] = pack_bf16(e[pair & 1][0], e[pair & 1][1]);
-      }
-      if constexpr (i >= 13 && i < 29 && (i & 1) == 1) {  // every row of the product is the lane's own four summed
-        constexpr int pair = i - 13;
-        const bf16x4 ones = {1.0f, 1.0f, 1.0f, 1.0f};
-        sums = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(__builtin_bit_cast(short4v, ones), __builtin_bit_cast(short4v, make_uint2(pw[pair], pw[pair + 1])), sums, 0, 0, 0);
+        sums[0] += e[pair & 1][0];
+        sums[1] += e[pair & 1][1];
       }
       if constexpr (i >= 10 && i < 26) {
         constexpr int pair = i - 10;
@@ -693,7 +689,7 @@ __global__ __launch_bounds__(kAttnThreads) void kv_attention_kernel(AttnParams p
       }
     };
     each_index(one_slot, std::make_integer_sequence<int, 64>{});
-    l_run += sums[0];
+    l_run += sums[0] + sums[1];
   };
 
   // prologue: the segment's first iteration into its stage, raw registers <- the second one

@@ -207,19 +207,26 @@ inline int64_t small_product_units(int cus) { return 2 * (int64_t)cus; }  // mos
 // 0.9 us for two of the smaller ones (us, 64 x 64 / 64 x 96: 512 x 3072 x 3072 15.2 / 13.7, 736 x 1536 x 1536 9.9 / 9.4, x
 // 8960 33.3 / 30.5, 440 x 3072 x 14336 50.4 / 45.2).  Larger ones were measured too: 64 x 128 and 96 x 128 were never ahead
 // of both, 128 x 128 by 6 % on 2048 x 2048 x 3072.
+// Two sets of four waves (one workgroup per unit, so a second wave on every SIMD) from 2048 elements of K on: a step then takes
+// 0.71 us where every unit is busy, with one set 0.83, and the sets' sums meet at the end.  us, one set / two: 736 x 1536 x 8960
+// 33.9 / 30.2, 512 x 3072 x 14336 53.2 / 47.0, x 3072 16.0 / 15.3, 450 x 2816 x 3328 16.65 / 15.9, 736 x 1536 x 2304 12.75 / 12.55, x 2048
+// 11.9 / 11.8, but 512 x 3072 x 1792 11.5 / 11.7, 736 x 1536 x 1536 10.4 / 10.5, 512 x 3072 x 1024 9.0 / 9.3.
+constexpr int64_t kSmallSetsK = 2048;
 struct SmallGemmPlan {
   int fb;  // tiles of 64 rows by 32 fb columns
   int parts;
   int tiles_m, tiles_n_each;
   int64_t tiles;
+  int sets;  // of four waves: K steps are dealt to one or two
 };
 inline SmallGemmPlan plan_small_gemm(int64_t M, int64_t N, int64_t Kp, int n_products, int cus) {
-  SmallGemmPlan p{2, 1, (int)((M + 63) / 64), (int)((N + 63) / 64), 0};
+  SmallGemmPlan p{2, 1, (int)((M + 63) / 64), (int)((N + 63) / 64), 0, 1};
   p.tiles = (int64_t)p.tiles_m * p.tiles_n_each * n_products;
   if (const int64_t each = (N + 95) / 96, wide = p.tiles_m * each * n_products; Kp >= 1024 && p.tiles > cus && wide <= cus) {
     p.fb = 3;
     p.tiles_n_each = (int)each;
     p.tiles = wide;
+    p.sets = Kp >= kSmallSetsK ? 2 : 1;
     return p;
   }
   const int64_t steps = (Kp + 255) / 256;

@@ -594,23 +594,23 @@ __global__ __launch_bounds__(256) void gemm_w4a4_persistent_kernel(PersistentPar
 // x 2048 8.2 / 9.6, 736 x 1536 x 8960 30.5 / 35.5 / 56.2, 40 x 2048 x 2048 8.1 / 9.5.  The kernel above keeps short contractions
 // (small_kernel_takes) and LL_GEMM_TILES_COMPILED (one order of summation for every shape).
 constexpr int kSmallThreads = 256;
-constexpr int kSmallStages = 4;
 constexpr int kSmallK = 256;                                  // K elements per step: 64 per wave
 constexpr int kSmallRow = kSmallK / 2;                        // bytes per row and stage; pieces stored at piece ^ (row % 8)
 constexpr int kSmallFragment = 32 * kSmallRow;                // the values of 32 rows of a stage
 constexpr int kSmallScales = 4 * 512;                         // the scales of 128 rows of a stage: four 128 x 4 tiles
 constexpr int kSmallFA = 2;                                   // fragments of 32 rows of A in a tile
 // A tile of 64 rows of A by 32 FB rows of B.  96 rows may lie in two of the 128-row blocks of the scales.
-template <int FB>
+template <int FB, int SETS = 1>
 struct SmallTile {
   static constexpr int kBlocks = 1 + (FB == 3 ? 2 : 1);       // of scales: A's, B's
   static constexpr int kValues = (kSmallFA + FB) * kSmallFragment;
   static constexpr int kStage = kValues + kBlocks * kSmallScales;
   static constexpr int kScaleLoads = (2 * kBlocks + 3) / 4;   // per wave and step, 1 KB each
   static constexpr int kLoads = kSmallFA + FB + kScaleLoads;
-  static constexpr int kRing = kSmallStages * kStage;
+  static constexpr int kStages = SETS == 2 ? 3 : 4;           // of a set of four waves
+  static constexpr int kRing = SETS * kStages * kStage;
   static constexpr int kExchange = FB * 4 * 4096;             // half of each wave's sums
-  static_assert(kExchange + 16 <= kRing && kRing <= 160 * 1024, "the exchange and a flag fit the ring");
+  static_assert(SETS * kExchange + 16 <= kRing && kRing <= 160 * 1024, "the exchange and a flag fit the ring");
 };
 static_assert(2 * SmallTile<2>::kRing <= 160 * 1024, "two workgroups fit a unit");
 constexpr int kSmallWholeSmem = SmallTile<2>::kRing + SmallTile<2>::kExchange;  // WHOLE: the exchange lies behind the ring, which stays full
@@ -635,8 +635,12 @@ __device__ __forceinline__ void load_fragments_to_lds(const uint8_t* const (&bas
 // parts.  The loads run on across the parts; what a part costs is its exchange through LDS, 2 us.  Four parts (the workgroups
 // that share them / one for all / the 64 x 64 tile kernel above): 64 x 512 x 5888 10.6 / 24.2 / 25.5 us, 112 x 2944 x 8192 15.3 /
 // 28.6 / 34.7, 128 x 3072 x 14336 21.8 / 41.8 / 58.3, 48 x 1024 x 4096 10.2 / 20.1 / 18.7.
-template <bool WHOLE, int FB>
-__global__ __launch_bounds__(kSmallThreads, WHOLE ? 1 : 2) void gemm_w4a4_small_kernel(
+//
+// SETS = 2: eight waves, two sets of four that take every other K step, each with three stages of its own.  A wave alone on its
+// SIMD pays 5 cycles for each of the 8 instructions that go with an MFMA; two share the issue (736 x 1536 x 8960 33.9 us with
+// one set, so 30.2; plan_small_gemm has more).  At the end the sets' sums are added, (set 0) + (set 1).
+template <bool WHOLE, int FB, int SETS = 1>
+__global__ __launch_bounds__(SETS * kSmallThreads, WHOLE ? 1 : 2) void gemm_w4a4_small_kernel(
     const uint8_t* __restrict__ Av, const uint8_t* __restrict__ As, const uint8_t* __restrict__ Bv0,
     const uint8_t* __restrict__ Bs0, const float* __restrict__ alpha_ptr0, const float* __restrict__ amax_a,
     const float* __restrict__ amax_b0, float inv_denom_a, float inv_denom_b0, int M, int N, int Mp, int Np, int Kp,
@@ -677,16 +681,18 @@ __global__ __launch_bounds__(kSmallThreads, WHOLE ? 1 : 2) void gemm_w4a4_small_
       epi.sink = gg.sink;
     }
   }
-  using S = SmallTile<FB>;
+  using S = SmallTile<FB, SETS>;
   constexpr int FA = kSmallFA;
   constexpr int kFragments = FA + FB;  // A first
   const int row0 = tile_m * (32 * FA), col0 = tile_n * (32 * FB);
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, lh = lane >> 5;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave = __builtin_amdgcn_readfirstlane((tid >> 6) & 3), set = SETS == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 8);
+  uint8_t* const ring = smem + set * (S::kStages * S::kStage);
   const int all_steps = (Kp + kSmallK - 1) / kSmallK;
   auto first_step = [&](int p) { return (int)((int64_t)p * all_steps / parts); };  // of part p, which has at least one: the host sees to it
-  const int t0 = WHOLE ? 0 : first_step(part);
-  const int nk = WHOLE ? all_steps : first_step(part + 1) - t0;
+  const int t0 = (WHOLE || SETS > 1 ? 0 : first_step(part)) + set;
+  // Both sets ask for as many steps, zeros behind the end of K.
+  const int nk = WHOLE ? all_steps : SETS > 1 ? (all_steps + 1) / 2 : first_step(part + 1) - t0;
 
   // ---- global -> LDS: a load instruction covers 1 KB = 8 rows of 128 bytes.  Wave w brings rows 8 w .. 8 w + 7 of every
   // fragment and one or two KB of scales.  The matrices are padded to 128 rows; a fragment of B behind them is the last one again.
@@ -704,13 +710,13 @@ __global__ __launch_bounds__(kSmallThreads, WHOLE ? 1 : 2) void gemm_w4a4_small_
     const int at = min(wave + 4 * i, 2 * S::kBlocks - 1), block = at >> 1;  // behind the last: the last again
     const int64_t first = block == 0 ? row0 >> 7 : min((col0 >> 7) + block - 1, (Np >> 7) - 1);
     s_src[i] = (block == 0 ? As : Bs) + first * (Kp >> 6) * 512 + (at & 1) * 1024 + (int64_t)t0 * 2048;
-    s_dst[i] = lds_address(smem) + S::kValues + at * 1024;
+    s_dst[i] = lds_address(ring) + S::kValues + at * 1024;
   }
   uint32_t voff = (uint32_t)(lane >> 3) * (uint32_t)row_bytes + (uint32_t)piece * 16u, soff = (uint32_t)lane * 16u;
-  const uint32_t v_dst = lds_address(smem) + wave * 1024;
+  const uint32_t v_dst = lds_address(ring) + wave * 1024;
   auto load_step = [&](int step, auto stage) __attribute__((always_inline)) {  // called for the steps in order
     constexpr int kBase = decltype(stage)::value * S::kStage;
-    const int k0 = (t0 + step) * kSmallK;
+    const int k0 = (t0 + SETS * step) * kSmallK;
     if (k0 + kSmallK <= Kp) {
       load_fragments_to_lds<kBase>(src, voff, v_dst);
 #pragma unroll
@@ -726,8 +732,8 @@ __global__ __launch_bounds__(kSmallThreads, WHOLE ? 1 : 2) void gemm_w4a4_small_
         load_to_lds_b128(k0 + 64 * (2 * half + (lane >> 5)) < Kp ? s_src[i] + soff : zero16, s_dst[i] + kBase);
       }
     }
-    voff += kSmallRow;
-    soff += 2048;
+    voff += SETS * kSmallRow;
+    soff += SETS * 2048;
   };
 
   // ---- the lane's LDS reads: row l32 of a fragment, piece 2 wave + lh; the scale bytes of the piece's two blocks.  A wave
@@ -739,10 +745,10 @@ __global__ __launch_bounds__(kSmallThreads, WHOLE ? 1 : 2) void gemm_w4a4_small_
 #pragma unroll
   for (int f = 0; f < kFragments; ++f) {
     const int own = f < FA ? (odd ? 1 - f : f) : FA + (upper ? (f - FA + kKeepB) % FB : f - FA);
-    v_rd[f] = smem + l32 * kSmallRow + 16 * ((2 * wave + lh) ^ (l32 & 7)) + own * kSmallFragment;
+    v_rd[f] = ring + l32 * kSmallRow + 16 * ((2 * wave + lh) ^ (l32 & 7)) + own * kSmallFragment;
     const int first = f < FA ? row0 : col0, at = first + 32 * (f < FA ? own : own - FA);  // of the operand's rows
     const int block = (at >> 7) - (first >> 7) + (f < FA ? 0 : 1);
-    s_rd[f] = smem + S::kValues + block * kSmallScales + 512 * wave + l32 * 16 + 2 * lh + ((at & 127) >> 5) * 4;
+    s_rd[f] = ring + S::kValues + block * kSmallScales + 512 * wave + l32 * 16 + 2 * lh + ((at & 127) >> 5) * 4;
   }
   struct Raw {
     uint4 v[kFragments];
@@ -867,14 +873,14 @@ __global__ __launch_bounds__(kSmallThreads, WHOLE ? 1 : 2) void gemm_w4a4_small_
     }
     mma_under(o[0], h, s2, 0, o[1]);
     mma_under(o[1], h, s2, 1, o[0]);
-    constexpr std::integral_constant<int, (kStageNo + 1) % kSmallStages> kNext{};
-    if (const int behind = nk - 2 - t; behind >= 3) {
-      wait_loads(kS2);
+    constexpr std::integral_constant<int, (kStageNo + 1) % S::kStages> kNext{};
+    if (const int behind = nk - 2 - t; behind >= S::kStages - 1) {
+      wait_loads(std::integral_constant<int, S::kStages - 2>{});
       __syncthreads();
-      load_step(t + kSmallStages, stage);
+      load_step(t + S::kStages, stage);
       read_raw(next, kNext);
     } else if (behind >= 0) {
-      if (behind == 2) wait_loads(kS2);
+      if (S::kStages > 3 && behind == 2) wait_loads(kS2);
       else if (behind == 1) wait_loads(kS1);
       else wait_loads(kS0);
       __syncthreads();
@@ -886,9 +892,9 @@ __global__ __launch_bounds__(kSmallThreads, WHOLE ? 1 : 2) void gemm_w4a4_small_
   load_step(0, kS0);
   if (1 < nk) load_step(1, kS1);
   if (2 < nk) load_step(2, kS2);
-  if (3 < nk) load_step(3, kS3);
-  if (nk > 3) wait_loads(kS3);
-  else if (nk == 3) wait_loads(kS2);
+  if (S::kStages > 3 && 3 < nk) load_step(3, kS3);
+  if (S::kStages > 3 && nk > 3) wait_loads(kS3);
+  else if (nk >= 3) wait_loads(kS2);
   else if (nk == 2) wait_loads(kS1);
   else wait_loads(kS0);
   __syncthreads();
@@ -917,6 +923,23 @@ __global__ __launch_bounds__(kSmallThreads, WHOLE ? 1 : 2) void gemm_w4a4_small_
       if (++p == parts) break;
       end = first_step(p + 1);
     }
+  } else if constexpr (SETS == 2) {
+    const int end = all_steps > 1 ? (all_steps + 1 - set) / 2 : 1;  // no barrier stands in the last step, which set 1 may have none of
+#pragma unroll 1
+    for (int t = 0;;) {
+      step(t, kS0, h0, h1);
+      if (++t == end) break;
+      step(t, kS1, h1, h0);
+      if (++t == end) break;
+      step(t, kS2, h0, h1);
+      if (++t == end) break;
+      step(t, kS0, h1, h0);
+      if (++t == end) break;
+      step(t, kS1, h0, h1);
+      if (++t == end) break;
+      step(t, kS2, h1, h0);
+      if (++t == end) break;
+    }
   } else {
     int t = 0;
 #pragma unroll 1
@@ -935,7 +958,31 @@ __global__ __launch_bounds__(kSmallThreads, WHOLE ? 1 : 2) void gemm_w4a4_small_
   } else {
     mma_last();
     __syncthreads();  // every wave has left the ring, which the exchange and then the patches of the epilogue take
-    exchange_quarters(reinterpret_cast<float*>(smem));
+    exchange_quarters(reinterpret_cast<float*>(smem + set * S::kExchange));
+  }
+  // Of the two fragments that waves 0 and 1 keep, set 0 finishes the first and set 1 the second; the one of waves 2 and 3 is set 0's.
+  if constexpr (SETS == 2) {
+    static_assert(FB == 3 && kKeepB == 2);
+    float* sums = reinterpret_cast<float*>(smem) + lane * 4;
+    const float16v &give = upper || set == 1 ? acc[0][0] : acc[1][0], &keep = upper || set == 0 ? acc[0][0] : acc[1][0];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      *reinterpret_cast<float4*>(sums + (4 * set + wave) * 1024 + i * 256) = make_float4(give[4 * i], give[4 * i + 1], give[4 * i + 2], give[4 * i + 3]);
+    __syncthreads();
+    if (upper && set == 1) return;
+    float16v kept[1][1];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float4 x = *reinterpret_cast<const float4*>(sums + (4 * (set ^ 1) + wave) * 1024 + i * 256);
+      kept[0][0][4 * i] = keep[4 * i] + x.x;
+      kept[0][0][4 * i + 1] = keep[4 * i + 1] + x.y;
+      kept[0][0][4 * i + 2] = keep[4 * i + 2] + x.z;
+      kept[0][0][4 * i + 3] = keep[4 * i + 3] + x.w;
+    }
+    const float alpha = alpha_ptr ? alpha_ptr[0] : (amax_a[0] * amax_b[0]) * (inv_denom_a * inv_denom_b);
+    gemm_epilogue<1, 1, 4>(kept, alpha, smem + 8 * 4096, 4 * set + wave, lane, row0 + (odd ? 32 : 0), col0 + (upper ? 64 : 32 * set), M, N, D, ldd,
+                           bias, act, epi, (uint32_t)blockIdx.x * 8 + 4 * set + wave);
+    return;
   }
   if (FB == 2 && !WHOLE && parts > 1) {
     // Part of a tile: the workgroup that arrives last adds the parts up in the order of their K ranges, so the sum does
@@ -1491,21 +1538,22 @@ int dispatch_gemm(const uint8_t* A_values, const uint8_t* A_scales, const uint8_
     const SmallGemmPlan plan = plan_small_gemm(M, N, Kp, groups.n, cus);
     GemmGroups gr = groups;
     gr.tiles_n_each = plan.tiles_n_each;
-#define LL_SMALL_LAUNCH(WHOLE, FB, wgs, lds, records, arrivals)                                                            \
+#define LL_SMALL_LAUNCH(WHOLE, FB, SETS, wgs, lds, records, arrivals)                                                            \
   do {                                                                                                                       \
     static std::atomic<uint64_t> lds_allowed{0};                                                                              \
-    if (int rc = allow_dynamic_lds(reinterpret_cast<const void*>(&gemm_w4a4_small_kernel<WHOLE, FB>), lds, lds_allowed, "ll_nvfp4_gemm_tnt")) return rc; \
-    hipLaunchKernelGGL((gemm_w4a4_small_kernel<WHOLE, FB>), dim3((unsigned)(((wgs) + 7) / 8 * 8)), dim3(kSmallThreads), lds, s, A_values, A_scales, \
+    if (int rc = allow_dynamic_lds(reinterpret_cast<const void*>(&gemm_w4a4_small_kernel<WHOLE, FB, SETS>), lds, lds_allowed, "ll_nvfp4_gemm_tnt")) return rc; \
+    hipLaunchKernelGGL((gemm_w4a4_small_kernel<WHOLE, FB, SETS>), dim3((unsigned)(((wgs) + 7) / 8 * 8)), dim3(SETS * kSmallThreads), lds, s, A_values, A_scales, \
                        B_values, B_scales, alpha, amax_a, amax_b, 1.0f / denom_a, 1.0f / denom_b, (int)M, (int)N, (int)Mp, (int)Np, (int)Kp, \
                        static_cast<uint16_t*>(D), ldd, plan.tiles_m, plan.tiles_n_each * gr.n, epi, gr, plan.parts, records, arrivals);   \
   } while (0)
     StreamScratch w;
     if (plan.fb == 3) {
-      LL_SMALL_LAUNCH(false, 3, plan.tiles, SmallTile<3>::kRing, nullptr, nullptr);
+      if (plan.sets == 2) LL_SMALL_LAUNCH(false, 3, 2, plan.tiles, (SmallTile<3, 2>::kRing), nullptr, nullptr);
+      else LL_SMALL_LAUNCH(false, 3, 1, plan.tiles, SmallTile<3>::kRing, nullptr, nullptr);
     } else if (plan.parts > 1 && !small_product_scratch(dev, s, cus, w)) {
-      LL_SMALL_LAUNCH(true, 2, plan.tiles, kSmallWholeSmem, nullptr, nullptr);
+      LL_SMALL_LAUNCH(true, 2, 1, plan.tiles, kSmallWholeSmem, nullptr, nullptr);
     } else {
-      LL_SMALL_LAUNCH(false, 2, plan.tiles * plan.parts, SmallTile<2>::kRing, reinterpret_cast<float*>(w.records), w.counters);
+      LL_SMALL_LAUNCH(false, 2, 1, plan.tiles * plan.parts, SmallTile<2>::kRing, reinterpret_cast<float*>(w.records), w.counters);
     }
 #undef LL_SMALL_LAUNCH
     LL_CHECK_LAUNCH("gemm_w4a4_small_kernel");

@@ -885,6 +885,9 @@ def test_small_products_with_k_shared_between_waves_and_workgroups(gpu, M, N, K,
     (1030, 1000, 1088, 1),    # 64 x 96 tiles: the last one reaches behind the padded matrix, tiles across 128-row scale blocks
     (1100, 930, 1024, 1),     # the same where it ends inside, N no multiple of 8
     (500, 700, 1344, 3),      # three products, a ragged last step
+    (512, 3072, 2048, 1),     # two sets of waves: the shortest K, as many steps for either
+    (1030, 1000, 2112, 1),    # the second set has a step less, the last one of the first is a quarter; ragged both ways
+    (700, 1000, 2496, 2),     # the last step, of the second set, three quarters; two products
 ])
 def test_small_products_of_more_tiles_than_compute_units(gpu, M, N, K, groups):
     test_small_products_with_k_shared_between_waves_and_workgroups(gpu, M, N, K, groups)

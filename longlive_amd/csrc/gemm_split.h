@@ -183,6 +183,16 @@ inline TileKernelChoice choose_tile_kernel(int64_t M, int64_t N, int64_t Kp, int
   return {best, generated_ok && best >= 2};
 }
 
+// Sets of four waves of a workgroup that computes a tile of 128 x 128: two while every tile has a unit to itself, where the
+// four waves of one had a SIMD each and waited for every instruction.  us, one set / two: 736 x 4608 x 1536 19.2 / 17.3, 1000 x
+// 4096 x 2048 24.7 / 22.3, 800 x 4096 x 4096 41.0 / 36.0, 640 x 6400 x 896 14.6 / 13.8, with gate or residual 2 to 4 more off; x 384
+// 9.74 / 9.69.  One order of summation for every shape (LL_GEMM_TILES_COMPILED) needs one set.
+constexpr int64_t kTileSetsK = 512;
+inline int tile_kernel_sets(int64_t M, int64_t N, int64_t Kp, int n_products, int cus, int schedule) {
+  const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128) * n_products;
+  return schedule != 2 /* LL_GEMM_TILES_COMPILED */ && tiles <= cus && Kp >= kTileSetsK ? 2 : 1;
+}
+
 // How the small-product kernel divides a launch: 64 x 64 tiles, each by `parts` workgroups that share its K range (steps of
 // 256 elements).  Measured when a step took 0.55 us (0.47 now) with one workgroup on every compute unit; handing two to
 // four parts over and adding them up takes 2.4 us (their records are read four at a time: five to eight 3.6); with more

@@ -23,6 +23,7 @@
 #include "gemm_epilogue.h"
 #include "gemm_split.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace ll {
@@ -56,8 +57,11 @@ struct GemmSmem {
   static constexpr int kStage = kAVals + kBVals + kAScales + kBScales;
 };
 
-template <int FA, int FB>
-__global__ __launch_bounds__(kGemmThreads, 2) void gemm_w4a4_kernel(
+// SETS = 2 (tiles of 128 x 128, no more than compute units: tile_kernel_sets): eight waves, two sets of four that take every other K
+// step in stages of their own, where the four waves of one would each have a SIMD to itself; each set finishes half of the
+// sums.
+template <int FA, int FB, int SETS = 1>
+__global__ __launch_bounds__(SETS * kGemmThreads, 2) void gemm_w4a4_kernel(
     const uint8_t* __restrict__ Av, const uint8_t* __restrict__ As, const uint8_t* __restrict__ Bv0,
     const uint8_t* __restrict__ Bs0, const float* __restrict__ alpha_ptr0, const float* __restrict__ amax_a,
     const float* __restrict__ amax_b0, float inv_denom_a, float inv_denom_b0, int M, int N, int Mp, int Np, int Kp,
@@ -122,7 +126,9 @@ __global__ __launch_bounds__(kGemmThreads, 2) void gemm_w4a4_kernel(
   const int row0 = tile_m * BM;  // first row of A (output row)
   const int col0 = tile_n * BN;  // first row of B (output column)
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x % kGemmThreads, set = SETS == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / kGemmThreads);
+  const int lane = tid & 63, wave = tid >> 6;
+  uint8_t* const stages = smem + set * 2 * S::kStage;
   const int wm = wave & 1, wn = wave >> 1;
   const int l32 = lane & 31, lh = lane >> 5;
 
@@ -170,8 +176,8 @@ __global__ __launch_bounds__(kGemmThreads, 2) void gemm_w4a4_kernel(
   // Kp is a multiple of 64 but maybe not of 128: in the last step the second 64 elements may not exist; the
   // lanes that would fetch them fetch zeros instead.
   auto load_step = [&](int t, int stage) {
-    const uint32_t base = lds_address(smem + stage * S::kStage + wave * 1024);
-    const uint32_t sbase = lds_address(smem + stage * S::kStage + s_dst);
+    const uint32_t base = lds_address(stages + stage * S::kStage + wave * 1024);
+    const uint32_t sbase = lds_address(stages + stage * S::kStage + s_dst);
     const bool second_half_valid = (t * kBK + 64) < Kp;
     if (second_half_valid) {
 #pragma unroll
@@ -223,7 +229,7 @@ __global__ __launch_bounds__(kGemmThreads, 2) void gemm_w4a4_kernel(
     half2v as[FA][2], bs[FB][2];
   };
   auto read_half = [&](Half& h, int stage, int cc) {
-    const uint8_t* base = smem + stage * S::kStage;
+    const uint8_t* base = stages + stage * S::kStage;
 #pragma unroll
     for (int f = 0; f < FA; ++f) {
       h.a[f] = *reinterpret_cast<const uint4*>(base + (a_voff[f] ^ (32 * cc)));
@@ -265,7 +271,7 @@ __global__ __launch_bounds__(kGemmThreads, 2) void gemm_w4a4_kernel(
   // ---- main loop: two LDS stages, the loads of step t+1 in flight into the other stage while step t is
   // computed.
   {
-    load_step(0, 0);
+    if (set < nk) load_step(set, 0);
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's pieces are in LDS
     __syncthreads();
     // A wave whose rows (or columns) all lie beyond M (N) only helps with the staging: in the last row of
@@ -278,9 +284,9 @@ __global__ __launch_bounds__(kGemmThreads, 2) void gemm_w4a4_kernel(
       // issue until the matrix pipe is free again).  The MFMAs of the last sub-step of a K step are issued after
       // the barrier, behind the LDS reads of the next step, whose latency they cover.
       Operands o[2];
-      for (int t = 0; t < nk; ++t) {
-        if (t + 1 < nk) load_step(t + 1, (t + 1) & 1);
-        if (wave_has_output) {
+      for (int t = 0; t < (nk + SETS - 1) / SETS; ++t) {  // the set's steps: SETS t + set
+        if (SETS * (t + 1) + set < nk) load_step(SETS * (t + 1) + set, (t + 1) & 1);
+        if (wave_has_output && SETS * t + set < nk) {
           Half h[2];
           read_half(h[0], t & 1, 0);
           read_half(h[1], t & 1, 1);
@@ -300,7 +306,7 @@ __global__ __launch_bounds__(kGemmThreads, 2) void gemm_w4a4_kernel(
         __builtin_amdgcn_s_waitcnt(0x0F70);
         __syncthreads();
       }
-      if (wave_has_output) mma(o[1]);
+      if (wave_has_output && set < nk) mma(o[1]);
     } else {
       // Large tiles (8 fragments pairs per wave): the same software pipeline, with the packed dwords read from LDS
       // one sub-step ahead instead of a whole K step at a time, which is what lets it fit 256 registers.
@@ -378,6 +384,35 @@ __global__ __launch_bounds__(kGemmThreads, 2) void gemm_w4a4_kernel(
     alpha = alpha_ptr[0];
   } else {
     alpha = (amax_a[0] * amax_b[0]) * (inv_denom_a * inv_denom_b);
+  }
+  if constexpr (SETS == 2) {  // set 0 finishes the first fragment of A, set 1 the second
+    static_assert(FA == 2);
+    constexpr int kExchange = 8 * FB * 4096;
+    float* sums = reinterpret_cast<float*>(smem) + lane * 4;
+    float16v kept[FB][1];
+#pragma unroll
+    for (int g = 0; g < FB; ++g) {
+      const float16v give = set == 0 ? acc[g][1] : acc[g][0];
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        *reinterpret_cast<float4*>(sums + ((4 * set + wave) * FB + g) * 1024 + i * 256) = make_float4(give[4 * i], give[4 * i + 1], give[4 * i + 2], give[4 * i + 3]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int g = 0; g < FB; ++g) {
+      const float16v keep = set == 0 ? acc[g][0] : acc[g][1];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float4 x = *reinterpret_cast<const float4*>(sums + ((4 * (set ^ 1) + wave) * FB + g) * 1024 + i * 256);
+        kept[g][0][4 * i] = keep[4 * i] + x.x;
+        kept[g][0][4 * i + 1] = keep[4 * i + 1] + x.y;
+        kept[g][0][4 * i + 2] = keep[4 * i + 2] + x.z;
+        kept[g][0][4 * i + 3] = keep[4 * i + 3] + x.w;
+      }
+    }
+    gemm_epilogue<1, FB, 4>(kept, alpha, smem + kExchange, 4 * set + wave, lane, row0 + wm * 32 * FA + 32 * set, col0 + wn * 32 * FB, M, N, D, ldd,
+                            bias, act, epi, (uint32_t)blockIdx.x * 8 + 4 * set + wave);
+    return;
   }
   gemm_epilogue<FA, FB, FA * FB < 8 ? 4 : 2>(acc, alpha, smem, wave, lane, row0 + wm * 32 * FA, col0 + wn * 32 * FB, M, N, D, ldd, bias, act, epi,
                         (uint32_t)blockIdx.x * 4 + wave);
@@ -1357,7 +1392,7 @@ __global__ __launch_bounds__(kSplitThreads) void gemm_w4a4_asm8_kernel(
 
 static std::atomic<int> g_gemm_schedule{LL_GEMM_AUTO};
 
-template <int FA, int FB>
+template <int FA, int FB, int SETS = 1>
 int launch_gemm(const uint8_t* Av, const uint8_t* As, const uint8_t* Bv, const uint8_t* Bs, const float* alpha,
                 const float* amax_a, const float* amax_b, float denom_a, float denom_b, int M, int N, int Mp, int Np,
                 int Kp, void* D, int64_t ldd, const GemmEpilogue& epi, GemmGroups groups, hipStream_t stream,
@@ -1380,10 +1415,11 @@ int launch_gemm(const uint8_t* Av, const uint8_t* As, const uint8_t* Bv, const u
       return LL_OK;
     }
   }
-  const size_t smem = 2 * S::kStage;
+  // two sets: their sums and the epilogue's patches behind those
+  const size_t smem = SETS == 1 ? 2 * S::kStage : std::max(SETS * 2 * S::kStage, 8 * FB * 4096 + 8 * 32 * (64 * FB + 16));
   static std::atomic<uint64_t> lds_allowed{0};  // one per tile configuration
-  if (int rc = allow_dynamic_lds(reinterpret_cast<const void*>(&gemm_w4a4_kernel<FA, FB>), smem, lds_allowed, "ll_nvfp4_gemm_tnt")) return rc;
-  hipLaunchKernelGGL((gemm_w4a4_kernel<FA, FB>), dim3((unsigned)(tiles_m * tiles_n)), dim3(kGemmThreads), smem, stream,
+  if (int rc = allow_dynamic_lds(reinterpret_cast<const void*>(&gemm_w4a4_kernel<FA, FB, SETS>), smem, lds_allowed, "ll_nvfp4_gemm_tnt")) return rc;
+  hipLaunchKernelGGL((gemm_w4a4_kernel<FA, FB, SETS>), dim3((unsigned)(tiles_m * tiles_n)), dim3(SETS * kGemmThreads), smem, stream,
                      Av, As, Bv, Bs, alpha, amax_a, amax_b, 1.0f / denom_a, 1.0f / denom_b, M, N, Mp, Np, Kp,
                      static_cast<uint16_t*>(D), ldd, tiles_m, tiles_n, epi, groups);
   LL_CHECK_LAUNCH("gemm_w4a4_kernel");
@@ -1564,7 +1600,9 @@ int dispatch_gemm(const uint8_t* A_values, const uint8_t* A_scales, const uint8_
   switch (choice.kernel) {
     case LL_GEMM_KERNEL_256X128: return launch_gemm<4, 2>(LL_GEMM_ARGS);
     case LL_GEMM_KERNEL_128X256: return launch_gemm<2, 4>(LL_GEMM_ARGS);
-    case LL_GEMM_KERNEL_128X128: return launch_gemm<2, 2>(LL_GEMM_ARGS);
+    case LL_GEMM_KERNEL_128X128:
+      return tile_kernel_sets(M, N, Kp, groups.n, cus, g_gemm_schedule.load(std::memory_order_relaxed)) == 2 ? launch_gemm<2, 2, 2>(LL_GEMM_ARGS)
+                                                                                                           : launch_gemm<2, 2>(LL_GEMM_ARGS);
     default: return launch_gemm<1, 1>(LL_GEMM_ARGS);
   }
 #undef LL_GEMM_ARGS

@@ -893,6 +893,37 @@ def test_small_products_of_more_tiles_than_compute_units(gpu, M, N, K, groups):
     test_small_products_with_k_shared_between_waves_and_workgroups(gpu, M, N, K, groups)
 
 
+@pytest.mark.parametrize("M,N,K,groups", [
+    (640, 6400, 512, 1),     # the shortest K that two sets share, two steps each
+    (1020, 4088, 1088, 1),   # nine steps, the last one, of the first set, a half; ragged both ways
+    (640, 1800, 896, 3),     # seven steps, three products, a ragged last column of tiles
+    (600, 6160, 1216, 1),    # ten steps, the last one, of the second set, a half; waves without rows or columns
+])
+def test_tiles_in_two_sets_of_waves(gpu, M, N, K, groups):
+    """128 x 128 tiles of which every one has a compute unit to itself deal K to two sets of waves: the bound of the small
+    products, and the same bits twice; residual and the maximum of the results."""
+    cfg = QuantizationConfig(scale_rule="mse")
+    xq = quantize_to_fp4(activations((M, K), 25).to(gpu), cfg)
+    ws = [quantize_to_fp4((weights((N, K), 26 + i) * (1 + i)).to(gpu), cfg) for i in range(groups)]
+    assert _native.gemm_kernel(M, N, xq.padded_shape[1], groups)["kernel"] == "128x128"
+
+    def run():
+        return list(_native.gemm_grouped(xq.values, xq.scale_factors, xq.amax, 1536.0, M, N,
+                                         [dict(values=w.values, scales=w.scale_factors, amax=w.amax, denom=1536.0) for w in ws]))
+
+    with _native.gemm_schedule("tiles_compiled"):
+        want = run()
+    for a, b, c in zip(run(), run(), want):
+        assert torch.equal(a, b)
+        _ulp_close(a, c, frac=5e-3)
+    if groups == 1:
+        ticket = _native.amax_ticket(gpu)
+        residual = activations((M, N), 5).to(gpu)
+        y = fp4_matmul(xq, ws[0], residual=residual, amax_out=ticket)
+        assert torch.equal(y, residual + a)
+        assert float(quantize_to_fp4(y, cfg, amax=ticket).amax) == float(y.float().abs().max())
+
+
 def test_recorded_small_products_replayed_at_the_same_time(gpu):
     """Products whose K range several workgroups share, recorded twice on one stream that has run them before and replayed
     on two streams beside the same work on the recording stream: every result has the bits of the launch by itself."""

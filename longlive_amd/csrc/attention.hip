@@ -29,7 +29,6 @@
 #include <cfloat>
 #include <map>
 #include <mutex>
-#include <type_traits>
 #include <utility>
 
 namespace ll {
@@ -80,7 +79,6 @@ struct SlotTable {
   const uint8_t* vs[kMaxSlots];
   float kg[kMaxSlots];
   float vg[kMaxSlots];
-  int direct;        // whether this workgroup's probabilities keep the reference point that a segment's first keys gave them
   int last_arrival;  // whether this workgroup completed the tile it just left a partial result for
 };
 
@@ -276,12 +274,6 @@ __device__ __forceinline__ void write_rows(const float16v (&o)[N], float inv_l, 
   }
 }
 
-// f(0), f(1), ... with every index a constant of its own type.
-template <typename F, int... I>
-__device__ __forceinline__ void each_index(F& f, std::integer_sequence<int, I...>) {
-  (f(std::integral_constant<int, I>{}), ...);
-}
-
 template <bool WIDE>
 __global__ __launch_bounds__(kAttnThreads) void kv_attention_kernel(AttnParams p) {
   constexpr int kQueries = WIDE ? 2 * kWgQueries : kWgQueries;  // queries per workgroup
@@ -306,7 +298,6 @@ __global__ __launch_bounds__(kAttnThreads) void kv_attention_kernel(AttnParams p
     tab.kg[tid] = load_global<float>(reinterpret_cast<const void*>(p.ka_ptrs[tid])) * p.inv_denom;
     tab.vg[tid] = load_global<float>(reinterpret_cast<const void*>(p.va_ptrs[tid])) * p.inv_denom;
   }
-  if (threadIdx.x == 0) tab.direct = 1;
 
   __syncthreads();
 
@@ -318,20 +309,16 @@ __global__ __launch_bounds__(kAttnThreads) void kv_attention_kernel(AttnParams p
   // tail of one tile followed by the head of the next, and with the head (keys from 0) first and the tail
   // (keys up to the end) last, all workgroups of the launch move through the key range together, a few
   // iterations apart at most, which is what lets those of one head find each other's K/V lines in the L2.
-  int tile_id, seg_begin, seg_end;
-  bool again = false;  // the same segment once more, with the maximum followed
   for (;;) {
+  int tile_id, seg_begin, seg_end;
   bf16x8 qf[8];
   if constexpr (WIDE) {
-    if (!again) {
-      const auto& c = reread_params();
-      Segment seg;
-      if (!next_segment(at, group_number(c.d.G), division_of(c), seg)) break;
-      tile_id = (int)seg.tile;
-      seg_begin = seg.begin;
-      seg_end = seg.end;
-    }
-    again = false;
+    const auto& c = reread_params();
+    Segment seg;
+    if (!next_segment(at, group_number(c.d.G), division_of(c), seg)) break;
+    tile_id = (int)seg.tile;
+    seg_begin = seg.begin;
+    seg_end = seg.end;
   } else {
     const uint32_t g = group_number(p.d.G), part = g % p.parts;
     tile_id = (int)(g / p.parts);
@@ -544,154 +531,6 @@ __global__ __launch_bounds__(kAttnThreads) void kv_attention_kernel(AttnParams p
     l_run += sum;
   };
 
-  // 256-query tiles, tiles of 128 keys that are all there.  The reference point of the exponentials is the maximum over a segment's
-  // first 32 keys and stays there: no maximum per tile, no wait for it, and the exponentials of 32 keys begin while the MFMAs of
-  // the next 32 run.  Probabilities then reach beyond 1, which fp32 and bf16 hold as exactly; where a query's scores grow by some
-  // 2^100 or its results leave the range, the segment is run once more with the maximum followed (`again`, below), and the
-  // workgroup follows it from then on.
-  // What bounds the loop is the power limit: the MFMA pipe is busy 55 % of the cycles at 1.93 GHz, and with zeros for operands the same
-  // cycles take 15 % less time, so what counts is what is not executed.  160 vector instructions per wave and iteration convert,
-  // 160 are the softmax.  The iteration is 64 slots of one MFMA with what is to run beside it, held in place by scheduling barriers,
-  // in which no instruction waits for another.  Row sums are added up in fp32, of the probabilities ahead of their rounding to bf16:
-  // of the rounded ones, four to an MFMA of 4 x 4 x 4, they cost 0.6 % less (a chunk step of 2640 x 24 418.9 us, so 421.9), but where one
-  // probability outweighs the others its rounding would scale what the others add by up to 2^-8.  Raw bytes are asked for
-  // without branches, behind which the compiler waits for every load under way (one busy wave per SIMD: 247 us, so 202).
-  // With the maximum followed per tile (as softmax_pv does) / so, us: 7040 queries x 24 heads over 21120 cached + 7040 keys 2276 /
-  // 2135, 2560 x 24 over 10560 + 2640 452 / 425, one tile of 80 queries per unit over 13200 keys 226 / 202.
-  const bool direct = WIDE && __builtin_amdgcn_readfirstlane(tab.direct) != 0;
-  int it = seg_begin;
-  float neg_direct = 0.0f;
-  auto direct_iteration = [&](auto convert_tag) __attribute__((always_inline)) {
-    constexpr bool kConvert = decltype(convert_tag)::value;
-    typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
-    typedef __attribute__((address_space(3))) bf16x4* lds_bf16x4_t;
-    const uint8_t* cur = smem + (it & 1) * kStageBytes;
-    uint8_t* nxt = smem + ((it + 1) & 1) * kStageBytes;
-    const uint8_t* k_lane = cur + l32 * kKPitch + lh * 16;
-    const uint8_t* v_lane = cur + 2 * kKTileBytes + (4 * lh + ((lane & 15) >> 2)) * kVPitch + (16 * ((lane >> 4) & 1) + 4 * (lane & 3)) * 2;
-    uint8_t* kdst = nxt + k_dst_off;
-    uint8_t* vdst = nxt + v_dst_off;
-    constexpr int kAhead = 5, kRing = 6;
-    uint4 fk[kRing];
-    bf16x4 fv[2][4][2];
-    float16v sc[2];
-    uint32_t pw[16];
-    half2v s2[2], t[4];
-    float v8[8], x[2][2], e[2][2];
-    float sums[2] = {0.0f, 0.0f};
-    const float gs_k = k_gs, gs_v = v_gs;
-    const uint8_t *values, *scales;  // where the raw registers are filled from next
-    uint32_t vo, so;
-    int next_slot;
-    auto read_k = [&](auto tag) __attribute__((always_inline)) {  // fragment f % 16 of the 64 keys f / 16
-      constexpr int f = decltype(tag)::value;
-      fk[f % kRing] = *reinterpret_cast<const uint4*>(k_lane + (f >> 4) * kKTileBytes + ((f >> 3) & 1) * 32 * kKPitch + (f & 7) * 32);
-    };
-    each_index(read_k, std::make_integer_sequence<int, kAhead>{});
-    __builtin_amdgcn_sched_barrier(0);
-    auto one_slot = [&](auto slot_tag) __attribute__((always_inline)) {
-      constexpr int slot = decltype(slot_tag)::value, h = slot >> 5, i = slot & 31;
-      // LDS reads: K five slots ahead of its MFMA, V four
-      if constexpr (i < 16 - kAhead) read_k(std::integral_constant<int, h * 16 + i + kAhead>{});
-      if constexpr (h == 0 && i >= 32 - kAhead) read_k(std::integral_constant<int, 16 + i - (32 - kAhead)>{});
-      if constexpr (i >= 12 && i < 28) {
-        constexpr int step = (i - 12) >> 2, dt = i & 3;
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-          fv[step & 1][dt][j] = __builtin_amdgcn_ds_read_tr16_b64_v4bf16(
-              (lds_bf16x4_t)(v_lane + h * kVTileBytes + (16 * step + 8 * j) * kVPitch + dt * 64));
-      }
-      __builtin_amdgcn_sched_barrier(0);
-      // S^T in slots 0-15 (32 keys after 32 keys), O^T in slots 16-31
-      if constexpr (i < 16) {
-        constexpr int kt = i >> 3, ks = i & 7;
-        const float16v zero = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-        sc[kt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, fk[(h * 16 + i) % kRing]), qf[ks], ks == 0 ? zero : sc[kt], 0, 0, 0);
-      } else {
-        constexpr int step = (i - 16) >> 2, dt = i & 3;
-        const bf16x4(&v)[2] = fv[step & 1][dt];
-        const bf16x8 a = __builtin_shufflevector(v[0], v[1], 0, 1, 2, 3, 4, 5, 6, 7);
-        const bf16x8 b = __builtin_bit_cast(bf16x8, make_uint4(pw[4 * step], pw[4 * step + 1], pw[4 * step + 2], pw[4 * step + 3]));
-        o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, o[dt], 0, 0, 0);
-      }
-      if constexpr (slot == 8) {
-        if (it == seg_begin) {
-          float mx = sc[0][0];
-#pragma unroll
-          for (int r = 1; r < 16; ++r) mx = fmaxf(mx, sc[0][r]);
-          m_run = max_over_wave_halves(mx);
-          neg_direct = -m_run * p.scale_log2;
-        }
-      }
-      // probabilities: pair p's multiply-adds, exponentials, packing and sum in four slots in a row
-      if constexpr (i >= 11 && i < 27) {
-        constexpr int pair = i - 11;
-        pw[pair] = pack_bf16(e[pair & 1][0], e[pair & 1][1]);
-        sums[0] += e[pair & 1][0];
-        sums[1] += e[pair & 1][1];
-      }
-      if constexpr (i >= 10 && i < 26) {
-        constexpr int pair = i - 10;
-        e[pair & 1][0] = __builtin_amdgcn_exp2f(x[pair & 1][0]);
-        e[pair & 1][1] = __builtin_amdgcn_exp2f(x[pair & 1][1]);
-      }
-      if constexpr (i >= 9 && i < 25) {
-        constexpr int pair = i - 9, kt = pair >> 3, r = 2 * (pair & 7);
-        x[pair & 1][0] = fmaf(sc[kt][r], p.scale_log2, neg_direct);
-        x[pair & 1][1] = fmaf(sc[kt][r + 1], p.scale_log2, neg_direct);
-      }
-      // conversion of the next tile: a dword's conversions, scaling, widening and packing in four slots in a row
-      if constexpr (kConvert && (i < 9 || i >= 25)) {
-        constexpr int piece = i < 9 ? i : i - 16, j = piece >> 2;  // dword j of the row, K under the first tile, V under the second
-        const KRaw& raw = h == 0 ? kf : vf;
-        const uint32_t w = j == 0 ? raw.v.x : j == 1 ? raw.v.y : j == 2 ? raw.v.z : raw.v.w;
-        const float gs = h == 0 ? gs_k : gs_v;
-        if constexpr (piece == 0) block_scales_f16(raw.scales, s2);
-        if constexpr ((piece & 3) == 0) {
-          t[0] = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 0);
-          t[1] = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 1);
-          t[2] = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 2);
-          t[3] = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 3);
-        }
-        if constexpr ((piece & 3) == 1) {
-#pragma unroll
-          for (int n = 0; n < 4; ++n) t[n] = t[n] * s2[j >> 1];
-        }
-        if constexpr ((piece & 3) == 2) {
-#pragma unroll
-          for (int n = 0; n < 4; ++n) {
-            v8[2 * n] = widen_mul_lo(t[n], gs);
-            v8[2 * n + 1] = widen_mul_hi(t[n], gs);
-          }
-        }
-        if constexpr ((piece & 3) == 3)
-          reinterpret_cast<uint4*>(h == 0 ? kdst : vdst)[j] =
-              make_uint4(pack_bf16(v8[0], v8[1]), pack_bf16(v8[2], v8[3]), pack_bf16(v8[4], v8[5]), pack_bf16(v8[6], v8[7]));
-      }
-      __builtin_amdgcn_sched_barrier(0);
-      // raw bytes of the tile behind the next one: K once its registers are free, V half an iteration later
-      if constexpr (kConvert && slot == 9) {
-        advance();
-        const bool there = it + 2 < seg_end && iter_base + k_local < n_cached;
-        vo = there ? k_vo : 0;
-        so = there ? k_so : 0;
-        next_slot = there ? k_slot : 0;
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      if constexpr (kConvert && (slot == 26 || slot == 58)) {
-        values = (h == 0 ? tab.kv : tab.vv)[next_slot];
-        scales = (h == 0 ? tab.ks : tab.vs)[next_slot];
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      if constexpr (kConvert && (slot == 31 || slot == 63)) {
-        fetch_row(values, scales, vo, so, h == 0 ? kf : vf);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    };
-    each_index(one_slot, std::make_integer_sequence<int, 64>{});
-    l_run += sums[0] + sums[1];
-  };
-
   // prologue: the segment's first iteration into its stage, raw registers <- the second one
   fetch_next();
   if constexpr (!WIDE) {
@@ -711,11 +550,12 @@ __global__ __launch_bounds__(kAttnThreads) void kv_attention_kernel(AttnParams p
   __builtin_amdgcn_s_waitcnt(0x0F70);
 
   // Iterations whose own 128 keys all exist and whose successor is all FP4 form a prefix of the key range;
-  // they run the interleaved body (128-query tiles): S^T (64 keys x 32 queries) = 16 MFMAs in eight steps of two, each step
+  // they run the interleaved body: S^T (64 keys x 32 queries) = 16 MFMAs in eight steps of two, each step
   // also converting one dword of the prefetched K row (even steps) or V row (odd steps) into the other LDS
-  // stage.  The rest (the bf16 chunk, the tail; 256-query tiles that follow the maximum) runs the plain
+  // stage.  The rest (the bf16 chunk, the tail) runs the plain
   // body in a loop of its own.
   const int n_fast = min(n_cached / kIterKeys, seg_end) - 1;
+  int it = seg_begin;
   if (wave_idle) {
     // A wave without queries: the conversion of its rows, the same number of barriers, nothing else.
     for (; it < n_fast; ++it) {
@@ -742,15 +582,13 @@ __global__ __launch_bounds__(kAttnThreads) void kv_attention_kernel(AttnParams p
       __syncthreads();
     }
   }
-  if constexpr (WIDE) {
-    if (direct) {
-      for (; it < n_fast; ++it) {
-        direct_iteration(std::true_type{});
-        __syncthreads();
-      }
-    }
-  }
-  for (; !WIDE && it < n_fast; ++it) {
+  // Where this loop of 5 KB begins is worth 0.5 to 2 %: 256-query tiles whose key ranges are shared are fastest with its first
+  // instruction 32 bytes behind a 64-byte line, where these put it together with the register copies that the compiler sets in
+  // between.  us, 28 / 32 bytes behind the line: 2328 queries x 16 heads over 9312 cached + 2328 keys 244 / 241, on another card
+  // 237.5 / 235.7, 2856 x 16 over 11424 + 2856 338 / 333 and 331.7 / 329.4, 3088 x 24 over 3088 + 3088 263 / 259 and 256.2 / 254.7;
+  // whole tiles: 2640 x 24 over 10560 + 2640 413 / 411.5 and 408.9 / 406.9.
+  if constexpr (WIDE) asm volatile(".p2align 6\n\ts_nop 0\n\ts_nop 0\n\ts_nop 0\n\ts_nop 0");
+  for (; it < n_fast; ++it) {
     const uint8_t* cur = smem + (it & 1) * kStageBytes;
     uint8_t* nxt = smem + ((it + 1) & 1) * kStageBytes;
     const bool has_next2 = it + 2 < seg_end;
@@ -760,9 +598,11 @@ __global__ __launch_bounds__(kAttnThreads) void kv_attention_kernel(AttnParams p
     block_scales_f16(vf.scales, vs2);
     uint8_t* kdst = nxt + k_dst_off;
     uint8_t* vdst = nxt + v_dst_off;
-    {
+#pragma unroll
+    for (int h = 0; h < kHalves; ++h) {
+      const int tile = WIDE ? h : kp;
       float16v sc[2];
-      const uint8_t* krow0 = cur + kp * kKTileBytes + l32 * kKPitch + lh * 16;
+      const uint8_t* krow0 = cur + tile * kKTileBytes + l32 * kKPitch + lh * 16;
       const uint8_t* krow1 = krow0 + 32 * kKPitch;
 #pragma unroll
       for (int kt = 0; kt < 2; ++kt)
@@ -785,10 +625,11 @@ __global__ __launch_bounds__(kAttnThreads) void kv_attention_kernel(AttnParams p
         const bf16x8 fa0 = __builtin_bit_cast(bf16x8, fk[ks % 3][0]), fa1 = __builtin_bit_cast(bf16x8, fk[ks % 3][1]);
         sc[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa0, qf[ks], sc[0], 0, 0, 0);
         sc[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa1, qf[ks], sc[1], 0, 0, 0);
-        // One dword (8 elements) of the prefetched rows at a time, K in the even steps, V in the odd ones.
-        {
+        // One dword (8 elements) of the prefetched rows at a time.  One tile per wave: K in the even steps, V in the
+        // odd ones.  Two tiles per wave: every second step, K under the first tile's MFMAs and V under the second's.
+        if (!WIDE || (ks & 1) == 0) {
           const int j = ks >> 1;
-          const bool is_k = (ks & 1) == 0;
+          const bool is_k = WIDE ? h == 0 : (ks & 1) == 0;
           float v8[8];
           fp4x8_to_f32(is_k ? wk[j] : wv[j], is_k ? ks2[j >> 1] : vs2[j >> 1], is_k ? k_gs : v_gs, v8);
           reinterpret_cast<uint4*>(is_k ? kdst : vdst)[j] = make_uint4(pack_bf16(v8[0], v8[1]), pack_bf16(v8[2], v8[3]),
@@ -796,9 +637,11 @@ __global__ __launch_bounds__(kAttnThreads) void kv_attention_kernel(AttnParams p
         }
         __builtin_amdgcn_sched_barrier(0);
       }
-      advance();
-      if (has_next2) fetch_next();
-      softmax_pv(sc, cur + 2 * kKTileBytes + kp * kVTileBytes);
+      if (h == kHalves - 1) {
+        advance();
+        if (has_next2) fetch_next();
+      }
+      softmax_pv(sc, cur + 2 * kKTileBytes + tile * kVTileBytes);
     }
     __syncthreads();
   }
@@ -851,12 +694,8 @@ __global__ __launch_bounds__(kAttnThreads) void kv_attention_kernel(AttnParams p
         load_to_lds_b128(source(64 - kKPieces + chunk_wave, kVPitch), v_base, dst + 2 * kKTileBytes + (64 - kKPieces) * 1024);
       }
     }
-    const bool whole = WIDE && direct && (it + 1) * kIterKeys <= Lk_i;  // decoded or copied above, no key missing
-    if constexpr (WIDE) {
-      if (whole && !wave_idle) direct_iteration(std::false_type{});
-    }
 #pragma unroll 1
-    for (int h = whole ? kHalves : 0; h < kHalves; ++h) {
+    for (int h = 0; h < kHalves; ++h) {
       const int tile = WIDE ? h : kp;
       const int tile_base = it * kIterKeys + tile * kTileKeys;
       if (tile_base >= Lk_i || wave_idle) break;
@@ -907,19 +746,6 @@ __global__ __launch_bounds__(kAttnThreads) void kv_attention_kernel(AttnParams p
   }
 
   l_run += __shfl_xor(l_run, 32, 64);  // row sums were per wave half so far
-  if constexpr (WIDE) {
-    if (direct) {  // the vote of the workgroup; its waves share the conversion, so all of them go again or none
-      float odd = l_run < 0x1p100f ? 0.0f : 1.0f;  // stays 0 unless a sum or a result is out of range
-#pragma unroll
-      for (int dt = 0; dt < 4; ++dt)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) odd = fmaf(o[dt][i], 0.0f, odd);
-      if (odd != 0.0f) tab.direct = 0;
-      __syncthreads();
-      again = __builtin_amdgcn_readfirstlane(tab.direct) == 0;
-      if (again) continue;
-    }
-  }
   {  // epilogue of the segment, with its own copies of the thread's coordinates (see fresh_thread_index)
   const auto& c = reread_params();
   const int tid = fresh_thread_index(), lane = tid & 63, wave = tid >> 6;
@@ -928,16 +754,6 @@ __global__ __launch_bounds__(kAttnThreads) void kv_attention_kernel(AttnParams p
     // Every wave has seen its segment of the key range for its 32 queries.
     bool write_out = true;
     if (seg_begin != 0 || seg_end != n_iter) {
-      if (direct && __builtin_amdgcn_ballot_w64(l_run > 0x1p20f) != 0 && p.scale_log2 > 0.0f) {
-        // A part's weight beside the others' is 2^reference point times its sum: bring the reference point back near the maximum.
-        const int e = l_run > 0x1p20f ? __builtin_amdgcn_frexp_expf(l_run) : 0;
-        m_run += (float)e / p.scale_log2;
-        l_run = __builtin_amdgcn_ldexpf(l_run, -e);
-#pragma unroll
-        for (int dt = 0; dt < 4; ++dt)
-#pragma unroll
-          for (int i = 0; i < 16; ++i) o[dt][i] = __builtin_amdgcn_ldexpf(o[dt][i], -e);
-      }
       // Part of a tile.  Whoever arrives last at a tile combines the parts; the others leave their state in a
       // record (two records per workgroup: one for the first tile it touches, one for the last) and count
       // their arrival.  The parts are combined from the end of the key range backwards whoever does it, so

@@ -1151,10 +1151,10 @@ def test_tiles_whose_scores_are_all_minus_infinity_weigh_nothing(gpu, policy, go
 @pytest.mark.parametrize("high,far", [(60.0, (40,)), (60.0, (200, 700, 1190)), (150.0, (40,)), (150.0, (700,)), (150.0, (1100,)), (150.0, (1190,)),
                                       (400.0, (0, 500, 1150))])
 def test_scores_far_above_those_of_the_first_keys(gpu, policy, high, far):
-    """256-query tiles keep the reference point of a segment's first 32 keys and run the segment again where that is too low: keys
-    whose scores lie `high` above the others', within what fp32 holds and beyond, behind the first 32 keys, in later cached tiles, in
-    the chunk and in its ragged last tile; a full and a light group of queries, half of the queries without such keys.  Bound,
-    element by element: half a step of bf16 is at most 2^-8 of a number, of every probability and of the result."""
+    """256-query tiles and keys whose scores lie `high` above the others', within what fp32 holds as exponentials and beyond, behind
+    the first 32 keys, in later cached tiles, in the chunk and in its ragged last tile; a full and a light group of queries, half of
+    the queries without such keys.  Bound, element by element: half a step of bf16 is at most 2^-8 of a number, of every
+    probability and of the result."""
     Lq, H, T, cached, n_new = 300, 2, 384, 1000, 200
     q, k, v = (_randn((n, H, 128), s).to(gpu) for n, s in ((Lq, 71), (cached + n_new, 72), (cached + n_new, 73)))
     q[..., 0], k[..., 0] = 0.0, 0.0
@@ -1176,6 +1176,35 @@ def test_scores_far_above_those_of_the_first_keys(gpu, policy, high, far):
     p = [torch.softmax(q[:, h].double() @ K[:, h].T.contiguous() * 128 ** -0.5, -1) for h in range(H)]
     ref, size = (torch.stack([ph @ x[:, h] for h, ph in enumerate(p)], 1) for x in (V, V.abs()))
     assert ((out.double() - ref).abs() <= 2 ** -8 * (size + ref.abs())).all()
+
+
+@pytest.mark.parametrize("policy", ["wide", "split"])
+@pytest.mark.parametrize("Lq,H,T,cached,n_new", [(300, 2, 384, 1000, 200), (1344, 4, 0, 0, 1344)])
+def test_wide_tiles_weigh_a_dominating_key_exactly(gpu, policy, Lq, H, T, cached, n_new):
+    """Queries along three times a key of their own, spread over all keys: its score lies some 19 or more above zero and the others'
+    within 11 of it, more than 2^8 apart as weights.  The softmax then takes it for its reference point and its weight of 1 costs
+    nothing as bf16.  Bound, element by element: half a step of bf16, 2^-8, of the result and of the other probabilities, and
+    2^-13 of sum p |v| for the scores' and sums' fp32."""
+    q, k, v = (_randn((n, H, 128), s).to(gpu) for n, s in ((Lq, 81), (cached + n_new, 82), (cached + n_new, 83)))
+    from longlive_amd.utils.quant import SlotPointerTable
+    tables, slots, K, V = None, [[], []], [], []
+    if cached:
+        for x, own, rows in ((k, slots[0], K), (v, slots[1], V)):
+            padded = torch.cat([x[:cached], x.new_zeros(-cached % T, H, 128)])
+            own.extend(quantize_to_fp4(padded[i:i + T].reshape(-1, 128), CFG) for i in range(0, len(padded), T))
+            rows.append(dequantize_kv_cache(own, len(own), H, T, torch.bfloat16, gpu)[0][:cached])
+        kt, vt = (SlotPointerTable(own) for own in slots)
+        tables = (kt.values, kt.scales, kt.amax, vt.values, vt.scales, vt.amax)
+    K, V = torch.cat([*K, k[cached:]]), torch.cat([*V, v[cached:]])
+    at = (torch.arange(Lq, device=gpu)[:, None] * len(K) // Lq + torch.arange(H, device=gpu) * 37) % len(K)
+    q = 3 * torch.gather(K, 0, at[:, :, None].expand(Lq, H, 128))
+    with _native.attention_policy(policy):
+        out = _native.kv_attention(q, tables, cached, T, 6.0, 256.0, k[cached:].contiguous(), v[cached:].contiguous(), 128 ** -0.5)
+    K, V = K.double(), V.double()
+    p = [torch.softmax(q[:, h].double() @ K[:, h].T.contiguous() * 128 ** -0.5, -1) for h in range(H)]
+    ref, size = (torch.stack([ph @ x[:, h] for h, ph in enumerate(p)], 1) for x in (V, V.abs()))
+    top = torch.stack([torch.gather(ph, 1, at[:, h:h + 1]) * V[at[:, h], h].abs() for h, ph in enumerate(p)], 1)
+    assert ((out.double() - ref).abs() <= 2 ** -8 * ref.abs() + 2 ** -8 * (size - top) + 2 ** -13 * size).all()
 
 
 @pytest.mark.parametrize("Lq,H,T,cached,n_new", [(512, 16, 512, 0, 4000), (512, 16, 512, 3584, 416), (520, 24, 480, 0, 1900),

@@ -494,8 +494,8 @@ typedef struct ll_row_norm {
  * ll_layer_norm_quantize (weight and bias, either may be NULL) of x bf16 [M, C], contiguous, and ll_nvfp4_gemm_tnt_grouped of
  * the result with `activation` on every product (alpha NULL), in one launch and with the same bits.  For small activations:
  * LL_ENOSUP, and nothing is launched, unless C is a multiple of 64 up to 256, the products ones that ll_nvfp4_gemm_tnt_grouped
- * computes in plain 64 x 64 tiles, and their tiles of 32 x 256 no more than two per compute unit.  row_norms (NULL or n_products, N <= 256):
- * D receives the rows after WanRMSNorm with row_eps and, where asked for, RoPE; the product's sink their maximum.  exchange and spin_limit as
+ * computes in plain 64 x 64 tiles, and their tiles of 32 x 256 no more than two per compute unit.  row_norms (NULL or n_products; LL_ENOSUP
+ * unless N <= 256 and the normed products' biases are 8-byte aligned): D receives the rows after WanRMSNorm with row_eps and, where asked for, RoPE; the product's sink their maximum.  exchange and spin_limit as
  * amax_sink and spin_limit of ll_adaln_quantize; the products' own sinks may be later epochs of the same buffer.
  */
 int ll_nvfp4_norm_gemm(const void* x, int64_t M, int C, const void* scale, const void* shift, int64_t scale_stride,

@@ -479,9 +479,10 @@ extern "C" int ll_nvfp4_norm_gemm(const void* x, int64_t M, int C, const void* s
                      (!rn.rope || (cos && sin && seq_len >= 0)),
                  "%s: product %d: a row norm needs N and ldd of whole 16-byte pieces, no activation, heads of 128 and angles for RoPE", what, i);
       LL_REQUIRE(((reinterpret_cast<uintptr_t>(rn.weight) | reinterpret_cast<uintptr_t>(rn.smooth) | reinterpret_cast<uintptr_t>(products[i].D) |
-                   reinterpret_cast<uintptr_t>(cos) | reinterpret_cast<uintptr_t>(sin)) & 15) == 0 && (reinterpret_cast<uintptr_t>(products[i].bias) & 7) == 0,
-                 "%s: product %d: row norm operands must be 16-byte aligned (bias 8-byte)", what, i);
-      if (N > fused_cols(kAdalnRows)) return LL_ENOSUP;
+                   reinterpret_cast<uintptr_t>(cos) | reinterpret_cast<uintptr_t>(sin)) & 15) == 0,
+                 "%s: product %d: row norm operands must be 16-byte aligned", what, i);
+      // a bias at any element, which the product by itself takes, is loaded here by eights of bytes
+      if (N > fused_cols(kAdalnRows) || (reinterpret_cast<uintptr_t>(products[i].bias) & 7) != 0) return LL_ENOSUP;
       p.row_norm[i] = rn;
     }
     p.row_eps = row_eps;

@@ -1027,6 +1027,32 @@ def test_native_block_call_equals_the_separate_operations(gpu, F, h, w, heads, f
                     assert (a is None and b is None) or torch.equal(a, b), i
 
 
+@pytest.mark.parametrize("heads,h,w", [(2, 8, 8), (4, 16, 24)])
+def test_block_takes_biases_at_any_element(gpu, heads, h, w):
+    """Biases that are views into one parameter buffer, at odd elements: the bits of a block whose biases lie by themselves, where a
+    block's projections share a launch with their norms and where they do not."""
+    torch.manual_seed(0)
+    dim, L = heads * 128, h * w
+    block, _ = quantize_model_with_filter(DiTBlock(dim, 512, heads).to(gpu), ModelQuantizationConfig(), use_default_filtered_modules=True,
+                                          materialize_for_inference=True, verbose=False)
+    g = torch.Generator().manual_seed(6)
+    x, ctx = (torch.randn(1, n, dim, generator=g).bfloat16().to(gpu) for n in (L, 16))
+    e = torch.randn(1, 1, 6, dim, generator=g).bfloat16().to(gpu)
+    cos, sin = rope_cos_sin(build_rope_angles(128), 1, h, w, 0, gpu)
+    outs = []
+    with torch.no_grad():
+        for offset in (0, 1, 3):
+            for linear in [m for m in block.modules() if getattr(m, "bias", None) is not None and hasattr(m, "quantized_weight")]:
+                own = torch.zeros(linear.bias.numel() + 8, dtype=linear.bias.dtype, device=gpu)[offset:offset + linear.bias.numel()]
+                linear.bias = torch.nn.Parameter(own.copy_(linear.bias), requires_grad=False)
+                assert linear.bias.data_ptr() % 8 == 2 * offset
+            cache = kvc.initialize_kv_cache(1, L, 1, heads, 128, KV, gpu)[0]
+            y, (_, _, info) = block(x, e, cos, sin, ctx, cache, 0, L)
+            outs.append((y, info["new_k"], info["new_v"]))
+    for other in outs[1:]:
+        assert all(torch.equal(a, b) for a, b in zip(outs[0], other))
+
+
 @pytest.mark.parametrize("dim,channels,patch,latent", [
     (256, 48, (1, 2, 2), (3, 8, 32)),     # the suite's model: 192 tokens
     (384, 16, (1, 2, 2), (2, 10, 14)),    # 70 tokens: ragged tiles of tokens, N = 64

@@ -84,6 +84,21 @@ def test_one_launch_entry_points_check_their_arguments_before_touching_the_gpu()
     assert b"null amax sink" in lib.ll_last_error()
 
 
+@pytest.mark.parametrize("offset", [2, 4, 6])
+def test_a_bias_at_any_element_is_left_to_the_separate_launches(offset):
+    """ll_nvfp4_norm_gemm with a row norm: the product by itself takes a bias that is a view into a larger buffer, so the launch
+    that does not is not available (LL_ENOSUP = -3) and refuses nothing (LL_EINVAL = -1)."""
+    import ctypes
+    lib = _native.load()
+    buf = (ctypes.c_uint8 * 4096)()                     # aligned host memory: only its address is looked at
+    ptr = ctypes.addressof(buf) + (-ctypes.addressof(buf)) % 256
+    sink = _native.AmaxSinkStruct(ptr, 1, None)
+    product = _native.GemmProduct(ptr, ptr, None, ptr, 1536.0, ptr, 256, ptr + offset, _native.AmaxSinkStruct())
+    row_norm = _native.RowNorm(ptr, None, 0)
+    assert lib.ll_nvfp4_norm_gemm(ptr, 64, 256, None, None, 0, 0, 1, 0, None, None, 1e-6, 3, ctypes.byref(sink), 64, 1536.0, 256, 256, 1,
+                                  ctypes.byref(product), 0, ctypes.byref(row_norm), 1e-6, None, None, 0, None) == -3
+
+
 def test_noalloc_quantize_refuses_inputs_beyond_its_limit_before_touching_the_gpu():
     lib = _native.load()
     limit = lib.ll_nvfp4_quantize_noalloc_max_elements()

@@ -30,7 +30,8 @@ def initialize_kv_cache(num_layers: int, block_token_size: int, max_blocks: int,
     parts = (zero.values, zero.scale_factors.view(torch.uint8), zero.amax)
     buffers = [[torch.empty_like(t) for _ in range(num_layers * 2 * max_blocks)] for t in parts]
     for t, copies in zip(parts, buffers):
-        torch._foreach_copy_(copies, [t] * len(copies))
+        if copies:   # no layers or no blocks: no slots, and nothing that an empty list could be refused for
+            torch._foreach_copy_(copies, [t] * len(copies))
     made = iter([QuantizedTensor(v, s.view(zero.scale_factors.dtype), a, zero.dtype, zero.original_shape, zero.scale_rule, zero.padded_shape)
                  for v, s, a in zip(*buffers)])
     cache = []

@@ -269,6 +269,19 @@ def test_cache_policy_fill_then_roll_matches_reference_numbers():
         kvc.plan_cache_step(_fake_cache(blk, 5), 0, blk // 2, blk)
 
 
+@pytest.mark.parametrize("layers,blocks", [(0, 3), (2, 0), (0, 0), (2, 3)])
+def test_cache_of_no_layers_or_no_blocks(monkeypatch, layers, blocks):
+    """A list of as many layers, each with as many slots of its own buffers, none included."""
+    zero = QuantizedTensor(torch.zeros(128, 64, dtype=torch.uint8), torch.zeros(1024, dtype=torch.uint8).view(torch.float8_e4m3fn),
+                           torch.zeros(1), "nvfp4", (128, 128), "mse", (128, 128))
+    monkeypatch.setattr(kvc, "quantize_to_fp4", lambda *a, **k: zero)
+    cache = kvc.initialize_kv_cache(layers, 128, blocks, 1, 128, QuantizationConfig(), "cpu")
+    assert len(cache) == layers and all(len(layer[name]) == blocks for layer in cache for name in "kv")
+    slots = [slot for layer in cache for name in "kv" for slot in layer[name]]
+    assert len({slot.values.data_ptr() for slot in slots}) == len(slots)
+    assert all(torch.equal(slot.values, zero.values) and torch.equal(slot.amax, zero.amax) for slot in slots)
+
+
 def test_nvfp4_checkpoint_helpers_on_plain_dictionaries():
     from types import SimpleNamespace
 

@@ -221,7 +221,8 @@ int ll_nvfp4_gemm_tnt_fused(const uint8_t* A_values, const uint8_t* A_scales, co
  * ll_nvfp4_quantize (x_sink NULL) or ll_nvfp4_quantize_from_sink of x [M, K] and ll_nvfp4_gemm_tnt_fused of the result, in one
  * launch and with the same bits.  For small activations: LL_ENOSUP, and nothing is launched, unless K is a multiple of 64 up to
  * 512, ldx a multiple of 8, x 16-byte aligned, the product one that ll_nvfp4_gemm_tnt computes in plain 64 x 64 tiles, for K
- * beyond 256 of no more tiles of 32 x 128 than compute units, and, without x_sink, M * K <= 65536.  B [Np, K], Np a multiple of 128.
+ * beyond 256 of no more tiles of 32 x 128 than compute units, and, without x_sink, M * K <= 65536, or where D overlaps x or the
+ * epilogue's sink is x_sink's buffer, which early workgroups would write while late ones read.  B [Np, K], Np a multiple of 128.
  */
 int ll_nvfp4_quantize_gemm(const void* x, int64_t M, int64_t K, int64_t ldx, int rule, const ll_amax_sink* x_sink,
                            float denom_a, const uint8_t* B_values, const uint8_t* B_scales, const float* amax_b,
@@ -494,9 +495,11 @@ typedef struct ll_row_norm {
  * ll_layer_norm_quantize (weight and bias, either may be NULL) of x bf16 [M, C], contiguous, and ll_nvfp4_gemm_tnt_grouped of
  * the result with `activation` on every product (alpha NULL), in one launch and with the same bits.  For small activations:
  * LL_ENOSUP, and nothing is launched, unless C is a multiple of 64 up to 256, the products ones that ll_nvfp4_gemm_tnt_grouped
- * computes in plain 64 x 64 tiles, and their tiles of 32 x 256 no more than two per compute unit.  row_norms (NULL or n_products; LL_ENOSUP
- * unless N <= 256 and the normed products' biases are 8-byte aligned): D receives the rows after WanRMSNorm with row_eps and, where asked for, RoPE; the product's sink their maximum.  exchange and spin_limit as
- * amax_sink and spin_limit of ll_adaln_quantize; the products' own sinks may be later epochs of the same buffer.
+ * computes in plain 64 x 64 tiles, and their tiles of 32 x 256 no more than two per compute unit, or where a D (or smooth) overlaps
+ * x or an operand of its normalization.  row_norms (NULL or n_products; LL_ENOSUP unless N <= 256 and the normed products' biases
+ * are 8-byte aligned): D receives the rows after WanRMSNorm with row_eps and, where asked for, RoPE; the product's sink their
+ * maximum.  exchange and spin_limit as amax_sink and spin_limit of ll_adaln_quantize; the products' own sinks may be later epochs
+ * of the same buffer.
  */
 int ll_nvfp4_norm_gemm(const void* x, int64_t M, int C, const void* scale, const void* shift, int64_t scale_stride,
                        int64_t shift_stride, int64_t frame_rows, int add_one_to_scale, const void* weight, const void* bias,

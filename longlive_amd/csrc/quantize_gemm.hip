@@ -368,6 +368,13 @@ void launch_quantize_gemm(const typename FusedParamsOf<ROWS>::type& p, int rule,
   }
 }
 
+// Whether two ranges of memory have a byte in common (none of them null and long).
+inline bool overlap(const void* a, int64_t bytes_a, const void* b, int64_t bytes_b) {
+  const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+  return a && b && x < y + (uintptr_t)bytes_b && y < x + (uintptr_t)bytes_a;
+}
+inline int64_t matrix_bytes(int64_t rows, int64_t cols, int64_t ld) { return 2 * ((rows - 1) * ld + cols); }
+
 }  // namespace ll
 
 extern "C" int ll_nvfp4_quantize_gemm(const void* x, int64_t M, int64_t K, int64_t ldx, int rule, const ll_amax_sink* x_sink, float denom_a,
@@ -385,6 +392,12 @@ extern "C" int ll_nvfp4_quantize_gemm(const void* x, int64_t M, int64_t K, int64
              "ll_nvfp4_quantize_gemm: operands must be 16-byte, D and bias 2-byte aligned");
   FusedParams p{};
   if (int rc = make_epilogue(*epilogue, N, p.epi)) return rc;
+  // Workgroups that begin late still read x and its maximum when others write results and leave their maxima: two launches do not mind
+  // where either lies in the place of the other.
+  constexpr int64_t kSinkBytes = (int64_t)kAmaxParts * sizeof(uint64_t);
+  if (overlap(D, matrix_bytes(M, N, ldd), x, matrix_bytes(M, K, ldx)) ||
+      (x_sink && overlap(x_sink->parts, kSinkBytes, epilogue->amax_sink.parts, kSinkBytes)))
+    return LL_ENOSUP;
   // Where the launch is ahead of quantization and product of their own.  A workgroup that reads the whole tensor for its maximum: up
   // to 65536 elements (a call with its host time, two launches / one, us: 64 x 512 x 512 12.4 / 9.9, 128 x 512 x 256 12.4 / 11.3; 192 x 512
   // x 512, beyond the line, 12.6 / 12.5 and on the GPU 9.9 / 12.2).
@@ -490,6 +503,15 @@ extern "C" int ll_nvfp4_norm_gemm(const void* x, int64_t M, int C, const void* s
     p.sinp = sin;
     p.seq_len = (int)(seq_len < M ? seq_len : M);
   }
+  // as in ll_nvfp4_quantize_gemm, and the recomputation of a late workgroup's share reads all of it again; the maxima have slots of their own
+  const int64_t frames = scale ? M / frame_rows : 1;
+  const struct { const void* at; int64_t bytes; } read[] = {{x, matrix_bytes(M, C, C)}, {scale, matrix_bytes(frames, C, scale_stride)},
+      {shift, matrix_bytes(frames, C, shift_stride)}, {weight, matrix_bytes(1, C, C)}, {bias, matrix_bytes(1, C, C)}};
+  for (int i = 0; i < n_products; ++i)
+    for (const auto& r : read)
+      if (overlap(products[i].D, matrix_bytes(M, N, products[i].ldd), r.at, r.bytes) ||
+          overlap(p.row_norm[i].smooth, matrix_bytes(M, N, products[i].ldd), r.at, r.bytes))
+        return LL_ENOSUP;
   if (C % 64 != 0 || C > kNormMaxK || M > (1 << 20) || N > (1 << 20)) return LL_ENOSUP;
   int dev = 0, cus = 0;
   if (hipGetDevice(&dev) != hipSuccess) {

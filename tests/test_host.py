@@ -99,6 +99,45 @@ def test_a_bias_at_any_element_is_left_to_the_separate_launches(offset):
                                   ctypes.byref(product), 0, ctypes.byref(row_norm), 1e-6, None, None, 0, None) == -3
 
 
+@pytest.mark.parametrize("x,d,x_sink,d_sink", [
+    (0, 0, None, None),            # D in the place of x
+    (0, 64, None, None),           # behind x's first rows
+    (64, 64 - 4 * 2 * 64 + 2, None, None),   # D's last element in x's first
+    (0, 4096, 16384, 16384),       # the maximum of x and that of D, epochs of one buffer
+    (0, 4096, 16384, 16384 + 8 * 1023),      # buffers with one slot in common
+])
+def test_a_small_layer_whose_result_lies_where_it_reads_is_left_to_two_launches(x, d, x_sink, d_sink):
+    """ll_nvfp4_quantize_gemm (LL_ENOSUP = -3): workgroups that begin late read x and its maximum after others have written results
+    and left their maxima."""
+    import ctypes
+    lib = _native.load()
+    buf = (ctypes.c_uint8 * 65536)()                    # aligned host memory: only its address is looked at
+    ptr = ctypes.addressof(buf) + (-ctypes.addressof(buf)) % 256 + 1024
+    sink = lambda at, epoch: _native.AmaxSinkStruct() if at is None else _native.AmaxSinkStruct(ptr + at, epoch, None)
+    epilogue = _native.GemmEpilogue(None, 0, None, 0, 0, None, 0, sink(d_sink, 2))
+    given = sink(x_sink, 1)
+    assert lib.ll_nvfp4_quantize_gemm(ptr + x, 4, 64, 64, 3, None if x_sink is None else ctypes.byref(given), 1536.0, ptr + 60000 // 16 * 16,
+                                      ptr, ptr, 1536.0, 64, 128, ptr + d, 64, ctypes.byref(epilogue), None) == -3
+
+
+@pytest.mark.parametrize("given", ["x", "scale", "shift", "weight", "bias"])
+@pytest.mark.parametrize("where", ["D", "smooth"])
+def test_small_layers_behind_a_norm_whose_results_lie_where_it_reads_are_left_to_separate_launches(given, where):
+    import ctypes
+    lib = _native.load()
+    buf = (ctypes.c_uint8 * (1 << 17))()
+    ptr = ctypes.addressof(buf) + (-ctypes.addressof(buf)) % 256
+    at = {name: ptr + 16384 * i for i, name in enumerate(("x", "scale", "shift", "weight", "bias", "rest", "D"))}
+    adaln = given in ("x", "scale", "shift")
+    d = at[given] if where == "D" else at["D"]
+    product = _native.GemmProduct(at["rest"], at["rest"], None, at["rest"], 1536.0, d, 128, None, _native.AmaxSinkStruct())
+    row_norm = _native.RowNorm(at["rest"], at[given] if where == "smooth" else None, 0)
+    exchange = _native.AmaxSinkStruct(at["rest"], 1, None)
+    norm = (at["scale"], at["shift"], 64, 64, 16, 1, None, None) if adaln else (None, None, 0, 0, 1, 0, at["weight"], at["bias"])
+    assert lib.ll_nvfp4_norm_gemm(at["x"], 32, 64, *norm, 1e-6, 3, ctypes.byref(exchange), 64, 1536.0, 128, 128, 1, ctypes.byref(product), 0,
+                                  ctypes.byref(row_norm), 1e-6, None, None, 0, None) == -3
+
+
 def test_noalloc_quantize_refuses_inputs_beyond_its_limit_before_touching_the_gpu():
     lib = _native.load()
     limit = lib.ll_nvfp4_quantize_noalloc_max_elements()

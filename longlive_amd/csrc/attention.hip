@@ -1207,6 +1207,8 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) 
   // that either is under way while the other is worked on.
   if (t < n_tiles) {
     if (CACHED) {
+      // The last cached tile's V rows are read: the loads that replace them are none that the compiler would wait ahead of.
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       fetch_k(t);
       fetch_v();
     }

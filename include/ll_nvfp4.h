@@ -483,6 +483,9 @@ int ll_layer_norm_quantize(const void* x, int64_t rows, int C, const void* weigh
                            int rule, uint8_t* values, uint8_t* scales, float* amax, const ll_amax_sink* amax_sink,
                            int64_t spin_limit, void* stream);
 
+/* The widest activation that ll_nvfp4_norm_gemm takes. */
+#define LL_NORM_GEMM_MAX_C 256
+
 /* What ll_nvfp4_norm_gemm does with whole rows of a product, as ll_rms_norm and ll_qk_norm_rope_pair_amax do with them. */
 typedef struct ll_row_norm {
   const void* weight; /* bf16 [N] of WanRMSNorm; NULL: the rows stay as they are */
@@ -494,7 +497,7 @@ typedef struct ll_row_norm {
  * ll_adaln_quantize (scale and shift given: bf16 rows scale_stride and shift_stride elements apart, one per frame_rows rows of x) or
  * ll_layer_norm_quantize (weight and bias, either may be NULL) of x bf16 [M, C], contiguous, and ll_nvfp4_gemm_tnt_grouped of
  * the result with `activation` on every product (alpha NULL), in one launch and with the same bits.  For small activations:
- * LL_ENOSUP, and nothing is launched, unless C is a multiple of 64 up to 256, the products ones that ll_nvfp4_gemm_tnt_grouped
+ * LL_ENOSUP, and nothing is launched, unless C is a multiple of 64 up to LL_NORM_GEMM_MAX_C, the products ones that ll_nvfp4_gemm_tnt_grouped
  * computes in plain 64 x 64 tiles, and their tiles of 32 x 256 no more than two per compute unit, or where a D (or smooth) overlaps
  * x or an operand of its normalization.  row_norms (NULL or n_products; LL_ENOSUP unless N <= 256 and the normed products' biases
  * are 8-byte aligned): D receives the rows after WanRMSNorm with row_eps and, where asked for, RoPE; the product's sink their

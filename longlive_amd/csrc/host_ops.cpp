@@ -483,12 +483,10 @@ PyObject* py_block_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
     return code ? code : c.quantize_from(y, L, C, q, again);
   };
   // The layers behind a normalization of h [L, C] (adaLN with the modulation vectors `scale` and `shift`, or norm3 where scale is
-  // negative): one launch for small activations, else `operand(exchange)` and `product()`.  result_sink: the sink of the first
-  // product where it is to have a fresh epoch, which has to be newer than those of the launches before it.
-  TempOperand xq{};  // allocated by the first that needs it
-  const bool whole_rows = C <= 256;  // a workgroup of ll_nvfp4_norm_gemm has them: the norms and RoPE of q and k are part of it
+  // negative) in one launch, for small activations.  LL_ENOSUP, as for every wider block: nothing is launched, `exchange` is unused.
   auto norm_gemm = [&](const void* h, int scale, int shift, const ll_amax_sink& exchange, const Layer* const* layers, int n, void* const* outs,
                        const ll_amax_sink* sinks, int activation, const ll_row_norm* row_norms, float row_eps) -> int {
+    if (C > LL_NORM_GEMM_MAX_C) return LL_ENOSUP;
     ll_gemm_product p[4];
     BlockCall::products(layers, n, outs, sinks, p);
     const bool adaln = scale >= 0;
@@ -497,17 +495,7 @@ PyObject* py_block_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
                               c.denom_a, layers[0]->n, layers[0]->np, n, p, activation, row_norms, row_eps, cos->data_ptr<float>(),
                               sin->data_ptr<float>(), L, c.stream);
   };
-  auto normed_layers = [&](const void* h, int scale, int shift, const Layer* const* layers, int n, void* const* outs, const ll_amax_sink* sinks,
-                           ll_amax_sink* result_sink, int activation, auto operand, auto product) -> int {
-    const ll_amax_sink exchange = ep.take();
-    if (result_sink) *result_sink = ep.take();
-    int code = norm_gemm(h, scale, shift, exchange, layers, n, outs, sinks ? sinks : result_sink, activation, nullptr, 0.f);
-    if (code != LL_ENOSUP) return code;
-    if (!xq.values) xq = c.operand(L, C);
-    if ((code = operand(exchange))) return code;
-    if (result_sink) *result_sink = ep.take();
-    return product();
-  };
+  TempOperand xq{};  // allocated by the first that needs it
 
   // ---- self-attention
   const Tensor value = empty({1, L, H, 128}, at::kBFloat16, dev), key = empty({1, L, H, 128}, at::kBFloat16, dev);
@@ -516,21 +504,17 @@ PyObject* py_block_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
   {
     const Tensor roped_q = empty({L, C}, at::kBFloat16, dev), smooth_k = empty({L, C}, at::kBFloat16, dev);
     const Layer* const layers[3] = {&w[Q], &w[K], &w[V]};
-    int code = LL_ENOSUP;
-    if (whole_rows) {
-      void* const outs[3] = {roped_q.data_ptr(), key.data_ptr(), value.data_ptr()};
-      const ll_row_norm row_norms[3] = {{norm[0], nullptr, 1}, {norm[1], smooth_k.data_ptr(), 1}, {nullptr, nullptr, 0}};
-      const ll_amax_sink sinks[3] = {{nullptr, 0, nullptr}, kv_sink[0], kv_sink[1]};
-      code = norm_gemm(x.data_ptr(), 1, 0, ep.take(), layers, 3, outs, sinks, LL_ACT_NONE, row_norms, eps[1]);
-    }
+    void* const normed[3] = {roped_q.data_ptr(), key.data_ptr(), value.data_ptr()};
+    const ll_row_norm row_norms[3] = {{norm[0], nullptr, 1}, {norm[1], smooth_k.data_ptr(), 1}, {nullptr, nullptr, 0}};
+    const ll_amax_sink exchange = ep.take(), normed_sinks[3] = {{nullptr, 0, nullptr}, kv_sink[0], kv_sink[1]};
+    int code = norm_gemm(x.data_ptr(), 1, 0, exchange, layers, 3, normed, normed_sinks, LL_ACT_NONE, row_norms, eps[1]);
     if (code == LL_ENOSUP) {
       const Tensor q = empty({L, C}, at::kBFloat16, dev), k = empty({L, C}, at::kBFloat16, dev);
       void* const outs[3] = {q.data_ptr(), k.data_ptr(), value.data_ptr()};
       const ll_amax_sink sinks[3] = {{nullptr, 0, nullptr}, {nullptr, 0, nullptr}, kv_sink[1]};
-      LL_TRY(normed_layers(x.data_ptr(), 1, 0, layers, 3, outs, sinks, nullptr, LL_ACT_NONE,
-                           [&](const ll_amax_sink& sink) { return adaln_operand(x.data_ptr(), 1, 0, xq, sink); },
-                           [&] { return c.grouped(xq, layers, 3, L, outs, sinks); }),
-             "adaLN and q / k / v projections");
+      xq = c.operand(L, C);
+      LL_TRY(adaln_operand(x.data_ptr(), 1, 0, xq, exchange), "adaLN");
+      LL_TRY(c.grouped(xq, layers, 3, L, outs, sinks), "q / k / v projections");
       code = ll_qk_norm_rope_pair_amax(q.data_ptr(), k.data_ptr(), L, H, norm[0], norm[1], eps[1], cos->data_ptr<float>(), sin->data_ptr<float>(),
                                        L, roped_q.data_ptr(), key.data_ptr(), smooth_k.data_ptr(), &kv_sink[0], c.stream);
     }
@@ -574,18 +558,15 @@ PyObject* py_block_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
   {
     const Tensor qn = empty({L, C}, at::kBFloat16, dev);
     const Layer* const layers[1] = {&w[CQ]};
-    int code = LL_ENOSUP;
-    if (whole_rows) {
-      void* const outs[1] = {qn.data_ptr()};
-      const ll_row_norm row_norms[1] = {{norm[4], nullptr, 0}};
-      code = norm_gemm(x1.data_ptr(), -1, -1, ep.take(), layers, 1, outs, nullptr, LL_ACT_NONE, row_norms, eps[3]);
-    }
+    void* const normed[1] = {qn.data_ptr()};
+    const ll_row_norm row_norms[1] = {{norm[4], nullptr, 0}};
+    const ll_amax_sink exchange = ep.take();
+    int code = norm_gemm(x1.data_ptr(), -1, -1, exchange, layers, 1, normed, nullptr, LL_ACT_NONE, row_norms, eps[3]);
     if (code == LL_ENOSUP) {
       const Tensor q = empty({L, C}, at::kBFloat16, dev);
-      void* const outs[1] = {q.data_ptr()};
-      LL_TRY(normed_layers(x1.data_ptr(), -1, -1, layers, 1, outs, nullptr, nullptr, LL_ACT_NONE, norm3_operand,
-                           [&] { return c.gemm(xq, w[CQ], L, q.data_ptr(), plain_epilogue); }),
-             "norm3 and cross-attention q");
+      if (!xq.values) xq = c.operand(L, C);
+      LL_TRY(norm3_operand(exchange), "norm3");
+      LL_TRY(c.gemm(xq, w[CQ], L, q.data_ptr(), plain_epilogue), "cross-attention q");
       code = ll_rms_norm(q.data_ptr(), L, (int)C, norm[4], eps[3], qn.data_ptr(), c.stream);
     }
     LL_TRY(code, "cross-attention q");
@@ -627,10 +608,16 @@ PyObject* py_block_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
   {
     const Layer* const layers[1] = {&w[UP]};
     void* const outs[1] = {hidden.data_ptr()};
-    LL_TRY(normed_layers(x2.data_ptr(), 4, 3, layers, 1, outs, nullptr, &gelu.amax_sink, LL_ACT_GELU_TANH,
-                         [&](const ll_amax_sink& sink) { return adaln_operand(x2.data_ptr(), 4, 3, xq, sink); },
-                         [&] { return c.gemm(xq, w[UP], L, hidden.data_ptr(), gelu); }),
-           "adaLN and FFN up");
+    const ll_amax_sink exchange = ep.take();
+    gelu.amax_sink = ep.take();  // newer than the exchange, and below newer than what adaLN may take behind it
+    int code = norm_gemm(x2.data_ptr(), 4, 3, exchange, layers, 1, outs, &gelu.amax_sink, LL_ACT_GELU_TANH, nullptr, 0.f);
+    if (code == LL_ENOSUP) {
+      if (!xq.values) xq = c.operand(L, C);
+      LL_TRY(adaln_operand(x2.data_ptr(), 4, 3, xq, exchange), "adaLN");
+      gelu.amax_sink = ep.take();
+      code = c.gemm(xq, w[UP], L, hidden.data_ptr(), gelu);
+    }
+    LL_TRY(code, "FFN up");
   }
   TempOperand hq{};
   const Tensor& out = attended;  // its memory is free by now

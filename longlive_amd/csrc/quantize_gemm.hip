@@ -21,7 +21,7 @@ namespace ll {
 // workgroup fewer compute units are busy (48 x 256 x 512 7.2 instead of 6.1 us).
 constexpr int kFusedThreads = 512;
 constexpr int kFusedRows = 32;  // of a workgroup's tile: a wave multiplies all rows and 32 columns
-constexpr int kFusedMaxK = 512, kNormMaxK = 256;
+constexpr int kFusedMaxK = 512, kNormMaxK = LL_NORM_GEMM_MAX_C;
 constexpr int kFusedPatch = 32 * (64 + 16);       // bytes of a wave's patch in the epilogue
 
 struct FusedParams {

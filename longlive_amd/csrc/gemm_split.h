@@ -218,9 +218,11 @@ inline int64_t small_product_units(int cus) { return 2 * (int64_t)cus; }  // mos
 // 8960 33.3 / 30.5, 440 x 3072 x 14336 50.4 / 45.2).  Larger ones were measured too: 64 x 128 and 96 x 128 were never ahead
 // of both, 128 x 128 by 6 % on 2048 x 2048 x 3072.
 // Two sets of four waves (one workgroup per unit, so a second wave on every SIMD) from 2048 elements of K on: a step then takes
-// 0.71 us where every unit is busy, with one set 0.83, and the sets' sums meet at the end.  us, one set / two: 736 x 1536 x 8960
-// 33.9 / 30.2, 512 x 3072 x 14336 53.2 / 47.0, x 3072 16.0 / 15.3, 450 x 2816 x 3328 16.65 / 15.9, 736 x 1536 x 2304 12.75 / 12.55, x 2048
-// 11.9 / 11.8, but 512 x 3072 x 1792 11.5 / 11.7, 736 x 1536 x 1536 10.4 / 10.5, 512 x 3072 x 1024 9.0 / 9.3.
+// 0.71 us where every unit is busy, with one set 0.83, and the sets' sums meet at the end.  us, one set / two, the product by
+// itself: 736 x 1536 x 8960 33.9 / 30.2, 512 x 3072 x 14336 53.2 / 47.0, 736 x 1536 x 2304 12.75 / 12.55, x 2048 11.9 / 11.8, but 512 x
+// 3072 x 1792 11.5 / 11.7, 736 x 1536 x 1536 10.4 / 10.5, 512 x 3072 x 1024 9.0 / 9.3; a call of a linear layer, its quantization with
+// it: 736 x 1536 x 8960 43.1 / 38.8, x 6144 34.6 / 31.9, x 3072 22.95 / 22.2, x 2560 20.3 / 19.9, x 2304 19.2 / 19.0, x 2048 18.0 / 18.0, 512 x
+// 3072 x 14336 58.4 / 54.1, x 4096 24.6 / 23.5, x 3072 21.1 / 20.4, x 2560 19.3 / 19.0, x 2048 17.9 / 17.85, 450 x 2816 x 3328 22.1 / 21.4.
 constexpr int64_t kSmallSetsK = 2048;
 struct SmallGemmPlan {
   int fb;  // tiles of 64 rows by 32 fb columns

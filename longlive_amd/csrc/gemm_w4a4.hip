@@ -895,7 +895,7 @@ __global__ __launch_bounds__(SETS * kSmallThreads, WHOLE ? 1 : 2) void gemm_w4a4
   };
   // One K step from the packed words in h; the words of the step behind it are read into `next` half way through,
   // when every wave has its loads of that step in LDS and has read this step's stage for the last time (the stage is
-  // then refilled with the step four further on), so that neither the barrier nor the LDS latency is waited out.
+  // then refilled with the step kStages further on), so that neither the barrier nor the LDS latency is waited out.
   auto step = [&](int t, auto stage, Raw& h, Raw& next) __attribute__((always_inline)) {
     constexpr int kStageNo = decltype(stage)::value;
     half2v s2[kFragments][2];
@@ -959,7 +959,8 @@ __global__ __launch_bounds__(SETS * kSmallThreads, WHOLE ? 1 : 2) void gemm_w4a4
       end = first_step(p + 1);
     }
   } else if constexpr (SETS == 2) {
-    const int end = all_steps > 1 ? (all_steps + 1 - set) / 2 : 1;  // no barrier stands in the last step, which set 1 may have none of
+    static_assert(kSmallSetsK >= 2 * kSmallK, "a step for either set");
+    const int end = (all_steps + 1 - set) / 2;  // no barrier stands in the last step, which set 1 may have none of
 #pragma unroll 1
     for (int t = 0;;) {
       step(t, kS0, h0, h1);

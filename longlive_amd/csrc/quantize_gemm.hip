@@ -127,7 +127,7 @@ __global__ __launch_bounds__(kFusedThreads, fused_waves(ROWS)) void quantize_gem
     lo[i] = src[0];
     hi[i] = src[1];
   }
-  // normalized rows: the wave's eight rows of the tile (behind the last row: the last again), with their operands
+  // normalized rows: the wave's four rows of the tile, two pairs (behind the last row: the last again), with their operands
   constexpr int kPairs = kWaveRows / 2;
   uint4 xraw[kPairs][1], araw[kPairs][1], braw[kPairs][1];
   if constexpr (kNorm) {

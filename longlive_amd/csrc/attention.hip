@@ -29,6 +29,7 @@
 #include <cfloat>
 #include <map>
 #include <mutex>
+#include <type_traits>
 #include <utility>
 
 namespace ll {
@@ -135,7 +136,7 @@ __device__ __forceinline__ void fp4x8_to_f32(uint32_t w, half2v s2, float gs, fl
 // is re-derived from the key index when the data is decoded.
 struct KRaw {         // K or V of one key, one quarter of the head dimension (32 elements)
   uint4 v;            // 16 packed bytes
-  uint32_t scales;    // 2 e4m3 block scales (low 16 bits)
+  uint16_t scales;    // 2 e4m3 block scales (low 16 bits)
 };
 
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
@@ -272,6 +273,12 @@ __device__ __forceinline__ void write_rows(const float16v (&o)[N], float inv_l, 
       out_max = abs_max_bf16x8(v, out_max);
     }
   }
+}
+
+// f(0), f(1), ... with every index a constant of its own type.
+template <typename F, int... I>
+__device__ __forceinline__ void each_index(F& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
 }
 
 template <bool WIDE>
@@ -531,6 +538,179 @@ __global__ __launch_bounds__(kAttnThreads) void kv_attention_kernel(AttnParams p
     l_run += sum;
   };
 
+  // 256-query tiles, iterations whose 128 keys are all there: 64 slots of one MFMA with what is to run beside it, held in place by
+  // scheduling barriers, in which no instruction waits for another.  S^T of both tiles of 64 keys comes first, then O^T of both;
+  // the probabilities of the first tile are formed under the second S^T, those of the second under the first O^T, and the next
+  // iteration's K and V are converted under the first S^T and the second O^T.
+  // The reference point is softmax_pv's, bit for bit, without a maximum per tile: while the probabilities that a lane has of a tile
+  // add up to no more than 128, none of them is above 2^7, and softmax_pv would have raised nothing.  Where they add up to more (a
+  // segment's first tile and a handful behind it; NaN, too) follow_maximum does what softmax_pv does and forms the tile's
+  // probabilities again, and it is to be reached before the first of them is multiplied: hence this order.
+  // What bounds the loop is the power limit: the MFMA pipe is busy 59 % of the cycles at 1.74 GHz with 7.1 vector instructions per
+  // MFMA, where with a maximum per tile it was 54 % at 1.81 GHz with 8.0, so what counts is what is not executed.  Raw bytes are
+  // asked for without branches, behind which the compiler waits for every load under way.  us, with a maximum per tile and the
+  // softmax in a burst behind each S^T / so: 2640 queries x 24 heads over 10560 cached + 2640 keys 419 / 404, 7040 x 24 over 21120 +
+  // 7040 2254 / 2152, 2328 x 16 over 9312 + 2328 232 / 221; where a key far above the others raises the reference point every
+  // fourth iteration, the first shape 398 / 392.  With the packing left to the compiler, which sinks it behind the branch, so
+  // that 32 values stay in place of 16, 453.
+  int it = seg_begin;
+  auto wide_iteration = [&](auto convert_tag) __attribute__((always_inline)) {
+    constexpr bool kConvert = decltype(convert_tag)::value;
+    typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(3))) bf16x4* lds_bf16x4_t;
+    const uint8_t* cur = smem + (it & 1) * kStageBytes;
+    uint8_t* nxt = smem + ((it + 1) & 1) * kStageBytes;
+    const uint8_t* k_lane = cur + l32 * kKPitch + lh * 16;
+    const uint8_t* v_lane = cur + 2 * kKTileBytes + (4 * lh + ((lane & 15) >> 2)) * kVPitch + (16 * ((lane >> 4) & 1) + 4 * (lane & 3)) * 2;
+    uint8_t* kdst = nxt + k_dst_off;
+    uint8_t* vdst = nxt + v_dst_off;
+    constexpr int kAhead = 5, kRing = 6;
+    uint4 fk[kRing];
+    bf16x4 fv[2][4][2];
+    float16v sc[2][2];
+    uint32_t pw[2][16];
+    half2v s2[2], t[4];
+    float v8[8], x[2][2], e[2][2];
+    float neg = -m_run * p.scale_log2, sum = 0.0f;
+    const float gs_k = k_gs, gs_v = v_gs;
+    const uint8_t *values, *scales;  // where the raw registers are filled from next
+    bool there;
+    auto read_k = [&](auto tag) __attribute__((always_inline)) {  // fragment f % 16 of the 64 keys f / 16
+      constexpr int f = decltype(tag)::value;
+      fk[f % kRing] = *reinterpret_cast<const uint4*>(k_lane + (f >> 4) * kKTileBytes + ((f >> 3) & 1) * 32 * kKPitch + (f & 7) * 32);
+    };
+    // The tile's probabilities are there, none of them multiplied yet.
+    auto follow_maximum = [&](float16v (&s)[2], uint32_t (&w)[16]) __attribute__((always_inline)) {
+      if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(sum <= 128.0f)) != 0, 0)) {
+        float mx = s[0][0];
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[kt][r]);
+        mx = max_over_wave_halves(mx);
+        const bool raise = (mx - m_run) * p.scale_log2 > kRescaleStep;
+        if (__builtin_amdgcn_ballot_w64(raise) != 0) {
+          const float alpha = raise ? __builtin_amdgcn_exp2f((m_run - mx) * p.scale_log2) : 1.0f;
+          m_run = raise ? mx : m_run;
+          neg = -m_run * p.scale_log2;
+          l_run *= alpha;
+#pragma unroll
+          for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) o[dt][i] *= alpha;
+          sum = 0.0f;
+#pragma unroll
+          for (int pair = 0; pair < 16; ++pair) {
+            const float p0 = __builtin_amdgcn_exp2f(fmaf(s[pair >> 3][2 * (pair & 7)], p.scale_log2, neg));
+            const float p1 = __builtin_amdgcn_exp2f(fmaf(s[pair >> 3][2 * (pair & 7) + 1], p.scale_log2, neg));
+            sum += p0 + p1;
+            w[pair] = pack_bf16(p0, p1);
+          }
+        }
+      }
+      l_run += sum;
+      sum = 0.0f;
+    };
+    each_index(read_k, std::make_integer_sequence<int, kAhead>{});
+    __builtin_amdgcn_sched_barrier(0);
+    auto one_slot = [&](auto slot_tag) __attribute__((always_inline)) {
+      constexpr int slot = decltype(slot_tag)::value;
+      // LDS reads: K five slots ahead of its MFMA, V four
+      if constexpr (slot + kAhead < 32) read_k(std::integral_constant<int, slot + kAhead>{});
+      if constexpr (slot >= 28 && slot < 60) {
+        constexpr int u = slot - 28, step = (u >> 2) & 3, dt = u & 3;
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          fv[step & 1][dt][j] = __builtin_amdgcn_ds_read_tr16_b64_v4bf16(
+              (lds_bf16x4_t)(v_lane + (u >> 4) * kVTileBytes + (16 * step + 8 * j) * kVPitch + dt * 64));
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      // S^T of the first and the second 64 keys in slots 0-31 (32 keys after 32 keys), their O^T in slots 32-63
+      if constexpr (slot < 32) {
+        constexpr int h = slot >> 4, kt = (slot >> 3) & 1, ks = slot & 7;
+        const float16v zero = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+        sc[h][kt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, fk[slot % kRing]), qf[ks], ks == 0 ? zero : sc[h][kt], 0, 0, 0);
+      } else {
+        constexpr int u = slot - 32, h = u >> 4, step = (u >> 2) & 3, dt = u & 3;
+        const bf16x4(&v)[2] = fv[step & 1][dt];
+        const bf16x8 a = __builtin_shufflevector(v[0], v[1], 0, 1, 2, 3, 4, 5, 6, 7);
+        const bf16x8 b = __builtin_bit_cast(bf16x8, make_uint4(pw[h][4 * step], pw[h][4 * step + 1], pw[h][4 * step + 2], pw[h][4 * step + 3]));
+        o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, o[dt], 0, 0, 0);
+      }
+      // probabilities: a pair's multiply-adds, exponentials, packing and sum in three slots in a row
+      constexpr int kFirst[2] = {9, 29};
+      constexpr int g = slot < kFirst[1] ? 0 : 1, i = slot - kFirst[g];
+      if constexpr (i >= 2 && i < 18) {
+        constexpr int pair = i - 2;
+        pw[g][pair] = pack_bf16(e[pair & 1][0], e[pair & 1][1]);
+        asm volatile("" : "+v"(pw[g][pair]));  // here, and not sunk behind the branch to the MFMA that reads it
+        sum += e[pair & 1][0] + e[pair & 1][1];
+      }
+      if constexpr (i >= 1 && i < 17) {
+        constexpr int pair = i - 1;
+        e[pair & 1][0] = __builtin_amdgcn_exp2f(x[pair & 1][0]);
+        e[pair & 1][1] = __builtin_amdgcn_exp2f(x[pair & 1][1]);
+      }
+      if constexpr (i >= 0 && i < 16) {
+        constexpr int pair = i, kt = pair >> 3, r = 2 * (pair & 7);
+        x[pair & 1][0] = fmaf(sc[g][kt][r], p.scale_log2, neg);
+        x[pair & 1][1] = fmaf(sc[g][kt][r + 1], p.scale_log2, neg);
+      }
+      // conversion of the next tile: a dword's conversions, scaling, widening and packing in four slots in a row
+      constexpr int kK = slot < 8 ? slot : slot >= 28 && slot < 36 ? slot - 20 : -1, kV = slot >= 47 && slot < 63 ? slot - 47 : -1;
+      if constexpr (kConvert && (kK >= 0 || kV >= 0)) {
+        constexpr bool is_k = kK >= 0;
+        constexpr int piece = is_k ? kK : kV, j = piece >> 2;  // dword j of the row
+        const KRaw& raw = is_k ? kf : vf;
+        const uint32_t w = j == 0 ? raw.v.x : j == 1 ? raw.v.y : j == 2 ? raw.v.z : raw.v.w;
+        const float gs = is_k ? gs_k : gs_v;
+        if constexpr (piece == 0) block_scales_f16(raw.scales, s2);
+        if constexpr ((piece & 3) == 0) {
+          t[0] = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 0);
+          t[1] = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 1);
+          t[2] = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 2);
+          t[3] = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 3);
+        }
+        if constexpr ((piece & 3) == 1) {
+#pragma unroll
+          for (int n = 0; n < 4; ++n) t[n] = t[n] * s2[j >> 1];
+        }
+        if constexpr ((piece & 3) == 2) {
+#pragma unroll
+          for (int n = 0; n < 4; ++n) {
+            v8[2 * n] = widen_mul_lo(t[n], gs);
+            v8[2 * n + 1] = widen_mul_hi(t[n], gs);
+          }
+        }
+        if constexpr ((piece & 3) == 3)
+          reinterpret_cast<uint4*>(is_k ? kdst : vdst)[j] =
+              make_uint4(pack_bf16(v8[0], v8[1]), pack_bf16(v8[2], v8[3]), pack_bf16(v8[4], v8[5]), pack_bf16(v8[6], v8[7]));
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (slot == 28 || slot == 47) {
+        follow_maximum(sc[slot == 28 ? 0 : 1], pw[slot == 28 ? 0 : 1]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      // raw bytes of the iteration behind the next one, K and V each once its registers are free
+      if constexpr (kConvert && slot == 9) {
+        advance();
+        there = it + 2 < seg_end && iter_base + k_local < n_cached;
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if constexpr (kConvert && (slot == 32 || slot == 58)) {
+        const int from = there ? k_slot : 0;
+        values = (slot == 32 ? tab.kv : tab.vv)[from];
+        scales = (slot == 32 ? tab.ks : tab.vs)[from];
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if constexpr (kConvert && (slot == 37 || slot == 63)) {
+        fetch_row(values, scales, there ? k_vo : 0u, there ? k_so : 0u, slot == 37 ? kf : vf);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    each_index(one_slot, std::make_integer_sequence<int, 64>{});
+  };
+
   // prologue: the segment's first iteration into its stage, raw registers <- the second one
   fetch_next();
   if constexpr (!WIDE) {
@@ -550,12 +730,11 @@ __global__ __launch_bounds__(kAttnThreads) void kv_attention_kernel(AttnParams p
   __builtin_amdgcn_s_waitcnt(0x0F70);
 
   // Iterations whose own 128 keys all exist and whose successor is all FP4 form a prefix of the key range;
-  // they run the interleaved body: S^T (64 keys x 32 queries) = 16 MFMAs in eight steps of two, each step
-  // also converting one dword of the prefetched K row (even steps) or V row (odd steps) into the other LDS
-  // stage.  The rest (the bf16 chunk, the tail) runs the plain
-  // body in a loop of its own.
+  // they run the interleaved body: wide_iteration for 256-query tiles, and for 128-query tiles S^T (64 keys x 32 queries) = 16
+  // MFMAs in eight steps of two, each step also converting one dword of the prefetched K row (even steps) or V row (odd
+  // steps) into the other LDS stage.  The rest (the bf16 chunk, the tail) runs in a loop of its own, without conversion beside
+  // the MFMAs.
   const int n_fast = min(n_cached / kIterKeys, seg_end) - 1;
-  int it = seg_begin;
   if (wave_idle) {
     // A wave without queries: the conversion of its rows, the same number of barriers, nothing else.
     for (; it < n_fast; ++it) {
@@ -582,13 +761,13 @@ __global__ __launch_bounds__(kAttnThreads) void kv_attention_kernel(AttnParams p
       __syncthreads();
     }
   }
-  // Where this loop of 5 KB begins is worth 0.5 to 2 %: 256-query tiles whose key ranges are shared are fastest with its first
-  // instruction 32 bytes behind a 64-byte line, where these put it together with the register copies that the compiler sets in
-  // between.  us, 28 / 32 bytes behind the line: 2328 queries x 16 heads over 9312 cached + 2328 keys 244 / 241, on another card
-  // 237.5 / 235.7, 2856 x 16 over 11424 + 2856 338 / 333 and 331.7 / 329.4, 3088 x 24 over 3088 + 3088 263 / 259 and 256.2 / 254.7;
-  // whole tiles: 2640 x 24 over 10560 + 2640 413 / 411.5 and 408.9 / 406.9.
-  if constexpr (WIDE) asm volatile(".p2align 6\n\ts_nop 0\n\ts_nop 0\n\ts_nop 0\n\ts_nop 0");
-  for (; it < n_fast; ++it) {
+  if constexpr (WIDE) {
+    for (; it < n_fast; ++it) {
+      wide_iteration(std::true_type{});
+      __syncthreads();
+    }
+  }
+  for (; !WIDE && it < n_fast; ++it) {
     const uint8_t* cur = smem + (it & 1) * kStageBytes;
     uint8_t* nxt = smem + ((it + 1) & 1) * kStageBytes;
     const bool has_next2 = it + 2 < seg_end;
@@ -598,11 +777,9 @@ __global__ __launch_bounds__(kAttnThreads) void kv_attention_kernel(AttnParams p
     block_scales_f16(vf.scales, vs2);
     uint8_t* kdst = nxt + k_dst_off;
     uint8_t* vdst = nxt + v_dst_off;
-#pragma unroll
-    for (int h = 0; h < kHalves; ++h) {
-      const int tile = WIDE ? h : kp;
+    {
       float16v sc[2];
-      const uint8_t* krow0 = cur + tile * kKTileBytes + l32 * kKPitch + lh * 16;
+      const uint8_t* krow0 = cur + kp * kKTileBytes + l32 * kKPitch + lh * 16;
       const uint8_t* krow1 = krow0 + 32 * kKPitch;
 #pragma unroll
       for (int kt = 0; kt < 2; ++kt)
@@ -625,11 +802,10 @@ __global__ __launch_bounds__(kAttnThreads) void kv_attention_kernel(AttnParams p
         const bf16x8 fa0 = __builtin_bit_cast(bf16x8, fk[ks % 3][0]), fa1 = __builtin_bit_cast(bf16x8, fk[ks % 3][1]);
         sc[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa0, qf[ks], sc[0], 0, 0, 0);
         sc[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa1, qf[ks], sc[1], 0, 0, 0);
-        // One dword (8 elements) of the prefetched rows at a time.  One tile per wave: K in the even steps, V in the
-        // odd ones.  Two tiles per wave: every second step, K under the first tile's MFMAs and V under the second's.
-        if (!WIDE || (ks & 1) == 0) {
+        // One dword (8 elements) of the prefetched rows at a time, K in the even steps, V in the odd ones.
+        {
           const int j = ks >> 1;
-          const bool is_k = WIDE ? h == 0 : (ks & 1) == 0;
+          const bool is_k = (ks & 1) == 0;
           float v8[8];
           fp4x8_to_f32(is_k ? wk[j] : wv[j], is_k ? ks2[j >> 1] : vs2[j >> 1], is_k ? k_gs : v_gs, v8);
           reinterpret_cast<uint4*>(is_k ? kdst : vdst)[j] = make_uint4(pack_bf16(v8[0], v8[1]), pack_bf16(v8[2], v8[3]),
@@ -637,11 +813,9 @@ __global__ __launch_bounds__(kAttnThreads) void kv_attention_kernel(AttnParams p
         }
         __builtin_amdgcn_sched_barrier(0);
       }
-      if (h == kHalves - 1) {
-        advance();
-        if (has_next2) fetch_next();
-      }
-      softmax_pv(sc, cur + 2 * kKTileBytes + tile * kVTileBytes);
+      advance();
+      if (has_next2) fetch_next();
+      softmax_pv(sc, cur + 2 * kKTileBytes + kp * kVTileBytes);
     }
     __syncthreads();
   }
@@ -694,8 +868,12 @@ __global__ __launch_bounds__(kAttnThreads) void kv_attention_kernel(AttnParams p
         load_to_lds_b128(source(64 - kKPieces + chunk_wave, kVPitch), v_base, dst + 2 * kKTileBytes + (64 - kKPieces) * 1024);
       }
     }
+    const bool whole = WIDE && (it + 1) * kIterKeys <= Lk_i;  // no key missing
+    if constexpr (WIDE) {
+      if (whole && !wave_idle) wide_iteration(std::false_type{});
+    }
 #pragma unroll 1
-    for (int h = 0; h < kHalves; ++h) {
+    for (int h = whole ? kHalves : 0; h < kHalves; ++h) {
       const int tile = WIDE ? h : kp;
       const int tile_base = it * kIterKeys + tile * kTileKeys;
       if (tile_base >= Lk_i || wave_idle) break;

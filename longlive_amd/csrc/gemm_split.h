@@ -221,8 +221,9 @@ inline int64_t small_product_units(int cus) { return 2 * (int64_t)cus; }  // mos
 // 0.71 us where every unit is busy, with one set 0.83, and the sets' sums meet at the end.  us, one set / two, the product by
 // itself: 736 x 1536 x 8960 33.9 / 30.2, 512 x 3072 x 14336 53.2 / 47.0, 736 x 1536 x 2304 12.75 / 12.55, x 2048 11.9 / 11.8, but 512 x
 // 3072 x 1792 11.5 / 11.7, 736 x 1536 x 1536 10.4 / 10.5, 512 x 3072 x 1024 9.0 / 9.3; a call of a linear layer, its quantization with
-// it: 736 x 1536 x 8960 43.1 / 38.8, x 6144 34.6 / 31.9, x 3072 22.95 / 22.2, x 2560 20.3 / 19.9, x 2304 19.2 / 19.0, x 2048 18.0 / 18.0, 512 x
-// 3072 x 14336 58.4 / 54.1, x 4096 24.6 / 23.5, x 3072 21.1 / 20.4, x 2560 19.3 / 19.0, x 2048 17.9 / 17.85, 450 x 2816 x 3328 22.1 / 21.4.
+// it: 736 x 1536 x 8960 43.0 / 38.8, x 6144 34.5 / 31.9, x 3072 22.95 / 22.2, x 2560 20.3 / 19.95, x 2304 19.2 / 19.0, x 2048 18.2 / 18.2, 512 x
+// 3072 x 14336 59.6 / 54.5, x 4096 24.6 / 23.8, x 2560 19.3 / 19.0, x 2048 18.0 / 18.0, 450 x 2816 x 3328 22.15 / 21.4.  The same on two other
+// cards, but 512 x 3072 x 3072 21.1 / 20.4 on one and 21.1 / 21.1 to 21.5 on the others.
 constexpr int64_t kSmallSetsK = 2048;
 struct SmallGemmPlan {
   int fb;  // tiles of 64 rows by 32 fb columns

@@ -1179,6 +1179,14 @@ def test_scores_far_above_those_of_the_first_keys(gpu, policy, high, far):
 
 
 @pytest.mark.parametrize("policy", ["wide", "split"])
+@pytest.mark.parametrize("high,far", [(4.0, tuple(range(130, 1190, 5))), (7.6, (200, 700)), (7.6, tuple(range(1, 1200, 64))), (9.0, (100, 300, 1050))])
+def test_scores_about_the_step_of_the_reference_point(gpu, policy, high, far):
+    """The same where sums of probabilities pass the bound of wide tiles below which nothing can be raised, with and without a
+    query whose reference point then is, in the first and the second tile of an iteration."""
+    test_scores_far_above_those_of_the_first_keys(gpu, policy, high, far)
+
+
+@pytest.mark.parametrize("policy", ["wide", "split"])
 @pytest.mark.parametrize("Lq,H,T,cached,n_new", [(300, 2, 384, 1000, 200), (1344, 4, 0, 0, 1344)])
 def test_wide_tiles_weigh_a_dominating_key_exactly(gpu, policy, Lq, H, T, cached, n_new):
     """Queries along three times a key of their own, spread over all keys: its score lies some 19 or more above zero and the others'

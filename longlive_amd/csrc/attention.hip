@@ -868,7 +868,10 @@ __global__ __launch_bounds__(kAttnThreads) void kv_attention_kernel(AttnParams p
         load_to_lds_b128(source(64 - kKPieces + chunk_wave, kVPitch), v_base, dst + 2 * kKTileBytes + (64 - kKPieces) * 1024);
       }
     }
-    const bool whole = WIDE && (it + 1) * kIterKeys <= Lk_i;  // no key missing
+    // No key missing, and not the only such iteration of the segment, whose first tile has its probabilities formed twice: 2640
+    // queries x 24 heads over 226 keys 21.1 us in the plain body, 21.8 in slots, over 256 19.95 and 19.9, over 512 27.35 and 26.65, 7040 x
+    // 24 over 128 33.2 and 34.2, over 256 44.0 and 43.0, over 1024 105.7 and 99.7.
+    const bool whole = WIDE && (it + 1) * kIterKeys <= Lk_i && min(seg_end, Lk_i / kIterKeys) - seg_begin > 1;
     if constexpr (WIDE) {
       if (whole && !wave_idle) wide_iteration(std::false_type{});
     }

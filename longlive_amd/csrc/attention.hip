@@ -552,7 +552,8 @@ __global__ __launch_bounds__(kAttnThreads) void kv_attention_kernel(AttnParams p
   // softmax in a burst behind each S^T / so: 2640 queries x 24 heads over 10560 cached + 2640 keys 419 / 404, 7040 x 24 over 21120 +
   // 7040 2254 / 2152, 2328 x 16 over 9312 + 2328 232 / 221; where a key far above the others raises the reference point every
   // fourth iteration, the first shape 398 / 392.  With the packing left to the compiler, which sinks it behind the branch, so
-  // that 32 values stay in place of 16, 453.
+  // that 32 values stay in place of 16, 453.  The kernel then takes all 256 registers; the thread's index waits in scratch memory
+  // for the segment's end.
   int it = seg_begin;
   auto wide_iteration = [&](auto convert_tag) __attribute__((always_inline)) {
     constexpr bool kConvert = decltype(convert_tag)::value;
